@@ -1,0 +1,41 @@
+// Kernel arguments of the batched matrix products (matmul.hip, split_gemm.hip).
+#pragma once
+
+#include "common.hpp"
+#include "device_utils.hpp"
+
+namespace cg {
+
+struct MmArgs {
+    const uint32_t *A;
+    const uint32_t *B;
+    uint32_t *C;
+    uint32_t M, N, K;
+    int64_t a_sm, a_sk, b_sk, b_sn;
+    uint32_t nb;                    // collapsed batch axes
+    uint32_t bd[kMaxBatchAxes];     // extents, innermost first
+    FastDiv bdiv[kMaxBatchAxes];
+    int64_t a_bs[kMaxBatchAxes], b_bs[kMaxBatchAxes];
+    uint32_t batch;
+    uint32_t a_vec, b_vec;          // 16-byte loads along the unit-stride axis are legal
+    uint32_t ksplit;                // tiled kernels: values of k per workgroup along grid.z (a multiple of 32), 0 = all of K
+    uint32_t c_fmt;                 // mfma_gemm_dlds_kernel: kFmtWords, or the operands' narrow format: C holds its patterns, rounded in the store
+};
+
+__device__ __forceinline__ void batch_offsets(const MmArgs &a, uint32_t b, int64_t &oa, int64_t &ob) {
+    oa = 0;
+    ob = 0;
+    for (uint32_t d = 0; d < a.nb; d++) {
+        uint32_t q = fastdiv(b, a.bdiv[d]);
+        int64_t i = (int64_t)(b - q * a.bd[d]);
+        b = q;
+        oa += i * a.a_bs[d];
+        ob += i * a.b_bs[d];
+    }
+}
+
+// The f32 products of more than eight rows (split_gemm.hip).  `a` complete but for ksplit; C is the row-major result.
+// a_mfast / b_nfast: the operand's rows, not k, are its unit-stride axis.
+int launch_split_gemm(cg_backend *be, MmArgs a, bool a_mfast, bool b_nfast);
+
+} // namespace cg

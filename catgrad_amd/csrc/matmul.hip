@@ -9,21 +9,16 @@
 // axes form one run, the batch is folded into M (one tall GEMM instead of B small ones).
 //
 // Kernels
-//   mfma_gemm_kernel   256 threads = 2x2 waves, one template for three macro tiles: 128x128x32 (2x2
-//                      v_mfma_f32_32x32x2_f32 accumulators per wave, two workgroups per compute unit) for
-//                      f32 products, 128x64x32 when N is a small multiple of 64 or the product has at
-//                      most one 128x128 tile per compute unit, 256x256x32 (each wave a 128x128 block as
-//                      4x4 accumulators, all 256 accumulation registers, 144 KiB of LDS) for the 16-bit
-//                      and fp8 products and for x.y with a row-contiguous right operand when there is at
-//                      least one such tile per compute unit; HALF variants
-//                      narrow the tiles to bf16 / f16 on their way into LDS, or read operands that
-//                      pack_operand_kernel narrowed in memory (bf16 / f16 / fp8), and issue
-//                      v_mfma_f32_32x32x16_{bf16,f16} / v_mfma_scale_f32_32x32x64_f8f6f4.  Tiles of
-//                      k-contiguous operands are staged K-fastest in LDS (pitch 36 words: 128-bit fragment
-//                      reads and tile stores are both free of bank conflicts), those of row-contiguous f32
-//                      operands rows-fastest; whole tiles are loaded at fixed per-lane offsets without
-//                      tests; two LDS buffers, next tile's global loads in flight during
-//                      the MFMAs, XCD-aware tile order.  MFMA-bound: 2*M*N*K flop.
+//   split_gemm_kernel  (split_gemm.hip) every f32 product of more than eight rows.
+//   mfma_gemm_kernel   products of the narrow dtypes: 256 threads = 2x2 waves, 128x128x32 macro tiles (2x2 32x32
+//                      accumulators per wave) or, with at least one such tile per compute unit, 256x256x32
+//                      (each wave a 128x128 block as 4x4 accumulators, all 256 accumulation registers, 144 KiB
+//                      of LDS).  Tiles of words are narrowed to bf16 / f16 on their way into LDS (fp8 words to
+//                      bf16, which holds them exactly), or operands lie narrow in memory (pack_operand_kernel);
+//                      v_mfma_f32_32x32x16_{bf16,f16} / v_mfma_scale_f32_32x32x64_f8f6f4.  Staged K-fastest in
+//                      LDS; whole tiles are loaded at fixed per-lane offsets without tests; two LDS buffers,
+//                      next tile's global loads in flight during the MFMAs, XCD-aware tile order.
+//                      MFMA-bound: 2*M*N*K flop.
 //   skinny_kt_*        M <= 8 with K-contiguous B rows (decode-time linear layers and q.K^T),
 //                      HBM-bound streams of B (4*K*N bytes):
 //                      skinny_kt_wide / _narrow: a wave per output column (or per 4 columns, or a
@@ -43,8 +38,7 @@
 // Accumulation is f32 with fused multiply-add; the summation order differs from the
 // reference's `matrixmultiply::sgemm`, which is why the contract for matmul is 1e-3
 // relative (ndarray.rs:750-816 makes no promise on order either).
-#include "common.hpp"
-#include "device_utils.hpp"
+#include "gemm_args.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -52,34 +46,6 @@
 namespace cg {
 
 namespace {
-
-struct MmArgs {
-    const uint32_t *A;
-    const uint32_t *B;
-    uint32_t *C;
-    uint32_t M, N, K;
-    int64_t a_sm, a_sk, b_sk, b_sn;
-    uint32_t nb;                    // collapsed batch axes
-    uint32_t bd[kMaxBatchAxes];     // extents, innermost first
-    FastDiv bdiv[kMaxBatchAxes];
-    int64_t a_bs[kMaxBatchAxes], b_bs[kMaxBatchAxes];
-    uint32_t batch;
-    uint32_t a_vec, b_vec;          // 16-byte loads along the unit-stride axis are legal
-    uint32_t ksplit;                // mfma_gemm_kernel: values of k per workgroup along grid.z (a multiple of 32), 0 = all of K
-    uint32_t c_fmt;                 // mfma_gemm_dlds_kernel: kFmtWords, or the operands' narrow format: C holds its patterns, rounded in the store
-};
-
-__device__ __forceinline__ void batch_offsets(const MmArgs &a, uint32_t b, int64_t &oa, int64_t &ob) {
-    oa = 0;
-    ob = 0;
-    for (uint32_t d = 0; d < a.nb; d++) {
-        uint32_t q = fastdiv(b, a.bdiv[d]);
-        int64_t i = (int64_t)(b - q * a.bd[d]);
-        b = q;
-        oa += i * a.a_bs[d];
-        ob += i * a.b_bs[d];
-    }
-}
 
 // ------------------------------------------------------------------------------------------
 // MFMA kernel
@@ -159,22 +125,13 @@ __device__ __forceinline__ void load_tile(TileRegs<TR> &t, const uint32_t *base,
     }
 }
 
-// Stores the registers into an LDS tile: K-fastest, [TR][PITCH], for k-contiguous operands; rows-fastest, [BK][TR], for
-// row-contiguous ones.
-template <bool ROWS_FAST, int TR> __device__ __forceinline__ void store_tile(const TileRegs<TR> &t, float *lds) {
+// Stores the registers of a k-contiguous operand into an LDS tile, [TR][PITCH].
+template <int TR> __device__ __forceinline__ void store_tile(const TileRegs<TR> &t, float *lds) {
 #pragma unroll
     for (int h = 0; h < TileRegs<TR>::slots; h++) {
         uint32_t slot = threadIdx.x + h * kThreads;
-        if (!ROWS_FAST) {
-            uint32_t row = slot / (BK / 4), k = (slot % (BK / 4)) * 4;
-            *reinterpret_cast<float4v *>(lds + row * PITCH + k) = t.v[h];
-        } else {
-            // rows stay the fastest axis in LDS too, [BK][TR]: one 16-byte store, no transposition (eight lanes cover 32
-            // consecutive words); the fragments are then read a word at a time, 32 consecutive words per half wave
-            uint32_t row, k;
-            rows_fast_slot<TR>(slot, row, k);
-            *reinterpret_cast<float4v *>(lds + k * TR + row) = t.v[h];
-        }
+        uint32_t row = slot / (BK / 4), k = (slot % (BK / 4)) * 4;
+        *reinterpret_cast<float4v *>(lds + row * PITCH + k) = t.v[h];
     }
 }
 
@@ -229,18 +186,15 @@ template <bool ROWS_FAST, int HALF, int TR> __device__ __forceinline__ void stor
     }
 }
 
-// NT / MT: 32-wide MFMA tiles per wave along N / M (the block is 2 x 2 waves).  NT = 2, MT = 2: the
-// 128 x 128 macro tile; NT = 1: 128 x 64 (each wave a 64 x 32 strip) for products whose N is a small
-// multiple of 64, such as p.V with head_dim 64; NT = MT = 4: 256 x 256, each wave a 128 x 128 block in
-// 256 accumulation registers, one wave per SIMD: four times the matrix instructions between two
+// NT / MT: 32-wide MFMA tiles per wave along N / M (the block is 2 x 2 waves).  2: the 128 x 128 macro tile; 4: 256 x 256,
+// each wave a 128 x 128 block in 256 accumulation registers, one wave per SIMD: four times the matrix instructions between two
 // barriers and half the LDS traffic per flop, for products with enough tiles to fill the chip.
-// HALF: 0 f32 operands (v_mfma_f32_32x32x2_f32); 1 / 2: bfloat16 / binary16 operands (see above).
+// HALF: 1 / 2: words that are bfloat16 / binary16 values (see above; fp8 values are bfloat16 values too).
 // 3 / 4 / 5: operands that are ALREADY narrow in memory — bfloat16 / binary16 / fp8 (E4M3) patterns, k contiguous,
-// addressed as 32-bit words of 2 or 4 values (a.K counts words; see pack_operand).  The tile pipeline is the f32 one
-// word for word (16-byte global loads, K-fastest LDS rows of 32 words + 4, one 128-bit LDS read per fragment); a
+// addressed as 32-bit words of 2 or 4 values (a.K counts words; see pack_operand): (16-byte global loads, K-fastest LDS rows of 32 words + 4, one 128-bit LDS read per fragment); a
 // fragment then is 8 (16) consecutive k of a row and feeds one v_mfma_f32_32x32x16_{bf16,f16} (two
 // v_mfma_f32_32x32x16_fp8_fp8): a tile is 64 (128) deep in k, and half (a quarter) of the bytes move per flop.
-template <bool A_MFAST, bool B_NFAST, int NT, int MT = 2, int HALF = 0>
+template <bool A_MFAST, bool B_NFAST, int NT, int MT, int HALF>
 __global__ __launch_bounds__(kThreads) void mfma_gemm_kernel(const MmArgs a) {
     constexpr int BN = 64 * NT, BM = 64 * MT; // shadow the defaults
     constexpr bool WIDEN = HALF == 1 || HALF == 2; // f32 words narrowed on their way into LDS
@@ -255,8 +209,8 @@ __global__ __launch_bounds__(kThreads) void mfma_gemm_kernel(const MmArgs a) {
             store_tile_half<A_MFAST, HALF>(ta, reinterpret_cast<uint32_t *>(lds_a(buf)));
             store_tile_half<B_NFAST, HALF>(tb, reinterpret_cast<uint32_t *>(lds_b(buf)));
         } else {
-            store_tile<A_MFAST>(ta, lds_a(buf));
-            store_tile<B_NFAST>(tb, lds_b(buf));
+            store_tile(ta, lds_a(buf));
+            store_tile(tb, lds_b(buf));
         }
     };
 
@@ -281,14 +235,9 @@ __global__ __launch_bounds__(kThreads) void mfma_gemm_kernel(const MmArgs a) {
     const uint32_t m0 = tile_m * BM, n0 = tile_n * BN;
     int64_t oa, ob;
     batch_offsets(a, blockIdx.y, oa, ob);
-    // A product with too few tiles for the device is cut along k over grid.z: this workgroup multiplies k0 .. k0 + Kk and
-    // leaves its tile in slot (batch entry, split) of a.C, which then is scratch memory that splitk_reduce_kernel sums up
-    // in a fixed order.
-    const uint32_t k0 = blockIdx.z * a.ksplit;
-    const uint32_t Kk = a.ksplit ? min(a.K - k0, a.ksplit) : a.K;
-    const uint32_t *A = a.A + oa + (int64_t)k0 * a.a_sk;
-    const uint32_t *B = a.B + ob + (int64_t)k0 * a.b_sk;
-    uint32_t *C = a.C + ((uint64_t)blockIdx.y * gridDim.z + blockIdx.z) * a.M * a.N;
+    const uint32_t Kk = a.K;
+    const uint32_t *A = a.A + oa, *B = a.B + ob;
+    uint32_t *C = a.C + (uint64_t)blockIdx.y * a.M * a.N;
 
     const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     const uint32_t wm = (wave / 2) * (32 * MT), wn = (wave % 2) * (32 * NT); // wave quadrant
@@ -575,36 +524,6 @@ __global__ __launch_bounds__(kThreads) void mfma_gemm_kernel(const MmArgs a) {
         const uint32_t cur = kt & 1;
         const bool more = decltype(whole_next)::value || kt + 1 < nk;
         const float *la = lds_a(cur), *lb = lds_b(cur);
-        // One 8-deep chunk of the tile: lane group g supplies k = 8*kc + 4*g + t to the t-th MFMA,
-        // for A and B alike, so one 128-bit LDS read feeds four MFMAs.
-        auto chunk = [&](const int kc) {
-            float4v fa[MT], fb[NT];
-#pragma unroll
-            for (int i = 0; i < MT; i++) {
-                if constexpr (A_MFAST) {
-#pragma unroll
-                    for (int t = 0; t < 4; t++) fa[i][t] = la[(kc * 8 + lg * 4 + t) * BM + wm + i * 32 + li];
-                } else {
-                    fa[i] = *reinterpret_cast<const float4v *>(la + (wm + i * 32 + li) * PITCH + kc * 8 + lg * 4);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < NT; j++) {
-                if constexpr (B_NFAST) {
-#pragma unroll
-                    for (int t = 0; t < 4; t++) fb[j][t] = lb[(kc * 8 + lg * 4 + t) * BN + wn + j * 32 + li];
-                } else {
-                    fb[j] = *reinterpret_cast<const float4v *>(lb + (wn + j * 32 + li) * PITCH + kc * 8 + lg * 4);
-                }
-            }
-#pragma unroll
-            for (int t = 0; t < 4; t++)
-#pragma unroll
-                for (int i = 0; i < MT; i++)
-#pragma unroll
-                    for (int j = 0; j < NT; j++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][t], fb[j][t], acc[i][j], 0, 0, 0);
-        };
         // While a wave is in its burst of matrix instructions it wins issue arbitration against the other
         // wave of its SIMD (which is loading or storing a tile): the two stop advancing in lock-step and
         // their stalls at the barrier no longer coincide.
@@ -644,21 +563,9 @@ __global__ __launch_bounds__(kThreads) void mfma_gemm_kernel(const MmArgs a) {
                                                                                __builtin_bit_cast(f16x8, fb[j]), acc[i][j], 0, 0, 0);
                     }
             }
-        } else if constexpr (MT == 4) {
-            // one wave per SIMD: nobody else fills the time the staging of the next tile takes (for a row-contiguous
-            // operand 4-byte LDS stores and their addresses), so it goes between the two halves of the burst, by when
-            // the tile's global loads have long arrived; the other LDS buffer is written, the current one read
-#pragma unroll
-            for (int kc = 0; kc < BK / 16; kc++) chunk(kc);
-            if (more) stage(ra, rb, cur ^ 1);
-#pragma unroll
-            for (int kc = BK / 16; kc < BK / 8; kc++) chunk(kc);
-        } else {
-#pragma unroll
-            for (int kc = 0; kc < BK / 8; kc++) chunk(kc);
         }
         __builtin_amdgcn_s_setprio(0);
-        if (more && (HALF || MT != 4)) stage(ra, rb, cur ^ 1);
+        if (more) stage(ra, rb, cur ^ 1);
         __syncthreads();
         };
     {
@@ -1893,22 +1800,6 @@ __global__ __launch_bounds__(kThreads) void skinny_nn_kernel(const MmArgs a, uin
 }
 
 // The same four elements at a time (mn a multiple of 4, both arrays 16-byte aligned): the sums in the same fixed order.
-__global__ __launch_bounds__(kThreads) void splitk_reduce4_kernel(const float4v *part, float4v *C, uint32_t splits, uint32_t mn4, uint64_t total4) {
-    const uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (i >= total4) return;
-    const uint64_t b = i / mn4, e = i % mn4;
-    float4v v = {0.f, 0.f, 0.f, 0.f};
-    for (uint32_t s = 0; s < splits; s++) {
-        const float4v p = __builtin_nontemporal_load(part + (b * splits + s) * mn4 + e);
-        v[0] += p[0];
-        v[1] += p[1];
-        v[2] += p[2];
-        v[3] += p[3];
-    }
-    C[i] = v;
-}
-
-// C[b][e] = sum over s of part[b][s][e]   (e < M*N)
 __global__ __launch_bounds__(kThreads) void splitk_reduce_kernel(const uint32_t *part, uint32_t *C, uint32_t splits,
                                                                  uint32_t mn, uint64_t total) {
     uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
@@ -2552,37 +2443,14 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
     const int kind = half ? half : x->dt == CG_F8 ? 3 : 0;           // the narrow kernels' operand format (0: none)
     hipStream_t s = be->stream;
 
-    // ---- the tiled kernels' plan (used by the last branch below; here because it decides how operands are addressed) ----
-    // the narrow tile when the wide one would leave over a seventh of its columns empty, and when the product has at
-    // most one 128 x 128 tile per compute unit: twice the workgroups then fill the chip (4096 x 2048 x 512: 148 -> 83 us)
-    // or at least put two on a unit (8192 x 2048 x 512: 148 -> 145 us); with more tiles than that the wide one wins
-    // (env CG_GEMM_NARROW_BELOW=n moves the limit, for measurements)
-    const int64_t cols128 = (N + 127) / 128 * 128, cols64 = (N + 63) / 64 * 64;
-    static const int64_t narrow_below = [] { const char *e = getenv("CG_GEMM_NARROW_BELOW"); return e ? atoll(e) : 256ll; }();
-    const int64_t tiles128 = ((M + BM - 1) / BM) * (cols128 / 128) * (int64_t)batch;
-    const bool narrow = (cols128 * 7 > cols64 * 8 || (tiles128 <= narrow_below && N >= 128)) && !half; // (the 16-bit kernels come in the two square tiles)
-    const int bn = narrow ? 64 : 128;
-    // the 64 x 64 tile when even the narrow tile leaves most compute units without one (the linear layers of a short prompt on
-    // a narrow model: 512 x 576 is 36 tiles of 128 x 64): twice the workgroups, each cut along k half as often
-    // below 128 tiles of 128 x 64 — the SmolLM2-135M shape's prefill of 512 tokens 7.34 -> 6.84 ms, the Qwen3-0.6B shape's of
-    // 1024 unchanged (env CG_GEMM_TINY_BELOW=n moves the limit, for measurements; 0: never)
-    static const int64_t tiny_below = [] { const char *e = getenv("CG_GEMM_TINY_BELOW"); return e ? atoll(e) : 128ll; }();
-    const bool tiny = narrow && !kind && ((M + BM - 1) / BM) * (cols64 / 64) * (int64_t)batch < tiny_below && M > 64;
-    const int bm = tiny ? 64 : BM;
+    // ---- the narrow dtypes' tiled kernels' plan (used by the last branch below; here because it decides how operands are addressed) ----
     // the 256 x 256 tile when it covers the chip at least once (env CG_GEMM_BIG=0 switches it off)
     const uint64_t tiles_big = (uint64_t)((M + 255) / 256) * ((N + 255) / 256) * batch;
     static const bool big_allowed = [] {
         const char *e = getenv("CG_GEMM_BIG");
         return !(e && e[0] == '0');
     }();
-    const bool fits_big = big_allowed && !narrow && tiles_big >= 256 && M >= 256 && N >= 256;
-    // f32 words: since whole tiles are loaded without tests, two workgroups of the 128 x 128 tile per compute unit (two
-    // waves per SIMD covering each other's barriers) are as fast as one of the wide tile or faster — 137-138 against
-    // 134-135 TFLOP/s on the 1B shape's linear layers, and a partial last round costs a quarter as much (8192 x 2048 x
-    // 3072: 755 against 1015 us) — except with a k-contiguous left and a row-contiguous right operand (x.y: 1 % behind).
-    // The 16-bit and fp8 paths keep the wide tile (half the L2 bytes per flop, which is what bounds them).
-    const bool narrow_dtype = kind != 0;
-    const bool big = fits_big && (narrow_dtype || (!a_mfast && b_nfast));
+    const bool big = big_allowed && kind && tiles_big >= 256 && M >= 256 && N >= 256;
     // Operands of a narrow dtype in a product big enough for the 256 x 256 tile are multiplied from 2-byte / 1-byte
     // patterns: as they lie in memory when their buffer holds that format, else narrowed in memory first (the right
     // operand once per buffer) (env CG_GEMM_PACKED=0 switches it off).
@@ -2620,6 +2488,7 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
     const double bytes = distinct_bytes(x) + distinct_bytes(y) + distinct_bytes(out);
     const bool simple = K == 0 || !f32, skinny = !simple && M <= 8 && (a.b_sk == 1 || a.b_sn == 1);
     ProfScope prof(be, simple ? CG_K_GEMM_SIMPLE : skinny ? CG_K_GEMM_SKINNY : CG_K_GEMM_MFMA, skinny ? bytes : flop);
+    if (!simple && !skinny && !kind) return launch_split_gemm(be, a, a_mfast, b_nfast); // (no narrow dtype)
     if (K == 0 || !f32) {
         uint64_t elems = (uint64_t)M * N;
         dim3 grid((uint32_t)((elems + kThreads - 1) / kThreads), (uint32_t)batch);
@@ -2745,48 +2614,12 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
         }
 #undef CG_MM_SWITCH
     } else {
-        uint64_t tiles = big ? tiles_big / batch : (uint64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+        const uint64_t tiles = big ? tiles_big / batch : (uint64_t)((M + BM - 1) / BM) * ((N + 127) / 128);
         if (tiles > 0x7FFFFFFFull) return fail(CG_ERR_UNSUPPORTED, "matmul: too many tiles");
-        // Too few tiles for the device (the linear layers of a short prefill on a narrow model): cut along k as well, so that
-        // about two workgroups per compute unit run, each with at least 128 values of k; the partial tiles go to scratch memory
-        // and are summed in a fixed order (the same shape always gets the same cut: results are identical from run to run).
-        // (env CG_GEMM_SPLITK=0 switches it off)
-        static const bool splitk_allowed = [] {
-            const char *e = getenv("CG_GEMM_SPLITK");
-            return !(e && e[0] == '0');
-        }();
-        static const int64_t splitk_below = [] { const char *e = getenv("CG_GEMM_SPLITK_BELOW"); return e ? atoll(e) : 256ll; }();
-        static const int64_t splitk_target = [] { const char *e = getenv("CG_GEMM_SPLITK_TARGET"); return e ? atoll(e) : 512ll; }();
-        int64_t splits = 1;
-        uint32_t kchunk = 0;
-        if (splitk_allowed && !narrow_dtype && !big && (int64_t)(tiles * (uint64_t)batch) < splitk_below && K >= 256) {
-            const int64_t wgs = (int64_t)tiles * batch;
-            splits = std::min<int64_t>(std::min<int64_t>((splitk_target + wgs - 1) / wgs, K / 128), 16);
-            kchunk = (uint32_t)(((K + splits - 1) / splits + BK - 1) / BK * BK);
-            splits = (K + kchunk - 1) / kchunk;
-            if (splits < 2) {
-                splits = 1;
-                kchunk = 0;
-            }
-        }
-        void *kscratch = nullptr;
-        size_t kscratch_cls = 0;
-        if (splits > 1) {
-            int src = be->pool.alloc((size_t)batch * splits * M * N * 4, &kscratch, &kscratch_cls);
-            if (src) return src;
-            a.C = static_cast<uint32_t *>(kscratch);
-            a.ksplit = kchunk;
-        }
-        dim3 grid((uint32_t)tiles, (uint32_t)batch, (uint32_t)splits);
+        dim3 grid((uint32_t)tiles, (uint32_t)batch);
         static const bool lds_ok = [] { // the tiles need more than the default 64 KiB of dynamic LDS
             bool ok = true;
 #define CG_LDS(AF, BF)                                                                                                \
-    ok &= hipFuncSetAttribute(reinterpret_cast<const void *>(&mfma_gemm_kernel<AF, BF, 2>),                           \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_lds_bytes(128)) == hipSuccess;    \
-    ok &= hipFuncSetAttribute(reinterpret_cast<const void *>(&mfma_gemm_kernel<AF, BF, 1>),                           \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_lds_bytes(64)) == hipSuccess;     \
-    ok &= hipFuncSetAttribute(reinterpret_cast<const void *>(&mfma_gemm_kernel<AF, BF, 4, 4>),                        \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_lds_bytes(256, 256)) == hipSuccess; \
     ok &= hipFuncSetAttribute(reinterpret_cast<const void *>(&mfma_gemm_kernel<AF, BF, 4, 4, 1>),                     \
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_lds_bytes(256, 256, true)) == hipSuccess; \
     ok &= hipFuncSetAttribute(reinterpret_cast<const void *>(&mfma_gemm_kernel<AF, BF, 4, 4, 2>),                     \
@@ -2857,20 +2690,10 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
         else                                                                                                       \
             hipLaunchKernelGGL((mfma_gemm_kernel<AF, BF, 2, 2, H>), grid, dim3(kThreads), gemm_lds_bytes(128, 128, true), s, a); \
     } while (0)
-#define CG_GEMM(AF, BF)                                                                                            \
-    do {                                                                                                           \
-        if (half == 1) {                                                                                           \
-            CG_GEMM_HALF(AF, BF, 1);                                                                               \
-        } else if (half == 2) {                                                                                    \
-            CG_GEMM_HALF(AF, BF, 2);                                                                               \
-        } else if (big)                                                                                            \
-            hipLaunchKernelGGL((mfma_gemm_kernel<AF, BF, 4, 4>), grid, dim3(kThreads), gemm_lds_bytes(256, 256), s, a); \
-        else if (tiny)                                                                                             \
-            hipLaunchKernelGGL((mfma_gemm_kernel<AF, BF, 1, 1>), grid, dim3(kThreads), gemm_lds_bytes(64, 64), s, a); \
-        else if (narrow)                                                                                           \
-            hipLaunchKernelGGL((mfma_gemm_kernel<AF, BF, 1>), grid, dim3(kThreads), gemm_lds_bytes(64), s, a);     \
-        else                                                                                                       \
-            hipLaunchKernelGGL((mfma_gemm_kernel<AF, BF, 2>), grid, dim3(kThreads), gemm_lds_bytes(128), s, a);    \
+#define CG_GEMM(AF, BF)                    \
+    do {                                   \
+        if (half == 2) CG_GEMM_HALF(AF, BF, 2); \
+        else CG_GEMM_HALF(AF, BF, 1);      \
     } while (0)
         if (a_mfast) {
             if (b_nfast) CG_GEMM(true, true);
@@ -2881,18 +2704,6 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
         }
 #undef CG_GEMM
 #undef CG_GEMM_HALF
-        if (splits > 1) {
-            uint32_t *const dst = static_cast<uint32_t *>(out->buf->ptr);
-            const uint64_t mn = (uint64_t)M * N, total = mn * batch;
-            if (mn % 4 == 0 && reinterpret_cast<uintptr_t>(dst) % 16 == 0)
-                hipLaunchKernelGGL(splitk_reduce4_kernel, dim3((uint32_t)((total / 4 + kThreads - 1) / kThreads)), dim3(kThreads), 0, s,
-                                   static_cast<const float4v *>(kscratch), reinterpret_cast<float4v *>(dst), (uint32_t)splits,
-                                   (uint32_t)(mn / 4), total / 4);
-            else
-                hipLaunchKernelGGL(splitk_reduce_kernel, dim3((uint32_t)((total + kThreads - 1) / kThreads)), dim3(kThreads), 0, s,
-                                   static_cast<const uint32_t *>(kscratch), dst, (uint32_t)splits, (uint32_t)mn, total);
-            be->pool.free(kscratch, kscratch_cls); // stream-ordered: later users queue behind the reduce
-        }
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "matmul launch");

@@ -1,0 +1,74 @@
+"""f32 products of more than eight rows: multiplied in pieces of 8 significant bits, whatever the layout and wherever the tiles
+end, to the accuracy of 32-bit arithmetic; rows that the pieces cannot hold are multiplied as they are."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# edges of the tiles (32 x 256, 64 x 128, 128 x 128, 256 x 256), of a stage (16 values of k) and of the cuts along k
+SIZES = [(9, 16, 8), (9, 1, 33), (17, 33, 31), (32, 2048, 260), (33, 96, 128), (64, 100, 129), (65, 576, 192), (128, 160, 256), (129, 31, 4), (255, 64, 260),
+         (300, 1000, 520), (1030, 48, 1028), (2048, 64, 8192)]
+
+
+def operands(be, M, K, N, a_rows_fast, b_rows_fast, batch=1, seed=0):
+    rng = np.random.default_rng(seed)
+    a = rng.standard_normal((batch, M, K), dtype=np.float32)
+    b = rng.standard_normal((batch, K, N), dtype=np.float32) * np.float32(0.1)
+    x = be.transpose(be.from_numpy(np.ascontiguousarray(a.transpose(0, 2, 1))), 1, 2) if a_rows_fast else be.from_numpy(a)
+    y = be.from_numpy(b) if b_rows_fast else be.transpose(be.from_numpy(np.ascontiguousarray(b.transpose(0, 2, 1))), 1, 2)
+    return a, b, x, y
+
+
+def check(got, a, b):
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    K = a.shape[-1]
+    # three left-out products of pieces (2^-22 together at most), a rounding per 16 values of k and kept product, and up to 16
+    # partial sums, each relative to the sum of magnitudes
+    bound = (4.0 + 6 * ((K + 15) // 16) + 16) * 2.0 ** -24 * (np.abs(a) @ np.abs(b)) + 1e-37
+    assert (np.abs(got - a @ b) <= bound).all()
+
+
+@pytest.mark.parametrize("size", SIZES, ids=str)
+@pytest.mark.parametrize("layout", ["nt", "nn", "tt", "tn"])
+def test_layouts_and_edges(hip, size, layout):
+    M, K, N = size
+    a, b, x, y = operands(hip, M, K, N, layout[0] == "t", layout[1] == "n")
+    check(hip.to_numpy(hip.matmul(x, y)), a, b)
+
+
+def test_batches_and_unaligned_views(hip):
+    a, b, x, y = operands(hip, 70, 200, 90, False, False, batch=3)
+    check(hip.to_numpy(hip.matmul(x, y)), a, b)
+    x, y = hip.slice(x, 2, 3, 190), hip.slice(y, 1, 3, 190)   # rows begin 12 bytes behind a multiple of 16
+    check(hip.to_numpy(hip.matmul(x, y)), a[:, :, 3:193], b[:, 3:193])
+
+
+def test_a_row_of_the_unit_matrix_hands_values_through(hip):
+    rng = np.random.default_rng(5)
+    w = rng.standard_normal((1, 96, 200), dtype=np.float32) * np.exp(rng.uniform(-20, 20, (1, 96, 200))).astype(np.float32)
+    eye = np.eye(96, dtype=np.float32)[None]
+    np.testing.assert_array_equal(hip.to_numpy(hip.matmul(hip.from_numpy(eye), hip.from_numpy(w))), w)
+
+
+@pytest.mark.parametrize("M", [16, 40, 130])
+@pytest.mark.parametrize("side", ["left", "right"])
+def test_ends_of_the_range(hip, M, side):
+    """Infinities, values that round up beyond bfloat16's largest, rows of tiny values, NaN: as in 32-bit arithmetic."""
+    K, N = 64, 130
+    rng = np.random.default_rng(M)
+    a = rng.standard_normal((1, M, K), dtype=np.float32)
+    b = np.zeros((1, K, N), dtype=np.float32)
+    b[0, rng.integers(0, K, N), np.arange(N)] = rng.choice(np.float32([1.0, -0.5, 2.0 ** -10]), N)   # a scaled choice: exact products
+    a[0, 3] = np.float32(3.4028235e38) * np.sign(a[0, 3])
+    a[0, 5] *= np.float32(1e-34)
+    a[0, 7, 1] = np.inf
+    a[0, 9, 2] = np.nan
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = (a[0].astype(np.float64)[:, :, None] * b[0].astype(np.float64)[None]).sum(1).astype(np.float32)
+    if side == "left":
+        got = hip.to_numpy(hip.matmul(hip.from_numpy(a), hip.from_numpy(b)))[0]
+    else:
+        got = hip.to_numpy(hip.matmul(hip.transpose(hip.from_numpy(np.ascontiguousarray(b.transpose(0, 2, 1)).reshape(1, N, K)), 1, 1),
+                                      hip.transpose(hip.from_numpy(a), 1, 2)))[0].T
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(got[~np.isnan(want)], want[~np.isnan(want)])
