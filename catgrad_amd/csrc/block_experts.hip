@@ -10,6 +10,7 @@
 //                                       in the store of the first; 16 / 32 values of k per row and stage by loads straight
 //                                       into a ring of LDS stages, one barrier a stage
 #include "block_stream.hpp"
+#include "split_tile.hpp"
 
 #include <algorithm>
 
@@ -304,13 +305,13 @@ struct ExpertTileArgs {
     float limit, slope;
 };
 
-// 64 MT x 128 tiles of an expert's rows, four waves of 32 MT x 64 each.  A stage is 64 bytes of k per row, by loads straight
+// 64 MT x 128 tiles of an expert's rows in bfloat16, four waves of 32 MT x 64 each.  A stage is 64 bytes of k per row, by loads straight
 // into LDS in a ring of four: one multiplied, three in flight, one barrier a stage.  A row's four 16-byte columns lie at column
 // c ^ ((row >> 2) & 3), so that the lanes that a 128-bit read serves together cover all banks.  FIRST: the tile's 128 weight
 // rows are 64 of each first matrix, 32 in turn, so that a lane finds both factors of its activations; the left operand's rows
-// come through the list.  f32: lane group g supplies k = 4 (2 c + g) + t to the t-th of four instructions.
-template <bool BF16, bool FIRST, int MT> __global__ __launch_bounds__(kThreads) void expert_tile_kernel(const ExpertTileArgs a) {
-    constexpr uint32_t TM = 64 * MT, A_BYTES = TM * 64, STAGE = A_BYTES + kTileN * 64, EB = BF16 ? 2 : 4, STAGE_K = 64 / EB;
+// come through the list.
+template <bool FIRST, int MT> __global__ __launch_bounds__(kThreads) void expert_tile_kernel(const ExpertTileArgs a) {
+    constexpr uint32_t TM = 64 * MT, A_BYTES = TM * 64, STAGE = A_BYTES + kTileN * 64, EB = 2, STAGE_K = 64 / EB;
     constexpr uint32_t OUT_N = FIRST ? 64 : 128; // output columns of a tile
     extern __shared__ float lds_dyn[];
     typedef __attribute__((address_space(3))) char lds_char;
@@ -381,12 +382,7 @@ template <bool BF16, bool FIRST, int MT> __global__ __launch_bounds__(kThreads) 
             for (int i = 0; i < MT; i++)
 #pragma unroll
                 for (int j = 0; j < 2; j++) {
-                    if constexpr (BF16) {
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[i]), __builtin_bit_cast(bf16x8, fb[j]), acc[i][j], 0, 0, 0);
-                    } else {
-#pragma unroll
-                        for (int t = 0; t < 4; t++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][t], fb[j][t], acc[i][j], 0, 0, 0);
-                    }
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[i]), __builtin_bit_cast(bf16x8, fb[j]), acc[i][j], 0, 0, 0);
                 }
         }
     }
@@ -405,15 +401,54 @@ template <bool BF16, bool FIRST, int MT> __global__ __launch_bounds__(kThreads) 
                 const uint32_t f = n0 + (wave % 2) * 32 + li;
                 if (f >= a.N) continue;
                 const float h = a.weights[choice] * activation(acc[i][0][v], acc[i][1][v], a.limit, a.slope);
-                if constexpr (BF16) static_cast<uint16_t *>(a.out)[(uint64_t)place * a.N + f] = (uint16_t)(round_bf16(h) >> 16);
-                else static_cast<float *>(a.out)[(uint64_t)place * a.N + f] = h;
+                static_cast<uint16_t *>(a.out)[(uint64_t)place * a.N + f] = (uint16_t)(round_bf16(h) >> 16);
             } else {
 #pragma unroll
                 for (int j = 0; j < 2; j++) {
                     const uint32_t n = n0 + wn + j * 32 + li;
                     if (n >= a.N) continue;
-                    if constexpr (BF16) static_cast<uint16_t *>(a.out)[(uint64_t)choice * a.N + n] = (uint16_t)(round_bf16(acc[i][j][v]) >> 16);
-                    else static_cast<float *>(a.out)[(uint64_t)choice * a.N + n] = acc[i][j][v];
+                    static_cast<uint16_t *>(a.out)[(uint64_t)choice * a.N + n] = (uint16_t)(round_bf16(acc[i][j][v]) >> 16);
+                }
+            }
+        }
+}
+
+// The same in 32 bits, as products of pieces (split_tile.hpp): WM x 2 waves of MT x 2 blocks.
+template <bool FIRST, int WM, int MT, bool CARE> __global__ __launch_bounds__(128 * WM, 2) void expert_split_kernel(const ExpertTileArgs a) {
+    constexpr uint32_t OUT_N = FIRST ? 64 : 128;
+    extern __shared__ float lds_dyn[];
+    const uint32_t tile = blockIdx.x / a.tiles_n, n0 = (blockIdx.x - tile * a.tiles_n) * OUT_N;
+    const uint4 job = a.tiles[tile];
+    const uint32_t m = job.z, K = a.K, N = a.N, top = a.top;
+    if (m == 0) return;
+    const uint32_t *const list = a.list + job.y;
+    const split::TileSide x = {reinterpret_cast<const uint32_t *>(a.x) + (FIRST ? 0 : (uint64_t)job.y * K), 1};
+    const split::TileSide w = {reinterpret_cast<const uint32_t *>(a.w) + (uint64_t)job.x * (FIRST ? 2 : 1) * N * K, 1};
+    float16v acc[MT][2];
+    split::product<WM, 2, MT, 2, false, false, CARE>(
+        acc, (split::lds_char *)lds_dyn, x, [=](uint32_t r) { return (int64_t)(FIRST ? list[r] / top : r) * K; }, m - 1, w,
+        [=](uint32_t r) {
+            const uint32_t n = FIRST ? min(n0 + (r >> 6) * 32 + (r & 31), N - 1) + ((r >> 5) & 1) * N : min(n0 + r, N - 1);
+            return (int64_t)n * K;
+        },
+        127, K);
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), li = threadIdx.x % 32, lg = threadIdx.x % 64 / 32;
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const uint32_t r = (wave / 2 * MT + i) * 32 + 8 * (v / 4) + 4 * lg + (v % 4);
+            if (v % 4 == 0) __builtin_amdgcn_sched_barrier(0); // (few rows' places in registers at a time)
+            if (r >= m) continue;
+            const uint32_t choice = list[r];
+            if constexpr (FIRST) {
+                const uint32_t f = n0 + (wave % 2) * 32 + li;
+                if (f < N) static_cast<float *>(a.out)[(uint64_t)(job.y + r) * N + f] = a.weights[choice] * activation(acc[i][0][v], acc[i][1][v], a.limit, a.slope);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const uint32_t n = n0 + (wave % 2) * 64 + j * 32 + li;
+                    if (n < N) static_cast<float *>(a.out)[(uint64_t)choice * N + n] = acc[i][j][v];
                 }
             }
         }
@@ -445,9 +480,16 @@ bool vector_rows(const ExpertsPlan &p) {
 }
 double first_bytes(const ExpertsPlan &p, double used) { return used * 2.0 * p.ff * p.width * (p.fmt == kFmtBF16 ? 2.0 : 4.0); }
 
-template <bool BF16, bool FIRST, int MT> int launch_tiles(cg_backend *be, const ExpertTileArgs &a, uint32_t tiles) {
-    const size_t lds = (size_t)kStages * (64 * MT + kTileN) * 64;
-    hipLaunchKernelGGL((expert_tile_kernel<BF16, FIRST, MT>), dim3(tiles * a.tiles_n), dim3(kThreads), lds, be->stream, a);
+template <bool FIRST> int launch_tiles(cg_backend *be, const ExpertTileArgs &a, uint32_t tiles, bool bf16, bool low, bool far) {
+    const dim3 grid(tiles * a.tiles_n);
+    const uint32_t tm = low ? 64 : 128;
+    const size_t lds = bf16 ? (size_t)kStages * (tm + kTileN) * 64 : split::lds_bytes(tm, kTileN);
+    if (bf16 && low) hipLaunchKernelGGL((expert_tile_kernel<FIRST, 1>), grid, dim3(kThreads), lds, be->stream, a);
+    else if (bf16) hipLaunchKernelGGL((expert_tile_kernel<FIRST, 2>), grid, dim3(kThreads), lds, be->stream, a);
+    else if (low && far) hipLaunchKernelGGL((expert_split_kernel<FIRST, 2, 1, true>), grid, dim3(kThreads), lds, be->stream, a);
+    else if (low) hipLaunchKernelGGL((expert_split_kernel<FIRST, 2, 1, false>), grid, dim3(kThreads), lds, be->stream, a);
+    else if (far) hipLaunchKernelGGL((expert_split_kernel<FIRST, 2, 2, true>), grid, dim3(kThreads), lds, be->stream, a);
+    else hipLaunchKernelGGL((expert_split_kernel<FIRST, 2, 2, false>), grid, dim3(kThreads), lds, be->stream, a);
     return launched("expert_tiles");
 }
 
@@ -542,6 +584,8 @@ int launch_experts(cg_backend *be, const ExpertsPlan &p, float *y, int *y_fmt) {
         return launched("expert_slots");
     }
     *y_fmt = bf16 ? kFmtBF16 : kFmtWords;
+    // rows or matrices further apart than 32-bit byte offsets reach
+    const bool far = (uint64_t)p.rows * p.width >= (1ull << 30) || 2ull * p.ff * p.width >= (1ull << 30);
     // lists
     const bool low = n <= 64ull * p.experts; // few rows per expert: short tiles
     const uint32_t tm = low ? 64 : 128, max_tiles = (uint32_t)(n / tm + std::min<uint64_t>(p.experts, n));
@@ -578,8 +622,7 @@ int launch_experts(cg_backend *be, const ExpertsPlan &p, float *y, int *y_fmt) {
     int rc;
     {
         ProfScope prof(be, CG_K_GEMM_MFMA, 4.0 * (double)n * p.ff * p.width);
-        rc = bf16 ? (low ? launch_tiles<true, true, 1>(be, a, max_tiles) : launch_tiles<true, true, 2>(be, a, max_tiles))
-                  : (low ? launch_tiles<false, true, 1>(be, a, max_tiles) : launch_tiles<false, true, 2>(be, a, max_tiles));
+        rc = launch_tiles<true>(be, a, max_tiles, bf16, low, far);
     }
     if (rc) return rc;
     a.x = static_cast<const char *>(hid.p);
@@ -589,8 +632,7 @@ int launch_experts(cg_backend *be, const ExpertsPlan &p, float *y, int *y_fmt) {
     a.K = p.ff;
     a.tiles_n = (p.width + kTileN - 1) / kTileN;
     ProfScope prof(be, CG_K_GEMM_MFMA, 2.0 * (double)n * p.ff * p.width);
-    return bf16 ? (low ? launch_tiles<true, false, 1>(be, a, max_tiles) : launch_tiles<true, false, 2>(be, a, max_tiles))
-                : (low ? launch_tiles<false, false, 1>(be, a, max_tiles) : launch_tiles<false, false, 2>(be, a, max_tiles));
+    return launch_tiles<false>(be, a, max_tiles, bf16, low, far);
 }
 
 } // namespace cg
