@@ -1,7 +1,8 @@
-// Products of bfloat16 patterns with the sums in 32-bit, for prompts that do not fill the device with 256 x 256 tiles:
-// y[M, N] = x[M, K] . w[N, K]^T, cut along k as well when there are few tiles.
+// Products of operands that lie narrow in memory (bfloat16, binary16 or fp8 patterns, k contiguous) with the sums in 32 bits, for
+// shapes that do not fill the device with 256 x 256 tiles: y[M, N] = x[M, K] . w[N, K]^T, cut along k as well when there are few
+// tiles.  The result is 32-bit words, or rounded to the operands' format in the last store.
 #include "blocks.hpp"
-#include "device_utils.hpp"
+#include "gemm_args.hpp"
 
 #include <algorithm>
 
@@ -9,26 +10,41 @@ namespace cg {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr uint32_t kTileN = 128, kStages = 4, kStageK = 32, kXcds = 8, kGroupM = 8;
+constexpr uint32_t kTileN = 128, kStages = 4, kStageBytes = 64, kXcds = 8, kGroupM = 8;
 typedef float float16v __attribute__((ext_vector_type(16)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef int int4v __attribute__((ext_vector_type(4)));
 
 struct TileArgs {
     const char *x, *w;
-    float *y;                  // split s of y at y + s * M * N
-    uint32_t M, N, K;
-    uint32_t x_pitch, w_pitch; // bytes
-    uint32_t k_part;           // values of k per split, a multiple of kStageK
+    void *y;                   // split s of y at y + s * M * N
+    uint32_t M, N;
+    uint32_t K;                // bytes, as the pitches
+    uint32_t x_pitch, w_pitch;
+    uint32_t k_part;           // bytes of k per split, a multiple of kStageBytes
 };
+
+template <int FMT> __device__ __forceinline__ uint32_t pattern(float v) {
+    if constexpr (FMT == kFmtBF16) return round_bf16_bits(asu(v)) >> 16;
+    else if constexpr (FMT == kFmtF16) return __half_as_ushort(__float2half_rn(v));
+    else return f8_byte_of(round_f8_bits(asu(v)));
+}
+template <int FMT> __device__ __forceinline__ void put(void *y, uint64_t at, float v) {
+    if constexpr (FMT == kFmtWords) static_cast<float *>(y)[at] = v;
+    else if constexpr (FMT == kFmtF8) static_cast<uint8_t *>(y)[at] = (uint8_t)pattern<FMT>(v);
+    else static_cast<uint16_t *>(y)[at] = (uint16_t)pattern<FMT>(v);
+}
 
 __device__ const uint32_t kZeros[4] __attribute__((aligned(16))) = {0, 0, 0, 0};
 
 // 64 MT x 128 tiles, four waves of 32 MT x 64 each.  A stage is 64 bytes of k per row, fetched by loads straight into LDS in
 // a ring of four: one multiplied, three in flight, one barrier a stage.  A row's four 16-byte columns lie at column
 // c ^ ((row >> 2) & 3), so that the lanes that a 128-bit read serves together cover all banks; a load instruction of a wave
-// fills 16 rows in lane order.  Rows beyond the edge are clamped, columns beyond K come from a block of zeros.
-template <int MT> __global__ __launch_bounds__(kThreads) void bf16_tile_kernel(const TileArgs a) {
+// fills 16 rows in lane order.  Rows beyond the edge are clamped, columns beyond K come from a block of zeros.  FMT: the operands'
+// format; OUT: the result's.
+template <int FMT, int OUT, int MT> __global__ __launch_bounds__(kThreads) void narrow_tile_kernel(const TileArgs a) {
     constexpr uint32_t TM = 64 * MT, A_BYTES = TM * 64, STAGE = A_BYTES + kTileN * 64;
     extern __shared__ float lds_dyn[];
     typedef __attribute__((address_space(3))) char lds_char;
@@ -41,7 +57,7 @@ template <int MT> __global__ __launch_bounds__(kThreads) void bf16_tile_kernel(c
     const uint32_t group = lin / (kGroupM * tiles_n), in_group = lin % (kGroupM * tiles_n), first_m = group * kGroupM;
     const uint32_t gsize = min(tiles_m - first_m, kGroupM);
     const uint32_t m0 = (first_m + in_group % gsize) * TM, n0 = (in_group / gsize) * kTileN;
-    const uint32_t k_first = blockIdx.y * a.k_part, k_end = min(k_first + a.k_part, a.K), nk = (k_end - k_first + kStageK - 1) / kStageK;
+    const uint32_t k_first = blockIdx.y * a.k_part, k_end = min(k_first + a.k_part, a.K), nk = (k_end - k_first + kStageBytes - 1) / kStageBytes;
 
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
     const uint32_t wm = (wave / 2) * 32 * MT, wn = (wave % 2) * 64, li = lane % 32, lg = lane / 32;
@@ -54,11 +70,11 @@ template <int MT> __global__ __launch_bounds__(kThreads) void bf16_tile_kernel(c
 #pragma unroll
     for (int q = 0; q < 2; q++) off[MT + q] = min(n0 + (wave * 2 + q) * 16 + lane / 4, a.N - 1) * a.w_pitch + col * 16;
     auto issue = [&](const uint32_t stage, const uint32_t place) {
-        const uint32_t k0 = k_first + stage * kStageK;
-        const bool tail = k0 + kStageK > a.K, outside = k0 + col * 8 >= a.K;
+        const uint32_t k0 = k_first + stage * kStageBytes;
+        const bool tail = k0 + kStageBytes > a.K, outside = k0 + col * 16 >= a.K;
 #pragma unroll
         for (int q = 0; q < MT + 2; q++) {
-            const char *p = (q < MT ? a.x : a.w) + (uint64_t)k0 * 2 + off[q];
+            const char *p = (q < MT ? a.x : a.w) + k0 + off[q];
             if (tail && outside) p = reinterpret_cast<const char *>(kZeros);
             lds_char *const l = lds + place * STAGE + (q < MT ? (wave * MT + q) * 1024 : A_BYTES + (wave * 2 + q - MT) * 1024);
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)p, (__attribute__((address_space(3))) void *)l, 16, 0, 0);
@@ -66,7 +82,7 @@ template <int MT> __global__ __launch_bounds__(kThreads) void bf16_tile_kernel(c
     };
     const uint32_t sw = (li >> 2) & 3;
     auto frag = [&](const uint32_t base, const uint32_t c) {
-        return __builtin_bit_cast(bf16x8, *reinterpret_cast<const __attribute__((address_space(3))) float4v *>(lds + base + li * 64 + ((c ^ sw) * 16)));
+        return *reinterpret_cast<const __attribute__((address_space(3))) int4v *>(lds + base + li * 64 + ((c ^ sw) * 16));
     };
 
     float16v acc[MT][2];
@@ -89,21 +105,42 @@ template <int MT> __global__ __launch_bounds__(kThreads) void bf16_tile_kernel(c
         const uint32_t base = (kt % kStages) * STAGE;
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-            bf16x8 fa[MT], fb[2];
+            constexpr int STEPS = FMT == kFmtF8 ? 2 : 1; // matrix instructions per 16-byte column
+            int4v fa[MT][STEPS], fb[2][STEPS];
+            auto read = [&](const uint32_t at, int4v(&f)[STEPS]) {
+                const int4v v = frag(at, c * 2 + lg);
+                if constexpr (FMT != kFmtF8) f[0] = v;
+                else {
+                    // fp8 values are bfloat16 values: the fp8 instructions keep 3.5e-6 of a sum (64 and 2048 values of k alike),
+                    // the bfloat16 ones all of its 32 bits
 #pragma unroll
-            for (int i = 0; i < MT; i++) fa[i] = frag(base + (wm + i * 32) * 64, c * 2 + lg);
+                    for (int w = 0; w < 4; w++) {
+                        f[w / 2][w % 2 * 2] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((uint32_t)v[w], 1.0f, false));
+                        f[w / 2][w % 2 * 2 + 1] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((uint32_t)v[w], 1.0f, true));
+                    }
+                }
+            };
 #pragma unroll
-            for (int j = 0; j < 2; j++) fb[j] = frag(base + A_BYTES + (wn + j * 32) * 64, c * 2 + lg);
+            for (int i = 0; i < MT; i++) read(base + (wm + i * 32) * 64, fa[i]);
 #pragma unroll
-            for (int i = 0; i < MT; i++)
+            for (int j = 0; j < 2; j++) read(base + A_BYTES + (wn + j * 32) * 64, fb[j]);
 #pragma unroll
-                for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+            for (int t = 0; t < STEPS; t++)
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) {
+                        if constexpr (FMT == kFmtF16)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, fa[i][t]), __builtin_bit_cast(f16x8, fb[j][t]), acc[i][j], 0, 0, 0);
+                        else
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[i][t]), __builtin_bit_cast(bf16x8, fb[j][t]), acc[i][j], 0, 0, 0);
+                    }
         }
     }
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0x0070); // no load may write LDS that another workgroup gets
 
-    float *const y = a.y + (uint64_t)blockIdx.y * a.M * a.N;
+    const uint64_t first = (uint64_t)blockIdx.y * a.M * a.N;
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
@@ -113,18 +150,21 @@ template <int MT> __global__ __launch_bounds__(kThreads) void bf16_tile_kernel(c
 #pragma unroll
             for (int v = 0; v < 16; v++) { // the instruction's result: row 8 (v / 4) + 4 lg + v % 4, column li
                 const uint32_t m = m0 + wm + i * 32 + 8 * (v / 4) + 4 * lg + (v % 4);
-                if (m < a.M) y[(uint64_t)m * a.N + n] = acc[i][j][v];
+                if (m < a.M) put<OUT>(a.y, first + (uint64_t)m * a.N + n, acc[i][j][v]);
             }
         }
 }
 
 // y[e] = the parts' sum, in their order
-__global__ __launch_bounds__(kThreads) void sum_parts_kernel(const float4v *part, float4v *y, uint32_t parts, uint64_t n4) {
+template <int OUT> __global__ __launch_bounds__(kThreads) void sum_parts_kernel(const float4v *part, void *y, uint32_t parts, uint64_t n4) {
     const uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
     if (i >= n4) return;
     float4v v = __builtin_nontemporal_load(part + i);
     for (uint32_t s = 1; s < parts; s++) v += __builtin_nontemporal_load(part + s * n4 + i);
-    y[i] = v;
+    if constexpr (OUT == kFmtWords) static_cast<float4v *>(y)[i] = v;
+    else if constexpr (OUT == kFmtF8)
+        static_cast<uint32_t *>(y)[i] = pattern<OUT>(v[0]) | pattern<OUT>(v[1]) << 8 | pattern<OUT>(v[2]) << 16 | pattern<OUT>(v[3]) << 24;
+    else static_cast<uint2 *>(y)[i] = make_uint2(pattern<OUT>(v[0]) | pattern<OUT>(v[1]) << 16, pattern<OUT>(v[2]) | pattern<OUT>(v[3]) << 16);
 }
 
 int launched(const char *what) {
@@ -132,48 +172,71 @@ int launched(const char *what) {
     return e == hipSuccess ? CG_OK : hip_fail(e, what);
 }
 
+template <int FMT, int OUT> int run_tiles(cg_backend *be, TileArgs a) {
+    const bool low = a.M <= 64;
+    const uint32_t tm = low ? 64 : 128;
+    const uint64_t tiles = (uint64_t)((a.M + tm - 1) / tm) * ((a.N + kTileN - 1) / kTileN);
+    if (tiles > 0x7FFFFFFFull) return kDeclined;
+    // two workgroups per compute unit, each with at least 512 bytes of k; the same shape always gets the same cut
+    const uint64_t mn = (uint64_t)a.M * a.N, room = 2 * (uint64_t)be->compute_units;
+    uint32_t splits = mn % 4 ? 1 : (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({room / tiles, a.K / 512, 16}));
+    a.k_part = ((a.K + splits - 1) / splits + kStageBytes - 1) / kStageBytes * kStageBytes;
+    splits = (a.K + a.k_part - 1) / a.k_part;
+    void *parts = nullptr, *const y = a.y;
+    size_t cls = 0;
+    if (splits > 1) {
+        if (int rc = be->pool.alloc(mn * splits * 4, &parts, &cls)) return rc;
+        a.y = parts;
+    }
+    const dim3 grid((uint32_t)tiles, splits);
+    const size_t lds = (size_t)kStages * (tm + kTileN) * kStageBytes;
+    if (splits > 1) {
+        if (low) hipLaunchKernelGGL((narrow_tile_kernel<FMT, kFmtWords, 1>), grid, dim3(kThreads), lds, be->stream, a);
+        else hipLaunchKernelGGL((narrow_tile_kernel<FMT, kFmtWords, 2>), grid, dim3(kThreads), lds, be->stream, a);
+        hipLaunchKernelGGL((sum_parts_kernel<OUT>), dim3((uint32_t)((mn / 4 + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream,
+                           static_cast<const float4v *>(parts), y, splits, mn / 4);
+        be->pool.free(parts, cls); // stream-ordered
+    } else {
+        if (low) hipLaunchKernelGGL((narrow_tile_kernel<FMT, OUT, 1>), grid, dim3(kThreads), lds, be->stream, a);
+        else hipLaunchKernelGGL((narrow_tile_kernel<FMT, OUT, 2>), grid, dim3(kThreads), lds, be->stream, a);
+    }
+    return launched("narrow_tiles");
+}
+
 } // namespace
 
-int launch_bf16_tiles(cg_backend *be, const void *x, uint32_t rows, const Weight &w, float *y) {
-    const uint64_t x_bytes = (uint64_t)rows * w.k * 2, w_bytes = (uint64_t)w.n * (uint64_t)w.pitch * 2;
-    if (!takes_bf16_tiles(rows, w) || reinterpret_cast<uintptr_t>(x) % 16) return kDeclined;
-    const bool low = rows <= 64;
-    const uint32_t tm = low ? 64 : 128;
-    const uint64_t tiles = (uint64_t)((rows + tm - 1) / tm) * ((w.n + kTileN - 1) / kTileN);
-    if (x_bytes >= (1ull << 32) || w_bytes >= (1ull << 32) || tiles > 0x7FFFFFFFull) return kDeclined;
+int launch_narrow_tiles(cg_backend *be, int fmt, const void *x, int64_t x_pitch, int64_t rows, const void *w, int64_t w_pitch, int64_t n, int64_t k, void *y, int y_fmt) {
+    const int64_t eb = (int64_t)fmt_bytes(fmt);
+    if (!fits_narrow_tiles(fmt, x, x_pitch, rows, w, w_pitch, n, k)) return kDeclined;
     TileArgs a{};
     a.x = static_cast<const char *>(x);
-    a.w = static_cast<const char *>(w.p);
-    a.M = rows;
-    a.N = w.n;
-    a.K = w.k;
-    a.x_pitch = w.k * 2;
-    a.w_pitch = (uint32_t)(w.pitch * 2);
-    // two workgroups per compute unit, each with at least 256 values of k; the same shape always gets the same cut
-    const uint64_t mn = (uint64_t)rows * w.n, room = 2 * (uint64_t)be->compute_units;
-    uint32_t splits = mn % 4 ? 1 : (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({room / tiles, w.k / 256, 16}));
-    a.k_part = ((w.k + splits - 1) / splits + kStageK - 1) / kStageK * kStageK;
-    splits = (w.k + a.k_part - 1) / a.k_part;
-    ProfScope prof(be, CG_K_GEMM_MFMA, 2.0 * (double)mn * w.k);
-    void *parts = nullptr;
-    size_t cls = 0;
-    if (splits > 1)
-        if (int rc = be->pool.alloc(mn * splits * 4, &parts, &cls)) return rc;
-    a.y = splits > 1 ? static_cast<float *>(parts) : y;
-    const dim3 grid((uint32_t)tiles, splits);
-    const size_t lds = (size_t)kStages * (tm + kTileN) * 64;
-    if (low) hipLaunchKernelGGL((bf16_tile_kernel<1>), grid, dim3(kThreads), lds, be->stream, a);
-    else hipLaunchKernelGGL((bf16_tile_kernel<2>), grid, dim3(kThreads), lds, be->stream, a);
-    if (splits > 1) {
-        hipLaunchKernelGGL(sum_parts_kernel, dim3((uint32_t)((mn / 4 + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream,
-                           static_cast<const float4v *>(parts), reinterpret_cast<float4v *>(y), splits, mn / 4);
-        be->pool.free(parts, cls); // stream-ordered
-    }
-    return launched("bf16_tiles");
+    a.w = static_cast<const char *>(w);
+    a.y = y;
+    a.M = (uint32_t)rows;
+    a.N = (uint32_t)n;
+    a.K = (uint32_t)(k * eb);
+    a.x_pitch = (uint32_t)(x_pitch * eb);
+    a.w_pitch = (uint32_t)(w_pitch * eb);
+    const bool words = y_fmt == kFmtWords;
+    if (fmt == kFmtBF16) return words ? run_tiles<kFmtBF16, kFmtWords>(be, a) : run_tiles<kFmtBF16, kFmtBF16>(be, a);
+    if (fmt == kFmtF16) return words ? run_tiles<kFmtF16, kFmtWords>(be, a) : run_tiles<kFmtF16, kFmtF16>(be, a);
+    return words ? run_tiles<kFmtF8, kFmtWords>(be, a) : run_tiles<kFmtF8, kFmtF8>(be, a);
 }
 
-bool takes_bf16_tiles(uint32_t rows, const Weight &w) {
-    return rows > 0 && w.fmt == kFmtBF16 && w.k % 8 == 0 && w.pitch % 8 == 0 && reinterpret_cast<uintptr_t>(w.p) % 16 == 0;
+bool fits_narrow_tiles(int fmt, const void *x, int64_t x_pitch, int64_t rows, const void *w, int64_t w_pitch, int64_t n, int64_t k) {
+    const int64_t eb = (int64_t)fmt_bytes(fmt);
+    auto side = [&](const void *p, int64_t pitch, int64_t r) {
+        return r > 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0 && pitch >= 0 && pitch * eb % 16 == 0 && r * pitch * eb < (1ll << 32) && r < (1ll << 31);
+    };
+    return fmt != kFmtWords && k > 0 && k * eb % 16 == 0 && k * eb < (1ll << 31) && side(x, x_pitch, rows) && side(w, w_pitch, n);
 }
+
+int launch_bf16_tiles(cg_backend *be, const void *x, uint32_t rows, const Weight &w, float *y) {
+    if (!takes_bf16_tiles(rows, w)) return kDeclined;
+    ProfScope prof(be, CG_K_GEMM_MFMA, 2.0 * (double)rows * w.n * w.k);
+    return launch_narrow_tiles(be, kFmtBF16, x, w.k, rows, w.p, w.pitch, w.n, w.k, y, kFmtWords);
+}
+
+bool takes_bf16_tiles(uint32_t rows, const Weight &w) { return w.fmt == kFmtBF16 && fits_narrow_tiles(kFmtBF16, nullptr, w.k, rows, w.p, w.pitch, w.n, w.k); }
 
 } // namespace cg

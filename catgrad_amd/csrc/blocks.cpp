@@ -156,7 +156,7 @@ int product_operand(cg_backend *be, int64_t rows, const Weight &weight, cg_tenso
     if (w->dt == CG_BF16 && K % 8 == 0 && (rows >= 256 || takes_bf16_tiles((uint32_t)rows, weight))) {
         if (int rc = new_dense(be, CG_BF16, xd, 2, &x, 0, kFmtBF16)) return rc;
         ProductViews v(be, w, rows, nullptr);
-        *tiles = rows < 256 || launch_matmul(be, x, &v.wt, nullptr) != CG_OK;
+        *tiles = rows < 256 || launch_matmul(be, x, &v.wt, nullptr, true) != CG_OK;
         if (*tiles && !takes_bf16_tiles((uint32_t)rows, weight)) {
             *tiles = false;
             release(x);

@@ -580,7 +580,7 @@ int launch_any_diff(cg_backend *be, const cg_tensor *x, const cg_tensor *y);
 
 // out == nullptr: nothing is launched; CG_OK if this product would run on the kernel that can round a narrow dtype's
 // result in its store (then `out` may hold that dtype's format), kDeclined if not.
-int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_tensor *out);
+int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_tensor *out, bool wide_only = false);
 
 // The batch structure of x . y after collapsing: batch axes that both operands walk as one run
 // are merged, a split axis contributes its two parts, and the innermost batch axis is folded

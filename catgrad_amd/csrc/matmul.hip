@@ -683,11 +683,6 @@ template <int HALF, bool NARROW_OUT> __global__ __launch_bounds__(kThreads) void
     // would give, bit for bit) and stored as its patterns, a quarter or an eighth of the bytes of that f32 result and pass:
     // lanes exchange values so that each stores 32 bits — two columns of one row (16-bit: lanes pair up, the even lane takes
     // the first of two rows, the odd lane the second) or four (fp8: a quad transposes its 4 x 4 values).
-    auto pattern = [&](const float x) -> uint32_t {
-        if constexpr (HALF == 3) return round_bf16_bits(asu(x)) >> 16;
-        else if constexpr (HALF == 4) return (uint32_t)__half_as_ushort(__float2half_rn(x));
-        else return (uint32_t)f8_byte_of(round_f8_bits(asu(x)));
-    };
     const uint32_t lane_off = ((wm + 4 * lg) * a.N + wn + li) * 4;
     const uint32_t sub = HALF == 5 ? (li & 3) : (li & 1); // this lane's row among the 4 (2) that its group exchanges
     const uint32_t lane_off_narrow = ((wm + 4 * lg + sub) * a.N + wn + li - sub) * (HALF == 5 ? 1 : 2);
@@ -713,56 +708,67 @@ template <int HALF, bool NARROW_OUT> __global__ __launch_bounds__(kThreads) void
                 }
             return;
         }
-        if (whole) {
-            constexpr uint32_t EB = HALF == 5 ? 1 : 2;
-            char *const base = reinterpret_cast<char *>(a.C) + ((uint64_t)m0 * a.N + n0) * EB;
+        if constexpr (NARROW_OUT) {
+            // (N is a multiple of 4: a lane's columns are all inside or all outside; the stores of an edge tile are masked, not made a
+            // value at a time, which took longer than the tile: 1500 x 2048 x 8192 on bf16 73 -> 67 us)
+            auto rounded = [&](auto whole_) {
+                auto inside = [&](const uint32_t r, const int j) {
+                    return decltype(whole_)::value || (m0 + wm + 4 * lg + sub + r < a.M && n0 + wn + j * 32 + li - sub < a.N);
+                };
+                constexpr uint32_t EB = HALF == 5 ? 1 : 2;
+                char *const base = reinterpret_cast<char *>(a.C) + ((uint64_t)m0 * a.N + n0) * EB;
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+                for (int i = 0; i < 4; i++)
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    if constexpr (HALF != 5) {
+                    for (int j = 0; j < 4; j++) {
+                        if constexpr (HALF != 5) {
 #pragma unroll
-                        for (int v = 0; v < 16; v += 2) {
-                            // v_cvt_pk_{bf16,f16}_f32 round two values as the rounding pass does (all 2^32 patterns compared)
-                            const float2v pair = {acc[i][j][v], acc[i][j][v + 1]};
-                            uint32_t mine;
-                            if constexpr (HALF == 3) mine = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, bf16x2));
-                            else mine = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, f16x2));
-                            const uint32_t theirs = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, 0xB1, 0xF, 0xF, true); // the pair's other lane
-                            // even lane: its and the other's first row; odd lane: the other's and its second row
-                            const uint32_t two = __builtin_amdgcn_perm(theirs, mine, sub ? 0x03020706u : 0x05040100u);
-                            const uint32_t r = i * 32 + 8 * (v / 4) + (v % 4);
-                            asm volatile("global_store_dword %0, %1, %2" ::"v"(lane_off_narrow), "v"(two), "s"(base + ((uint64_t)r * a.N + j * 32) * 2) : "memory");
-                        }
-                    } else {
-#pragma unroll
-                        for (int v = 0; v < 16; v += 4) {
-                            // v_cvt_pk_fp8_f32 rounds as the rounding pass does once the magnitude is clamped to 448 (it holds no
-                            // infinities) and NaNs are set apart: they become the clamped pattern 0x7e, which the 0x7f below completes
-                            // (all 2^32 patterns compared)
-                            float xs[4];
-                            uint32_t nans = 0;
-#pragma unroll
-                            for (int k = 0; k < 4; k++) {
-                                const uint32_t u = asu(acc[i][j][v + k]), mag = u & 0x7FFFFFFFu;
-                                xs[k] = asf(min(mag, 0x43E00000u) | (u & 0x80000000u));
-                                nans |= mag > 0x7F800000u ? 0x7Fu << (8 * k) : 0u;
+                            for (int v = 0; v < 16; v += 2) {
+                                // v_cvt_pk_{bf16,f16}_f32 round two values as the rounding pass does (all 2^32 patterns compared)
+                                const float2v pair = {acc[i][j][v], acc[i][j][v + 1]};
+                                uint32_t mine;
+                                if constexpr (HALF == 3) mine = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, bf16x2));
+                                else mine = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, f16x2));
+                                const uint32_t theirs = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, 0xB1, 0xF, 0xF, true); // the pair's other lane
+                                // even lane: its and the other's first row; odd lane: the other's and its second row
+                                const uint32_t two = __builtin_amdgcn_perm(theirs, mine, sub ? 0x03020706u : 0x05040100u);
+                                const uint32_t r = i * 32 + 8 * (v / 4) + (v % 4);
+                                if (inside(r, j))
+                                    asm volatile("global_store_dword %0, %1, %2" ::"v"(lane_off_narrow), "v"(two), "s"(base + ((uint64_t)r * a.N + j * 32) * 2) : "memory");
                             }
-                            int packed = __builtin_amdgcn_cvt_pk_fp8_f32(xs[0], xs[1], 0, false);
-                            packed = __builtin_amdgcn_cvt_pk_fp8_f32(xs[2], xs[3], packed, true);
-                            const uint32_t mine = (uint32_t)packed | nans; // byte k: row k of this lane's column
-                            // lane q of the quad keeps row q: byte q of every lane's word, at the place of that lane's column
-                            const uint32_t r1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, 0x39, 0xF, 0xF, true); // of lane q + 1
-                            const uint32_t r2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, 0x4E, 0xF, 0xF, true); // of lane q + 2
-                            const uint32_t r3 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, 0x93, 0xF, 0xF, true); // of lane q + 3
-                            const uint32_t four = __builtin_amdgcn_perm(r1, mine, quad_sel_a) | __builtin_amdgcn_perm(r3, r2, quad_sel_b);
-                            const uint32_t r = i * 32 + 8 * (v / 4);
-                            asm volatile("global_store_dword %0, %1, %2" ::"v"(lane_off_narrow), "v"(four), "s"(base + ((uint64_t)r * a.N + j * 32)) : "memory");
-                            __builtin_amdgcn_sched_barrier(0);
+                        } else {
+#pragma unroll
+                            for (int v = 0; v < 16; v += 4) {
+                                // v_cvt_pk_fp8_f32 rounds as the rounding pass does once the magnitude is clamped to 448 (it holds no
+                                // infinities) and NaNs are set apart: they become the clamped pattern 0x7e, which the 0x7f below completes
+                                // (all 2^32 patterns compared)
+                                float xs[4];
+                                uint32_t nans = 0;
+#pragma unroll
+                                for (int k = 0; k < 4; k++) {
+                                    const uint32_t u = asu(acc[i][j][v + k]), mag = u & 0x7FFFFFFFu;
+                                    xs[k] = asf(min(mag, 0x43E00000u) | (u & 0x80000000u));
+                                    nans |= mag > 0x7F800000u ? 0x7Fu << (8 * k) : 0u;
+                                }
+                                int packed = __builtin_amdgcn_cvt_pk_fp8_f32(xs[0], xs[1], 0, false);
+                                packed = __builtin_amdgcn_cvt_pk_fp8_f32(xs[2], xs[3], packed, true);
+                                const uint32_t mine = (uint32_t)packed | nans; // byte k: row k of this lane's column
+                                // lane q of the quad keeps row q: byte q of every lane's word, at the place of that lane's column
+                                const uint32_t r1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, 0x39, 0xF, 0xF, true); // of lane q + 1
+                                const uint32_t r2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, 0x4E, 0xF, 0xF, true); // of lane q + 2
+                                const uint32_t r3 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, 0x93, 0xF, 0xF, true); // of lane q + 3
+                                const uint32_t four = __builtin_amdgcn_perm(r1, mine, quad_sel_a) | __builtin_amdgcn_perm(r3, r2, quad_sel_b);
+                                const uint32_t r = i * 32 + 8 * (v / 4);
+                                if (inside(r, j))
+                                    asm volatile("global_store_dword %0, %1, %2" ::"v"(lane_off_narrow), "v"(four), "s"(base + ((uint64_t)r * a.N + j * 32)) : "memory");
+                                __builtin_amdgcn_sched_barrier(0);
+                            }
                         }
+                        __builtin_amdgcn_sched_barrier(0);
                     }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
+            };
+            if (whole) rounded(std::true_type{});
+            else rounded(std::false_type{});
             return;
         }
 #pragma unroll
@@ -776,9 +782,7 @@ template <int HALF, bool NARROW_OUT> __global__ __launch_bounds__(kThreads) void
                         const uint32_t row = m0 + wm + i * 32 + 8 * (v / 4) + 4 * lg + (v % 4);
                         if (row < a.M) {
                             const uint64_t at = (uint64_t)row * a.N + col;
-                            if constexpr (!NARROW_OUT) a.C[at] = asu(acc[i][j][v]);
-                            else if constexpr (HALF == 5) reinterpret_cast<uint8_t *>(a.C)[at] = (uint8_t)pattern(acc[i][j][v]);
-                            else reinterpret_cast<uint16_t *>(a.C)[at] = (uint16_t)pattern(acc[i][j][v]);
+                            a.C[at] = asu(acc[i][j][v]);
                         }
                     }
                 }
@@ -2427,7 +2431,7 @@ __global__ __launch_bounds__(kThreads) void skinny_kt_packed_kernel(const MmArgs
     }
 }
 
-int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_tensor *out) {
+int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_tensor *out, bool wide_only) {
     if (int frc = flush_deferred(be)) return frc;
     MmArgs a;
     MmFold f;
@@ -2444,26 +2448,30 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
     hipStream_t s = be->stream;
 
     // ---- the narrow dtypes' tiled kernels' plan (used by the last branch below; here because it decides how operands are addressed) ----
-    // the 256 x 256 tile when it covers the chip at least once (env CG_GEMM_BIG=0 switches it off)
+    // the 256 x 256 tile when it covers half of the chip (1024 x 2048 x 8192, 128 tiles: 53 us against 57 on 128 x 128 tiles, bf16;
+    // 2048 x 2048 x 2048, 64 tiles: 46 against 39), all of it for fp8, whose instructions keep less of a sum (env CG_GEMM_BIG=0 switches it off)
     const uint64_t tiles_big = (uint64_t)((M + 255) / 256) * ((N + 255) / 256) * batch;
     static const bool big_allowed = [] {
         const char *e = getenv("CG_GEMM_BIG");
         return !(e && e[0] == '0');
     }();
-    const bool big = big_allowed && kind && tiles_big >= 256 && M >= 256 && N >= 256;
-    // Operands of a narrow dtype in a product big enough for the 256 x 256 tile are multiplied from 2-byte / 1-byte
-    // patterns: as they lie in memory when their buffer holds that format, else narrowed in memory first (the right
-    // operand once per buffer) (env CG_GEMM_PACKED=0 switches it off).
-    const bool big_packed = f32 && K != 0 && M > 8 && kind && packed_narrow_ok() && big && batch == 1 && K % (kind == 3 ? 16 : 8) == 0 && x->buf && y->buf;
+    const bool big = big_allowed && kind && tiles_big >= (kind == 3 ? 256 : 128) && M >= 256 && N >= 256;
+    // Operands of a narrow dtype are multiplied from 2-byte / 1-byte patterns where rows of k are whole 16-byte pieces: as they
+    // lie in memory when their buffer holds that format, else narrowed in memory first (the right operand once per buffer)
+    // (env CG_GEMM_PACKED=0 switches it off).
+    const bool packable = f32 && K != 0 && M > 8 && kind && packed_narrow_ok() && batch == 1 && K % (kind == 3 ? 16 : 8) == 0 && x->buf && y->buf;
+    const bool x_lies = packable && native_rows(x, kind, a.a_sm, a.a_sk, K, false), y_lies = packable && native_rows(y, kind, a.b_sn, a.b_sk, K, false);
+    // on 256 x 256 tiles if there is one for every compute unit, else on 128 x 128 tiles, unless words are all there is
+    const bool big_packed = packable && big, low_packed = packable && !big && (x_lies || y_lies);
 
     // ---- the operands' addresses -------------------------------------------------------------------------------------
-    const bool x_native = big_packed && native_rows(x, kind, a.a_sm, a.a_sk, K, false);
+    const bool x_native = (big_packed || low_packed) && x_lies;
     rc = mm_operand(x, true, x_native, &a);
     if (rc) return rc;
     // a decode-time linear layer of a narrow dtype reads its weight matrix at 2 or 1 bytes a weight (see below)
     const bool skinny_packed = f32 && K != 0 && M <= (half ? 8 : 2) && packed_narrow_ok() && kind && batch == 1 && a.a_sk == 1 && a.a_vec &&
                                a.a_sm % 4 == 0 && K % 16 == 0 && K >= 256 && N >= 64 && y->buf;
-    const bool y_native = (skinny_packed && native_rows(y, kind, a.b_sn, a.b_sk, K, true)) || (big_packed && native_rows(y, kind, a.b_sn, a.b_sk, K, false));
+    const bool y_native = (skinny_packed && native_rows(y, kind, a.b_sn, a.b_sk, K, true)) || ((big_packed || low_packed) && y_lies);
     rc = mm_operand(y, false, y_native, &a);
     if (rc) return rc;
     // Whole stages of 64 bytes of k in whole turns of the ring, 16-byte rows, byte offsets that fit 32 bits: the wide tile
@@ -2480,7 +2488,9 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
                       (!x_native || reinterpret_cast<uintptr_t>(native_ptr(x)) % 16 == 0) && (!y_native || reinterpret_cast<uintptr_t>(native_ptr(y)) % 16 == 0) &&
                       (uint64_t)M * (uint64_t)a_pitch * 4 < (1ull << 32) && (uint64_t)N * (uint64_t)b_pitch * 4 < (1ull << 32) &&
                       (uint64_t)M * (uint64_t)N < (1ull << 30);
-    const bool can_round = dlds && N % 4 == 0;
+    const int64_t low_a = low_packed ? (x_native ? a.a_sm : K) : 0, low_b = low_packed ? (y_native ? a.b_sn : K) : 0; // row pitches in elements
+    const bool low = low_packed && !wide_only && fits_narrow_tiles(kind, nullptr, low_a, M, nullptr, low_b, N, K);
+    const bool can_round = (dlds && N % 4 == 0) || low;
     if (!out) return can_round ? CG_OK : kDeclined;
     const int c_fmt = out->buf->fmt;
     if (c_fmt != kFmtWords && !can_round) return fail(CG_ERR_ARG, "matmul: a narrow result needs the kernel that rounds in its store");
@@ -2533,6 +2543,16 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
         else { CG_PACKED(8) }
 #undef CG_PACKED
         if (tb) be->pool.free(tb, cb); // stream-ordered: later users queue behind the product
+    } else if (low) {
+        const void *pa = x_native ? native_ptr(x) : nullptr, *pb = y_native ? native_ptr(y) : nullptr;
+        void *ta = nullptr, *tb = nullptr;
+        size_t ca = 0, cb = 0;
+        int prc = x_native ? CG_OK : pack_operand(be, words_buffer(x), a.A, a.a_sm, a.a_sk, M, K, kind, x->rc.load() > 1 || x->buf->rc.load() > 1, &pa, &ta, &ca);
+        if (!prc && !y_native) prc = pack_operand(be, words_buffer(y), a.B, a.b_sn, a.b_sk, N, K, kind, true, &pb, &tb, &cb);
+        if (!prc) prc = launch_narrow_tiles(be, kind, pa, low_a, M, pb, low_b, N, K, out->buf->ptr, c_fmt);
+        if (ta) be->pool.free(ta, ca); // stream-ordered: later users queue behind the product
+        if (tb) be->pool.free(tb, cb);
+        return prc;
     } else if (M <= 8 && a.b_sk == 1) {
         const bool vec = a.a_vec && a.b_vec && a.a_sk == 1 && K % 4 == 0;
 #define CG_MM_SWITCH(CALL)        \

@@ -1,0 +1,61 @@
+"""Products of operands that lie in memory as bfloat16, binary16 or fp8 patterns, on 128-wide tiles (cut along k or not) and at the
+edges of the 256-wide ones: the sum in 32 bits, rounded once to the dtype."""
+import numpy as np
+import pytest
+
+from catgrad_amd import _abi as A
+
+pytestmark = pytest.mark.gpu
+
+UNIT = {"bf16": 2.0 ** -8, "f16": 2.0 ** -11, "fp8": 2.0 ** -4}   # largest relative rounding error
+# edges of tiles (64 / 128 rows, 128 columns), of stages (64 bytes of k), cuts along k, one column, odd results
+SIZES = [(9, 16, 640), (64, 512, 129), (65, 272, 1021), (130, 1040, 520), (300, 2048, 260), (513, 192, 128), (1100, 64, 72), (4100, 2048, 16)]
+WIDE = [("bf16", 1500, 256, 5632), ("f16", 1100, 128, 6660), ("fp8", 2100, 256, 8196)]   # whole turns of k, ragged rows and columns
+
+
+def backend_values(be, torch, name, x):
+    code, dt, bits, make = {"bf16": (A.BF16, torch.bfloat16, torch.int16, lambda r, s: be.ndarray_from_vec_bf16(r.view(np.uint16), s)),
+                            "f16": (A.F16, torch.float16, torch.int16, lambda r, s: be.ndarray_from_vec_f16(r.view(np.float16), s)),
+                            "fp8": (A.F8, torch.float8_e4m3fn, torch.uint8, be.ndarray_from_vec_fp8)}[name]
+    t = torch.from_numpy(x).to(dt)
+    return make(t.view(bits).numpy().reshape(-1), x.shape), t.double().numpy()
+
+
+def run(be, name, M, K, N):
+    import torch
+
+    rng = np.random.default_rng(M + K + N)
+    x, a = backend_values(be, torch, name, rng.standard_normal((1, M, K), dtype=np.float32))
+    w, b = backend_values(be, torch, name, rng.standard_normal((N, K), dtype=np.float32) * np.float32(K ** -0.5))
+    got = be.to_numpy(be.cast(be.matmul(x, be.broadcast(be.transpose(w, 0, 1), (1, K, N))), A.F32))[0]
+    want = a[0].astype(np.float32) @ b.T.astype(np.float32) if M * N * K > 1 << 31 else a[0] @ b.T
+    # the rounding to the dtype (fp8 below 2^-6: in steps of 2^-9) and the 32-bit sums of both sides
+    bound = UNIT[name] * np.abs(want) + (2.0 ** -10 if name == "fp8" else 2.0 ** -25) + 2 * K * 2.0 ** -24 * 8.0
+    assert (np.abs(got - want) <= bound).all()
+
+
+@pytest.mark.parametrize("name", ["bf16", "f16", "fp8"])
+@pytest.mark.parametrize("size", SIZES, ids=str)
+def test_against_float64(hip, name, size):
+    run(hip, name, *size)
+
+
+@pytest.mark.parametrize("case", WIDE, ids=str)
+def test_edges_of_the_wide_tile(hip, case):
+    run(hip, *case)
+
+
+def test_fp8_sums_keep_32_bits(hip):
+    """Sums that lie within 2^-20 of the middle between two fp8 values go to the right one."""
+    import torch
+
+    M, K, N = 80, 4096, 640
+    x = np.zeros((1, M, K), dtype=np.float32)
+    w = np.zeros((N, K), dtype=np.float32)
+    x[0, :, 0], w[:, 0] = 16.0, 1.0
+    x[0, :, 1], w[:, 1] = 1.0, 1.0                # half way between 16 and 18, and 16 is even
+    x[0, :, 2], w[:, 2] = 2.0 ** -6, 2.0 ** -9    # a push upwards
+    xs, _ = backend_values(hip, torch, "fp8", x)
+    ws, _ = backend_values(hip, torch, "fp8", w)
+    got = hip.to_numpy(hip.cast(hip.matmul(xs, hip.broadcast(hip.transpose(ws, 0, 1), (1, K, N))), A.F32))
+    assert (got == 18.0).all()                    # 16 + 1 + 2^-15
