@@ -1388,6 +1388,72 @@ __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_residual_kernel(
     skinny_kt_mfma_xreg_body<MM, 1, false, true, false, TRIPS>(a, blockIdx.x, blockIdx.y, nullptr, 0, &r);
 }
 // the same with the RMS norm of the left operand applied on load
+// The same sum with residual terms for up to four rows, eight columns and all of K by eight waves: an eighth of a chunk of K each,
+// every load of a chunk asked for before the first product.  The kernel above fetches as many bytes of activations as of weights
+// (four columns per workgroup), and a compute unit's path to L2 bounds it; here the activations are half of the weights' bytes.
+// 4 x 8192 x 2048 (64 MiB of weights): 17.2 us above, 15.9 here; 4 x 2048 x 2048: 6.5 and 6.2.
+constexpr int kEightThreads = 512;
+template <int TRIPS> __global__ __launch_bounds__(kEightThreads, 2) void skinny_kt_mfma_eight_residual_kernel(const MmArgs a, const MmResidual res) {
+    const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 4, b = lane / 4;
+    const uint32_t n0 = blockIdx.x * 8;
+    const uint32_t *const w0 = a.B + (int64_t)min(n0 + j, a.N - 1) * a.b_sn, *const w1 = a.B + (int64_t)min(n0 + 4 + j, a.N - 1) * a.b_sn;
+    const uint32_t *const x = a.A + (int64_t)min(j, a.M - 1) * a.a_sm;
+    // the sum's other terms for the value this thread will store
+    const uint32_t tc = threadIdx.x / 16, tm = threadIdx.x / 4 % 4, tcol = n0 + 4 * tc + threadIdx.x % 4;
+    const bool stored = threadIdx.x < 32 && tcol < a.N && tm < a.M;
+    uint32_t term[4] = {};
+    if (stored) {
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+            if ((uint32_t)t != res.slot && (uint32_t)t < res.nterms) term[t] = res.term[t][(uint64_t)tm * a.N + tcol];
+    }
+    float4v acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    for (uint32_t k0 = wave * (TRIPS * 64) + b * 4; k0 < a.K; k0 += TRIPS * kEightThreads) { // (K: whole chunks)
+        float4v xr[TRIPS], wr[2][TRIPS];
+#pragma unroll
+        for (int t = 0; t < TRIPS; t++) {
+            wr[0][t] = *reinterpret_cast<const float4v *>(w0 + k0 + 64 * t);
+            wr[1][t] = *reinterpret_cast<const float4v *>(w1 + k0 + 64 * t);
+            xr[t] = *reinterpret_cast<const float4v *>(x + k0 + 64 * t);
+        }
+        __builtin_amdgcn_sched_barrier(0); // (or the compiler asks for a few at a time)
+#pragma unroll
+        for (int t = 0; t < TRIPS; t++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int c = 0; c < 2; c++) acc[c] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[t][e], wr[c][t][e], acc[c], 0, 0, 0);
+    }
+    __shared__ float part[8][32];
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float v = acc[c][i];
+#pragma unroll
+            for (int s = 32; s >= 4; s >>= 1) v += __shfl_xor(v, s);
+            if (lane < 4) part[wave][c * 16 + i * 4 + j] = v;
+        }
+    __syncthreads();
+    if (threadIdx.x >= 32) return;
+    const uint32_t t = threadIdx.x;
+    uint32_t v = asu(((part[0][t] + part[1][t]) + (part[2][t] + part[3][t])) + ((part[4][t] + part[5][t]) + (part[6][t] + part[7][t])));
+#pragma unroll
+    for (int k = 0; k < 4; k++) term[k] = (uint32_t)k == res.slot ? v : term[k];
+    v = residual_sum(res, term);
+    if (stored) a.C[(uint64_t)tm * a.N + tcol] = v;
+    if (res.partials) { // the rows' sums of squares over four columns each, as above
+        float q = stored ? asf(v) * asf(v) : 0.0f;
+        q += __shfl_xor(q, 1);
+        q += __shfl_xor(q, 2);
+        if (t % 4 == 0 && n0 + 4 * tc < a.N) res.partials[((uint64_t)blockIdx.x * 2 + tc) * 4 + tm] = q;
+    }
+}
+// trips of 64 values of k per wave and chunk; 0: K is not whole chunks, or there are too few columns for a workgroup per compute unit
+static inline int eight_trips(const cg_backend *be, uint32_t M, uint32_t N, uint32_t K) {
+    if (M > 4 || (uint64_t)N < 8ull * be->compute_units) return 0;
+    return K % 8192 == 0 ? 16 : K % 4096 == 0 ? 8 : K % 2048 == 0 ? 4 : 0;
+}
 template <int TRIPS = 8>
 __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_gated_norm_kernel(const MmArgs a, const uint32_t *second, uint32_t one,
                                                                                   const NormFuse nf) {
@@ -2184,7 +2250,12 @@ int launch_matmul_residual(cg_backend *be, const cg_tensor *x, const cg_tensor *
     }
     ProfScope prof(be, CG_K_GEMM_SKINNY, distinct_bytes(x) + distinct_bytes(y) + 4.0 * distinct_bytes(out));
     dim3 grid((uint32_t)((a.N + 3) / 4));
-    if (xreg_narrow(a.M, a.K)) {
+    const int eight = eight_trips(be, a.M, a.N, a.K);
+    const dim3 grid8((uint32_t)((a.N + 7) / 8));
+    if (eight == 16) hipLaunchKernelGGL(skinny_kt_mfma_eight_residual_kernel<16>, grid8, dim3(kEightThreads), 0, be->stream, a, r);
+    else if (eight == 8) hipLaunchKernelGGL(skinny_kt_mfma_eight_residual_kernel<8>, grid8, dim3(kEightThreads), 0, be->stream, a, r);
+    else if (eight == 4) hipLaunchKernelGGL(skinny_kt_mfma_eight_residual_kernel<4>, grid8, dim3(kEightThreads), 0, be->stream, a, r);
+    else if (xreg_narrow(a.M, a.K)) {
         if (xreg_trips(a.K) == 8)
             hipLaunchKernelGGL((skinny_kt_mfma_xreg_residual_kernel<4, 8>), grid, dim3(kThreads), 0, be->stream, a, r);
         else
