@@ -127,7 +127,7 @@ int launch_split_gemm(cg_backend *be, MmArgs a, bool a_mfast, bool b_nfast) {
     const bool care = !a.a_vec || !a.b_vec || !fits(a_mfast, a.a_sm, a.a_sk, a.M) || !fits(b_nfast, a.b_sn, a.b_sk, a.N);
     auto count = [&](int t) { return (uint64_t)((a.M + all[t].bm - 1) / all[t].bm) * ((a.N + all[t].bn - 1) / all[t].bn) * a.batch; };
     const uint64_t mn = (uint64_t)a.M * a.N;
-    // The tile, and over how many workgroups k is cut (at least 96 values each, partial results of at most 64 MB), by what a
+    // The tile, and over how many workgroups k is cut (at least 64 values each, partial results of at most 64 MB), by what a
     // round of workgroups over the compute units takes: measured over M = 16 .. 4096 at the models' widths, where this picks the
     // fastest of all pairs or one within 5 % of it.  512 x 2048 x 2048: 38 us in four parts of 128 x 128 tiles, 47 in two of the
     // wide one; 2048 x 2048 x 8192: 305 with the wide one, 357 without; 32 x 2048 x 8192: 23 with 32 x 256, 35 with 128 x 128.
@@ -136,7 +136,7 @@ int launch_split_gemm(cg_backend *be, MmArgs a, bool a_mfast, bool b_nfast) {
     double best = 0;
     auto consider = [&](int tile) {
         const uint64_t wgs = count(tile);
-        for (uint64_t p = 1; p <= 16 && (p == 1 || (a.K / p >= 96 && p * a.batch * mn <= (16u << 20))); p++) {
+        for (uint64_t p = 1; p <= 16 && (p == 1 || (a.K / p >= 64 && p * a.batch * mn <= (16u << 20))); p++) {
             const uint32_t part = p > 1 ? (uint32_t)((a.K + p - 1) / p + 31) / 32 * 32 : a.K;
             if (p > 1 && (a.K + part - 1) / part != p) continue;
             const double rounds = (double)((wgs * p + be->compute_units - 1) / be->compute_units);

