@@ -1,6 +1,7 @@
 // Launchers of the attention kernels (attention.hpp): decode-time attention over a KV cache in one
 // pass, in segments or in chunks with a combine, and prefill attention on the matrix cores.
 #include "interp.hpp"
+#include "split_tile.hpp"
 
 namespace cg {
 

@@ -841,12 +841,13 @@ __global__ __launch_bounds__(kBlock) void decode_attention_combine_kernel(const 
 //     S^T[t][m] = K[t] . Q[m] / scale  first MFMA operand K (from LDS), second Q / scale (registers, loaded once)
 //     running maximum / sum per query  = per lane: in-register over its 32 values + one exchange with lane ^ 32
 //     O^T[d][m] += V^T[d][t] P^T[t][m] first operand V^T (columns of the LDS tile), second P^T — which, in the accumulator
-//                                      layout of v_mfma_f32_32x32x2 (column = lane % 32, rows 8*(v/4) + 4*(lane/32)
-//                                      + v%4), already is the operand layout: no trip through LDS, no transposition
+//                                      layout of the 32x32 instructions (column = lane % 32, rows 8*(v/4) +
+//                                      4*(lane/32) + v%4), already is the operand layout: no trip through LDS
 // The scores are divided by the scale and masked exactly as the soft-max program does (x / d + f32(i < j) * m with
 // i the query's position, j the key's); masked keys get weight zero, which is what exp(x - max) rounds to for them.
 // out = O / l at the end (the program divides the weights first: same value up to rounding).
-// MFMA-bound: 2 x 2 x 32 x 64 x 64 flop per wave and tile over ~half of the [rows, T] rectangle.
+// Bound by the matrix pipes, and in pieces by them and the splitting together: 2 x 2 x 32 x 64 x 64 flop per wave and tile over
+// ~half of the [rows, T] rectangle.
 struct PrefillArgs {
     uint32_t *out;      // [batch][M][hd], dense
     uint32_t S;         // query positions per head: row m of a group is position m % S
@@ -863,16 +864,24 @@ struct PrefillArgs {
 };
 
 constexpr int kPfRows = 128, kPfKeys = 64;
-// K and V tiles, [64 keys][head_dim + 4] each (a row starts 4 banks after the one before), double buffered:
-// 68 KiB for head_dim 64 (two workgroups per CU), 132 KiB for 128 (one)
+// The 32-bit instructions' K and V tiles, [64 keys][head_dim + 4] each (a row starts 4 banks after the one before), double
+// buffered: 68 KiB for head_dim 64 (two workgroups per CU), 132 KiB for 128 (one).  The pieces take 48 KiB of it, one buffer:
+// the next tile waits in registers (and at head_dim 64 the other workgroup covers the second barrier).
 constexpr size_t prefill_lds_bytes(int hd) { return 2 * 2 * (size_t)kPfKeys * (hd + 4) * sizeof(float); }
 
-template <int HD>
-__global__ __launch_bounds__(kBlock) void prefill_attention_kernel(const AttnArgs g, const PrefillArgs e) {
+// PIECES: both products as products of bfloat16 pieces (split_tile.hpp), 2.67 times the rate of the 32-bit instructions: the
+// queries' pieces stay in registers, those of K and V are made on the way into LDS, once for the four waves (V turned, so that a
+// fragment's eight keys are the eight that a lane holds weights of), and the weights are split in place.  Returns true, and has
+// stored nothing, if a value lies at the ends of the range that pieces cover; !PIECES: the 32-bit instructions.
+// Measured, 32-bit instructions -> pieces: 4 x 2048 tokens, 32 heads of 64 over 8 KV heads 626 -> 427 us (159 TFLOP/s of the visible
+// half); 1024 tokens, 16 heads of 128 over 8 85 -> 75; 512 tokens, 9 heads of 64 over 3 19.6 -> 16.4; 4 x 8 tokens 12.7 -> 12.9.  The
+// products are no longer what bounds it alone: splitting K, V and the weights, the exponentials and the two barriers of a tile weigh as
+// much.  Error against 64 bits: no larger (a sum is rounded once per 16 terms and piece).
+template <int HD, bool PIECES> __device__ __forceinline__ bool prefill_rows(const AttnArgs &g, const PrefillArgs &e, float *const pf_lds) {
     static_assert(HD == 64 || HD == 128, "head_dim 64 or 128");
+    constexpr int KEYS = PIECES && HD == 128 ? 32 : kPfKeys; // per tile
     constexpr int kPfPitch = HD + 4;
     typedef float float16v __attribute__((ext_vector_type(16)));
-    extern __shared__ float pf_lds[]; // above the static limit
     float (*Ks)[kPfKeys][kPfPitch] = reinterpret_cast<float (*)[kPfKeys][kPfPitch]>(pf_lds);                       // [2][t][d]
     float (*Vs)[kPfKeys][kPfPitch] = reinterpret_cast<float (*)[kPfKeys][kPfPitch]>(pf_lds + 2 * kPfKeys * kPfPitch); // [2][t][d]
     const uint32_t tid = threadIdx.x, lane = tid % 64, wave = tid / 64, li = lane % 32, lg = lane / 32;
@@ -919,21 +928,49 @@ __global__ __launch_bounds__(kBlock) void prefill_attention_kernel(const AttnArg
         kmax = min(g.T - 1, e.pos0 + smax);
     }
     const uint32_t ntiles_all = kmax / kPfKeys + 1;
-    // this workgroup's share of the key tiles (all of them without a split)
+    // this workgroup's share of the key tiles (all of them without a split), the same for either way to multiply
     const uint32_t per_part = (ntiles_all + e.ksplit - 1) / e.ksplit;
-    const uint32_t it_first = blockIdx.y * per_part, ntiles = min(ntiles_all, it_first + per_part);
+    const uint32_t it_first = blockIdx.y * per_part * (kPfKeys / KEYS);
+    const uint32_t ntiles = min(kmax / KEYS + 1, (blockIdx.y + 1) * per_part * (kPfKeys / KEYS));
 
     // the query rows, as second MFMA operands: chunk c covers d = 8c .. 8c+7, this lane holds 4*lg .. 4*lg+3 of them.
     // The program divides every score by the scale; dividing the query once instead is the same value up to
     // rounding and takes the division out of the loop.
     const float scale = asf(e.scale);
-    float4v qf[HD / 8];
+    typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+    typedef uint32_t uint4w __attribute__((ext_vector_type(4)));
+    float4v qf[PIECES ? 1 : HD / 8];
+    bf16x8 qp[PIECES ? HD / 16 : 1][3]; // chunk c: d = 16 c + 8 lg .. + 7
+    float top_qk = 0.0f, top_v[4] = {}; // largest magnitudes seen, V's by the columns that this thread loads
+    if constexpr (!PIECES) {
 #pragma unroll
-    for (int c = 0; c < HD / 8; c++) {
-        qf[c] = (float4v){0.f, 0.f, 0.f, 0.f};
-        if (live) qf[c] = *reinterpret_cast<const float4v *>(g.Q + oq + (int64_t)m * g.q_sm + c * 8 + lg * 4);
+        for (int c = 0; c < HD / 8; c++) {
+            qf[c] = (float4v){0.f, 0.f, 0.f, 0.f};
+            if (live) qf[c] = *reinterpret_cast<const float4v *>(g.Q + oq + (int64_t)m * g.q_sm + c * 8 + lg * 4);
 #pragma unroll
-        for (int r = 0; r < 4; r++) qf[c][r] = qf[c][r] / scale;
+            for (int r = 0; r < 4; r++) qf[c][r] = qf[c][r] / scale;
+        }
+    } else {
+#pragma unroll
+        for (int c = 0; c < HD / 16; c++) {
+            uint4w w[3];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                float4v q = {0.f, 0.f, 0.f, 0.f};
+                if (live) q = *reinterpret_cast<const float4v *>(g.Q + oq + (int64_t)m * g.q_sm + c * 16 + lg * 8 + h * 4);
+#pragma unroll
+                for (int r = 0; r < 4; r++) q[r] = q[r] / scale;
+                split::grow(top_qk, q[0], q[1]);
+                split::grow(top_qk, q[2], q[3]);
+                uint32_t a[3], b[3];
+                split::split2(q[0], q[1], a);
+                split::split2(q[2], q[3], b);
+#pragma unroll
+                for (int p = 0; p < 3; p++) w[p][2 * h] = a[p], w[p][2 * h + 1] = b[p];
+            }
+#pragma unroll
+            for (int p = 0; p < 3; p++) qp[c][p] = __builtin_bit_cast(bf16x8, w[p]);
+        }
     }
     float16v acc_o[HD / 32];
 #pragma unroll
@@ -943,65 +980,114 @@ __global__ __launch_bounds__(kBlock) void prefill_attention_kernel(const AttnArg
     float run_max = -INFINITY, run_sum = 0.0f;
     constexpr float kLog2e = 1.4426950408889634f;
 
-    // K / V tile: 64 positions x HD floats each = 16 * HD float4 per operand, HD / 16 per thread
-    constexpr int kSlots = kPfKeys * (HD / 4) / kBlock, kQpr = HD / 4;
+    // K / V tile: KEYS positions x HD floats each, in 16-byte slots
+    constexpr int kSlots = KEYS * (HD / 4) / kBlock, kQpr = HD / 4;
     float4v kr[kSlots], vr[kSlots];
+    typedef __attribute__((address_space(3))) char lds_char;
+    lds_char *const lds = (lds_char *)pf_lds;
+    constexpr uint32_t PIECE = KEYS * HD * 2; // bytes of a piece of K, and of V behind K's three
     auto load_kv = [&](uint32_t t0) {
 #pragma unroll
         for (int h = 0; h < kSlots; h++) {
-            const uint32_t slot = tid + h * kBlock, t = t0 + slot / kQpr, dq = slot % kQpr;
+            // (pieces: K a row's 16 values by four lanes; V four positions of four columns)
+            const uint32_t slot = tid + h * kBlock;
+            const uint32_t tk = t0 + (PIECES ? tid / 4 % KEYS : slot / kQpr), dk = PIECES ? (tid / (4 * KEYS) + h * (kBlock / (4 * KEYS))) * 4 + tid % 4 : slot % kQpr;
+            const uint32_t tv = t0 + (PIECES ? tid / kQpr * 4 + h : slot / kQpr), dv = PIECES ? tid % kQpr : slot % kQpr;
             kr[h] = (float4v){0.f, 0.f, 0.f, 0.f};
             vr[h] = (float4v){0.f, 0.f, 0.f, 0.f};
-            if (t < g.T) {
-                kr[h] = *reinterpret_cast<const float4v *>(g.Kc + ok + (int64_t)t * g.k_st + dq * 4);
-                vr[h] = *reinterpret_cast<const float4v *>(g.V + ov + (int64_t)t * g.v_st + dq * 4);
-            }
+            if (tk < g.T) kr[h] = *reinterpret_cast<const float4v *>(g.Kc + ok + (int64_t)tk * g.k_st + dk * 4);
+            if (tv < g.T) vr[h] = *reinterpret_cast<const float4v *>(g.V + ov + (int64_t)tv * g.v_st + dv * 4);
         }
     };
     auto store_kv = [&](uint32_t buf) {
+        if constexpr (!PIECES) {
 #pragma unroll
-        for (int h = 0; h < kSlots; h++) {
-            const uint32_t slot = tid + h * kBlock, t = slot / kQpr, dq = slot % kQpr;
-            *reinterpret_cast<float4v *>(&Ks[buf][t][dq * 4]) = kr[h];
-            *reinterpret_cast<float4v *>(&Vs[buf][t][dq * 4]) = vr[h];
+            for (int h = 0; h < kSlots; h++) {
+                const uint32_t slot = tid + h * kBlock, t = slot / kQpr, dq = slot % kQpr;
+                *reinterpret_cast<float4v *>(&Ks[buf][t][dq * 4]) = kr[h];
+                *reinterpret_cast<float4v *>(&Vs[buf][t][dq * 4]) = vr[h];
+            }
+        } else {
+            typedef __attribute__((address_space(3))) split::uint2v lds_pair;
+            // K: blocks of 32 keys x 16 d in the order of the fragments' lanes (rows of the second lane group at row ^ 12)
+            const uint32_t t = tid / 4 % KEYS, kg = tid % 4 / 2;
+            const uint32_t k_at = (tid / (4 * KEYS) * (KEYS / 32) + t / 32) * 1024 + kg * 512 + ((t % 32) ^ (kg * 12)) * 16 + tid % 2 * 8;
+            // V: blocks of 32 d x 16 keys; four rows change places by (d / 16) so that the lanes' stores cover all banks
+            const uint32_t u = tid / kQpr, w = tid % kQpr, vg = u & 1;
+            const uint32_t v_at = 3 * PIECE + (u / 4 * (HD / 32) + w / 8) * 1024 + vg * 512 + (u >> 1 & 1) * 8;
+#pragma unroll
+            for (int h = 0; h < kSlots; h++) {
+                uint32_t a[3], b[3];
+                split::grow(top_qk, kr[h][0], kr[h][1]);
+                split::grow(top_qk, kr[h][2], kr[h][3]);
+                split::split2(kr[h][0], kr[h][1], a);
+                split::split2(kr[h][2], kr[h][3], b);
+#pragma unroll
+                for (int p = 0; p < 3; p++) *reinterpret_cast<lds_pair *>(lds + p * PIECE + k_at + h * (kBlock / (4 * KEYS)) * (KEYS / 32) * 1024) = (split::uint2v){a[p], b[p]};
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                uint32_t a[3], b[3];
+                split::grow(top_v[r], vr[0][r], vr[1][r]);
+                split::grow(top_v[r], vr[2][r], vr[3][r]);
+                split::split2(vr[0][r], vr[1][r], a);
+                split::split2(vr[2][r], vr[3][r], b);
+                const uint32_t row = (w % 8 * 4 + (r ^ (w / 4 & 3))) ^ (vg * 12);
+#pragma unroll
+                for (int p = 0; p < 3; p++) *reinterpret_cast<lds_pair *>(lds + p * PIECE + v_at + row * 16) = (split::uint2v){a[p], b[p]};
+            }
         }
     };
+    auto piece = [&](uint32_t at) { return __builtin_bit_cast(bf16x8, *reinterpret_cast<__attribute__((address_space(3))) float4v *>(lds + at)); };
     if (it_first < ntiles) { // (a part beyond the last key tile of these rows has nothing to do but to say so)
-        load_kv(it_first * kPfKeys);
+        load_kv(it_first * KEYS);
         store_kv(it_first & 1);
     }
     __syncthreads();
 
     for (uint32_t it = it_first; it < ntiles; it++) {
-        const uint32_t cur = it & 1, t0 = it * kPfKeys;
+        const uint32_t cur = it & 1, t0 = it * KEYS;
         const bool more = it + 1 < ntiles;
-        if (more) load_kv(t0 + kPfKeys);
-        // ---- S^T = K Q^T for the tile: two blocks of 32 keys x this wave's 32 queries
-        float16v acc_s[kPfKeys / 32];
+        if (more) load_kv(t0 + KEYS);
+        // ---- S^T = K Q^T for the tile: blocks of 32 keys x this wave's 32 queries
+        float16v acc_s[KEYS / 32];
 #pragma unroll
-        for (int tb = 0; tb < kPfKeys / 32; tb++) {
+        for (int tb = 0; tb < KEYS / 32; tb++) {
 #pragma unroll
             for (int v = 0; v < 16; v++) acc_s[tb][v] = 0.0f;
+            if constexpr (PIECES) continue;
 #pragma unroll
-            for (int c = 0; c < HD / 8; c++) {
+            for (int c = 0; c < (PIECES ? 0 : HD / 8); c++) {
                 const float4v kf = *reinterpret_cast<const float4v *>(&Ks[cur][tb * 32 + li][c * 8 + lg * 4]);
 #pragma unroll
                 for (int r = 0; r < 4; r++) acc_s[tb] = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[r], qf[c][r], acc_s[tb], 0, 0, 0);
             }
         }
+        if constexpr (PIECES) {
+#pragma unroll
+            for (int c = 0; c < HD / 16; c++)
+#pragma unroll
+                for (int tb = 0; tb < KEYS / 32; tb++) {
+                    bf16x8 kf[3];
+#pragma unroll
+                    for (int p = 0; p < 3; p++) kf[p] = piece(p * PIECE + (c * (KEYS / 32) + tb) * 1024 + lg * 512 + (li ^ (lg * 12)) * 16);
+#pragma unroll
+                    for (int k = 0; k < 6; k++) acc_s[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[split::kPairA[k]], qp[c][split::kPairB[k]], acc_s[tb], 0, 0, 0);
+                }
+        }
         // ---- mask, running soft-max statistics of this lane's query.  Weights are 2^((x - max) log2 e) on the
         // hardware's exp2 (relative error ~1e-6 for the arguments that matter: inside the 1e-4 of element-wise math).
         // A tile that every query of the wave sees whole (the common case below the diagonal) needs no per-key test.
-        const bool whole = __all((int)(live && t0 + kPfKeys - 1 <= iq && t0 + kPfKeys <= g.T));
+        const bool whole = __all((int)(live && t0 + KEYS - 1 <= iq && t0 + KEYS <= g.T));
         float tile_max = -INFINITY;
         if (whole) {
 #pragma unroll
-            for (int tb = 0; tb < kPfKeys / 32; tb++)
+            for (int tb = 0; tb < KEYS / 32; tb++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) tile_max = fmaxf(tile_max, acc_s[tb][v]);
         } else {
 #pragma unroll
-            for (int tb = 0; tb < kPfKeys / 32; tb++)
+            for (int tb = 0; tb < KEYS / 32; tb++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
                     // the program's x / d + f32(i < j) * m: nothing is added to a visible key, and an invisible one
@@ -1018,7 +1104,7 @@ __global__ __launch_bounds__(kBlock) void prefill_attention_kernel(const AttnArg
         const float alpha = __builtin_amdgcn_exp2f((run_max - base) * kLog2e);
         float tile_sum = 0.0f;
 #pragma unroll
-        for (int tb = 0; tb < kPfKeys / 32; tb++)
+        for (int tb = 0; tb < KEYS / 32; tb++)
 #pragma unroll
             for (int v = 0; v < 16; v++) {
                 const float p = __builtin_amdgcn_exp2f((acc_s[tb][v] - base) * kLog2e); // 2^-inf = 0 for a hidden key
@@ -1028,24 +1114,60 @@ __global__ __launch_bounds__(kBlock) void prefill_attention_kernel(const AttnArg
         tile_sum += __shfl_xor(tile_sum, 32);
         run_sum = run_sum * alpha + tile_sum;
         run_max = new_max;
-        // ---- O^T = alpha O^T + V^T P^T: the V operand is read column-wise from the [t][d] tile (32 lanes, 32 banks)
+        if constexpr (!PIECES) {
+            // ---- O^T = alpha O^T + V^T P^T: the V operand is read column-wise from the [t][d] tile (32 lanes, 32 banks)
 #pragma unroll
-        for (int db = 0; db < HD / 32; db++) {
+            for (int db = 0; db < HD / 32; db++) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc_o[db][v] *= alpha;
+                for (int v = 0; v < 16; v++) acc_o[db][v] *= alpha;
 #pragma unroll
-            for (int tb = 0; tb < kPfKeys / 32; tb++)
+                for (int tb = 0; tb < KEYS / 32; tb++)
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
+                    for (int q = 0; q < 4; q++) {
 #pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const float vf = Vs[cur][tb * 32 + q * 8 + lg * 4 + r][db * 32 + li];
-                        acc_o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf, acc_s[tb][q * 4 + r], acc_o[db], 0, 0, 0);
+                        for (int r = 0; r < 4; r++) {
+                            const float vf = Vs[cur][tb * 32 + q * 8 + lg * 4 + r][db * 32 + li];
+                            acc_o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf, acc_s[tb][q * 4 + r], acc_o[db], 0, 0, 0);
+                        }
                     }
+            }
+        } else {
+#pragma unroll
+            for (int db = 0; db < HD / 32; db++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc_o[db][v] *= alpha;
+#pragma unroll
+            for (int q = 0; q < KEYS / 16; q++) { // 16 keys: the eight weights that a lane holds of them, and V's rows in that order
+                uint4w pw[3];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    uint32_t x[3];
+                    split::split2(acc_s[q / 2][q % 2 * 8 + 2 * r], acc_s[q / 2][q % 2 * 8 + 2 * r + 1], x);
+#pragma unroll
+                    for (int p = 0; p < 3; p++) pw[p][r] = x[p];
                 }
+#pragma unroll
+                for (int db = 0; db < HD / 32; db++) {
+                    bf16x8 vf[3];
+                    const uint32_t row = (li ^ ((db * 2 + li / 16) & 3)) ^ (lg * 12);
+#pragma unroll
+                    for (int p = 0; p < 3; p++) vf[p] = piece((3 + p) * PIECE + (q * (HD / 32) + db) * 1024 + lg * 512 + row * 16);
+#pragma unroll
+                    for (int k = 0; k < 6; k++)
+                        acc_o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[split::kPairA[k]], __builtin_bit_cast(bf16x8, pw[split::kPairB[k]]), acc_o[db], 0, 0, 0);
+                }
+            }
+            __syncthreads(); // (one buffer: the tile is read)
         }
         if (more) store_kv(cur ^ 1);
         __syncthreads();
+    }
+    if constexpr (PIECES) {
+        // (a score is a sum of products of magnitudes below 1e18: what the smallest values' pieces lose of it is nothing beside 1)
+        bool bad = top_qk > 1.0e18f;
+#pragma unroll
+        for (int r = 0; r < 4; r++) bad = bad || split::out_of_range(top_v[r]);
+        if (__syncthreads_or(bad)) return true;
     }
     if (e.ksplit > 1) { // the part's statistics and un-normalised O; lane group 0 of a wave writes the statistics
         if (live) {
@@ -1065,7 +1187,7 @@ __global__ __launch_bounds__(kBlock) void prefill_attention_kernel(const AttnArg
                 e.part_ml[row * 2 + 1] = run_sum;
             }
         }
-        return;
+        return false;
     }
     // ---- out[m][d] = O^T[d][m] / l[m]
     if (live) {
@@ -1080,6 +1202,12 @@ __global__ __launch_bounds__(kBlock) void prefill_attention_kernel(const AttnArg
                 *reinterpret_cast<float4v *>(orow + db * 32 + j * 8 + lg * 4) = o;
             }
     }
+    return false;
+}
+
+template <int HD> __global__ __launch_bounds__(kBlock, HD == 64 ? 2 : 1) void prefill_attention_kernel(const AttnArgs g, const PrefillArgs e) {
+    extern __shared__ float pf_lds[]; // above the static limit
+    if (prefill_rows<HD, true>(g, e, pf_lds)) prefill_rows<HD, false>(g, e, pf_lds);
 }
 
 // out[row][d] = sum_p 2^((m_p - g) log2 e) O_p[row][d] / sum_p 2^((m_p - g) log2 e) l_p, g = max_p m_p: the parts of a
