@@ -184,10 +184,12 @@ template <int FMT, int OUT> int run_tiles(cg_backend *be, TileArgs a) {
     splits = (a.K + a.k_part - 1) / a.k_part;
     void *parts = nullptr, *const y = a.y;
     size_t cls = 0;
-    if (splits > 1) {
-        if (int rc = be->pool.alloc(mn * splits * 4, &parts, &cls)) return rc;
-        a.y = parts;
+    if (splits > 1 && be->pool.alloc(mn * splits * 4, &parts, &cls)) {
+        (void)hipGetLastError();
+        splits = 1; // no room for the parts: uncut
+        a.k_part = (a.K + kStageBytes - 1) / kStageBytes * kStageBytes;
     }
+    if (splits > 1) a.y = parts;
     const dim3 grid((uint32_t)tiles, splits);
     const size_t lds = (size_t)kStages * (tm + kTileN) * kStageBytes;
     if (splits > 1) {

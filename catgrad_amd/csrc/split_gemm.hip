@@ -163,8 +163,11 @@ int launch_split_gemm(cg_backend *be, MmArgs a, bool a_mfast, bool b_nfast) {
         a.ksplit = (uint32_t)((a.K + splits - 1) / splits + 31) / 32 * 32;
         splits = (a.K + a.ksplit - 1) / a.ksplit;
     }
+    if (splits > 1 && be->pool.alloc(a.batch * splits * mn * 4, &parts, &cls)) {
+        (void)hipGetLastError();
+        splits = 1; // no room for the parts: uncut
+    }
     if (splits > 1) {
-        if (int rc = be->pool.alloc(a.batch * splits * mn * 4, &parts, &cls)) return rc;
         a.C = static_cast<uint32_t *>(parts);
     } else {
         splits = 1;
