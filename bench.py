@@ -30,14 +30,18 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK = 8.0e12       # B/s, MI355X HBM3E
-MFMA_F32_PEAK = 157.3e12  # flop/s, MI355X dense f32 matrix
+MFMA_BF16_PEAK = 2.5e15  # flop/s, MI355X dense bf16 matrix
+# f32 products and the prefill's attention multiply three bfloat16 pieces of every value, six instructions for one product at f32
+# precision: the ceiling of that (the f32 matrix instructions' own peak is 157.3e12)
+SPLIT_PEAK = MFMA_BF16_PEAK / 6
+TRAFFIC_FILE = "split_gemm_llama1b_prefill_pmc.txt"
 
 
 def profiled_traffic():
-    """HBM bytes per launch of the dominant kernel (mfma_gemm_kernel) on the config-5 prefill, as the rocprofv3
+    """HBM bytes per launch of the dominant kernel (split_gemm_kernel) on the config-5 prefill, as the rocprofv3
     FETCH_SIZE / WRITE_SIZE passes measured them: read from the committed summary (its line
     `traffic_bytes_per_launch: <n>`), not measured by this process (counters need the profiler)."""
-    path = os.path.join(ROOT, "profiles", "mfma_gemm_llama1b_prefill_pmc.txt")
+    path = os.path.join(ROOT, "profiles", TRAFFIC_FILE)
     try:
         for line in open(path):
             if line.startswith("traffic_bytes_per_launch:"):
@@ -55,7 +59,7 @@ def micro_bench(iters=20):
     rng = np.random.default_rng(0)
     out = {}
 
-    def run(name, cls, fn, unit, launches_per_call=1, mfma_peak=MFMA_F32_PEAK):
+    def run(name, cls, fn, unit, launches_per_call=1, mfma_peak=SPLIT_PEAK):
         # warm up to steady clocks: the uploads before a line leave the card idle long enough for it to clock down, and
         # the first few milliseconds of launches after that run up to 15 % slow
         t_warm = time.perf_counter()
@@ -102,7 +106,7 @@ def micro_bench(iters=20):
     # rounded to the dtype in the product's store; against the dense peaks of those instructions
     x32 = be.from_numpy(rng.standard_normal((1, 8192, 2048), dtype=np.float32) * np.float32(0.25))
     w32 = be.from_numpy(rng.standard_normal((8192, 2048), dtype=np.float32) * np.float32(0.25))
-    for dt, tag, peak in ((A.BF16, "bf16", 2.5e15), (A.F8, "fp8", 5.0e15)):
+    for dt, tag, peak in ((A.BF16, "bf16", MFMA_BF16_PEAK), (A.F8, "fp8", 5.0e15)):
         wn = be.cast(w32, dt)
         be.realize(wn)
         wv = be.broadcast(be.transpose(wn, 0, 1), (1, 2048, 8192))
@@ -285,25 +289,25 @@ def measure(config, steps, warmup, batch=None, prefill=None, decode=None, seed=0
         "decode_ms_per_step": round(tg_s / K / T * 1e3, 4),
         # the whole prefill against the matrix peak: algorithmic flop (all linear layers + dense attention) / prefill time
         "prefill_flop": prefill_flop,
-        "prefill_mfma_frac": round(prefill_flop / (pp_s / K) / MFMA_F32_PEAK, 4),
+        "prefill_mfma_frac": round(prefill_flop / (pp_s / K) / SPLIT_PEAK, 4),
         "backend_calls": {"prefill": calls[0], "per_decode_step": round(calls[1] / max(T, 1), 1)},
         "backend": sess.backend_name,
         "roofline": {
-            "kernel": "mfma_gemm_kernel (f32 v_mfma_f32_32x32x2; 128x128x32 tiles, two workgroups per compute unit; 128x64 and "
-                      "split-k variants for products that do not fill the device)",
-            "bound": "mfma", "achieved": round(mfma_rate / 1e12, 3), "peak": MFMA_F32_PEAK / 1e12, "unit": "TFLOP/s",
-            "frac": round(mfma_rate / MFMA_F32_PEAK, 4),
+            "kernel": "split_gemm_kernel (f32 operands in three bfloat16 pieces, six v_mfma_f32_32x32x16_bf16 per product; 256x256 "
+                      "tiles; smaller ones and cuts along k for products that do not fill the device)",
+            "bound": "mfma", "achieved": round(mfma_rate / 1e12, 3), "peak": SPLIT_PEAK / 1e12, "unit": "TFLOP/s",
+            "frac": round(mfma_rate / SPLIT_PEAK, 4),
             # from the committed rocprofv3 counter summary of this very workload (null for any other)
             "traffic": profiled_traffic() if (config, B, S) == (5, 4, 2048) else None,
-            "traffic_source": "profiles/mfma_gemm_llama1b_prefill_pmc.txt" if (config, B, S) == (5, 4, 2048) else None,
+            "traffic_source": "profiles/" + TRAFFIC_FILE + " (256x256 tile)" if (config, B, S) == (5, 4, 2048) else None,
             "launches_timed": n_m, "avg_launch_ms": round(ms_m / max(n_m, 1), 4),
             "flop_per_launch_avg": flop_m / max(n_m, 1),
         },
         # the one-pass causal attention of the prefill (q.K^T, soft-max, p.V): flop of the visible half only
         "prefill_attention": {
-            "kernel": "prefill_attention_kernel (f32 v_mfma_f32_32x32x2, 128 query rows x 64 keys per step)",
-            "bound": "mfma", "achieved": round(attn_rate / 1e12, 3), "peak": MFMA_F32_PEAK / 1e12, "unit": "TFLOP/s",
-            "frac": round(attn_rate / MFMA_F32_PEAK, 4), "launches_timed": n_a,
+            "kernel": "prefill_attention_kernel (bfloat16 pieces as above, 128 query rows x 64 keys per step)",
+            "bound": "mfma", "achieved": round(attn_rate / 1e12, 3), "peak": SPLIT_PEAK / 1e12, "unit": "TFLOP/s",
+            "frac": round(attn_rate / SPLIT_PEAK, 4), "launches_timed": n_a,
             "avg_launch_ms": round(ms_a / max(n_a, 1), 4), "timed_in": "an untimed pass of its own, before the timed region",
         },
         "decode_roofline": {
@@ -432,7 +436,7 @@ def measure_blocks(design, size, dtype, steps, warmup, seed=0):
         "decode_ms_per_step": round(tg / T * 1e3, 4), "decode_tok_s": round(B * T / tg, 1),
         "weight_bytes_per_step": int(weights * wb), "decode_hbm_frac_weights": round(weights * wb / (tg / T) / HBM_PEAK, 4),
         "prefill_linear_flop": linear_flop,
-        "prefill_linear_peak_frac": round(linear_flop / pp / (2.5e15 if dtype == "bfloat16" else MFMA_F32_PEAK), 4),
+        "prefill_linear_peak_frac": round(linear_flop / pp / (MFMA_BF16_PEAK if dtype == "bfloat16" else SPLIT_PEAK), 4),
         "window": window, "kernel_classes": per_class, "first_tokens": tokens[:2].tolist(),
     }
     return out
