@@ -85,18 +85,24 @@ template <int WM, int WN, int MT, int NT, bool AF, bool BF, bool CARE> Kernel pr
     return hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess ? k : nullptr;
 }
 // microseconds that a round of workgroups (one per compute unit) takes per stage, by tile
-constexpr double kStage[5] = {2.4, 0.72, 0.5, 0.55, 0.8};
+constexpr double kStage[7] = {2.4, 0.72, 0.5, 0.55, 1.65, 0.375, 0.7};
 // In the order of `kStage`: the wide tile, the tile for what does not fill the device with it, two for a few rows, and the second
-// one's twin for any alignment.
+// one's twin for any alignment; 64 x 64 for k-contiguous operands whose results are small or narrow, and its twin.  What the
+// 64 x 64 tile gains over the others (cuts along k included): 1800 x 100 x 400 12.8 -> 9.0 us, 200 x 1001 x 333 23.7 -> 17.3,
+// 64 x 256 x 512 10.8 -> 9.9, 100 x 17 x 100 9.7 -> 7.0; from 1024 x 1024 x 1024 on (29 against 25 us) it loses to 128 x 128.
 const Tile *tiles() {
 #define CG_TILE(WM, WN, MT, NT, CARE)                                                                       \
     {32 * WM * MT, 32 * WN * NT, 64 * WM * WN, {{prepared<WM, WN, MT, NT, false, false, CARE>(), prepared<WM, WN, MT, NT, false, true, CARE>()}, \
                                   {prepared<WM, WN, MT, NT, true, false, CARE>(), prepared<WM, WN, MT, NT, true, true, CARE>()}}}
+#define CG_SMALL_TILE(CARE) \
+    {64, 64, 256, {{prepared<2, 2, 1, 1, false, false, CARE>(), nullptr}, {nullptr, nullptr}}}
 #define CG_LOW_TILE(WM, WN, MT, NT) \
     {32 * WM * MT, 32 * WN * NT, 64 * WM * WN, {{prepared<WM, WN, MT, NT, false, false, false>(), prepared<WM, WN, MT, NT, false, true, false>()}, {nullptr, nullptr}}}
-    static const Tile t[5] = {CG_TILE(2, 4, 4, 2, false), CG_TILE(2, 2, 2, 2, false), CG_LOW_TILE(1, 4, 2, 1), CG_LOW_TILE(1, 4, 1, 2), CG_TILE(2, 2, 2, 2, true)};
+    static const Tile t[7] = {CG_TILE(2, 4, 4, 2, false), CG_TILE(2, 2, 2, 2, false), CG_LOW_TILE(1, 4, 2, 1), CG_LOW_TILE(1, 4, 1, 2), CG_TILE(2, 2, 2, 2, true),
+                              CG_SMALL_TILE(false), CG_SMALL_TILE(true)};
 #undef CG_TILE
 #undef CG_LOW_TILE
+#undef CG_SMALL_TILE
     return t;
 }
 
@@ -140,10 +146,13 @@ int launch_split_gemm(cg_backend *be, MmArgs a, bool a_mfast, bool b_nfast) {
             const uint32_t part = p > 1 ? (uint32_t)((a.K + p - 1) / p + 31) / 32 * 32 : a.K;
             if (p > 1 && (a.K + part - 1) / part != p) continue;
             const double rounds = (double)((wgs * p + be->compute_units - 1) / be->compute_units);
-            const double us = rounds * (2.0 + kStage[tile] * ((part + kDepth - 1) / kDepth)) + (p > 1 ? 4.0 + 1e-6 * p * a.batch * mn : 0.0);
+            const double stages = kStage[tile] * ((part + kDepth - 1) / kDepth);
+            // (small tiles: several to a compute unit, which hide each other's waits)
+            const double us = (tile < 5 ? rounds * ((tile == 1 || tile == 2 ? 3.0 : 2.0) + stages) : 2.0 + stages * std::max(1.0, 0.85 * rounds)) + (p > 1 ? 4.0 + 1e-6 * p * a.batch * mn : 0.0);
             if (t < 0 || us < best) t = tile, splits = p, best = us;
         }
     };
+    if (!a_mfast && !b_nfast) consider(care ? 6 : 5);
     if (care) consider(4);
     else {
         consider(1);

@@ -5,9 +5,10 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-# edges of the tiles (32 x 256, 64 x 128, 128 x 128, 256 x 256), of a stage (16 values of k) and of the cuts along k
+# edges of the tiles (64 x 64, 32 x 256, 64 x 128, 128 x 128, 256 x 256), of a stage (16 values of k) and of the cuts along k
 SIZES = [(9, 16, 8), (9, 1, 33), (17, 33, 31), (32, 2048, 260), (33, 96, 128), (64, 100, 129), (65, 576, 192), (128, 160, 256), (129, 31, 4), (255, 64, 260),
-         (300, 1000, 520), (1030, 48, 1028), (2048, 64, 8192)]
+         (300, 1000, 520), (1030, 48, 1028), (2048, 64, 8192),
+         (64, 64, 64), (65, 63, 65), (1800, 100, 400), (200, 1001, 333), (1500, 700, 50)]
 
 
 def operands(be, M, K, N, a_rows_fast, b_rows_fast, batch=1, seed=0):
