@@ -209,7 +209,8 @@ template <int FMT, int OUT> int run_tiles(cg_backend *be, TileArgs a) {
 
 int launch_narrow_tiles(cg_backend *be, int fmt, const void *x, int64_t x_pitch, int64_t rows, const void *w, int64_t w_pitch, int64_t n, int64_t k, void *y, int y_fmt) {
     const int64_t eb = (int64_t)fmt_bytes(fmt);
-    if (!fits_narrow_tiles(fmt, x, x_pitch, rows, w, w_pitch, n, k)) return kDeclined;
+    if (fmt == kFmtWords || !fits_narrow_tiles(fmt, x_pitch, rows, w_pitch, n, k)) return kDeclined;
+    if (!x || !w || reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16) return kDeclined;
     TileArgs a{};
     a.x = static_cast<const char *>(x);
     a.w = static_cast<const char *>(w);
@@ -225,20 +226,14 @@ int launch_narrow_tiles(cg_backend *be, int fmt, const void *x, int64_t x_pitch,
     return words ? run_tiles<kFmtF8, kFmtWords>(be, a) : run_tiles<kFmtF8, kFmtF8>(be, a);
 }
 
-bool fits_narrow_tiles(int fmt, const void *x, int64_t x_pitch, int64_t rows, const void *w, int64_t w_pitch, int64_t n, int64_t k) {
-    const int64_t eb = (int64_t)fmt_bytes(fmt);
-    auto side = [&](const void *p, int64_t pitch, int64_t r) {
-        return r > 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0 && pitch >= 0 && pitch * eb % 16 == 0 && r * pitch * eb < (1ll << 32) && r < (1ll << 31);
-    };
-    return fmt != kFmtWords && k > 0 && k * eb % 16 == 0 && k * eb < (1ll << 31) && side(x, x_pitch, rows) && side(w, w_pitch, n);
-}
-
 int launch_bf16_tiles(cg_backend *be, const void *x, uint32_t rows, const Weight &w, float *y) {
     if (!takes_bf16_tiles(rows, w)) return kDeclined;
     ProfScope prof(be, CG_K_GEMM_MFMA, 2.0 * (double)rows * w.n * w.k);
     return launch_narrow_tiles(be, kFmtBF16, x, w.k, rows, w.p, w.pitch, w.n, w.k, y, kFmtWords);
 }
 
-bool takes_bf16_tiles(uint32_t rows, const Weight &w) { return w.fmt == kFmtBF16 && fits_narrow_tiles(kFmtBF16, nullptr, w.k, rows, w.p, w.pitch, w.n, w.k); }
+bool takes_bf16_tiles(uint32_t rows, const Weight &w) {
+    return w.fmt == kFmtBF16 && reinterpret_cast<uintptr_t>(w.p) % 16 == 0 && fits_narrow_tiles(kFmtBF16, w.k, rows, w.pitch, w.n, w.k);
+}
 
 } // namespace cg

@@ -3,6 +3,7 @@
 
 #include "common.hpp"
 #include "device_utils.hpp"
+#include "narrow_route.hpp"
 
 namespace cg {
 
@@ -40,8 +41,7 @@ int launch_split_gemm(cg_backend *be, MmArgs a, bool a_mfast, bool b_nfast);
 
 
 // y[rows, n] = x[rows, k] . w[n, k]^T of patterns of one narrow format (block_products.hip); pitches in elements; y dense, words or
-// patterns of that format.  kDeclined: operands that fits_narrow_tiles does not take (addresses may be null there).
+// patterns of that format.  kDeclined: operands that fits_narrow_tiles does not take or that are not 16-byte aligned.
 int launch_narrow_tiles(cg_backend *be, int fmt, const void *x, int64_t x_pitch, int64_t rows, const void *w, int64_t w_pitch, int64_t n, int64_t k, void *y, int y_fmt);
-bool fits_narrow_tiles(int fmt, const void *x, int64_t x_pitch, int64_t rows, const void *w, int64_t w_pitch, int64_t n, int64_t k);
 
 } // namespace cg

@@ -2532,19 +2532,9 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
     // (env CG_GEMM_PACKED=0 switches it off).
     const bool packable = f32 && K != 0 && M > 8 && kind && packed_narrow_ok() && batch == 1 && K % (kind == 3 ? 16 : 8) == 0 && x->buf && y->buf;
     const bool x_lies = packable && native_rows(x, kind, a.a_sm, a.a_sk, K, false), y_lies = packable && native_rows(y, kind, a.b_sn, a.b_sk, K, false);
-    // on 256 x 256 tiles if there is one for every compute unit, else on 128 x 128 tiles, unless words are all there is
-    const bool big_packed = packable && big, low_packed = packable && !big && (x_lies || y_lies);
-
-    // ---- the operands' addresses -------------------------------------------------------------------------------------
-    const bool x_native = (big_packed || low_packed) && x_lies;
-    rc = mm_operand(x, true, x_native, &a);
-    if (rc) return rc;
-    // a decode-time linear layer of a narrow dtype reads its weight matrix at 2 or 1 bytes a weight (see below)
-    const bool skinny_packed = f32 && K != 0 && M <= (half ? 8 : 2) && packed_narrow_ok() && kind && batch == 1 && a.a_sk == 1 && a.a_vec &&
-                               a.a_sm % 4 == 0 && K % 16 == 0 && K >= 256 && N >= 64 && y->buf;
-    const bool y_native = (skinny_packed && native_rows(y, kind, a.b_sn, a.b_sk, K, true)) || ((big_packed || low_packed) && y_lies);
-    rc = mm_operand(y, false, y_native, &a);
-    if (rc) return rc;
+    const NarrowRoute route = narrow_route(kind, {M, a.a_sm, x_lies}, {N, a.b_sn, y_lies}, K, packable, big, wide_only);
+    const bool big_packed = route == NarrowRoute::wide, low = route == NarrowRoute::low;
+    const bool x_native = (big_packed || low) && x_lies, y_native_rows = (big_packed || low) && y_lies;
     // Whole stages of 64 bytes of k in whole turns of the ring, 16-byte rows, byte offsets that fit 32 bits: the wide tile
     // fed by loads straight into LDS (env CG_GEMM_DLDS=0: the register-staged one).  Only that kernel can round the result
     // to the operands' format in its store; without `out` the call just says whether this product would run on it.
@@ -2554,15 +2544,23 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
     }();
     const int64_t per = kind == 3 ? 4 : 2;           // elements per 32-bit word
     const int64_t kw = kind ? K / per : 0;           // words per row
-    const int64_t a_pitch = x_native ? a.a_sm / per : kw, b_pitch = y_native ? a.b_sn / per : kw; // (a view taken as it lies keeps its own row pitch)
+    const int64_t a_pitch = x_native ? a.a_sm / per : kw, b_pitch = y_native_rows ? a.b_sn / per : kw; // (a view taken as it lies keeps its own row pitch)
     const bool dlds = big_packed && dlds_allowed && kw % (16 * kDldsStages) == 0 && a_pitch % 4 == 0 && b_pitch % 4 == 0 &&
-                      (!x_native || reinterpret_cast<uintptr_t>(native_ptr(x)) % 16 == 0) && (!y_native || reinterpret_cast<uintptr_t>(native_ptr(y)) % 16 == 0) &&
+                      (!x_native || reinterpret_cast<uintptr_t>(native_ptr(x)) % 16 == 0) && (!y_native_rows || reinterpret_cast<uintptr_t>(native_ptr(y)) % 16 == 0) &&
                       (uint64_t)M * (uint64_t)a_pitch * 4 < (1ull << 32) && (uint64_t)N * (uint64_t)b_pitch * 4 < (1ull << 32) &&
                       (uint64_t)M * (uint64_t)N < (1ull << 30);
-    const int64_t low_a = low_packed ? (x_native ? a.a_sm : K) : 0, low_b = low_packed ? (y_native ? a.b_sn : K) : 0; // row pitches in elements
-    const bool low = low_packed && !wide_only && fits_narrow_tiles(kind, nullptr, low_a, M, nullptr, low_b, N, K);
     const bool can_round = (dlds && N % 4 == 0) || low;
     if (!out) return can_round ? CG_OK : kDeclined;
+
+    // ---- the operands' addresses -------------------------------------------------------------------------------------
+    rc = mm_operand(x, true, x_native, &a);
+    if (rc) return rc;
+    // a decode-time linear layer of a narrow dtype reads its weight matrix at 2 or 1 bytes a weight (see below)
+    const bool skinny_packed = f32 && K != 0 && M <= (half ? 8 : 2) && packed_narrow_ok() && kind && batch == 1 && a.a_sk == 1 && a.a_vec &&
+                               a.a_sm % 4 == 0 && K % 16 == 0 && K >= 256 && N >= 64 && y->buf;
+    const bool y_native = (skinny_packed && native_rows(y, kind, a.b_sn, a.b_sk, K, true)) || y_native_rows;
+    rc = mm_operand(y, false, y_native, &a);
+    if (rc) return rc;
     const int c_fmt = out->buf->fmt;
     if (c_fmt != kFmtWords && !can_round) return fail(CG_ERR_ARG, "matmul: a narrow result needs the kernel that rounds in its store");
     const double flop = 2.0 * (double)M * (double)N * (double)K * (double)batch;
@@ -2620,7 +2618,7 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
         size_t ca = 0, cb = 0;
         int prc = x_native ? CG_OK : pack_operand(be, words_buffer(x), a.A, a.a_sm, a.a_sk, M, K, kind, x->rc.load() > 1 || x->buf->rc.load() > 1, &pa, &ta, &ca);
         if (!prc && !y_native) prc = pack_operand(be, words_buffer(y), a.B, a.b_sn, a.b_sk, N, K, kind, true, &pb, &tb, &cb);
-        if (!prc) prc = launch_narrow_tiles(be, kind, pa, low_a, M, pb, low_b, N, K, out->buf->ptr, c_fmt);
+        if (!prc) prc = launch_narrow_tiles(be, kind, pa, x_native ? a.a_sm : K, M, pb, y_native ? a.b_sn : K, N, K, out->buf->ptr, c_fmt);
         if (ta) be->pool.free(ta, ca); // stream-ordered: later users queue behind the product
         if (tb) be->pool.free(tb, cb);
         return prc;
