@@ -2502,6 +2502,29 @@ __global__ __launch_bounds__(kThreads) void skinny_kt_packed_kernel(const MmArgs
     }
 }
 
+// x . y -> out on the 128-wide tiles, an operand that does not lie narrow packed first.  kDeclined: the pool has no room for that.
+static int low_product(cg_backend *be, int kind, const cg_tensor *x, bool x_lies, const cg_tensor *y, bool y_lies, MmArgs a, int64_t M, int64_t N, int64_t K,
+                       cg_tensor *out) {
+    int rc = mm_operand(x, true, x_lies, &a);
+    if (!rc) rc = mm_operand(y, false, y_lies, &a);
+    if (rc) return rc;
+    const void *pa = x_lies ? native_ptr(x) : nullptr, *pb = y_lies ? native_ptr(y) : nullptr;
+    void *ta = nullptr, *tb = nullptr;
+    size_t ca = 0, cb = 0;
+    rc = x_lies ? CG_OK : pack_operand(be, words_buffer(x), a.A, a.a_sm, a.a_sk, M, K, kind, x->rc.load() > 1 || x->buf->rc.load() > 1, &pa, &ta, &ca);
+    if (!rc && !y_lies) rc = pack_operand(be, words_buffer(y), a.B, a.b_sn, a.b_sk, N, K, kind, true, &pb, &tb, &cb);
+    if (rc) {
+        (void)hipGetLastError();
+        rc = kDeclined;
+    } else {
+        ProfScope prof(be, CG_K_GEMM_MFMA, 2.0 * (double)M * (double)N * (double)K);
+        rc = launch_narrow_tiles(be, kind, pa, x_lies ? a.a_sm : K, M, pb, y_lies ? a.b_sn : K, N, K, out->buf->ptr, out->buf->fmt);
+    }
+    if (ta) be->pool.free(ta, ca); // stream-ordered: later users queue behind the product
+    if (tb) be->pool.free(tb, cb);
+    return rc;
+}
+
 int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_tensor *out, bool wide_only) {
     if (int frc = flush_deferred(be)) return frc;
     MmArgs a;
@@ -2534,7 +2557,7 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
     const bool x_lies = packable && native_rows(x, kind, a.a_sm, a.a_sk, K, false), y_lies = packable && native_rows(y, kind, a.b_sn, a.b_sk, K, false);
     const NarrowRoute route = narrow_route(kind, {M, a.a_sm, x_lies}, {N, a.b_sn, y_lies}, K, packable, big, wide_only);
     const bool big_packed = route == NarrowRoute::wide, low = route == NarrowRoute::low;
-    const bool x_native = (big_packed || low) && x_lies, y_native_rows = (big_packed || low) && y_lies;
+    bool x_native = (big_packed || low) && x_lies, y_native_rows = (big_packed || low) && y_lies;
     // Whole stages of 64 bytes of k in whole turns of the ring, 16-byte rows, byte offsets that fit 32 bits: the wide tile
     // fed by loads straight into LDS (env CG_GEMM_DLDS=0: the register-staged one).  Only that kernel can round the result
     // to the operands' format in its store; without `out` the call just says whether this product would run on it.
@@ -2553,6 +2576,12 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
     if (!out) return can_round ? CG_OK : kDeclined;
 
     // ---- the operands' addresses -------------------------------------------------------------------------------------
+    if (low) {
+        rc = low_product(be, kind, x, x_native, y, y_native_rows, a, M, N, K, out);
+        if (rc != kDeclined) return rc;
+        x_native = y_native_rows = false; // no room to pack an operand: from words, as they lie or widened
+        if (out->buf->fmt != kFmtWords) return kDeclined;
+    }
     rc = mm_operand(x, true, x_native, &a);
     if (rc) return rc;
     // a decode-time linear layer of a narrow dtype reads its weight matrix at 2 or 1 bytes a weight (see below)
@@ -2612,16 +2641,6 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
         else { CG_PACKED(8) }
 #undef CG_PACKED
         if (tb) be->pool.free(tb, cb); // stream-ordered: later users queue behind the product
-    } else if (low) {
-        const void *pa = x_native ? native_ptr(x) : nullptr, *pb = y_native ? native_ptr(y) : nullptr;
-        void *ta = nullptr, *tb = nullptr;
-        size_t ca = 0, cb = 0;
-        int prc = x_native ? CG_OK : pack_operand(be, words_buffer(x), a.A, a.a_sm, a.a_sk, M, K, kind, x->rc.load() > 1 || x->buf->rc.load() > 1, &pa, &ta, &ca);
-        if (!prc && !y_native) prc = pack_operand(be, words_buffer(y), a.B, a.b_sn, a.b_sk, N, K, kind, true, &pb, &tb, &cb);
-        if (!prc) prc = launch_narrow_tiles(be, kind, pa, x_native ? a.a_sm : K, M, pb, y_native ? a.b_sn : K, N, K, out->buf->ptr, c_fmt);
-        if (ta) be->pool.free(ta, ca); // stream-ordered: later users queue behind the product
-        if (tb) be->pool.free(tb, cb);
-        return prc;
     } else if (M <= 8 && a.b_sk == 1) {
         const bool vec = a.a_vec && a.b_vec && a.a_sk == 1 && K % 4 == 0;
 #define CG_MM_SWITCH(CALL)        \

@@ -2954,6 +2954,13 @@ static int matmul_entry(cg_backend *b, cg_tensor *x, cg_tensor *y, cg_tensor **o
     if (rc) return rc;
     if (numel(o) > 0) {
         rc = launch_matmul(b, x, y, o);
+        if (rc == kDeclined) { // no room after all to multiply patterns: a result in words, rounded by the caller
+            release(o);
+            fmt = kFmtWords;
+            rc = new_dense(b, x->dt, od, r, &o, 0, fmt);
+            if (rc) return rc;
+            rc = launch_matmul(b, x, y, o);
+        }
         if (rc) {
             release(o);
             return rc;
