@@ -11,7 +11,9 @@
 // The pieces share the 32-bit exponent's range but not infinity's company: a piece may round up to infinity beyond 3.38e38, and
 // infinity times a zero piece is no number.  Values below 2^-126 lose bits of their lower pieces.  While it splits, a
 // workgroup keeps the largest magnitude of every row of both operands, and a tile with a row at either end of the range (or
-// an infinity) is multiplied again on the 32-bit instructions (plain_product).
+// an infinity) is multiplied again on the 32-bit instructions (plain_product).  So is a tile whose products could leave the range:
+// the product of two first pieces may be above that of the values, and the products of the others, which are added first, have
+// signs of their own and meet infinity alone.
 #pragma once
 
 #include "common.hpp"
@@ -62,6 +64,17 @@ __device__ __forceinline__ void grow(float &m, float x, float y) { // m = max(m,
 }
 // A row whose largest magnitude is m cannot be multiplied in pieces at full precision.
 __device__ __forceinline__ bool out_of_range(float m) { return m > 3.0e38f || (m > 0.0f && m < 8.0e-28f); }
+// Operands of magnitudes up to a and b: any number of products of their pieces adds up to less than 2^127.
+__device__ __forceinline__ bool in_range(float a, float b) { return a * b < 0x1p95f; }
+// the largest of a wave's values, none of them negative
+template <int CTRL> __device__ __forceinline__ float with_lane(float m) {
+    return fmaxf(m, asf((uint32_t)__builtin_amdgcn_update_dpp(0, (int)asu(m), CTRL, 0xF, 0xF, false)));
+}
+__device__ __forceinline__ float wave_max(float m) {
+    m = with_lane<0x118>(with_lane<0x114>(with_lane<0x112>(with_lane<0x111>(m)))); // a row's 16 lanes: its last one has the largest
+    m = with_lane<0x143>(with_lane<0x142>(m));                                       // the last lanes of rows to the rows behind
+    return asf((uint32_t)__builtin_amdgcn_readlane((int)asu(m), 63));
+}
 
 // One operand's way into LDS: R rows, its share of a stage in registers, its pieces in fragment order.
 //
@@ -172,6 +185,12 @@ template <int R, bool ROWS_FAST, int THREADS> struct Feed {
             b |= out_of_range(m);
         }
         return b;
+    }
+    __device__ __forceinline__ float most() {
+        float m = top[0];
+#pragma unroll
+        for (int u = 1; u < UNITS; u++) m = fmaxf(m, top[u]);
+        return wave_max(m);
     }
 };
 
@@ -375,16 +394,16 @@ __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const
         }
     }
 
-    __attribute__((address_space(3))) uint32_t *const flags = reinterpret_cast<__attribute__((address_space(3))) uint32_t *>(lds + 2 * STAGE);
+    __attribute__((address_space(3))) float2v *const tops = reinterpret_cast<__attribute__((address_space(3))) float2v *>(lds + 2 * STAGE);
     const bool bad_a = fa.bad(), bad_b = fb.bad(); // (both: every lane takes part in the exchanges)
     const bool some = __builtin_amdgcn_ballot_w64(bad_a || bad_b) != 0;
-    if (lane == 0) flags[wave] = some;
+    const float2v top = {some ? INFINITY : fa.most(), fb.most()};
+    if (lane == 0) tops[wave] = top;
     meet();
-    uint32_t any = 0;
+    float2v most = tops[0];
 #pragma unroll
-    for (int w = 0; w < WM * WN; w++) any |= flags[w];
-    if (any)
-        plain_product<MT, NT, AF, BF>(acc, oa, row_a, last_a, ob, row_b, last_b, K, bma * 32, bnb * 32);
+    for (int w = 1; w < WM * WN; w++) most = {fmaxf(most[0], tops[w][0]), fmaxf(most[1], tops[w][1])};
+    if (most[0] == INFINITY || !in_range(most[0], most[1])) plain_product<MT, NT, AF, BF>(acc, oa, row_a, last_a, ob, row_b, last_b, K, bma * 32, bnb * 32);
 }
 
 } // namespace split

@@ -73,3 +73,54 @@ def test_ends_of_the_range(hip, M, side):
                                       hip.transpose(hip.from_numpy(a), 1, 2)))[0].T
     assert np.array_equal(np.isnan(got), np.isnan(want))
     np.testing.assert_array_equal(got[~np.isnan(want)], want[~np.isnan(want)])
+
+
+# by layout: the 256 x 256 tile in all four; 64 x 64, 64 x 128 and 128 x 128; 32 x 256; the same cut along k; any alignment
+TILES = [(2048, 64, 8192), (72, 64, 2048), (32, 64, 8192), (32, 2048, 8192), (200, 512, 256), (130, 63, 130)]
+
+
+def check_chosen(be, size, layout, rows, scales):
+    """Every column of the right operand holds one value (a power of two): every result is one product, exact or out of range."""
+    M, K, N = size
+    rng = np.random.default_rng(M + K + N)
+    a, b = rng.standard_normal((M, K), dtype=np.float32), np.zeros((K, N), dtype=np.float32)
+    at, s = rng.integers(0, K, N), rng.choice(np.float32(scales), N)
+    b[at, np.arange(N)] = s
+    for r, make in rows.items():
+        a[r] = make(rng, K)
+    with np.errstate(all="ignore"):
+        want = a[:, at].astype(np.float64) * s
+        want = want.astype(np.float32)
+        others = np.isfinite(a).sum(1)[:, None] - np.isfinite(a[:, at]) < K - 1   # infinity (or NaN) times zero among the terms
+        want[others] = np.nan
+    x = be.transpose(be.from_numpy(np.ascontiguousarray(a.T)), 0, 1) if layout[0] == "t" else be.from_numpy(a)
+    y = be.from_numpy(b) if layout[1] == "n" else be.transpose(be.from_numpy(np.ascontiguousarray(b.T)), 0, 1)
+    got = be.to_numpy(be.matmul(x, y))
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(got[~np.isnan(want)], want[~np.isnan(want)])
+
+
+def one(value):
+    def make(rng, K):
+        r = rng.standard_normal(K, dtype=np.float32)
+        r[K // 3] = value
+        return r
+    return make
+
+
+@pytest.mark.parametrize("size", TILES, ids=str)
+@pytest.mark.parametrize("layout", ["nt", "nn", "tt", "tn"])
+def test_rows_at_the_ends_of_the_range(hip, size, layout):
+    last = size[0] - 1
+    check_chosen(hip, size, layout, {
+        last: lambda rng, K: np.float32(3.4028235e38) * rng.choice(np.float32([1, -1]), K), 5: lambda rng, K: rng.standard_normal(K, dtype=np.float32) * np.float32(1e-34),
+        last // 2: one(np.inf), last // 3: one(np.nan), last - 3: one(-np.inf)}, [1.0, -0.5, 2.0 ** -10])
+
+
+@pytest.mark.parametrize("size", TILES, ids=str)
+@pytest.mark.parametrize("layout", ["nt", "nn", "tt", "tn"])
+def test_products_beyond_the_range(hip, size, layout):
+    """Finite values whose products are infinite have the product's sign, whatever the pieces' are."""
+    last = size[0] - 1
+    signs = lambda rng, K: np.float32(1.01e22) * rng.choice(np.float32([1, -1]), K)    # noqa: E731  (a second piece of the other sign)
+    check_chosen(hip, size, layout, {last: signs, 3: signs, last // 2: one(-1.1e38)}, [1.0, 2.0 ** 70, -2.0 ** 70])
