@@ -2,12 +2,14 @@
 //
 // A 32-bit float is the exact sum of three bfloat16 numbers (24 bits of significand = 3 x 8, each piece the nearest to what
 // the ones before leave over), and products of bfloat16 numbers are exact in the matrix unit's 32-bit sums.  Of the nine
-// piece products of x y the three of weight 2^-24 and below are left out; what the other six add up to is off by less than the
-// rounding of one 32-bit multiplication (x y (1 + d), |d| <= 2^-23.4, and 2^-26 in the root mean square), and a chain over k
-// rounds once per 16 values of k and piece instead of once per value.  Measured against 64 bits on 2048 values of k drawn from
-// N(0, 1): relative error 7.0e-7 against 8.1e-7 of v_mfma_f32_32x32x2_f32 (8192: 1.5e-6 against 1.6e-6; all positive:
-// 4.3e-7 against 6.5e-7).  Six instructions of 32 cycles for 16 values of k against eight of 64: 2.67 times the peak rate.
+// piece products of x y the three of weight 2^-25 and below are left out: together at most 2^-24.0 of |x y|, which is the
+// largest rounding of one 32-bit multiplication, and 2^-27.5 in the root mean square, a fifth of that rounding's.
 //
+// The matrix instruction cuts what it adds off towards minus infinity below its sum's last bits, so a chain of them over all of k
+// moves every output, of either sign, to the same side (by 8e-8 of their root mean square at 2048 values of k), which does not
+// average out over a model's rows and layers as roundings do.  The six piece products of 16 values of k are therefore a chain of
+// their own that starts from zero, of the negated left operand for every other 16, and a vector instruction adds its sum to the
+// total or takes it away: one rounding to nearest per 16 values of k, where the 32-bit matrix instructions round 8 times.
 // The pieces share the 32-bit exponent's range but not infinity's company: a piece may round up to infinity beyond 3.38e38, and
 // infinity times a zero piece is no number.  Values below 2^-126 lose bits of their lower pieces.  While it splits, a
 // workgroup keeps the largest magnitude of every row of both operands, and a tile with a row at either end of the range (or
@@ -40,8 +42,8 @@ struct TileSide {
     int64_t s_k;
 };
 
-// the six piece products, small ones first
-constexpr int kPairA[6] = {0, 2, 1, 0, 1, 0}, kPairB[6] = {2, 0, 1, 1, 0, 0};
+// the six piece products, the largest last, in an order that is done with the left side's small pieces early
+constexpr int kPairA[6] = {2, 1, 1, 0, 0, 0}, kPairB[6] = {0, 1, 0, 2, 1, 0};
 
 constexpr uint32_t lds_bytes(int bm, int bn) { return 2 * (uint32_t)(bm + bn) * kDepth * 6 + 64; }
 
@@ -134,13 +136,13 @@ template <int R, bool ROWS_FAST, int THREADS> struct Feed {
             for (int i = 0; i < 4; i++) r[set][h][i] = k < K ? r[set][h][i] : 0.0f;
         }
     }
-    // splits unit u of a set into the stage at `lds`
-    __device__ __forceinline__ void store(lds_char *lds, int set, int u) {
+    // splits unit u of a set, times `up`, into the stage at `lds`
+    __device__ __forceinline__ void store(lds_char *lds, int set, int u, float up) {
         if constexpr (!ROWS_FAST) {
             const float4v v = r[set][u];
             uint32_t a[3], b[3];
-            split2(v[0], v[1], a);
-            split2(v[2], v[3], b);
+            split2(v[0] * up, v[1] * up, a);
+            split2(v[2] * up, v[3] * up, b);
             grow(top[u], v[0], v[1]);
             grow(top[u], v[2], v[3]);
             if (R >= STEP || threadIdx.x < R * 4) {
@@ -154,7 +156,7 @@ template <int R, bool ROWS_FAST, int THREADS> struct Feed {
             uint32_t w[KQ / 2][3];
 #pragma unroll
             for (int t = 0; t < KQ / 2; t++) {
-                split2(r[set][2 * t][u], r[set][2 * t + 1][u], w[t]);
+                split2(r[set][2 * t][u] * up, r[set][2 * t + 1][u] * up, w[t]);
                 grow(top[u], r[set][2 * t][u], r[set][2 * t + 1][u]);
             }
 #pragma unroll
@@ -194,28 +196,55 @@ template <int R, bool ROWS_FAST, int THREADS> struct Feed {
     }
 };
 
-// The 32-bit instructions on operands straight from memory: what is left for tiles that pieces do not cover.
+// The 32-bit instructions on operands straight from memory: what is left for tiles that pieces do not cover.  A row of blocks after
+// the other; eight values of k at a time, four of them per lane group, asked for while the eight before them multiply.
 template <int MT, int NT, bool AF, bool BF, class RowA, class RowB>
 __device__ __forceinline__ void plain_product(float16v (&acc)[MT][NT], const TileSide &a, RowA row_a, uint32_t last_a, const TileSide &b, RowB row_b,
                                            uint32_t last_b, uint32_t K, uint32_t wm, uint32_t wn) {
-    const uint32_t li = threadIdx.x % 32, lg = threadIdx.x % 64 / 32;
+    typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+    const uint32_t li = threadIdx.x % 32, lg = threadIdx.x % 64 / 32, eights = K / 8;
+    auto four = [&](const uint32_t *p, const int64_t s_k, const bool fast, const uint32_t k) {
+        if (!fast && s_k == 1) return (float4v)*reinterpret_cast<const float4u *>(p + k);
+        float4v v;
 #pragma unroll
-    for (int i = 0; i < MT; i++)
+        for (int t = 0; t < 4; t++) v[t] = asf(p[(int64_t)(k + t) * s_k]);
+        return v;
+    };
+    const uint32_t *pb[NT];
 #pragma unroll
-        for (int j = 0; j < NT; j++)
+    for (int j = 0; j < NT; j++) pb[j] = b.p + row_b(min(wn + j * 32 + li, last_b));
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.0f;
-    for (uint32_t k = 0; k < K; k += 2) {
-        const uint32_t kk = k + lg;
-        float fa[MT], fb[NT];
+    for (int i = 0; i < MT; i++) {
+        const uint32_t *const pa = a.p + row_a(min(wm + i * 32 + li, last_a));
 #pragma unroll
-        for (int i = 0; i < MT; i++) fa[i] = kk < K ? asf(a.p[(int64_t)kk * a.s_k + row_a(min(wm + i * 32 + li, last_a))]) : 0.0f;
+        for (int j = 0; j < NT; j++) acc[i][j] = (float16v){};
+        float4v fa, fb[NT];
+        auto ask = [&](const uint32_t k) {
+            fa = four(pa, a.s_k, AF, k + lg * 4);
 #pragma unroll
-        for (int j = 0; j < NT; j++) fb[j] = kk < K ? asf(b.p[(int64_t)kk * b.s_k + row_b(min(wn + j * 32 + li, last_b))]) : 0.0f;
+            for (int j = 0; j < NT; j++) fb[j] = four(pb[j], b.s_k, BF, k + lg * 4);
+        };
+        if (eights) ask(0);
+        for (uint32_t c = 0; c < eights; c++) {
+            const float4v ga = fa;
+            float4v gb[NT];
 #pragma unroll
-        for (int i = 0; i < MT; i++)
+            for (int j = 0; j < NT; j++) gb[j] = fb[j];
+            ask(min(c + 1, eights - 1) * 8);
 #pragma unroll
-            for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i], fb[j], acc[i][j], 0, 0, 0);
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(ga[t], gb[j][t], acc[i][j], 0, 0, 0);
+        }
+        for (uint32_t k = eights * 8; k < K; k += 2) {
+            const uint32_t kk = k + lg, at = min(kk, K - 1);
+            const float x = asf(pa[(int64_t)at * a.s_k]);
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                const float y = asf(pb[j][(int64_t)at * b.s_k]);
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(kk < K ? x : 0.0f, kk < K ? y : 0.0f, acc[i][j], 0, 0, 0);
+            }
+        }
     }
 }
 
@@ -224,9 +253,12 @@ __device__ __forceinline__ void plain_product(float16v (&acc)[MT][NT], const Til
 // the last one.
 //
 // A stage is 16 values of k.  While a stage is multiplied, the next one goes from registers through split2 into the other half of
-// LDS and the one after it (two where a tile is small: LEAD) is asked for, a unit at a time between groups of NT matrix
-// instructions; the fragments of a row of blocks are read while the row before it multiplies.  The barrier stands before the
-// stage's last row: everybody has read the stage and written the next by then, whose fragments are read under that row.
+// LDS and the one after it (two where a tile is small: LEAD) is asked for, a unit at a time between the matrix instructions; the
+// fragments of a row of blocks are read while the row before it multiplies.  A block's chain of six is added to its total while the
+// next block's chain runs (SETS: the registers for that; the wide tile has none and waits, which its other wave on the SIMD
+// fills).  The barrier stands before the stage's last row: everybody has read the stage and written the next by then, whose
+// fragments are read under that row.
+// Up to four values of k are multiplied by the 32-bit instructions alone, which lose less of so short a sum.
 template <int WM, int WN, int MT, int NT, bool AF, bool BF, bool CARE, class RowA, class RowB>
 __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const lds, const TileSide &oa, RowA row_a, const uint32_t last_a, const TileSide &ob,
                                         RowB row_b, const uint32_t last_b, const uint32_t K) {
@@ -234,6 +266,10 @@ __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const
     typedef Feed<BM, AF, 64 * WM * WN> FA;
     typedef Feed<BN, BF, 64 * WM * WN> FB;
     constexpr int LEAD = FA::SLOTS + FB::SLOTS > 4 ? 1 : 2;
+    constexpr bool WIDE = MT * NT >= 8;
+    constexpr int TOGETHER = WIDE ? 1 : NT;                            // blocks of a row whose chains run side by side
+    constexpr int GROUPS = MT * NT / TOGETHER, SETS = WIDE ? 1 : 2;    // of such chains in a stage; of their sums in registers
+    constexpr bool CARRY = GROUPS == 1;                                // a stage's sums are added in the next stage
     constexpr uint32_t STAGE = 3 * (FA::PIECE + FB::PIECE);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, li = lane % 32, lg = lane / 32;
     const uint32_t bma = wave / WN * MT, bnb = wave % WN * NT; // this wave's first block of rows and of columns
@@ -243,7 +279,7 @@ __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const
     FB fb;
     fa.start(oa, row_a, last_a);
     fb.start(ob, row_b, last_b);
-    const uint32_t nk = CARE ? (K + kDepth - 1) / kDepth : K / kDepth; // stages of the loop (CARE: with the last, ragged one)
+    const uint32_t nk = K <= 4 ? 0 : CARE ? (K + kDepth - 1) / kDepth : K / kDepth; // stages of the loop (CARE: with the last, ragged one)
     // (behind the last stage the last one is asked for again: one way through the loop, and values that nobody multiplies)
     auto ask_a = [&](uint32_t s, int set, int h) {
         if constexpr (CARE) fa.load_careful(oa, row_a, last_a, K, s, set, h);
@@ -253,81 +289,93 @@ __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const
         if constexpr (CARE) fb.load_careful(ob, row_b, last_b, K, s, set, h);
         else fb.load(ob, min(s, nk - 1), set, h);
     };
+    const float16v zero = {};
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int j = 0; j < NT; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.0f;
+        for (int j = 0; j < NT; j++) acc[i][j] = zero;
     auto meet = [&]() {
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0)
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
-    constexpr int AS = MT > 1 ? 2 : 1;
+    constexpr int AS = MT > 1 && !WIDE ? 2 : 1; // (the wide tile reads the left side's next fragments under a row's last chain)
     bf16x8 a[AS][3], b[NT][3];
     auto read = [&](lds_char *p) { return __builtin_bit_cast(bf16x8, *reinterpret_cast<__attribute__((address_space(3))) float4v *>(p)); };
     auto read_a = [&](const int par, const int i, const int p) { a[i % AS][p] = read(fa_base + par * STAGE + p * FA::PIECE + i * 1024); };
     auto read_b = [&](const int par, const int j, const int p) { b[j][p] = read(fb_base + par * STAGE + p * FB::PIECE + j * 1024); };
-    // One stage (PAR: its half of LDS): the small products first.
+    float16v sum[SETS][TOGETHER]; // chains of six
+    if (CARRY)
+        for (int t = 0; t < TOGETHER; t++) sum[SETS - 1][t] = zero;
+    auto add = [&](const int group, const int set, const float down) {
+#pragma unroll
+        for (int t = 0; t < TOGETHER; t++) {
+            float16v &to = acc[group * TOGETHER / NT][group * TOGETHER % NT + t];
+#pragma unroll
+            for (int v = 0; v < 16; v++) to[v] = __builtin_fmaf(sum[set][t][v], down, to[v]);
+        }
+    };
+    // One stage (PAR: its half of LDS, 1: its left operand is negated)
     auto stage = [&](const uint32_t s, auto par_) {
         constexpr int PAR = decltype(par_)::value;
         constexpr int SET = LEAD == 2 ? (PAR + 1) % 2 : 0; // registers of stage s + 1, to be filled with stage s + 1 + LEAD
-        constexpr int UNITS = FA::UNITS + FB::UNITS, GROUPS = MT > 1 ? (MT - 1) * 6 : 6;
+        constexpr int UNITS = FA::UNITS + FB::UNITS, SLOTS = (MT > 1 ? MT - 1 : 1) * NT / TOGETHER * 6; // places between the matrix instructions before the barrier
+        constexpr float down = PAR ? -1.0f : 1.0f;
         lds_char *const to = lds + (PAR ^ 1) * STAGE;
         auto unit = [&](const int u) {
             if (u < FA::UNITS) {
-                fa.store(to, SET, u);
+                fa.store(to, SET, u, PAR ? 1.0f : -1.0f);
                 if (!AF) ask_a(s + 1 + LEAD, SET, u);
                 else if (u == 3)
                     for (int h = 0; h < FA::SLOTS; h++) ask_a(s + 1 + LEAD, SET, h);
             } else {
                 const int v = u - FA::UNITS;
-                fb.store(to + 3 * FA::PIECE, SET, v);
+                fb.store(to + 3 * FA::PIECE, SET, v, 1.0f);
                 if (!BF) ask_b(s + 1 + LEAD, SET, v);
                 else if (v == 3)
                     for (int h = 0; h < FB::SLOTS; h++) ask_b(s + 1 + LEAD, SET, h);
             }
         };
 #pragma unroll
-        for (int i = 0; i < MT; i++) {
-            if (MT > 1 && i == MT - 1) meet();
+        for (int group = 0; group < GROUPS; group++) {
+            const int i = group * TOGETHER / NT, j0 = group * TOGETHER % NT, set = (PAR * GROUPS + group) % SETS, before = (set + 1) % SETS;
+            if (MT > 1 && i == MT - 1 && j0 == 0) meet();
 #pragma unroll
             for (int g = 0; g < 6; g++) {
 #pragma unroll
-                for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i % AS][kPairA[g]], b[j][kPairB[g]], acc[i][j], 0, 0, 0);
-                const int group = i * 6 + g;
-                if (group < GROUPS) {
+                for (int t = 0; t < TOGETHER; t++)
+                    sum[set][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i % AS][kPairA[g]], b[j0 + t][kPairB[g]], g ? sum[set][t] : zero, 0, 0, 0);
+                if (SETS == 2 && g == 4 && (group || CARRY)) add(group ? group - 1 : GROUPS - 1, before, group ? down : -down);
+                const int slot = group * 6 + g;
+                if (slot < SLOTS) {
 #pragma unroll
                     for (int u = 0; u < UNITS; u++)
-                        if (u * GROUPS / UNITS == group) unit(u);
+                        if (u * SLOTS / UNITS == slot) unit(u);
                 }
                 if (MT > 1) {
-                    if (g < 3) {
-                        if (i + 1 < MT) read_a(PAR, i + 1, kPairA[g]);
-                        else read_a(PAR ^ 1, 0, kPairA[g]);
-                    }
-                    if (i == MT - 1) {
-                        const int gone = g == 0 ? 2 : g == 3 ? 1 : g == 5 ? 0 : -1; // the piece of B that was used for the last time
-                        if (gone >= 0) {
+                    const int next = (i + 1) % MT, par = i + 1 < MT ? PAR : PAR ^ 1;
+                    if (WIDE ? j0 + TOGETHER == NT && (g == 0 || g == 2 || g == 5) : j0 == 0 && g < 3) read_a(par, next, WIDE ? kPairA[g] : g);
+                    if (i == MT - 1 && g >= 3) { // (used for the last time)
 #pragma unroll
-                            for (int j = 0; j < NT; j++) read_b(PAR ^ 1, j, gone);
-                        }
+                        for (int t = 0; t < TOGETHER; t++) read_b(PAR ^ 1, j0 + t, kPairB[g]);
                     }
                 }
-                if constexpr (!CARE) {
-#pragma unroll
-                    for (int j = 0; j < NT; j++) { // what goes along, between the matrix instructions
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x002, 24 / NT + 1, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
+                if (MT * NT < 4) __builtin_amdgcn_sched_barrier(0); // (or all of a unit's work would stand behind the chain)
             }
+            if (WIDE) add(group, 0, down);
+            if constexpr (!CARE && MT * NT >= 4) {
+#pragma unroll
+                for (int g = 0; g < 6 * TOGETHER; g++) { // what goes along, between the matrix instructions
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, WIDE ? 6 : 8, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
+        if (SETS == 2 && !CARRY) add(GROUPS - 1, (PAR * GROUPS + GROUPS - 1) % SETS, down);
         if (MT == 1) {
             meet();
 #pragma unroll
@@ -348,9 +396,9 @@ __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const
             for (int h = 0; h < FB::SLOTS; h++) ask_b(1, 1, h);
         }
 #pragma unroll
-        for (int u = 0; u < FA::UNITS; u++) fa.store(lds, 0, u);
+        for (int u = 0; u < FA::UNITS; u++) fa.store(lds, 0, u, 1.0f);
 #pragma unroll
-        for (int u = 0; u < FB::UNITS; u++) fb.store(lds + 3 * FA::PIECE, 0, u);
+        for (int u = 0; u < FB::UNITS; u++) fb.store(lds + 3 * FA::PIECE, 0, u, 1.0f);
         for (int h = 0; h < FA::SLOTS; h++) ask_a(LEAD, 0, h);
         for (int h = 0; h < FB::SLOTS; h++) ask_b(LEAD, 0, h);
 
@@ -363,21 +411,27 @@ __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const
             for (int j = 0; j < NT; j++) read_b(0, j, p);
         for (uint32_t s = 0;; s += 2) {
             stage(s, P0{});
-            if (s + 1 >= nk) break;
+            if (s + 1 >= nk) {
+                if (CARRY) add(0, 0, 1.0f);
+                break;
+            }
             stage(s + 1, P1{});
-            if (s + 2 >= nk) break;
+            if (s + 2 >= nk) {
+                if (CARRY) add(0, SETS - 1, -1.0f);
+                break;
+            }
         }
     }
-    if (MT * NT < 8 && !CARE && K % kDepth) { // what is left of k, a stage by itself (the wide tile has no registers for it)
+    if (MT * NT < 8 && !CARE && K > 4 && K % kDepth) { // what is left of k, a stage by itself (the wide tile has no registers for it)
 #pragma unroll
         for (int h = 0; h < FA::SLOTS; h++) fa.load_careful(oa, row_a, last_a, K, nk, 0, h);
 #pragma unroll
         for (int h = 0; h < FB::SLOTS; h++) fb.load_careful(ob, row_b, last_b, K, nk, 0, h);
         meet(); // (nobody reads the half that is written now)
 #pragma unroll
-        for (int u = 0; u < FA::UNITS; u++) fa.store(lds, 0, u);
+        for (int u = 0; u < FA::UNITS; u++) fa.store(lds, 0, u, nk % 2 ? -1.0f : 1.0f);
 #pragma unroll
-        for (int u = 0; u < FB::UNITS; u++) fb.store(lds + 3 * FA::PIECE, 0, u);
+        for (int u = 0; u < FB::UNITS; u++) fb.store(lds + 3 * FA::PIECE, 0, u, 1.0f);
         meet();
 #pragma unroll
         for (int p = 0; p < 3; p++)
@@ -388,22 +442,30 @@ __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const
 #pragma unroll
             for (int p = 0; p < 3; p++) read_a(0, i, p);
 #pragma unroll
-            for (int g = 0; g < 6; g++)
+            for (int j = 0; j < NT; j++) {
+                float16v &t = sum[0][j % TOGETHER];
 #pragma unroll
-                for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i % AS][kPairA[g]], b[j][kPairB[g]], acc[i][j], 0, 0, 0);
+                for (int g = 0; g < 6; g++) t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i % AS][kPairA[g]], b[j][kPairB[g]], g ? t : zero, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[i][j][v] = __builtin_fmaf(t[v], nk % 2 ? -1.0f : 1.0f, acc[i][j][v]);
+            }
         }
     }
 
-    __attribute__((address_space(3))) float2v *const tops = reinterpret_cast<__attribute__((address_space(3))) float2v *>(lds + 2 * STAGE);
-    const bool bad_a = fa.bad(), bad_b = fb.bad(); // (both: every lane takes part in the exchanges)
-    const bool some = __builtin_amdgcn_ballot_w64(bad_a || bad_b) != 0;
-    const float2v top = {some ? INFINITY : fa.most(), fb.most()};
-    if (lane == 0) tops[wave] = top;
-    meet();
-    float2v most = tops[0];
+    bool plain = K <= 4;
+    if (!plain) {
+        __attribute__((address_space(3))) float2v *const tops = reinterpret_cast<__attribute__((address_space(3))) float2v *>(lds + 2 * STAGE);
+        const bool bad_a = fa.bad(), bad_b = fb.bad(); // (both: every lane takes part in the exchanges)
+        const bool some = __builtin_amdgcn_ballot_w64(bad_a || bad_b) != 0;
+        const float2v top = {some ? INFINITY : fa.most(), fb.most()};
+        if (lane == 0) tops[wave] = top;
+        meet();
+        float2v most = tops[0];
 #pragma unroll
-    for (int w = 1; w < WM * WN; w++) most = {fmaxf(most[0], tops[w][0]), fmaxf(most[1], tops[w][1])};
-    if (most[0] == INFINITY || !in_range(most[0], most[1])) plain_product<MT, NT, AF, BF>(acc, oa, row_a, last_a, ob, row_b, last_b, K, bma * 32, bnb * 32);
+        for (int w = 1; w < WM * WN; w++) most = {fmaxf(most[0], tops[w][0]), fmaxf(most[1], tops[w][1])};
+        plain = most[0] == INFINITY || !in_range(most[0], most[1]);
+    }
+    if (__builtin_amdgcn_readfirstlane(plain)) plain_product<MT, NT, AF, BF>(acc, oa, row_a, last_a, ob, row_b, last_b, K, bma * 32, bnb * 32);
 }
 
 } // namespace split

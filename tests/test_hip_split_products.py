@@ -124,3 +124,14 @@ def test_products_beyond_the_range(hip, size, layout):
     last = size[0] - 1
     signs = lambda rng, K: np.float32(1.01e22) * rng.choice(np.float32([1, -1]), K)    # noqa: E731  (a second piece of the other sign)
     check_chosen(hip, size, layout, {last: signs, 3: signs, last // 2: one(-1.1e38)}, [1.0, 2.0 ** 70, -2.0 ** 70])
+
+
+@pytest.mark.parametrize("size,layout", [((512, 576, 1536), "nt"), ((512, 576, 1536), "nn"), ((512, 576, 1536), "tt"), ((512, 576, 1536), "tn"), ((1024, 1024, 2048), "nt"),
+                                         ((4096, 256, 4096), "nt"), ((4096, 256, 4096), "tn"), ((1023, 2047, 513), "nt"), ((30, 1024, 8192), "nt")], ids=str)
+def test_roundings_have_no_direction(hip, size, layout):
+    """The error's mean over all results, against their root mean square: a rounding to nearest per 16 values of k has none (over
+    these numbers of results its mean is below 2^-28), sums cut off below have 2^-27 and more."""
+    a, b, x, y = operands(hip, *size, layout[0] == "t", layout[1] == "n", seed=3)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    d = hip.to_numpy(hip.matmul(x, y)) - want
+    assert abs(d.mean()) <= 2.0 ** -28 * np.sqrt((want ** 2).mean()), d.mean() / np.sqrt((want ** 2).mean())
