@@ -10,12 +10,10 @@
 // average out over a model's rows and layers as roundings do.  The six piece products of 16 values of k are therefore a chain of
 // their own that starts from zero, of the negated left operand for every other 16, and a vector instruction adds its sum to the
 // total or takes it away: one rounding to nearest per 16 values of k, where the 32-bit matrix instructions round 8 times.
-// The pieces share the 32-bit exponent's range but not infinity's company: a piece may round up to infinity beyond 3.38e38, and
-// infinity times a zero piece is no number.  Values below 2^-126 lose bits of their lower pieces.  While it splits, a
-// workgroup keeps the largest magnitude of every row of both operands, and a tile with a row at either end of the range (or
-// an infinity) is multiplied again on the 32-bit instructions (plain_product).  So is a tile whose products could leave the range:
-// the product of two first pieces may be above that of the values, and the products of the others, which are added first, have
-// signs of their own and meet infinity alone.
+// Both operands are multiplied by 2^16 on their way into pieces, and the chains' sums by 2^-32 as they are added: then the three
+// pieces of every 32-bit number, the subnormal ones included, are bfloat16 numbers (multiples of 2^-133).  What the pieces do
+// not hold are infinities and products at the upper end of the range: while it splits, a workgroup keeps the largest magnitude of
+// either operand, and a tile whose products could leave the range is multiplied again on the 32-bit instructions (plain_product).
 #pragma once
 
 #include "common.hpp"
@@ -51,6 +49,7 @@ __device__ __forceinline__ uint32_t cvt2(float x, float y) {
     const float2v v = {x, y};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
+constexpr float kUp = 65536.0f, kDown = 1.0f / (65536.0f * 65536.0f); // both operands' scale, and the products' way back
 __device__ __forceinline__ float lo2(uint32_t h) { return asf(h << 16); }
 __device__ __forceinline__ float hi2(uint32_t h) { return asf(h & 0xFFFF0000u); }
 // Two values' three pieces, two to a word.
@@ -66,8 +65,8 @@ __device__ __forceinline__ void grow(float &m, float x, float y) { // m = max(m,
 }
 // A row whose largest magnitude is m cannot be multiplied in pieces at full precision.
 __device__ __forceinline__ bool out_of_range(float m) { return m > 3.0e38f || (m > 0.0f && m < 8.0e-28f); }
-// Operands of magnitudes up to a and b: any number of products of their pieces adds up to less than 2^127.
-__device__ __forceinline__ bool in_range(float a, float b) { return a * b < 0x1p95f; }
+// Operands of magnitudes up to a and b: 16 products of scaled pieces stay below 2^127.
+__device__ __forceinline__ bool in_range(float a, float b) { return a < 0x1p110f && b < 0x1p110f && a * b < 0x1p90f; }
 // the largest of a wave's values, none of them negative
 template <int CTRL> __device__ __forceinline__ float with_lane(float m) {
     return fmaxf(m, asf((uint32_t)__builtin_amdgcn_update_dpp(0, (int)asu(m), CTRL, 0xF, 0xF, false)));
@@ -94,13 +93,12 @@ template <int R, bool ROWS_FAST, int THREADS> struct Feed {
     static_assert(!ROWS_FAST || KQ == 2 || KQ == 4, "a thread's share of a stage");
     uint32_t off[SLOTS]; // byte offsets of the 16-byte loads from the stage's first value
     uint32_t at;         // where this thread's pieces go
-    float top[UNITS];    // largest magnitude per row seen
+    float top;           // largest magnitude seen
     float4v r[2][SLOTS];
 
     template <class Row> __device__ __forceinline__ void start(const TileSide &o, Row row, uint32_t last) {
         const uint32_t t = threadIdx.x;
-#pragma unroll
-        for (int u = 0; u < UNITS; u++) top[u] = 0.0f;
+        top = 0.0f;
         if constexpr (!ROWS_FAST) {
             const uint32_t q = t % 4, l = t / 4;
 #pragma unroll
@@ -143,8 +141,8 @@ template <int R, bool ROWS_FAST, int THREADS> struct Feed {
             uint32_t a[3], b[3];
             split2(v[0] * up, v[1] * up, a);
             split2(v[2] * up, v[3] * up, b);
-            grow(top[u], v[0], v[1]);
-            grow(top[u], v[2], v[3]);
+            grow(top, v[0], v[1]);
+            grow(top, v[2], v[3]);
             if (R >= STEP || threadIdx.x < R * 4) {
 #pragma unroll
                 for (int p = 0; p < 3; p++) {
@@ -157,7 +155,7 @@ template <int R, bool ROWS_FAST, int THREADS> struct Feed {
 #pragma unroll
             for (int t = 0; t < KQ / 2; t++) {
                 split2(r[set][2 * t][u] * up, r[set][2 * t + 1][u] * up, w[t]);
-                grow(top[u], r[set][2 * t][u], r[set][2 * t + 1][u]);
+                grow(top, r[set][2 * t][u], r[set][2 * t + 1][u]);
             }
 #pragma unroll
             for (int p = 0; p < 3; p++) {
@@ -169,30 +167,6 @@ template <int R, bool ROWS_FAST, int THREADS> struct Feed {
                 }
             }
         }
-    }
-    // any row out of the range that pieces cover (the lanes that share a row meet first)
-    __device__ __forceinline__ bool bad() {
-        bool b = false;
-#pragma unroll
-        for (int u = 0; u < UNITS; u++) {
-            float m = top[u];
-            if constexpr (!ROWS_FAST) {
-                m = fmaxf(m, __shfl_xor(m, 1));
-                m = fmaxf(m, __shfl_xor(m, 2));
-            } else {
-                m = fmaxf(m, __shfl_xor(m, 8));
-                m = fmaxf(m, __shfl_xor(m, 16));
-                if constexpr (KQ == 2) m = fmaxf(m, __shfl_xor(m, 32));
-            }
-            b |= out_of_range(m);
-        }
-        return b;
-    }
-    __device__ __forceinline__ float most() {
-        float m = top[0];
-#pragma unroll
-        for (int u = 1; u < UNITS; u++) m = fmaxf(m, top[u]);
-        return wave_max(m);
     }
 };
 
@@ -321,17 +295,17 @@ __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const
         constexpr int PAR = decltype(par_)::value;
         constexpr int SET = LEAD == 2 ? (PAR + 1) % 2 : 0; // registers of stage s + 1, to be filled with stage s + 1 + LEAD
         constexpr int UNITS = FA::UNITS + FB::UNITS, SLOTS = (MT > 1 ? MT - 1 : 1) * NT / TOGETHER * 6; // places between the matrix instructions before the barrier
-        constexpr float down = PAR ? -1.0f : 1.0f;
+        constexpr float down = PAR ? -kDown : kDown;
         lds_char *const to = lds + (PAR ^ 1) * STAGE;
         auto unit = [&](const int u) {
             if (u < FA::UNITS) {
-                fa.store(to, SET, u, PAR ? 1.0f : -1.0f);
+                fa.store(to, SET, u, PAR ? kUp : -kUp);
                 if (!AF) ask_a(s + 1 + LEAD, SET, u);
                 else if (u == 3)
                     for (int h = 0; h < FA::SLOTS; h++) ask_a(s + 1 + LEAD, SET, h);
             } else {
                 const int v = u - FA::UNITS;
-                fb.store(to + 3 * FA::PIECE, SET, v, 1.0f);
+                fb.store(to + 3 * FA::PIECE, SET, v, kUp);
                 if (!BF) ask_b(s + 1 + LEAD, SET, v);
                 else if (v == 3)
                     for (int h = 0; h < FB::SLOTS; h++) ask_b(s + 1 + LEAD, SET, h);
@@ -396,9 +370,9 @@ __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const
             for (int h = 0; h < FB::SLOTS; h++) ask_b(1, 1, h);
         }
 #pragma unroll
-        for (int u = 0; u < FA::UNITS; u++) fa.store(lds, 0, u, 1.0f);
+        for (int u = 0; u < FA::UNITS; u++) fa.store(lds, 0, u, kUp);
 #pragma unroll
-        for (int u = 0; u < FB::UNITS; u++) fb.store(lds + 3 * FA::PIECE, 0, u, 1.0f);
+        for (int u = 0; u < FB::UNITS; u++) fb.store(lds + 3 * FA::PIECE, 0, u, kUp);
         for (int h = 0; h < FA::SLOTS; h++) ask_a(LEAD, 0, h);
         for (int h = 0; h < FB::SLOTS; h++) ask_b(LEAD, 0, h);
 
@@ -412,12 +386,12 @@ __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const
         for (uint32_t s = 0;; s += 2) {
             stage(s, P0{});
             if (s + 1 >= nk) {
-                if (CARRY) add(0, 0, 1.0f);
+                if (CARRY) add(0, 0, kDown);
                 break;
             }
             stage(s + 1, P1{});
             if (s + 2 >= nk) {
-                if (CARRY) add(0, SETS - 1, -1.0f);
+                if (CARRY) add(0, SETS - 1, -kDown);
                 break;
             }
         }
@@ -429,9 +403,9 @@ __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const
         for (int h = 0; h < FB::SLOTS; h++) fb.load_careful(ob, row_b, last_b, K, nk, 0, h);
         meet(); // (nobody reads the half that is written now)
 #pragma unroll
-        for (int u = 0; u < FA::UNITS; u++) fa.store(lds, 0, u, nk % 2 ? -1.0f : 1.0f);
+        for (int u = 0; u < FA::UNITS; u++) fa.store(lds, 0, u, nk % 2 ? -kUp : kUp);
 #pragma unroll
-        for (int u = 0; u < FB::UNITS; u++) fb.store(lds + 3 * FA::PIECE, 0, u, 1.0f);
+        for (int u = 0; u < FB::UNITS; u++) fb.store(lds + 3 * FA::PIECE, 0, u, kUp);
         meet();
 #pragma unroll
         for (int p = 0; p < 3; p++)
@@ -447,23 +421,21 @@ __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const
 #pragma unroll
                 for (int g = 0; g < 6; g++) t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i % AS][kPairA[g]], b[j][kPairB[g]], g ? t : zero, 0, 0, 0);
 #pragma unroll
-                for (int v = 0; v < 16; v++) acc[i][j][v] = __builtin_fmaf(t[v], nk % 2 ? -1.0f : 1.0f, acc[i][j][v]);
+                for (int v = 0; v < 16; v++) acc[i][j][v] = __builtin_fmaf(t[v], nk % 2 ? -kDown : kDown, acc[i][j][v]);
             }
         }
     }
 
-    bool plain = K <= 4;
+    uint32_t plain = K <= 4;
     if (!plain) {
         __attribute__((address_space(3))) float2v *const tops = reinterpret_cast<__attribute__((address_space(3))) float2v *>(lds + 2 * STAGE);
-        const bool bad_a = fa.bad(), bad_b = fb.bad(); // (both: every lane takes part in the exchanges)
-        const bool some = __builtin_amdgcn_ballot_w64(bad_a || bad_b) != 0;
-        const float2v top = {some ? INFINITY : fa.most(), fb.most()};
+        const float2v top = {wave_max(fa.top), wave_max(fb.top)};
         if (lane == 0) tops[wave] = top;
         meet();
         float2v most = tops[0];
 #pragma unroll
         for (int w = 1; w < WM * WN; w++) most = {fmaxf(most[0], tops[w][0]), fmaxf(most[1], tops[w][1])};
-        plain = most[0] == INFINITY || !in_range(most[0], most[1]);
+        plain = !in_range(most[0], most[1]);
     }
     if (__builtin_amdgcn_readfirstlane(plain)) plain_product<MT, NT, AF, BF>(acc, oa, row_a, last_a, ob, row_b, last_b, K, bma * 32, bnb * 32);
 }

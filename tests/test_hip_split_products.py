@@ -135,3 +135,28 @@ def test_roundings_have_no_direction(hip, size, layout):
     want = a.astype(np.float64) @ b.astype(np.float64)
     d = hip.to_numpy(hip.matmul(x, y)) - want
     assert abs(d.mean()) <= 2.0 ** -28 * np.sqrt((want ** 2).mean()), d.mean() / np.sqrt((want ** 2).mean())
+
+
+@pytest.mark.parametrize("size", TILES, ids=str)
+@pytest.mark.parametrize("layout", ["nt", "nn", "tt", "tn"])
+def test_small_values_beside_large_ones(hip, size, layout):
+    """All bits of values down to the smallest subnormal, in rows that also hold ordinary ones."""
+    def mixed(low, high):
+        def make(rng, K):
+            r = rng.standard_normal(K, dtype=np.float32)
+            small = rng.random(K) < 0.7
+            return np.where(small, np.ldexp(1 + rng.random(K), rng.integers(low, high, K)) * rng.choice([1, -1], K), r).astype(np.float32)
+        return make
+
+    last = size[0] - 1
+    check_chosen(hip, size, layout, {last: mixed(-126, -100), 3: mixed(-149, -126), last // 2: mixed(-120, -110), last // 3: mixed(-149, 20)},
+                 [1.0, -0.5, 2.0 ** 60, -2.0 ** -7])
+
+
+def test_sums_of_small_and_large_products(hip):
+    rng = np.random.default_rng(9)
+    M, K, N = 150, 96, 200
+    a = np.ldexp(rng.standard_normal((1, M, K)), rng.integers(-126, -120, (1, M, K))).astype(np.float32)
+    b = np.ldexp(rng.standard_normal((1, K, N)), rng.integers(95, 100, (1, K, N))).astype(np.float32)
+    a[0, :, 0], b[0, 0] = 1.0, 0.0          # a row's largest value meets nothing
+    check(hip.to_numpy(hip.matmul(hip.from_numpy(a), hip.from_numpy(b))), a, b)
