@@ -1132,17 +1132,17 @@ template <int HD, bool PIECES> __device__ __forceinline__ bool prefill_rows(cons
                     }
             }
         } else {
-#pragma unroll
-            for (int db = 0; db < HD / 32; db++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) acc_o[db][v] *= alpha;
+            // the tile's share of O, from zero and of negated weights every other time (split_tile.hpp)
+            float16v sum[HD / 32];
+            const bool odd = (it + __builtin_amdgcn_readfirstlane(wave)) % 2;
+            const float up = odd ? -1.0f : 1.0f, down = up;
 #pragma unroll
             for (int q = 0; q < KEYS / 16; q++) { // 16 keys: the eight weights that a lane holds of them, and V's rows in that order
                 uint4w pw[3];
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     uint32_t x[3];
-                    split::split2(acc_s[q / 2][q % 2 * 8 + 2 * r], acc_s[q / 2][q % 2 * 8 + 2 * r + 1], x);
+                    split::split2(acc_s[q / 2][q % 2 * 8 + 2 * r] * up, acc_s[q / 2][q % 2 * 8 + 2 * r + 1] * up, x);
 #pragma unroll
                     for (int p = 0; p < 3; p++) pw[p][r] = x[p];
                 }
@@ -1154,9 +1154,14 @@ template <int HD, bool PIECES> __device__ __forceinline__ bool prefill_rows(cons
                     for (int p = 0; p < 3; p++) vf[p] = piece((3 + p) * PIECE + (q * (HD / 32) + db) * 1024 + lg * 512 + row * 16);
 #pragma unroll
                     for (int k = 0; k < 6; k++)
-                        acc_o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[split::kPairA[k]], __builtin_bit_cast(bf16x8, pw[split::kPairB[k]]), acc_o[db], 0, 0, 0);
+                        sum[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[split::kPairA[k]], __builtin_bit_cast(bf16x8, pw[split::kPairB[k]]),
+                                                                         q || k ? sum[db] : (float16v){}, 0, 0, 0);
                 }
             }
+#pragma unroll
+            for (int db = 0; db < HD / 32; db++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc_o[db][v] = __builtin_fmaf(sum[db][v], down, acc_o[db][v] * alpha);
             __syncthreads(); // (one buffer: the tile is read)
         }
         if (more) store_kv(cur ^ 1);

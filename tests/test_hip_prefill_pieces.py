@@ -34,3 +34,19 @@ def test_against_64_bits(hip, hd, rep, S, pos0, far):
     err = np.abs(got - np.matmul(p, v))
     print("error / bound: max %.3f, mean %.5f" % ((err / bound).max(), (err / bound).mean()), flush=True)
     assert (err <= bound).all()
+
+
+@pytest.mark.parametrize("hd,rep,S", [(64, 3, 512), (64, 4, 1500), (128, 2, 1024)])
+def test_roundings_have_no_direction(hip, hd, rep, S):
+    """The outputs' error in the mean, against their root mean square per query: roundings to nearest have none (over these numbers of
+    outputs below 2^-28), sums that are cut off below have 2^-26 and more."""
+    rng = np.random.default_rng(S)
+    q, k, v = (rng.standard_normal(s, dtype=np.float32) for s in ((2, 4 * rep, S, hd), (2, 4, S, hd), (2, 4, S, hd)))
+    got = hip.to_numpy(cases.decode_attention_ops(hip, hip.from_numpy(q), hip.from_numpy(k), hip.from_numpy(v), rep))
+    q, k, v = (x.astype(np.float64) for x in (q, np.repeat(k, rep, 1), np.repeat(v, rep, 1)))
+    s = np.matmul(q, k.transpose(0, 1, 3, 2)) / np.sqrt(hd)
+    s[..., np.triu(np.ones((S, S), dtype=bool), 1)] = -np.inf
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = np.matmul(p / p.sum(-1, keepdims=True), v)
+    d = (got - want) / np.sqrt((want ** 2).mean(-1, keepdims=True))
+    assert abs(d.mean()) <= 2.0 ** -28, d.mean()
