@@ -941,7 +941,7 @@ template <int HD, bool PIECES> __device__ __forceinline__ bool prefill_rows(cons
     typedef uint32_t uint4w __attribute__((ext_vector_type(4)));
     float4v qf[PIECES ? 1 : HD / 8];
     bf16x8 qp[PIECES ? HD / 16 : 1][3]; // chunk c: d = 16 c + 8 lg .. + 7
-    float top_qk = 0.0f, top_v[4] = {}; // largest magnitudes seen, V's by the columns that this thread loads
+    float top_qk = 0.0f, top_v = 0.0f; // largest magnitudes seen
     if constexpr (!PIECES) {
 #pragma unroll
         for (int c = 0; c < HD / 8; c++) {
@@ -1028,10 +1028,10 @@ template <int HD, bool PIECES> __device__ __forceinline__ bool prefill_rows(cons
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 uint32_t a[3], b[3];
-                split::grow(top_v[r], vr[0][r], vr[1][r]);
-                split::grow(top_v[r], vr[2][r], vr[3][r]);
-                split::split2(vr[0][r], vr[1][r], a);
-                split::split2(vr[2][r], vr[3][r], b);
+                split::grow(top_v, vr[0][r], vr[1][r]);
+                split::grow(top_v, vr[2][r], vr[3][r]);
+                split::split2(vr[0][r] * split::kUp, vr[1][r] * split::kUp, a);
+                split::split2(vr[2][r] * split::kUp, vr[3][r] * split::kUp, b);
                 const uint32_t row = (w % 8 * 4 + (r ^ (w / 4 & 3))) ^ (vg * 12);
 #pragma unroll
                 for (int p = 0; p < 3; p++) *reinterpret_cast<lds_pair *>(lds + p * PIECE + v_at + row * 16) = (split::uint2v){a[p], b[p]};
@@ -1135,7 +1135,7 @@ template <int HD, bool PIECES> __device__ __forceinline__ bool prefill_rows(cons
             // the tile's share of O, from zero and of negated weights every other time (split_tile.hpp)
             float16v sum[HD / 32];
             const bool odd = (it + __builtin_amdgcn_readfirstlane(wave)) % 2;
-            const float up = odd ? -1.0f : 1.0f, down = up;
+            const float up = odd ? -split::kUp : split::kUp, down = odd ? -split::kDown : split::kDown;
 #pragma unroll
             for (int q = 0; q < KEYS / 16; q++) { // 16 keys: the eight weights that a lane holds of them, and V's rows in that order
                 uint4w pw[3];
@@ -1168,10 +1168,9 @@ template <int HD, bool PIECES> __device__ __forceinline__ bool prefill_rows(cons
         __syncthreads();
     }
     if constexpr (PIECES) {
-        // (a score is a sum of products of magnitudes below 1e18: what the smallest values' pieces lose of it is nothing beside 1)
-        bool bad = top_qk > 1.0e18f;
-#pragma unroll
-        for (int r = 0; r < 4; r++) bad = bad || split::out_of_range(top_v[r]);
+        // (a score is a sum of products of magnitudes below 1e18: what the smallest values' pieces lose of it is nothing beside 1;
+        // 64 keys' products of weights up to 1 and V, both scaled by 2^16, stay below 2^127)
+        const bool bad = !(top_qk <= 1.0e18f && top_v < 0x1p88f);
         if (__syncthreads_or(bad)) return true;
     }
     if (e.ksplit > 1) { // the part's statistics and un-normalised O; lane group 0 of a wave writes the statistics

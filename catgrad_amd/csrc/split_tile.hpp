@@ -63,8 +63,6 @@ __device__ __forceinline__ void split2(float x, float y, uint32_t (&w)[3]) {
 __device__ __forceinline__ void grow(float &m, float x, float y) { // m = max(m, |x|, |y|)
     asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(x), "v"(y));
 }
-// A row whose largest magnitude is m cannot be multiplied in pieces at full precision.
-__device__ __forceinline__ bool out_of_range(float m) { return m > 3.0e38f || (m > 0.0f && m < 8.0e-28f); }
 // Operands of magnitudes up to a and b: 16 products of scaled pieces stay below 2^127.
 __device__ __forceinline__ bool in_range(float a, float b) { return a < 0x1p110f && b < 0x1p110f && a * b < 0x1p90f; }
 // the largest of a wave's values, none of them negative

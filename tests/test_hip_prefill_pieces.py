@@ -50,3 +50,22 @@ def test_roundings_have_no_direction(hip, hd, rep, S):
     want = np.matmul(p / p.sum(-1, keepdims=True), v)
     d = (got - want) / np.sqrt((want ** 2).mean(-1, keepdims=True))
     assert abs(d.mean()) <= 2.0 ** -28, d.mean()
+
+
+@pytest.mark.parametrize("hd,rep,S", [(64, 3, 200), (128, 2, 140)])
+@pytest.mark.parametrize("low,high", [(-149, -126), (-126, -115), (-149, 3), (80, 95)])
+def test_values_of_any_size(hip, hd, rep, S, low, high):
+    """V with small (or very large) values beside ordinary ones: queries that see only such keys get all of their bits."""
+    rng = np.random.default_rng(S + high)
+    q, k, v = (rng.standard_normal(s, dtype=np.float32) for s in ((1, 2 * rep, S, hd), (1, 2, S, hd), (1, 2, S, hd)))
+    v[:, :, :70, ::3] = np.ldexp(v[:, :, :70, ::3], rng.integers(low, high, v[:, :, :70, ::3].shape)).astype(np.float32)
+    got = hip.to_numpy(cases.decode_attention_ops(hip, hip.from_numpy(q), hip.from_numpy(k), hip.from_numpy(v), rep))
+    q, k, v = (x.astype(np.float64) for x in (q, np.repeat(k, rep, 1), np.repeat(v, rep, 1)))
+    s = np.matmul(q, k.transpose(0, 1, 3, 2)) / np.sqrt(hd)
+    s[..., np.triu(np.ones((S, S), dtype=bool), 1)] = -np.inf
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    score = (hd + 8) * 2.0 ** -24 * (np.matmul(np.abs(q), np.abs(k).transpose(0, 1, 3, 2)) / np.sqrt(hd)).max(-1, keepdims=True)
+    # as above, and the spacing of subnormal numbers per key and step of the division
+    bound = (2 * score + 64 * 2.0 ** -24 + 2 * (S + 16) * 2.0 ** -24) * np.matmul(p, np.abs(v)) + (S + 8) * 2.0 ** -149
+    assert (np.abs(got - np.matmul(p, v)) <= bound).all()
