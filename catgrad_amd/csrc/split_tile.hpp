@@ -13,7 +13,7 @@
 // Both operands are multiplied by 2^16 on their way into pieces, and the chains' sums by 2^-32 as they are added: then the three
 // pieces of every 32-bit number, the subnormal ones included, are bfloat16 numbers (multiples of 2^-133).  What the pieces do
 // not hold are infinities and products at the upper end of the range: while it splits, a workgroup keeps the largest magnitude of
-// either operand, and a tile whose products could leave the range is multiplied again on the 32-bit instructions (plain_product).
+// either operand, and a tile whose products could leave the range is multiplied again on the 32-bit instructions (`plain`).
 #pragma once
 
 #include "common.hpp"
@@ -43,6 +43,7 @@ struct TileSide {
 // the six piece products, the largest last, in an order that is done with the left side's small pieces early
 constexpr int kPairA[6] = {2, 1, 1, 0, 0, 0}, kPairB[6] = {0, 1, 0, 2, 1, 0};
 
+constexpr uint32_t kPitch = kDepth + 4; // words from row to row where a stage lies in LDS in 32 bits
 constexpr uint32_t lds_bytes(int bm, int bn) { return 2 * (uint32_t)(bm + bn) * kDepth * 6 + 64; }
 
 __device__ __forceinline__ uint32_t cvt2(float x, float y) {
@@ -166,59 +167,22 @@ template <int R, bool ROWS_FAST, int THREADS> struct Feed {
             }
         }
     }
-};
-
-// The 32-bit instructions on operands straight from memory: what is left for tiles that pieces do not cover.  A row of blocks after
-// the other; eight values of k at a time, four of them per lane group, asked for while the eight before them multiply.
-template <int MT, int NT, bool AF, bool BF, class RowA, class RowB>
-__device__ __forceinline__ void plain_product(float16v (&acc)[MT][NT], const TileSide &a, RowA row_a, uint32_t last_a, const TileSide &b, RowB row_b,
-                                           uint32_t last_b, uint32_t K, uint32_t wm, uint32_t wn) {
-    typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
-    const uint32_t li = threadIdx.x % 32, lg = threadIdx.x % 64 / 32, eights = K / 8;
-    auto four = [&](const uint32_t *p, const int64_t s_k, const bool fast, const uint32_t k) {
-        if (!fast && s_k == 1) return (float4v)*reinterpret_cast<const float4u *>(p + k);
-        float4v v;
+    // the values of a set as they are, rows of kPitch
+    __device__ __forceinline__ void store_plain(__attribute__((address_space(3))) float *lds, int set) {
+        const uint32_t t = threadIdx.x;
+        if constexpr (!ROWS_FAST) {
 #pragma unroll
-        for (int t = 0; t < 4; t++) v[t] = asf(p[(int64_t)(k + t) * s_k]);
-        return v;
-    };
-    const uint32_t *pb[NT];
+            for (int h = 0; h < SLOTS; h++)
+                if (R >= STEP || t < R * 4) *reinterpret_cast<__attribute__((address_space(3))) float4v *>(lds + (t / 4 + h * STEP) * kPitch + t % 4 * 4) = r[set][h];
+        } else {
+            const uint32_t row = t / (128 / KQ) * 32 + t % 8 * 4, k = t / 8 % (16 / KQ) * KQ;
 #pragma unroll
-    for (int j = 0; j < NT; j++) pb[j] = b.p + row_b(min(wn + j * 32 + li, last_b));
+            for (int h = 0; h < SLOTS; h++)
 #pragma unroll
-    for (int i = 0; i < MT; i++) {
-        const uint32_t *const pa = a.p + row_a(min(wm + i * 32 + li, last_a));
-#pragma unroll
-        for (int j = 0; j < NT; j++) acc[i][j] = (float16v){};
-        float4v fa, fb[NT];
-        auto ask = [&](const uint32_t k) {
-            fa = four(pa, a.s_k, AF, k + lg * 4);
-#pragma unroll
-            for (int j = 0; j < NT; j++) fb[j] = four(pb[j], b.s_k, BF, k + lg * 4);
-        };
-        if (eights) ask(0);
-        for (uint32_t c = 0; c < eights; c++) {
-            const float4v ga = fa;
-            float4v gb[NT];
-#pragma unroll
-            for (int j = 0; j < NT; j++) gb[j] = fb[j];
-            ask(min(c + 1, eights - 1) * 8);
-#pragma unroll
-            for (int t = 0; t < 4; t++)
-#pragma unroll
-                for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(ga[t], gb[j][t], acc[i][j], 0, 0, 0);
-        }
-        for (uint32_t k = eights * 8; k < K; k += 2) {
-            const uint32_t kk = k + lg, at = min(kk, K - 1);
-            const float x = asf(pa[(int64_t)at * a.s_k]);
-#pragma unroll
-            for (int j = 0; j < NT; j++) {
-                const float y = asf(pb[j][(int64_t)at * b.s_k]);
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(kk < K ? x : 0.0f, kk < K ? y : 0.0f, acc[i][j], 0, 0, 0);
-            }
+                for (int i = 0; i < 4; i++) lds[(row + i) * kPitch + k + h] = r[set][h][i];
         }
     }
-}
+};
 
 // acc = the workgroup's tile of A B^T: WM x WN waves of MT x NT blocks of 32 x 32 each (lane (li, lg), register v of a block: row
 // 8 (v / 4) + 4 lg + v % 4, column li).  row_a / row_b: tile row -> element offset of that row; rows beyond last_a / last_b repeat
@@ -435,7 +399,54 @@ __device__ __forceinline__ void product(float16v (&acc)[MT][NT], lds_char *const
         for (int w = 1; w < WM * WN; w++) most = {fmaxf(most[0], tops[w][0]), fmaxf(most[1], tops[w][1])};
         plain = !in_range(most[0], most[1]);
     }
-    if (__builtin_amdgcn_readfirstlane(plain)) plain_product<MT, NT, AF, BF>(acc, oa, row_a, last_a, ob, row_b, last_b, K, bma * 32, bnb * 32);
+    if (!__builtin_amdgcn_readfirstlane(plain)) return;
+    // The 32-bit instructions, for what the pieces do not hold: a stage is multiplied while the next one is on its way.  Lane group
+    // lg multiplies k = 8 c + 4 lg + t in the t-th of four instructions.
+    typedef __attribute__((address_space(3))) float lds_float;
+    lds_float *const whole = (lds_float *)lds;
+    constexpr uint32_t WHOLE = (BM + BN) * kPitch;
+    static_assert(2 * WHOLE * 4 <= 2 * STAGE, "both stages fit where the pieces were");
+    const uint32_t stages = (K + kDepth - 1) / kDepth;
+    auto fetch = [&](const uint32_t s) {
+        if (CARE || (s + 1) * kDepth > K) {
+#pragma unroll
+            for (int h = 0; h < FA::SLOTS; h++) fa.load_careful(oa, row_a, last_a, K, s, 0, h);
+#pragma unroll
+            for (int h = 0; h < FB::SLOTS; h++) fb.load_careful(ob, row_b, last_b, K, s, 0, h);
+        } else {
+#pragma unroll
+            for (int h = 0; h < FA::SLOTS; h++) fa.load(oa, s, 0, h);
+#pragma unroll
+            for (int h = 0; h < FB::SLOTS; h++) fb.load(ob, s, 0, h);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[i][j] = zero;
+    fetch(0);
+    meet(); // (everybody is done with the pieces)
+    for (uint32_t s = 0; s < stages; s++) {
+        lds_float *const at = whole + s % 2 * WHOLE;
+        fa.store_plain(at, 0);
+        fb.store_plain(at + BM * kPitch, 0);
+        meet(); // (the stage is there, and nobody reads the one before the last)
+        fetch(min(s + 1, stages - 1));
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            float4v x[MT], y[NT];
+#pragma unroll
+            for (int i = 0; i < MT; i++) x[i] = *reinterpret_cast<__attribute__((address_space(3))) float4v *>(at + ((bma + i) * 32 + li) * kPitch + c * 8 + lg * 4);
+#pragma unroll
+            for (int j = 0; j < NT; j++) y[j] = *reinterpret_cast<__attribute__((address_space(3))) float4v *>(at + (BM + (bnb + j) * 32 + li) * kPitch + c * 8 + lg * 4);
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i][t], y[j][t], acc[i][j], 0, 0, 0);
+        }
+    }
 }
 
 } // namespace split
