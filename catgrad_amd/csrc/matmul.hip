@@ -2525,7 +2525,8 @@ static int low_product(cg_backend *be, int kind, const cg_tensor *x, bool x_lies
     return rc;
 }
 
-int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_tensor *out, bool wide_only) {
+// patterns: operands of a narrow dtype may be multiplied from patterns; kDeclined: they would be, and the pool has no room to pack one.
+static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_tensor *out, bool wide_only, bool patterns) {
     if (int frc = flush_deferred(be)) return frc;
     MmArgs a;
     MmFold f;
@@ -2553,11 +2554,11 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
     // Operands of a narrow dtype are multiplied from 2-byte / 1-byte patterns where rows of k are whole 16-byte pieces: as they
     // lie in memory when their buffer holds that format, else narrowed in memory first (the right operand once per buffer)
     // (env CG_GEMM_PACKED=0 switches it off).
-    const bool packable = f32 && K != 0 && M > 8 && kind && packed_narrow_ok() && batch == 1 && K % (kind == 3 ? 16 : 8) == 0 && x->buf && y->buf;
+    const bool packable = patterns && f32 && K != 0 && M > 8 && kind && packed_narrow_ok() && batch == 1 && K % (kind == 3 ? 16 : 8) == 0 && x->buf && y->buf;
     const bool x_lies = packable && native_rows(x, kind, a.a_sm, a.a_sk, K, false), y_lies = packable && native_rows(y, kind, a.b_sn, a.b_sk, K, false);
     const NarrowRoute route = narrow_route(kind, {M, a.a_sm, x_lies}, {N, a.b_sn, y_lies}, K, packable, big, wide_only);
     const bool big_packed = route == NarrowRoute::wide, low = route == NarrowRoute::low;
-    bool x_native = (big_packed || low) && x_lies, y_native_rows = (big_packed || low) && y_lies;
+    const bool x_native = (big_packed || low) && x_lies, y_native_rows = (big_packed || low) && y_lies;
     // Whole stages of 64 bytes of k in whole turns of the ring, 16-byte rows, byte offsets that fit 32 bits: the wide tile
     // fed by loads straight into LDS (env CG_GEMM_DLDS=0: the register-staged one).  Only that kernel can round the result
     // to the operands' format in its store; without `out` the call just says whether this product would run on it.
@@ -2576,12 +2577,7 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
     if (!out) return can_round ? CG_OK : kDeclined;
 
     // ---- the operands' addresses -------------------------------------------------------------------------------------
-    if (low) {
-        rc = low_product(be, kind, x, x_native, y, y_native_rows, a, M, N, K, out);
-        if (rc != kDeclined) return rc;
-        x_native = y_native_rows = false; // no room to pack an operand: from words, as they lie or widened
-        if (out->buf->fmt != kFmtWords) return kDeclined;
-    }
+    if (low) return low_product(be, kind, x, x_native, y, y_native_rows, a, M, N, K, out);
     rc = mm_operand(x, true, x_native, &a);
     if (rc) return rc;
     // a decode-time linear layer of a narrow dtype reads its weight matrix at 2 or 1 bytes a weight (see below)
@@ -2752,7 +2748,10 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
             const bool x_shared = x->rc.load() > 1 || x->buf->rc.load() > 1;
             int prc = x_native ? CG_OK : pack_operand(be, words_buffer(x), a.A, a.a_sm, a.a_sk, M, K, kind, x_shared, &pa, &ta, &ca);
             if (!prc && !y_native) prc = pack_operand(be, words_buffer(y), a.B, a.b_sn, a.b_sk, N, K, kind, true, &pb, &tb, &cb);
-            if (!prc) {
+            if (prc) {
+                (void)hipGetLastError();
+                prc = kDeclined;
+            } else {
                 MmArgs p = a;
                 p.A = static_cast<const uint32_t *>(pa);
                 p.B = static_cast<const uint32_t *>(pb);
@@ -2815,6 +2814,12 @@ int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_ten
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "matmul launch");
+}
+
+int launch_matmul(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_tensor *out, bool wide_only) {
+    const int rc = product(be, x, y, out, wide_only, true);
+    // no room to pack an operand: from words, as they lie or widened (a result in patterns is the caller's to ask for again in words)
+    return rc == kDeclined && out && out->buf->fmt == kFmtWords ? product(be, x, y, out, wide_only, false) : rc;
 }
 
 } // namespace cg
