@@ -1,14 +1,16 @@
 // C[b, M, N] = A[b, M, K] B[b, K, N] of 32-bit floats for more than eight rows, on the bfloat16 matrix instructions (split_tile.hpp).
 //
-// 8192 x 2048 x 8192: 1185 us = 232 TFLOP/s, where the 32-bit instructions took 1990 us = 138 (88 % of their peak); 1024 x 1024 x
-// 3072: 47 against 76 us; 32 x 2048 x 8192: 23 against 47 us.  The wide tile is bound by power: matrix pipes busy 76 % of
-// the cycles at 1.64 GHz (64 SQ_VALU_MFMA_BUSY_CYCLES per instruction pair and GRBM_GUI_ACTIVE over the time), so what it saves
+// 8192 x 2048 x 8192: 1250 us = 220 TFLOP/s, where the 32-bit instructions took 1990 us = 138 (88 % of their peak); 1024 x 1024 x
+// 3072: 53 against 74 us; 32 x 2048 x 8192: 22 against 46 us.  A few small shapes stay above the 32-bit instructions, whose tiles
+// started sooner: with contiguous rows 100 x 576 x 1536 13.1 against 10.7, 4096 x 700 x 50 18.8 against 14.7 and 100 x 64 x 1024 6.6
+// against 5.3; 333 x 1001 x 333 16.4 against 15.5.  The wide tile is bound by the clock at the card's power limit, so what it saves
 // elsewhere comes back as clock: eight waves that share one 256 x 256 tile split a third less than two workgroups of four with
 // 256 x 128 each and run 8 % faster.  Splitting by v_dot2c_f32_bf16 (one instruction for the shift and the subtraction): slower.
 #include "gemm_args.hpp"
 #include "split_tile.hpp"
 
 #include <algorithm>
+#include <cmath>
 
 namespace cg {
 namespace {
@@ -84,25 +86,33 @@ template <int WM, int WN, int MT, int NT, bool AF, bool BF, bool CARE> Kernel pr
     const int lds = (int)lds_bytes(32 * WM * MT, 32 * WN * NT);
     return hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess ? k : nullptr;
 }
-// microseconds that a round of workgroups (one per compute unit) takes per stage, by tile
-constexpr double kStage[7] = {2.4, 0.72, 0.5, 0.55, 1.65, 0.375, 0.7};
-// In the order of `kStage`: the wide tile, the tile for what does not fill the device with it, two for a few rows, and the second
-// one's twin for any alignment; 64 x 64 for k-contiguous operands whose results are small or narrow, and its twin.  What the
-// 64 x 64 tile gains over the others (cuts along k included): 1800 x 100 x 400 12.8 -> 9.0 us, 200 x 1001 x 333 23.7 -> 17.3,
-// 64 x 256 x 512 10.8 -> 9.9, 100 x 17 x 100 9.7 -> 7.0; from 1024 x 1024 x 1024 on (29 against 25 us) it loses to 128 x 128.
+// What a launch takes, in microseconds: before and behind the stages, a stage, and the share of a stage that each workgroup of a
+// compute unit takes when there are several (they hide each other's waits).
+struct Cost {
+    double start, stage, share;
+};
+// In the order of `tiles`: the wide tile, the tile for what does not fill the device with it, two for a few rows, and the second
+// one's twin for any alignment; 64 x 64 for k-contiguous operands, and its twin; 64 x 64 for operands with contiguous rows, which
+// two waves turn in registers, and its twin.  Fitted to 474 shapes of 16 to 8192 rows in all layouts, every tile and cut timed: what this
+// picks is 1 % above the fastest in the mean.
+constexpr Cost kCost[9] = {{9.8, 1.64, 1.0}, {5.8, 0.70, 0.83}, {4.4, 0.61, 0.68}, {5.2, 0.42, 1.45}, {5.6, 1.44, 0.835},
+                           {4.0, 0.37, 0.705}, {4.5, 0.68, 0.937}, {4.85, 0.40, 1.03}, {5.0, 0.817, 0.85}};
 const Tile *tiles() {
 #define CG_TILE(WM, WN, MT, NT, CARE)                                                                       \
     {32 * WM * MT, 32 * WN * NT, 64 * WM * WN, {{prepared<WM, WN, MT, NT, false, false, CARE>(), prepared<WM, WN, MT, NT, false, true, CARE>()}, \
                                   {prepared<WM, WN, MT, NT, true, false, CARE>(), prepared<WM, WN, MT, NT, true, true, CARE>()}}}
 #define CG_SMALL_TILE(CARE) \
     {64, 64, 256, {{prepared<2, 2, 1, 1, false, false, CARE>(), nullptr}, {nullptr, nullptr}}}
+#define CG_ROWS_TILE(CARE) \
+    {64, 64, 128, {{nullptr, prepared<1, 2, 2, 1, false, true, CARE>()}, {prepared<1, 2, 2, 1, true, false, CARE>(), prepared<1, 2, 2, 1, true, true, CARE>()}}}
 #define CG_LOW_TILE(WM, WN, MT, NT) \
     {32 * WM * MT, 32 * WN * NT, 64 * WM * WN, {{prepared<WM, WN, MT, NT, false, false, false>(), prepared<WM, WN, MT, NT, false, true, false>()}, {nullptr, nullptr}}}
-    static const Tile t[7] = {CG_TILE(2, 4, 4, 2, false), CG_TILE(2, 2, 2, 2, false), CG_LOW_TILE(1, 4, 2, 1), CG_LOW_TILE(1, 4, 1, 2), CG_TILE(2, 2, 2, 2, true),
-                              CG_SMALL_TILE(false), CG_SMALL_TILE(true)};
+    static const Tile t[9] = {CG_TILE(2, 4, 4, 2, false), CG_TILE(2, 2, 2, 2, false), CG_LOW_TILE(1, 4, 2, 1), CG_LOW_TILE(1, 4, 1, 2), CG_TILE(2, 2, 2, 2, true),
+                              CG_SMALL_TILE(false), CG_SMALL_TILE(true), CG_ROWS_TILE(false), CG_ROWS_TILE(true)};
 #undef CG_TILE
 #undef CG_LOW_TILE
 #undef CG_SMALL_TILE
+#undef CG_ROWS_TILE
     return t;
 }
 
@@ -133,26 +143,26 @@ int launch_split_gemm(cg_backend *be, MmArgs a, bool a_mfast, bool b_nfast) {
     const bool care = !a.a_vec || !a.b_vec || !fits(a_mfast, a.a_sm, a.a_sk, a.M) || !fits(b_nfast, a.b_sn, a.b_sk, a.N);
     auto count = [&](int t) { return (uint64_t)((a.M + all[t].bm - 1) / all[t].bm) * ((a.N + all[t].bn - 1) / all[t].bn) * a.batch; };
     const uint64_t mn = (uint64_t)a.M * a.N;
-    // The tile, and over how many workgroups k is cut (at least 64 values each, partial results of at most 64 MB), by what a
-    // round of workgroups over the compute units takes: measured over M = 16 .. 4096 at the models' widths, where this picks the
-    // fastest of all pairs or one within 5 % of it.  512 x 2048 x 2048: 38 us in four parts of 128 x 128 tiles, 47 in two of the
-    // wide one; 2048 x 2048 x 8192: 305 with the wide one, 357 without; 32 x 2048 x 8192: 23 with 32 x 256, 35 with 128 x 128.
+    // The tile, and over how many workgroups k is cut (at least 64 values each, partial results of at most 64 MB), by what the launch
+    // takes: in us, 512 x 2048 x 2048 37 in four parts of 128 x 128 tiles, 45 in 16 of the wide one; 2048 x 2048 x 8192 342 with
+    // the wide one, 401 without; 32 x 2048 x 8192 21 with 32 x 256, 34 with 128 x 128; 333 x 1536 x 576 16 with 64 x 64, 20 without; and where rows are contiguous, on the two-wave
+    // tile and without it (before: on the 32-bit instructions), 100 x 64 x 1024 6.7 and 9.1 (5.2), 1500 x 700 x 50 15.6 and 19.8 (13.0).
     int t = -1;
     uint64_t splits = 1;
     double best = 0;
     auto consider = [&](int tile) {
+        const Cost &c = kCost[tile];
         const uint64_t wgs = count(tile);
         for (uint64_t p = 1; p <= 16 && (p == 1 || (a.K / p >= 64 && p * a.batch * mn <= (16u << 20))); p++) {
             const uint32_t part = p > 1 ? (uint32_t)((a.K + p - 1) / p + 31) / 32 * 32 : a.K;
             if (p > 1 && (a.K + part - 1) / part != p) continue;
-            const double rounds = (double)((wgs * p + be->compute_units - 1) / be->compute_units);
-            const double stages = kStage[tile] * ((part + kDepth - 1) / kDepth);
-            // (small tiles: several to a compute unit, which hide each other's waits)
-            const double us = (tile < 5 ? rounds * ((tile == 1 || tile == 2 ? 3.0 : 2.0) + stages) : 2.0 + stages * std::max(1.0, 0.85 * rounds)) + (p > 1 ? 4.0 + 1e-6 * p * a.batch * mn : 0.0);
+            const double rounds = std::ceil((double)(wgs * p) / be->compute_units), stages = c.stage * ((part + kDepth - 1) / kDepth);
+            const double us = (tile == 0 ? rounds * (c.start + stages) : c.start + stages * std::max(1.0, c.share * rounds)) +
+                              (p > 1 ? 2.15 + 0.19 * p + 1.05e-6 * p * a.batch * mn : 0.0);
             if (t < 0 || us < best) t = tile, splits = p, best = us;
         }
     };
-    if (!a_mfast && !b_nfast) consider(care ? 6 : 5);
+    consider((a_mfast || b_nfast ? 7 : 5) + care);
     if (care) consider(4);
     else {
         consider(1);

@@ -8,7 +8,8 @@ pytestmark = pytest.mark.gpu
 # edges of the tiles (64 x 64, 32 x 256, 64 x 128, 128 x 128, 256 x 256), of a stage (16 values of k) and of the cuts along k
 SIZES = [(9, 16, 8), (9, 1, 33), (17, 33, 31), (32, 2048, 260), (33, 96, 128), (64, 100, 129), (65, 576, 192), (128, 160, 256), (129, 31, 4), (255, 64, 260),
          (300, 1000, 520), (1030, 48, 1028), (2048, 64, 8192),
-         (64, 64, 64), (65, 63, 65), (1800, 100, 400), (200, 1001, 333), (1500, 700, 50)]
+         (64, 64, 64), (65, 63, 65), (1800, 100, 400), (200, 1001, 333), (1500, 700, 50),
+         (2048, 128, 8192), (1024, 64, 4096), (1030, 63, 4098), (20, 512, 8192)]
 
 
 def operands(be, M, K, N, a_rows_fast, b_rows_fast, batch=1, seed=0):
@@ -75,8 +76,9 @@ def test_ends_of_the_range(hip, M, side):
     np.testing.assert_array_equal(got[~np.isnan(want)], want[~np.isnan(want)])
 
 
-# by layout: the 256 x 256 tile in all four; 64 x 64, 64 x 128 and 128 x 128; 32 x 256; the same cut along k; any alignment
-TILES = [(2048, 64, 8192), (72, 64, 2048), (32, 64, 8192), (32, 2048, 8192), (200, 512, 256), (130, 63, 130)]
+# the 128 x 128 tile; 64 x 64 of four waves (nt) and of two; 32 x 256 and 128 x 128 cut along k; 64 x 64 cut; 64 x 64 for any alignment;
+# 256 x 256; 64 x 128 and 128 x 128; 128 x 128 for any alignment
+TILES = [(2048, 64, 8192), (72, 64, 2048), (32, 64, 8192), (32, 2048, 8192), (200, 512, 256), (130, 63, 130), (2048, 128, 8192), (1024, 64, 4096), (1030, 63, 4098)]
 
 
 def check_chosen(be, size, layout, rows, scales):
