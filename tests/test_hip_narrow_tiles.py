@@ -59,3 +59,30 @@ def test_fp8_sums_keep_32_bits(hip):
     ws, _ = backend_values(hip, torch, "fp8", w)
     got = hip.to_numpy(hip.cast(hip.matmul(xs, hip.broadcast(hip.transpose(ws, 0, 1), (1, K, N))), A.F32))
     assert (got == 18.0).all()                    # 16 + 1 + 2^-15
+
+
+@pytest.mark.parametrize("M", [40, 200])
+def test_fp8_results_at_the_ends_of_the_range(hip, M):
+    """Sums beyond the largest value are that value, NaN stays NaN, small ones round to multiples of 2^-9."""
+    import torch
+
+    K, N = 256, 1024
+    rng = np.random.default_rng(M)
+    x = rng.standard_normal((1, M, K), dtype=np.float32)
+    x[0, ::3] *= 100.0
+    x[0, 1::3] = np.where(np.arange(K) < 2, rng.integers(-8, 9, (len(x[0, 1::3]), K)) * 2.0 ** -9, 0.0)
+    x[0, 5, 7] = np.nan
+    w = np.where(np.arange(K) < 2, 0.5, rng.standard_normal((N, K))).astype(np.float32)
+    xs, a = backend_values(hip, torch, "fp8", x)
+    ws, b = backend_values(hip, torch, "fp8", w)
+    got = hip.to_numpy(hip.cast(hip.matmul(xs, hip.broadcast(hip.transpose(ws, 0, 1), (1, K, N))), A.F32))[0]
+    exact = a[0] @ b.T
+    want = torch.from_numpy(np.clip(exact, -448, 448)).float().to(torch.float8_e4m3fn).float().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isnan(got[5]).all()
+    small = np.arange(M) % 3 == 1
+    np.testing.assert_array_equal(got[small & (np.arange(M) != 5)], want[small & (np.arange(M) != 5)])    # sums of two multiples of 2^-10: exact
+    far = np.abs(exact) > 500
+    assert far.sum() > 100 and (got[far] == 448 * np.sign(exact[far])).all()
+    # everything from 448 up is 448; below, one rounding to the dtype of a sum of 256 roundings of at most 448 * 2^-24 each
+    near, keep = np.clip(exact, -448, 448), ~np.isnan(want)
+    assert (np.abs(got - near)[keep] <= UNIT["fp8"] * np.abs(near[keep]) + 2.0 ** -10 + 2 * K * 2.0 ** -24 * 448).all()
