@@ -24,9 +24,9 @@ def operands(be, M, K, N, a_rows_fast, b_rows_fast, batch=1, seed=0):
 def check(got, a, b):
     a, b = a.astype(np.float64), b.astype(np.float64)
     K = a.shape[-1]
-    # three left-out products of pieces (2^-22 together at most), a rounding per 16 values of k and kept product, and up to 16
+    # three left-out products of pieces (2^-24 together at most), a rounding per 16 values of k and kept product, and up to 16
     # partial sums, each relative to the sum of magnitudes
-    bound = (4.0 + 6 * ((K + 15) // 16) + 16) * 2.0 ** -24 * (np.abs(a) @ np.abs(b)) + 1e-37
+    bound = (1.0 + 6 * ((K + 15) // 16) + 16) * 2.0 ** -24 * (np.abs(a) @ np.abs(b)) + 1e-37
     assert (np.abs(got - a @ b) <= bound).all()
 
 
