@@ -873,10 +873,11 @@ constexpr size_t prefill_lds_bytes(int hd) { return 2 * 2 * (size_t)kPfKeys * (h
 // queries' pieces stay in registers, those of K and V are made on the way into LDS, once for the four waves (V turned, so that a
 // fragment's eight keys are the eight that a lane holds weights of), and the weights are split in place.  Returns true, and has
 // stored nothing, if a value lies at the ends of the range that pieces cover; !PIECES: the 32-bit instructions.
-// Measured, 32-bit instructions -> pieces: 4 x 2048 tokens, 32 heads of 64 over 8 KV heads 626 -> 427 us (159 TFLOP/s of the visible
-// half); 1024 tokens, 16 heads of 128 over 8 85 -> 75; 512 tokens, 9 heads of 64 over 3 19.6 -> 16.4; 4 x 8 tokens 12.7 -> 12.9.  The
+// Measured, 32-bit instructions -> pieces: 4 x 2048 tokens, 32 heads of 64 over 8 KV heads 626 -> 433 us (159 TFLOP/s of the visible
+// half); 1024 tokens, 16 heads of 128 over 8 85 -> 78; 512 tokens, 9 heads of 64 over 3 19.6 -> 17.0; 4 x 8 tokens 12.7 -> 12.9.  The
 // products are no longer what bounds it alone: splitting K, V and the weights, the exponentials and the two barriers of a tile weigh as
-// much.  Error against 64 bits: no larger (a sum is rounded once per 16 terms and piece).
+// much.  Error against 64 bits: 4.0e-7 -> 2.1e-7 (the first of these).  With a value beyond the range in every head both ways are run:
+// the whole call of the first 666 -> 841 us (442 without such a value), of the second 95 -> 110.
 template <int HD, bool PIECES> __device__ __forceinline__ bool prefill_rows(const AttnArgs &g, const PrefillArgs &e, float *const pf_lds) {
     static_assert(HD == 64 || HD == 128, "head_dim 64 or 128");
     constexpr int KEYS = PIECES && HD == 128 ? 32 : kPfKeys; // per tile

@@ -10,10 +10,13 @@
 //
 // Kernels
 //   split_gemm_kernel  (split_gemm.hip) every f32 product of more than eight rows.
-//   mfma_gemm_kernel   products of the narrow dtypes: 256 threads = 2x2 waves, 128x128x32 macro tiles (2x2 32x32
-//                      accumulators per wave) or, with at least one such tile per compute unit, 256x256x32
-//                      (each wave a 128x128 block as 4x4 accumulators, all 256 accumulation registers, 144 KiB
-//                      of LDS).  Tiles of words are narrowed to bf16 / f16 on their way into LDS (fp8 words to
+//   narrow_tile_kernel (block_products.hip) products of the narrow dtypes with an operand that lies in memory as
+//                      patterns, on 128-wide tiles (narrow_route.hpp decides).
+//   mfma_gemm_kernel   the other products of the narrow dtypes: 256 threads = 2x2 waves, 128x128x32 macro tiles (2x2
+//                      32x32 accumulators per wave) or, with enough of them (one per two compute units for the 16-bit
+//                      dtypes, one per unit for fp8), 256x256x32 (each wave a 128x128 block as 4x4 accumulators, all 256
+//                      accumulation registers, 144 KiB of LDS), fed by loads straight into LDS where k is whole turns
+//                      of the ring (mfma_gemm_dlds_kernel).  Tiles of words are narrowed to bf16 / f16 on their way into LDS (fp8 words to
 //                      bf16, which holds them exactly), or operands lie narrow in memory (pack_operand_kernel);
 //                      v_mfma_f32_32x32x16_{bf16,f16} / v_mfma_scale_f32_32x32x64_f8f6f4.  Staged K-fastest in
 //                      LDS; whole tiles are loaded at fixed per-lane offsets without tests; two LDS buffers,
@@ -191,9 +194,10 @@ template <bool ROWS_FAST, int HALF, int TR> __device__ __forceinline__ void stor
 // barriers and half the LDS traffic per flop, for products with enough tiles to fill the chip.
 // HALF: 1 / 2: words that are bfloat16 / binary16 values (see above; fp8 values are bfloat16 values too).
 // 3 / 4 / 5: operands that are ALREADY narrow in memory — bfloat16 / binary16 / fp8 (E4M3) patterns, k contiguous,
-// addressed as 32-bit words of 2 or 4 values (a.K counts words; see pack_operand): (16-byte global loads, K-fastest LDS rows of 32 words + 4, one 128-bit LDS read per fragment); a
-// fragment then is 8 (16) consecutive k of a row and feeds one v_mfma_f32_32x32x16_{bf16,f16} (two
-// v_mfma_f32_32x32x16_fp8_fp8): a tile is 64 (128) deep in k, and half (a quarter) of the bytes move per flop.
+// addressed as 32-bit words of 2 or 4 values (a.K counts words; see pack_operand).  The tiles are loaded and staged as words
+// (16-byte loads, K-fastest LDS rows of 32 words + 4, one 128-bit LDS read per fragment); a fragment then is 8 (16) consecutive k of
+// a row and feeds one v_mfma_f32_32x32x16_{bf16,f16} (two v_mfma_f32_32x32x16_fp8_fp8): a tile is 64 (128) deep in k, and half (a
+// quarter) of the bytes move per flop.
 template <bool A_MFAST, bool B_NFAST, int NT, int MT, int HALF>
 __global__ __launch_bounds__(kThreads) void mfma_gemm_kernel(const MmArgs a) {
     constexpr int BN = 64 * NT, BM = 64 * MT; // shadow the defaults
@@ -1387,11 +1391,12 @@ template <int MM, int TRIPS = 8>
 __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_residual_kernel(const MmArgs a, const MmResidual r) {
     skinny_kt_mfma_xreg_body<MM, 1, false, true, false, TRIPS>(a, blockIdx.x, blockIdx.y, nullptr, 0, &r);
 }
-// the same with the RMS norm of the left operand applied on load
 // The same sum with residual terms for up to four rows, eight columns and all of K by eight waves: an eighth of a chunk of K each,
 // every load of a chunk asked for before the first product.  The kernel above fetches as many bytes of activations as of weights
 // (four columns per workgroup), and a compute unit's path to L2 bounds it; here the activations are half of the weights' bytes.
-// 4 x 8192 x 2048 (64 MiB of weights): 17.2 us above, 15.9 here; 4 x 2048 x 2048: 6.5 and 6.2.
+// 4 x 8192 x 2048 (64 MiB of weights): 17.2 us above, 15.9 here; 4 x 2048 x 2048: 6.5 and 6.2.  With an arg-max of the sum behind
+// both: 4 x 4096 x 2048 24.8 and 24.4, 4 x 6144 x 2048 28.4 and 27.9, 4 x 16384 x 2048 45.8 and 45.4; from 3072 columns on
+// equal within 1 %.
 constexpr int kEightThreads = 512;
 template <int TRIPS> __global__ __launch_bounds__(kEightThreads, 2) void skinny_kt_mfma_eight_residual_kernel(const MmArgs a, const MmResidual res) {
     const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 4, b = lane / 4;
@@ -1454,6 +1459,7 @@ static inline int eight_trips(const cg_backend *be, uint32_t M, uint32_t N, uint
     if (M > 4 || (uint64_t)N < 8ull * be->compute_units) return 0;
     return K % 8192 == 0 ? 16 : K % 4096 == 0 ? 8 : K % 2048 == 0 ? 4 : 0;
 }
+// the gated pair with the RMS norm of the left operand applied on load
 template <int TRIPS = 8>
 __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_gated_norm_kernel(const MmArgs a, const uint32_t *second, uint32_t one,
                                                                                   const NormFuse nf) {
@@ -1869,7 +1875,7 @@ __global__ __launch_bounds__(kThreads) void skinny_nn_kernel(const MmArgs a, uin
     }
 }
 
-// The same four elements at a time (mn a multiple of 4, both arrays 16-byte aligned): the sums in the same fixed order.
+// C[b][e] = sum over s of part[b][s][e]   (e < M*N), in a fixed order
 __global__ __launch_bounds__(kThreads) void splitk_reduce_kernel(const uint32_t *part, uint32_t *C, uint32_t splits,
                                                                  uint32_t mn, uint64_t total) {
     uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x;

@@ -3,9 +3,11 @@
 // 8192 x 2048 x 8192: 1250 us = 220 TFLOP/s, where the 32-bit instructions took 1990 us = 138 (88 % of their peak); 1024 x 1024 x
 // 3072: 53 against 74 us; 32 x 2048 x 8192: 22 against 46 us.  A few small shapes stay above the 32-bit instructions, whose tiles
 // started sooner: with contiguous rows 100 x 576 x 1536 13.1 against 10.7, 4096 x 700 x 50 18.8 against 14.7 and 100 x 64 x 1024 6.6
-// against 5.3; 333 x 1001 x 333 16.4 against 15.5.  The wide tile is bound by the clock at the card's power limit, so what it saves
-// elsewhere comes back as clock: eight waves that share one 256 x 256 tile split a third less than two workgroups of four with
-// 256 x 128 each and run 8 % faster.  Splitting by v_dot2c_f32_bf16 (one instruction for the shift and the subtraction): slower.
+// against 5.3; 333 x 1001 x 333 16.4 against 15.5.  The wide tile is bound by issuing: matrix pipes busy 66 % of the
+// cycles at 1.77 GHz (64 SQ_VALU_MFMA_BUSY_CYCLES per instruction pair and GRBM_GUI_ACTIVE over the time); with one chain over all of
+// k, without the additions of the chains' sums, 76 % at 1.74 GHz and 1150 us, but with sums off to one side.  Eight waves that share one
+// 256 x 256 tile split a third less than two workgroups of four with 256 x 128 each and run 8 % faster.  Splitting by
+// v_dot2c_f32_bf16 (one instruction for the shift and the subtraction): slower.
 #include "gemm_args.hpp"
 #include "split_tile.hpp"
 
