@@ -529,6 +529,48 @@ def _():
     return run, expect
 
 
+@case("kv_cache_growth_from_few_tokens")
+def _():
+    """The same from one to five tokens on (each number its own cache): a token at a time, more tokens than the room that a
+    small cache's store is given at first, two tokens at once in between, a fork of an earlier cache, and a cache of one
+    sequence and head beside them."""
+    L, D = 2, 16
+    shapes = [(2, 2, 1), (1, 3, 2), (2, 1, 3), (1, 1, 1), (2, 2, 5)]
+    steps = [1] * 3 + [2] + [1] * 70
+    bases = [f32(140 + i, (L, B, H, T, D)) for i, (B, H, T) in enumerate(shapes)]
+    news = [[f32(150 + 7 * i + s, (L, B, H, n, D)) for s, n in enumerate(steps)] for i, (B, H, _) in enumerate(shapes)]
+
+    def run(be):
+        outs = []
+        for (B, H, _), base, new in zip(shapes, bases, news):
+            cache, old = be.from_numpy(base), None
+            for s, rows in enumerate(new):
+                layers = []
+                for l in range(L):
+                    c = be.reshape(be.slice(cache, 0, l, 1).move(), (B, H, cache.shape[3], D))
+                    if s == 1 and l == 1:
+                        outs.append(be.to_numpy(be.concat(c, be.from_numpy(-rows[l]).move(), 2)))
+                    layers.append(be.concat(c.move(), be.from_numpy(rows[l]).move(), 2))
+                shp = (1, B, H, layers[0].shape[2], D)
+                out = be.reshape(layers[0].move(), shp)
+                for l in range(1, L):
+                    out = be.concat(out.move(), be.reshape(layers[l].move(), shp).move(), 0)
+                if s == 2:
+                    old = cache.clone()
+                cache = out
+            outs += [be.to_numpy(old), be.to_numpy(cache)]
+        return outs
+
+    def expect():
+        outs = []
+        for base, new in zip(bases, news):
+            upto = [np.concatenate([base] + new[:s], 3) for s in range(len(steps) + 1)]
+            outs += [np.concatenate([upto[1][1], -new[1][1]], 2), upto[2], upto[-1]]
+        return outs
+
+    return run, expect
+
+
 @case("kv_deferred_row_writes", "red")
 def _():
     """Rows appended to a cache from element-wise programs (as the rotary embedding of k is) may be written
