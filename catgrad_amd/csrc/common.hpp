@@ -215,12 +215,12 @@ struct Buffer : Pooled<Buffer> {
     RowStore *rs = nullptr;      // owned
     bool constant = false;       // the contents depend on constants only (iota, programs over such buffers)
     Buffer *successor = nullptr; // retained: the roomier buffer that blocks of this one migrate to on append
-    // Set by the product kernels that store a residual stream [rows <= 4, N]: per workgroup (4 columns) and row
-    // the sum of squares of what it stored, [side_blocks][4] floats.  An RMS norm over these rows that feeds
+    // Set by the product kernels that store a residual stream [rows <= 8, N]: per group of 4 columns and row
+    // the sum of squares of what was stored there, [side_blocks][side_rows] floats (4 for up to four rows, else 8).  An RMS norm over these rows that feeds
     // decode-time products needs no pass of its own then (see NormFuse).  Owned (pool memory).
     void *side = nullptr;
     size_t side_cls = 0;
-    uint32_t side_blocks = 0;
+    uint32_t side_blocks = 0, side_rows = 0;
     // Narrow copies of 2-D views of this buffer for the matrix instructions of its dtype (launch_matmul): [rows][k] of
     // 2-byte (f16 / bf16) or 1-byte (fp8) patterns, k contiguous, one entry per view (several slices of one weight buffer
     // each keep theirs; the oldest goes when the list is full).  A weight matrix is narrowed once and the copy kept while
@@ -407,7 +407,7 @@ struct DeferredWrite {
 // x / pow(sum(x*x) / n + eps, e) * gamma applied to the left operand while a decode-time product loads it:
 // the row sums come from the per-workgroup partial sums that the kernel which stored x left behind.
 struct NormFuse {
-    const float *partials; // [blocks][4]
+    const float *partials; // [blocks][4], [blocks][8] for more than four rows
     uint32_t blocks;
     const uint32_t *gamma; // [K]
     uint32_t n_bits, eps_bits, exp_bits;
@@ -598,7 +598,7 @@ struct MmFold {
 int fold_matmul(const cg_tensor *x, const cg_tensor *y, MmFold *f);
 // Several skinny products x . ys[i] -> outs[i] (n of them, the same x) in one launch; kDeclined (declared
 // below) when the shapes do not allow it.
-// nf != null: x is the residual stream and the kernel applies the RMS norm to it on load (needs M <= 4 and K a
+// nf != null: x is the residual stream and the kernel applies the RMS norm to it on load (needs M <= 8 and K a
 // multiple of 2048; kDeclined otherwise, before anything is launched).
 int launch_matmul_gated(cg_backend *be, const cg_tensor *x, const cg_tensor *yg, const cg_tensor *yu, uint32_t one,
                         cg_tensor *out, const NormFuse *nf = nullptr);

@@ -27,7 +27,7 @@
 //                      skinny_kt_wide / _narrow: a wave per output column (or per 4 columns, or a
 //                      column per 16/32 lanes for short K), 16-byte loads along K, wave shuffle
 //                      reduction;
-//                      skinny_kt_mfma_xreg_*: M <= 4 on the 4x4x1 matrix instruction with the
+//                      skinny_kt_mfma_xreg_*: M <= 8 on the 4x4x1 matrix instruction with the
 //                      activations held in registers, in the variants the decode step needs:
 //                      _group (products that share their left operand in one launch), _group_rope
 //                      (the same with the rotary embedding and the KV-cache row writes in the
@@ -1015,7 +1015,7 @@ struct MmResidual {
     const uint32_t *term[4];
     uint32_t slot, order;
     uint32_t nterms;  // 4, or 2: out = t0 + t1
-    float *partials;  // null, or [workgroups][4]: per row the sum of squares of the four columns stored
+    float *partials;  // null, or [groups of four columns][4 or 8 rows]: per row the sum of squares of the four columns stored
 };
 // the sum, given all its terms
 __device__ __forceinline__ uint32_t residual_sum(const MmResidual &r, const uint32_t (&t)[4]) {
@@ -1155,7 +1155,11 @@ static inline uint32_t xreg_cols_iters(uint64_t groups) {
     const uint64_t it = groups / 512;
     return (uint32_t)(it < 1 ? 1 : it > 4 ? 4 : it);
 }
-static inline bool xreg_narrow(uint32_t M, uint32_t K) { return M >= 1 && M <= 4 && xreg_trips(K) != 0; }
+// Five to eight rows run on the same kernels with a second group of four rows: two activation loads and eight matrix
+// instructions per weight load instead of one and four.  Against the vector-unit kernels without the norms, gates and cache rows in
+// their loads and stores (up to 14 launches a layer instead of 5): Llama-3.2-1B shape, six sequences 2.44 -> 1.67 ms a step; SmolLM2-135M
+// shape, eight 1.93 -> 1.27; Qwen3-0.6B shape, five 2.8 -> 2.2.
+static inline bool xreg_narrow(uint32_t M, uint32_t K) { return M >= 1 && M <= 8 && xreg_trips(K) != 0; }
 constexpr int kMaxGroup = 4;
 struct MmGroup {
     MmArgs p[kMaxGroup];
@@ -1209,7 +1213,7 @@ template <int TRIPS, bool WHOLE = false> __device__ __forceinline__ void xreg_la
 template <bool WHOLE, int MM, int CG, bool GATED, bool RESIDUAL, bool NORM, int TRIPS>
 __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, const uint32_t block_x, const uint32_t block_y, const uint32_t *second,
                                                               const uint32_t one, const MmResidual *res, const NormFuse *nf) {
-    static_assert(!NORM || MM == 4, "the norm's row sums are kept for four rows");
+    static_assert(MM == 4 || MM == 8, "one or two groups of four rows");
     static_assert(!GATED || CG == 2, "a gated pair is two column groups");
     static_assert(!(GATED && RESIDUAL), "one epilogue at a time");
     constexpr int G = MM / 4;
@@ -1246,14 +1250,14 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
     }
     // NORM: the products are taken of x * gamma and divided by d_m = pow(sum(x[m]^2) / n + eps, e) where they are stored:
     // (x / d * gamma) . w = ((x * gamma) . w) / d.  The row sums are put together from the partial sums that the kernel
-    // which stored x left (always in the same order); thread t takes entries t, t + 256, ... of [blocks][4], all of row
-    // t % 4.  The first eight per thread are asked for here and added up after the walk along K: nothing waits for them.
-    float pv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    // which stored x left (always in the same order); thread t takes entries t, t + 256, ... of [blocks][MM], all of row
+    // t % MM.  The first 512 blocks' are asked for here and added up after the walk along K: nothing waits for them.
+    float pv[NORM ? 2 * MM : 1] = {};
     if constexpr (NORM) {
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
+        for (int u = 0; u < 2 * MM; u++) {
             const uint32_t i = threadIdx.x + u * kThreads;
-            if (i < nf->blocks * 4) pv[u] = nf->partials[i];
+            if (i < nf->blocks * MM) pv[u] = nf->partials[i];
         }
     }
     // of every chunk of TRIPS * 256 values of k (2048 or 1024) a wave takes a quarter in a row (TRIPS trips of 64)
@@ -1311,15 +1315,15 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
         }
     }
     __shared__ float part[4][CG * MM * 4];
-    __shared__ float nsum[4][4];
+    __shared__ float nsum[4][MM];
     if constexpr (NORM) {
         float s = 0.0f;
 #pragma unroll
-        for (int u = 0; u < 8; u++) s += pv[u];
-        for (uint32_t i = threadIdx.x + 8 * kThreads; i < nf->blocks * 4; i += kThreads) s += nf->partials[i];
+        for (int u = 0; u < 2 * MM; u++) s += pv[u];
+        for (uint32_t i = threadIdx.x + 2 * MM * kThreads; i < nf->blocks * MM; i += kThreads) s += nf->partials[i];
 #pragma unroll
-        for (int sh = 32; sh >= 4; sh >>= 1) s += __shfl_xor(s, sh);
-        if (lane < 4) nsum[wave][lane] = s;
+        for (int sh = 32; sh >= MM; sh >>= 1) s += __shfl_xor(s, sh);
+        if (lane < MM) nsum[wave][lane] = s;
     }
 #pragma unroll
     for (int c = 0; c < CG; c++)
@@ -1339,7 +1343,7 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
             uint32_t gv = asu((part[0][t] + part[1][t]) + (part[2][t] + part[3][t]));
             uint32_t uv = asu((part[0][u_at] + part[1][u_at]) + (part[2][u_at] + part[3][u_at]));
             if constexpr (NORM) {
-                const uint32_t d = norm_divisor(*nf, (nsum[0][m % 4] + nsum[1][m % 4]) + (nsum[2][m % 4] + nsum[3][m % 4]));
+                const uint32_t d = norm_divisor(*nf, (nsum[0][m] + nsum[1][m]) + (nsum[2][m] + nsum[3][m]));
                 gv = apply<kDiv, true>(gv, d, 0, nullptr);
                 uv = apply<kDiv, true>(uv, d, 0, nullptr);
             }
@@ -1353,7 +1357,7 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
         const uint32_t c = threadIdx.x / (MM * 4), m = threadIdx.x / 4 % MM, col = n0 + 4 * c + threadIdx.x % 4;
         uint32_t v = asu((part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]));
         if constexpr (NORM)
-            v = apply<kDiv, true>(v, norm_divisor(*nf, (nsum[0][m % 4] + nsum[1][m % 4]) + (nsum[2][m % 4] + nsum[3][m % 4])), 0, nullptr);
+            v = apply<kDiv, true>(v, norm_divisor(*nf, (nsum[0][m] + nsum[1][m]) + (nsum[2][m] + nsum[3][m])), 0, nullptr);
         if constexpr (RESIDUAL) {
 #pragma unroll
             for (int t = 0; t < 4; t++) term[t] = (uint32_t)t == res->slot ? v : term[t];
@@ -1362,12 +1366,12 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
         const bool stored = col < a.N && m < a.M;
         if (stored) a.C[((uint64_t)block_y * a.M + m) * a.N + col] = v;
         if constexpr (RESIDUAL) {
-            // threads 0..15 = (row m, column n0 + t % 4): the row's sum of squares over the block's four columns
+            // threads 0 .. 4 MM - 1 = (row m, column n0 + t % 4): the row's sum of squares over the block's four columns
             if (res->partials) {
                 float q = stored ? asf(v) * asf(v) : 0.0f;
                 q += __shfl_xor(q, 1);
                 q += __shfl_xor(q, 2);
-                if (threadIdx.x % 4 == 0) res->partials[(uint64_t)block_x * 4 + m] = q;
+                if (threadIdx.x % 4 == 0) res->partials[(uint64_t)block_x * MM + m] = q;
             }
         }
     }
@@ -1398,28 +1402,33 @@ __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_residual_kernel(
 // both: 4 x 4096 x 2048 24.8 and 24.4, 4 x 6144 x 2048 28.4 and 27.9, 4 x 16384 x 2048 45.8 and 45.4; from 3072 columns on
 // equal within 1 %.
 constexpr int kEightThreads = 512;
-template <int TRIPS> __global__ __launch_bounds__(kEightThreads, 2) void skinny_kt_mfma_eight_residual_kernel(const MmArgs a, const MmResidual res) {
+template <int MM, int TRIPS>
+__global__ __launch_bounds__(kEightThreads, 2) void skinny_kt_mfma_eight_residual_kernel(const MmArgs a, const MmResidual res) {
     const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 4, b = lane / 4;
     const uint32_t n0 = blockIdx.x * 8;
     const uint32_t *const w0 = a.B + (int64_t)min(n0 + j, a.N - 1) * a.b_sn, *const w1 = a.B + (int64_t)min(n0 + 4 + j, a.N - 1) * a.b_sn;
-    const uint32_t *const x = a.A + (int64_t)min(j, a.M - 1) * a.a_sm;
+    constexpr int G = MM / 4, kOut = 8 * MM; // row groups; values of the workgroup's result
+    const uint32_t *x[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) x[g] = a.A + (int64_t)min((uint32_t)(4 * g) + j, a.M - 1) * a.a_sm;
     // the sum's other terms for the value this thread will store
-    const uint32_t tc = threadIdx.x / 16, tm = threadIdx.x / 4 % 4, tcol = n0 + 4 * tc + threadIdx.x % 4;
-    const bool stored = threadIdx.x < 32 && tcol < a.N && tm < a.M;
+    const uint32_t tc = threadIdx.x / (4 * MM), tm = threadIdx.x / 4 % MM, tcol = n0 + 4 * tc + threadIdx.x % 4;
+    const bool stored = threadIdx.x < kOut && tcol < a.N && tm < a.M;
     uint32_t term[4] = {};
     if (stored) {
 #pragma unroll
         for (int t = 0; t < 4; t++)
             if ((uint32_t)t != res.slot && (uint32_t)t < res.nterms) term[t] = res.term[t][(uint64_t)tm * a.N + tcol];
     }
-    float4v acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    float4v acc[2][G] = {};
     for (uint32_t k0 = wave * (TRIPS * 64) + b * 4; k0 < a.K; k0 += TRIPS * kEightThreads) { // (K: whole chunks)
-        float4v xr[TRIPS], wr[2][TRIPS];
+        float4v xr[G][TRIPS], wr[2][TRIPS];
 #pragma unroll
         for (int t = 0; t < TRIPS; t++) {
             wr[0][t] = *reinterpret_cast<const float4v *>(w0 + k0 + 64 * t);
             wr[1][t] = *reinterpret_cast<const float4v *>(w1 + k0 + 64 * t);
-            xr[t] = *reinterpret_cast<const float4v *>(x + k0 + 64 * t);
+#pragma unroll
+            for (int g = 0; g < G; g++) xr[g][t] = *reinterpret_cast<const float4v *>(x[g] + k0 + 64 * t);
         }
         __builtin_amdgcn_sched_barrier(0); // (or the compiler asks for a few at a time)
 #pragma unroll
@@ -1427,20 +1436,22 @@ template <int TRIPS> __global__ __launch_bounds__(kEightThreads, 2) void skinny_
 #pragma unroll
             for (int e = 0; e < 4; e++)
 #pragma unroll
-                for (int c = 0; c < 2; c++) acc[c] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[t][e], wr[c][t][e], acc[c], 0, 0, 0);
+                for (int c = 0; c < 2; c++)
+#pragma unroll
+                    for (int g = 0; g < G; g++) acc[c][g] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[g][t][e], wr[c][t][e], acc[c][g], 0, 0, 0);
     }
-    __shared__ float part[8][32];
+    __shared__ float part[8][kOut];
 #pragma unroll
     for (int c = 0; c < 2; c++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float v = acc[c][i];
+        for (int i = 0; i < MM; i++) {
+            float v = acc[c][i / 4][i % 4];
 #pragma unroll
             for (int s = 32; s >= 4; s >>= 1) v += __shfl_xor(v, s);
-            if (lane < 4) part[wave][c * 16 + i * 4 + j] = v;
+            if (lane < 4) part[wave][(c * MM + i) * 4 + j] = v;
         }
     __syncthreads();
-    if (threadIdx.x >= 32) return;
+    if (threadIdx.x >= kOut) return;
     const uint32_t t = threadIdx.x;
     uint32_t v = asu(((part[0][t] + part[1][t]) + (part[2][t] + part[3][t])) + ((part[4][t] + part[5][t]) + (part[6][t] + part[7][t])));
 #pragma unroll
@@ -1451,42 +1462,42 @@ template <int TRIPS> __global__ __launch_bounds__(kEightThreads, 2) void skinny_
         float q = stored ? asf(v) * asf(v) : 0.0f;
         q += __shfl_xor(q, 1);
         q += __shfl_xor(q, 2);
-        if (t % 4 == 0 && n0 + 4 * tc < a.N) res.partials[((uint64_t)blockIdx.x * 2 + tc) * 4 + tm] = q;
+        if (t % 4 == 0 && n0 + 4 * tc < a.N) res.partials[((uint64_t)blockIdx.x * 2 + tc) * MM + tm] = q;
     }
 }
 // trips of 64 values of k per wave and chunk; 0: K is not whole chunks, or there are too few columns for a workgroup per compute unit
 static inline int eight_trips(const cg_backend *be, uint32_t M, uint32_t N, uint32_t K) {
-    if (M > 4 || (uint64_t)N < 8ull * be->compute_units) return 0;
-    return K % 8192 == 0 ? 16 : K % 4096 == 0 ? 8 : K % 2048 == 0 ? 4 : 0;
+    if (M > 8 || (uint64_t)N < 8ull * be->compute_units) return 0;
+    return K % 8192 == 0 && M <= 4 ? 16 : K % 4096 == 0 ? 8 : K % 2048 == 0 ? 4 : 0; // (16 trips of eight rows: more registers than there are)
 }
 // the gated pair with the RMS norm of the left operand applied on load
-template <int TRIPS = 8>
+template <int MM, int TRIPS = 8>
 __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_gated_norm_kernel(const MmArgs a, const uint32_t *second, uint32_t one,
                                                                                   const NormFuse nf) {
-    skinny_kt_mfma_xreg_body<4, 2, true, false, true, TRIPS>(a, blockIdx.x, blockIdx.y, second, one, nullptr, &nf);
+    skinny_kt_mfma_xreg_body<MM, 2, true, false, true, TRIPS>(a, blockIdx.x, blockIdx.y, second, one, nullptr, &nf);
 }
 template <int MM, int CG, int TRIPS = 8> __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_group_kernel(const MmGroup g) {
     uint32_t bx;
     const uint32_t p = group_problem(g, bx);
     skinny_kt_mfma_xreg_body<MM, CG, false, false, false, TRIPS>(g.p[p], bx, 0);
 }
-template <int TRIPS = 8>
+template <int MM, int TRIPS = 8>
 __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_group_norm_kernel(const MmGroup g, const NormFuse nf) {
     uint32_t bx;
     const uint32_t p = group_problem(g, bx);
-    skinny_kt_mfma_xreg_body<4, 1, false, false, true, TRIPS>(g.p[p], bx, 0, nullptr, 0, nullptr, &nf);
+    skinny_kt_mfma_xreg_body<MM, 1, false, false, true, TRIPS>(g.p[p], bx, 0, nullptr, 0, nullptr, &nf);
 }
 
 // The grouped products of an attention block's decode step (q, k, v: a few rows, the same left operand) with the
 // rotary embedding and the move into the KV cache done where they are stored: a workgroup owns two groups of four
 // columns half a head apart (the pair the embedding mixes; next to each other for a product stored as it is) and
 // writes column n = head * hd + d of row m to dst[m * sb + head * sh + d] (see RopeStore).  The embedding's ops are
-// those of the deferred program cos * x + sin * concat(-x2, x1), in its order.  M <= 4, K a multiple of TRIPS * 256,
+// those of the deferred program cos * x + sin * concat(-x2, x1), in its order.  M <= MM, K a multiple of TRIPS * 256,
 // N a multiple of hd (of 8 without the embedding).
 struct RopeGroup {
     RopeStore s[kMaxGroup];
 };
-template <bool WHOLE, bool NORM, int TRIPS>
+template <bool WHOLE, int MM, bool NORM, int TRIPS>
 __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGroup &g, const RopeGroup &rg, const NormFuse &nf) {
     static_assert(TRIPS == 8 || TRIPS == 4, "chunks of 2048 or 1024");
     uint32_t bx;
@@ -1501,21 +1512,24 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGrou
     const uint32_t *wrow[2];
 #pragma unroll
     for (int c = 0; c < 2; c++) wrow[c] = a.B + (int64_t)min(nc[c] + j, a.N - 1) * a.b_sn;
-    const uint32_t *xrow = a.A + (int64_t)min(j, a.M - 1) * a.a_sm;
-    float4v acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    constexpr int G = MM / 4, kOut = 8 * MM; // row groups; values of the workgroup's result: at most a wave's lanes
+    const uint32_t *xrow[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) xrow[g] = a.A + (int64_t)min((uint32_t)(4 * g) + j, a.M - 1) * a.a_sm;
+    float4v acc[2][G] = {};
     // the embedding's factors for the value this thread will store: asked for before the walk along K
     uint32_t cs = 0, sn = 0;
-    if (rs.rope && threadIdx.x < 32) {
-        const uint32_t d = (nc[threadIdx.x / 16] + threadIdx.x % 4) % rs.hd;
+    if (rs.rope && threadIdx.x < kOut) {
+        const uint32_t d = (nc[threadIdx.x / (4 * MM)] + threadIdx.x % 4) % rs.hd;
         cs = rs.cos[d];
         sn = rs.sin[d];
     }
-    float pv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float pv[NORM ? 2 * MM : 1] = {};
     if constexpr (NORM) {
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
+        for (int u = 0; u < 2 * MM; u++) {
             const uint32_t i = threadIdx.x + u * kThreads;
-            if (i < nf.blocks * 4) pv[u] = nf.partials[i];
+            if (i < nf.blocks * MM) pv[u] = nf.partials[i];
         }
     }
     uint32_t kb, ks;
@@ -1527,9 +1541,11 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGrou
         return v;
     };
     for (uint32_t k0 = 0; k0 < a.K; k0 += TRIPS * 256) {
-        float4v xr[TRIPS];
+        float4v xr[G][TRIPS];
 #pragma unroll
-        for (int t = 0; t < TRIPS; t++) xr[t] = at(xrow, k0 + kb + ks * t);
+        for (int t = 0; t < TRIPS; t++)
+#pragma unroll
+            for (int g = 0; g < G; g++) xr[g][t] = at(xrow[g], k0 + kb + ks * t);
         float4v gm[NORM ? TRIPS : 1];
         if constexpr (NORM) {
 #pragma unroll
@@ -1545,56 +1561,57 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGrou
 #pragma unroll
                     for (int t = 0; t < TRIPS; t++)
 #pragma unroll
-                        for (int e = 0; e < 4; e++) xr[t][e] = asf(apply<kMul, true>(asu(xr[t][e]), asu(gm[t][e]), 0, nullptr));
+                        for (int g = 0; g < G; g++)
+#pragma unroll
+                            for (int e = 0; e < 4; e++) xr[g][t][e] = asf(apply<kMul, true>(asu(xr[g][t][e]), asu(gm[t][e]), 0, nullptr));
                 }
             }
 #pragma unroll
-            for (int t = 0; t < TRIPS; t++) {
-                acc[c] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[t][0], w[t][0], acc[c], 0, 0, 0);
-                acc[c] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[t][1], w[t][1], acc[c], 0, 0, 0);
-                acc[c] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[t][2], w[t][2], acc[c], 0, 0, 0);
-                acc[c] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[t][3], w[t][3], acc[c], 0, 0, 0);
-            }
+            for (int t = 0; t < TRIPS; t++)
+#pragma unroll
+                for (int g = 0; g < G; g++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[c][g] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[g][t][e], w[t][e], acc[c][g], 0, 0, 0);
         }
     }
-    __shared__ float part[4][32];
-    __shared__ float nsum[4][4];
+    __shared__ float part[4][kOut];
+    __shared__ float nsum[4][MM];
     if constexpr (NORM) {
         float s = 0.0f;
 #pragma unroll
-        for (int u = 0; u < 8; u++) s += pv[u];
-        for (uint32_t i = threadIdx.x + 8 * kThreads; i < nf.blocks * 4; i += kThreads) s += nf.partials[i];
+        for (int u = 0; u < 2 * MM; u++) s += pv[u];
+        for (uint32_t i = threadIdx.x + 2 * MM * kThreads; i < nf.blocks * MM; i += kThreads) s += nf.partials[i];
 #pragma unroll
-        for (int sh = 32; sh >= 4; sh >>= 1) s += __shfl_xor(s, sh);
-        if (lane < 4) nsum[wave][lane] = s;
+        for (int sh = 32; sh >= MM; sh >>= 1) s += __shfl_xor(s, sh);
+        if (lane < MM) nsum[wave][lane] = s;
     }
 #pragma unroll
     for (int c = 0; c < 2; c++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float v = acc[c][i];
+        for (int i = 0; i < MM; i++) {
+            float v = acc[c][i / 4][i % 4];
 #pragma unroll
             for (int s = 32; s >= 4; s >>= 1) v += __shfl_xor(v, s);
-            if (lane < 4) part[wave][(c * 4 + i) * 4 + j] = v;
+            if (lane < 4) part[wave][(c * MM + i) * 4 + j] = v;
         }
     __syncthreads();
-    if (threadIdx.x < 64) { // the first wave: lanes 0..31 hold (column group, row, column), the others idle along
-        const uint32_t t = threadIdx.x % 32, c = t / 16, m = t / 4 % 4, col = nc[c] + t % 4;
+    if (threadIdx.x < 64) { // the first wave: lanes 0 .. kOut - 1 hold (column group, row, column), any others idle along
+        const uint32_t t = threadIdx.x % kOut, c = t / (4 * MM), m = t / 4 % MM, col = nc[c] + t % 4;
         uint32_t v = asu((part[0][t] + part[1][t]) + (part[2][t] + part[3][t]));
         if constexpr (NORM) v = apply<kDiv, true>(v, norm_divisor(nf, (nsum[0][m] + nsum[1][m]) + (nsum[2][m] + nsum[3][m])), 0, nullptr);
-        const uint32_t other = __shfl_xor(v, 16); // the same row's column half a head away
+        const uint32_t other = __shfl_xor(v, 4 * MM); // the same row's column half a head away
         if (rs.rope) {
             // lower half: rotate_half reads -x[d + hd / 2]; upper half: x[d - hd / 2]
             const uint32_t rot = c == 0 ? apply<kNeg, true>(other, 0, 0, nullptr) : other;
             v = apply<kAdd, true>(apply<kMul, true>(cs, v, 0, nullptr), apply<kMul, true>(sn, rot, 0, nullptr), 0, nullptr);
         }
-        if (threadIdx.x < 32 && col < a.N && m < a.M) rs.dst[(int64_t)m * rs.sb + (int64_t)(col / rs.hd) * rs.sh + col % rs.hd] = v;
+        if (threadIdx.x < kOut && col < a.N && m < a.M) rs.dst[(int64_t)m * rs.sb + (int64_t)(col / rs.hd) * rs.sh + col % rs.hd] = v;
     }
 }
-template <bool NORM, int TRIPS>
+template <int MM, bool NORM, int TRIPS>
 __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_group_rope_kernel(const MmGroup g, const RopeGroup rg, const NormFuse nf) {
-    if (g.p[0].K % (TRIPS * 256) == 0) skinny_kt_mfma_xreg_group_rope_impl<true, NORM, TRIPS>(g, rg, nf); // (the problems of a group share k)
-    else skinny_kt_mfma_xreg_group_rope_impl<false, NORM, TRIPS>(g, rg, nf);
+    if (g.p[0].K % (TRIPS * 256) == 0) skinny_kt_mfma_xreg_group_rope_impl<true, MM, NORM, TRIPS>(g, rg, nf); // (the problems of a group share k)
+    else skinny_kt_mfma_xreg_group_rope_impl<false, MM, NORM, TRIPS>(g, rg, nf);
 }
 
 // The store above for products whose heads go through an RMS norm of their own first (RopeStore::hgamma, the q / k norm of
@@ -1613,14 +1630,14 @@ struct HeadFinish {
     uint32_t first[kMaxGroup + 1]; // prefix sums of the products' head counts
     uint32_t n, M;
 };
-constexpr int kFinishThreads = 512;
+constexpr int kFinishThreads = 1024;
 __global__ __launch_bounds__(kFinishThreads) void head_norm_rope_finish_kernel(const HeadFinish f) {
     uint32_t p = 0;
     while (p + 1 < f.n && blockIdx.x >= f.first[p + 1]) p++;
     const uint32_t head = blockIdx.x - f.first[p];
     const RopeStore &rs = f.s[p];
     const uint32_t e = threadIdx.x, m = e / rs.hd, d = e % rs.hd;
-    const bool mine = e < f.M * rs.hd; // (M <= 4, hd <= 128: at most 512 threads)
+    const bool mine = e < f.M * rs.hd; // (M <= 8, hd <= 128: at most 1024 threads)
     uint32_t hg = 0, cs = 0, sn = 0, v = 0;
     if (mine) v = f.src[p][(int64_t)m * f.N[p] + head * rs.hd + d];
     if (mine && rs.hgamma) hg = rs.hgamma[d];
@@ -1628,7 +1645,7 @@ __global__ __launch_bounds__(kFinishThreads) void head_norm_rope_finish_kernel(c
         cs = rs.cos[d];
         sn = rs.sin[d];
     }
-    __shared__ float hv[4][128], hy[4][128];
+    __shared__ float hv[8][128], hy[8][128];
     if (rs.hgamma) { // (the same for the whole workgroup)
         if (mine) hv[m][d] = asf(v);
         __syncthreads();
@@ -1662,28 +1679,32 @@ __global__ __launch_bounds__(kFinishThreads) void head_norm_rope_finish_kernel(c
 // are three quarters as many bytes again as the weights); four groups per workgroup take 29.5 instead of 34.3 us for
 // the 128 MiB of gate + up, more leave too few workgroups in flight.  For q / k / v and o (a quarter of the columns)
 // one group per workgroup stays the fastest.  Weights are read with the non-temporal hint.
-// M <= 4, batch folded away (one batch entry).  Epilogues as in skinny_kt_mfma_xreg_body.
-template <bool WHOLE, bool NORM, int TRIPS>
+// M <= MM, batch folded away (one batch entry).  Epilogues as in skinny_kt_mfma_xreg_body.
+template <bool WHOLE, int MM, bool NORM, int TRIPS>
 __device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs &a, const uint32_t *second, uint32_t one, uint32_t iters, const NormFuse &nf) {
     static_assert(TRIPS == 8 || TRIPS == 4, "chunks of 2048 or 1024");
     const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     const uint32_t j = lane % 4, b = lane / 4;
     uint32_t kb, ks; // this lane's k: kb + ks t (beyond K, in a chunk that K does not fill: zeros)
     xreg_lane_k<TRIPS, WHOLE>(a.K, wave, b, kb, ks);
-    const uint32_t *xrow = a.A + (int64_t)min(j, a.M - 1) * a.a_sm;
-    float4v xr[TRIPS];
+    constexpr int G = MM / 4, kOut = 4 * MM; // row groups; values of one product in a group of columns
+    float4v xr[G][TRIPS];
 #pragma unroll
-    for (int t = 0; t < TRIPS; t++) {
-        xr[t] = (float4v){0.f, 0.f, 0.f, 0.f};
-        if (WHOLE || kb + ks * t < a.K) xr[t] = *reinterpret_cast<const float4v *>(xrow + kb + ks * t);
+    for (int g = 0; g < G; g++) {
+        const uint32_t *xrow = a.A + (int64_t)min((uint32_t)(4 * g) + j, a.M - 1) * a.a_sm;
+#pragma unroll
+        for (int t = 0; t < TRIPS; t++) {
+            xr[g][t] = (float4v){0.f, 0.f, 0.f, 0.f};
+            if (WHOLE || kb + ks * t < a.K) xr[g][t] = *reinterpret_cast<const float4v *>(xrow + kb + ks * t);
+        }
     }
-    float pv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float pv[NORM ? 2 * MM : 1] = {};
     float4v gm[NORM ? TRIPS : 1];
     if constexpr (NORM) {
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
+        for (int u = 0; u < 2 * MM; u++) {
             const uint32_t i = threadIdx.x + u * kThreads;
-            if (i < nf.blocks * 4) pv[u] = nf.partials[i];
+            if (i < nf.blocks * MM) pv[u] = nf.partials[i];
         }
 #pragma unroll
         for (int t = 0; t < TRIPS; t++) {
@@ -1691,8 +1712,8 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs
             if (WHOLE || kb + ks * t < a.K) gm[t] = *reinterpret_cast<const float4v *>(nf.gamma + kb + ks * t);
         }
     }
-    __shared__ float part[2][4][32];
-    __shared__ float nsum[4][4];
+    __shared__ float part[2][4][2 * kOut];
+    __shared__ float nsum[4][MM];
     const uint32_t groups = (a.N + 3) / 4;
     float4v wg[TRIPS], wu[TRIPS]; // the group's four columns of the two weight matrices
     auto ask = [&](float4v (&w)[TRIPS], const uint32_t *base, uint32_t n0) {
@@ -1703,14 +1724,13 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs
             if (WHOLE || kb + ks * t < a.K) w[t] = __builtin_nontemporal_load(reinterpret_cast<const float4v *>(row + ks * t));
         }
     };
-    auto multiply = [&](float4v &sum, const float4v (&w)[TRIPS]) {
+    auto multiply = [&](float4v (&sum)[G], const float4v (&w)[TRIPS]) {
 #pragma unroll
-        for (int t = 0; t < TRIPS; t++) {
-            sum = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[t][0], w[t][0], sum, 0, 0, 0);
-            sum = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[t][1], w[t][1], sum, 0, 0, 0);
-            sum = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[t][2], w[t][2], sum, 0, 0, 0);
-            sum = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[t][3], w[t][3], sum, 0, 0, 0);
-        }
+        for (int t = 0; t < TRIPS; t++)
+#pragma unroll
+            for (int g = 0; g < G; g++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) sum[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[g][t][e], w[t][e], sum[g], 0, 0, 0);
     };
     const uint32_t first_grp = blockIdx.x * iters;
     if (first_grp >= groups) return; // the same for every thread of the workgroup
@@ -1721,29 +1741,31 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs
 #pragma unroll
         for (int t = 0; t < TRIPS; t++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) xr[t][e] = asf(apply<kMul, true>(asu(xr[t][e]), asu(gm[t][e]), 0, nullptr));
+            for (int g = 0; g < G; g++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) xr[g][t][e] = asf(apply<kMul, true>(asu(xr[g][t][e]), asu(gm[t][e]), 0, nullptr));
         float s = 0.0f;
 #pragma unroll
-        for (int u = 0; u < 8; u++) s += pv[u];
-        for (uint32_t i = threadIdx.x + 8 * kThreads; i < nf.blocks * 4; i += kThreads) s += nf.partials[i];
+        for (int u = 0; u < 2 * MM; u++) s += pv[u];
+        for (uint32_t i = threadIdx.x + 2 * MM * kThreads; i < nf.blocks * MM; i += kThreads) s += nf.partials[i];
 #pragma unroll
-        for (int sh = 32; sh >= 4; sh >>= 1) s += __shfl_xor(s, sh);
-        if (lane < 4) nsum[wave][lane] = s;
+        for (int sh = 32; sh >= MM; sh >>= 1) s += __shfl_xor(s, sh);
+        if (lane < MM) nsum[wave][lane] = s;
     }
     uint32_t divisor = 0;
     for (uint32_t it = 0; it < iters; it++) {
         const uint32_t grp = first_grp + it;
         if (grp >= groups) break;
         const uint32_t n0 = grp * 4;
-        float4v acc_g = {0.f, 0.f, 0.f, 0.f}, acc_u = {0.f, 0.f, 0.f, 0.f};
+        float4v acc_g[G] = {}, acc_u[G] = {};
         ask(wu, second, n0);
         multiply(acc_g, wg);
         if (it + 1 < iters && grp + 1 < groups) ask(wg, a.B, n0 + 4); // on its way through the rest of this group
         multiply(acc_u, wu);
-        float (*pt)[32] = part[it & 1];
+        float (*pt)[2 * kOut] = part[it & 1];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float vg = acc_g[i], vu = acc_u[i];
+        for (int i = 0; i < MM; i++) {
+            float vg = acc_g[i / 4][i % 4], vu = acc_u[i / 4][i % 4];
 #pragma unroll
             for (int s = 32; s >= 4; s >>= 1) {
                 vg += __shfl_xor(vg, s);
@@ -1751,14 +1773,14 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs
             }
             if (lane < 4) {
                 pt[wave][i * 4 + j] = vg;
-                pt[wave][16 + i * 4 + j] = vu;
+                pt[wave][kOut + i * 4 + j] = vu;
             }
         }
         __syncthreads(); // (the buffer written two groups ago was read before the barrier of the group in between)
-        if (threadIdx.x < 16) {
+        if (threadIdx.x < kOut) {
             const uint32_t t = threadIdx.x, m = t / 4, col = n0 + t % 4;
             uint32_t gv = asu((pt[0][t] + pt[1][t]) + (pt[2][t] + pt[3][t]));
-            uint32_t uv = asu((pt[0][16 + t] + pt[1][16 + t]) + (pt[2][16 + t] + pt[3][16 + t]));
+            uint32_t uv = asu((pt[0][kOut + t] + pt[1][kOut + t]) + (pt[2][kOut + t] + pt[3][kOut + t]));
             if constexpr (NORM) {
                 if (it == 0) divisor = norm_divisor(nf, (nsum[0][m] + nsum[1][m]) + (nsum[2][m] + nsum[3][m]));
                 gv = apply<kDiv, true>(gv, divisor, 0, nullptr);
@@ -1772,11 +1794,11 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs
         }
     }
 }
-template <bool NORM, int TRIPS>
+template <int MM, bool NORM, int TRIPS>
 __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_cols_gated_kernel(const MmArgs a, const uint32_t *second, uint32_t one,
                                                                                   uint32_t iters, const NormFuse nf) {
-    if (a.K % (TRIPS * 256) == 0) skinny_kt_mfma_xreg_cols_gated_impl<true, NORM, TRIPS>(a, second, one, iters, nf);
-    else skinny_kt_mfma_xreg_cols_gated_impl<false, NORM, TRIPS>(a, second, one, iters, nf);
+    if (a.K % (TRIPS * 256) == 0) skinny_kt_mfma_xreg_cols_gated_impl<true, MM, NORM, TRIPS>(a, second, one, iters, nf);
+    else skinny_kt_mfma_xreg_cols_gated_impl<false, MM, NORM, TRIPS>(a, second, one, iters, nf);
 }
 
 // Vectorised skinny kernel for short K (K <= 4*LPC, e.g. q.K^T of a decode step with
@@ -2083,16 +2105,17 @@ int launch_matmul_group(cg_backend *be, const cg_tensor *x, const cg_tensor *con
     g.first[n] = blocks;
     g.n = (uint32_t)n;
     ProfScope prof(be, CG_K_GEMM_SKINNY, bytes);
-    if (xreg)
-        hipLaunchKernelGGL((skinny_kt_mfma_xreg_group_kernel<4, 2, 8>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
-    else if (nf && xreg_trips(g.p[0].K) == 8)
-        hipLaunchKernelGGL(skinny_kt_mfma_xreg_group_norm_kernel<8>, dim3(blocks), dim3(kThreads), 0, be->stream, g, *nf);
-    else if (nf)
-        hipLaunchKernelGGL(skinny_kt_mfma_xreg_group_norm_kernel<4>, dim3(blocks), dim3(kThreads), 0, be->stream, g, *nf);
-    else if (xreg1 && xreg_trips(g.p[0].K) == 8)
-        hipLaunchKernelGGL((skinny_kt_mfma_xreg_group_kernel<4, 1, 8>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
-    else if (xreg1)
-        hipLaunchKernelGGL((skinny_kt_mfma_xreg_group_kernel<4, 1, 4>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
+    const bool eight = g.p[0].M > 4, deep = xreg_trips(g.p[0].K) == 8;
+    auto launch = [&](auto kernel, auto... args) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, be->stream, args...); };
+    if (xreg) launch(skinny_kt_mfma_xreg_group_kernel<4, 2, 8>, g);
+    else if (nf && deep && eight) launch(skinny_kt_mfma_xreg_group_norm_kernel<8, 8>, g, *nf);
+    else if (nf && deep) launch(skinny_kt_mfma_xreg_group_norm_kernel<4, 8>, g, *nf);
+    else if (nf && eight) launch(skinny_kt_mfma_xreg_group_norm_kernel<8, 4>, g, *nf);
+    else if (nf) launch(skinny_kt_mfma_xreg_group_norm_kernel<4, 4>, g, *nf);
+    else if (xreg1 && deep && eight) launch(skinny_kt_mfma_xreg_group_kernel<8, 1, 8>, g);
+    else if (xreg1 && deep) launch(skinny_kt_mfma_xreg_group_kernel<4, 1, 8>, g);
+    else if (xreg1 && eight) launch(skinny_kt_mfma_xreg_group_kernel<8, 1, 4>, g);
+    else if (xreg1) launch(skinny_kt_mfma_xreg_group_kernel<4, 1, 4>, g);
     else if (g.p[0].M <= 1)
         hipLaunchKernelGGL((skinny_kt_wide_group_kernel<1>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
     else if (g.p[0].M <= 4)
@@ -2168,10 +2191,18 @@ int launch_matmul_group_rope(cg_backend *be, const cg_tensor *x, const cg_tensor
         hf.first[hf.n] = heads;
         finish_heads = heads;
     }
-    if (nf && wide) hipLaunchKernelGGL((skinny_kt_mfma_xreg_group_rope_kernel<true, 8>), dim3(blocks), dim3(kThreads), 0, be->stream, g, rg, *nf);
-    else if (nf) hipLaunchKernelGGL((skinny_kt_mfma_xreg_group_rope_kernel<true, 4>), dim3(blocks), dim3(kThreads), 0, be->stream, g, rg, *nf);
-    else if (wide) hipLaunchKernelGGL((skinny_kt_mfma_xreg_group_rope_kernel<false, 8>), dim3(blocks), dim3(kThreads), 0, be->stream, g, rg, none);
-    else hipLaunchKernelGGL((skinny_kt_mfma_xreg_group_rope_kernel<false, 4>), dim3(blocks), dim3(kThreads), 0, be->stream, g, rg, none);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, be->stream, g, rg, nf ? *nf : none); };
+    if (g.p[0].M > 4) {
+        if (nf && wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<8, true, 8>);
+        else if (nf) launch(skinny_kt_mfma_xreg_group_rope_kernel<8, true, 4>);
+        else if (wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<8, false, 8>);
+        else launch(skinny_kt_mfma_xreg_group_rope_kernel<8, false, 4>);
+    } else {
+        if (nf && wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<4, true, 8>);
+        else if (nf) launch(skinny_kt_mfma_xreg_group_rope_kernel<4, true, 4>);
+        else if (wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<4, false, 8>);
+        else launch(skinny_kt_mfma_xreg_group_rope_kernel<4, false, 4>);
+    }
     if (by_head) {
         const uint32_t threads = (hf.M * 128 + 63) / 64 * 64;
         hipLaunchKernelGGL(head_norm_rope_finish_kernel, dim3(finish_heads), dim3(threads), 0, be->stream, hf);
@@ -2195,7 +2226,7 @@ int launch_matmul_gated(cg_backend *be, const cg_tensor *x, const cg_tensor *yg,
     if (!rc) rc = make_mm_args(x, yu, c, &au, &fu);
     if (rc) return rc;
     const bool vec = ag.a_vec && ag.b_vec && au.b_vec && ag.a_sk == 1 && ag.K % 4 == 0;
-    if (fg.batch != 1 || fu.batch != 1 || ag.M > 4 || ag.b_sk != 1 || au.b_sk != 1 || !vec || ag.K <= 256 || ag.N < 512 ||
+    if (fg.batch != 1 || fu.batch != 1 || ag.M > 8 || ag.b_sk != 1 || au.b_sk != 1 || !vec || ag.K <= 256 || ag.N < 512 ||
         au.N != ag.N || au.K != ag.K || au.M != ag.M || au.b_sn != ag.b_sn)
         return kDeclined;
     if (nf && xreg_trips(ag.K) == 0) return kDeclined;
@@ -2203,23 +2234,38 @@ int launch_matmul_gated(cg_backend *be, const cg_tensor *x, const cg_tensor *yg,
     ProfScope prof(be, CG_K_GEMM_SKINNY, distinct_bytes(x) + distinct_bytes(yg) + distinct_bytes(yu) + distinct_bytes(out));
     const dim3 ggrid((ag.N + 3) / 4);
     if (xreg_trips(ag.K) == 0) return kDeclined;
+    const bool eight = ag.M > 4;
     if ((int)ag.K <= xreg_trips(ag.K) * 256) { // one chunk of k (full or not): see skinny_kt_mfma_xreg_cols_gated_kernel
         NormFuse none;
         memset(&none, 0, sizeof none);
         const uint32_t groups = (ag.N + 3) / 4, iters = xreg_cols_iters(groups);
         const dim3 cgrid((groups + iters - 1) / iters);
-        if (nf && short_chunks) hipLaunchKernelGGL((skinny_kt_mfma_xreg_cols_gated_kernel<true, 4>), cgrid, dim3(kThreads), 0, be->stream, ag, au.B, one, iters, *nf);
-        else if (nf) hipLaunchKernelGGL((skinny_kt_mfma_xreg_cols_gated_kernel<true, 8>), cgrid, dim3(kThreads), 0, be->stream, ag, au.B, one, iters, *nf);
-        else if (short_chunks) hipLaunchKernelGGL((skinny_kt_mfma_xreg_cols_gated_kernel<false, 4>), cgrid, dim3(kThreads), 0, be->stream, ag, au.B, one, iters, none);
-        else hipLaunchKernelGGL((skinny_kt_mfma_xreg_cols_gated_kernel<false, 8>), cgrid, dim3(kThreads), 0, be->stream, ag, au.B, one, iters, none);
-    } else if (nf && short_chunks)
-        hipLaunchKernelGGL(skinny_kt_mfma_xreg_gated_norm_kernel<4>, ggrid, dim3(kThreads), 0, be->stream, ag, au.B, one, *nf);
-    else if (nf)
-        hipLaunchKernelGGL(skinny_kt_mfma_xreg_gated_norm_kernel<8>, ggrid, dim3(kThreads), 0, be->stream, ag, au.B, one, *nf);
-    else if (short_chunks)
-        hipLaunchKernelGGL((skinny_kt_mfma_xreg_gated_kernel<4, 4>), ggrid, dim3(kThreads), 0, be->stream, ag, au.B, one);
-    else
-        hipLaunchKernelGGL((skinny_kt_mfma_xreg_gated_kernel<4, 8>), ggrid, dim3(kThreads), 0, be->stream, ag, au.B, one);
+        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, cgrid, dim3(kThreads), 0, be->stream, ag, au.B, one, iters, nf ? *nf : none); };
+        if (eight) {
+            if (nf && short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<8, true, 4>);
+            else if (nf) launch(skinny_kt_mfma_xreg_cols_gated_kernel<8, true, 8>);
+            else if (short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<8, false, 4>);
+            else launch(skinny_kt_mfma_xreg_cols_gated_kernel<8, false, 8>);
+        } else {
+            if (nf && short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<4, true, 4>);
+            else if (nf) launch(skinny_kt_mfma_xreg_cols_gated_kernel<4, true, 8>);
+            else if (short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<4, false, 4>);
+            else launch(skinny_kt_mfma_xreg_cols_gated_kernel<4, false, 8>);
+        }
+    } else {
+        auto launch = [&](auto kernel, auto... more) { hipLaunchKernelGGL(kernel, ggrid, dim3(kThreads), 0, be->stream, ag, au.B, one, more...); };
+        if (eight) {
+            if (nf && short_chunks) launch(skinny_kt_mfma_xreg_gated_norm_kernel<8, 4>, *nf);
+            else if (nf) launch(skinny_kt_mfma_xreg_gated_norm_kernel<8, 8>, *nf);
+            else if (short_chunks) launch(skinny_kt_mfma_xreg_gated_kernel<8, 4>);
+            else launch(skinny_kt_mfma_xreg_gated_kernel<8, 8>);
+        } else {
+            if (nf && short_chunks) launch(skinny_kt_mfma_xreg_gated_norm_kernel<4, 4>, *nf);
+            else if (nf) launch(skinny_kt_mfma_xreg_gated_norm_kernel<4, 8>, *nf);
+            else if (short_chunks) launch(skinny_kt_mfma_xreg_gated_kernel<4, 4>);
+            else launch(skinny_kt_mfma_xreg_gated_kernel<4, 8>);
+        }
+    }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "gated matmul launch");
 }
@@ -2247,8 +2293,10 @@ int launch_matmul_residual(cg_backend *be, const cg_tensor *x, const cg_tensor *
     if (keep_sums && out->offset == 0 && xreg_narrow(a.M, a.K) && !out->buf->side) {
         // the stored rows' sums of squares per workgroup, for an RMS norm that may follow (Buffer::side)
         Buffer *ob = out->buf;
-        if (be->pool.alloc((size_t)blocks * 4 * sizeof(float), &ob->side, &ob->side_cls) == CG_OK) {
+        const uint32_t rows = a.M > 4 ? 8 : 4;
+        if (be->pool.alloc((size_t)blocks * rows * sizeof(float), &ob->side, &ob->side_cls) == CG_OK) {
             ob->side_blocks = blocks;
+            ob->side_rows = rows;
             r.partials = static_cast<float *>(ob->side);
         } else {
             ob->side = nullptr;
@@ -2258,14 +2306,20 @@ int launch_matmul_residual(cg_backend *be, const cg_tensor *x, const cg_tensor *
     dim3 grid((uint32_t)((a.N + 3) / 4));
     const int eight = eight_trips(be, a.M, a.N, a.K);
     const dim3 grid8((uint32_t)((a.N + 7) / 8));
-    if (eight == 16) hipLaunchKernelGGL(skinny_kt_mfma_eight_residual_kernel<16>, grid8, dim3(kEightThreads), 0, be->stream, a, r);
-    else if (eight == 8) hipLaunchKernelGGL(skinny_kt_mfma_eight_residual_kernel<8>, grid8, dim3(kEightThreads), 0, be->stream, a, r);
-    else if (eight == 4) hipLaunchKernelGGL(skinny_kt_mfma_eight_residual_kernel<4>, grid8, dim3(kEightThreads), 0, be->stream, a, r);
+    auto launch8 = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid8, dim3(kEightThreads), 0, be->stream, a, r); };
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, be->stream, a, r); };
+    const bool rows8 = a.M > 4;
+    if (eight == 16) launch8(skinny_kt_mfma_eight_residual_kernel<4, 16>);
+    else if (eight == 8 && rows8) launch8(skinny_kt_mfma_eight_residual_kernel<8, 8>);
+    else if (eight == 8) launch8(skinny_kt_mfma_eight_residual_kernel<4, 8>);
+    else if (eight == 4 && rows8) launch8(skinny_kt_mfma_eight_residual_kernel<8, 4>);
+    else if (eight == 4) launch8(skinny_kt_mfma_eight_residual_kernel<4, 4>);
     else if (xreg_narrow(a.M, a.K)) {
-        if (xreg_trips(a.K) == 8)
-            hipLaunchKernelGGL((skinny_kt_mfma_xreg_residual_kernel<4, 8>), grid, dim3(kThreads), 0, be->stream, a, r);
-        else
-            hipLaunchKernelGGL((skinny_kt_mfma_xreg_residual_kernel<4, 4>), grid, dim3(kThreads), 0, be->stream, a, r);
+        const bool deep = xreg_trips(a.K) == 8;
+        if (deep && rows8) launch(skinny_kt_mfma_xreg_residual_kernel<8, 8>);
+        else if (deep) launch(skinny_kt_mfma_xreg_residual_kernel<4, 8>);
+        else if (rows8) launch(skinny_kt_mfma_xreg_residual_kernel<8, 4>);
+        else launch(skinny_kt_mfma_xreg_residual_kernel<4, 4>);
     } else if (a.M <= 1)
         hipLaunchKernelGGL((skinny_kt_wide_residual_kernel<1>), grid, dim3(kThreads), 0, be->stream, a, r);
     else if (a.M <= 4)
@@ -2680,7 +2734,11 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
                     hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<4, 2, 8>), grid, dim3(kThreads), 0, s, a);
             } else if (cols >= 2048 && xreg_narrow((uint32_t)M, (uint32_t)K)) {
                 dim3 grid((uint32_t)((N + 3) / 4), (uint32_t)batch);
-                if (xreg_trips((uint32_t)K) == 4)
+                if (M > 4 && xreg_trips((uint32_t)K) == 4)
+                    hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<8, 1, 4>), grid, dim3(kThreads), 0, s, a);
+                else if (M > 4)
+                    hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<8, 1, 8>), grid, dim3(kThreads), 0, s, a);
+                else if (xreg_trips((uint32_t)K) == 4)
                     hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<4, 1, 4>), grid, dim3(kThreads), 0, s, a);
                 else
                     hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<4, 1, 8>), grid, dim3(kThreads), 0, s, a);

@@ -153,7 +153,7 @@ Pending::~Pending() {
 }
 
 // Is x (still) the deferred program  h / pow(sum(h * h) / n + eps, e) * gamma  over the rows of a residual stream h
-// [1..4 rows, K] whose kernel left the partial sums of squares (Buffer::side)?  Then a decode-time product can apply
+// [1..8 rows, K] whose kernel left the partial sums of squares (Buffer::side)?  Then a decode-time product can apply
 // the norm while it loads h (K a multiple of 4 above 256) and the norm needs no launch.  Fills nf and the stand-in tensor
 // h (a borrowed view of the leaf's buffer: set h->buf to null before it goes out of scope).
 static bool norm_fuse_of(const cg_tensor *x, NormFuse *nf, cg_tensor *h) {
@@ -166,9 +166,11 @@ static bool norm_fuse_of(const cg_tensor *x, NormFuse *nf, cg_tensor *h) {
         if (p->ins[i].op != code[i][0] || p->ins[i].a != code[i][1] || p->ins[i].b != code[i][2] || p->ins[i].c != code[i][3]) return false;
     const int r = x->rank;
     const int64_t K = x->dims[r - 1], rows = K > 0 ? numel(x) / K : 0;
-    if (K <= 256 || K % 4 != 0 || rows < 1 || rows > 4 || p->rowlen != K) return false;
+    if (K <= 256 || K % 4 != 0 || rows < 1 || rows > 8 || p->rowlen != K) return false;
     const LeafView &lh = p->leaf[0], &lg = p->leaf[4];
-    if (lh.uniform || lh.pw || lh.lazy || !lh.buf || !lh.buf->side || lh.offset != 0 || (int64_t)lh.buf->side_blocks * 4 != K) return false;
+    if (lh.uniform || lh.pw || lh.lazy || !lh.buf || !lh.buf->side || lh.offset != 0 || (int64_t)lh.buf->side_blocks * 4 != K ||
+        lh.buf->side_rows != (rows > 4 ? 8u : 4u))
+        return false;
     if (is_narrow_buf(lh.buf) || is_narrow_buf(lg.buf)) return false; // (the kernels read 32-bit words)
     if (!p->leaf[1].uniform || !p->leaf[2].uniform || !p->leaf[3].uniform) return false;
     if (lg.uniform || lg.pw || lg.lazy || !lg.buf || lg.offset % 4 != 0) return false;
@@ -1293,7 +1295,7 @@ static int try_rope_stores(cg_backend *be, std::vector<DeferredWrite> &w, const 
         const int64_t N = m->dims[m->rank - 1];
         int64_t rows = 1;
         for (int d = 0; d + 1 < m->rank; d++) rows *= m->dims[d];
-        if (H * hd != N || rows != B || B > 4 || (m->head_norm && m->hn_hd != (uint32_t)hd)) return kDeclined;
+        if (H * hd != N || rows != B || B > 8 || (m->head_norm && m->hn_hd != (uint32_t)hd)) return kDeclined;
         auto whole = [&](const int64_t *s, int64_t off, int64_t want_off) { // the view [B, H, 1, hd] of the product's rows, from `want_off`
             return (B == 1 || s[0] == N) && (H == 1 || s[1] == hd) && s[3] == 1 && off == want_off;
         };
@@ -1753,7 +1755,7 @@ static int defer_reduce(cg_backend *be, int kind, cg_tensor *x, const int64_t *o
 }
 
 // x: the deferred RMS norm  v / pow(sum(v * v) / n + eps, e) * gamma  over the rows of [R, hd], v the whole of a decode-time
-// product [rows <= 4, N = heads * hd] that nobody has needed yet (the q / k norm of Qwen3, qwen3.rs:249-279).  Then x
+// product [rows <= 8, N = heads * hd] that nobody has needed yet (the q / k norm of Qwen3, qwen3.rs:249-279).  Then x
 // becomes a plain view of a NEW open product that carries the norm (LazyMm::head_norm): the views, the rotary embedding and
 // the cache write that follow treat it like any open product, and the kernel that stores the embedded heads norms them on
 // the way (try_rope_stores).  False: not that shape; x is untouched.
