@@ -68,6 +68,13 @@ CG_PROGRAM(RowsSoftmaxCausal, 5, 0x12, -1, {19, 0, 1, 0}, {149, 2, 3, 2}, {169, 
 // log(sum(exp(x - m))) + m, m one value per row           (log-sum-exp behind the rows' maxima; 4096 x 8192: 256 us
 // interpreted, 26 compiled = 5.2 TB/s)
 CG_PROGRAM(RowsLogSumExp, 2, 0x0, -1, {17, 0, 1, 0}, {3, 8, 8, 8}, {48, 9, 9, 9}, {4, 10, 10, 10}, {16, 11, 1, 11})
+// log(sum(exp(x - max x))) + max x: the same with the maxima taken in the kernel, from the row in registers (4096 x 8192, with
+// the maxima's launch before: 51 us, now 27); with the maxima also in memory, because somebody holds them; and what is left of it
+// when somebody reads x - max x or its exponentials
+CG_PROGRAM(RowsLogSumExpMax, 1, 0x0, -1, {49, 0, 0, 0}, {17, 0, 8, 0}, {3, 9, 9, 9}, {48, 10, 10, 10}, {4, 11, 11, 11}, {16, 12, 8, 12})
+CG_PROGRAM(RowsLogSumExpMaxKept, 2, 0x0, -1, {49, 0, 0, 0}, {17, 0, 8, 0}, {3, 9, 9, 9}, {48, 10, 10, 10}, {4, 11, 11, 11}, {16, 12, 1, 12})
+CG_PROGRAM(RowsShift, 1, 0x0, -1, {49, 0, 0, 0}, {17, 0, 8, 0})
+CG_PROGRAM(RowsShiftExp, 1, 0x0, -1, {49, 0, 0, 0}, {17, 0, 8, 0}, {3, 9, 9, 9})
 // exp(x - max x) / sum                                    (soft-max)
 CG_PROGRAM(RowsSoftmax, 1, 0x0, -1, {49, 0, 0, 0}, {17, 0, 8, 0}, {3, 9, 9, 9}, {48, 10, 10, 10}, {19, 10, 11, 10})
 
@@ -81,7 +88,8 @@ template <class P> struct words_only_of<P, std::void_t<decltype(P::words_only)>>
 
 template <class... P> struct ProgramList {};
 using MapPrograms = ProgramList<MapRope, MapSiluMul, MapResidual3a, MapResidual3b, MapSiluMulBF16, MapSiluMulF16, MapSiluMulF8, MapBiasSigmoid>;
-using RowsPrograms = ProgramList<RowsRmsNorm, RowsRmsNormAdd, RowsRmsNormAdd2a, RowsRmsNormAdd2b, RowsSoftmaxCausal, RowsLogSumExp, RowsSoftmax>;
+using RowsPrograms = ProgramList<RowsRmsNorm, RowsRmsNormAdd, RowsRmsNormAdd2a, RowsRmsNormAdd2b, RowsSoftmaxCausal, RowsLogSumExp, RowsSoftmax, RowsLogSumExpMax, RowsLogSumExpMaxKept,
+                                RowsShift, RowsShiftExp>;
 
 template <class P> bool program_matches(const Pending &p) {
     if (p.nleaf != P::nleaf || p.ninstr != P::ninstr) return false;
@@ -396,8 +404,8 @@ bool aot_map_dispatch(const Pending &p, const FusedArgs &a, dim3 grid, hipStream
     return aot_map_dispatch(p, a, grid, s, ProgramList<Rest...>{});
 }
 
-// Cached items per lane: 3 vectors of four (rows up to 12 * TPR elements) or 10 single
-// elements (rows up to 10 * TPR); longer rows take the re-reading instantiation.
+// Cached items per lane: 3 vectors of four (rows up to 12 * TPR elements; programs of a single leaf up to 16 vectors by 256 lanes,
+// rows up to 16384) or 10 single elements (rows up to 10 * TPR); longer rows take the re-reading instantiation.
 template <class P, int VEC> void aot_rows_launch(const FusedArgs &a, uint32_t *rowout, int tpr, dim3 grid, hipStream_t s) {
     constexpr int CI = VEC == 4 ? 3 : 10;
     const bool fits = (uint64_t)(a.n / VEC) <= (uint64_t)CI * (uint32_t)tpr;
@@ -408,6 +416,13 @@ template <class P, int VEC> void aot_rows_launch(const FusedArgs &a, uint32_t *r
         else                                                                                                \
             hipLaunchKernelGGL((aot_rows_kernel<P, VEC, TPR, 0>), grid, dim3(kBlock), 0, s, a, rowout);      \
     } while (0)
+    if constexpr (VEC == 4 && P::nleaf == 1) {
+        if (!fits && tpr == 256 && a.n <= 16384) {
+            if (a.n <= 8192) hipLaunchKernelGGL((aot_rows_kernel<P, VEC, 256, 8>), grid, dim3(kBlock), 0, s, a, rowout);
+            else hipLaunchKernelGGL((aot_rows_kernel<P, VEC, 256, 16>), grid, dim3(kBlock), 0, s, a, rowout);
+            return;
+        }
+    }
     if (tpr == 16) CG_ROWS(16);
     else if (tpr == 64) CG_ROWS(64);
     else CG_ROWS(256);

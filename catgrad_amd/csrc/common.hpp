@@ -261,6 +261,9 @@ struct cg_tensor : cg::Pooled<cg_tensor> {
     uint32_t ubits = 0;
     // A deferred element-wise result: no buffer yet, `pend` says how to compute it.
     cg::Pending *pend = nullptr;
+    // Set (and retained) on the broadcast of deferred row maxima that somebody else holds too: `pend` computes them anew, for
+    // the one consumer to which that costs nothing (x - max x: the row is in registers); settle() gives every other the maxima.
+    cg_tensor *row_of = nullptr;
     // Split axis: logical axis `split` (extent outer * split_inner) is addressed as
     // (i / split_inner) * split_os + (i % split_inner) * strides[split].  This is what
     // `reshape` makes of two adjacent axes that cannot share one stride — the merged
@@ -549,7 +552,8 @@ int launch_fused_reduce(cg_backend *be, int kind, bool f32, const Pending &p, in
 int launch_fused_rows(cg_backend *be, const cg_tensor *out, const Pending &p, const int64_t *dims, int rank);
 int launch_arange(cg_backend *be, cg_tensor *out);
 // Copies n <= kReadbackWords words to be->rb_dev and then stores `seq` at word kReadbackWords of it, visible to the host.
-constexpr uint32_t kReadbackWords = 1024;
+// (64 KiB: the runtime's staged copy and its wake-up cost 20 us more than the kernel's stores over the bus)
+constexpr uint32_t kReadbackWords = 16384;
 int launch_small_readback(cg_backend *be, const uint32_t *src, uint32_t n, uint32_t seq);
 // A few words from the host travel with the launch, as kernel arguments: n <= kUploadWords words to dst.
 constexpr uint32_t kUploadWords = 64;

@@ -230,7 +230,10 @@ int launch_elementwise(cg_backend *be, int op, cg_dtype dt, const cg_tensor *out
 }
 
 __global__ void small_readback_kernel(const uint32_t *src, uint32_t n, uint32_t *dst, uint32_t seq) {
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
+    // one workgroup, since the number behind the words must not be seen before any of them: 16 bytes a lane where src allows it
+    const uint32_t quads = reinterpret_cast<uintptr_t>(src) % 16 == 0 ? n / 4 : 0;
+    for (uint32_t i = threadIdx.x; i < quads; i += blockDim.x) reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+    for (uint32_t i = quads * 4 + threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
     __threadfence_system();
     __syncthreads();
     if (threadIdx.x == 0) __hip_atomic_store(dst + kReadbackWords, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -253,7 +256,7 @@ int launch_small_upload(cg_backend *be, uint32_t *dst, const uint32_t *host_word
 }
 
 int launch_small_readback(cg_backend *be, const uint32_t *src, uint32_t n, uint32_t seq) {
-    hipLaunchKernelGGL(small_readback_kernel, dim3(1), dim3(256), 0, be->stream, src, n, be->rb_dev, seq);
+    hipLaunchKernelGGL(small_readback_kernel, dim3(1), dim3(n > 1024 ? 1024 : 256), 0, be->stream, src, n, be->rb_dev, seq);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "read-back launch");
 }

@@ -2230,6 +2230,7 @@ int launch_matmul_gated(cg_backend *be, const cg_tensor *x, const cg_tensor *yg,
         au.N != ag.N || au.K != ag.K || au.M != ag.M || au.b_sn != ag.b_sn)
         return kDeclined;
     if (nf && xreg_trips(ag.K) == 0) return kDeclined;
+    if (ag.M > 4 && !nf) return kDeclined; // (more than four rows: a decode step's, whose norm comes along; others as a grouped product and the program)
     const bool short_chunks = xreg_trips(ag.K) == 4; // K a multiple of 1024 but not of 2048
     ProfScope prof(be, CG_K_GEMM_SKINNY, distinct_bytes(x) + distinct_bytes(yg) + distinct_bytes(yu) + distinct_bytes(out));
     const dim3 ggrid((ag.N + 3) / 4);
@@ -2242,10 +2243,8 @@ int launch_matmul_gated(cg_backend *be, const cg_tensor *x, const cg_tensor *yg,
         const dim3 cgrid((groups + iters - 1) / iters);
         auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, cgrid, dim3(kThreads), 0, be->stream, ag, au.B, one, iters, nf ? *nf : none); };
         if (eight) {
-            if (nf && short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<8, true, 4>);
-            else if (nf) launch(skinny_kt_mfma_xreg_cols_gated_kernel<8, true, 8>);
-            else if (short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<8, false, 4>);
-            else launch(skinny_kt_mfma_xreg_cols_gated_kernel<8, false, 8>);
+            if (short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<8, true, 4>);
+            else launch(skinny_kt_mfma_xreg_cols_gated_kernel<8, true, 8>);
         } else {
             if (nf && short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<4, true, 4>);
             else if (nf) launch(skinny_kt_mfma_xreg_cols_gated_kernel<4, true, 8>);
@@ -2255,10 +2254,8 @@ int launch_matmul_gated(cg_backend *be, const cg_tensor *x, const cg_tensor *yg,
     } else {
         auto launch = [&](auto kernel, auto... more) { hipLaunchKernelGGL(kernel, ggrid, dim3(kThreads), 0, be->stream, ag, au.B, one, more...); };
         if (eight) {
-            if (nf && short_chunks) launch(skinny_kt_mfma_xreg_gated_norm_kernel<8, 4>, *nf);
-            else if (nf) launch(skinny_kt_mfma_xreg_gated_norm_kernel<8, 8>, *nf);
-            else if (short_chunks) launch(skinny_kt_mfma_xreg_gated_kernel<8, 4>);
-            else launch(skinny_kt_mfma_xreg_gated_kernel<8, 8>);
+            if (short_chunks) launch(skinny_kt_mfma_xreg_gated_norm_kernel<8, 4>, *nf);
+            else launch(skinny_kt_mfma_xreg_gated_norm_kernel<8, 8>, *nf);
         } else {
             if (nf && short_chunks) launch(skinny_kt_mfma_xreg_gated_norm_kernel<4, 4>, *nf);
             else if (nf) launch(skinny_kt_mfma_xreg_gated_norm_kernel<4, 8>, *nf);

@@ -23,6 +23,7 @@ static thread_local std::string g_err;
 static std::recursive_mutex g_lazy_mu; // guards lazy backing of uniform tensors and of deferred ones (computing one may compute another)
 
 static int run_pending(cg_backend *be, const cg_tensor *dst, const Pending &p, bool fresh);
+static int settle(cg_tensor *t);
 
 int fail(int code, const char *fmt, ...) {
     char buf[512];
@@ -342,6 +343,7 @@ void release(cg_tensor *t) {
         cg_backend *be = t->be;
         buffer_release(t->buf);
         delete t->pend;
+        release(t->row_of);
         delete t;
         be->live_tensors.fetch_sub(1, std::memory_order_relaxed);
     }
@@ -790,6 +792,9 @@ static int run_pending(cg_backend *be, const cg_tensor *dst, const Pending &p) {
 
 // Row-major copy of a view (the materialising half of reshape / to_vec).
 int materialize(cg_backend *be, const cg_tensor *x, cg_tensor **out) {
+    if (x->row_of) {
+        if (int rc = settle(const_cast<cg_tensor *>(x))) return rc;
+    }
     cg_tensor *o;
     // a copy of a view of a narrow buffer keeps the buffer's format (whatever dtype tags the view); a program without row
     // reductions stores the format of its dtype
@@ -1412,8 +1417,37 @@ static bool may_wait(const cg_backend *be, const cg_tensor *dst, const Pending *
     return be->fuse && be->aot && p && p->nred == 0 && !p->reduced && numel(dst) > 0 && numel(dst) <= 16384;
 }
 
+// A broadcast of shared row maxima (cg_tensor::row_of) becomes the view of them that it stands for.
+static int settle(cg_tensor *t) {
+    std::lock_guard<std::recursive_mutex> lk(g_lazy_mu);
+    if (!t->row_of) return CG_OK;
+    cg_tensor *m = t->row_of;
+    const int rc = ensure_concrete(m);
+    if (rc) return rc;
+    t->buf = m->buf;
+    t->buf->rc.fetch_add(1);
+    memcpy(t->strides, m->strides, sizeof t->strides);
+    t->strides[t->rank - 1] = 0;
+    t->offset = m->offset;
+    delete t->pend;
+    t->pend = nullptr;
+    t->row_of = nullptr;
+    release(m);
+    return CG_OK;
+}
+
+// The maxima of x's rows, nothing else: cheap to compute again inside a program that has the row in registers, up to the 16384
+// values that it keeps there (log-sum-exp and arg-max of 2000 x 12000: 101 us with the maxima's own pass, 79 without; 100 x 60000,
+// walked twice by one workgroup a row: 75 and 85).
+static bool lone_row_max(const cg_tensor *x) {
+    const Pending *p = x->pend;
+    return p && p->reduced && p->nleaf == 1 && p->ninstr == 1 && p->ins[0].op == kRowMax && !p->overflow && !p->leaf[0].uniform && !p->leaf[0].pw &&
+           !p->leaf[0].lazy && x->dt == CG_F32 && x->be->aot && p->rowlen <= 16384;
+}
+
 // Turns a deferred tensor into a concrete one, in place (every holder of the handle sees it).
 int ensure_concrete(cg_tensor *t) {
+    if (t->row_of) return settle(t);
     if (t->split >= 0) { // a split-axis view becomes a plain dense tensor, in place
         std::lock_guard<std::recursive_mutex> lk(g_lazy_mu);
         if (t->split < 0) return CG_OK;
@@ -1594,6 +1628,13 @@ static uint8_t splice_program(Pending *p, const Pending *src, const int64_t *dim
     return last;
 }
 
+// x is deferred, but nothing more than a view of f32 values in a buffer (what a cast of values held in a narrower format leaves).
+static bool deferred_view(const cg_tensor *x) {
+    const Pending *p = x->pend;
+    return p && !p->reduced && p->nleaf == 1 && p->ninstr == 1 && p->nred == 0 && p->ins[0].op == kCopy && !p->leaf[0].uniform && !p->leaf[0].pw &&
+           !p->leaf[0].lazy && p->leaf[0].buf;
+}
+
 // The result of applying `op` element-wise to `ins` (all of ins[0]'s shape) as a deferred
 // tensor.  Deferred inputs that this call owns alone, or that are cheap, are spliced in;
 // other deferred inputs are made concrete first so that their value is computed once.
@@ -1609,6 +1650,24 @@ static int defer_elementwise(cg_backend *be, int op, cg_dtype in_dt, cg_dtype ou
         if (x->split >= 0) {
             int rc = ensure_concrete(x);
             if (rc) return rc;
+        }
+        if (x->row_of) { // row maxima that somebody else holds too: computed anew for x - max x alone
+            const cg_tensor *l = ins[0];
+            LeafView lv{};
+            bool of_buffer = false;
+            if (l->pend) {
+                of_buffer = deferred_view(l);
+                if (of_buffer) lv = l->pend->leaf[0];
+            } else if (l->buf && !l->uniform && l->split < 0) {
+                of_buffer = true;
+                lv.buf = l->buf;
+                memcpy(lv.strides, l->strides, sizeof lv.strides);
+                lv.offset = l->offset;
+            }
+            if (op != kSub || k != 1 || in_dt != CG_F32 || x->rc.load() != 1 || !of_buffer || !same_leaf(lv, x->pend->leaf[0], x->dims, rank)) {
+                int rc = settle(x);
+                if (rc) return rc;
+            }
         }
         if (op != kAdd && x->pend && residual_sum_open(x)) { // see there; a further add may still join the sum
             int rc = ensure_concrete(x);
@@ -1711,13 +1770,16 @@ static int defer_elementwise(cg_backend *be, int op, cg_dtype in_dt, cg_dtype ou
 static int defer_reduce(cg_backend *be, int kind, cg_tensor *x, const int64_t *odims, cg_tensor **out) {
     *out = nullptr;
     const int rank = x->rank;
-    if (x->split >= 0 || (x->pend && x->pend->reduced)) {
+    if (x->split >= 0 || x->row_of || (x->pend && x->pend->reduced)) {
         int rc = ensure_concrete(x);
         if (rc) return rc;
     }
     Pending *p;
     uint8_t src;
-    if (x->pend) {
+    if (x->pend && x->dt == CG_F32 && deferred_view(x)) { // the values as they lie: a lone reduction, on its own kernels
+        p = new Pending;
+        src = (uint8_t)add_leaf(p, x->pend->leaf[0], x->dims, rank);
+    } else if (x->pend) {
         if (x->pend->nred >= kMaxRowReduce || x->pend->ninstr >= kMaxInstr) return CG_OK;
         p = new Pending(*x->pend);
         src = (uint8_t)(kMaxLeaves + p->ninstr - 1);
@@ -1777,7 +1839,8 @@ static bool head_norm_lazy(cg_tensor *x) {
     int64_t n = 1;
     for (int d = 0; d < m->rank; d++) n *= m->dims[d];
     const int64_t N = m->dims[m->rank - 1], K = m->x->rank > 0 ? m->x->dims[m->x->rank - 1] : 0;
-    if (n != R * hd || N % hd || n / N > 4 || K <= 256 || K % 4) return false; // (what the kernels of launch_matmul_group_rope take)
+    if (n != R * hd || N % hd || n / N > 8 || K <= 256 || K % 4) return false; // (what the kernels of launch_matmul_group_rope take)
+    if (n / N > 1 && (m->rank != 3 || m->dims[1] != 1)) return false; // (one position each: the rows of a prompt have no such store)
     if (!p->leaf[1].uniform || !p->leaf[2].uniform || !p->leaf[3].uniform) return false;
     if (lg.uniform || lg.pw || lg.lazy || !lg.buf || is_narrow_buf(lg.buf) || lg.strides[1] != 1 || (R > 1 && lg.strides[0] != 0)) return false;
     LazyMm *m2 = new LazyMm;
@@ -2303,6 +2366,7 @@ cg_dtype cg_tensor_dtype(const cg_tensor *t) { return t->dt; }
 size_t cg_tensor_numel(const cg_tensor *t) { return (size_t)numel(t); }
 int cg_tensor_is_contiguous(const cg_tensor *t) {
     Enter entered(t->be); // a deferred tensor may be being computed, in place, by another thread
+    if (t->row_of) return t->dims[t->rank - 1] == 1; // (a view of its rows' maxima)
     if (t->pend) return 1; // a deferred result is row-major once computed
     return (t->uniform && numel(t) > 1) ? 0 : (is_contiguous(t) ? 1 : 0);
 }
@@ -3094,7 +3158,8 @@ int cg_broadcast(cg_backend *b, cg_tensor *x, const size_t *dims, size_t rank, c
         if (x->dims[i] != d[i + shift] && x->dims[i] != 1)
             return fail(CG_ERR_SHAPE, "broadcast: incompatible shape (axis %d: %lld -> %lld)", i, (long long)x->dims[i],
                         (long long)d[i + shift]);
-    if (x->pend && x->pend->reduced && x->rc.load() == 1 && (int)rank == x->rank && d[rank - 1] == x->pend->rowlen) {
+    const bool alone = x->rc.load() == 1;
+    if (x->pend && x->pend->reduced && (alone || lone_row_max(x)) && (int)rank == x->rank && d[rank - 1] == x->pend->rowlen) {
         // row results broadcast back over their rows: the same program, seen at full shape
         bool same = true;
         for (int i = 0; i + 1 < (int)rank; i++) same = same && d[i] == x->dims[i];
@@ -3108,6 +3173,10 @@ int cg_broadcast(cg_backend *b, cg_tensor *x, const size_t *dims, size_t rank, c
             memcpy(t->dims, d, sizeof(int64_t) * rank);
             set_row_major(t);
             t->pend = p;
+            if (!alone) {
+                retain(x);
+                t->row_of = x;
+            }
             *out = t;
             return CG_OK;
         }
