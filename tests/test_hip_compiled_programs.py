@@ -58,3 +58,36 @@ def test_compiled_and_interpreted_agree(hip, interpreter, name):
     got, want = (CASES[name](be, np.random.default_rng(11)) for be in (hip, interpreter))
     for g, w in zip(got, want):
         np.testing.assert_array_equal(g, w)
+
+
+def gating(be, dtype, gate, up):
+    raw = {A.BF16: be.ndarray_from_vec_bf16, A.F8: be.ndarray_from_vec_fp8}[dtype]
+    g, u = raw(gate, gate.shape), raw(up, up.shape)
+    one = be.broadcast(be.cast(be.ndarray_from_vec_f32([1.0], ()), dtype).move(), gate.shape)
+    e = be.exp(be.neg(g).move())
+    e = be.div(g.move(), be.add(one.move(), e.move()).move())
+    return be.to_numpy(be.cast(be.mul(e.move(), u.move()).move(), A.F32))
+
+
+@pytest.mark.parametrize("extra", [0, 1, 7, 9, 15, 4097])
+@pytest.mark.parametrize("dtype", [A.BF16, A.F8])
+def test_gating_of_every_value(hip, interpreter, dtype, extra):
+    """All patterns of the dtype as gates, beside several factors; counts that end inside a lane's share, a workgroup's, and beyond."""
+    rng = np.random.default_rng(extra)
+    bits, kind = (16, np.uint16) if dtype == A.BF16 else (8, np.uint8)
+    # (large enough to lie in memory as patterns, not words; many whole rounds of the patterns in a run, so that fast and slow meet)
+    gate = np.concatenate([np.arange(1 << bits, dtype=kind)] * max(2, (1 << 18) >> bits) + [rng.integers(0, 1 << bits, extra, dtype=kind)])
+    up = rng.integers(0, 1 << bits, gate.size, dtype=kind)
+    up[: 1 << bits] = {A.BF16: 0x3F80, A.F8: 0x38}[dtype]  # one
+    got, want = (gating(be, dtype, gate, up) for be in (hip, interpreter))
+    np.testing.assert_array_equal(got, want)
+    small = rng.integers(0, 0x4281 if dtype == A.BF16 else 256, gate.size, dtype=kind)  # gates of the fast range alone, both signs
+    if dtype == A.BF16:
+        small |= (rng.integers(0, 2, gate.size, dtype=kind) << 15).astype(kind)
+    got, want = (gating(be, dtype, small, up) for be in (hip, interpreter))
+    np.testing.assert_array_equal(got, want)
+    if dtype == A.BF16:
+        every = np.concatenate([np.arange(0x4281, dtype=kind), np.arange(0x8000, 0xC281, dtype=kind)] * 8)
+        ones = np.full(every.size, 0x3F80, kind)
+        got, want = (gating(be, dtype, every, ones) for be in (hip, interpreter))
+        np.testing.assert_array_equal(got, want)
