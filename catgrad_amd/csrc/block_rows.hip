@@ -252,6 +252,7 @@ __global__ __launch_bounds__(kThreads) void few_rows_residual_kernel(const Rows 
 // the factors of a norm are the same for a whole row, so they are applied to the sums, and the row sums they need are formed
 // from what a wave loads anyway.  The polynomial norm is linear in z, z^2, z^3 and 1: four sums instead of one.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef f32x4 f32x4_words __attribute__((aligned(4))); // from any word's address
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bfx2 __attribute__((ext_vector_type(2)));
 
@@ -317,6 +318,9 @@ __device__ __forceinline__ float blocks_sum(float v) {
 }
 
 // A workgroup holds all of its waves' activations in registers (STEPS of 64 lanes' worth each) and walks column groups.
+// Weights, activations and the norm's gains are all asked for before anything is done with any of them: with the gains asked
+// for step by step behind the activations, 8328 x 1024 f32 took 10.6 us, 9.5 so (34 MB: 5.5 us at the device's rate, 5 before and
+// behind a launch's stream).
 template <bool BF16, int STEPS, int WAVES>
 __device__ __forceinline__ void four_rows_linear(const ProductInput &in, const uint32_t rows, const Weight &w, const uint32_t block, const uint32_t iters,
                                                  const float *__restrict__ bias, const float scale, float *__restrict__ out) {
@@ -333,25 +337,32 @@ __device__ __forceinline__ void four_rows_linear(const ProductInput &in, const u
     };
     ask(g0);
     Frag<BF16> x[STEPS];
-    float ss = 0.0f;
+    float z[STEPS][W];
 #pragma unroll
-    for (int s = 0; s < STEPS; s++) {
-        const uint32_t k = k0 + s * WAVES * SPAN;
-        float z[W];
-        load_input<BF16>(in, min(j, rows - 1), j < rows, k, z);
-        if (in.gamma) {
+    for (int s = 0; s < STEPS; s++) load_input<BF16>(in, min(j, rows - 1), j < rows, k0 + s * WAVES * SPAN, z[s]);
+    if (in.gamma) {
+        float gm[STEPS][W], ss = 0.0f;
+#pragma unroll
+        for (int s = 0; s < STEPS; s++)
+#pragma unroll
+            for (uint32_t i = 0; i < W; i += 4) { // (in.k is a multiple of W; behind it the activations are zero)
+                const f32x4 t = *reinterpret_cast<const f32x4_words *>(in.gamma + min(k0 + s * WAVES * SPAN + i, in.k - 4));
+#pragma unroll
+                for (int e = 0; e < 4; e++) gm[s][i + e] = t[e];
+            }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < STEPS; s++)
 #pragma unroll
             for (uint32_t i = 0; i < W; i++) {
-                ss = fmaf(z[i], z[i], ss);
-                z[i] *= in.gamma[min(k + i, in.k - 1)];
+                ss = fmaf(z[s][i], z[s][i], ss);
+                z[s][i] *= gm[s][i];
             }
-        }
-        x[s] = pack<BF16>(z);
-    }
-    if (in.gamma) {
         ss = blocks_sum(ss);
         if (lane < 4) squares[wave][lane] = ss;
     }
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) x[s] = pack<BF16>(z[s]);
     float rstd = scale;
     for (uint32_t g = g0; g < g1; g++) {
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -402,55 +413,70 @@ template <int NG> struct BranchSums {
     f32x4 acc[NG][4]; // of z, z^2, z^3, 1
     float m[3];
 };
-template <bool BF16, int NG, int WAVES, bool POLY>
-__device__ __forceinline__ void walk_branch(const ResidualBranch &b, uint32_t rows, uint32_t width, uint32_t n0, BranchSums<NG> &o) {
-    constexpr uint32_t W = Frag<BF16>::W, SPAN = 16 * W, STEP = WAVES * SPAN;
-    constexpr int AHEAD = 4;
-    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 3;
-    uint32_t n[NG];
+// Four steps of a branch (AHEAD * WAVES * 64 or 128 values of k) in registers: both branches' first ones are asked for before any is
+// multiplied.  2048 columns of 2048 + 8192 values of k, f32: 23.9 us with one branch behind the other, 21.1 so; bf16 14.7 and 14.1;
+// 1024 columns of 2048 + 3072: 10.2 and 10.1 (eight steps at a time: 10.4).
+template <bool BF16, int NG> struct BranchLoads {
+    static constexpr int AHEAD = 4;
+    Frag<BF16> wt[AHEAD][NG];
+    float z[AHEAD][Frag<BF16>::W];
+};
+template <bool BF16, int NG, int WAVES>
+__device__ __forceinline__ void ask_branch(const ResidualBranch &b, uint32_t rows, uint32_t width, uint32_t n0, uint32_t base, BranchLoads<BF16, NG> &l) {
+    constexpr uint32_t W = Frag<BF16>::W, STEP = WAVES * 16 * W;
+    const uint32_t lane = threadIdx.x & 63, j = lane & 3, k0 = base + (lane >> 2) * W;
 #pragma unroll
-    for (int g = 0; g < NG; g++) n[g] = min(n0 + 4 * g + j, width - 1);
+    for (int a = 0; a < l.AHEAD; a++)
+#pragma unroll
+        for (int g = 0; g < NG; g++) l.wt[a][g] = load_weights<BF16>(b.w, min(n0 + 4 * g + j, width - 1), k0 + a * STEP);
+#pragma unroll
+    for (int a = 0; a < l.AHEAD; a++) load_input<BF16>(b.in, min(j, rows - 1), j < rows, k0 + a * STEP, l.z[a]);
+}
+template <bool BF16, int NG, int WAVES, bool POLY>
+__device__ __forceinline__ void multiply_branch(const ResidualBranch &b, uint32_t base, BranchLoads<BF16, NG> &l, BranchSums<NG> &o) {
+    constexpr uint32_t W = Frag<BF16>::W, STEP = WAVES * 16 * W;
+    const uint32_t k0 = base + ((threadIdx.x & 63) >> 2) * W;
     float one[W];
 #pragma unroll
     for (uint32_t i = 0; i < W; i++) one[i] = 1.0f;
     const Frag<BF16> ones = pack<BF16>(one);
-    for (uint32_t base = wave * SPAN; base < b.w.k; base += AHEAD * STEP) { // (the same trips for every lane: the instruction does not mask)
-        const uint32_t k0 = base + (lane >> 2) * W;
-        Frag<BF16> wt[AHEAD][NG];
-        float z[AHEAD][W];
 #pragma unroll
-        for (int a = 0; a < AHEAD; a++)
+    for (int a = 0; a < l.AHEAD; a++) {
+        Frag<BF16> x = pack<BF16>(l.z[a]);
 #pragma unroll
-            for (int g = 0; g < NG; g++) wt[a][g] = load_weights<BF16>(b.w, n[g], k0 + a * STEP);
+        for (int g = 0; g < NG; g++) o.acc[g][0] = multiply<BF16>(l.wt[a][g], x, o.acc[g][0]);
+        if constexpr (POLY) {
+            float p[W], c[W];
 #pragma unroll
-        for (int a = 0; a < AHEAD; a++) load_input<BF16>(b.in, min(j, rows - 1), j < rows, k0 + a * STEP, z[a]);
-#pragma unroll
-        for (int a = 0; a < AHEAD; a++) {
-            Frag<BF16> x = pack<BF16>(z[a]);
-#pragma unroll
-            for (int g = 0; g < NG; g++) o.acc[g][0] = multiply<BF16>(wt[a][g], x, o.acc[g][0]);
-            if constexpr (POLY) {
-                float p[W], c[W];
-#pragma unroll
-                for (uint32_t i = 0; i < W; i++) {
-                    p[i] = z[a][i] * z[a][i];
-                    c[i] = p[i] * z[a][i];
-                    o.m[0] += p[i];
-                    o.m[1] = fmaf(p[i], p[i], o.m[1]);
-                    o.m[2] = fmaf(c[i], c[i], o.m[2]);
-                }
-                x = pack<BF16>(p);
-#pragma unroll
-                for (int g = 0; g < NG; g++) o.acc[g][1] = multiply<BF16>(wt[a][g], x, o.acc[g][1]);
-                x = pack<BF16>(c);
-#pragma unroll
-                for (int g = 0; g < NG; g++) o.acc[g][2] = multiply<BF16>(wt[a][g], x, o.acc[g][2]);
-#pragma unroll
-                for (int i = 0; i < 4; i++) x.v[i] = k0 + a * STEP < b.w.k ? ones.v[i] : 0;
-#pragma unroll
-                for (int g = 0; g < NG; g++) o.acc[g][3] = multiply<BF16>(wt[a][g], x, o.acc[g][3]);
+            for (uint32_t i = 0; i < W; i++) {
+                p[i] = l.z[a][i] * l.z[a][i];
+                c[i] = p[i] * l.z[a][i];
+                o.m[0] += p[i];
+                o.m[1] = fmaf(p[i], p[i], o.m[1]);
+                o.m[2] = fmaf(c[i], c[i], o.m[2]);
             }
+            x = pack<BF16>(p);
+#pragma unroll
+            for (int g = 0; g < NG; g++) o.acc[g][1] = multiply<BF16>(l.wt[a][g], x, o.acc[g][1]);
+            x = pack<BF16>(c);
+#pragma unroll
+            for (int g = 0; g < NG; g++) o.acc[g][2] = multiply<BF16>(l.wt[a][g], x, o.acc[g][2]);
+#pragma unroll
+            for (int i = 0; i < 4; i++) x.v[i] = k0 + a * STEP < b.w.k ? ones.v[i] : 0;
+#pragma unroll
+            for (int g = 0; g < NG; g++) o.acc[g][3] = multiply<BF16>(l.wt[a][g], x, o.acc[g][3]);
         }
+    }
+}
+// What is left of a branch behind its first loads (the same trips for every lane: the instruction does not mask)
+template <bool BF16, int NG, int WAVES, bool POLY>
+__device__ __forceinline__ void walk_branch(const ResidualBranch &b, uint32_t rows, uint32_t width, uint32_t n0, BranchLoads<BF16, NG> &l, BranchSums<NG> &o) {
+    constexpr uint32_t SPAN = 16 * Frag<BF16>::W, TRIP = BranchLoads<BF16, NG>::AHEAD * WAVES * SPAN;
+    uint32_t base = (threadIdx.x >> 6) * SPAN;
+    multiply_branch<BF16, NG, WAVES, POLY>(b, base, l, o);
+    for (base += TRIP; base < b.w.k; base += TRIP) {
+        ask_branch<BF16, NG, WAVES>(b, rows, width, n0, base, l);
+        multiply_branch<BF16, NG, WAVES, POLY>(b, base, l, o);
     }
 }
 
@@ -478,8 +504,13 @@ __global__ __launch_bounds__(WAVES * 64) void four_rows_residual_kernel(const Ro
         if (b0.gate.p) gate[0] = b0.gate.p[(int64_t)mr * b0.gate.pitch + n] + (b0.gate_bias ? b0.gate_bias[n] : 0.0f);
         if (NB > 1 && b1.gate.p) gate[NB - 1] = b1.gate.p[(int64_t)mr * b1.gate.pitch + n] + (b1.gate_bias ? b1.gate_bias[n] : 0.0f);
     }
-    walk_branch<BF16, NG, WAVES, POLY0>(b0, rows, width, n0, s[0]);
-    if (NB > 1) walk_branch<BF16, NG, WAVES, POLY1>(b1, rows, width, n0, s[NB - 1]);
+    BranchLoads<BF16, NG> loads[NB];
+    const uint32_t first = wave * 16 * Frag<BF16>::W;
+    ask_branch<BF16, NG, WAVES>(b0, rows, width, n0, first, loads[0]);
+    if (NB > 1) ask_branch<BF16, NG, WAVES>(b1, rows, width, n0, first, loads[NB - 1]);
+    __builtin_amdgcn_sched_barrier(0); // (or the compiler asks for a few at a time)
+    walk_branch<BF16, NG, WAVES, POLY0>(b0, rows, width, n0, loads[0], s[0]);
+    if (NB > 1) walk_branch<BF16, NG, WAVES, POLY1>(b1, rows, width, n0, loads[NB - 1], s[NB - 1]);
 #pragma unroll
     for (int b = 0; b < NB; b++) {
         const bool poly = b == 0 ? POLY0 : POLY1;
