@@ -21,7 +21,7 @@ typedef int int4v __attribute__((ext_vector_type(4)));
 struct TileArgs {
     const char *x, *w;
     void *y;                   // split s of y at y + s * M * N
-    uint32_t M, N;
+    uint32_t M, N, ld;         // ld: elements from row to row of y
     uint32_t K;                // bytes, as the pitches
     uint32_t x_pitch, w_pitch;
     uint32_t k_part;           // bytes of k per split, a multiple of kStageBytes
@@ -156,17 +156,18 @@ template <int FMT, int OUT, int MT> __global__ __launch_bounds__(kThreads) void 
 #pragma unroll
             for (int v = 0; v < 16; v++) { // the instruction's result: row 8 (v / 4) + 4 lg + v % 4, column li
                 const uint32_t m = m0 + wm + i * 32 + 8 * (v / 4) + 4 * lg + (v % 4);
-                if (m < a.M) put<OUT>(a.y, first + (uint64_t)m * a.N + n, acc[i][j][v]);
+                if (m < a.M) put<OUT>(a.y, first + (uint64_t)m * a.ld + n, acc[i][j][v]);
             }
         }
 }
 
-// y[e] = the parts' sum, in their order
-template <int OUT> __global__ __launch_bounds__(kThreads) void sum_parts_kernel(const float4v *part, void *y, uint32_t parts, uint64_t n4) {
-    const uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
+// y[e] = the parts' sum, in their order; row4 and ld4: fours of columns in a row of the parts, and from row to row of y
+template <int OUT> __global__ __launch_bounds__(kThreads) void sum_parts_kernel(const float4v *part, void *y, uint32_t parts, uint64_t n4, uint32_t row4, uint32_t ld4) {
+    uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
     if (i >= n4) return;
     float4v v = __builtin_nontemporal_load(part + i);
     for (uint32_t s = 1; s < parts; s++) v += __builtin_nontemporal_load(part + s * n4 + i);
+    if (row4 != ld4) i = i / row4 * ld4 + i % row4;
     if constexpr (OUT == kFmtWords) static_cast<float4v *>(y)[i] = v;
     else if constexpr (OUT == kFmtF8)
         static_cast<uint32_t *>(y)[i] = pattern<OUT>(v[0]) | pattern<OUT>(v[1]) << 8 | pattern<OUT>(v[2]) << 16 | pattern<OUT>(v[3]) << 24;
@@ -192,7 +193,8 @@ template <int FMT, int OUT> int run_tiles(cg_backend *be, TileArgs a) {
     const double start = low ? (f8 ? 4.2 : 6.1) : f8 ? 5.4 : 6.8, stage = low ? (f8 ? 0.31 : 0.114) : f8 ? 0.58 : 0.236, share = low ? (f8 ? 0.83 : 1.0) : f8 ? 0.68 : 0.765;
     uint32_t splits = 1;
     double best = 0;
-    for (uint32_t p = 1; p == 1 || (mn % 4 == 0 && p <= 16 && p * tiles <= room && a.K / p >= 256); p++) {
+    const bool fours = mn % 4 == 0 && (a.ld == a.N || (a.N % 4 == 0 && a.ld % 4 == 0));
+    for (uint32_t p = 1; p == 1 || (fours && p <= 16 && p * tiles <= room && a.K / p >= 256); p++) {
         const double rounds = std::ceil((double)(tiles * p) / be->compute_units), stages = ((a.K + p - 1) / p + kStageBytes - 1) / kStageBytes;
         const double us = start + stage * stages * std::max(1.0, share * rounds) + (p > 1 ? 0.9 + 0.15 * p + 1.44e-6 * p * mn : 0.0);
         if (p == 1 || us < best) splits = p, best = us;
@@ -206,14 +208,15 @@ template <int FMT, int OUT> int run_tiles(cg_backend *be, TileArgs a) {
         splits = 1; // no room for the parts: uncut
         a.k_part = (a.K + kStageBytes - 1) / kStageBytes * kStageBytes;
     }
-    if (splits > 1) a.y = parts;
+    const uint32_t ld = a.ld;
+    if (splits > 1) a.y = parts, a.ld = a.N;
     const dim3 grid((uint32_t)tiles, splits);
     const size_t lds = (size_t)kStages * (tm + kTileN) * kStageBytes;
     if (splits > 1) {
         if (low) hipLaunchKernelGGL((narrow_tile_kernel<FMT, kFmtWords, 1>), grid, dim3(kThreads), lds, be->stream, a);
         else hipLaunchKernelGGL((narrow_tile_kernel<FMT, kFmtWords, 2>), grid, dim3(kThreads), lds, be->stream, a);
         hipLaunchKernelGGL((sum_parts_kernel<OUT>), dim3((uint32_t)((mn / 4 + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream,
-                           static_cast<const float4v *>(parts), y, splits, mn / 4);
+                           static_cast<const float4v *>(parts), y, splits, mn / 4, a.N / 4, ld == a.N ? a.N / 4 : ld / 4);
         be->pool.free(parts, cls); // stream-ordered
     } else {
         if (low) hipLaunchKernelGGL((narrow_tile_kernel<FMT, OUT, 1>), grid, dim3(kThreads), lds, be->stream, a);
@@ -224,9 +227,11 @@ template <int FMT, int OUT> int run_tiles(cg_backend *be, TileArgs a) {
 
 } // namespace
 
-int launch_narrow_tiles(cg_backend *be, int fmt, const void *x, int64_t x_pitch, int64_t rows, const void *w, int64_t w_pitch, int64_t n, int64_t k, void *y, int y_fmt) {
+int launch_narrow_tiles(cg_backend *be, int fmt, const void *x, int64_t x_pitch, int64_t rows, const void *w, int64_t w_pitch, int64_t n, int64_t k, void *y, int y_fmt,
+                        int64_t y_pitch) {
     const int64_t eb = (int64_t)fmt_bytes(fmt);
     if (fmt == kFmtWords || !fits_narrow_tiles(fmt, x_pitch, rows, w_pitch, n, k)) return kDeclined;
+    if (y_pitch != 0 && (y_pitch < n || y_pitch >= (1ll << 31))) return kDeclined;
     if (!x || !w || reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16) return kDeclined;
     TileArgs a{};
     a.x = static_cast<const char *>(x);
@@ -234,6 +239,7 @@ int launch_narrow_tiles(cg_backend *be, int fmt, const void *x, int64_t x_pitch,
     a.y = y;
     a.M = (uint32_t)rows;
     a.N = (uint32_t)n;
+    a.ld = (uint32_t)(y_pitch ? y_pitch : n);
     a.K = (uint32_t)(k * eb);
     a.x_pitch = (uint32_t)(x_pitch * eb);
     a.w_pitch = (uint32_t)(w_pitch * eb);

@@ -20,6 +20,7 @@ struct MmArgs {
     uint32_t batch;
     uint32_t a_vec, b_vec;          // 16-byte loads along the unit-stride axis are legal
     uint32_t ksplit;                // tiled kernels: values of k per workgroup along grid.z (a multiple of 32), 0 = all of K
+    uint32_t n_tiles;               // mfma_gemm_dlds_kernel: columns of tiles that it computes, from the first; 0 = all
     uint32_t c_fmt;                 // mfma_gemm_dlds_kernel: kFmtWords, or the operands' narrow format: C holds its patterns, rounded in the store
 };
 
@@ -40,8 +41,9 @@ __device__ __forceinline__ void batch_offsets(const MmArgs &a, uint32_t b, int64
 int launch_split_gemm(cg_backend *be, MmArgs a, bool a_mfast, bool b_nfast);
 
 
-// y[rows, n] = x[rows, k] . w[n, k]^T of patterns of one narrow format (block_products.hip); pitches in elements; y dense, words or
-// patterns of that format.  kDeclined: operands that fits_narrow_tiles does not take or that are not 16-byte aligned.
-int launch_narrow_tiles(cg_backend *be, int fmt, const void *x, int64_t x_pitch, int64_t rows, const void *w, int64_t w_pitch, int64_t n, int64_t k, void *y, int y_fmt);
+// y[rows, n] = x[rows, k] . w[n, k]^T of patterns of one narrow format (block_products.hip); pitches in elements; y's rows y_pitch
+// apart (0: dense), words or patterns of that format.  kDeclined: operands that fits_narrow_tiles does not take or that are not 16-byte aligned.
+int launch_narrow_tiles(cg_backend *be, int fmt, const void *x, int64_t x_pitch, int64_t rows, const void *w, int64_t w_pitch, int64_t n, int64_t k, void *y, int y_fmt,
+                        int64_t y_pitch = 0);
 
 } // namespace cg

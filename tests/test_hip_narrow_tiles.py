@@ -86,3 +86,30 @@ def test_fp8_results_at_the_ends_of_the_range(hip, M):
     # everything from 448 up is 448; below, one rounding to the dtype of a sum of 256 roundings of at most 448 * 2^-24 each
     near, keep = np.clip(exact, -448, 448), ~np.isnan(want)
     assert (np.abs(got - near)[keep] <= UNIT["fp8"] * np.abs(near[keep]) + 2.0 ** -10 + 2 * K * 2.0 ** -24 * 448).all()
+
+
+@pytest.mark.parametrize("dtype", [A.BF16, A.F16])
+@pytest.mark.parametrize("shape", [(1024, 16484, 256), (1024, 16387, 128), (1030, 13412, 384), (2048, 8448, 1280), (8192, 2052, 128), (300, 65600, 128), (66600, 200, 128), (66600, 500, 128)])
+def test_columns_left_over_by_the_rounds_of_wide_tiles(hip, dtype, shape):
+    """Results whose last few 256-wide tiles would be a round of their own: those columns come from the 128-wide tiles, beside the others in
+    the same rows (rounded in the store, or as words where a row is no whole number of fours), cut along k or not."""
+    import torch
+
+    M, N, K = shape
+    rng = np.random.default_rng(M + N + K)
+    x, w = (torch.from_numpy(rng.standard_normal(s, dtype=np.float32)) for s in ((M, K), (N, K)))
+    kind = torch.bfloat16 if dtype == A.BF16 else torch.float16
+    x, w = x.to(kind), w.to(kind)
+
+    def up(t):
+        if dtype == A.BF16:
+            return hip.ndarray_from_vec_bf16(t.view(torch.int16).numpy().view(np.uint16), tuple(t.shape))
+        return hip.ndarray_from_vec_f16(t.view(torch.int16).numpy().view(np.float16), tuple(t.shape))
+
+    tx, tw = hip.reshape(up(x).move(), (1, M, K)), up(w)
+    y = hip.matmul(tx, hip.broadcast(hip.transpose(tw, 0, 1), (1, K, N)).move())
+    got = hip.to_numpy(hip.cast(y.move(), A.F32))[0]
+    want = (x.cuda().float() @ w.cuda().float().T).cpu().numpy()
+    # the result's rounding, and the sums' in 32 bits
+    unit = 2.0 ** -8 if dtype == A.BF16 else 2.0 ** -11
+    assert (np.abs(got - want) <= unit * np.abs(want) + 1e-5 * K ** 0.5).all()
