@@ -39,17 +39,27 @@ __device__ __forceinline__ float softplus(float z) {
 }
 
 // Channel c of the three projections side by side: where its column of tokens begins (at sequence b, token 0), and its taps.
-// (Values are selected, not references: a reference into the arguments would have them fetched lane by lane.)
+// (Arguments are pinned to scalar registers before a lane chooses among them: left to itself the compiler chooses their place in
+// the argument block and has every lane fetch from there, a trip to memory in front of all others.)
+typedef const __attribute__((address_space(1))) float global_float;
+__device__ __forceinline__ int64_t pinned(int64_t v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+__device__ __forceinline__ global_float *pinned(const float *p) { return reinterpret_cast<global_float *>(pinned(reinterpret_cast<int64_t>(p))); }
 struct Channel {
-    const float *x, *taps;
+    global_float *x, *taps;
     int64_t pitch;
 };
 __device__ __forceinline__ Channel channel(const DeltaPlan &p, uint32_t b, uint32_t c) {
     const uint32_t kc = p.kv_heads * p.dim;
     const bool is_q = c < kc, is_k = c < 2 * kc;
     const uint32_t e = is_q ? c : is_k ? c - kc : c - 2 * kc;
-    const float *x = is_q ? p.q.p : is_k ? p.k.p : p.v.p, *w = is_q ? p.conv_q : is_k ? p.conv_k : p.conv_v;
-    const int64_t pitch = is_q ? p.q.pitch : is_k ? p.k.pitch : p.v.pitch;
+    global_float *const xq = pinned(p.q.p), *const xk = pinned(p.k.p), *const xv = pinned(p.v.p);
+    global_float *const wq = pinned(p.conv_q), *const wk = pinned(p.conv_k), *const wv = pinned(p.conv_v);
+    const int64_t pq = pinned(p.q.pitch), pk = pinned(p.k.pitch), pv = pinned(p.v.pitch);
+    global_float *x = is_q ? xq : is_k ? xk : xv, *w = is_q ? wq : is_k ? wk : wv;
+    const int64_t pitch = is_q ? pq : is_k ? pk : pv;
     return {x + (int64_t)b * p.S * pitch + e, w + (int64_t)e * p.taps, pitch};
 }
 // its input at time t (t < 0: what the state kept)
@@ -70,8 +80,9 @@ constexpr uint32_t kChunk = 16;
 __device__ __forceinline__ float exp2_of(float x) { return __builtin_amdgcn_exp2f(x); } // (x <= 0)
 
 // log2 of the decay of key channel d of head h
+__device__ __forceinline__ float log2_decay(float a_log, float dt) { return -expf(a_log) * softplus(dt) * kLog2e; }
 __device__ __forceinline__ float log2_decay(const DeltaPlan &p, float a, uint32_t h, uint32_t d) {
-    return -expf(p.a_log[h]) * softplus(a + p.dt_bias[h * p.dim + d]) * kLog2e;
+    return log2_decay(p.a_log[h], a + p.dt_bias[h * p.dim + d]);
 }
 
 // The last taps - 1 inputs of head h's channels (of its q and k channels if it is the first head that uses them).
@@ -99,7 +110,7 @@ __device__ __host__ constexpr uint32_t chunk_floats(uint32_t dp) { return 48 * d
 template <int TAPS> __device__ __forceinline__ void conv_chunk(const DeltaPlan &p, uint32_t b, uint32_t t0, uint32_t n, uint32_t c, float (&y)[kChunk]) {
     if constexpr (TAPS > 0) {
         const Channel ch = channel(p, b, c);
-        const float *x = ch.x + (int64_t)t0 * ch.pitch;
+        global_float *x = ch.x + (int64_t)t0 * ch.pitch;
         float in[kChunk + TAPS - 1], wt[TAPS];
 #pragma unroll
         for (uint32_t t = 0; t < kChunk; t++) in[t + TAPS - 1] = x[(int64_t)min(t, n - 1) * ch.pitch]; // (clamped, not tested: no load waits)
@@ -392,6 +403,17 @@ __device__ __forceinline__ float step_sum(float v, float *red) { // over the wor
     for (int i = 0; i < kStepThreads / 64; i++) s += red[i];
     return s;
 }
+// the same for two values
+__device__ __forceinline__ void step_sum2(float &a, float &b, float2 *red) {
+    a = wave_sum(a);
+    b = wave_sum(b);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = make_float2(a, b);
+    __syncthreads();
+    a = b = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kStepThreads / 64; i++) a += red[i].x, b += red[i].y;
+}
 // w[row, :] . x, four lanes of a quad together
 __device__ __forceinline__ float quad_dot(const float *__restrict__ w, const float *__restrict__ x, uint32_t n, uint32_t sub) {
     float s = 0.0f;
@@ -419,52 +441,121 @@ __device__ __forceinline__ float quad_dot(const float *__restrict__ w, const flo
     return s;
 }
 
-// conv_silu with the inputs and taps asked for together when there are TAPS of them
-template <int TAPS> __device__ __forceinline__ float conv_step(const DeltaPlan &p, uint32_t b, int t, uint32_t c) {
-    if constexpr (TAPS == 0) {
-        return conv_silu(p, b, t, c);
-    } else {
+// conv_silu of TAPS taps in two halves: its inputs and taps asked for, and the rest
+template <int TAPS> struct ConvLoads {
+    float x[TAPS], tap[TAPS];
+    __device__ __forceinline__ void ask(const DeltaPlan &p, uint32_t b, int t, uint32_t c) {
         const uint32_t C = 2 * p.kv_heads * p.dim + p.heads * p.vdim;
         const Channel ch = channel(p, b, c);
-        const float *now = ch.x + (int64_t)t * ch.pitch;
-        const float *kept = p.conv_state ? p.conv_state + ((int64_t)b * (TAPS - 1) + t + TAPS - 1) * C + c : now;
+        global_float *now = ch.x + (int64_t)t * ch.pitch;
+        global_float *kept = p.conv_state ? (global_float *)p.conv_state + ((int64_t)b * (TAPS - 1) + t + TAPS - 1) * C + c : now;
         const int64_t kept_pitch = p.conv_state ? C : 0;
-        float x[TAPS], tap[TAPS], s = 0.0f;
 #pragma unroll
         for (int i = 0; i < TAPS; i++) {
             const int back = TAPS - 1 - i; // tokens before t
             tap[i] = ch.taps[i];
             x[i] = *(back <= t ? now - (int64_t)back * ch.pitch : kept - (int64_t)back * kept_pitch); // (one load, whichever it is)
         }
+    }
+    __device__ __forceinline__ float value(const DeltaPlan &p, int t) const {
+        float s = 0.0f;
 #pragma unroll
-        for (int i = 0; i < TAPS; i++) x[i] = TAPS - 1 - i <= t || p.conv_state ? x[i] : 0.0f;
-#pragma unroll
-        for (int i = 0; i < TAPS; i++) s = fmaf(x[i], tap[i], s);
+        for (int i = 0; i < TAPS; i++) s = fmaf(TAPS - 1 - i <= t || p.conv_state ? x[i] : 0.0f, tap[i], s);
         return s * sigmoid(s);
+    }
+};
+template <int TAPS> __device__ __forceinline__ float conv_step(const DeltaPlan &p, uint32_t b, int t, uint32_t c) {
+    if constexpr (TAPS == 0) {
+        return conv_silu(p, b, t, c);
+    } else {
+        ConvLoads<TAPS> l;
+        l.ask(p, b, t, c);
+        return l.value(p, t);
     }
 }
 
+// A lane's quarter of w . x for up to kDotQuads * 16 values of k, 16 bytes at a time: asked for, and added up over its quad of lanes
+constexpr int kDotQuads = 8;
+struct DotLoads {
+    float4 a[kDotQuads], c[kDotQuads];
+    // (w and x: the same for all lanes, so that a lane's addresses are 32-bit offsets)
+    __device__ __forceinline__ void ask(const float *__restrict__ w, uint32_t row, const float *__restrict__ x, uint32_t n, uint32_t sub) {
+#pragma unroll
+        for (int j = 0; j < kDotQuads; j++) {
+            const uint32_t at = min(sub + 4 * j, n / 4 - 1);
+            a[j] = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(w) + (row * n + at * 4) * 4);
+            c[j] = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(x) + at * 16);
+        }
+    }
+    __device__ __forceinline__ float value(uint32_t n, uint32_t sub) const {
+        float s = 0.0f;
+#pragma unroll
+        for (int j = 0; j < kDotQuads; j++) {
+            const float t = fmaf(a[j].x, c[j].x, fmaf(a[j].y, c[j].y, fmaf(a[j].z, c[j].z, a[j].w * c[j].w)));
+            s += sub + 4 * j < n / 4 ? t : 0.0f;
+        }
+        s += __shfl_xor(s, 1, 64);
+        s += __shfl_xor(s, 2, 64);
+        return s;
+    }
+};
+
 // Thread (c, group) holds rows group, group + groups, ... (at most R) of column c of the head's state.
-template <int R, int TAPS> __global__ __launch_bounds__(kStepThreads) void delta_step_kernel(const DeltaPlan p, const uint32_t lanes) {
+// DIRECT: one token behind a state; a thread has at most one channel of the convolutions and a row of each factored projection, and these have ranks of at
+// most 128 in 16-byte pieces (launch_delta_step).  Then all of a token's loads are asked for together, and ahead of the state, whose
+// 64 KB for 128 x 128 a compute unit takes 2 us to fetch: nothing of the token waits for it.  One after the other: 14.9 us, 13.1 so
+// (what is left is mostly the state and the factors, 200 KB through one compute unit).
+template <int R, int TAPS, bool DIRECT> __global__ __launch_bounds__(kStepThreads) void delta_step_kernel(const DeltaPlan p, const uint32_t lanes) {
     __shared__ float q[257], k[257], g[257], v[kStepThreads], gate[kStepThreads], part[kStepThreads], red[kStepThreads / 64];
+    __shared__ float2 red2[kStepThreads / 64];
     const uint32_t h = blockIdx.x, b = blockIdx.y, rep = p.heads / p.kv_heads, kh = h / rep, D = p.dim, V = p.vdim, kc = p.kv_heads * D;
     const uint32_t tid = threadIdx.x, c = tid & (lanes - 1), group = tid / lanes, groups = kStepThreads / lanes;
     const int64_t sb = ((int64_t)b * p.heads + h) * D * V;
+    constexpr uint32_t ROWS = kStepThreads / 4; // rows of the factored projections per round
+    ConvLoads<TAPS ? TAPS : 1> conv;
+    DotLoads dot[DIRECT ? 2 : 1];
+    auto channel_of = [&](uint32_t u) { return u < D ? kh * D + u : u < 2 * D ? kc + kh * D + u - D : 2 * kc + h * V + u - 2 * D; };
+    auto ask = [&](uint32_t t) {
+        const int64_t r = (int64_t)b * p.S + t;
+        conv.ask(p, b, (int)t, channel_of(min(tid, 2 * D + V - 1)));
+        dot[0].ask(p.decay_w + (int64_t)h * D * p.decay_rank, min(tid / 4, D - 1), p.decay.p + r * p.decay.pitch, p.decay_rank, tid & 3);
+        dot[DIRECT].ask(p.gate_w + (int64_t)h * V * p.gate_rank, min(tid / 4, V - 1), p.gate.p + r * p.gate.pitch, p.gate_rank, tid & 3);
+    };
+    float dt_bias = 0.0f, a_log = 0.0f, beta_in = 0.0f, weight = 0.0f;
+    if constexpr (DIRECT) {
+        ask(0);
+        a_log = p.a_log[h];
+        dt_bias = p.dt_bias[h * D + min(tid / 4, D - 1)];
+        beta_in = p.beta.p[(int64_t)b * p.beta.pitch + h];
+        weight = p.norm[min(c, V - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+    }
     float S[R];
-    if (p.state) { // (clamped, not tested: no load waits)
-        const float *src = p.state + sb + min(c, V - 1);
+    if (DIRECT || p.state) { // (clamped, not tested: no load waits)
+        const char *const src = reinterpret_cast<const char *>(p.state + sb);
+        const uint32_t col = min(c, V - 1);
 #pragma unroll
-        for (int i = 0; i < R; i++) S[i] = src[(int64_t)min(group + i * groups, D - 1) * V];
-#pragma unroll
-        for (int i = 0; i < R; i++) S[i] = group + i * groups < D ? S[i] : 0.0f;
+        for (int i = 0; i < R; i++) S[i] = *reinterpret_cast<const float *>(src + (min(group + i * groups, D - 1) * V + col) * 4); // (D, V: a few hundred)
     } else {
 #pragma unroll
         for (int i = 0; i < R; i++) S[i] = 0.0f;
     }
     if (tid == 0) q[D] = k[D] = g[D] = 0.0f; // what the rows behind the last one read
-    for (uint32_t t = 0; t < p.S; t++) {
+    for (uint32_t t = 0; t < (DIRECT ? 1 : p.S); t++) {
         const int64_t r = (int64_t)b * p.S + t;
         float sq = 0.0f, sk = 0.0f;
+        if constexpr (DIRECT) {
+            const float x = conv.value(p, (int)t);
+            if (tid < 2 * D + V) {
+                (tid < D ? q[tid] : tid < 2 * D ? k[tid - D] : v[tid - 2 * D]) = x;
+                sq = tid < D ? x * x : 0.0f;
+                sk = tid >= D && tid < 2 * D ? x * x : 0.0f;
+            }
+            const uint32_t e = tid / 4;
+            const float decay = dot[0].value(p.decay_rank, tid & 3), open = dot[DIRECT].value(p.gate_rank, tid & 3);
+            if ((tid & 3) == 0 && e < D) g[e] = exp2_of(log2_decay(a_log, decay + dt_bias));
+            if ((tid & 3) == 0 && e < V) gate[e] = sigmoid(open);
+        } else
         for (uint32_t u = tid; u < 2 * D + V; u += kStepThreads) {
             const bool is_q = u < D, is_k = !is_q && u < 2 * D;
             const uint32_t e = is_q ? u : is_k ? u - D : u - 2 * D;
@@ -473,7 +564,7 @@ template <int R, int TAPS> __global__ __launch_bounds__(kStepThreads) void delta
             sk = is_k ? fmaf(x, x, sk) : sk;
             (is_q ? q : is_k ? k : v)[e] = x;
         }
-        for (uint32_t u = tid / 4; u < D + V; u += kStepThreads / 4) { // the two factored projections
+        for (uint32_t u = tid / 4; !DIRECT && u < D + V; u += ROWS) { // the two factored projections
             const bool is_g = u < D;
             const uint32_t e = is_g ? u : u - D;
             const float a = quad_dot(is_g ? p.decay_w + ((int64_t)h * D + e) * p.decay_rank : p.gate_w + ((int64_t)h * V + e) * p.gate_rank,
@@ -483,8 +574,12 @@ template <int R, int TAPS> __global__ __launch_bounds__(kStepThreads) void delta
                 else gate[e] = sigmoid(a);
             }
         }
-        const float fq = 1.0f / sqrtf(step_sum(sq, red) + 1e-6f) * (1.0f / sqrtf((float)D)), fk = 1.0f / sqrtf(step_sum(sk, red) + 1e-6f);
-        const float beta = sigmoid(p.beta.p[r * p.beta.pitch + h]);
+        step_sum2(sq, sk, red2);
+        if (DIRECT || t == 0) // rows behind the last one hold what the clamped loads brought
+#pragma unroll
+            for (int i = 0; i < R; i++) S[i] = group + i * groups < D ? S[i] : 0.0f;
+        const float fq = 1.0f / sqrtf(sq + 1e-6f) * (1.0f / sqrtf((float)D)), fk = 1.0f / sqrtf(sk + 1e-6f);
+        const float beta = sigmoid(DIRECT ? beta_in : p.beta.p[r * p.beta.pitch + h]);
         float read = 0.0f; // (the sums above end behind a barrier: q, k, v, g and gate are there)
 #pragma unroll
         for (int i = 0; i < R; i++) {
@@ -511,8 +606,8 @@ template <int R, int TAPS> __global__ __launch_bounds__(kStepThreads) void delta
         if (group == 0)
             for (uint32_t i = 0; i < groups; i++) y += part[i * lanes + c];
         const float f = 1.0f / sqrtf(step_sum(group == 0 && c < V ? y * y : 0.0f, red) / (float)V + p.eps);
-        if (group == 0 && c < V) p.out[r * p.heads * V + h * V + c] = y * f * p.norm[c] * gate[c];
-        __syncthreads(); // the next token overwrites what this one reads
+        if (group == 0 && c < V) p.out[r * p.heads * V + h * V + c] = y * f * (DIRECT ? weight : p.norm[c]) * gate[c];
+        if (!DIRECT) __syncthreads(); // the next token overwrites what this one reads
     }
     keep_inputs(p, b, h);
 #pragma unroll
@@ -632,13 +727,22 @@ int launch_channel_delta(cg_backend *be, const DeltaPlan &p) {
     if (step_shape(p, &lanes, &held)) {
         ProfScope prof(be, CG_K_RECURRENCE, flop * rows);
         const dim3 grid(p.heads, p.B);
-#define CG_STEP(R)                                                                                                          \
-    if (p.taps == 4) hipLaunchKernelGGL((delta_step_kernel<R, 4>), grid, dim3(kStepThreads), 0, be->stream, p, lanes);      \
-    else hipLaunchKernelGGL((delta_step_kernel<R, 0>), grid, dim3(kStepThreads), 0, be->stream, p, lanes)
-        if (held <= 4) { CG_STEP(4); }
-        else if (held <= 16) { CG_STEP(16); }
-        else if (held <= 32) { CG_STEP(32); }
-        else { CG_STEP(64); }
+        auto pieces = [](const float *w, uint32_t rank, const Rows &x) {
+            return rank >= 4 && rank <= 16 * kDotQuads && rank % 4 == 0 && x.pitch % 4 == 0 && ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x.p)) & 15) == 0;
+        };
+        const bool direct = p.S == 1 && p.state && p.taps == 4 && 2 * p.dim + p.vdim <= kStepThreads && p.dim <= kStepThreads / 4 && p.vdim <= kStepThreads / 4 && pieces(p.decay_w, p.decay_rank, p.decay) &&
+                            pieces(p.gate_w, p.gate_rank, p.gate);
+#define CG_STEP(R, DIRECT)                                                                                                                \
+    if (DIRECT) hipLaunchKernelGGL((delta_step_kernel<R, 4, DIRECT>), grid, dim3(kStepThreads), 0, be->stream, p, lanes);                \
+    else if (p.taps == 4) hipLaunchKernelGGL((delta_step_kernel<R, 4, false>), grid, dim3(kStepThreads), 0, be->stream, p, lanes);       \
+    else hipLaunchKernelGGL((delta_step_kernel<R, 0, false>), grid, dim3(kStepThreads), 0, be->stream, p, lanes)
+        if (direct && held <= 4) { CG_STEP(4, true); }
+        else if (direct && held <= 16) { CG_STEP(16, true); }
+        else if (direct) { CG_STEP(32, true); } // (128 rows by four groups)
+        else if (held <= 4) { CG_STEP(4, false); }
+        else if (held <= 16) { CG_STEP(16, false); }
+        else if (held <= 32) { CG_STEP(32, false); }
+        else { CG_STEP(64, false); }
 #undef CG_STEP
         return launched("channel_delta step");
     }
