@@ -152,14 +152,14 @@ __device__ __forceinline__ void aot_load_leaf(const FusedArgs &a, const int64_t 
         for (int j = 0; j < VEC; j++) t[j] = a.leaf[L].ubits;
     } else if constexpr (L == P::pw) {
         const bool second = e >= a.pw_split;
-        if (second) load_words<VEC, false, words_only_of<P>::value>(a.leaf2, off[P::nleaf], t);
-        else load_words<VEC, false, words_only_of<P>::value>(a.leaf[L], off[L], t);
+        if (second) load_words<VEC, false, words_only_of<P>::value, true>(a.leaf2, off[P::nleaf], t);
+        else load_words<VEC, false, words_only_of<P>::value, true>(a.leaf[L], off[L], t);
         if ((a.pw_neg >> (second ? 1 : 0)) & 1u) {
 #pragma unroll
             for (int j = 0; j < VEC; j++) t[j] ^= 0x80000000u;
         }
     } else {
-        load_words<VEC, false, words_only_of<P>::value>(a.leaf[L], off[L], t);
+        load_words<VEC, false, words_only_of<P>::value, true>(a.leaf[L], off[L], t);
     }
 }
 

@@ -120,7 +120,16 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
         g.q_bs[d] = f1.a_bs[d];
         g.k_bs[d] = f1.b_bs[d];
         g.v_bs[d] = f2.b_bs[d];
-        g.p_bs[d] = f2.a_bs[d];
+        g.p_rows[d] = f2.a_bs[d] / T;
+    }
+    // (the kernels read two axes of the entries and of the program's rows whatever their number: see entry_offsets)
+    for (int d = f1.nb; d < kMaxBatchAxes; d++) {
+        g.bd[d] = 1;
+        g.bdiv[d] = make_fastdiv(1);
+    }
+    for (uint32_t d = a.g.nouter; d < (uint32_t)kMaxOuter; d++) {
+        a.g.od[d] = 1;
+        a.g.odiv[d] = make_fastdiv(1);
     }
     g.q_sm = f1.a_sm;
     g.k_st = f1.b_sn;
@@ -219,6 +228,7 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
         const int passes = seglen <= 5 * per_pass ? 5 : seglen <= 10 * per_pass ? 10 : seglen <= 16 * per_pass ? 16 : 0;
         const bool halves = qrows * nseg * 2 <= attn_row_halves_below(); // two workgroups per row still leave compute units idle
         const dim3 grid((uint32_t)((f1.batch + 7) / 8 * 8 * g.M * (halves ? 2 : 1)), nseg), block(kRowBlock);
+        g.groups = make_fastdiv(g.M * (halves ? 2 : 1));
 #define CG_ROW_KERNEL(LPT, VS)                                                                                                     \
     do {                                                                                                                           \
         if (passes == 5) hipLaunchKernelGGL((decode_attention_row_kernel<P, LPT, 5, false, VS>), grid, block, 0, be->stream, g, a, po);   \

@@ -53,9 +53,12 @@ struct AttnArgs {
     float *part_ml; // [batch][splits][M][2]
     uint32_t M, T, hd, splits, chunk;
     uint32_t nb;
+    FastDiv groups; // decode, a workgroup per row: rows x parts of an entry
+    // batch axes; decode: the slots behind nb hold axes of extent one
     uint32_t bd[kMaxBatchAxes];
     FastDiv bdiv[kMaxBatchAxes];
-    int64_t q_bs[kMaxBatchAxes], k_bs[kMaxBatchAxes], v_bs[kMaxBatchAxes], p_bs[kMaxBatchAxes];
+    int64_t q_bs[kMaxBatchAxes], k_bs[kMaxBatchAxes], v_bs[kMaxBatchAxes];
+    int64_t p_rows[kMaxBatchAxes]; // decode: rows of the soft-max program per step of the axis
     int64_t q_sm; // stride between the query rows of a group
     int64_t k_st; // stride between cached positions of K (head_dim contiguous)
     int64_t v_st; // stride between cached positions of V (head_dim contiguous)
@@ -64,6 +67,41 @@ struct AttnArgs {
     uint32_t vbd[kMaxBatchAxes];
     FastDiv vbdiv[kMaxBatchAxes];
 };
+
+// Operand offsets of batch entry b, and its first row in the soft-max program's [rows, T] space.  Two axes are read without a test (as a
+// rule there are no more): a test in front of every axis is a trip to the argument block for every axis, a third of a microsecond each
+// before the first load of K goes out.
+__device__ __forceinline__ void entry_offsets(const AttnArgs &g, uint32_t b, int64_t &oq, int64_t &ok, int64_t &ov, uint32_t &row) {
+    oq = ok = ov = 0;
+    row = 0;
+    auto axis = [&](const uint32_t d) {
+        const uint32_t q = fastdiv(b, g.bdiv[d]), i = b - q * g.bd[d];
+        b = q;
+        oq += (int64_t)i * g.q_bs[d];
+        ok += (int64_t)i * g.k_bs[d];
+        ov += (int64_t)i * g.v_bs[d];
+        row += i * (uint32_t)g.p_rows[d];
+    };
+    axis(0);
+    axis(1);
+    if (g.nb > 2)
+        for (uint32_t d = 2; d < g.nb; d++) axis(d);
+}
+// the offsets of a row of that space in the program's leaves but the first, likewise
+template <class P> __device__ __forceinline__ void leaf_offsets(const FusedArgs &a, uint32_t row, int64_t (&base)[P::nleaf + 1]) {
+#pragma unroll
+    for (int i = 0; i <= P::nleaf; i++) base[i] = 0;
+    auto axis = [&](const uint32_t d) {
+        const uint32_t q = fastdiv(row, a.g.odiv[d]), i = row - q * a.g.od[d];
+        row = q;
+#pragma unroll
+        for (int lf = 1; lf < P::nleaf; lf++) base[lf] += (int64_t)i * a.leaf[lf].os[d];
+    };
+    axis(0);
+    axis(1);
+    if (a.g.nouter > 2)
+        for (uint32_t d = 2; d < a.g.nouter; d++) axis(d);
+}
 
 constexpr int kAttnRows = 8;    // most query rows per KV head
 constexpr int kAttnPasses = 8; // cached positions per lane group and workgroup
@@ -89,24 +127,9 @@ __global__ __launch_bounds__(kBlock) void decode_attention_kernel(const AttnArgs
     const uint32_t split = blockIdx.x, b = blockIdx.y;
     const uint32_t t0 = split * g.chunk, t1 = min(g.T, t0 + g.chunk);
     // operand offsets of this batch entry
-    int64_t oq = 0, ok = 0, ov = 0, op = 0;
-    {
-        uint32_t bb = b;
-        // (every axis slot is visited, so that the fields are read from the argument block at once instead of one
-        // dependent scalar load after the other)
-#pragma unroll
-        for (uint32_t d = 0; d < (uint32_t)kMaxBatchAxes; d++) {
-            if (d >= g.nb) break;
-            const uint32_t q = fastdiv(bb, g.bdiv[d]);
-            const int64_t i = (int64_t)(bb - q * g.bd[d]);
-            bb = q;
-            oq += i * g.q_bs[d];
-            ok += i * g.k_bs[d];
-            ov += i * g.v_bs[d];
-            op += i * g.p_bs[d];
-        }
-    }
-    const uint32_t row0 = (uint32_t)(op / g.T); // first row of this group in the program's [rows, T] space
+    int64_t oq, ok, ov;
+    uint32_t row0; // first row of this group in the program's [rows, T] space
+    entry_offsets(g, b, oq, ok, ov, row0);
     const uint32_t l = tid % LPT, sub = tid / LPT;
 
     float4v kf[kAttnPasses], vf[kAttnPasses];
@@ -290,96 +313,44 @@ __global__ __launch_bounds__(kRowBlock) void decode_attention_row_kernel(const A
     const uint32_t seg = blockIdx.y, t_first = seg * g.chunk;
     const uint32_t T = min(g.T, t_first + g.chunk) - t_first; // positions of this workgroup
     // block -> (batch entry, query row, half): the workgroups of an entry eight blocks apart
-    const uint32_t rest = blockIdx.x / 8, inner = rest % (g.M * VS), m = inner / VS, part = inner % VS;
-    const uint32_t b = rest / (g.M * VS) * 8 + blockIdx.x % 8;
+    const uint32_t rest = blockIdx.x / 8, eight = fastdiv(rest, g.groups), inner = rest - eight * g.M * VS, m = inner / VS, part = inner % VS;
+    const uint32_t b = eight * 8 + blockIdx.x % 8;
     if (b >= g.splits) return; // (the number of batch entries; the same for the whole workgroup)
-    int64_t oq = 0, ok = 0, ov = 0, op = 0;
-    {
-        uint32_t bb = b;
-        // (every axis slot is visited, so that the fields are read from the argument block up front and at once
-        // instead of one dependent scalar load after the other)
-#pragma unroll
-        for (uint32_t d = 0; d < (uint32_t)kMaxBatchAxes; d++) {
-            if (d >= g.nb) break;
-            const uint32_t q = fastdiv(bb, g.bdiv[d]);
-            const int64_t i = (int64_t)(bb - q * g.bd[d]);
-            bb = q;
-            oq += i * g.q_bs[d];
-            ok += i * g.k_bs[d];
-            ov += i * g.v_bs[d];
-            op += i * g.p_bs[d];
-        }
-    }
+    int64_t oq, ok, ov;
+    uint32_t row0; // first row of this group in the program's [rows, T] space
+    entry_offsets(g, b, oq, ok, ov, row0);
     const uint32_t l = tid % LPT, sub = tid / LPT, lv = tid % LPV, subv = tid / LPV;
     const uint32_t *kbase = g.Kc + ok + (int64_t)t_first * g.k_st + l * 4;
     const uint32_t *vbase = g.V + ov + (int64_t)t_first * g.v_st + (part * LPV + lv) * 4;
-    // FULL (a tag type): the trip lies inside the T positions, nothing is checked
-    const int64_t k_step = (int64_t)TPB * g.k_st, v_step = (int64_t)TPV * g.v_st;
-    auto ask_k = [&](float4v (&f)[PASSES], uint32_t first, auto full) {
-        const uint32_t *p = kbase + (int64_t)(first + sub) * g.k_st;
-#pragma unroll
-        for (int ps = 0; ps < PASSES; ps++) {
-            if constexpr (decltype(full)::value) {
-                f[ps] = *reinterpret_cast<const float4v *>(p);
-            } else {
-                f[ps] = (float4v){0.f, 0.f, 0.f, 0.f};
-                if (first + sub + ps * TPB < T) f[ps] = *reinterpret_cast<const float4v *>(p);
-            }
-            p += k_step;
-        }
-    };
-    auto ask_v = [&](float4v (&f)[PASSES_V], uint32_t first, auto full) {
-        const uint32_t *p = vbase + (int64_t)(first + subv) * g.v_st;
-#pragma unroll
-        for (int ps = 0; ps < PASSES_V; ps++) {
-            if constexpr (decltype(full)::value) {
-                f[ps] = *reinterpret_cast<const float4v *>(p);
-            } else {
-                f[ps] = (float4v){0.f, 0.f, 0.f, 0.f};
-                if (first + subv + ps * TPV < T) f[ps] = *reinterpret_cast<const float4v *>(p);
-            }
-            p += v_step;
-        }
-    };
-    constexpr std::true_type whole_trip{};
-    constexpr std::false_type ragged{};
-    // the trip that starts at `first`, checked only when it reaches beyond T
+    // the trip that starts at `first`.  Positions beyond the last are clamped, not tested: with a test in front of every load the
+    // compiler knows of none that is on its way, and the first score waits for all of K and V.  (What they bring is not used.)
     auto ask_k_at = [&](float4v (&f)[PASSES], uint32_t first) {
-        if (first + SPAN <= T) ask_k(f, first, whole_trip);
-        else ask_k(f, first, ragged);
+#pragma unroll
+        for (int ps = 0; ps < PASSES; ps++) f[ps] = *reinterpret_cast<const float4v *>(kbase + (int64_t)min(first + sub + ps * TPB, T - 1) * g.k_st);
     };
     auto ask_v_at = [&](float4v (&f)[PASSES_V], uint32_t first) {
-        if (first + SPAN_V <= T) ask_v(f, first, whole_trip);
-        else ask_v(f, first, ragged);
+#pragma unroll
+        for (int ps = 0; ps < PASSES_V; ps++) f[ps] = *reinterpret_cast<const float4v *>(vbase + (int64_t)min(first + subv + ps * TPV, T - 1) * g.v_st);
     };
+    // (tag types: a trip inside the T positions, and one that ends beyond them)
+    constexpr std::true_type whole_trip{};
+    constexpr std::false_type ragged{};
     float4v ka[PASSES], kb[LOOP ? PASSES : 1];
     float4v va[PASSES_V], vb[LOOP ? PASSES_V : 1];
-    ask_k_at(ka, 0);
-    if constexpr (V_EARLY) ask_v_at(va, 0);
+    // (loads come back in the order in which they are asked for: the query and K, the leaves, V)
     const float4v qf = *reinterpret_cast<const float4v *>(g.Q + oq + (int64_t)m * g.q_sm + l * 4);
+    ask_k_at(ka, 0);
     // the soft-max program's other leaves at this thread's positions (tid, tid + 1024, ...)
     LeafWords<P, 1> w[IPL];
     int64_t base[P::nleaf + 1];
-    {
-#pragma unroll
-        for (int i = 0; i <= P::nleaf; i++) base[i] = 0;
-        uint32_t rr = (uint32_t)(op / g.T) + m; // the row in the program's [rows, T] space
-#pragma unroll
-        for (uint32_t d = 0; d < (uint32_t)kMaxOuter; d++) {
-            if (d >= a.g.nouter) break;
-            const uint32_t q = fastdiv(rr, a.g.odiv[d]);
-            const int64_t i = (int64_t)(rr - q * a.g.od[d]);
-            rr = q;
-#pragma unroll
-            for (int lf = 1; lf < P::nleaf; lf++) base[lf] += i * a.leaf[lf].os[d];
-        }
-    }
+    leaf_offsets<P>(a, row0 + m, base);
     auto fetch_leaves = [&]() {
 #pragma unroll
         for (int c = 0; c < IPL; c++)
-            if (tid + c * kRowBlock < T) aot_fetch_from<P, 1>(a, base, t_first + tid + c * kRowBlock, w[c]);
+            aot_fetch_from<P, 1>(a, base, t_first + min(tid + c * kRowBlock, T - 1), w[c]);
     };
     if constexpr (!LOOP) fetch_leaves(); // nothing waits for them yet
+    if constexpr (V_EARLY) ask_v_at(va, 0);
 
     // ---- scores of the whole row
     auto score = [&](const float4v (&f)[PASSES], uint32_t first, auto full) {
@@ -545,83 +516,38 @@ __global__ __launch_bounds__(kSegBlock) void decode_attention_seg_kernel(const A
     const uint32_t tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     const uint32_t split = blockIdx.x, b = blockIdx.y;
     const uint32_t t0 = split * g.chunk, n = min(g.T, t0 + g.chunk) - t0; // (the host makes no empty segment)
-    int64_t oq = 0, ok = 0, ov = 0, op = 0;
-    {
-        uint32_t bb = b;
-        // (every axis slot is visited, so that the fields are read from the argument block at once instead of one
-        // dependent scalar load after the other)
-#pragma unroll
-        for (uint32_t d = 0; d < (uint32_t)kMaxBatchAxes; d++) {
-            if (d >= g.nb) break;
-            const uint32_t q = fastdiv(bb, g.bdiv[d]);
-            const int64_t i = (int64_t)(bb - q * g.bd[d]);
-            bb = q;
-            oq += i * g.q_bs[d];
-            ok += i * g.k_bs[d];
-            ov += i * g.v_bs[d];
-            op += i * g.p_bs[d];
-        }
-    }
+    int64_t oq, ok, ov;
+    uint32_t row0; // first row of this group in the program's [rows, T] space
+    entry_offsets(g, b, oq, ok, ov, row0);
     const uint32_t l = tid % LPT, sub = tid / LPT;
     const uint32_t *kbase = g.Kc + ok + (int64_t)t0 * g.k_st + l * 4;
     const uint32_t *vbase = g.V + ov + (int64_t)t0 * g.v_st + l * 4;
-    const int64_t k_step = (int64_t)TPB * g.k_st, v_step = (int64_t)TPB * g.v_st;
-    // the trip that starts at `first`: FULL (a tag type) when it lies inside the segment, nothing is checked then
-    auto ask = [&](float4v (&f)[PASSES], const uint32_t *base, int64_t st, int64_t step, uint32_t first, auto full) {
-        const uint32_t *p = base + (int64_t)(first + sub) * st;
+    // the trip that starts at `first` (positions clamped as in the kernel above)
+    auto ask = [&](float4v (&f)[PASSES], const uint32_t *base, int64_t st, uint32_t first) {
 #pragma unroll
-        for (int ps = 0; ps < PASSES; ps++) {
-            if constexpr (decltype(full)::value) {
-                f[ps] = *reinterpret_cast<const float4v *>(p);
-            } else {
-                f[ps] = (float4v){0.f, 0.f, 0.f, 0.f};
-                if (first + sub + ps * TPB < n) f[ps] = *reinterpret_cast<const float4v *>(p);
-            }
-            p += step;
-        }
+        for (int ps = 0; ps < PASSES; ps++) f[ps] = *reinterpret_cast<const float4v *>(base + (int64_t)min(first + sub + ps * TPB, n - 1) * st);
     };
     constexpr std::true_type whole_trip{};
     constexpr std::false_type ragged{};
-    auto ask_k = [&](float4v (&f)[PASSES], uint32_t first) {
-        if (first + SPAN <= n) ask(f, kbase, g.k_st, k_step, first, whole_trip);
-        else ask(f, kbase, g.k_st, k_step, first, ragged);
-    };
-    auto ask_v = [&](float4v (&f)[PASSES], uint32_t first) {
-        if (first + SPAN <= n) ask(f, vbase, g.v_st, v_step, first, whole_trip);
-        else ask(f, vbase, g.v_st, v_step, first, ragged);
-    };
+    auto ask_k = [&](float4v (&f)[PASSES], uint32_t first) { ask(f, kbase, g.k_st, first); };
+    auto ask_v = [&](float4v (&f)[PASSES], uint32_t first) { ask(f, vbase, g.v_st, first); };
     float4v ka[PASSES], kb[LOOP ? PASSES : 1];
     float4v va[PASSES], vb[LOOP ? PASSES : 1];
-    ask_k(ka, 0);
-    if constexpr (!LOOP) ask_v(va, 0); // the whole segment is in flight from the start: the registers hold both
     float4v qf[MM];
 #pragma unroll
     for (int m = 0; m < MM; m++) {
-        qf[m] = (float4v){0.f, 0.f, 0.f, 0.f};
-        if ((uint32_t)m < g.M) qf[m] = *reinterpret_cast<const float4v *>(g.Q + oq + (int64_t)m * g.q_sm + l * 4);
+        qf[m] = *reinterpret_cast<const float4v *>(g.Q + oq + (int64_t)min((uint32_t)m, g.M - 1) * g.q_sm + l * 4);
     }
+    ask_k(ka, 0);
     // the soft-max phase gives a wave a query row (waves M.. have none); its lanes take positions lane, lane + 64, ...
     const uint32_t my_row = wave; // < g.M: this wave runs the program on row my_row
     int64_t base[P::nleaf + 1];
     LeafWords<P, 1> w[IPL];
-    if (my_row < g.M) {
+    leaf_offsets<P>(a, row0 + min(my_row, g.M - 1), base);
+    if constexpr (!LOOP) { // nothing waits for them yet
 #pragma unroll
-        for (int i = 0; i <= P::nleaf; i++) base[i] = 0;
-        uint32_t rr = (uint32_t)(op / g.T) + my_row; // the row in the program's [rows, T] space
-#pragma unroll
-        for (uint32_t d = 0; d < (uint32_t)kMaxOuter; d++) {
-            if (d >= a.g.nouter) break;
-            const uint32_t q = fastdiv(rr, a.g.odiv[d]);
-            const int64_t i = (int64_t)(rr - q * a.g.od[d]);
-            rr = q;
-#pragma unroll
-            for (int lf = 1; lf < P::nleaf; lf++) base[lf] += i * a.leaf[lf].os[d];
-        }
-        if constexpr (!LOOP) { // nothing waits for them yet
-#pragma unroll
-            for (int c = 0; c < IPL; c++)
-                if (lane + c * 64 < n) aot_fetch_from<P, 1>(a, base, t0 + lane + c * 64, w[c]);
-        }
+        for (int c = 0; c < IPL; c++) aot_fetch_from<P, 1>(a, base, t0 + min(lane + c * 64, n - 1), w[c]);
+        ask_v(va, 0); // the whole segment is in flight: the registers hold both
     }
 
     // ---- scores of the segment, all rows of the group

@@ -123,11 +123,14 @@ __device__ __forceinline__ void store_narrow(const Operand &o, int64_t off, cons
     }
 }
 
+// (Operands lie in device memory, which the compiler does not know of a pointer that it finds in an argument block; it would load
+// through the general address space, whose loads wait for everything asked for before them, LDS included.)
 // WORDS: the caller knows that the operand lies in 32-bit words (kernels compiled for launches whose operands all do:
 // without the narrow formats' code between its loads a program keeps them all in flight).
-template <int VEC, bool STREAM = false, bool WORDS = false>
+// IN_MEMORY: nor is it a constant (a compiled program knows which of its leaves are).
+template <int VEC, bool STREAM = false, bool WORDS = false, bool IN_MEMORY = false>
 __device__ __forceinline__ void load_words(const Operand &o, int64_t off, uint32_t (&r)[VEC]) {
-    if (o.uniform) {
+    if (!IN_MEMORY && o.uniform) {
 #pragma unroll
         for (int j = 0; j < VEC; j++) r[j] = o.ubits;
         return;
@@ -136,12 +139,14 @@ __device__ __forceinline__ void load_words(const Operand &o, int64_t off, uint32
         load_narrow<VEC>(o, off, r);
         return;
     }
-    const uint32_t *p = reinterpret_cast<const uint32_t *>(o.ptr) + off;
+    typedef const __attribute__((address_space(1))) uint32_t global_word;
+    global_word *p = reinterpret_cast<global_word *>(reinterpret_cast<uintptr_t>(o.ptr)) + off;
     if (VEC >= 4 && o.is == 1) {
         typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+        typedef const __attribute__((address_space(1))) u4 global_u4;
 #pragma unroll
         for (int q = 0; q < VEC / 4; q++) {
-            const u4 t = STREAM ? __builtin_nontemporal_load(reinterpret_cast<const u4 *>(p) + q) : reinterpret_cast<const u4 *>(p)[q];
+            const u4 t = STREAM ? __builtin_nontemporal_load(reinterpret_cast<global_u4 *>(p) + q) : reinterpret_cast<global_u4 *>(p)[q];
             r[(4 * q) % VEC] = t[0];
             r[(4 * q + 1) % VEC] = t[1];
             r[(4 * q + 2) % VEC] = t[2];
