@@ -162,7 +162,7 @@ __global__ __launch_bounds__(kBlock) void decode_attention_kernel(const AttnArgs
                     if ((uint32_t)m < g.M) {
                         float v = fmaf(qf[m][3], kf[ps][3], fmaf(qf[m][2], kf[ps][2], fmaf(qf[m][1], kf[ps][1], qf[m][0] * kf[ps][0])));
                         v = row16_sum(v);
-                        if (LPT == 32) v += __shfl_xor(v, 16);
+                        if (LPT == 32) v = asf(fold_rows(asu(v), AddWords{}));
                         if (l == 0 && t < t1) sc[m][t - t0] = v;
                     }
                 }
@@ -207,8 +207,7 @@ __global__ __launch_bounds__(kBlock) void decode_attention_kernel(const AttnArgs
                 acc = row_merge(true, true, acc, s.v[src0][0]);
             }
         }
-#pragma unroll
-        for (int sft = 32; sft >= 1; sft >>= 1) acc = row_merge(true, true, acc, (uint32_t)__shfl_xor((int)acc, sft));
+        acc = wave_fold<1>(acc, [](uint32_t x, uint32_t y) { return row_merge(true, true, x, y); });
         rs[0] = acc;
         uint32_t sum = row_init(false, true);
 #pragma unroll
@@ -220,8 +219,7 @@ __global__ __launch_bounds__(kBlock) void decode_attention_kernel(const AttnArgs
                 sc[m][i] = asf(s.v[src1][0]); // the un-normalised weight
             }
         }
-#pragma unroll
-        for (int sft = 32; sft >= 1; sft >>= 1) sum = row_merge(false, true, sum, (uint32_t)__shfl_xor((int)sum, sft));
+        sum = wave_fold<1>(sum, [](uint32_t x, uint32_t y) { return row_merge(false, true, x, y); });
         if (lane == 0) {
             float *ml = g.part_ml + (((uint64_t)b * g.splits + split) * g.M + m) * 2;
             ml[0] = asf(acc);
@@ -360,7 +358,7 @@ __global__ __launch_bounds__(kRowBlock) void decode_attention_row_kernel(const A
             if (decltype(full)::value || first + ps * TPB < T) { // the same for the whole workgroup
                 float v = fmaf(qf[3], f[ps][3], fmaf(qf[2], f[ps][2], fmaf(qf[1], f[ps][1], qf[0] * f[ps][0])));
                 v = row16_sum(v);
-                if (LPT == 32) v += __shfl_xor(v, 16);
+                if (LPT == 32) v = asf(fold_rows(asu(v), AddWords{}));
                 if (l == 0 && (decltype(full)::value || t < T)) sc[t] = v;
             }
         }
@@ -397,8 +395,7 @@ __global__ __launch_bounds__(kRowBlock) void decode_attention_row_kernel(const A
                 acc = row_merge(true, true, acc, s.v[src0][0]);
             }
         }
-#pragma unroll
-        for (int sft = 32; sft >= 1; sft >>= 1) acc = row_merge(true, true, acc, (uint32_t)__shfl_xor((int)acc, sft));
+        acc = wave_fold<1>(acc, [](uint32_t x, uint32_t y) { return row_merge(true, true, x, y); });
         if (lane == 0) cross[0][wave] = acc;
         __syncthreads();
         acc = cross[0][0];
@@ -416,8 +413,7 @@ __global__ __launch_bounds__(kRowBlock) void decode_attention_row_kernel(const A
                 sc[i] = asf(s.v[src1][0]); // the un-normalised weight
             }
         }
-#pragma unroll
-        for (int sft = 32; sft >= 1; sft >>= 1) sum = row_merge(false, true, sum, (uint32_t)__shfl_xor((int)sum, sft));
+        sum = wave_fold<1>(sum, [](uint32_t x, uint32_t y) { return row_merge(false, true, x, y); });
         if (lane == 0) cross[1][wave] = sum;
         __syncthreads();
         sum = cross[1][0];
@@ -457,12 +453,7 @@ __global__ __launch_bounds__(kRowBlock) void decode_attention_row_kernel(const A
     }
     // the wave's position groups (lanes lv, lv + LPV, ...) first, then the waves through LDS
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        float v = o[j];
-#pragma unroll
-        for (int sft = LPV; sft < 64; sft <<= 1) v += __shfl_xor(v, sft);
-        o[j] = v;
-    }
+    for (int j = 0; j < 4; j++) o[j] = wave_sum_up<LPV>(o[j]);
     if (lane < LPV) *reinterpret_cast<float4v *>(&red[wave][lv * 4]) = o;
     __syncthreads();
     if (tid < HD / VS) {
@@ -561,7 +552,7 @@ __global__ __launch_bounds__(kSegBlock) void decode_attention_seg_kernel(const A
                     if ((uint32_t)m < g.M) {
                         float v = fmaf(qf[m][3], f[ps][3], fmaf(qf[m][2], f[ps][2], fmaf(qf[m][1], f[ps][1], qf[m][0] * f[ps][0])));
                         v = row16_sum(v);
-                        if (LPT == 32) v += __shfl_xor(v, 16);
+                        if (LPT == 32) v = asf(fold_rows(asu(v), AddWords{}));
                         if (l == 0 && (decltype(full)::value || t < n)) sc[m * cap + t] = v;
                     }
                 }
@@ -608,8 +599,7 @@ __global__ __launch_bounds__(kSegBlock) void decode_attention_seg_kernel(const A
                 acc = row_merge(true, true, acc, s.v[src0][0]);
             }
         }
-#pragma unroll
-        for (int sft = 32; sft >= 1; sft >>= 1) acc = row_merge(true, true, acc, (uint32_t)__shfl_xor((int)acc, sft));
+        acc = wave_fold<1>(acc, [](uint32_t x, uint32_t y) { return row_merge(true, true, x, y); });
         rs[0] = acc;
         uint32_t sum = row_init(false, true);
         if constexpr (!LOOP) {
@@ -631,8 +621,7 @@ __global__ __launch_bounds__(kSegBlock) void decode_attention_seg_kernel(const A
                 sc[m * cap + i] = asf(s.v[src1][0]);
             }
         }
-#pragma unroll
-        for (int sft = 32; sft >= 1; sft >>= 1) sum = row_merge(false, true, sum, (uint32_t)__shfl_xor((int)sum, sft));
+        sum = wave_fold<1>(sum, [](uint32_t x, uint32_t y) { return row_merge(false, true, x, y); });
         if (lane == 0) {
             float *ml = g.part_ml + (((uint64_t)b * g.splits + split) * g.M + m) * 2;
             ml[0] = asf(acc);
@@ -682,12 +671,7 @@ __global__ __launch_bounds__(kSegBlock) void decode_attention_seg_kernel(const A
     for (int m = 0; m < MM; m++) {
         if ((uint32_t)m < g.M) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                float v = o[m][j];
-#pragma unroll
-                for (int sft = LPT; sft < 64; sft <<= 1) v += __shfl_xor(v, sft);
-                o[m][j] = v;
-            }
+            for (int j = 0; j < 4; j++) o[m][j] = wave_sum_up<LPT>(o[m][j]);
             if (lane < LPT) *reinterpret_cast<float4v *>(&red[(wave * MM + m) * HD + l * 4]) = o[m];
         }
     }
@@ -753,8 +737,7 @@ __global__ __launch_bounds__(kBlock) void decode_attention_combine_kernel(const 
             num1 = fmaf(wk, v1[k], num1);
         }
     }
-#pragma unroll
-    for (int sft = 32; sft >= 1; sft >>= 1) den += __shfl_xor(den, sft);
+    den = wave_sum<1>(den);
     if (lane < hd) out[r * hd + lane] = asu(num0 / den);
     if (lane + 64 < hd) out[r * hd + lane + 64] = asu(num1 / den);
 }

@@ -329,6 +329,65 @@ __device__ __forceinline__ float wave_total(float v) {
     return asf((uint32_t)__builtin_amdgcn_readlane((int)asu(v), 63));
 }
 
+// f over the lanes of a wave at distances 32, 16 .. LOW, left in all of them: what a butterfly of shuffles gives, to the bit, where f
+// does not mind the order of its two operands.  (Below 16 lanes by rotation: the values repeat by then.)  A shuffle is a trip through
+// LDS, and a chain of six of them, 64 cycles each, is longer than the memory's latency behind which nothing else is left to do.
+template <int CTRL> __device__ __forceinline__ uint32_t row_rotated(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+}
+template <class F> __device__ __forceinline__ uint32_t fold_halves(uint32_t v, F f) { // lanes 32 apart
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return f((uint32_t)r[0], (uint32_t)r[1]);
+}
+template <class F> __device__ __forceinline__ uint32_t fold_rows(uint32_t v, F f) { // lanes 16 apart
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return f((uint32_t)r[0], (uint32_t)r[1]);
+}
+template <int LOW, class F> __device__ __forceinline__ uint32_t wave_fold(uint32_t v, F f) {
+    static_assert(LOW == 1 || LOW == 2 || LOW == 4 || LOW == 8 || LOW == 16 || LOW == 32, "a distance between lanes");
+    v = fold_halves(v, f);
+    if constexpr (LOW <= 16) v = fold_rows(v, f);
+    if constexpr (LOW <= 8) v = f(v, row_rotated<0x128>(v));
+    if constexpr (LOW <= 4) v = f(v, row_rotated<0x124>(v));
+    if constexpr (LOW <= 2) v = f(v, row_rotated<0x122>(v));
+    if constexpr (LOW <= 1) v = f(v, row_rotated<0x121>(v));
+    return v;
+}
+struct AddWords {
+    __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const { return asu(asf(a) + asf(b)); }
+};
+template <int LOW> __device__ __forceinline__ float wave_sum(float v) { return asf(wave_fold<LOW>(asu(v), AddWords{})); }
+// ... and in the other order, LOW, 2 LOW .. 32 (where the lanes' values do not repeat yet, only rows and halves can be folded)
+template <int LOW> __device__ __forceinline__ float wave_sum_up(float v) {
+#pragma unroll
+    for (int s = LOW; s < 8; s <<= 1) v += __shfl_xor(v, s);
+    if constexpr (LOW <= 8) v += asf(row_rotated<0x128>(asu(v)));
+    if constexpr (LOW <= 16) v = asf(fold_rows(asu(v), AddWords{}));
+    return asf(fold_halves(asu(v), AddWords{}));
+}
+// The value of the lane DIST away (16 or 32)
+template <int DIST> __device__ __forceinline__ uint32_t across(uint32_t v) {
+    static_assert(DIST == 16 || DIST == 32, "a row or a half");
+    if constexpr (DIST == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return threadIdx.x & 32 ? (uint32_t)r[0] : (uint32_t)r[1];
+    } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return threadIdx.x & 16 ? (uint32_t)r[0] : (uint32_t)r[1];
+    }
+}
+// The sums of four values over the lanes at distances 32, 16, 8 and 4, in that order: of v[r] in row r (lanes 16 r .. 16 r + 15).  Two
+// values share a register from the first step on, four from the second.
+__device__ __forceinline__ float four_sums(float a, float b, float c, float d) {
+    const auto ac = __builtin_amdgcn_permlane32_swap(asu(a), asu(c), false, false);
+    const auto bd = __builtin_amdgcn_permlane32_swap(asu(b), asu(d), false, false);
+    const float x = asf((uint32_t)ac[0]) + asf((uint32_t)ac[1]), y = asf((uint32_t)bd[0]) + asf((uint32_t)bd[1]);
+    const auto xy = __builtin_amdgcn_permlane16_swap(asu(x), asu(y), false, false);
+    float v = asf((uint32_t)xy[0]) + asf((uint32_t)xy[1]);
+    v += asf(row_rotated<0x128>(asu(v)));
+    return v + asf(row_rotated<0x124>(asu(v)));
+}
+
 // Offset (in elements) of row `row` of a view whose outer axes are described by
 // (od, odiv, os), innermost first.
 __device__ __forceinline__ int64_t row_offset(uint32_t row, uint32_t nouter, const uint32_t *od, const FastDiv *odiv,

@@ -996,9 +996,7 @@ template <int MM> __global__ __launch_bounds__(kThreads) void skinny_kt_kernel(c
     }
 #pragma unroll
     for (int m = 0; m < MM; m++) {
-        float v = acc[m];
-#pragma unroll
-        for (int s = 32; s >= 1; s >>= 1) v += __shfl_xor(v, s);
+        const float v = wave_sum<1>(acc[m]);
         if (lane == 0 && (uint32_t)m < a.M) a.C[((uint64_t)blockIdx.y * a.M + m) * a.N + n] = asu(v);
     }
 }
@@ -1087,10 +1085,7 @@ __device__ __forceinline__ void skinny_kt_wide_body(const MmArgs &a, const uint3
 #pragma unroll
     for (int c = 0; c < COLS; c++)
 #pragma unroll
-        for (int m = 0; m < MM; m++) {
-#pragma unroll
-            for (int s = 32; s >= 1; s >>= 1) acc[c][m] += __shfl_xor(acc[c][m], s);
-        }
+        for (int m = 0; m < MM; m++) acc[c][m] = wave_sum<1>(acc[c][m]);
     if (SPLIT) {
         __shared__ float part[4][COLS * MM];
         if (lane == 0) {
@@ -1172,7 +1167,8 @@ __device__ __forceinline__ uint32_t group_problem(const MmGroup &g, uint32_t &bl
     uint32_t p = 0;
 #pragma unroll
     for (int i = 1; i < kMaxGroup; i++) p += (uint32_t)i < g.n && blockIdx.x >= g.first[i] ? 1u : 0u;
-    block_x = blockIdx.x - g.first[p];
+    const uint32_t first = p == 0 ? g.first[0] : p == 1 ? g.first[1] : p == 2 ? g.first[2] : g.first[3];
+    block_x = blockIdx.x - first;
     return p;
 }
 template <int MM> __global__ __launch_bounds__(kThreads) void skinny_kt_wide_group_kernel(const MmGroup g) {
@@ -1210,6 +1206,38 @@ template <int TRIPS, bool WHOLE = false> __device__ __forceinline__ void xreg_la
     kb = (ragged ? wave * 64 : wave * (TRIPS * 64)) + b * 4;
     ks = ragged ? 256u : 64u;
 }
+// Four values of a row from k on, and what they count for: zeros behind K.  Loads behind K are clamped, not tested: a test in front of
+// every load leaves the compiler without a count of what is on its way, and it then waits for all of it before each of several groups.
+// The kernels below run for a few microseconds, most of them one trip to memory; around it nothing waits that need not: every load of
+// a chunk is on its way before the first wait, the sums over lanes stay out of LDS (four_sums), a norm's divisor is worked out
+// meanwhile, and the arguments come in two trips.  One row, us a launch with guarded loads, shuffles, the divisor at the end and
+// arguments field by field, and so: q, k and v with the rotary embedding 576 -> 960 7.3 and 5.2, 1024 -> 4096 9.0 and 6.7; gate and up
+// 576 -> 1536 7.4 and 5.9, 1024 -> 3072 8.5 and 7.8; the sums 576 -> 576 3.8 and 3.6, 2048 -> 1024 5.8 and 5.5.  Four rows: q, k and v
+// 2048 -> 3072 11.8 and 9.7, gate and up 2048 -> 8192 26.4 and 24.3.
+template <bool WHOLE, bool NT = false> __device__ __forceinline__ float4v xreg_at(const uint32_t *row, uint32_t k, uint32_t K) {
+    const float4v *const p = reinterpret_cast<const float4v *>(row + (WHOLE ? k : min(k, K - 4)));
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+template <bool WHOLE> __device__ __forceinline__ float4v xreg_within(float4v v, uint32_t k, uint32_t K) {
+    if constexpr (!WHOLE) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = k < K ? v[e] : 0.0f;
+    }
+    return v;
+}
+// This thread's share of a norm's partial sums, [blocks][MM] floats: the first 2 * MM rounds, clamped likewise, and their sum with the rest
+template <int MM> __device__ __forceinline__ void xreg_ask_sums(const NormFuse &nf, float (&pv)[2 * MM]) {
+#pragma unroll
+    for (int u = 0; u < 2 * MM; u++) pv[u] = nf.partials[min(threadIdx.x + u * kThreads, nf.blocks * MM - 1)];
+}
+template <int MM> __device__ __forceinline__ float xreg_sums(const NormFuse &nf, const float (&pv)[2 * MM]) {
+    float s = 0.0f;
+#pragma unroll
+    for (int u = 0; u < 2 * MM; u++) s += threadIdx.x + u * kThreads < nf.blocks * MM ? pv[u] : 0.0f;
+    for (uint32_t i = threadIdx.x + 2 * MM * kThreads; i < nf.blocks * MM; i += kThreads) s += nf.partials[i];
+    return s;
+}
 template <bool WHOLE, int MM, int CG, bool GATED, bool RESIDUAL, bool NORM, int TRIPS>
 __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, const uint32_t block_x, const uint32_t block_y, const uint32_t *second,
                                                               const uint32_t one, const MmResidual *res, const NormFuse *nf) {
@@ -1238,28 +1266,20 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
     // the sum's other terms for the value this thread will store: asked for before the walk along K
     uint32_t term[4] = {};
     if constexpr (RESIDUAL) {
-        if (threadIdx.x < CG * MM * 4) {
-            const uint32_t c = threadIdx.x / (MM * 4), m = threadIdx.x / 4 % MM, col = n0 + 4 * c + threadIdx.x % 4;
-            if (col < a.N && m < a.M) {
+        const uint32_t c = threadIdx.x / (MM * 4) % CG, m = min(threadIdx.x / 4 % MM, a.M - 1), col = min(n0 + 4 * c + threadIdx.x % 4, a.N - 1);
 #pragma unroll
-                for (int t = 0; t < 4; t++)
-                    if ((uint32_t)t != res->slot && (uint32_t)t < res->nterms)
-                        term[t] = res->term[t][((uint64_t)block_y * a.M + m) * a.N + col];
-            }
-        }
+        for (int t = 0; t < 4; t++)
+            if ((uint32_t)t != res->slot && (uint32_t)t < res->nterms) term[t] = res->term[t][((uint64_t)block_y * a.M + m) * a.N + col];
     }
     // NORM: the products are taken of x * gamma and divided by d_m = pow(sum(x[m]^2) / n + eps, e) where they are stored:
     // (x / d * gamma) . w = ((x * gamma) . w) / d.  The row sums are put together from the partial sums that the kernel
     // which stored x left (always in the same order); thread t takes entries t, t + 256, ... of [blocks][MM], all of row
-    // t % MM.  The first 512 blocks' are asked for here and added up after the walk along K: nothing waits for them.
-    float pv[NORM ? 2 * MM : 1] = {};
-    if constexpr (NORM) {
-#pragma unroll
-        for (int u = 0; u < 2 * MM; u++) {
-            const uint32_t i = threadIdx.x + u * kThreads;
-            if (i < nf->blocks * MM) pv[u] = nf->partials[i];
-        }
-    }
+    // t % MM.  They are asked for in front of all else, and the divisor (a power, in a few hundred instructions that nothing hides
+    // at a kernel's end) is worked out while the first weights are on their way.
+    __shared__ float nsum[4][MM];
+    uint32_t divisor = 0;
+    float pv[2 * MM];
+    if constexpr (NORM) xreg_ask_sums<MM>(*nf, pv);
     // of every chunk of TRIPS * 256 values of k (2048 or 1024) a wave takes a quarter in a row (TRIPS trips of 64)
     static_assert(TRIPS == 8 || TRIPS == 4, "chunks of 2048 or 1024");
     uint32_t kb, ks;
@@ -1270,28 +1290,37 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
         for (int t = 0; t < TRIPS; t++) {
             const uint32_t k = k0 + kb + ks * t;
 #pragma unroll
-            for (int g = 0; g < G; g++) {
-                xr[g][t] = (float4v){0.f, 0.f, 0.f, 0.f};
-                if (WHOLE || k < a.K) xr[g][t] = *reinterpret_cast<const float4v *>(xrow[g] + k);
-            }
+            for (int g = 0; g < G; g++) xr[g][t] = xreg_at<WHOLE>(xrow[g], k, a.K);
         }
         float4v gm[NORM ? TRIPS : 1]; // asked for with the activations, multiplied in once the first weights are on their way
         if constexpr (NORM) {
 #pragma unroll
             for (int t = 0; t < TRIPS; t++) {
                 const uint32_t k = k0 + kb + ks * t;
-                gm[t] = (float4v){0.f, 0.f, 0.f, 0.f};
-                if (WHOLE || k < a.K) gm[t] = *reinterpret_cast<const float4v *>(nf->gamma + k);
+                gm[t] = xreg_at<WHOLE>(nf->gamma, k, a.K);
             }
+        }
+        float4v ws[CG][TRIPS];
+        auto ask = [&](int c) {
+#pragma unroll
+            for (int t = 0; t < TRIPS; t++) ws[c][t] = xreg_at<WHOLE>(wrow[c], k0 + kb + ks * t, a.K);
+        };
+        if constexpr (NORM) { // all in front of the wait for the partial sums
+#pragma unroll
+            for (int c = 0; c < CG; c++) ask(c);
         }
 #pragma unroll
         for (int c = 0; c < CG; c++) {
-            float4v w[TRIPS];
-#pragma unroll
-            for (int t = 0; t < TRIPS; t++) {
-                const uint32_t k = k0 + kb + ks * t;
-                w[t] = (float4v){0.f, 0.f, 0.f, 0.f};
-                if (WHOLE || k < a.K) w[t] = *reinterpret_cast<const float4v *>(wrow[c] + k);
+            float4v (&w)[TRIPS] = ws[c];
+            if constexpr (!NORM) ask(c);
+            if constexpr (!WHOLE || NORM) __builtin_amdgcn_sched_barrier(0); // (what follows stays behind all of the loads)
+            if constexpr (NORM) {
+                if (c == 0 && k0 == 0) { // (the same for every thread)
+                    const float s = wave_sum<MM>(xreg_sums<MM>(*nf, pv));
+                    if (lane < MM) nsum[wave][lane] = s;
+                    __syncthreads();
+                    if (threadIdx.x < MM * 4 * (GATED ? 1 : CG)) divisor = norm_divisor(*nf, (nsum[0][threadIdx.x / 4 % MM] + nsum[1][threadIdx.x / 4 % MM]) + (nsum[2][threadIdx.x / 4 % MM] + nsum[3][threadIdx.x / 4 % MM]));
+                }
             }
             if constexpr (NORM) {
                 if (c == 0) {
@@ -1301,6 +1330,15 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
                         for (int g = 0; g < G; g++)
 #pragma unroll
                             for (int e = 0; e < 4; e++) xr[g][t][e] = asf(apply<kMul, true>(asu(xr[g][t][e]), asu(gm[t][e]), 0, nullptr));
+                }
+            }
+            if constexpr (!WHOLE) {
+#pragma unroll
+                for (int t = 0; t < TRIPS; t++) {
+                    w[t] = xreg_within<WHOLE>(w[t], k0 + kb + ks * t, a.K);
+#pragma unroll
+                    for (int g = 0; g < G; g++)
+                        if (c == 0) xr[g][t] = xreg_within<WHOLE>(xr[g][t], k0 + kb + ks * t, a.K);
                 }
             }
 #pragma unroll
@@ -1315,27 +1353,13 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
         }
     }
     __shared__ float part[4][CG * MM * 4];
-    __shared__ float nsum[4][MM];
-    if constexpr (NORM) {
-        float s = 0.0f;
-#pragma unroll
-        for (int u = 0; u < 2 * MM; u++) s += pv[u];
-        for (uint32_t i = threadIdx.x + 2 * MM * kThreads; i < nf->blocks * MM; i += kThreads) s += nf->partials[i];
-#pragma unroll
-        for (int sh = 32; sh >= MM; sh >>= 1) s += __shfl_xor(s, sh);
-        if (lane < MM) nsum[wave][lane] = s;
-    }
 #pragma unroll
     for (int c = 0; c < CG; c++)
 #pragma unroll
-        for (int g = 0; g < G; g++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                float v = acc[c][g][i];
-#pragma unroll
-                for (int s = 32; s >= 4; s >>= 1) v += __shfl_xor(v, s);
-                if (lane < 4) part[wave][(c * MM + 4 * g + i) * 4 + j] = v;
-            }
+        for (int g = 0; g < G; g++) {
+            const float v = four_sums(acc[c][g][0], acc[c][g][1], acc[c][g][2], acc[c][g][3]); // of row g * 4 + b / 4
+            if (b % 4 == 0) part[wave][(c * MM + 4 * g) * 4 + b + j] = v;
+        }
     __syncthreads();
     if constexpr (GATED) {
         if (threadIdx.x < MM * 4) {
@@ -1343,9 +1367,8 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
             uint32_t gv = asu((part[0][t] + part[1][t]) + (part[2][t] + part[3][t]));
             uint32_t uv = asu((part[0][u_at] + part[1][u_at]) + (part[2][u_at] + part[3][u_at]));
             if constexpr (NORM) {
-                const uint32_t d = norm_divisor(*nf, (nsum[0][m] + nsum[1][m]) + (nsum[2][m] + nsum[3][m]));
-                gv = apply<kDiv, true>(gv, d, 0, nullptr);
-                uv = apply<kDiv, true>(uv, d, 0, nullptr);
+                gv = apply<kDiv, true>(gv, divisor, 0, nullptr);
+                uv = apply<kDiv, true>(uv, divisor, 0, nullptr);
             }
             // the ops of the deferred program, in its order
             const uint32_t e = apply<kExp, true>(apply<kNeg, true>(gv, 0, 0, nullptr), 0, 0, nullptr);
@@ -1356,8 +1379,7 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
     } else if (threadIdx.x < CG * MM * 4) {
         const uint32_t c = threadIdx.x / (MM * 4), m = threadIdx.x / 4 % MM, col = n0 + 4 * c + threadIdx.x % 4;
         uint32_t v = asu((part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]));
-        if constexpr (NORM)
-            v = apply<kDiv, true>(v, norm_divisor(*nf, (nsum[0][m] + nsum[1][m]) + (nsum[2][m] + nsum[3][m])), 0, nullptr);
+        if constexpr (NORM) v = apply<kDiv, true>(v, divisor, 0, nullptr);
         if constexpr (RESIDUAL) {
 #pragma unroll
             for (int t = 0; t < 4; t++) term[t] = (uint32_t)t == res->slot ? v : term[t];
@@ -1369,8 +1391,8 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
             // threads 0 .. 4 MM - 1 = (row m, column n0 + t % 4): the row's sum of squares over the block's four columns
             if (res->partials) {
                 float q = stored ? asf(v) * asf(v) : 0.0f;
-                q += __shfl_xor(q, 1);
-                q += __shfl_xor(q, 2);
+                q += asf(row_rotated<0xB1>(asu(q))); // (of the lane 1 away, then 2)
+                q += asf(row_rotated<0x4E>(asu(q)));
                 if (threadIdx.x % 4 == 0) res->partials[(uint64_t)block_x * MM + m] = q;
             }
         }
@@ -1415,11 +1437,10 @@ __global__ __launch_bounds__(kEightThreads, 2) void skinny_kt_mfma_eight_residua
     const uint32_t tc = threadIdx.x / (4 * MM), tm = threadIdx.x / 4 % MM, tcol = n0 + 4 * tc + threadIdx.x % 4;
     const bool stored = threadIdx.x < kOut && tcol < a.N && tm < a.M;
     uint32_t term[4] = {};
-    if (stored) {
+    const uint64_t term_at = (uint64_t)min(tm, a.M - 1) * a.N + min(tcol, a.N - 1);
 #pragma unroll
-        for (int t = 0; t < 4; t++)
-            if ((uint32_t)t != res.slot && (uint32_t)t < res.nterms) term[t] = res.term[t][(uint64_t)tm * a.N + tcol];
-    }
+    for (int t = 0; t < 4; t++)
+        if ((uint32_t)t != res.slot && (uint32_t)t < res.nterms) term[t] = res.term[t][term_at];
     float4v acc[2][G] = {};
     for (uint32_t k0 = wave * (TRIPS * 64) + b * 4; k0 < a.K; k0 += TRIPS * kEightThreads) { // (K: whole chunks)
         float4v xr[G][TRIPS], wr[2][TRIPS];
@@ -1444,11 +1465,9 @@ __global__ __launch_bounds__(kEightThreads, 2) void skinny_kt_mfma_eight_residua
 #pragma unroll
     for (int c = 0; c < 2; c++)
 #pragma unroll
-        for (int i = 0; i < MM; i++) {
-            float v = acc[c][i / 4][i % 4];
-#pragma unroll
-            for (int s = 32; s >= 4; s >>= 1) v += __shfl_xor(v, s);
-            if (lane < 4) part[wave][(c * MM + i) * 4 + j] = v;
+        for (int g = 0; g < G; g++) {
+            const float v = four_sums(acc[c][g][0], acc[c][g][1], acc[c][g][2], acc[c][g][3]); // of row g * 4 + b / 4
+            if (b % 4 == 0) part[wave][(c * MM + 4 * g) * 4 + b + j] = v;
         }
     __syncthreads();
     if (threadIdx.x >= kOut) return;
@@ -1460,8 +1479,8 @@ __global__ __launch_bounds__(kEightThreads, 2) void skinny_kt_mfma_eight_residua
     if (stored) a.C[(uint64_t)tm * a.N + tcol] = v;
     if (res.partials) { // the rows' sums of squares over four columns each, as above
         float q = stored ? asf(v) * asf(v) : 0.0f;
-        q += __shfl_xor(q, 1);
-        q += __shfl_xor(q, 2);
+        q += asf(row_rotated<0xB1>(asu(q)));
+        q += asf(row_rotated<0x4E>(asu(q)));
         if (t % 4 == 0 && n0 + 4 * tc < a.N) res.partials[((uint64_t)blockIdx.x * 2 + tc) * MM + tm] = q;
     }
 }
@@ -1500,10 +1519,27 @@ struct RopeGroup {
 template <bool WHOLE, int MM, bool NORM, int TRIPS>
 __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGroup &g, const RopeGroup &rg, const NormFuse &nf) {
     static_assert(TRIPS == 8 || TRIPS == 4, "chunks of 2048 or 1024");
+    __shared__ float nsum[4][MM];
+    uint32_t divisor = 0;
+    float pv[2 * MM];
+    if constexpr (NORM) xreg_ask_sums<MM>(nf, pv); // (the norm as in skinny_kt_mfma_xreg_body)
     uint32_t bx;
     const uint32_t p = group_problem(g, bx);
-    const MmArgs &a = g.p[p];
-    const RopeStore &rs = rg.s[p];
+    // (everything that the problem's number leads to asked for at once, not field by field on the way)
+    struct {
+        const uint32_t *A, *B;
+        uint32_t M, N, K;
+        int64_t a_sm, b_sn;
+    } a = {g.p[p].A, g.p[p].B, g.p[p].M, g.p[p].N, g.p[p].K, g.p[p].a_sm, g.p[p].b_sn};
+    struct {
+        uint32_t *dst;
+        int64_t sb, sh;
+        const uint32_t *cos, *sin;
+        uint32_t hd, rope;
+    } rs = {rg.s[p].dst, rg.s[p].sb, rg.s[p].sh, rg.s[p].cos, rg.s[p].sin, rg.s[p].hd, rg.s[p].rope};
+    asm volatile("" : "+s"(a.M), "+s"(a.N), "+s"(a.K), "+s"(a.a_sm), "+s"(a.b_sn), "+s"(rs.sb), "+s"(rs.sh), "+s"(rs.hd), "+s"(rs.rope)
+                 : "s"(a.A), "s"(a.B), "s"(rs.dst), "s"(rs.cos), "s"(rs.sin));
+    if constexpr (NORM) asm volatile("" ::"s"(nf.gamma), "s"(nf.n_bits), "s"(nf.eps_bits), "s"(nf.exp_bits));
     const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     const uint32_t j = lane % 4, b = lane / 4;
     const uint32_t span = rs.rope ? rs.hd : 8, per = span / 8;
@@ -1524,22 +1560,9 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGrou
         cs = rs.cos[d];
         sn = rs.sin[d];
     }
-    float pv[NORM ? 2 * MM : 1] = {};
-    if constexpr (NORM) {
-#pragma unroll
-        for (int u = 0; u < 2 * MM; u++) {
-            const uint32_t i = threadIdx.x + u * kThreads;
-            if (i < nf.blocks * MM) pv[u] = nf.partials[i];
-        }
-    }
     uint32_t kb, ks;
     xreg_lane_k<TRIPS, WHOLE>(a.K, wave, b, kb, ks);
-    // (a value of k beyond K contributes zeros: only a ragged last chunk has any)
-    auto at = [&](const uint32_t *row, uint32_t k) {
-        float4v v = {0.f, 0.f, 0.f, 0.f};
-        if (WHOLE || k < a.K) v = *reinterpret_cast<const float4v *>(row + k);
-        return v;
-    };
+    auto at = [&](const uint32_t *row, uint32_t k) { return xreg_at<WHOLE>(row, k, a.K); };
     for (uint32_t k0 = 0; k0 < a.K; k0 += TRIPS * 256) {
         float4v xr[G][TRIPS];
 #pragma unroll
@@ -1551,11 +1574,23 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGrou
 #pragma unroll
             for (int t = 0; t < TRIPS; t++) gm[t] = at(nf.gamma, k0 + kb + ks * t);
         }
+        float4v ws[2][TRIPS];
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int t = 0; t < TRIPS; t++) ws[c][t] = at(wrow[c], k0 + kb + ks * t);
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-            float4v w[TRIPS];
-#pragma unroll
-            for (int t = 0; t < TRIPS; t++) w[t] = at(wrow[c], k0 + kb + ks * t);
+            float4v (&w)[TRIPS] = ws[c];
+            if constexpr (!WHOLE || NORM) __builtin_amdgcn_sched_barrier(0); // (what follows stays behind all of the loads)
+            if constexpr (NORM) {
+                if (c == 0 && k0 == 0) { // (the same for every thread)
+                    const float s = wave_sum<MM>(xreg_sums<MM>(nf, pv));
+                    if (lane < MM) nsum[wave][lane] = s;
+                    __syncthreads();
+                    if (threadIdx.x < 64) divisor = norm_divisor(nf, (nsum[0][threadIdx.x / 4 % MM] + nsum[1][threadIdx.x / 4 % MM]) + (nsum[2][threadIdx.x / 4 % MM] + nsum[3][threadIdx.x / 4 % MM]));
+                }
+            }
             if constexpr (NORM) {
                 if (c == 0) {
 #pragma unroll
@@ -1564,6 +1599,15 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGrou
                         for (int g = 0; g < G; g++)
 #pragma unroll
                             for (int e = 0; e < 4; e++) xr[g][t][e] = asf(apply<kMul, true>(asu(xr[g][t][e]), asu(gm[t][e]), 0, nullptr));
+                }
+            }
+            if constexpr (!WHOLE) {
+#pragma unroll
+                for (int t = 0; t < TRIPS; t++) {
+                    w[t] = xreg_within<WHOLE>(w[t], k0 + kb + ks * t, a.K);
+#pragma unroll
+                    for (int g = 0; g < G; g++)
+                        if (c == 0) xr[g][t] = xreg_within<WHOLE>(xr[g][t], k0 + kb + ks * t, a.K);
                 }
             }
 #pragma unroll
@@ -1575,31 +1619,19 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGrou
         }
     }
     __shared__ float part[4][kOut];
-    __shared__ float nsum[4][MM];
-    if constexpr (NORM) {
-        float s = 0.0f;
-#pragma unroll
-        for (int u = 0; u < 2 * MM; u++) s += pv[u];
-        for (uint32_t i = threadIdx.x + 2 * MM * kThreads; i < nf.blocks * MM; i += kThreads) s += nf.partials[i];
-#pragma unroll
-        for (int sh = 32; sh >= MM; sh >>= 1) s += __shfl_xor(s, sh);
-        if (lane < MM) nsum[wave][lane] = s;
-    }
 #pragma unroll
     for (int c = 0; c < 2; c++)
 #pragma unroll
-        for (int i = 0; i < MM; i++) {
-            float v = acc[c][i / 4][i % 4];
-#pragma unroll
-            for (int s = 32; s >= 4; s >>= 1) v += __shfl_xor(v, s);
-            if (lane < 4) part[wave][(c * MM + i) * 4 + j] = v;
+        for (int g = 0; g < G; g++) {
+            const float v = four_sums(acc[c][g][0], acc[c][g][1], acc[c][g][2], acc[c][g][3]); // of row g * 4 + b / 4
+            if (b % 4 == 0) part[wave][(c * MM + 4 * g) * 4 + b + j] = v;
         }
     __syncthreads();
     if (threadIdx.x < 64) { // the first wave: lanes 0 .. kOut - 1 hold (column group, row, column), any others idle along
         const uint32_t t = threadIdx.x % kOut, c = t / (4 * MM), m = t / 4 % MM, col = nc[c] + t % 4;
         uint32_t v = asu((part[0][t] + part[1][t]) + (part[2][t] + part[3][t]));
-        if constexpr (NORM) v = apply<kDiv, true>(v, norm_divisor(nf, (nsum[0][m] + nsum[1][m]) + (nsum[2][m] + nsum[3][m])), 0, nullptr);
-        const uint32_t other = __shfl_xor(v, 4 * MM); // the same row's column half a head away
+        if constexpr (NORM) v = apply<kDiv, true>(v, divisor, 0, nullptr);
+        const uint32_t other = across<4 * MM>(v); // the same row's column half a head away
         if (rs.rope) {
             // lower half: rotate_half reads -x[d + hd / 2]; upper half: x[d - hd / 2]
             const uint32_t rot = c == 0 ? apply<kNeg, true>(other, 0, 0, nullptr) : other;
@@ -1688,43 +1720,34 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs
     uint32_t kb, ks; // this lane's k: kb + ks t (beyond K, in a chunk that K does not fill: zeros)
     xreg_lane_k<TRIPS, WHOLE>(a.K, wave, b, kb, ks);
     constexpr int G = MM / 4, kOut = 4 * MM; // row groups; values of one product in a group of columns
+    float pv[2 * MM];
+    if constexpr (NORM) xreg_ask_sums<MM>(nf, pv);
     float4v xr[G][TRIPS];
 #pragma unroll
     for (int g = 0; g < G; g++) {
         const uint32_t *xrow = a.A + (int64_t)min((uint32_t)(4 * g) + j, a.M - 1) * a.a_sm;
 #pragma unroll
-        for (int t = 0; t < TRIPS; t++) {
-            xr[g][t] = (float4v){0.f, 0.f, 0.f, 0.f};
-            if (WHOLE || kb + ks * t < a.K) xr[g][t] = *reinterpret_cast<const float4v *>(xrow + kb + ks * t);
-        }
+        for (int t = 0; t < TRIPS; t++) xr[g][t] = xreg_at<WHOLE>(xrow, kb + ks * t, a.K);
     }
-    float pv[NORM ? 2 * MM : 1] = {};
     float4v gm[NORM ? TRIPS : 1];
     if constexpr (NORM) {
 #pragma unroll
-        for (int u = 0; u < 2 * MM; u++) {
-            const uint32_t i = threadIdx.x + u * kThreads;
-            if (i < nf.blocks * MM) pv[u] = nf.partials[i];
-        }
-#pragma unroll
-        for (int t = 0; t < TRIPS; t++) {
-            gm[t] = (float4v){0.f, 0.f, 0.f, 0.f};
-            if (WHOLE || kb + ks * t < a.K) gm[t] = *reinterpret_cast<const float4v *>(nf.gamma + kb + ks * t);
-        }
+        for (int t = 0; t < TRIPS; t++) gm[t] = xreg_at<WHOLE>(nf.gamma, kb + ks * t, a.K);
     }
     __shared__ float part[2][4][2 * kOut];
     __shared__ float nsum[4][MM];
     const uint32_t groups = (a.N + 3) / 4;
     float4v wg[TRIPS], wu[TRIPS]; // the group's four columns of the two weight matrices
     auto ask = [&](float4v (&w)[TRIPS], const uint32_t *base, uint32_t n0) {
-        const uint32_t *row = base + (int64_t)min(n0 + j, a.N - 1) * a.b_sn + kb;
+        const uint32_t *row = base + (int64_t)min(n0 + j, a.N - 1) * a.b_sn;
 #pragma unroll
-        for (int t = 0; t < TRIPS; t++) {
-            w[t] = (float4v){0.f, 0.f, 0.f, 0.f};
-            if (WHOLE || kb + ks * t < a.K) w[t] = __builtin_nontemporal_load(reinterpret_cast<const float4v *>(row + ks * t));
-        }
+        for (int t = 0; t < TRIPS; t++) w[t] = xreg_at<WHOLE, true>(row, kb + ks * t, a.K);
     };
-    auto multiply = [&](float4v (&sum)[G], const float4v (&w)[TRIPS]) {
+    auto multiply = [&](float4v (&sum)[G], float4v (&w)[TRIPS]) {
+        if constexpr (!WHOLE) {
+#pragma unroll
+            for (int t = 0; t < TRIPS; t++) w[t] = xreg_within<WHOLE>(w[t], kb + ks * t, a.K);
+        }
 #pragma unroll
         for (int t = 0; t < TRIPS; t++)
 #pragma unroll
@@ -1735,7 +1758,17 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs
     const uint32_t first_grp = blockIdx.x * iters;
     if (first_grp >= groups) return; // the same for every thread of the workgroup
     ask(wg, a.B, first_grp * 4);
-    if constexpr (NORM) {
+    ask(wu, second, first_grp * 4);
+    if constexpr (!WHOLE || NORM) __builtin_amdgcn_sched_barrier(0); // (what follows stays behind the loads)
+    uint32_t divisor = 0;
+    if constexpr (NORM) { // (the norm as in skinny_kt_mfma_xreg_body)
+        const float s = wave_sum<MM>(xreg_sums<MM>(nf, pv));
+        if (lane < MM) nsum[wave][lane] = s;
+        __syncthreads();
+        if (threadIdx.x < kOut) {
+            const uint32_t m = threadIdx.x / 4;
+            divisor = norm_divisor(nf, (nsum[0][m] + nsum[1][m]) + (nsum[2][m] + nsum[3][m]));
+        }
         // (x / d * gamma) . w = ((x * gamma) . w) / d: gamma goes in once, while the first weights are on their way; the row
         // sums of squares are put together from the partial sums, always in the same order
 #pragma unroll
@@ -1744,36 +1777,31 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs
             for (int g = 0; g < G; g++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) xr[g][t][e] = asf(apply<kMul, true>(asu(xr[g][t][e]), asu(gm[t][e]), 0, nullptr));
-        float s = 0.0f;
-#pragma unroll
-        for (int u = 0; u < 2 * MM; u++) s += pv[u];
-        for (uint32_t i = threadIdx.x + 2 * MM * kThreads; i < nf.blocks * MM; i += kThreads) s += nf.partials[i];
-#pragma unroll
-        for (int sh = 32; sh >= MM; sh >>= 1) s += __shfl_xor(s, sh);
-        if (lane < MM) nsum[wave][lane] = s;
     }
-    uint32_t divisor = 0;
+    if constexpr (!WHOLE) {
+#pragma unroll
+        for (int g = 0; g < G; g++)
+#pragma unroll
+            for (int t = 0; t < TRIPS; t++) xr[g][t] = xreg_within<WHOLE>(xr[g][t], kb + ks * t, a.K);
+    }
     for (uint32_t it = 0; it < iters; it++) {
         const uint32_t grp = first_grp + it;
         if (grp >= groups) break;
         const uint32_t n0 = grp * 4;
         float4v acc_g[G] = {}, acc_u[G] = {};
-        ask(wu, second, n0);
+        const bool more = it + 1 < iters && grp + 1 < groups;
         multiply(acc_g, wg);
-        if (it + 1 < iters && grp + 1 < groups) ask(wg, a.B, n0 + 4); // on its way through the rest of this group
+        if (more) ask(wg, a.B, n0 + 4); // on its way through the rest of this group
         multiply(acc_u, wu);
+        if (more) ask(wu, second, n0 + 4);
         float (*pt)[2 * kOut] = part[it & 1];
 #pragma unroll
-        for (int i = 0; i < MM; i++) {
-            float vg = acc_g[i / 4][i % 4], vu = acc_u[i / 4][i % 4];
-#pragma unroll
-            for (int s = 32; s >= 4; s >>= 1) {
-                vg += __shfl_xor(vg, s);
-                vu += __shfl_xor(vu, s);
-            }
-            if (lane < 4) {
-                pt[wave][i * 4 + j] = vg;
-                pt[wave][kOut + i * 4 + j] = vu;
+        for (int g = 0; g < G; g++) {
+            const float vg = four_sums(acc_g[g][0], acc_g[g][1], acc_g[g][2], acc_g[g][3]); // of row g * 4 + b / 4
+            const float vu = four_sums(acc_u[g][0], acc_u[g][1], acc_u[g][2], acc_u[g][3]);
+            if (b % 4 == 0) {
+                pt[wave][16 * g + b + j] = vg;
+                pt[wave][kOut + 16 * g + b + j] = vu;
             }
         }
         __syncthreads(); // (the buffer written two groups ago was read before the barrier of the group in between)
@@ -1782,7 +1810,6 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs
             uint32_t gv = asu((pt[0][t] + pt[1][t]) + (pt[2][t] + pt[3][t]));
             uint32_t uv = asu((pt[0][kOut + t] + pt[1][kOut + t]) + (pt[2][kOut + t] + pt[3][kOut + t]));
             if constexpr (NORM) {
-                if (it == 0) divisor = norm_divisor(nf, (nsum[0][m] + nsum[1][m]) + (nsum[2][m] + nsum[3][m]));
                 gv = apply<kDiv, true>(gv, divisor, 0, nullptr);
                 uv = apply<kDiv, true>(uv, divisor, 0, nullptr);
             }
@@ -2505,13 +2532,8 @@ __global__ __launch_bounds__(kThreads) void skinny_kt_packed_mfma_kernel(const M
         }
         if (it + 1 < iters && grp + 1 < groups) ask(grp + 1); // on its way through the reduction of this group
         float (*pt)[16] = part[it & 1];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float v = acc[i];
-#pragma unroll
-            for (int s = 32; s >= 4; s >>= 1) v += __shfl_xor(v, s);
-            if (lane < 4) pt[wave][i * 4 + j] = v;
-        }
+        const float v = four_sums(acc[0], acc[1], acc[2], acc[3]);
+        if (lane / 4 % 4 == 0) pt[wave][lane / 4 + j] = v;
         __syncthreads(); // (the buffer written two groups ago was read before the barrier of the group in between)
         if (threadIdx.x < 16) {
             const uint32_t m = threadIdx.x / 4, col = grp * 4 + threadIdx.x % 4;
@@ -2553,8 +2575,7 @@ __global__ __launch_bounds__(kThreads) void skinny_kt_packed_kernel(const MmArgs
     }
 #pragma unroll
     for (int m = 0; m < MM; m++) {
-#pragma unroll
-        for (int s = 32; s >= 1; s >>= 1) acc[m] += __shfl_xor(acc[m], s);
+        acc[m] = wave_sum<1>(acc[m]);
         if (lane == 0 && (uint32_t)m < a.M) a.C[(uint64_t)m * a.N + n] = asu(acc[m]);
     }
 }

@@ -30,7 +30,21 @@ def session():
 @pytest.mark.parametrize("rows", [5, 8])
 @pytest.mark.parametrize("shape", list(SHAPES))
 def test_steps_of_five_to_eight_rows(session, shape, rows):
-    arch, hidden, heads, kv, ff, hd = SHAPES[shape]
+    check(session, SHAPES[shape], rows)
+
+
+# last chunks that end inside a run of 64 values of k, with no chunk before them and with one
+ENDS = {"hidden_580": ("qwen3", 580, 9, 3, 1156, 64), "hidden_1156": ("llama", 1156, 17, 17, 580, 0), "hidden_3332": ("qwen3", 3332, 8, 4, 2308, 128)}
+
+
+@pytest.mark.parametrize("rows", [1, 4, 7])
+@pytest.mark.parametrize("shape", ["ragged_short", "ragged_long", "short_chunks", *ENDS])
+def test_steps_with_ragged_chunks(session, shape, rows):
+    check(session, ENDS.get(shape) or SHAPES[shape], rows)
+
+
+def check(session, shape, rows):
+    arch, hidden, heads, kv, ff, hd = shape
     cfg = LlmConfig(arch, hidden, 2, heads, kv, ff, 521, head_dim=hd, rms_norm_eps=1e-5, rope_theta=10000.0, tie_word_embeddings=True)
     params = params_of(cfg, seed=rows, scale=1.5)
     rng = np.random.default_rng(7)
