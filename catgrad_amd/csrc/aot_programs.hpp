@@ -265,8 +265,7 @@ __device__ __forceinline__ Values<P, VEC> aot_eval(const LeafWords<P, VEC> &w, c
 
 template <bool IS_MAX, bool F, int TPR> __device__ __forceinline__ uint32_t aot_row_combine(uint32_t acc) {
     constexpr int W = TPR < 64 ? TPR : 64;
-#pragma unroll
-    for (int m = W / 2; m >= 1; m >>= 1) acc = row_merge(IS_MAX, F, acc, (uint32_t)__shfl_xor((int)acc, m));
+    acc = group_fold<W>(acc, [](uint32_t x, uint32_t y) { return row_merge(IS_MAX, F, x, y); });
     if constexpr (TPR > 64) {
         __shared__ uint32_t part[kBlock / 64];
         if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = acc;

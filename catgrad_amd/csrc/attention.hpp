@@ -453,7 +453,7 @@ __global__ __launch_bounds__(kRowBlock) void decode_attention_row_kernel(const A
     }
     // the wave's position groups (lanes lv, lv + LPV, ...) first, then the waves through LDS
 #pragma unroll
-    for (int j = 0; j < 4; j++) o[j] = wave_sum_up<LPV>(o[j]);
+    for (int j = 0; j < 4; j++) o[j] = wave_add_up<LPV>(o[j]);
     if (lane < LPV) *reinterpret_cast<float4v *>(&red[wave][lv * 4]) = o;
     __syncthreads();
     if (tid < HD / VS) {
@@ -671,7 +671,7 @@ __global__ __launch_bounds__(kSegBlock) void decode_attention_seg_kernel(const A
     for (int m = 0; m < MM; m++) {
         if ((uint32_t)m < g.M) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) o[m][j] = wave_sum_up<LPT>(o[m][j]);
+            for (int j = 0; j < 4; j++) o[m][j] = wave_add_up<LPT>(o[m][j]);
             if (lane < LPT) *reinterpret_cast<float4v *>(&red[(wave * MM + m) * HD + l * 4]) = o[m];
         }
     }
@@ -719,8 +719,7 @@ __global__ __launch_bounds__(kBlock) void decode_attention_combine_kernel(const 
         const bool mine = lane < kGroup && c < splits;
         const float cm = mine ? ml[(uint64_t)c * M * 2] : kF32Min, cl = mine ? ml[(uint64_t)c * M * 2 + 1] : 0.0f;
         float m2 = fmaxf(gmax, cm);
-#pragma unroll
-        for (int sft = 16; sft >= 1; sft >>= 1) m2 = fmaxf(m2, __shfl_xor(m2, sft));
+        m2 = asf(group_fold<32>(asu(m2), LargerWords{}));
         m2 = __shfl(m2, 0);
         // what was summed so far is relative to the old maximum
         const float rescale = expf(gmax - m2);
@@ -737,7 +736,7 @@ __global__ __launch_bounds__(kBlock) void decode_attention_combine_kernel(const 
             num1 = fmaf(wk, v1[k], num1);
         }
     }
-    den = wave_sum<1>(den);
+    den = wave_add<1>(den);
     if (lane < hd) out[r * hd + lane] = asu(num0 / den);
     if (lane + 64 < hd) out[r * hd + lane + 64] = asu(num1 / den);
 }
@@ -1008,7 +1007,7 @@ template <int HD, bool PIECES> __device__ __forceinline__ bool prefill_rows(cons
                     tile_max = fmaxf(tile_max, acc_s[tb][v]);
                 }
         }
-        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
+        tile_max = asf(fold_halves(asu(tile_max), LargerWords{}));
         const float new_max = fmaxf(run_max, tile_max);
         const float base = new_max == -INFINITY ? 0.0f : new_max; // a lane without a live query: keep NaN out
         const float alpha = __builtin_amdgcn_exp2f((run_max - base) * kLog2e);
@@ -1021,7 +1020,7 @@ template <int HD, bool PIECES> __device__ __forceinline__ bool prefill_rows(cons
                 acc_s[tb][v] = p;
                 tile_sum += p;
             }
-        tile_sum += __shfl_xor(tile_sum, 32);
+        tile_sum = asf(fold_halves(asu(tile_sum), AddWords{}));
         run_sum = run_sum * alpha + tile_sum;
         run_max = new_max;
         if constexpr (!PIECES) {

@@ -21,9 +21,7 @@ constexpr int kThreads = 256, kWaves = 4;
 constexpr uint32_t kSeg = 128; // keys of a segment
 
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
-    return v;
+    return wave_add<1>(v);
 }
 __device__ __forceinline__ float block_sum(float v, float *red) {
     v = wave_sum(v);
@@ -153,8 +151,7 @@ template <int LANES> __global__ __launch_bounds__(kThreads) void attention_turn_
         float c = key ? 1.0f : temp;
         if (p.unit_heads) {
             float m = there ? fmaf(x.x, x.x, fmaf(x.y, x.y, fmaf(x.z, x.z, x.w * x.w))) : 0.0f;
-#pragma unroll
-            for (int e = 1; e < LANES; e <<= 1) m += __shfl_xor(m, e, 64);
+            m = asf(group_fold_up<LANES>(asu(m), AddWords{}));
             c /= sqrtf(m / (float)p.dim + p.eps);
         }
         if (!there || h0 + threadIdx.x / LANES >= heads) continue;
@@ -268,8 +265,7 @@ __global__ __launch_bounds__(kThreads) void attention_scores_kernel(const Attent
 #pragma unroll
         for (int h = 0; h < REP; h++) {
             float v = acc[h];
-            v += __shfl_xor(v, 1, 64);
-            v += __shfl_xor(v, 2, 64);
+            v = add_across<2>(add_across<1>(v));
             if (sub == 0) {
                 if (p.bias) v -= slope_of(h0 + h, p.heads) * (float)(int)(p.cached + s - j);
                 sc[h * kSeg + key] = j < hi ? v : -INFINITY;
@@ -281,8 +277,7 @@ __global__ __launch_bounds__(kThreads) void attention_scores_kernel(const Attent
     for (uint32_t h = wave; h < nh; h += kWaves) {
         const float a = sc[h * kSeg + lane], c = sc[h * kSeg + 64 + lane];
         float m = fmaxf(a, c);
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+        m = asf(wave_fold<1>(asu(m), LargerWords{}));
         const float l = m == -INFINITY ? 0.0f : wave_sum(expf(a - m) + expf(c - m));
         const int64_t head = (int64_t)blockIdx.z * p.heads + h0 + h;
         float *o = scores + (head * nseg + seg) * kSeg;

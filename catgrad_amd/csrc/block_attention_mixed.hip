@@ -26,9 +26,7 @@ constexpr uint32_t kSeg = 128; // keys of a segment of attention_scores_kernel
 constexpr float kLog2e = 1.44269504088896341f, kNone = -1e30f;
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v = fmaxf(v, __shfl_xor(v, d, 64));
-    return v;
+    return asf(wave_fold<1>(asu(v), LargerWords{}));
 }
 __device__ __forceinline__ float slope_of(uint32_t h, uint32_t heads) { return exp2f(-8.0f * (float)(h + 1) / (float)heads); }
 __device__ __forceinline__ uint32_t first_visible(const AttentionPlan &p, uint32_t i) { return p.window && i + 1 > p.window ? i + 1 - p.window : 0; }
@@ -333,8 +331,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_mixed_tiles_kernel(
 #pragma unroll
                 for (int i = 0; i < HPW; i++) {
                     float up = fmaxf(fmaxf(x[i][0], x[i][1]), fmaxf(x[i][2], x[i][3]));
-                    up = fmaxf(up, __shfl_xor(up, 16, 64));
-                    up = fmaxf(top[i], fmaxf(up, __shfl_xor(up, 32, 64)));
+                    up = fmaxf(top[i], asf(fold_halves(fold_rows(asu(up), LargerWords{}), LargerWords{})));
                     const float f = __builtin_amdgcn_exp2f(top[i] - up);
                     top[i] = up;
                     l[i] *= f;
@@ -387,9 +384,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_mixed_tiles_kernel(
     for (int i = 0; i < HPW; i++) {
         const uint32_t h = h0 + i;
         if (h >= p.heads) break;
-        float sum = l[i];
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
+        float sum = wave_add_up<16>(l[i]);
         if (splits > 1) {
             if (lg == 0 && s0 + li < p.S) stats[(split * rows + (uint64_t)b * p.S + s0 + li) * p.heads + h] = make_float2(top[i], sum);
             sum = 1.0f;
@@ -521,7 +516,7 @@ __global__ __launch_bounds__(kThreads, REP <= 4 ? 3 : 2) void attention_mixed_st
             float x[QV], m = 0.0f;
 #pragma unroll
             for (int v = 0; v < QV; v++) {
-                x[v] = fmaf(qv[i][v], turn[v].x, __shfl_xor(qv[i][v], 1, 64) * turn[v].y);
+                x[v] = fmaf(qv[i][v], turn[v].x, asf(across<1>(asu(qv[i][v]))) * turn[v].y);
                 if (lane + 64 * v < p.dim) m = fmaf(x[v], x[v], m);
             }
             float g = f;
@@ -580,8 +575,7 @@ __global__ __launch_bounds__(kThreads, REP <= 4 ? 3 : 2) void attention_mixed_st
                         const float y = fmaf(k[i][d][0], qv[0], fmaf(k[i][d][1], qv[1], fmaf(k[i][d][2], qv[2], k[i][d][3] * qv[3])));
                         x += e < p.dim ? y : 0.0f;
                     }
-                    x += __shfl_xor(x, 1, 64);
-                    x += __shfl_xor(x, 2, 64);
+                    x = add_across<2>(add_across<1>(x));
                     if (sub == 0 && there && h0 + h < rep) {
                         if (p.bias) x -= slope_of(hh, p.heads) * (float)(int)(p.cached + s - j);
                         lds[at.raw + hh * pitch + key] = key < keys ? x : 0.0f;
@@ -606,15 +600,13 @@ __global__ __launch_bounds__(kThreads, REP <= 4 ? 3 : 2) void attention_mixed_st
             const float top = lds[at.state + h];
             float m = top, l = 0.0f;
             for (uint32_t key = i % 4; key < chunk; key += 4) m = fmaxf(m, x[key]);
-            m = fmaxf(m, __shfl_xor(m, 1, 64));
-            m = fmaxf(m, __shfl_xor(m, 2, 64));
+            m = asf(group_fold_up<4>(asu(m), LargerWords{}));
             for (uint32_t key = i % 4; key < chunk; key += 4) {
                 const float e = __builtin_amdgcn_exp2f(x[key] - m);
                 x[key] = e;
                 l += e;
             }
-            l += __shfl_xor(l, 1, 64);
-            l += __shfl_xor(l, 2, 64);
+            l = add_across<2>(add_across<1>(l));
             if (i % 4 == 0) {
                 const float f = __builtin_amdgcn_exp2f(top - m);
                 lds[at.state + h] = m;

@@ -149,9 +149,7 @@ __global__ __launch_bounds__(kStatWaves * 64) void attention_row_stats_kernel(co
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     float up = x[r] * kLog2e;
-#pragma unroll
-                    for (int d = 1; d < 16; d <<= 1) up = fmaxf(up, __shfl_xor(up, d, 64)); // over the lanes that share the row
-                    up = fmaxf(top[i][r], up);
+                    up = fmaxf(top[i][r], asf(group_fold_up<16>(asu(up), LargerWords{}))); // over the lanes that share the row
                     l[i][r] *= __builtin_amdgcn_exp2f(top[i][r] - up);
                     top[i][r] = up;
                 }
@@ -164,9 +162,7 @@ __global__ __launch_bounds__(kStatWaves * 64) void attention_row_stats_kernel(co
     for (int i = 0; i < HPW; i++) {
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            float sum = l[i][r];
-#pragma unroll
-            for (int d = 1; d < 16; d <<= 1) sum += __shfl_xor(sum, d, 64);
+            float sum = asf(group_fold_up<16>(asu(l[i][r]), AddWords{}));
             if (p.zero_sink) sum += __builtin_amdgcn_exp2f(-top[i][r]);
             const uint32_t s = at.s0 + 4 * at.lg + r;
             if (at.li == 0 && s < p.S && h0 + i < p.heads) stats[((int64_t)at.b * p.S + s) * p.heads + h0 + i] = make_float2(top[i][r], 1.0f / sum);

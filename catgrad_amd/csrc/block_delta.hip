@@ -25,9 +25,7 @@ namespace {
 constexpr int kThreads = 256, kWaves = 4;
 
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
-    return v;
+    return wave_add<1>(v);
 }
 // on the hardware's exp2, log2 and reciprocal (about one unit in the last place each)
 __device__ __forceinline__ float sigmoid(float z) { return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.44269504088896341f)); }
@@ -198,8 +196,8 @@ template <int TAPS> __global__ __launch_bounds__(kThreads, 2) void delta_chunk_k
             m = fmaf(kt.x, ks.x, fmaf(kt.y, ks.y, fmaf(kt.z, ks.z, fmaf(kt.w, ks.w, m))));
             a = fmaf(qt.x, ks.x, fmaf(qt.y, ks.y, fmaf(qt.z, ks.z, fmaf(qt.w, ks.w, a))));
         }
-        m += __shfl_xor(m, 1, 64);
-        a += __shfl_xor(a, 1, 64);
+        m = add_across<1>(m);
+        a = add_across<1>(a);
         if ((tid & 1) == 0) {
             lower[t][s] = beta[t] * m;
             A[t * kChunk + s] = a;
@@ -436,9 +434,7 @@ __device__ __forceinline__ float quad_dot(const float *__restrict__ w, const flo
     } else {
         for (uint32_t i = sub; i < n; i += 4) s = fmaf(w[i], x[i], s);
     }
-    s += __shfl_xor(s, 1, 64);
-    s += __shfl_xor(s, 2, 64);
-    return s;
+    return add_across<2>(add_across<1>(s));
 }
 
 // conv_silu of TAPS taps in two halves: its inputs and taps asked for, and the rest
@@ -494,9 +490,7 @@ struct DotLoads {
             const float t = fmaf(a[j].x, c[j].x, fmaf(a[j].y, c[j].y, fmaf(a[j].z, c[j].z, a[j].w * c[j].w)));
             s += sub + 4 * j < n / 4 ? t : 0.0f;
         }
-        s += __shfl_xor(s, 1, 64);
-        s += __shfl_xor(s, 2, 64);
-        return s;
+        return add_across<2>(add_across<1>(s));
     }
 };
 

@@ -11,9 +11,7 @@ namespace {
 constexpr int kThreads = 256, kWaves = 4;
 
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
-    return v;
+    return wave_add<1>(v);
 }
 // sum over the 256 threads of a workgroup, for every thread; `red` has a slot per wave
 __device__ __forceinline__ float block_sum(float v, float *red) {
@@ -312,9 +310,7 @@ template <bool BF16> __device__ __forceinline__ void load_input(const ProductInp
 }
 // over the 16 lanes that share j
 __device__ __forceinline__ float blocks_sum(float v) {
-#pragma unroll
-    for (int d = 4; d < 64; d <<= 1) v += __shfl_xor(v, d, 64);
-    return v;
+    return wave_add_up<4>(v);
 }
 
 // A workgroup holds all of its waves' activations in registers (STEPS of 64 lanes' worth each) and walks column groups.

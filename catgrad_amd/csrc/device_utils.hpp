@@ -356,25 +356,59 @@ template <int LOW, class F> __device__ __forceinline__ uint32_t wave_fold(uint32
 struct AddWords {
     __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const { return asu(asf(a) + asf(b)); }
 };
-template <int LOW> __device__ __forceinline__ float wave_sum(float v) { return asf(wave_fold<LOW>(asu(v), AddWords{})); }
-// ... and in the other order, LOW, 2 LOW .. 32 (where the lanes' values do not repeat yet, only rows and halves can be folded)
-template <int LOW> __device__ __forceinline__ float wave_sum_up(float v) {
-#pragma unroll
-    for (int s = LOW; s < 8; s <<= 1) v += __shfl_xor(v, s);
-    if constexpr (LOW <= 8) v += asf(row_rotated<0x128>(asu(v)));
-    if constexpr (LOW <= 16) v = asf(fold_rows(asu(v), AddWords{}));
-    return asf(fold_halves(asu(v), AddWords{}));
-}
-// The value of the lane DIST away (16 or 32)
+template <int LOW> __device__ __forceinline__ float wave_add(float v) { return asf(wave_fold<LOW>(asu(v), AddWords{})); }
+// The value of the lane DIST away
 template <int DIST> __device__ __forceinline__ uint32_t across(uint32_t v) {
-    static_assert(DIST == 16 || DIST == 32, "a row or a half");
+    static_assert(DIST == 1 || DIST == 2 || DIST == 4 || DIST == 8 || DIST == 16 || DIST == 32, "a bit of the lane's number");
     if constexpr (DIST == 32) {
         const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
         return threadIdx.x & 32 ? (uint32_t)r[0] : (uint32_t)r[1];
-    } else {
+    } else if constexpr (DIST == 16) {
         const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
         return threadIdx.x & 16 ? (uint32_t)r[0] : (uint32_t)r[1];
+    } else if constexpr (DIST == 8) {
+        return row_rotated<0x128>(v);
+    } else if constexpr (DIST == 4) { // four up in the lower quads of a pair, four down in the upper
+        const uint32_t up = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x104, 0xF, 0x5, false);
+        return (uint32_t)__builtin_amdgcn_update_dpp((int)up, (int)v, 0x114, 0xF, 0xA, false);
+    } else {
+        return row_rotated<DIST == 2 ? 0x4E : 0xB1>(v);
     }
+}
+template <int DIST> __device__ __forceinline__ float add_across(float v) { return v + asf(across<DIST>(asu(v))); }
+struct LargerWords {
+    __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const { return asu(fmaxf(asf(a), asf(b))); }
+};
+// f over groups of W lanes, their nearest neighbours first (1, 2 .. W / 2): quads repeat by the time that they are mirrored
+template <int W, class F> __device__ __forceinline__ uint32_t group_fold_up(uint32_t v, F f) {
+    static_assert(W == 2 || W == 4 || W == 8 || W == 16 || W == 32 || W == 64, "a group of lanes");
+    v = f(v, across<1>(v));
+    if constexpr (W > 2) v = f(v, across<2>(v));
+    if constexpr (W > 4) v = f(v, row_rotated<0x141>(v)); // (eight lanes mirrored)
+    if constexpr (W > 8) v = f(v, row_rotated<0x140>(v)); // (sixteen)
+    if constexpr (W > 16) v = fold_rows(v, f);
+    if constexpr (W > 32) v = fold_halves(v, f);
+    return v;
+}
+// ... and their farthest ones first (W / 2 .. 1)
+template <int W, class F> __device__ __forceinline__ uint32_t group_fold(uint32_t v, F f) {
+    static_assert(W == 1 || W == 2 || W == 4 || W == 8 || W == 16 || W == 32 || W == 64, "a group of lanes");
+    if constexpr (W > 32) v = fold_halves(v, f);
+    if constexpr (W > 16) v = fold_rows(v, f);
+    if constexpr (W > 8) v = f(v, across<8>(v));
+    if constexpr (W > 4) v = f(v, across<4>(v));
+    if constexpr (W > 2) v = f(v, across<2>(v));
+    if constexpr (W > 1) v = f(v, across<1>(v));
+    return v;
+}
+// The sum over the lanes at distances LOW, 2 LOW .. 32, in that order
+template <int LOW> __device__ __forceinline__ float wave_add_up(float v) {
+    if constexpr (LOW <= 1) v = add_across<1>(v);
+    if constexpr (LOW <= 2) v = add_across<2>(v);
+    if constexpr (LOW <= 4) v = add_across<4>(v);
+    if constexpr (LOW <= 8) v += asf(row_rotated<0x128>(asu(v)));
+    if constexpr (LOW <= 16) v = asf(fold_rows(asu(v), AddWords{}));
+    return asf(fold_halves(asu(v), AddWords{}));
 }
 // The sums of four values over the lanes at distances 32, 16, 8 and 4, in that order: of v[r] in row r (lanes 16 r .. 16 r + 15).  Two
 // values share a register from the first step on, four from the second.

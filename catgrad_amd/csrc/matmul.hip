@@ -996,7 +996,7 @@ template <int MM> __global__ __launch_bounds__(kThreads) void skinny_kt_kernel(c
     }
 #pragma unroll
     for (int m = 0; m < MM; m++) {
-        const float v = wave_sum<1>(acc[m]);
+        const float v = wave_add<1>(acc[m]);
         if (lane == 0 && (uint32_t)m < a.M) a.C[((uint64_t)blockIdx.y * a.M + m) * a.N + n] = asu(v);
     }
 }
@@ -1085,7 +1085,7 @@ __device__ __forceinline__ void skinny_kt_wide_body(const MmArgs &a, const uint3
 #pragma unroll
     for (int c = 0; c < COLS; c++)
 #pragma unroll
-        for (int m = 0; m < MM; m++) acc[c][m] = wave_sum<1>(acc[c][m]);
+        for (int m = 0; m < MM; m++) acc[c][m] = wave_add<1>(acc[c][m]);
     if (SPLIT) {
         __shared__ float part[4][COLS * MM];
         if (lane == 0) {
@@ -1316,7 +1316,7 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
             if constexpr (!WHOLE || NORM) __builtin_amdgcn_sched_barrier(0); // (what follows stays behind all of the loads)
             if constexpr (NORM) {
                 if (c == 0 && k0 == 0) { // (the same for every thread)
-                    const float s = wave_sum<MM>(xreg_sums<MM>(*nf, pv));
+                    const float s = wave_add<MM>(xreg_sums<MM>(*nf, pv));
                     if (lane < MM) nsum[wave][lane] = s;
                     __syncthreads();
                     if (threadIdx.x < MM * 4 * (GATED ? 1 : CG)) divisor = norm_divisor(*nf, (nsum[0][threadIdx.x / 4 % MM] + nsum[1][threadIdx.x / 4 % MM]) + (nsum[2][threadIdx.x / 4 % MM] + nsum[3][threadIdx.x / 4 % MM]));
@@ -1585,7 +1585,7 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGrou
             if constexpr (!WHOLE || NORM) __builtin_amdgcn_sched_barrier(0); // (what follows stays behind all of the loads)
             if constexpr (NORM) {
                 if (c == 0 && k0 == 0) { // (the same for every thread)
-                    const float s = wave_sum<MM>(xreg_sums<MM>(nf, pv));
+                    const float s = wave_add<MM>(xreg_sums<MM>(nf, pv));
                     if (lane < MM) nsum[wave][lane] = s;
                     __syncthreads();
                     if (threadIdx.x < 64) divisor = norm_divisor(nf, (nsum[0][threadIdx.x / 4 % MM] + nsum[1][threadIdx.x / 4 % MM]) + (nsum[2][threadIdx.x / 4 % MM] + nsum[3][threadIdx.x / 4 % MM]));
@@ -1762,7 +1762,7 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs
     if constexpr (!WHOLE || NORM) __builtin_amdgcn_sched_barrier(0); // (what follows stays behind the loads)
     uint32_t divisor = 0;
     if constexpr (NORM) { // (the norm as in skinny_kt_mfma_xreg_body)
-        const float s = wave_sum<MM>(xreg_sums<MM>(nf, pv));
+        const float s = wave_add<MM>(xreg_sums<MM>(nf, pv));
         if (lane < MM) nsum[wave][lane] = s;
         __syncthreads();
         if (threadIdx.x < kOut) {
@@ -2575,7 +2575,7 @@ __global__ __launch_bounds__(kThreads) void skinny_kt_packed_kernel(const MmArgs
     }
 #pragma unroll
     for (int m = 0; m < MM; m++) {
-        acc[m] = wave_sum<1>(acc[m]);
+        acc[m] = wave_add<1>(acc[m]);
         if (lane == 0 && (uint32_t)m < a.M) a.C[(uint64_t)m * a.N + n] = asu(acc[m]);
     }
 }
