@@ -341,10 +341,11 @@ __device__ __forceinline__ void four_rows_linear(const ProductInput &in, const u
 #pragma unroll
         for (int s = 0; s < STEPS; s++)
 #pragma unroll
-            for (uint32_t i = 0; i < W; i += 4) { // (in.k is a multiple of W; behind it the activations are zero)
-                const f32x4 t = *reinterpret_cast<const f32x4_words *>(in.gamma + min(k0 + s * WAVES * SPAN + i, in.k - 4));
+            for (uint32_t i = 0; i < W; i += 4) { // (in.k is a multiple of W; zeros behind it, as the activations: the gains may be infinite)
+                const uint32_t k = k0 + s * WAVES * SPAN + i;
+                const f32x4 t = *reinterpret_cast<const f32x4_words *>(in.gamma + min(k, in.k - 4));
 #pragma unroll
-                for (int e = 0; e < 4; e++) gm[s][i + e] = t[e];
+                for (int e = 0; e < 4; e++) gm[s][i + e] = k < in.k ? t[e] : 0.0f;
             }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll

@@ -67,6 +67,19 @@ def run_linear(be, case, seed=0):
     close(be.to_numpy(out)[0], ref, 2e-5 if exact else 2e-2, f"linear {case}")
 
 
+def run_linear_infinite_gain(be, rows, K, dt):
+    """An infinite gain at each of the last columns: every product is that infinity with its term's sign, also where the kernel's
+    share of the columns ends behind the last one."""
+    rng = np.random.default_rng(K + rows)
+    x, w = rng.standard_normal((1, rows, K)).astype(np.float32), bf16(rng.standard_normal((40, K)))
+    xt, wt = be.from_numpy(x), weight(be, w, dt)
+    for at in range(K - 8, K):
+        gamma = np.ones(K, np.float32)
+        gamma[at] = np.inf
+        got = be.to_numpy(be.block_linear(xt, wt, gamma=be.from_numpy(gamma), eps=1e-3))[0]
+        np.testing.assert_array_equal(got, np.sign(x[0, :, at, None] * w[:, at]) * np.float32(np.inf))
+
+
 RESIDUAL = [  # rows, width, [(K, poly, gate)], weight dtype
     (1, 64, [(40, False, True), (96, True, True)], "f32"), (1, 520, [(257, True, False)], "f32"), (2, 256, [(512, False, True), (768, True, True)], "bf16"),
     (4, 2048, [(2048, False, True), (8192, True, True)], "f32"), (4, 1024, [(1024, False, True), (6144, True, True)], "bf16"),

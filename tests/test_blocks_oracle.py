@@ -9,6 +9,11 @@ def test_linear(oracle, case):
     C.run_linear(oracle, case)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_linear_infinite_gain(oracle, dtype):
+    C.run_linear_infinite_gain(oracle, 3, 520, dtype)
+
+
 @pytest.mark.parametrize("case", [c for c in C.RESIDUAL if c[0] * c[1] * sum(k for k, _, _ in c[2]) < 2e7], ids=str)
 def test_residual(oracle, case):
     C.run_residual(oracle, case)

@@ -12,6 +12,12 @@ def test_linear(hip, case):
     C.run_linear(hip, case)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("rows,K", [(1, 264), (4, 520), (3, 1032), (2, 1024), (1, 4104)])
+def test_linear_infinite_gain(hip, rows, K, dtype):
+    C.run_linear_infinite_gain(hip, rows, K, dtype)
+
+
 @pytest.mark.parametrize("case", C.RESIDUAL, ids=str)
 def test_residual(hip, case):
     C.run_residual(hip, case)
