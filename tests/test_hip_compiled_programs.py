@@ -7,13 +7,23 @@ from catgrad_amd import _abi as A
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module")
-def interpreter():
+@pytest.fixture(scope="module", autouse=True)
+def interpreter(hip):
     from backends import backend_with_env
 
     be = backend_with_env(CG_AOT="0")
+    hip.own_programs, be.own_programs = (1, 0), (0, 1)  # programs launched: compiled, interpreted
     yield be
     be.close()
+
+
+def realized(be, y):
+    """y computed in its own dtype, with a compiled program (or, on the backend without them, an interpreted one): a cast behind the
+    program would make it another."""
+    be.program_stats()
+    be.realize(y)
+    assert be.program_stats() == be.own_programs
+    return be.to_numpy(be.cast(y.move(), A.F32))
 
 
 def silu_mul(be, dtype, shape, rng):
@@ -22,7 +32,7 @@ def silu_mul(be, dtype, shape, rng):
     one = be.broadcast(be.cast(be.ndarray_from_vec_f32([1.0], ()), dtype).move(), shape)
     e = be.exp(be.neg(g).move())
     e = be.div(g.move(), be.add(one.move(), e.move()).move())
-    return [be.to_numpy(be.cast(be.mul(e.move(), u.move()).move(), A.F32))]
+    return [realized(be, be.mul(e.move(), u.move()))]
 
 
 def row_programs(be, shape, rng):
@@ -66,7 +76,7 @@ def gating(be, dtype, gate, up):
     one = be.broadcast(be.cast(be.ndarray_from_vec_f32([1.0], ()), dtype).move(), gate.shape)
     e = be.exp(be.neg(g).move())
     e = be.div(g.move(), be.add(one.move(), e.move()).move())
-    return be.to_numpy(be.cast(be.mul(e.move(), u.move()).move(), A.F32))
+    return realized(be, be.mul(e.move(), u.move()))
 
 
 @pytest.mark.parametrize("extra", [0, 1, 7, 9, 15, 4097])
