@@ -2044,6 +2044,7 @@ static bool try_row_append(cg_backend *b, cg_tensor *x, cg_tensor *y, size_t dim
     if (outer <= 1 || outer > 65536 || min_os % R) return false;
     if (!small && numel(x) * 4 < 65536) return false; // not worth the bookkeeping
     if (is_narrow_buf(x->buf)) { // rows are appended to 32-bit words
+        if (small) return false; // (the words of all of its buffer for a few rows: more than the copy)
         hipError_t she = hipSetDevice(b->device);
         *status = she == hipSuccess ? make_words(x) : hip_fail(she, "hipSetDevice");
         if (*status) return true;
@@ -2130,11 +2131,10 @@ static bool try_row_append(cg_backend *b, cg_tensor *x, cg_tensor *y, size_t dim
             nbuf->rs->nblocks = nb;
             nbuf->rs->fill.assign((size_t)nb, 0);
             int rc = b->pool.alloc((size_t)(nb * nbuf->rs->C * R) * 4, &nbuf->ptr, &nbuf->cls);
-            if (rc) {
+            if (rc) { // no room for the store: copied
                 delete nbuf->rs;
                 delete nbuf;
-                *status = rc;
-                return true;
+                return false;
             }
             nbuf->elems = nb * nbuf->rs->C * R;
             src->successor = nbuf;

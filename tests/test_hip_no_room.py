@@ -1,5 +1,5 @@
-"""Products whose scratch memory cannot be had give the results that they give with it: operands that are not packed are read as they
-are, sums over k are not cut.  A second process, in which the library's requests for device memory of chosen sizes are refused."""
+"""Calls whose scratch memory cannot be had give the results that they give with it: operands that are not packed are read as they
+are, sums over k are not cut, caches are copied without a store behind them.  A second process, in which the library's requests for device memory of chosen sizes are refused."""
 import os
 import subprocess
 import sys
@@ -79,6 +79,27 @@ for M, K, N, dtype, low, high in (
     assert np.array_equal(be.to_numpy(be.cast(z, A.F32)), want), (M, K, N, dtype)
     print(M, K, N, dtype, "requests refused:", seen, flush=True)
     assert seen, (M, K, N, dtype)
+
+# a cache, its dtype, the part of axis 2 that is appended to, the sizes that are refused, whether they are asked for at all
+for shape, dtype, part, low, high, asked in (
+        ((4, 4, 3, 256), A.F32, None, 500_000, 16 << 20, True),   # few tokens: a store with room for more
+        ((4, 4, 80, 256), A.F32, None, 4 << 20, 64 << 20, True),  # many
+        ((64, 16, 8, 128), A.BF16, 1, 3 << 20, 8 << 20, False)):  # a row of a tensor that lies in two bytes: not the words of all of it
+    a = whole(*shape)
+    row = whole(*shape[:2], 1, shape[3])
+    x, y = upload(a, dtype), upload(row, dtype)
+    if part is not None:
+        x, a = be.slice(x, 2, part, 1), a[:, :, part:part + 1]
+    be.pool_trim()
+    shim.refuse(low, high)
+    z = be.concat(x, y, 2)
+    z = be.concat(z.move(), y, 2)
+    be.sync()
+    seen = shim.count()
+    shim.refuse(1, 0)
+    assert np.array_equal(be.to_numpy(be.cast(z, A.F32)), np.concatenate([a, row, row], 2)), shape
+    print(shape, dtype, "requests refused:", seen, flush=True)
+    assert bool(seen) == asked, shape
 print("done", flush=True)
 """
 
