@@ -38,7 +38,7 @@ struct RowsArgs {
     int64_t os[kMaxOuter];
     uint32_t vec;         // 4: rows are unit-stride and 16-byte aligned; 8: the same for rows of a narrow format (one access of
                           // 16 bytes, fp8 8 bytes, holds 8 elements)
-    uint32_t fmt;         // how the elements lie in memory (kFmtWords, ...); narrow formats: reduce_rows_kernel only
+    uint32_t fmt;         // how the elements lie in memory (kFmtWords, ...); narrow formats: reduce_rows_kernel, reduce_segments_kernel
 };
 
 __device__ __forceinline__ int32_t total_key(uint32_t bits) { // Rust f32::total_cmp
@@ -262,7 +262,7 @@ template <int MODE, bool F, int VEC> __global__ __launch_bounds__(kBlock) void a
     if (hit) *a.flag = 1u;
 }
 
-// native: a view of a narrow buffer is described as it lies in memory (for reduce_rows_kernel); else as 32-bit words
+// native: a view of a narrow buffer is described as it lies in memory; else as 32-bit words
 int fill_rows_args(const cg_tensor *x, RowsArgs *a, bool native = false) {
     memset(a, 0, sizeof *a);
     const void *p;
@@ -310,13 +310,35 @@ int fill_rows_args(const cg_tensor *x, RowsArgs *a, bool native = false) {
 // Few, long rows (the arg-max over a 128 K vocabulary for a handful of sequences): a row per
 // workgroup would leave most of the chip idle, so every row is cut into segments, a workgroup
 // reduces one segment to a packed accumulator, and a second small kernel merges a row's segments.
+// Rows of a narrow format are read as they lie (widened first, all of the tensor that they are part of would be).
 template <int K, bool F>
 __global__ __launch_bounds__(kBlock) void reduce_segments_kernel(const RowsArgs a, long long *part, uint32_t seglen) {
     const uint32_t row = blockIdx.y, seg = blockIdx.x;
     const uint32_t lo = seg * seglen, hi = min(a.n, lo + seglen);
-    const uint32_t *p = reinterpret_cast<const uint32_t *>(a.x) + row_offset(row, a.nouter, a.od, a.odiv, a.os);
+    const int64_t base = row_offset(row, a.nouter, a.od, a.odiv, a.os);
+    const uint32_t *p = reinterpret_cast<const uint32_t *>(a.x) + base;
     Acc<K, F> acc;
-    if (a.vec == 4) { // seglen is a multiple of 4
+    if (a.fmt != kFmtWords) { // (the same for every lane: a launch parameter)
+        Operand o;
+        o.ptr = a.x;
+        o.is = a.sn;
+        o.uniform = 0;
+        o.fmt = a.fmt;
+        if (a.vec == 8) { // seglen and n are multiples of 8
+            for (uint32_t i = lo / 8 + threadIdx.x; i < hi / 8; i += kBlock) {
+                uint32_t t[8];
+                load_narrow<8>(o, base + 8 * (int64_t)i, t);
+#pragma unroll
+                for (int j = 0; j < 8; j++) acc.take(t[j], 8 * i + j);
+            }
+        } else {
+            for (uint32_t i = lo + threadIdx.x; i < hi; i += kBlock) {
+                uint32_t t[1];
+                load_narrow<1>(o, base + (int64_t)i * a.sn, t);
+                acc.take(t[0], i);
+            }
+        }
+    } else if (a.vec == 4) { // seglen is a multiple of 4
         for (uint32_t i = lo / 4 + threadIdx.x; i < hi / 4; i += kBlock) {
             const uint4 t = reinterpret_cast<const uint4 *>(p)[i];
             acc.take(t.x, 4 * i);
@@ -529,23 +551,24 @@ static int rows_route(const RowsArgs &a) {
 }
 
 template <int K, bool F> int launch_rows(cg_backend *be, const RowsArgs &a) {
-    if (rows_route(a) != 0 && a.fmt != kFmtWords) return fail(CG_ERR_ARG, "internal error: a narrow operand in a reduction kernel that reads words");
+    if (rows_route(a) == 1 && a.fmt != kFmtWords) return fail(CG_ERR_ARG, "internal error: a narrow operand in a reduction kernel that reads words");
     if (rows_route(a) == 1) return launch_cols<K, F>(be, a);
     if (rows_route(a) == 2) {
         uint32_t segs = std::min<uint32_t>(256, (a.n + 1023) / 1024);
-        const uint32_t seglen = ((a.n + segs - 1) / segs + 3) / 4 * 4;
+        const uint32_t unit = a.fmt == kFmtWords ? 4 : 8, seglen = ((a.n + segs - 1) / segs + unit - 1) / unit * unit;
         segs = (a.n + seglen - 1) / seglen;
         void *part = nullptr;
         size_t cls = 0;
-        int rc = be->pool.alloc((size_t)a.rows * segs * sizeof(long long), &part, &cls);
-        if (rc) return rc;
-        hipLaunchKernelGGL((reduce_segments_kernel<K, F>), dim3(segs, a.rows), dim3(kBlock), 0, be->stream, a,
-                           static_cast<long long *>(part), seglen);
-        hipLaunchKernelGGL((reduce_segments_final_kernel<K, F>), dim3(a.rows), dim3(64), 0, be->stream,
-                           static_cast<const long long *>(part), a.out, segs);
-        be->pool.free(part, cls); // stream-ordered: later users queue behind the merge
-        hipError_t e = hipGetLastError();
-        return e == hipSuccess ? CG_OK : hip_fail(e, "segmented reduction launch");
+        if (be->pool.alloc((size_t)a.rows * segs * sizeof(long long), &part, &cls) == CG_OK) {
+            hipLaunchKernelGGL((reduce_segments_kernel<K, F>), dim3(segs, a.rows), dim3(kBlock), 0, be->stream, a,
+                               static_cast<long long *>(part), seglen);
+            hipLaunchKernelGGL((reduce_segments_final_kernel<K, F>), dim3(a.rows), dim3(64), 0, be->stream,
+                               static_cast<const long long *>(part), a.out, segs);
+            be->pool.free(part, cls); // stream-ordered: later users queue behind the merge
+            hipError_t e = hipGetLastError();
+            return e == hipSuccess ? CG_OK : hip_fail(e, "segmented reduction launch");
+        }
+        // no room for the segments' results: a row per workgroup
     }
     // lanes per row: enough that a lane sees about eight elements, within {4,16,64,256}
     uint32_t want = (a.n + 7) / 8;
@@ -598,7 +621,7 @@ int launch_reduce(cg_backend *be, int kind, const cg_tensor *x, cg_tensor *out) 
     if (int frc = flush_deferred(be)) return frc;
     RowsArgs a;
     int rc = fill_rows_args(x, &a, true);
-    if (!rc && a.fmt != kFmtWords && rows_route(a) != 0) rc = fill_rows_args(x, &a); // those kernels read words
+    if (!rc && a.fmt != kFmtWords && rows_route(a) == 1) rc = fill_rows_args(x, &a); // those kernels read words
     if (rc) return rc;
     a.out = static_cast<uint32_t *>(out->buf->ptr);
     bool f = is_f(x->dt);

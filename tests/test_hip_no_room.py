@@ -100,6 +100,29 @@ for shape, dtype, part, low, high, asked in (
     assert np.array_equal(be.to_numpy(be.cast(z, A.F32)), np.concatenate([a, row, row], 2)), shape
     print(shape, dtype, "requests refused:", seen, flush=True)
     assert bool(seen) == asked, shape
+
+# sums and maxima of the rows of a tensor that lies in two bytes or one, as f32: neither its words nor a place for parts of rows is needed
+for shape, dtype, turn, low, high, asked in (
+        ((8, 262144), A.BF16, False, 10_000, 16 << 20, True),     # a few long rows: the parts
+        ((8, 262140), A.F16, False, 4 << 20, 16 << 20, False),
+        ((3, 400004), A.F8, False, 2 << 20, 16 << 20, False),
+        ((40000, 64), A.BF16, True, 8 << 20, 16 << 20, False),    # rows that lie side by side
+        ((1000, 2048), A.F8, True, 6 << 20, 16 << 20, False)):
+    a = whole(*shape)
+    x = upload(a, dtype)
+    if turn:
+        x, a = be.transpose(x, 0, 1), a.T
+    for op, want in ((be.sum, a.sum(-1, keepdims=True)), (be.max, a.max(-1, keepdims=True))):
+        be.pool_trim()
+        shim.refuse(low, high)
+        z = op(be.cast(x, A.F32).move())
+        be.realize(z)
+        be.sync()
+        seen = shim.count()
+        shim.refuse(1, 0)
+        assert np.array_equal(be.to_numpy(z), want), shape
+        print(shape, dtype, "requests refused:", seen, flush=True)
+        assert bool(seen) == asked, shape
 print("done", flush=True)
 """
 
