@@ -2580,17 +2580,6 @@ __global__ __launch_bounds__(kThreads) void skinny_kt_packed_kernel(const MmArgs
     }
 }
 
-// Columns of an [M, N] result that the 256-wide tiles compute.  Their workgroups, one per compute unit, walk the tiles in rounds; where
-// the last round leaves three quarters of the units idle, its columns go to the 128-wide tiles instead.  16-bit operands, us with a
-// last round and without: 1024 x 2048 x 16484 (4 tiles of 256 left over) 100 and 82, 18432 (32) 102 and 95, 20480 (64) 109 and 103, 24576
-// (128) 117 and 121; 2048 x 8192 x 8256 (8) 346 and 236, 10240 (64) 352 and 314, 12288 (128) 380 and 388.
-static int64_t wide_columns(const cg_backend *be, int kind, int64_t M, int64_t N, uint64_t tiles) {
-    const uint64_t units = (uint64_t)be->compute_units, over = tiles % units, rows = (uint64_t)(M + 255) / 256;
-    if (kind == 3 || tiles <= units || over == 0 || over * 4 > units) return N;
-    const int64_t columns = (int64_t)((tiles - over) / rows) * 256; // (whole columns of tiles)
-    return columns > 0 && N - columns <= N / 2 ? columns : N;
-}
-
 // x . y -> out on the 128-wide tiles, an operand that does not lie narrow packed first.  kDeclined: the pool has no room for that.
 static int low_product(cg_backend *be, int kind, const cg_tensor *x, bool x_lies, const cg_tensor *y, bool y_lies, MmArgs a, int64_t M, int64_t N, int64_t K,
                        cg_tensor *out) {
@@ -2866,7 +2855,7 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
                 if (dlds && !dlds_ok) prc = fail(CG_ERR_DEVICE, "matmul: cannot reserve %zu bytes of LDS", kDldsLdsBytes);
                 else if (dlds) {
                     const bool narrow_out = c_fmt != kFmtWords;
-                    const int64_t rest = N - wide_columns(be, kind, M, N, tiles);
+                    const int64_t rest = N - wide_columns(be->compute_units, kind, M, N);
                     if (rest > 0) {
                         const int64_t first = N - rest;
                         const int trc = launch_narrow_tiles(be, kind, pa, a_pitch * per, M, static_cast<const uint32_t *>(pb) + first * b_pitch, b_pitch * per, rest, K,

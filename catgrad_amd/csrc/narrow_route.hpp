@@ -37,4 +37,18 @@ inline NarrowRoute narrow_route(int kind, const NarrowSide &x, const NarrowSide 
     return fits_narrow_tiles(kind, x.lies ? x.pitch : k, x.rows, y.lies ? y.pitch : k, y.rows, k) ? NarrowRoute::low : NarrowRoute::words;
 }
 
+// Columns of an [M, N] result that the 256-wide tiles compute.  Their workgroups, one per compute unit, walk the tiles in rounds; where
+// the last round leaves three quarters of the units idle, its columns go to the 128-wide tiles instead.  16-bit operands, us with a
+// last round and without: 1024 x 2048 x 16484 (4 tiles of 256 left over) 100 and 82, 18432 (32) 102 and 95, 20480 (64) 109 and 103, 24576
+// (128) 117 and 121; 2048 x 8192 x 8256 (8) 346 and 236, 10240 (64) 352 and 314, 12288 (128) 380 and 388.
+// Whole columns of tiles move, of which a tall result has many in one, so how many tiles that are counts too: 5000 x 1024 x 4000 (64 left
+// over, 80 moved) 75 and 69, 20000 x 2048 x 1000 (60, 79) 120 and 107; 7424 x 512 x 2816 (63, 87) 39.5 and 40.9, with 2048 values of k
+// 101 and 100.5; 66600 x 1024 x 500 (10, 261) 116 and 127.  (What stays then fills its last round to eleven sixteenths or all of it.)
+inline int64_t wide_columns(int64_t units, int kind, int64_t M, int64_t N) {
+    const int64_t rows = (M + 255) / 256, tiles = rows * ((N + 255) / 256), over = tiles % units;
+    if (kind == 3 || tiles <= units || over == 0 || over * 4 > units) return N;
+    const int64_t columns = (tiles - over) / rows; // of tiles
+    return columns > 0 && (tiles - columns * rows) * 16 <= 5 * units ? columns * 256 : N;
+}
+
 } // namespace cg
