@@ -261,8 +261,9 @@ struct cg_tensor : cg::Pooled<cg_tensor> {
     uint32_t ubits = 0;
     // A deferred element-wise result: no buffer yet, `pend` says how to compute it.
     cg::Pending *pend = nullptr;
-    // Set (and retained) on the broadcast of deferred row maxima that somebody else holds too: `pend` computes them anew, for
-    // the one consumer to which that costs nothing (x - max x: the row is in registers); settle() gives every other the maxima.
+    // Set (and retained) on the broadcast of deferred row maxima that somebody else holds too, and on what follows from it: the first
+    // instruction of `pend` computes them anew, which costs nothing in a compiled program that has the row in registers.  settle() has
+    // the maxima read instead, before anything that no compiled program does.
     cg_tensor *row_of = nullptr;
     // Split axis: logical axis `split` (extent outer * split_inner) is addressed as
     // (i / split_inner) * split_os + (i % split_inner) * strides[split].  This is what
@@ -550,6 +551,9 @@ int launch_fused_reduce(cg_backend *be, int kind, bool f32, const Pending &p, in
 // Evaluates a program with row-reduce instructions over the iteration space `dims` (last axis = row).
 // reduced: `out` is dense with one element per row; else `out` is a (strided) view of shape `dims`.
 int launch_fused_rows(cg_backend *be, const cg_tensor *out, const Pending &p, const int64_t *dims, int rank);
+// Is there a kernel compiled for this program over rows of p.rowlen?  And do the compiled programs around a row's maximum begin like it?
+bool rows_program_compiled(const Pending &p);
+bool rows_max_program_begun(const Pending &p);
 int launch_arange(cg_backend *be, cg_tensor *out);
 // Copies n <= kReadbackWords words to be->rb_dev and then stores `seq` at word kReadbackWords of it, visible to the host.
 // (64 KiB: the runtime's staged copy and its wake-up cost 20 us more than the kernel's stores over the bus)

@@ -24,6 +24,7 @@ static std::recursive_mutex g_lazy_mu; // guards lazy backing of uniform tensors
 
 static int run_pending(cg_backend *be, const cg_tensor *dst, const Pending &p, bool fresh);
 static int settle(cg_tensor *t);
+static int settle_unless_compiled(cg_tensor *t);
 
 int fail(int code, const char *fmt, ...) {
     char buf[512];
@@ -793,7 +794,7 @@ static int run_pending(cg_backend *be, const cg_tensor *dst, const Pending &p) {
 // Row-major copy of a view (the materialising half of reshape / to_vec).
 int materialize(cg_backend *be, const cg_tensor *x, cg_tensor **out) {
     if (x->row_of) {
-        if (int rc = settle(const_cast<cg_tensor *>(x))) return rc;
+        if (int rc = settle_unless_compiled(const_cast<cg_tensor *>(x))) return rc;
     }
     cg_tensor *o;
     // a copy of a view of a narrow buffer keeps the buffer's format (whatever dtype tags the view); a program without row
@@ -1417,37 +1418,20 @@ static bool may_wait(const cg_backend *be, const cg_tensor *dst, const Pending *
     return be->fuse && be->aot && p && p->nred == 0 && !p->reduced && numel(dst) > 0 && numel(dst) <= 16384;
 }
 
-// A broadcast of shared row maxima (cg_tensor::row_of) becomes the view of them that it stands for.
-static int settle(cg_tensor *t) {
-    std::lock_guard<std::recursive_mutex> lk(g_lazy_mu);
-    if (!t->row_of) return CG_OK;
-    cg_tensor *m = t->row_of;
-    const int rc = ensure_concrete(m);
-    if (rc) return rc;
-    t->buf = m->buf;
-    t->buf->rc.fetch_add(1);
-    memcpy(t->strides, m->strides, sizeof t->strides);
-    t->strides[t->rank - 1] = 0;
-    t->offset = m->offset;
-    delete t->pend;
-    t->pend = nullptr;
-    t->row_of = nullptr;
-    release(m);
-    return CG_OK;
-}
-
 // The maxima of x's rows, nothing else: cheap to compute again inside a program that has the row in registers, up to the 16384
 // values that it keeps there (log-sum-exp and arg-max of 2000 x 12000: 101 us with the maxima's own pass, 79 without; 100 x 60000,
-// walked twice by one workgroup a row: 75 and 85).
+// walked twice by one workgroup a row: 75 and 85), and from 33 on (four lanes take a shorter one: no compiled program).
 static bool lone_row_max(const cg_tensor *x) {
     const Pending *p = x->pend;
     return p && p->reduced && p->nleaf == 1 && p->ninstr == 1 && p->ins[0].op == kRowMax && !p->overflow && !p->leaf[0].uniform && !p->leaf[0].pw &&
-           !p->leaf[0].lazy && x->dt == CG_F32 && x->be->aot && p->rowlen <= 16384;
+           !p->leaf[0].lazy && x->dt == CG_F32 && x->be->aot && p->rowlen > 32 && p->rowlen <= 16384;
 }
 
 // Turns a deferred tensor into a concrete one, in place (every holder of the handle sees it).
 int ensure_concrete(cg_tensor *t) {
-    if (t->row_of) return settle(t);
+    if (t->row_of) {
+        if (int rc = settle_unless_compiled(t)) return rc;
+    }
     if (t->split >= 0) { // a split-axis view becomes a plain dense tensor, in place
         std::lock_guard<std::recursive_mutex> lk(g_lazy_mu);
         if (t->split < 0) return CG_OK;
@@ -1628,6 +1612,72 @@ static uint8_t splice_program(Pending *p, const Pending *src, const int64_t *dim
     return last;
 }
 
+// What a deferred tensor computes from shared row maxima (cg_tensor::row_of) reads them from memory from here on: their broadcast is
+// a view of them, a program has them as one more leaf in the place of its first instruction.
+static int settle(cg_tensor *t) {
+    std::lock_guard<std::recursive_mutex> lk(g_lazy_mu);
+    if (!t->row_of) return CG_OK;
+    cg_tensor *m = t->row_of;
+    const int rc = ensure_concrete(m);
+    if (rc) return rc;
+    const int rank = t->rank;
+    if (t->pend->ninstr == 1) {
+        t->buf = m->buf;
+        t->buf->rc.fetch_add(1);
+        memcpy(t->strides, m->strides, sizeof t->strides);
+        t->strides[rank - 1] = 0;
+        t->offset = m->offset;
+        delete t->pend;
+        t->pend = nullptr;
+    } else {
+        const Pending *old = t->pend;
+        int64_t dims[kMaxRank]; // the program's iteration space
+        memcpy(dims, t->dims, sizeof dims);
+        if (old->reduced) dims[rank - 1] = old->rowlen;
+        Pending *p = new Pending;
+        uint8_t reg[kMaxLeaves + kMaxInstr];
+        for (int l = 0; l < old->nleaf; l++) reg[l] = (uint8_t)add_leaf(p, old->leaf[l], dims, rank);
+        LeafView lv{};
+        lv.buf = m->buf;
+        memcpy(lv.strides, m->strides, sizeof lv.strides);
+        lv.strides[rank - 1] = 0;
+        lv.offset = m->offset;
+        reg[kMaxLeaves] = (uint8_t)add_leaf(p, lv, dims, rank);
+        for (int i = 1; i < old->ninstr; i++) {
+            Instr in = old->ins[i];
+            in.a = reg[in.a];
+            in.b = reg[in.b];
+            in.c = reg[in.c];
+            reg[kMaxLeaves + i] = emit_instr(p, in);
+        }
+        if (p->nred > 0) {
+            p->rowlen = old->rowlen;
+            p->reduced = old->reduced;
+        }
+        if (!p->overflow && fused_program_fits(*p)) {
+            t->pend = p;
+            delete old;
+        } else {
+            delete p; // computed anew after all
+        }
+    }
+    t->row_of = nullptr;
+    release(m);
+    return CG_OK;
+}
+
+// A program that has its own kernel stays as it is: the maxima are taken from the row in registers.  (4096 x 8192, us with the maxima read
+// and so: x - max x 62 and 61, its exponentials 105 and 63, log-sum-exp 117 and 94.  What has no such kernel is interpreted, where
+// a second reduction costs most of the time: exp((x - max x) / 2) 116 and 361, rounded to bfloat16 59 and 304.)
+static int settle_unless_compiled(cg_tensor *t) {
+    std::lock_guard<std::recursive_mutex> lk(g_lazy_mu);
+    if (!t->row_of || !rows_program_compiled(*t->pend)) return settle(t);
+    cg_tensor *m = t->row_of;
+    t->row_of = nullptr;
+    release(m);
+    return CG_OK;
+}
+
 // x is deferred, but nothing more than a view of f32 values in a buffer (what a cast of values held in a narrower format leaves).
 static bool deferred_view(const cg_tensor *x) {
     const Pending *p = x->pend;
@@ -1651,31 +1701,13 @@ static int defer_elementwise(cg_backend *be, int op, cg_dtype in_dt, cg_dtype ou
             int rc = ensure_concrete(x);
             if (rc) return rc;
         }
-        if (x->row_of) { // row maxima that somebody else holds too: computed anew for x - max x alone
-            const cg_tensor *l = ins[0];
-            LeafView lv{};
-            bool of_buffer = false;
-            if (l->pend) {
-                of_buffer = deferred_view(l);
-                if (of_buffer) lv = l->pend->leaf[0];
-            } else if (l->buf && !l->uniform && l->split < 0) {
-                of_buffer = true;
-                lv.buf = l->buf;
-                memcpy(lv.strides, l->strides, sizeof lv.strides);
-                lv.offset = l->offset;
-            }
-            if (op != kSub || k != 1 || in_dt != CG_F32 || x->rc.load() != 1 || !of_buffer || !same_leaf(lv, x->pend->leaf[0], x->dims, rank)) {
-                int rc = settle(x);
-                if (rc) return rc;
-            }
-        }
         if (op != kAdd && x->pend && residual_sum_open(x)) { // see there; a further add may still join the sum
             int rc = ensure_concrete(x);
             if (rc) return rc;
         }
         if (!x->pend) continue;
         long mine = 0; // references to x that this very call consumes
-        for (int j = 0; j < nin; j++) mine += ins[j] == x;
+        for (int j = 0; j < nin; j++) mine += ins[j] == x || (ins[j]->row_of == x && ins[j]->rc.load() == 1);
         bool ok = x->rc.load() <= mine || cheap(x->pend);
         if (ok && x->pend->reduced) { // row results of different row lengths do not mix
             if (rowlen == 0) rowlen = x->pend->rowlen;
@@ -1699,6 +1731,7 @@ static int defer_elementwise(cg_backend *be, int op, cg_dtype in_dt, cg_dtype ou
         }
     }
     Pending *p = nullptr;
+    cg_tensor *maxima = nullptr; // shared ones that the program computes anew
     for (;;) { // build; while the program does not fit, compute the largest deferred input first and rebuild
         int64_t rl = 0;
         for (int k = 0; k < nin; k++)
@@ -1742,6 +1775,16 @@ static int defer_elementwise(cg_backend *be, int op, cg_dtype in_dt, cg_dtype ou
             p->rowlen = sdims[rank - 1];
             p->reduced = rl > 0;
         }
+        bool share = true;
+        maxima = nullptr;
+        for (int k = 0; k < nin; k++)
+            if (splice[k] && ins[k]->row_of) maxima = ins[k]->row_of, share = rows_max_program_begun(*p);
+        if (!share) { // nothing that ends in a compiled program: the maxima are read
+            delete p;
+            for (int k = 0; k < nin; k++)
+                if (int rc = settle(ins[k])) return rc;
+            return defer_elementwise(be, op, in_dt, out_dt, ins, nin, out);
+        }
         if (!p->overflow && p->nred <= kMaxRowReduce && fused_program_fits(*p)) break;
         delete p;
         int worst = -1;
@@ -1761,6 +1804,10 @@ static int defer_elementwise(cg_backend *be, int op, cg_dtype in_dt, cg_dtype ou
     memcpy(t->dims, shape_of->dims, sizeof t->dims);
     set_row_major(t);
     t->pend = p;
+    if (maxima) {
+        retain(maxima);
+        t->row_of = maxima;
+    }
     *out = t;
     return CG_OK;
 }
@@ -1770,7 +1817,7 @@ static int defer_elementwise(cg_backend *be, int op, cg_dtype in_dt, cg_dtype ou
 static int defer_reduce(cg_backend *be, int kind, cg_tensor *x, const int64_t *odims, cg_tensor **out) {
     *out = nullptr;
     const int rank = x->rank;
-    if (x->split >= 0 || x->row_of || (x->pend && x->pend->reduced)) {
+    if (x->split >= 0 || (x->pend && x->pend->reduced)) {
         int rc = ensure_concrete(x);
         if (rc) return rc;
     }
@@ -1804,6 +1851,11 @@ static int defer_reduce(cg_backend *be, int kind, cg_tensor *x, const int64_t *o
     emit_instr(p, in);
     p->rowlen = x->dims[rank - 1];
     p->reduced = true;
+    if (x->row_of && !rows_max_program_begun(*p)) {
+        delete p;
+        const int rc = settle(x);
+        return rc ? rc : defer_reduce(be, kind, x, odims, out);
+    }
     if (!fused_program_fits(*p)) {
         delete p;
         return CG_OK;
@@ -1815,6 +1867,10 @@ static int defer_reduce(cg_backend *be, int kind, cg_tensor *x, const int64_t *o
     memcpy(t->dims, odims, sizeof t->dims);
     set_row_major(t);
     t->pend = p;
+    if (x->row_of) {
+        retain(x->row_of);
+        t->row_of = x->row_of;
+    }
     *out = t;
     return CG_OK;
 }
@@ -1893,6 +1949,9 @@ static bool head_norm_lazy(cg_tensor *x) {
 template <class F>
 static int pending_view(cg_tensor *x, const int64_t *dims, int rank, F &&fn, cg_tensor **out, bool *handled) {
     *handled = false;
+    if (x->row_of) {
+        if (int rc = settle(x)) return rc;
+    }
     if (!x->pend) return CG_OK;
     if (x->pend->nred > 0 && !head_norm_lazy(x)) return ensure_concrete(x); // rows do not survive re-striding
     for (int l = 0; l < x->pend->nleaf; l++)
@@ -2369,7 +2428,7 @@ cg_dtype cg_tensor_dtype(const cg_tensor *t) { return t->dt; }
 size_t cg_tensor_numel(const cg_tensor *t) { return (size_t)numel(t); }
 int cg_tensor_is_contiguous(const cg_tensor *t) {
     Enter entered(t->be); // a deferred tensor may be being computed, in place, by another thread
-    if (t->row_of) return t->dims[t->rank - 1] == 1; // (a view of its rows' maxima)
+    if (t->row_of && t->pend->ninstr == 1) return t->dims[t->rank - 1] == 1; // (a view of its rows' maxima)
     if (t->pend) return 1; // a deferred result is row-major once computed
     return (t->uniform && numel(t) > 1) ? 0 : (is_contiguous(t) ? 1 : 0);
 }
@@ -3061,6 +3120,10 @@ static int reduce_entry(cg_backend *b, int kind, const char *what, cg_tensor *x,
     od[x->rank - 1] = 1;
     cg_tensor *o;
     int rc;
+    if (kind == kArgmax && x->row_of) {
+        rc = settle(x);
+        if (rc) return rc;
+    }
     if (b->fuse && kind != kArgmax && numel(x) > 0) {
         rc = defer_reduce(b, kind, x, od, out);
         if (rc || *out) return rc;
@@ -3161,6 +3224,10 @@ int cg_broadcast(cg_backend *b, cg_tensor *x, const size_t *dims, size_t rank, c
         if (x->dims[i] != d[i + shift] && x->dims[i] != 1)
             return fail(CG_ERR_SHAPE, "broadcast: incompatible shape (axis %d: %lld -> %lld)", i, (long long)x->dims[i],
                         (long long)d[i + shift]);
+    if (x->row_of) {
+        rc = settle(x);
+        if (rc) return rc;
+    }
     const bool alone = x->rc.load() == 1;
     if (x->pend && x->pend->reduced && (alone || lone_row_max(x)) && (int)rank == x->rank && d[rank - 1] == x->pend->rowlen) {
         // row results broadcast back over their rows: the same program, seen at full shape
@@ -3383,6 +3450,10 @@ int cg_concat(cg_backend *b, cg_tensor *x, cg_tensor *y, size_t dim, cg_tensor *
         *out = x;
         return CG_OK;
     }
+    for (cg_tensor *t : {x, y})
+        if (t->row_of) {
+            if (int src = settle(t)) return src;
+        }
     if (try_adjacent_merge(x, y, dim, out)) return CG_OK;
     {
         int arc;

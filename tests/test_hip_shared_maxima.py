@@ -104,6 +104,69 @@ def test_other_consumers_of_the_broadcast(hip, rows, cols):
     np.testing.assert_array_equal(hip.to_numpy(got), x.T - x.T.max(-1, keepdims=True))
 
 
+@pytest.mark.parametrize("rows,cols", [(70, 8192), (9, 130), (5, 64), (200, 24), (1, 33)])
+def test_programs_around_shared_maxima(hip, rows, cols):
+    """Every way on from x - max x: right, and the maxima taken anew only in a program that is compiled; the interpreter reads them,
+    from the reduction's own kernel (a launch of that class)."""
+    x, z = _x(rows, cols, False), _x(rows, cols, False)[:, ::-1].copy()
+    x[0, 0] = 9.0
+    m, d, e, lse = _want(x)
+    tx, tz, shape = hip.from_numpy(x), hip.from_numpy(z), (rows, cols)
+    half = hip.broadcast(hip.ndarray_from_vec_f32([0.5], ()), shape)
+    total = e.sum(-1, keepdims=True)
+    ways = {  # name: (what is made of x - max x and the maxima, its value, whether its program is a compiled one)
+        "shift": (lambda s, mx: s, d, True),
+        "exp": (lambda s, mx: hip.exp(s.move()), e, True),
+        "scaled": (lambda s, mx: hip.mul(s.move(), half), d * 0.5, False),
+        "temperature": (lambda s, mx: hip.exp(hip.mul(s.move(), half).move()), np.exp(d * 0.5), False),
+        "of_another": (lambda s, mx: hip.mul(s.move(), tz), d * z, False),
+        "sum": (lambda s, mx: hip.sum(s.move()), d.sum(-1, keepdims=True), False),
+        "largest": (lambda s, mx: hip.max(s.move()), np.zeros_like(m), False),
+        "sum_of_exp": (lambda s, mx: hip.sum(hip.exp(s.move()).move()), total, False),
+        "log_sum": (lambda s, mx: hip.log(hip.sum(hip.exp(s.move()).move()).move()), np.log(total), False),
+        "log_sum_exp_twice": (lambda s, mx: hip.mul(hip.add(hip.log(hip.sum(hip.exp(s.move()).move()).move()).move(), mx).move(),
+                                                    hip.broadcast(hip.ndarray_from_vec_f32([2.0], ()), (rows, 1)).move()), 2 * lse, False),
+        "maxima_first": (lambda s, mx: hip.add(mx, hip.log(hip.sum(hip.exp(s.move()).move()).move()).move()), lse, False),
+        "minus_log_sum": (lambda s, mx: hip.sub(s, hip.broadcast(hip.log(hip.sum(hip.exp(s).move()).move()).move(), shape).move()), d - np.log(total), None),
+        "soft_max": (lambda s, mx: (lambda ex: hip.div(ex, hip.broadcast(hip.sum(ex), shape).move()))(hip.exp(s.move())), e / total, None),
+        "maxima_again": (lambda s, mx: hip.sub(s.move(), hip.broadcast(mx, shape).move()), d - m, False),
+        "turned": (lambda s, mx: hip.exp(hip.transpose(s.move(), 0, 1).move()), e.T, False),
+        "part": (lambda s, mx: hip.exp(hip.slice(s.move(), 1, 1, cols - 3).move()), e[:, 1:cols - 2], False),
+        "reshaped": (lambda s, mx: hip.exp(hip.reshape(s.move(), (rows * cols, 1)).move()), e.reshape(-1, 1), False),
+        "beside": (lambda s, mx: hip.concat(s.move(), tz, 1), np.concatenate([d, z], 1), False),
+        "above": (lambda s, mx: hip.concat(tz, s.move(), 0), np.concatenate([z, d], 0), False),
+        "rounded": (lambda s, mx: hip.cast(s.move(), A.BF16), d, False),
+        "held": (lambda s, mx: hip.add(s, hip.exp(s).move()), d + e, None),
+        "where": (lambda s, mx: hip.where_cond(hip.lt(s, tz).move(), s, tz), np.minimum(d.astype(np.float32), z), None),
+    }
+    hip.profile_enable(A.K_REDUCE)
+    try:
+        for name, (way, want, compiled) in ways.items():
+            for kept in (True, False):
+                mx = hip.max(tx)
+                s = hip.sub(tx, hip.broadcast(mx, shape).move())
+                hip.sync()
+                hip.profile_read(A.K_REDUCE)
+                y = way(s, mx)
+                if not kept:
+                    del mx, s
+                hip.realize(y)
+                hip.sync()
+                launches = hip.profile_read(A.K_REDUCE)[0]
+                if compiled is not None and cols > 32:
+                    assert (launches == 0) == compiled, (name, kept, launches)
+                got = hip.to_numpy(hip.cast(y, A.F32))
+                if name == "rounded":
+                    assert (np.abs(got - want) <= 2.0 ** -8 * np.abs(want)).all(), name
+                else:
+                    tol = (cols / 256 + 32) * 2.0 ** -23
+                    assert (np.abs(got - want) <= tol * np.maximum(np.abs(want), np.abs(x).max() + np.abs(z).max())).all(), name
+                if kept:
+                    np.testing.assert_array_equal(hip.to_numpy(mx), m.astype(np.float32))
+    finally:
+        hip.profile_enable(A.K_REDUCE, 0)
+
+
 @pytest.mark.parametrize("rows,cols", [(300, 4096), (70, 16384), (9, 130)])
 def test_rows_that_lie_in_two_bytes(hip, rows, cols):
     x = _x(rows, cols, False)
