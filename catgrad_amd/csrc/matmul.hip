@@ -1201,10 +1201,29 @@ __device__ __forceinline__ uint32_t norm_divisor(const NormFuse &nf, float sum) 
 // interleaving the waves every 256 bytes).  A ragged last chunk: the waves interleaved every 64 values of k, so that what
 // there is of the chunk is shared by all four.
 // WHOLE: K is known to be whole chunks (the kernels branch once, at their top: loads without a test per trip).
-template <int TRIPS, bool WHOLE = false> __device__ __forceinline__ void xreg_lane_k(uint32_t K, uint32_t wave, uint32_t b, uint32_t &kb, uint32_t &ks) {
-    const bool ragged = !WHOLE && K % (TRIPS * 256) != 0;
-    kb = (ragged ? wave * 64 : wave * (TRIPS * 64)) + b * 4;
-    ks = ragged ? 256u : 64u;
+template <int TRIPS, bool WHOLE> __device__ __forceinline__ void xreg_lane_k(uint32_t wave, uint32_t b, uint32_t &kb, uint32_t &ks) {
+    kb = (WHOLE ? wave * (TRIPS * 64) : wave * 64) + b * 4;
+    ks = WHOLE ? 64u : 256u;
+}
+// A chunk's work with as many trips as what is left of K has (or one more): f(their number, as a constant).  Trips that lie behind K
+// altogether would be asked for like any others, clamped.  us with all of a chunk's trips and so: 4 x 512 x 8192 twice in a launch 23.6 and
+// 14.7, 4 x 2308 x 12288 24.7 and 19.1, with a residual sum 30.0 and 24.5.
+template <int TRIPS, bool WHOLE, class F> __device__ __forceinline__ void xreg_chunk(uint32_t left, F f) {
+    static_assert(TRIPS == 8 || TRIPS == 4, "chunks of 2048 or 1024");
+    constexpr std::integral_constant<int, TRIPS> all{};
+    if constexpr (WHOLE) {
+        f(all);
+    } else if constexpr (TRIPS == 8) {
+        if (left > 6 * 256) f(all);
+        else if (left > 4 * 256) f(std::integral_constant<int, 6>{});
+        else if (left > 3 * 256) f(std::integral_constant<int, 4>{});
+        else if (left > 2 * 256) f(std::integral_constant<int, 3>{});
+        else f(std::integral_constant<int, 2>{});
+    } else {
+        if (left > 3 * 256) f(all);
+        else if (left > 2 * 256) f(std::integral_constant<int, 3>{});
+        else f(std::integral_constant<int, 2>{});
+    }
 }
 // Four values of a row from k on, and what they count for: zeros behind K.  Loads behind K are clamped, not tested: a test in front of
 // every load leaves the compiler without a count of what is on its way, and it then waits for all of it before each of several groups.
@@ -1281,29 +1300,30 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
     float pv[2 * MM];
     if constexpr (NORM) xreg_ask_sums<MM>(*nf, pv);
     // of every chunk of TRIPS * 256 values of k (2048 or 1024) a wave takes a quarter in a row (TRIPS trips of 64)
-    static_assert(TRIPS == 8 || TRIPS == 4, "chunks of 2048 or 1024");
     uint32_t kb, ks;
-    xreg_lane_k<TRIPS, WHOLE>(a.K, wave, b, kb, ks);
-    for (uint32_t k0 = 0; k0 < a.K; k0 += TRIPS * 256) {
-        float4v xr[G][TRIPS];
+    xreg_lane_k<TRIPS, WHOLE>(wave, b, kb, ks);
+    uint32_t k0 = 0;
+    auto chunk = [&](auto trips) __attribute__((always_inline)) {
+        constexpr int T = decltype(trips)::value;
+        float4v xr[G][T];
 #pragma unroll
-        for (int t = 0; t < TRIPS; t++) {
+        for (int t = 0; t < T; t++) {
             const uint32_t k = k0 + kb + ks * t;
 #pragma unroll
             for (int g = 0; g < G; g++) xr[g][t] = xreg_at<WHOLE>(xrow[g], k, a.K);
         }
-        float4v gm[NORM ? TRIPS : 1]; // asked for with the activations, multiplied in once the first weights are on their way
+        float4v gm[NORM ? T : 1]; // asked for with the activations, multiplied in once the first weights are on their way
         if constexpr (NORM) {
 #pragma unroll
-            for (int t = 0; t < TRIPS; t++) {
+            for (int t = 0; t < T; t++) {
                 const uint32_t k = k0 + kb + ks * t;
                 gm[t] = xreg_at<WHOLE>(nf->gamma, k, a.K);
             }
         }
-        float4v ws[CG][TRIPS];
+        float4v ws[CG][T];
         auto ask = [&](int c) {
 #pragma unroll
-            for (int t = 0; t < TRIPS; t++) ws[c][t] = xreg_at<WHOLE>(wrow[c], k0 + kb + ks * t, a.K);
+            for (int t = 0; t < T; t++) ws[c][t] = xreg_at<WHOLE>(wrow[c], k0 + kb + ks * t, a.K);
         };
         if constexpr (NORM) { // all in front of the wait for the partial sums
 #pragma unroll
@@ -1311,7 +1331,7 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
         }
 #pragma unroll
         for (int c = 0; c < CG; c++) {
-            float4v (&w)[TRIPS] = ws[c];
+            float4v (&w)[T] = ws[c];
             if constexpr (!NORM) ask(c);
             if constexpr (!WHOLE || NORM) __builtin_amdgcn_sched_barrier(0); // (what follows stays behind all of the loads)
             if constexpr (NORM) {
@@ -1325,7 +1345,7 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
             if constexpr (NORM) {
                 if (c == 0) {
 #pragma unroll
-                    for (int t = 0; t < TRIPS; t++)
+                    for (int t = 0; t < T; t++)
 #pragma unroll
                         for (int g = 0; g < G; g++)
 #pragma unroll
@@ -1334,7 +1354,7 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
             }
             if constexpr (!WHOLE) {
 #pragma unroll
-                for (int t = 0; t < TRIPS; t++) {
+                for (int t = 0; t < T; t++) {
                     w[t] = xreg_within<WHOLE>(w[t], k0 + kb + ks * t, a.K);
 #pragma unroll
                     for (int g = 0; g < G; g++)
@@ -1342,7 +1362,7 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
                 }
             }
 #pragma unroll
-            for (int t = 0; t < TRIPS; t++)
+            for (int t = 0; t < T; t++)
 #pragma unroll
                 for (int g = 0; g < G; g++) {
                     acc[c][g] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[g][t][0], w[t][0], acc[c][g], 0, 0, 0);
@@ -1351,7 +1371,8 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
                     acc[c][g] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[g][t][3], w[t][3], acc[c][g], 0, 0, 0);
                 }
         }
-    }
+    };
+    for (; k0 < a.K; k0 += TRIPS * 256) xreg_chunk<TRIPS, WHOLE>(a.K - k0, chunk);
     __shared__ float part[4][CG * MM * 4];
 #pragma unroll
     for (int c = 0; c < CG; c++)
@@ -1518,7 +1539,6 @@ struct RopeGroup {
 };
 template <bool WHOLE, int MM, bool NORM, int TRIPS>
 __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGroup &g, const RopeGroup &rg, const NormFuse &nf) {
-    static_assert(TRIPS == 8 || TRIPS == 4, "chunks of 2048 or 1024");
     __shared__ float nsum[4][MM];
     uint32_t divisor = 0;
     float pv[2 * MM];
@@ -1561,27 +1581,29 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGrou
         sn = rs.sin[d];
     }
     uint32_t kb, ks;
-    xreg_lane_k<TRIPS, WHOLE>(a.K, wave, b, kb, ks);
+    xreg_lane_k<TRIPS, WHOLE>(wave, b, kb, ks);
     auto at = [&](const uint32_t *row, uint32_t k) { return xreg_at<WHOLE>(row, k, a.K); };
-    for (uint32_t k0 = 0; k0 < a.K; k0 += TRIPS * 256) {
-        float4v xr[G][TRIPS];
+    uint32_t k0 = 0;
+    auto chunk = [&](auto trips) __attribute__((always_inline)) {
+        constexpr int T = decltype(trips)::value;
+        float4v xr[G][T];
 #pragma unroll
-        for (int t = 0; t < TRIPS; t++)
+        for (int t = 0; t < T; t++)
 #pragma unroll
             for (int g = 0; g < G; g++) xr[g][t] = at(xrow[g], k0 + kb + ks * t);
-        float4v gm[NORM ? TRIPS : 1];
+        float4v gm[NORM ? T : 1];
         if constexpr (NORM) {
 #pragma unroll
-            for (int t = 0; t < TRIPS; t++) gm[t] = at(nf.gamma, k0 + kb + ks * t);
+            for (int t = 0; t < T; t++) gm[t] = at(nf.gamma, k0 + kb + ks * t);
         }
-        float4v ws[2][TRIPS];
+        float4v ws[2][T];
 #pragma unroll
         for (int c = 0; c < 2; c++)
 #pragma unroll
-            for (int t = 0; t < TRIPS; t++) ws[c][t] = at(wrow[c], k0 + kb + ks * t);
+            for (int t = 0; t < T; t++) ws[c][t] = at(wrow[c], k0 + kb + ks * t);
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-            float4v (&w)[TRIPS] = ws[c];
+            float4v (&w)[T] = ws[c];
             if constexpr (!WHOLE || NORM) __builtin_amdgcn_sched_barrier(0); // (what follows stays behind all of the loads)
             if constexpr (NORM) {
                 if (c == 0 && k0 == 0) { // (the same for every thread)
@@ -1594,7 +1616,7 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGrou
             if constexpr (NORM) {
                 if (c == 0) {
 #pragma unroll
-                    for (int t = 0; t < TRIPS; t++)
+                    for (int t = 0; t < T; t++)
 #pragma unroll
                         for (int g = 0; g < G; g++)
 #pragma unroll
@@ -1603,7 +1625,7 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGrou
             }
             if constexpr (!WHOLE) {
 #pragma unroll
-                for (int t = 0; t < TRIPS; t++) {
+                for (int t = 0; t < T; t++) {
                     w[t] = xreg_within<WHOLE>(w[t], k0 + kb + ks * t, a.K);
 #pragma unroll
                     for (int g = 0; g < G; g++)
@@ -1611,13 +1633,14 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGrou
                 }
             }
 #pragma unroll
-            for (int t = 0; t < TRIPS; t++)
+            for (int t = 0; t < T; t++)
 #pragma unroll
                 for (int g = 0; g < G; g++)
 #pragma unroll
                     for (int e = 0; e < 4; e++) acc[c][g] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[g][t][e], w[t][e], acc[c][g], 0, 0, 0);
         }
-    }
+    };
+    for (; k0 < a.K; k0 += TRIPS * 256) xreg_chunk<TRIPS, WHOLE>(a.K - k0, chunk);
     __shared__ float part[4][kOut];
 #pragma unroll
     for (int c = 0; c < 2; c++)
@@ -1712,13 +1735,12 @@ __global__ __launch_bounds__(kFinishThreads) void head_norm_rope_finish_kernel(c
 // the 128 MiB of gate + up, more leave too few workgroups in flight.  For q / k / v and o (a quarter of the columns)
 // one group per workgroup stays the fastest.  Weights are read with the non-temporal hint.
 // M <= MM, batch folded away (one batch entry).  Epilogues as in skinny_kt_mfma_xreg_body.
-template <bool WHOLE, int MM, bool NORM, int TRIPS>
+template <bool WHOLE, int MM, bool NORM, int CHUNK, int TRIPS>
 __device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs &a, const uint32_t *second, uint32_t one, uint32_t iters, const NormFuse &nf) {
-    static_assert(TRIPS == 8 || TRIPS == 4, "chunks of 2048 or 1024");
     const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     const uint32_t j = lane % 4, b = lane / 4;
     uint32_t kb, ks; // this lane's k: kb + ks t (beyond K, in a chunk that K does not fill: zeros)
-    xreg_lane_k<TRIPS, WHOLE>(a.K, wave, b, kb, ks);
+    xreg_lane_k<CHUNK, WHOLE>(wave, b, kb, ks);
     constexpr int G = MM / 4, kOut = 4 * MM; // row groups; values of one product in a group of columns
     float pv[2 * MM];
     if constexpr (NORM) xreg_ask_sums<MM>(nf, pv);
@@ -1824,8 +1846,11 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs
 template <int MM, bool NORM, int TRIPS>
 __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_cols_gated_kernel(const MmArgs a, const uint32_t *second, uint32_t one,
                                                                                   uint32_t iters, const NormFuse nf) {
-    if (a.K % (TRIPS * 256) == 0) skinny_kt_mfma_xreg_cols_gated_impl<true, MM, NORM, TRIPS>(a, second, one, iters, nf);
-    else skinny_kt_mfma_xreg_cols_gated_impl<false, MM, NORM, TRIPS>(a, second, one, iters, nf);
+    if (a.K % (TRIPS * 256) == 0) skinny_kt_mfma_xreg_cols_gated_impl<true, MM, NORM, TRIPS, TRIPS>(a, second, one, iters, nf);
+    else
+        xreg_chunk<TRIPS, false>(a.K, [&](auto trips) __attribute__((always_inline)) {
+            skinny_kt_mfma_xreg_cols_gated_impl<false, MM, NORM, TRIPS, decltype(trips)::value>(a, second, one, iters, nf);
+        });
 }
 
 // Vectorised skinny kernel for short K (K <= 4*LPC, e.g. q.K^T of a decode step with

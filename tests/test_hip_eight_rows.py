@@ -43,6 +43,38 @@ def test_steps_with_ragged_chunks(session, shape, rows):
     check(session, ENDS.get(shape) or SHAPES[shape], rows)
 
 
+# every number of trips that a last chunk can have, behind no chunk and behind one: heads of 64
+TRIPS = {f"hidden_{h}": ("llama", h, 8, 2, h + 4, 64) for h in (264, 772, 1796, 2564, 2820)}
+
+
+@pytest.mark.parametrize("rows", [1, 4, 8])
+@pytest.mark.parametrize("shape", list(TRIPS))
+def test_steps_with_every_last_chunk(session, shape, rows):
+    check(session, TRIPS[shape], rows)
+
+
+@pytest.mark.parametrize("K", [260, 512, 516, 768, 772, 1020, 1024, 1028, 1284, 1536, 1540, 1796, 2044, 2048, 2052, 2304, 2560, 2564, 2816, 2820, 3076, 3332, 4100])
+def test_products_of_every_last_chunk(hip, K):
+    """Alone, two and three in a launch, with a residual sum; columns for one and for two groups of four a workgroup.  Whole numbers: every order of
+    summation gives the same."""
+    rng = np.random.default_rng(K)
+    for N in (2052, 4100, 8196):
+        w = rng.integers(-3, 4, (3, N, K)).astype(np.float32)
+        tw = [hip.from_numpy(a) for a in w]
+        for rows in (1, 4, 5, 8):
+            x, r = rng.integers(-3, 4, (1, rows, K)).astype(np.float32), rng.integers(-9, 10, (1, rows, N)).astype(np.float32)
+            tx, want = hip.from_numpy(x), [x[0] @ a.T for a in w]
+
+            def product(i):
+                return hip.matmul(tx, hip.broadcast(hip.transpose(tw[i], 0, 1), (1, K, N)).move())
+
+            np.testing.assert_array_equal(hip.to_numpy(product(0))[0], want[0])
+            for n in (2, 3):
+                for i, y in enumerate([product(i) for i in range(n)]):
+                    np.testing.assert_array_equal(hip.to_numpy(y)[0], want[i])
+            np.testing.assert_array_equal(hip.to_numpy(hip.add(product(1).move(), hip.from_numpy(r)))[0], want[1] + r[0])
+
+
 def check(session, shape, rows):
     arch, hidden, heads, kv, ff, hd = shape
     cfg = LlmConfig(arch, hidden, 2, heads, kv, ff, 521, head_dim=hd, rms_norm_eps=1e-5, rope_theta=10000.0, tie_word_embeddings=True)
