@@ -502,12 +502,23 @@ __global__ __launch_bounds__(WAVES * 64) void four_rows_residual_kernel(const Ro
         if (NB > 1 && b1.gate.p) gate[NB - 1] = b1.gate.p[(int64_t)mr * b1.gate.pitch + n] + (b1.gate_bias ? b1.gate_bias[n] : 0.0f);
     }
     BranchLoads<BF16, NG> loads[NB];
-    const uint32_t first = wave * 16 * Frag<BF16>::W;
-    ask_branch<BF16, NG, WAVES>(b0, rows, width, n0, first, loads[0]);
-    if (NB > 1) ask_branch<BF16, NG, WAVES>(b1, rows, width, n0, first, loads[NB - 1]);
-    __builtin_amdgcn_sched_barrier(0); // (or the compiler asks for a few at a time)
-    walk_branch<BF16, NG, WAVES, POLY0>(b0, rows, width, n0, loads[0], s[0]);
-    if (NB > 1) walk_branch<BF16, NG, WAVES, POLY1>(b1, rows, width, n0, loads[NB - 1], s[NB - 1]);
+    const uint32_t first = __builtin_amdgcn_readfirstlane(wave) * 16 * Frag<BF16>::W;
+    const bool in0 = first < b0.w.k, in1 = NB > 1 && first < b1.w.k;
+    if (in0 && in1) {
+        ask_branch<BF16, NG, WAVES>(b0, rows, width, n0, first, loads[0]);
+        ask_branch<BF16, NG, WAVES>(b1, rows, width, n0, first, loads[NB - 1]);
+        __builtin_amdgcn_sched_barrier(0); // (or the compiler asks for a few at a time)
+        walk_branch<BF16, NG, WAVES, POLY0>(b0, rows, width, n0, loads[0], s[0]);
+        walk_branch<BF16, NG, WAVES, POLY1>(b1, rows, width, n0, loads[NB - 1], s[NB - 1]);
+    } else if (in0) { // a branch too short for the wave is none of its work (4096 columns of 128 + 128, f32: 17.0 us with it, 10.4 without)
+        ask_branch<BF16, NG, WAVES>(b0, rows, width, n0, first, loads[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        walk_branch<BF16, NG, WAVES, POLY0>(b0, rows, width, n0, loads[0], s[0]);
+    } else if (in1) {
+        ask_branch<BF16, NG, WAVES>(b1, rows, width, n0, first, loads[NB - 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        walk_branch<BF16, NG, WAVES, POLY1>(b1, rows, width, n0, loads[NB - 1], s[NB - 1]);
+    }
 #pragma unroll
     for (int b = 0; b < NB; b++) {
         const bool poly = b == 0 ? POLY0 : POLY1;
