@@ -37,8 +37,9 @@ __device__ __forceinline__ float softplus(float z) {
 }
 
 // Channel c of the three projections side by side: where its column of tokens begins (at sequence b, token 0), and its taps.
-// (Arguments are pinned to scalar registers before a lane chooses among them: left to itself the compiler chooses their place in
-// the argument block and has every lane fetch from there, a trip to memory in front of all others.)
+// (PIN: arguments are pinned to scalar registers before a lane chooses among them.  Left to itself the compiler chooses their place in
+// the argument block and has every lane fetch from there, a trip to memory in front of all others: 13.0 us for a
+// token and 11.8 pinned, states of 128 x 128.  In a loop over tokens the registers are worth more: two tokens 21.9 pinned, 19.0 not.)
 typedef const __attribute__((address_space(1))) float global_float;
 __device__ __forceinline__ int64_t pinned(int64_t v) {
     asm volatile("" : "+s"(v));
@@ -49,13 +50,15 @@ struct Channel {
     global_float *x, *taps;
     int64_t pitch;
 };
-__device__ __forceinline__ Channel channel(const DeltaPlan &p, uint32_t b, uint32_t c) {
+template <bool PIN> __device__ __forceinline__ Channel channel(const DeltaPlan &p, uint32_t b, uint32_t c) {
     const uint32_t kc = p.kv_heads * p.dim;
     const bool is_q = c < kc, is_k = c < 2 * kc;
     const uint32_t e = is_q ? c : is_k ? c - kc : c - 2 * kc;
-    global_float *const xq = pinned(p.q.p), *const xk = pinned(p.k.p), *const xv = pinned(p.v.p);
-    global_float *const wq = pinned(p.conv_q), *const wk = pinned(p.conv_k), *const wv = pinned(p.conv_v);
-    const int64_t pq = pinned(p.q.pitch), pk = pinned(p.k.pitch), pv = pinned(p.v.pitch);
+    auto held = [](const float *q) { return PIN ? pinned(q) : (global_float *)q; };
+    auto held_pitch = [](int64_t v) { return PIN ? pinned(v) : v; };
+    global_float *const xq = held(p.q.p), *const xk = held(p.k.p), *const xv = held(p.v.p);
+    global_float *const wq = held(p.conv_q), *const wk = held(p.conv_k), *const wv = held(p.conv_v);
+    const int64_t pq = held_pitch(p.q.pitch), pk = held_pitch(p.k.pitch), pv = held_pitch(p.v.pitch);
     global_float *x = is_q ? xq : is_k ? xk : xv, *w = is_q ? wq : is_k ? wk : wv;
     const int64_t pitch = is_q ? pq : is_k ? pk : pv;
     return {x + (int64_t)b * p.S * pitch + e, w + (int64_t)e * p.taps, pitch};
@@ -67,7 +70,7 @@ __device__ __forceinline__ float conv_input(const DeltaPlan &p, const Channel &c
     return p.conv_state ? p.conv_state[((int64_t)b * (p.taps - 1) + (t + (int)p.taps - 1)) * C + c] : 0.0f;
 }
 __device__ __forceinline__ float conv_silu(const DeltaPlan &p, uint32_t b, int t, uint32_t c) {
-    const Channel ch = channel(p, b, c);
+    const Channel ch = channel<false>(p, b, c);
     float s = 0.0f;
     for (uint32_t i = 0; i < p.taps; i++) s = fmaf(conv_input(p, ch, b, t - (int)(p.taps - 1 - i), c), ch.taps[i], s);
     return s * sigmoid(s);
@@ -90,7 +93,7 @@ __device__ void keep_inputs(const DeltaPlan &p, uint32_t b, uint32_t h) {
     for (uint32_t i = threadIdx.x; i < past * n; i += blockDim.x) {
         const uint32_t j = i / n, e = i - j * n;
         const uint32_t c = e < nq ? (h / rep) * p.dim + e : e < 2 * nq ? kc + (h / rep) * p.dim + (e - nq) : 2 * kc + h * p.vdim + (e - 2 * nq);
-        p.conv_out[((int64_t)b * past + j) * C + c] = conv_input(p, channel(p, b, c), b, (int)(p.S + j) - (int)past, c);
+        p.conv_out[((int64_t)b * past + j) * C + c] = conv_input(p, channel<false>(p, b, c), b, (int)(p.S + j) - (int)past, c);
     }
 }
 
@@ -107,7 +110,7 @@ __device__ __host__ constexpr uint32_t chunk_floats(uint32_t dp) { return 48 * d
 // Outputs of the convolution of channel c (of 16 tokens from t0; n of them are there), silu applied.  TAPS 0: any count.
 template <int TAPS> __device__ __forceinline__ void conv_chunk(const DeltaPlan &p, uint32_t b, uint32_t t0, uint32_t n, uint32_t c, float (&y)[kChunk]) {
     if constexpr (TAPS > 0) {
-        const Channel ch = channel(p, b, c);
+        const Channel ch = channel<false>(p, b, c);
         global_float *x = ch.x + (int64_t)t0 * ch.pitch;
         float in[kChunk + TAPS - 1], wt[TAPS];
 #pragma unroll
@@ -438,11 +441,11 @@ __device__ __forceinline__ float quad_dot(const float *__restrict__ w, const flo
 }
 
 // conv_silu of TAPS taps in two halves: its inputs and taps asked for, and the rest
-template <int TAPS> struct ConvLoads {
+template <int TAPS, bool PIN> struct ConvLoads {
     float x[TAPS], tap[TAPS];
     __device__ __forceinline__ void ask(const DeltaPlan &p, uint32_t b, int t, uint32_t c) {
         const uint32_t C = 2 * p.kv_heads * p.dim + p.heads * p.vdim;
-        const Channel ch = channel(p, b, c);
+        const Channel ch = channel<PIN>(p, b, c);
         global_float *now = ch.x + (int64_t)t * ch.pitch;
         global_float *kept = p.conv_state ? (global_float *)p.conv_state + ((int64_t)b * (TAPS - 1) + t + TAPS - 1) * C + c : now;
         const int64_t kept_pitch = p.conv_state ? C : 0;
@@ -464,7 +467,7 @@ template <int TAPS> __device__ __forceinline__ float conv_step(const DeltaPlan &
     if constexpr (TAPS == 0) {
         return conv_silu(p, b, t, c);
     } else {
-        ConvLoads<TAPS> l;
+        ConvLoads<TAPS, false> l;
         l.ask(p, b, t, c);
         return l.value(p, t);
     }
@@ -506,7 +509,7 @@ template <int R, int TAPS, bool DIRECT> __global__ __launch_bounds__(kStepThread
     const uint32_t tid = threadIdx.x, c = tid & (lanes - 1), group = tid / lanes, groups = kStepThreads / lanes;
     const int64_t sb = ((int64_t)b * p.heads + h) * D * V;
     constexpr uint32_t ROWS = kStepThreads / 4; // rows of the factored projections per round
-    ConvLoads<TAPS ? TAPS : 1> conv;
+    ConvLoads<TAPS ? TAPS : 1, true> conv;
     DotLoads dot[DIRECT ? 2 : 1];
     auto channel_of = [&](uint32_t u) { return u < D ? kh * D + u : u < 2 * D ? kc + kh * D + u - D : 2 * kc + h * V + u - 2 * D; };
     auto ask = [&](uint32_t t) {
