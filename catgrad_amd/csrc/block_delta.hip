@@ -110,7 +110,7 @@ __device__ __host__ constexpr uint32_t chunk_floats(uint32_t dp) { return 48 * d
 // Outputs of the convolution of channel c (of 16 tokens from t0; n of them are there), silu applied.  TAPS 0: any count.
 template <int TAPS> __device__ __forceinline__ void conv_chunk(const DeltaPlan &p, uint32_t b, uint32_t t0, uint32_t n, uint32_t c, float (&y)[kChunk]) {
     if constexpr (TAPS > 0) {
-        const Channel ch = channel<false>(p, b, c);
+        const Channel ch = channel<true>(p, b, c); // (1024 tokens of 16 heads of 32 x 32: 131 us without, 124.5)
         global_float *x = ch.x + (int64_t)t0 * ch.pitch;
         float in[kChunk + TAPS - 1], wt[TAPS];
 #pragma unroll
