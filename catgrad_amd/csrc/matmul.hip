@@ -1154,6 +1154,9 @@ static inline uint32_t xreg_cols_iters(uint64_t groups) {
 // instructions per weight load instead of one and four.  Against the vector-unit kernels without the norms, gates and cache rows in
 // their loads and stores (up to 14 launches a layer instead of 5): Llama-3.2-1B shape, six sequences 2.44 -> 1.67 ms a step; SmolLM2-135M
 // shape, eight 1.93 -> 1.27; Qwen3-0.6B shape, five 2.8 -> 2.2.
+// Products without any of that: weights from memory, as a model's are, in us on the vector-unit kernels and here: 5 x 3072 x 8192 34 and 29, 8 x
+// 4096 x 4096 31 and 28.6, two of them in a launch 60 and 46, 8 x 2048 x 8192 31 and 24.  Weights that the last-level cache still holds from the call
+// before are faster on those: 5 x 3072 x 8192 22 and 26, 8 x 4096 x 4096 23 and 28, 8 x 2048 x 8192 22 and 23.
 static inline bool xreg_narrow(uint32_t M, uint32_t K) { return M >= 1 && M <= 8 && xreg_trips(K) != 0; }
 constexpr int kMaxGroup = 4;
 struct MmGroup {
@@ -1200,10 +1203,14 @@ __device__ __forceinline__ uint32_t norm_divisor(const NormFuse &nf, float sum) 
 // takes a quarter of the chunk in a row (2 KiB in a row of each weight row: measured 12 % faster on the gate / up pair than
 // interleaving the waves every 256 bytes).  A ragged last chunk: the waves interleaved every 64 values of k, so that what
 // there is of the chunk is shared by all four.
-// WHOLE: K is known to be whole chunks (the kernels branch once, at their top: loads without a test per trip).
+// WHOLE: K is whole chunks (a kernel of its own: the registers of the other's branches would cost a workgroup per compute unit).
 template <int TRIPS, bool WHOLE> __device__ __forceinline__ void xreg_lane_k(uint32_t wave, uint32_t b, uint32_t &kb, uint32_t &ks) {
     kb = (WHOLE ? wave * (TRIPS * 64) : wave * 64) + b * 4;
     ks = WHOLE ? 64u : 256u;
+}
+template <class F> static void xreg_either(uint32_t K, int trips, F f) { // f(is K whole chunks of that many trips, as a constant)
+    if (trips && K % (trips * 256) == 0) f(std::true_type{});
+    else f(std::false_type{});
 }
 // A chunk's work with as many trips as what is left of K has (or one more): f(their number, as a constant).  Trips that lie behind K
 // altogether would be asked for like any others, clamped.  us with all of a chunk's trips and so: 4 x 512 x 8192 twice in a launch 23.6 and
@@ -1258,8 +1265,8 @@ template <int MM> __device__ __forceinline__ float xreg_sums(const NormFuse &nf,
     return s;
 }
 template <bool WHOLE, int MM, int CG, bool GATED, bool RESIDUAL, bool NORM, int TRIPS>
-__device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, const uint32_t block_x, const uint32_t block_y, const uint32_t *second,
-                                                              const uint32_t one, const MmResidual *res, const NormFuse *nf) {
+__device__ __forceinline__ void skinny_kt_mfma_xreg_body(const MmArgs &a, const uint32_t block_x, const uint32_t block_y, const uint32_t *second = nullptr,
+                                                         const uint32_t one = 0, const MmResidual *res = nullptr, const NormFuse *nf = nullptr) {
     static_assert(MM == 4 || MM == 8, "one or two groups of four rows");
     static_assert(!GATED || CG == 2, "a gated pair is two column groups");
     static_assert(!(GATED && RESIDUAL), "one epilogue at a time");
@@ -1419,24 +1426,16 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body_impl(const MmArgs &a, c
         }
     }
 }
-template <int MM, int CG, bool GATED = false, bool RESIDUAL = false, bool NORM = false, int TRIPS = 8>
-__device__ __forceinline__ void skinny_kt_mfma_xreg_body(const MmArgs &a, const uint32_t block_x, const uint32_t block_y,
-                                                         const uint32_t *second = nullptr, const uint32_t one = 0,
-                                                         const MmResidual *res = nullptr, const NormFuse *nf = nullptr) {
-    if (a.K % (TRIPS * 256) == 0) skinny_kt_mfma_xreg_body_impl<true, MM, CG, GATED, RESIDUAL, NORM, TRIPS>(a, block_x, block_y, second, one, res, nf);
-    else skinny_kt_mfma_xreg_body_impl<false, MM, CG, GATED, RESIDUAL, NORM, TRIPS>(a, block_x, block_y, second, one, res, nf);
+template <bool WHOLE, int MM, int CG, int TRIPS> __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_kernel(const MmArgs a) {
+    skinny_kt_mfma_xreg_body<WHOLE, MM, CG, false, false, false, TRIPS>(a, blockIdx.x, blockIdx.y);
 }
-
-template <int MM, int CG, int TRIPS = 8> __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_kernel(const MmArgs a) {
-    skinny_kt_mfma_xreg_body<MM, CG, false, false, false, TRIPS>(a, blockIdx.x, blockIdx.y);
-}
-template <int MM, int TRIPS = 8>
+template <bool WHOLE, int MM, int TRIPS>
 __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_gated_kernel(const MmArgs a, const uint32_t *second, uint32_t one) {
-    skinny_kt_mfma_xreg_body<MM, 2, true, false, false, TRIPS>(a, blockIdx.x, blockIdx.y, second, one);
+    skinny_kt_mfma_xreg_body<WHOLE, MM, 2, true, false, false, TRIPS>(a, blockIdx.x, blockIdx.y, second, one);
 }
-template <int MM, int TRIPS = 8>
+template <bool WHOLE, int MM, int TRIPS>
 __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_residual_kernel(const MmArgs a, const MmResidual r) {
-    skinny_kt_mfma_xreg_body<MM, 1, false, true, false, TRIPS>(a, blockIdx.x, blockIdx.y, nullptr, 0, &r);
+    skinny_kt_mfma_xreg_body<WHOLE, MM, 1, false, true, false, TRIPS>(a, blockIdx.x, blockIdx.y, nullptr, 0, &r);
 }
 // The same sum with residual terms for up to four rows, eight columns and all of K by eight waves: an eighth of a chunk of K each,
 // every load of a chunk asked for before the first product.  The kernel above fetches as many bytes of activations as of weights
@@ -1511,21 +1510,21 @@ static inline int eight_trips(const cg_backend *be, uint32_t M, uint32_t N, uint
     return K % 8192 == 0 && M <= 4 ? 16 : K % 4096 == 0 ? 8 : K % 2048 == 0 ? 4 : 0; // (16 trips of eight rows: more registers than there are)
 }
 // the gated pair with the RMS norm of the left operand applied on load
-template <int MM, int TRIPS = 8>
+template <bool WHOLE, int MM, int TRIPS>
 __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_gated_norm_kernel(const MmArgs a, const uint32_t *second, uint32_t one,
                                                                                   const NormFuse nf) {
-    skinny_kt_mfma_xreg_body<MM, 2, true, false, true, TRIPS>(a, blockIdx.x, blockIdx.y, second, one, nullptr, &nf);
+    skinny_kt_mfma_xreg_body<WHOLE, MM, 2, true, false, true, TRIPS>(a, blockIdx.x, blockIdx.y, second, one, nullptr, &nf);
 }
-template <int MM, int CG, int TRIPS = 8> __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_group_kernel(const MmGroup g) {
+template <bool WHOLE, int MM, int CG, int TRIPS> __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_group_kernel(const MmGroup g) {
     uint32_t bx;
     const uint32_t p = group_problem(g, bx);
-    skinny_kt_mfma_xreg_body<MM, CG, false, false, false, TRIPS>(g.p[p], bx, 0);
+    skinny_kt_mfma_xreg_body<WHOLE, MM, CG, false, false, false, TRIPS>(g.p[p], bx, 0);
 }
-template <int MM, int TRIPS = 8>
+template <bool WHOLE, int MM, int TRIPS>
 __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_group_norm_kernel(const MmGroup g, const NormFuse nf) {
     uint32_t bx;
     const uint32_t p = group_problem(g, bx);
-    skinny_kt_mfma_xreg_body<MM, 1, false, false, true, TRIPS>(g.p[p], bx, 0, nullptr, 0, nullptr, &nf);
+    skinny_kt_mfma_xreg_body<WHOLE, MM, 1, false, false, true, TRIPS>(g.p[p], bx, 0, nullptr, 0, nullptr, &nf);
 }
 
 // The grouped products of an attention block's decode step (q, k, v: a few rows, the same left operand) with the
@@ -1538,7 +1537,7 @@ struct RopeGroup {
     RopeStore s[kMaxGroup];
 };
 template <bool WHOLE, int MM, bool NORM, int TRIPS>
-__device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGroup &g, const RopeGroup &rg, const NormFuse &nf) {
+__global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_group_rope_kernel(const MmGroup g, const RopeGroup rg, const NormFuse nf) {
     __shared__ float nsum[4][MM];
     uint32_t divisor = 0;
     float pv[2 * MM];
@@ -1662,11 +1661,6 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_group_rope_impl(const MmGrou
         }
         if (threadIdx.x < kOut && col < a.N && m < a.M) rs.dst[(int64_t)m * rs.sb + (int64_t)(col / rs.hd) * rs.sh + col % rs.hd] = v;
     }
-}
-template <int MM, bool NORM, int TRIPS>
-__global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_group_rope_kernel(const MmGroup g, const RopeGroup rg, const NormFuse nf) {
-    if (g.p[0].K % (TRIPS * 256) == 0) skinny_kt_mfma_xreg_group_rope_impl<true, MM, NORM, TRIPS>(g, rg, nf); // (the problems of a group share k)
-    else skinny_kt_mfma_xreg_group_rope_impl<false, MM, NORM, TRIPS>(g, rg, nf);
 }
 
 // The store above for products whose heads go through an RMS norm of their own first (RopeStore::hgamma, the q / k norm of
@@ -1843,14 +1837,12 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs
         }
     }
 }
-template <int MM, bool NORM, int TRIPS>
+template <bool WHOLE, int MM, bool NORM, int TRIPS>
 __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_cols_gated_kernel(const MmArgs a, const uint32_t *second, uint32_t one,
                                                                                   uint32_t iters, const NormFuse nf) {
-    if (a.K % (TRIPS * 256) == 0) skinny_kt_mfma_xreg_cols_gated_impl<true, MM, NORM, TRIPS, TRIPS>(a, second, one, iters, nf);
-    else
-        xreg_chunk<TRIPS, false>(a.K, [&](auto trips) __attribute__((always_inline)) {
-            skinny_kt_mfma_xreg_cols_gated_impl<false, MM, NORM, TRIPS, decltype(trips)::value>(a, second, one, iters, nf);
-        });
+    xreg_chunk<TRIPS, WHOLE>(a.K, [&](auto trips) __attribute__((always_inline)) {
+        skinny_kt_mfma_xreg_cols_gated_impl<WHOLE, MM, NORM, TRIPS, decltype(trips)::value>(a, second, one, iters, nf);
+    });
 }
 
 // Vectorised skinny kernel for short K (K <= 4*LPC, e.g. q.K^T of a decode step with
@@ -2159,21 +2151,24 @@ int launch_matmul_group(cg_backend *be, const cg_tensor *x, const cg_tensor *con
     ProfScope prof(be, CG_K_GEMM_SKINNY, bytes);
     const bool eight = g.p[0].M > 4, deep = xreg_trips(g.p[0].K) == 8;
     auto launch = [&](auto kernel, auto... args) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, be->stream, args...); };
-    if (xreg) launch(skinny_kt_mfma_xreg_group_kernel<4, 2, 8>, g);
-    else if (nf && deep && eight) launch(skinny_kt_mfma_xreg_group_norm_kernel<8, 8>, g, *nf);
-    else if (nf && deep) launch(skinny_kt_mfma_xreg_group_norm_kernel<4, 8>, g, *nf);
-    else if (nf && eight) launch(skinny_kt_mfma_xreg_group_norm_kernel<8, 4>, g, *nf);
-    else if (nf) launch(skinny_kt_mfma_xreg_group_norm_kernel<4, 4>, g, *nf);
-    else if (xreg1 && deep && eight) launch(skinny_kt_mfma_xreg_group_kernel<8, 1, 8>, g);
-    else if (xreg1 && deep) launch(skinny_kt_mfma_xreg_group_kernel<4, 1, 8>, g);
-    else if (xreg1 && eight) launch(skinny_kt_mfma_xreg_group_kernel<8, 1, 4>, g);
-    else if (xreg1) launch(skinny_kt_mfma_xreg_group_kernel<4, 1, 4>, g);
-    else if (g.p[0].M <= 1)
-        hipLaunchKernelGGL((skinny_kt_wide_group_kernel<1>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
-    else if (g.p[0].M <= 4)
-        hipLaunchKernelGGL((skinny_kt_wide_group_kernel<4>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
-    else
-        hipLaunchKernelGGL((skinny_kt_wide_group_kernel<8>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
+    xreg_either(g.p[0].K, xreg ? 8 : xreg_trips(g.p[0].K), [&](auto whole) { // (the problems of a group share k)
+        constexpr bool W = decltype(whole)::value;
+        if (xreg) launch(skinny_kt_mfma_xreg_group_kernel<W, 4, 2, 8>, g);
+        else if (nf && deep && eight) launch(skinny_kt_mfma_xreg_group_norm_kernel<W, 8, 8>, g, *nf);
+        else if (nf && deep) launch(skinny_kt_mfma_xreg_group_norm_kernel<W, 4, 8>, g, *nf);
+        else if (nf && eight) launch(skinny_kt_mfma_xreg_group_norm_kernel<W, 8, 4>, g, *nf);
+        else if (nf) launch(skinny_kt_mfma_xreg_group_norm_kernel<W, 4, 4>, g, *nf);
+        else if (xreg1 && deep && eight) launch(skinny_kt_mfma_xreg_group_kernel<W, 8, 1, 8>, g);
+        else if (xreg1 && deep) launch(skinny_kt_mfma_xreg_group_kernel<W, 4, 1, 8>, g);
+        else if (xreg1 && eight) launch(skinny_kt_mfma_xreg_group_kernel<W, 8, 1, 4>, g);
+        else if (xreg1) launch(skinny_kt_mfma_xreg_group_kernel<W, 4, 1, 4>, g);
+        else if (g.p[0].M <= 1)
+            hipLaunchKernelGGL((skinny_kt_wide_group_kernel<1>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
+        else if (g.p[0].M <= 4)
+            hipLaunchKernelGGL((skinny_kt_wide_group_kernel<4>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
+        else
+            hipLaunchKernelGGL((skinny_kt_wide_group_kernel<8>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
+    });
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "grouped matmul launch");
 }
@@ -2244,17 +2239,20 @@ int launch_matmul_group_rope(cg_backend *be, const cg_tensor *x, const cg_tensor
         finish_heads = heads;
     }
     auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, be->stream, g, rg, nf ? *nf : none); };
-    if (g.p[0].M > 4) {
-        if (nf && wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<8, true, 8>);
-        else if (nf) launch(skinny_kt_mfma_xreg_group_rope_kernel<8, true, 4>);
-        else if (wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<8, false, 8>);
-        else launch(skinny_kt_mfma_xreg_group_rope_kernel<8, false, 4>);
-    } else {
-        if (nf && wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<4, true, 8>);
-        else if (nf) launch(skinny_kt_mfma_xreg_group_rope_kernel<4, true, 4>);
-        else if (wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<4, false, 8>);
-        else launch(skinny_kt_mfma_xreg_group_rope_kernel<4, false, 4>);
-    }
+    xreg_either(g.p[0].K, xreg_trips(g.p[0].K), [&](auto whole) { // (the problems of a group share k)
+        constexpr bool W = decltype(whole)::value;
+        if (g.p[0].M > 4) {
+            if (nf && wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 8, true, 8>);
+            else if (nf) launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 8, true, 4>);
+            else if (wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 8, false, 8>);
+            else launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 8, false, 4>);
+        } else {
+            if (nf && wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 4, true, 8>);
+            else if (nf) launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 4, true, 4>);
+            else if (wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 4, false, 8>);
+            else launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 4, false, 4>);
+        }
+    });
     if (by_head) {
         const uint32_t threads = (hf.M * 128 + 63) / 64 * 64;
         hipLaunchKernelGGL(head_norm_rope_finish_kernel, dim3(finish_heads), dim3(threads), 0, be->stream, hf);
@@ -2294,26 +2292,32 @@ int launch_matmul_gated(cg_backend *be, const cg_tensor *x, const cg_tensor *yg,
         const uint32_t groups = (ag.N + 3) / 4, iters = xreg_cols_iters(groups);
         const dim3 cgrid((groups + iters - 1) / iters);
         auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, cgrid, dim3(kThreads), 0, be->stream, ag, au.B, one, iters, nf ? *nf : none); };
-        if (eight) {
-            if (short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<8, true, 4>);
-            else launch(skinny_kt_mfma_xreg_cols_gated_kernel<8, true, 8>);
-        } else {
-            if (nf && short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<4, true, 4>);
-            else if (nf) launch(skinny_kt_mfma_xreg_cols_gated_kernel<4, true, 8>);
-            else if (short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<4, false, 4>);
-            else launch(skinny_kt_mfma_xreg_cols_gated_kernel<4, false, 8>);
-        }
+        xreg_either(ag.K, xreg_trips(ag.K), [&](auto whole) {
+            constexpr bool W = decltype(whole)::value;
+            if (eight) {
+                if (short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<W, 8, true, 4>);
+                else launch(skinny_kt_mfma_xreg_cols_gated_kernel<W, 8, true, 8>);
+            } else {
+                if (nf && short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<W, 4, true, 4>);
+                else if (nf) launch(skinny_kt_mfma_xreg_cols_gated_kernel<W, 4, true, 8>);
+                else if (short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<W, 4, false, 4>);
+                else launch(skinny_kt_mfma_xreg_cols_gated_kernel<W, 4, false, 8>);
+            }
+        });
     } else {
         auto launch = [&](auto kernel, auto... more) { hipLaunchKernelGGL(kernel, ggrid, dim3(kThreads), 0, be->stream, ag, au.B, one, more...); };
-        if (eight) {
-            if (short_chunks) launch(skinny_kt_mfma_xreg_gated_norm_kernel<8, 4>, *nf);
-            else launch(skinny_kt_mfma_xreg_gated_norm_kernel<8, 8>, *nf);
-        } else {
-            if (nf && short_chunks) launch(skinny_kt_mfma_xreg_gated_norm_kernel<4, 4>, *nf);
-            else if (nf) launch(skinny_kt_mfma_xreg_gated_norm_kernel<4, 8>, *nf);
-            else if (short_chunks) launch(skinny_kt_mfma_xreg_gated_kernel<4, 4>);
-            else launch(skinny_kt_mfma_xreg_gated_kernel<4, 8>);
-        }
+        xreg_either(ag.K, xreg_trips(ag.K), [&](auto whole) {
+            constexpr bool W = decltype(whole)::value;
+            if (eight) {
+                if (short_chunks) launch(skinny_kt_mfma_xreg_gated_norm_kernel<W, 8, 4>, *nf);
+                else launch(skinny_kt_mfma_xreg_gated_norm_kernel<W, 8, 8>, *nf);
+            } else {
+                if (nf && short_chunks) launch(skinny_kt_mfma_xreg_gated_norm_kernel<W, 4, 4>, *nf);
+                else if (nf) launch(skinny_kt_mfma_xreg_gated_norm_kernel<W, 4, 8>, *nf);
+                else if (short_chunks) launch(skinny_kt_mfma_xreg_gated_kernel<W, 4, 4>);
+                else launch(skinny_kt_mfma_xreg_gated_kernel<W, 4, 8>);
+            }
+        });
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "gated matmul launch");
@@ -2365,10 +2369,13 @@ int launch_matmul_residual(cg_backend *be, const cg_tensor *x, const cg_tensor *
     else if (eight == 4) launch8(skinny_kt_mfma_eight_residual_kernel<4, 4>);
     else if (xreg_narrow(a.M, a.K)) {
         const bool deep = xreg_trips(a.K) == 8;
-        if (deep && rows8) launch(skinny_kt_mfma_xreg_residual_kernel<8, 8>);
-        else if (deep) launch(skinny_kt_mfma_xreg_residual_kernel<4, 8>);
-        else if (rows8) launch(skinny_kt_mfma_xreg_residual_kernel<8, 4>);
-        else launch(skinny_kt_mfma_xreg_residual_kernel<4, 4>);
+        xreg_either(a.K, xreg_trips(a.K), [&](auto whole) {
+            constexpr bool W = decltype(whole)::value;
+            if (deep && rows8) launch(skinny_kt_mfma_xreg_residual_kernel<W, 8, 8>);
+            else if (deep) launch(skinny_kt_mfma_xreg_residual_kernel<W, 4, 8>);
+            else if (rows8) launch(skinny_kt_mfma_xreg_residual_kernel<W, 8, 4>);
+            else launch(skinny_kt_mfma_xreg_residual_kernel<W, 4, 4>);
+        });
     } else if (a.M <= 1)
         hipLaunchKernelGGL((skinny_kt_wide_residual_kernel<1>), grid, dim3(kThreads), 0, be->stream, a, r);
     else if (a.M <= 4)
@@ -2771,20 +2778,26 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
 #undef CG_CALL
             } else if (cols >= 4096 && M <= 4) { // the wider projections of a decode step: activations are fetched once per 8 columns
                 dim3 grid((uint32_t)((N + 7) / 8), (uint32_t)batch);
-                if (xreg_trips((uint32_t)K) == 4)
-                    hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<4, 2, 4>), grid, dim3(kThreads), 0, s, a);
-                else
-                    hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<4, 2, 8>), grid, dim3(kThreads), 0, s, a);
+                xreg_either((uint32_t)K, xreg_trips((uint32_t)K), [&](auto whole) {
+                    constexpr bool W = decltype(whole)::value;
+                    if (xreg_trips((uint32_t)K) == 4)
+                        hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<W, 4, 2, 4>), grid, dim3(kThreads), 0, s, a);
+                    else
+                        hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<W, 4, 2, 8>), grid, dim3(kThreads), 0, s, a);
+                });
             } else if (cols >= 2048 && xreg_narrow((uint32_t)M, (uint32_t)K)) {
                 dim3 grid((uint32_t)((N + 3) / 4), (uint32_t)batch);
-                if (M > 4 && xreg_trips((uint32_t)K) == 4)
-                    hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<8, 1, 4>), grid, dim3(kThreads), 0, s, a);
-                else if (M > 4)
-                    hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<8, 1, 8>), grid, dim3(kThreads), 0, s, a);
-                else if (xreg_trips((uint32_t)K) == 4)
-                    hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<4, 1, 4>), grid, dim3(kThreads), 0, s, a);
-                else
-                    hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<4, 1, 8>), grid, dim3(kThreads), 0, s, a);
+                xreg_either((uint32_t)K, xreg_trips((uint32_t)K), [&](auto whole) {
+                    constexpr bool W = decltype(whole)::value;
+                    if (M > 4 && xreg_trips((uint32_t)K) == 4)
+                        hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<W, 8, 1, 4>), grid, dim3(kThreads), 0, s, a);
+                    else if (M > 4)
+                        hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<W, 8, 1, 8>), grid, dim3(kThreads), 0, s, a);
+                    else if (xreg_trips((uint32_t)K) == 4)
+                        hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<W, 4, 1, 4>), grid, dim3(kThreads), 0, s, a);
+                    else
+                        hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<W, 4, 1, 8>), grid, dim3(kThreads), 0, s, a);
+                });
             } else if (cols >= 2048) {
                 dim3 grid((uint32_t)((N + 3) / 4), (uint32_t)batch);
 #define CG_CALL(MMV) hipLaunchKernelGGL((skinny_kt_wide_kernel<MMV, 1, false>), grid, dim3(kThreads), 0, s, a);
