@@ -556,7 +556,9 @@ bool rows_program_compiled(const Pending &p);
 bool rows_max_program_begun(const Pending &p);
 int launch_arange(cg_backend *be, cg_tensor *out);
 // Copies n <= kReadbackWords words to be->rb_dev and then stores `seq` at word kReadbackWords of it, visible to the host.
-// (64 KiB: the runtime's staged copy and its wake-up cost 20 us more than the kernel's stores over the bus)
+// (64 KiB.  The runtime's copy, us, and this one: behind a kernel 4096 words 30 and 23, 16384 33 and 27.  Behind a polled read-back, as of a step's
+// tokens, the runtime first retires all kernels in front of it: 6000 words 100 us more than here.  Only with nothing left to retire is its copy of
+// more than 16 KiB the faster one: 8192 words 13 and 17.)
 constexpr uint32_t kReadbackWords = 16384;
 int launch_small_readback(cg_backend *be, const uint32_t *src, uint32_t n, uint32_t seq);
 // A few words from the host travel with the launch, as kernel arguments: n <= kUploadWords words to dst.
