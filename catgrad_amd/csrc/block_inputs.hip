@@ -34,31 +34,37 @@ __global__ __launch_bounds__(kThreads) void pair_embedding_kernel(const PairEmbe
     for (uint32_t k = threadIdx.x; k < p.width; k += kThreads) p.out[(int64_t)r * p.width + k] = element(p.table, a + k) + element(p.pairs, c + k);
 }
 
-typedef const __attribute__((address_space(1))) float global_float;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-// A pointer that the compiler knows nothing of but its registers: what is chosen among such pointers is chosen, not branched for.
-__device__ __forceinline__ global_float *pinned(const float *p) {
-    int64_t v = reinterpret_cast<int64_t>(p);
-    asm volatile("" : "+s"(v));
-    return reinterpret_cast<global_float *>(v);
-}
 // ---- grouped norm and filter -----------------------------------------------------------------------------------------
+// h to the columns from o on of an output
+template <int VW> __device__ __forceinline__ void put_filtered(const ConvRowsPlan::Out &out, int64_t o, float (&h)[VW]) {
+    if (out.fmt == kFmtBF16) {
+        uint16_t *d = static_cast<uint16_t *>(out.dst) + o;
+        if constexpr (VW == 4)
+            *reinterpret_cast<uint2 *>(d) =
+                make_uint2((round_bf16(h[0]) >> 16) | (round_bf16(h[1]) & 0xFFFF0000u), (round_bf16(h[2]) >> 16) | (round_bf16(h[3]) & 0xFFFF0000u));
+        else *d = (uint16_t)(round_bf16(h[0]) >> 16);
+    } else {
+        float *d = static_cast<float *>(out.dst) + o;
+        if (out.round) {
+#pragma unroll
+            for (int j = 0; j < VW; j++) h[j] = asf(round_bf16(h[j]) & 0xFFFF0000u);
+        }
+        if constexpr (VW == 4) *reinterpret_cast<float4 *>(d) = make_float4(h[0], h[1], h[2], h[3]);
+        else *d = h[0];
+    }
+}
 // A workgroup takes `run` tokens of a sequence and `cols` columns of a group (blockIdx.y: group and part of it): the scales of
 // these tokens' rows and of the taps - 1 before them (a wave per row, four rows' pieces in flight), then, with a thread per VW
 // columns, the filter along the tokens; what the filter looks back on stays in registers.  TAPS: at most so many.
-// FEW: few tokens, four taps in four columns a thread: the taps and what the filter reads are asked for before the scales are known.
-// One new token of 1024 columns in 4 groups was six trips to memory one behind the other: 6.1 us, 5.4 so; where the device is full the
-// registers cost more than the wait (2048 tokens of 1024 columns: 21.8 us without, 23.7 with).
-template <int VW, int TAPS, bool FEW = false> __global__ __launch_bounds__(kThreads) void conv_rows_kernel(const ConvRowsPlan p, const uint32_t parts) {
+template <int VW, int TAPS> __global__ __launch_bounds__(kThreads) void conv_rows_kernel(const ConvRowsPlan p, const uint32_t parts) {
     extern __shared__ float scale[]; // [run + taps - 1]
-    const uint32_t past = FEW ? 3 : p.taps - 1, size = p.width / p.groups, group = blockIdx.y / parts, part = blockIdx.y - group * parts, g0 = group * size;
+    const uint32_t past = p.taps - 1, size = p.width / p.groups, group = blockIdx.y / parts, part = blockIdx.y - group * parts, g0 = group * size;
     const uint32_t runs = (p.S + p.run - 1) / p.run, b = blockIdx.x / runs, s0 = (blockIdx.x - b * runs) * p.run, n = min(p.run, p.S - s0);
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    auto load = [&](global_float *q, float(&v)[VW]) {
+    auto load = [&](const float *q, float(&v)[VW]) {
         if constexpr (VW == 4) {
-            const f32x4 t = *reinterpret_cast<const __attribute__((address_space(1))) f32x4 *>(q);
-#pragma unroll
-            for (int j = 0; j < VW; j++) v[j] = t[j];
+            const float4 t = *reinterpret_cast<const float4 *>(q);
+            v[0] = t.x, v[1] = t.y, v[2] = t.z, v[3] = t.w;
         } else {
             v[0] = *q;
         }
@@ -69,66 +75,26 @@ template <int VW, int TAPS, bool FEW = false> __global__ __launch_bounds__(kThre
     const uint32_t across = min(kThreads, ((per + VW - 1) / VW + 63) / 64 * 64), subs = kThreads / across, sub = threadIdx.x / across;
     const uint32_t sub_run = (n + subs - 1) / subs, i_first = min(n, sub * sub_run), i_end = min(n, i_first + sub_run);
     const uint32_t c_first = g0 + part * per + (threadIdx.x - sub * across) * VW;
-    // tap t counts from the present back; a second output that is not there reads the first's, a filter that is not there its gains
-    float gamma[2][VW], w[2][TAPS][VW];
-    const bool second = p.n > 1, filtered[2] = {p.out[0].conv != nullptr, second && p.out[1].conv != nullptr};
-    global_float *const gains[2] = {pinned(p.out[0].gamma), pinned(second ? p.out[1].gamma : p.out[0].gamma)};
-    global_float *const taps[2] = {pinned(filtered[0] ? p.out[0].conv : p.out[0].gamma), pinned(filtered[1] ? p.out[1].conv : p.out[0].gamma)};
-    global_float *const inputs = pinned(p.x.p), *const state = pinned(p.state ? p.state : p.x.p);
-    const bool has_state = p.state != nullptr;
+    float gamma[2][VW], w[2][TAPS][VW]; // tap t counts from the present back
     auto ask_filters = [&](uint32_t at) {
         at = min(at, p.width - VW);
 #pragma unroll
         for (int f = 0; f < 2; f++) {
-            load(gains[f] + at, gamma[f]);
-            if constexpr (FEW) {
+            if (f >= p.n) break;
+            load(p.out[f].gamma + at, gamma[f]);
 #pragma unroll
-                for (int j = 0; j < VW; j++) {
-                    float t[VW];
-                    load(taps[f] + (filtered[f] ? (int64_t)(at + j) * 4 : 0), t);
+            for (int j = 0; j < VW; j++) {
+                if (TAPS == 4 && VW == 4 && p.taps == 4 && p.out[f].conv) {
+                    const float4 t = *reinterpret_cast<const float4 *>(p.out[f].conv + (int64_t)(at + j) * 4);
+                    w[f][0][j] = t.w, w[f][1 % TAPS][j] = t.z, w[f][2 % TAPS][j] = t.y, w[f][3 % TAPS][j] = t.x;
+                } else {
 #pragma unroll
-                    for (int k = 0; k < VW; k++) w[f][TAPS - 1 - k][j] = t[k];
-                }
-            } else if (f < p.n) {
-#pragma unroll
-                for (int j = 0; j < VW; j++) {
-                    if (TAPS == 4 && VW == 4 && p.taps == 4 && p.out[f].conv) {
-                        const float4 t = *reinterpret_cast<const float4 *>(p.out[f].conv + (int64_t)(at + j) * 4);
-                        w[f][0][j] = t.w, w[f][1 % TAPS][j] = t.z, w[f][2 % TAPS][j] = t.y, w[f][3 % TAPS][j] = t.x;
-                    } else {
-#pragma unroll
-                        for (int t = 0; t < TAPS; t++) w[f][t][j] = p.out[f].conv && t < (int)p.taps ? p.out[f].conv[(int64_t)(at + j) * p.taps + (p.taps - 1 - t)] : 0.0f;
-                    }
+                    for (int t = 0; t < TAPS; t++) w[f][t][j] = p.out[f].conv && t < (int)p.taps ? p.out[f].conv[(int64_t)(at + j) * p.taps + (p.taps - 1 - t)] : 0.0f;
                 }
             }
         }
     };
-    // What the filter reads: z of token s0 - past + i, for the tokens in front of the sequence's new ones from its state.
-    constexpr int AHEAD = 4; // rows asked for together
-    float z[TAPS][VW], next[AHEAD][VW]; // z: the input t tokens back
-    auto ask_row = [&](uint32_t i, uint32_t at, float(&v)[VW]) {
-        const int32_t s = (int32_t)(s0 + i) - (int32_t)past;
-        const bool fresh = s >= 0 || !has_state;
-        const int64_t row = fresh ? (int64_t)b * p.S + max(s, 0) : (int64_t)b * past + (past + s);
-        global_float *const q = (fresh ? inputs : state) + row * (fresh ? p.x.pitch : (int64_t)p.width) + min(at, p.width - VW);
-        load(q, v);
-    };
-    auto ask_rows = [&](uint32_t i0, uint32_t at) {
-#pragma unroll
-        for (int e = 0; e < AHEAD; e++) ask_row(past + min(i0 + e, i_end - 1), at, next[e]);
-    };
-    auto ask_inputs = [&](uint32_t at) {
-#pragma unroll
-        for (int t = 0; t < TAPS; t++)
-#pragma unroll
-            for (int j = 0; j < VW; j++) z[t][j] = 0.0f;
-#pragma unroll
-        for (int t = TAPS - 1; t >= 1; t--)
-            if (t <= (int)past) ask_row(past + i_first - t, at, z[t - 1]); // (moved one back below)
-        ask_rows(i_first, at);
-    };
     ask_filters(c_first);
-    if constexpr (FEW) ask_inputs(c_first);
     constexpr int ROWS = 4; // of a wave at a time
     for (uint32_t i0 = wave; i0 < n + past; i0 += kWaves * ROWS) {
         float m[ROWS] = {};
@@ -137,7 +103,7 @@ template <int VW, int TAPS, bool FEW = false> __global__ __launch_bounds__(kThre
 #pragma unroll
             for (int e = 0; e < ROWS; e++) { // (clamped: rows that are not there are not stored)
                 const int32_t s = (int32_t)(s0 + min(i0 + e * kWaves, n + past - 1)) - (int32_t)past;
-                load(inputs + ((int64_t)b * p.S + max(s, 0)) * p.x.pitch + g0 + k, v[e]);
+                load(p.x.p + ((int64_t)b * p.S + max(s, 0)) * p.x.pitch + g0 + k, v[e]);
             }
 #pragma unroll
             for (int e = 0; e < ROWS; e++)
@@ -155,12 +121,19 @@ template <int VW, int TAPS, bool FEW = false> __global__ __launch_bounds__(kThre
     if (sub >= subs || i_first == i_end) return;
     for (uint32_t c = c_first; c < c_end; c += across * VW) {
         if (c != c_first) ask_filters(c);
-        if (!FEW || c != c_first) ask_inputs(c);
-        auto scaled = [&](uint32_t i, float(&v)[VW]) {
-            const bool fresh = (int32_t)(s0 + i) - (int32_t)past >= 0;
-            const float f = fresh ? scale[i] : 1.0f;
+        // z of token s0 - past + i, for the tokens in front of the sequence's new ones from its state
+        auto unit = [&](uint32_t i, float(&v)[VW]) {
+            const int32_t s = (int32_t)(s0 + i) - (int32_t)past;
+            if (s >= 0) {
+                load(p.x.p + ((int64_t)b * p.S + s) * p.x.pitch + c, v);
 #pragma unroll
-            for (int j = 0; j < VW; j++) v[j] = fresh ? v[j] * f : has_state ? v[j] : 0.0f;
+                for (int j = 0; j < VW; j++) v[j] *= scale[i];
+            } else if (p.state) {
+                load(p.state + ((int64_t)b * past + (past + s)) * p.width + c, v);
+            } else {
+#pragma unroll
+                for (int j = 0; j < VW; j++) v[j] = 0.0f;
+            }
         };
         // the inputs behind the sequence's end become its state
         auto keep = [&](int32_t s, const float(&v)[VW]) {
@@ -170,17 +143,23 @@ template <int VW, int TAPS, bool FEW = false> __global__ __launch_bounds__(kThre
             if constexpr (VW == 4) *reinterpret_cast<float4 *>(o) = make_float4(v[0], v[1], v[2], v[3]);
             else *o = v[0];
         };
+        float z[TAPS][VW]; // the input t tokens back
+#pragma unroll
+        for (int t = 0; t < TAPS; t++)
+#pragma unroll
+            for (int j = 0; j < VW; j++) z[t][j] = 0.0f;
 #pragma unroll
         for (int t = TAPS - 1; t >= 1; t--)
             if (t <= (int)past) {
                 const int32_t s = (int32_t)(s0 + i_first) - t;
-                scaled(past + i_first - t, z[t - 1]);
+                unit(past + i_first - t, z[t - 1]); // (moved one back below)
                 if (s0 + i_end == p.S && s < 0) keep(s, z[t - 1]);
             }
+        constexpr int AHEAD = 4; // rows asked for together
         for (uint32_t i0 = i_first; i0 < i_end; i0 += AHEAD) {
-            if (i0 != i_first) ask_rows(i0, c);
+            float next[AHEAD][VW];
 #pragma unroll
-            for (int e = 0; e < AHEAD; e++) scaled(past + min(i0 + e, i_end - 1), next[e]);
+            for (int e = 0; e < AHEAD; e++) unit(past + min(i0 + e, i_end - 1), next[e]);
 #pragma unroll
             for (int e = 0; e < AHEAD; e++) {
                 const uint32_t s = s0 + i0 + e;
@@ -201,26 +180,99 @@ template <int VW, int TAPS, bool FEW = false> __global__ __launch_bounds__(kThre
                     for (int j = 0; j < VW; j++) {
                         float a = 0.0f;
 #pragma unroll
-                        for (int t = TAPS - 1; t >= 0; t--) a = fmaf(!FEW || filtered[f] ? w[f][t][j] : 0.0f, z[t][j], a);
+                        for (int t = TAPS - 1; t >= 0; t--) a = fmaf(w[f][t][j], z[t][j], a);
                         h[j] = (a + z[0][j]) * gamma[f][j];
                     }
-                    if (p.out[f].fmt == kFmtBF16) {
-                        uint16_t *d = static_cast<uint16_t *>(p.out[f].dst) + o;
-                        if constexpr (VW == 4)
-                            *reinterpret_cast<uint2 *>(d) =
-                                make_uint2((round_bf16(h[0]) >> 16) | (round_bf16(h[1]) & 0xFFFF0000u), (round_bf16(h[2]) >> 16) | (round_bf16(h[3]) & 0xFFFF0000u));
-                        else *d = (uint16_t)(round_bf16(h[0]) >> 16);
-                    } else {
-                        float *d = static_cast<float *>(p.out[f].dst) + o;
-                        if (p.out[f].round) {
-#pragma unroll
-                            for (int j = 0; j < VW; j++) h[j] = asf(round_bf16(h[j]) & 0xFFFF0000u);
-                        }
-                        if constexpr (VW == 4) *reinterpret_cast<float4 *>(d) = make_float4(h[0], h[1], h[2], h[3]);
-                        else *d = h[0];
-                    }
+                    put_filtered<VW>(p.out[f], o, h);
                 }
             }
+        }
+    }
+}
+
+// The same for a token a workgroup, four taps (in 16 bytes) and four columns a thread: the taps and what the filter reads are asked for before the
+// scales are known, where the kernel above makes six trips to memory one behind the other.  us above and here, with its timing: a token of 1024
+// columns in 4 groups 7.7 and 6.7, 256 of them 10.3 and 8.7, 500 of 2048 columns in 8 groups 21.0 and 17.5, a token of 4096 columns 10.2 and 8.0.
+typedef const __attribute__((address_space(1))) float global_float;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+// A pointer that the compiler knows nothing of but its registers: what is chosen among such pointers is chosen, not branched for.
+__device__ __forceinline__ global_float *pinned(const float *p) {
+    int64_t v = reinterpret_cast<int64_t>(p);
+    asm volatile("" : "+s"(v));
+    return reinterpret_cast<global_float *>(v);
+}
+__global__ __launch_bounds__(kThreads) void conv_token_kernel(const ConvRowsPlan p, const uint32_t parts) {
+    constexpr int TAPS = 4, PAST = TAPS - 1;
+    static_assert(kWaves == TAPS, "a wave per row that a token looks at");
+    __shared__ float scale[TAPS];
+    const uint32_t size = p.width / p.groups, group = blockIdx.y / parts, part = blockIdx.y - group * parts, g0 = group * size;
+    const uint32_t b = blockIdx.x / p.S, s = blockIdx.x - b * p.S, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint32_t per = ((size + parts - 1) / parts + 3) / 4 * 4, c_end = g0 + min(size, (part + 1) * per), c_first = g0 + part * per + threadIdx.x * 4;
+    // a second output that is not there reads the first's, a state that is not there the inputs
+    const bool second = p.n > 1, has_state = p.state != nullptr;
+    global_float *const gains[2] = {pinned(p.out[0].gamma), pinned(p.out[second].gamma)}, *const taps[2] = {pinned(p.out[0].conv), pinned(p.out[second].conv)};
+    global_float *const inputs = pinned(p.x.p), *const state = pinned(has_state ? p.state : p.x.p);
+    auto load = [&](global_float *q) { return *reinterpret_cast<const __attribute__((address_space(1))) f32x4 *>(q); };
+    f32x4 gamma[2], w[2][4], z[TAPS]; // w: a column's taps, the oldest first; z: the input t tokens back
+    auto ask = [&](uint32_t c) {
+        const uint32_t at = min(c, p.width - 4);
+#pragma unroll
+        for (int f = 0; f < 2; f++) {
+            gamma[f] = load(gains[f] + at);
+#pragma unroll
+            for (int j = 0; j < 4; j++) w[f][j] = load(taps[f] + (int64_t)(at + j) * TAPS);
+        }
+#pragma unroll
+        for (int t = 0; t < TAPS; t++) {
+            const int32_t from = (int32_t)s - t;
+            const bool fresh = from >= 0 || !has_state;
+            const int64_t row = fresh ? (int64_t)b * p.S + max(from, 0) : (int64_t)b * PAST + (PAST + from);
+            z[t] = load((fresh ? inputs : state) + row * (fresh ? p.x.pitch : (int64_t)p.width) + at);
+        }
+    };
+    ask(c_first);
+    float m = 0.0f;
+    const int32_t mine = (int32_t)s - PAST + (int32_t)wave; // (the token whose scale this wave takes)
+    for (uint32_t k = lane * 4; k < size; k += 64 * 4) {
+        const f32x4 v = load(inputs + ((int64_t)b * p.S + max(mine, 0)) * p.x.pitch + g0 + k);
+#pragma unroll
+        for (int j = 0; j < 4; j++) m = fmaf(v[j], v[j], m);
+    }
+    const float sum = wave_total(m);
+    if (lane == 0) scale[wave] = 1.0f / sqrtf(sum / (float)size + p.eps);
+    __syncthreads();
+    for (uint32_t c = c_first; c < c_end; c += kThreads * 4) {
+        if (c != c_first) ask(c);
+#pragma unroll
+        for (int t = 0; t < TAPS; t++) {
+            const bool fresh = (int32_t)s - t >= 0;
+            const float f = fresh ? scale[PAST - t] : 1.0f;
+#pragma unroll
+            for (int j = 0; j < 4; j++) z[t][j] = fresh ? z[t][j] * f : has_state ? z[t][j] : 0.0f;
+        }
+        // the inputs behind the sequence's end become its state; the last token keeps what it saw of the old one
+        auto keep = [&](int32_t from, const f32x4 &v) {
+            const int32_t at = from - ((int32_t)p.S - PAST);
+            if (at >= 0) *reinterpret_cast<f32x4 *>(p.state_out + ((int64_t)b * PAST + at) * p.width + c) = v;
+        };
+        keep((int32_t)s, z[0]);
+        if (s + 1 == p.S) {
+#pragma unroll
+            for (int t = 1; t < TAPS; t++)
+                if ((int32_t)s - t < 0) keep((int32_t)s - t, z[t]);
+        }
+#pragma unroll
+        for (int f = 0; f < 2; f++) {
+            if (f >= p.n) break;
+            float h[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                float a = 0.0f;
+#pragma unroll
+                for (int t = PAST; t >= 0; t--) a = fmaf(w[f][j][PAST - t], z[t][j], a);
+                h[j] = (a + z[0][j]) * gamma[f][j];
+            }
+            put_filtered<4>(p.out[f], ((int64_t)b * p.S + s) * p.width + c, h);
         }
     }
 }
@@ -379,7 +431,9 @@ int launch_conv_rows(cg_backend *be, ConvRowsPlan p) {
     while (cols / (split * 2) >= 128 && (uint64_t)p.B * p.S * p.groups * split * 2 <= be->compute_units) split *= 2;
     double bytes = 4.0;
     bool vec = cols % 4 == 0 && p.x.pitch % 4 == 0 && aligned16(p.x.p) && aligned16(p.state) && aligned16(p.state_out);
+    bool taps = true; // every output has a filter
     for (int f = 0; f < p.n; f++) {
+        taps = taps && p.out[f].conv;
         bytes += p.out[f].fmt == kFmtBF16 ? 2.0 : 4.0;
         vec = vec && aligned16(p.out[f].dst) && aligned16(p.out[f].gamma) && aligned16(p.out[f].conv);
     }
@@ -394,7 +448,8 @@ int launch_conv_rows(cg_backend *be, ConvRowsPlan p) {
     if (p.taps <= 1) { CG_CONV(1); }
     else if (p.taps <= 2) { CG_CONV(2); }
     else if (p.taps <= 3) { CG_CONV(3); }
-    else if (p.taps == 4 && vec && p.run == 1) hipLaunchKernelGGL((conv_rows_kernel<4, 4, true>), grid, dim3(kThreads), lds, s, p, split); // (the device is not full)
+    else if (p.taps == 4 && vec && p.run == 1 && taps)
+        hipLaunchKernelGGL(conv_token_kernel, grid, dim3(kThreads), 0, s, p, split);
     else if (p.taps <= 4) { CG_CONV(4); }
     else if (p.taps <= 8) { CG_CONV(8); }
     else if (p.taps <= kMaxTaps) { CG_CONV(kMaxTaps); }

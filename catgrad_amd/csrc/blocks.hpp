@@ -102,7 +102,7 @@ struct ConvRowsPlan {
     const float *state; // null: zeros
     float *state_out;   // null with one tap
     int n;
-    struct {
+    struct Out {
         const float *gamma, *conv; // conv null: the norm alone
         void *dst;
         int fmt;    // words or bfloat16 patterns

@@ -388,6 +388,9 @@ DELTA = {  # name: (options, batch, taps, ranks, portions, dt_bias around)
     "one_head": (delta_options(1, 1, 40, 20), 2, 4, (16, 4), [33, 5], -3.0),
     "shared_keys": (delta_options(6, 2, 24, 48), 1, 4, (16, 16), [31, 1, 18], -3.0),
     "wide": (delta_options(2, 2, 128, 128), 1, 4, (64, 64), [70, 1, 16, 15, 1], -3.0),
+    "ranks_of_128": (delta_options(2, 1, 128, 128), 1, 4, (128, 128), [20, 1, 2, 1, 1], -3.0),
+    "ranks_of_124_and_4": (delta_options(2, 2, 100, 96), 2, 4, (124, 4), [3, 1, 1, 17, 1], -3.0),
+    "ranks_of_132": (delta_options(2, 2, 128, 128), 1, 4, (132, 128), [2, 1, 1], -3.0),
     "widest": (delta_options(1, 1, 256, 64), 1, 4, (16, 16), [40, 1, 3], -3.0),
     "chunk_edges": (delta_options(2, 1, 64, 80), 2, 4, (8, 8), [16, 15, 17, 32, 1, 31, 9, 12], -3.0),
     "fast_decay": (delta_options(2, 2, 32, 32), 1, 4, (8, 8), [60, 1, 20], 6.0),
@@ -422,7 +425,10 @@ CONV = [  # batch, portions, width, groups, taps, products, dtype
     (1, [30], 32, 4, 4, 2, "f32"), (2, [1] * 9, 32, 2, 4, 2, "f32"), (1, [2, 1, 2, 3, 9, 1, 40], 48, 3, 4, 2, "f32"), (1, [12, 2, 5], 30, 5, 3, 1, "f32"),
     (1, [12, 1, 5], 64, 1, 1, 2, "f32"), (2, [7, 2, 30], 64, 64, 2, 2, "f32"), (1, [3, 1, 2, 2, 40], 40, 2, 7, 2, "f32"), (1, [1, 1, 2, 40], 24, 2, 16, 1, "f32"),
     (1, [300, 1, 40], 520, 4, 4, 2, "bf16"), (3, [1, 1, 2, 90], 256, 4, 4, 2, "bf16"), (1, [20, 1, 9], 30, 2, 4, 2, "bf16"), (4, [600, 1], 128, 8, 4, 2, "bf16"),
-    (1, [2000], 96, 4, 5, 2, "f32"), (1, [300], 1024, 4, 4, 2, "bf16")]
+    (1, [2000], 96, 4, 5, 2, "f32"), (1, [300], 1024, 4, 4, 2, "bf16"),
+    # four taps on a token's own workgroup and not: one output, columns in parts of a group, more than a workgroup's, around the most workgroups
+    (1, [1, 1, 2, 3, 40], 64, 2, 4, 1, "f32"), (2, [3, 1, 1], 1024, 1, 4, 1, "bf16"), (1, [2, 1, 5], 2304, 2, 4, 2, "f32"), (1, [128, 129, 1], 256, 4, 4, 2, "f32"),
+    (3, [170, 1, 171], 32, 1, 4, 1, "bf16")]
 
 
 def run_conv_linear(be, case, seed=0):
