@@ -282,7 +282,7 @@ __global__ __launch_bounds__(kBlock) void decode_attention_kernel(const AttnArgs
 // kernels, which spread a KV head over many workgroups.
 // PASSES x (1024 / LPT) positions per trip to memory.  LOOP: several trips, the next always asked for before the
 // current one is used (PASSES registers twice); else one trip covers T, the soft-max program's other leaves are
-// asked for before K, and with at most ten passes V right behind K (the registers hold both).
+// asked for right behind K, and with at most ten passes V behind them (the registers hold both).
 // VS = 2: the workgroup computes all scores but only one half of head_dim of the output, so that twice as many compute
 // units pull on V (used when the launch would otherwise leave half of them idle).
 constexpr int kRowBlock = 1024;
@@ -480,10 +480,9 @@ __global__ __launch_bounds__(kRowBlock) void decode_attention_row_kernel(const A
 // segments a launch puts one workgroup on every compute unit, each with T / segments positions: 134 KB of K and V at
 // the 1B shape's T = 2100, in flight at once (PASSES x 1024 / LPT positions per trip, K and V of a trip in 2 x PASSES
 // sixteen-byte loads per lane).  A segment leaves its rows' maximum, sum and un-normalised weighted sum of V, as the
-// chunked kernel does; decode_attention_combine_kernel — or the load of the product that reads the result, see
-// AttnPartials — merges the segments.
+// chunked kernel does; decode_attention_combine_kernel merges the segments.
 // LOOP: several trips, the next always asked for before the current one is used; else one trip covers the segment and
-// the soft-max program's other leaves are asked for before K.  MM: most query rows per KV head (4 or 8).
+// the soft-max program's other leaves are asked for between K and V.  MM: most query rows per KV head (4 or 8).
 constexpr int kSegBlock = 1024;
 constexpr int kSegMaxChunk = 2048; // most positions per workgroup: their scores wait in LDS, MM x 8 KiB
 constexpr size_t seg_lds_bytes(int mm, int hd, uint32_t chunk) {

@@ -20,11 +20,8 @@ namespace {
 constexpr int kThreads = 256, kWaves = 4;
 constexpr uint32_t kSeg = 128; // keys of a segment
 
-__device__ __forceinline__ float wave_sum(float v) {
-    return wave_add<1>(v);
-}
 __device__ __forceinline__ float block_sum(float v, float *red) {
-    v = wave_sum(v);
+    v = wave_add<1>(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
@@ -121,7 +118,7 @@ __global__ __launch_bounds__(kThreads) void attention_turn_kernel(const Attentio
             const float v = value(d);
             m = fmaf(v, v, m);
         }
-        if (p.unit_heads) c /= sqrtf(wave_sum(m) / (float)p.dim + p.eps);
+        if (p.unit_heads) c /= sqrtf(wave_add<1>(m) / (float)p.dim + p.eps);
         for (uint32_t d = lane; d < p.dim; d += 64) dst[d] = (d == lane ? v0 : d == lane + 64 ? v1 : value(d)) * c;
     }
     float *vc = p.values + (int64_t)b * p.kv_heads * p.v_block + (int64_t)(p.cached + s) * p.vdim;
@@ -278,7 +275,7 @@ __global__ __launch_bounds__(kThreads) void attention_scores_kernel(const Attent
         const float a = sc[h * kSeg + lane], c = sc[h * kSeg + 64 + lane];
         float m = fmaxf(a, c);
         m = asf(wave_fold<1>(asu(m), LargerWords{}));
-        const float l = m == -INFINITY ? 0.0f : wave_sum(expf(a - m) + expf(c - m));
+        const float l = m == -INFINITY ? 0.0f : wave_add<1>(expf(a - m) + expf(c - m));
         const int64_t head = (int64_t)blockIdx.z * p.heads + h0 + h;
         float *o = scores + (head * nseg + seg) * kSeg;
         o[lane] = a;

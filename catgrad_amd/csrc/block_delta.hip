@@ -24,9 +24,6 @@ namespace {
 
 constexpr int kThreads = 256, kWaves = 4;
 
-__device__ __forceinline__ float wave_sum(float v) {
-    return wave_add<1>(v);
-}
 // on the hardware's exp2, log2 and reciprocal (about one unit in the last place each)
 __device__ __forceinline__ float sigmoid(float z) { return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.44269504088896341f)); }
 // max(z, 0) + ln(1 + e^-|z|), by its series where 1 + e^-|z| would lose what a slow decay lives on
@@ -40,12 +37,6 @@ __device__ __forceinline__ float softplus(float z) {
 // (PIN: arguments are pinned to scalar registers before a lane chooses among them.  Left to itself the compiler chooses their place in
 // the argument block and has every lane fetch from there, a trip to memory in front of all others: 13.0 us for a
 // token and 11.8 pinned, states of 128 x 128.  In a loop over tokens the registers are worth more: two tokens 21.9 pinned, 19.0 not.)
-typedef const __attribute__((address_space(1))) float global_float;
-__device__ __forceinline__ int64_t pinned(int64_t v) {
-    asm volatile("" : "+s"(v));
-    return v;
-}
-__device__ __forceinline__ global_float *pinned(const float *p) { return reinterpret_cast<global_float *>(pinned(reinterpret_cast<int64_t>(p))); }
 struct Channel {
     global_float *x, *taps;
     int64_t pitch;
@@ -173,7 +164,7 @@ template <int TAPS> __global__ __launch_bounds__(kThreads, 2) void delta_chunk_k
     for (uint32_t u = wave; u < 2 * kChunk; u += kWaves) { // the unit vectors: rows of q, then of k
         float *row = lds + u * pitch, ss = 0.0f;
         for (uint32_t d = lane; d < dp; d += 64) ss = fmaf(row[d], row[d], ss);
-        float f = 1.0f / sqrtf(wave_sum(ss) + 1e-6f);
+        float f = 1.0f / sqrtf(wave_add<1>(ss) + 1e-6f);
         if (u < kChunk) f *= 1.0f / sqrtf((float)D);
         for (uint32_t d = lane; d < dp; d += 64) row[d] *= f;
     }
@@ -395,7 +386,7 @@ __global__ __launch_bounds__(CT * 256) void delta_scan_kernel(const DeltaPlan p,
 constexpr int kStepThreads = 512;
 
 __device__ __forceinline__ float step_sum(float v, float *red) { // over the workgroup, for every thread
-    v = wave_sum(v);
+    v = wave_add<1>(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
@@ -406,8 +397,8 @@ __device__ __forceinline__ float step_sum(float v, float *red) { // over the wor
 }
 // the same for two values
 __device__ __forceinline__ void step_sum2(float &a, float &b, float2 *red) {
-    a = wave_sum(a);
-    b = wave_sum(b);
+    a = wave_add<1>(a);
+    b = wave_add<1>(b);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = make_float2(a, b);
     __syncthreads();
@@ -623,7 +614,7 @@ __global__ __launch_bounds__(kThreads) void delta_finish_kernel(const DeltaPlan 
     const float *gt = gate + w * p.vdim;
     float ss = 0.0f;
     for (uint32_t d = lane; d < p.vdim; d += 64) ss = fmaf(x[d], x[d], ss);
-    const float f = 1.0f / sqrtf(wave_sum(ss) / (float)p.vdim + p.eps);
+    const float f = 1.0f / sqrtf(wave_add<1>(ss) / (float)p.vdim + p.eps);
     for (uint32_t d = lane; d < p.vdim; d += 64) x[d] = x[d] * f * p.norm[d] * sigmoid(gt[d]);
 }
 

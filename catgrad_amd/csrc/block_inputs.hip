@@ -193,14 +193,7 @@ template <int VW, int TAPS> __global__ __launch_bounds__(kThreads) void conv_row
 // The same for a token a workgroup, four taps (in 16 bytes) and four columns a thread: the taps and what the filter reads are asked for before the
 // scales are known, where the kernel above makes six trips to memory one behind the other.  us above and here, with its timing: a token of 1024
 // columns in 4 groups 7.7 and 6.7, 256 of them 10.3 and 8.7, 500 of 2048 columns in 8 groups 21.0 and 17.5, a token of 4096 columns 10.2 and 8.0.
-typedef const __attribute__((address_space(1))) float global_float;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
-// A pointer that the compiler knows nothing of but its registers: what is chosen among such pointers is chosen, not branched for.
-__device__ __forceinline__ global_float *pinned(const float *p) {
-    int64_t v = reinterpret_cast<int64_t>(p);
-    asm volatile("" : "+s"(v));
-    return reinterpret_cast<global_float *>(v);
-}
 __global__ __launch_bounds__(kThreads) void conv_token_kernel(const ConvRowsPlan p, const uint32_t parts) {
     constexpr int TAPS = 4, PAST = TAPS - 1;
     static_assert(kWaves == TAPS, "a wave per row that a token looks at");

@@ -10,12 +10,9 @@ namespace {
 
 constexpr int kThreads = 256, kWaves = 4;
 
-__device__ __forceinline__ float wave_sum(float v) {
-    return wave_add<1>(v);
-}
 // sum over the 256 threads of a workgroup, for every thread; `red` has a slot per wave
 __device__ __forceinline__ float block_sum(float v, float *red) {
-    v = wave_sum(v);
+    v = wave_add<1>(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
@@ -194,7 +191,7 @@ __global__ __launch_bounds__(kThreads) void few_rows_linear_kernel(const Product
     for (int c = 0; c < NC; c++) {
 #pragma unroll
         for (int m = 0; m < M; m++) {
-            const float s = wave_sum(acc[c][m]);
+            const float s = wave_add<1>(acc[c][m]);
             if ((threadIdx.x & 63) == (uint32_t)m && m < (int)rows && n0 + c < w.n)
                 out[(int64_t)m * w.n + n0 + c] = s * scale + (bias ? bias[n0 + c] : 0.0f);
         }
@@ -229,7 +226,7 @@ __global__ __launch_bounds__(kThreads) void few_rows_residual_kernel(const Rows 
     float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll
     for (int m = 0; m < M; m++) {
-        const float t0 = wave_sum(a0[0][m]), t1 = NB > 1 ? wave_sum(a1[0][m]) : 0.0f;
+        const float t0 = wave_add<1>(a0[0][m]), t1 = NB > 1 ? wave_add<1>(a1[0][m]) : 0.0f;
         if (lane == (uint32_t)m) {
             s0 = t0;
             s1 = t1;

@@ -353,6 +353,14 @@ template <int LOW, class F> __device__ __forceinline__ uint32_t wave_fold(uint32
     if constexpr (LOW <= 1) v = f(v, row_rotated<0x121>(v));
     return v;
 }
+// Values and pointers that the compiler knows nothing of but their scalar registers: what a lane chooses among such is chosen, not branched
+// for, and not fetched from the argument block lane by lane.
+typedef const __attribute__((address_space(1))) float global_float;
+__device__ __forceinline__ int64_t pinned(int64_t v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+__device__ __forceinline__ global_float *pinned(const float *p) { return reinterpret_cast<global_float *>(pinned(reinterpret_cast<int64_t>(p))); }
 struct AddWords {
     __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const { return asu(asf(a) + asf(b)); }
 };

@@ -31,6 +31,9 @@ bool fused_program_fits(const Pending &p) {
 // compared in the tests).  g / d is g times the hardware's reciprocal, off by less than 2^-22 of it: a quotient of two 8-bit
 // significands lies at least 2^-17 of itself from the middle between two bfloat16 numbers, so it rounds as the exact one does
 // (d, a rounded 1 + exp(-g), is between 1 and 2^93; subnormal g have d = 2 and an exact product).
+//
+// f16 stays with MapSiluMulF16: quotients of its 11-bit significands come as close to the middle as 2^-23 of themselves, nearer than the
+// reciprocal is to them, so the same steps would not give its bits.
 template <int R> __device__ __forceinline__ uint32_t silu_exact(uint32_t g, uint32_t one) {
     const uint32_t e = apply<R, true>(apply<kExp, true>(apply<kNeg, true>(g, 0, 0, nullptr), 0, 0, nullptr), 0, 0, nullptr);
     const uint32_t d = apply<R, true>(apply<kAdd, true>(one, e, 0, nullptr), 0, 0, nullptr);
