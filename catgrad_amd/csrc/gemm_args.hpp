@@ -39,6 +39,10 @@ __device__ __forceinline__ void batch_offsets(const MmArgs &a, uint32_t b, int64
 // The f32 products of more than eight rows (split_gemm.hip).  `a` complete but for ksplit; C is the row-major result.
 // a_mfast / b_nfast: the operand's rows, not k, are its unit-stride axis.
 int launch_split_gemm(cg_backend *be, MmArgs a, bool a_mfast, bool b_nfast);
+// The same for a few dozen rows whose operands have k contiguous in 16-byte pieces (split_thin.hip), 16 `high` rows per workgroup, and
+// what that takes in microseconds.
+double thin_gemm_cost(const cg_backend *be, const MmArgs &a, int *high);
+int launch_thin_gemm(cg_backend *be, const MmArgs &a, int high);
 
 
 // y[rows, n] = x[rows, k] . w[n, k]^T of patterns of one narrow format (block_products.hip); pitches in elements; y's rows y_pitch

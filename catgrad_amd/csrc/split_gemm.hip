@@ -172,6 +172,13 @@ int launch_split_gemm(cg_backend *be, MmArgs a, bool a_mfast, bool b_nfast) {
         if (!a_mfast && a.M <= 1024) consider(2);
         if (!a_mfast && a.M <= 32) consider(3);
     }
+    // Few rows, or little work: without a second launch, where that is faster.  Up to four values of k are multiplied by the 32-bit
+    // instructions alone (split_tile.hpp).
+    if (!care && !a_mfast && !b_nfast && a.K % 4 == 0 && a.K > 4) {
+        int high = 0;
+        const double us = thin_gemm_cost(be, a, &high);
+        if (high && us < best) return launch_thin_gemm(be, a, high);
+    }
     const uint64_t tiles = count(t) / a.batch;
     if (tiles > 0x7FFFFFFFull) return fail(CG_ERR_UNSUPPORTED, "matmul: too many tiles");
     Kernel k = all[t].kernel[a_mfast][b_nfast];
