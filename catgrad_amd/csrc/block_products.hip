@@ -174,6 +174,119 @@ template <int OUT> __global__ __launch_bounds__(kThreads) void sum_parts_kernel(
     else static_cast<uint2 *>(y)[i] = make_uint2(pattern<OUT>(v[0]) | pattern<OUT>(v[1]) << 16, pattern<OUT>(v[2]) | pattern<OUT>(v[3]) << 16);
 }
 
+// A few dozen rows: 16 RT x 16 results per workgroup, whose waves take turns of 128 bytes of k.  The operands go from memory into the
+// matrix instruction's registers as they lie (16 bytes of a row per lane, four lanes side by side), two turns in flight, and the
+// waves' sums meet in LDS, so that k is cut eight ways without a second launch.  WHOLE: k is whole turns.
+// Bound by latency, as the tiles are at such sizes, but with one trip behind the other instead of a stage behind the other; tiles with
+// the launch that adds their parts, and here, in us: bf16 32 x 576 x 576 7.8 and 3.5, 64 x 1024 x 1024 9.2 and 4.4, 128 x 3072 x 1024
+// 13.5 and 10.9, 1500 x 16 x 2048 11.1 and 5.9; fp8 64 x 2048 x 2048 10.4 and 5.6.  Four row blocks: within 10 % of the better of one
+// and two where they were the fastest at all.
+constexpr int kThinWaves = 8, kTurnBytes = 128;
+template <int FMT, int OUT, int RT, bool WHOLE> __global__ __launch_bounds__(64 * kThinWaves) void narrow_thin_kernel(const TileArgs a) {
+    constexpr uint32_t TILE = RT * 256;
+    __shared__ float red[kThinWaves][TILE];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, li = lane % 16, lg = lane / 16;
+    const uint32_t n0 = blockIdx.x * 16, m0 = blockIdx.y * (16 * RT), turns = (a.K + kTurnBytes - 1) / kTurnBytes;
+    const char *const col = a.w + (uint64_t)min(n0 + li, a.N - 1) * a.w_pitch, *row[RT];
+#pragma unroll
+    for (int i = 0; i < RT; i++) row[i] = a.x + (uint64_t)min(m0 + 16 * i + li, a.M - 1) * a.x_pitch; // (rows behind the last repeat it)
+    int4v x[2][RT][2], y[2][2];
+    auto ask = [&](const uint32_t t, const int set) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const uint32_t k0 = t * kTurnBytes + h * 64 + lg * 16, k = WHOLE ? k0 : min(k0, a.K - 16);
+            y[set][h] = *reinterpret_cast<const int4v *>(col + k);
+#pragma unroll
+            for (int i = 0; i < RT; i++) x[set][i][h] = *reinterpret_cast<const int4v *>(row[i] + k);
+        }
+    };
+    float4v acc[RT];
+#pragma unroll
+    for (int i = 0; i < RT; i++) acc[i] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    constexpr int STEPS = FMT == kFmtF8 ? 2 : 1; // matrix instructions per 16 bytes
+    auto widen = [&](const int4v v, const bool in, int4v(&f)[STEPS]) { // (what was read elsewhere becomes zeros)
+        if constexpr (FMT != kFmtF8) f[0] = v;
+        else {
+#pragma unroll
+            for (int w = 0; w < 4; w++) { // (as bfloat16: see narrow_tile_kernel)
+                f[w / 2][w % 2 * 2] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((uint32_t)v[w], 1.0f, false));
+                f[w / 2][w % 2 * 2 + 1] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((uint32_t)v[w], 1.0f, true));
+            }
+        }
+        if (WHOLE) return;
+#pragma unroll
+        for (int t = 0; t < STEPS; t++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) f[t][j] = in ? f[t][j] : 0;
+    };
+    auto multiply = [&](const uint32_t t, const int set) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const bool in = t * kTurnBytes + h * 64 + lg * 16 < a.K;
+            int4v p[STEPS], q[STEPS];
+            widen(y[set][h], in, q);
+#pragma unroll
+            for (int i = 0; i < RT; i++) {
+                widen(x[set][i][h], in, p);
+#pragma unroll
+                for (int s = 0; s < STEPS; s++) {
+                    if constexpr (FMT == kFmtF16) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, p[s]), __builtin_bit_cast(f16x8, q[s]), acc[i], 0, 0, 0);
+                    else acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, p[s]), __builtin_bit_cast(bf16x8, q[s]), acc[i], 0, 0, 0);
+                }
+            }
+        }
+    };
+    if (wave < turns) { // (the loads stay where they stand, and every wait in the loop knows what else is on its way)
+        const uint32_t n = (turns - 1 - wave) / kThinWaves + 1;
+        uint32_t t = wave;
+        ask(t, 0);
+        if (n == 1) {
+            multiply(t, 0);
+        } else {
+            ask(t + kThinWaves, 1);
+            for (uint32_t left = n; left > 3; left -= 2, t += 2 * kThinWaves) {
+                multiply(t, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                ask(t + 2 * kThinWaves, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(t + kThinWaves, 1);
+                __builtin_amdgcn_sched_barrier(0);
+                ask(t + 3 * kThinWaves, 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            multiply(t, 0);
+            if (n % 2) {
+                ask(t + 2 * kThinWaves, 0);
+                multiply(t + kThinWaves, 1);
+                multiply(t + 2 * kThinWaves, 0);
+            } else {
+                multiply(t + kThinWaves, 1);
+            }
+        }
+    }
+    // (the last sums are on their way behind a branch, where the compiler does not always wait for them)
+#pragma unroll
+    for (int i = 0; i < RT; i++) asm volatile("s_nop 7" : "+v"(acc[i]));
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) red[wave][i * 256 + v * 64 + lane] = acc[i][v];
+    __syncthreads();
+    for (uint32_t e = threadIdx.x; e < TILE; e += 64 * kThinWaves) {
+        float s = red[0][e];
+#pragma unroll
+        for (int w = 1; w < kThinWaves; w++) s += red[w][e];
+        const uint32_t l = e % 64, r = m0 + e / 256 * 16 + l / 16 * 4 + e / 64 % 4, c = n0 + l % 16;
+        if (r < a.M && c < a.N) put<OUT>(a.y, (uint64_t)r * a.ld + c, s);
+    }
+}
+
+template <int FMT, int OUT, int RT> void launch_thin(cg_backend *be, const TileArgs &a) {
+    const dim3 grid((a.N + 15) / 16, (a.M + 16 * RT - 1) / (16 * RT));
+    if (a.K % kTurnBytes == 0) hipLaunchKernelGGL((narrow_thin_kernel<FMT, OUT, RT, true>), grid, dim3(64 * kThinWaves), 0, be->stream, a);
+    else hipLaunchKernelGGL((narrow_thin_kernel<FMT, OUT, RT, false>), grid, dim3(64 * kThinWaves), 0, be->stream, a);
+}
+
 int launched(const char *what) {
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, what);
@@ -198,6 +311,20 @@ template <int FMT, int OUT> int run_tiles(cg_backend *be, TileArgs a) {
         const double rounds = std::ceil((double)(tiles * p) / be->compute_units), stages = ((a.K + p - 1) / p + kStageBytes - 1) / kStageBytes;
         const double us = start + stage * stages * std::max(1.0, share * rounds) + (p > 1 ? 0.9 + 0.15 * p + 1.44e-6 * p * mn : 0.0);
         if (p == 1 || us < best) splits = p, best = us;
+    }
+    // Few rows, or little work: without a second launch, where that is faster.  Fitted to 136 shapes of 9 to 1500 rows, each format and both
+    // heights timed: one row block while a compute unit has one workgroup, two beyond.
+    int high = 0;
+    for (int rt = 1; rt <= 2; rt++) {
+        const uint64_t rows = (a.M + 16 * rt - 1) / (16 * rt);
+        const double rounds = (double)(rows * ((a.N + 15) / 16)) / be->compute_units, turns = a.K / (double)(kThinWaves * kTurnBytes);
+        const double us = 2.6 + (rt == 1 ? 0.9 : 1.32) * std::max(0.5, turns) * std::max(1.0, rounds);
+        if (rows <= 65535 && us < best) high = rt, best = us;
+    }
+    if (high) {
+        if (high == 1) launch_thin<FMT, OUT, 1>(be, a);
+        else launch_thin<FMT, OUT, 2>(be, a);
+        return launched("narrow_thin");
     }
     a.k_part = ((a.K + splits - 1) / splits + kStageBytes - 1) / kStageBytes * kStageBytes;
     splits = (a.K + a.k_part - 1) / a.k_part;

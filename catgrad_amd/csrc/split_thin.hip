@@ -89,19 +89,33 @@ template <int RT, bool WHOLE> __global__ __launch_bounds__(64 * kWaves, 4) void 
             asm volatile("" : "+v"(acc[i]));
         }
     };
-    if (wave < turns) {
-        const uint32_t last = wave + (turns - 1 - wave) / kWaves * kWaves; // this wave's last turn
-        ask(wave, 0);
-        if (wave != last) ask(wave + kWaves, 1);
-        for (uint32_t t = wave;;) {
-            multiply(t, 0, wave % 2);
-            if (t == last) break;
-            if (t + kWaves != last) ask(t + 2 * kWaves, 0);
-            t += kWaves;
-            multiply(t, 1, wave % 2 == 0);
-            if (t == last) break;
-            if (t + kWaves != last) ask(t + 2 * kWaves, 1);
-            t += kWaves;
+    if (wave < turns) { // (the loads stay where they stand, and every wait in the loop knows what else is on its way)
+        const uint32_t n = (turns - 1 - wave) / kWaves + 1;
+        const bool odd = wave % 2;
+        uint32_t t = wave;
+        ask(t, 0);
+        if (n == 1) {
+            multiply(t, 0, odd);
+        } else {
+            ask(t + kWaves, 1);
+            for (uint32_t left = n; left > 3; left -= 2, t += 2 * kWaves) {
+                multiply(t, 0, odd);
+                __builtin_amdgcn_sched_barrier(0);
+                ask(t + 2 * kWaves, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(t + kWaves, 1, !odd);
+                __builtin_amdgcn_sched_barrier(0);
+                ask(t + 3 * kWaves, 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            multiply(t, 0, odd);
+            if (n % 2) {
+                ask(t + 2 * kWaves, 0);
+                multiply(t + kWaves, 1, !odd);
+                multiply(t + 2 * kWaves, 0, odd);
+            } else {
+                multiply(t + kWaves, 1, !odd);
+            }
         }
     }
     auto leave = [&]() {

@@ -1,7 +1,9 @@
-"""f32 products of a few dozen rows with k contiguous in both operands: a workgroup's waves take turns of 32 values of k, and their
-sums meet in LDS; rows that the pieces cannot hold are multiplied as they are."""
+"""Products of a few dozen rows with k contiguous in both operands, of f32 and of the narrow dtypes: a workgroup's waves take turns of
+32 values (narrow: 128 bytes) of k, and their sums meet in LDS; f32 rows that the pieces cannot hold are multiplied as they are."""
 import numpy as np
 import pytest
+
+from catgrad_amd import _abi as A
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +71,26 @@ def test_roundings_have_no_direction(hip, size):
     want = a.astype(np.float64) @ b.astype(np.float64).transpose(0, 2, 1)
     d = hip.to_numpy(hip.matmul(x, y)) - want
     assert abs(d.mean()) <= 2.0 ** -28 * np.sqrt((want ** 2).mean())
+
+
+# a value beside a block of 16 rows and columns, a turn (64 16-bit or 128 8-bit values) and a round of the waves' turns; one and two row
+# blocks per workgroup; a tall narrow result
+NARROW = [(70, 1024, 65), (17, 4112, 17), (65, 1040, 128), (96, 1536, 600), (130, 560, 1500), (1500, 2048, 16), (64, 1008, 1000), (16, 8192, 100)]
+
+
+@pytest.mark.parametrize("size", NARROW, ids=str)
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16", "float8"])
+def test_narrow_dtypes(hip, size, dtype):
+    """Exact sums of small whole numbers, so that the one rounding of the result is all there may be."""
+    torch = pytest.importorskip("torch")
+    M, K, N = size
+    rng = np.random.default_rng(K)
+    a, b = rng.integers(-3, 4, (M, K)).astype(np.float32), rng.integers(-3, 4, (N, K)).astype(np.float32)
+    kind = {"bfloat16": torch.bfloat16, "float16": torch.float16, "float8": torch.float8_e4m3fn}[dtype]
+    make = {"bfloat16": lambda v: hip.ndarray_from_vec_bf16(torch.from_numpy(v).to(kind).view(torch.int16).numpy().view(np.uint16), v.shape),
+            "float16": lambda v: hip.ndarray_from_vec_f16(v.astype(np.float16), v.shape),
+            "float8": lambda v: hip.ndarray_from_vec_fp8(torch.from_numpy(v).to(kind).view(torch.uint8).numpy(), v.shape)}[dtype]
+    got = hip.to_numpy(hip.cast(hip.matmul(make(a), hip.transpose(make(b), 0, 1)), A.F32))
+    want = torch.from_numpy(a.astype(np.float64) @ b.astype(np.float64).T)
+    want = (want.clamp(-448, 448) if dtype == "float8" else want).to(kind).float().numpy()
+    np.testing.assert_array_equal(got, want)
