@@ -382,20 +382,20 @@ inline bool all_words(const FusedArgs &a) {
     for (uint32_t l = 0; l < a.nleaf; l++) words &= a.leaf[l].fmt == kFmtWords;
     return words;
 }
-template <class P> void aot_map_launch(const FusedArgs &a, dim3 grid, hipStream_t s) {
+template <class P> void aot_map_launch(const FusedArgs &a, dim3 grid, LaunchQueue &s) {
     const bool words = all_words(a);
     if (a.g.vec == 4 && words)
-        hipLaunchKernelGGL((aot_map_kernel<WordsOnly<P>, 4>), grid, dim3(kBlock), 0, s, a);
+        launch_kernel((aot_map_kernel<WordsOnly<P>, 4>), grid, dim3(kBlock), 0, s, a);
     else if (a.g.vec == 4)
-        hipLaunchKernelGGL((aot_map_kernel<P, 4>), grid, dim3(kBlock), 0, s, a);
+        launch_kernel((aot_map_kernel<P, 4>), grid, dim3(kBlock), 0, s, a);
     else if (words)
-        hipLaunchKernelGGL((aot_map_kernel<WordsOnly<P>, 1>), grid, dim3(kBlock), 0, s, a);
+        launch_kernel((aot_map_kernel<WordsOnly<P>, 1>), grid, dim3(kBlock), 0, s, a);
     else
-        hipLaunchKernelGGL((aot_map_kernel<P, 1>), grid, dim3(kBlock), 0, s, a);
+        launch_kernel((aot_map_kernel<P, 1>), grid, dim3(kBlock), 0, s, a);
 }
-inline bool aot_map_dispatch(const Pending &, const FusedArgs &, dim3, hipStream_t, ProgramList<>) { return false; }
+inline bool aot_map_dispatch(const Pending &, const FusedArgs &, dim3, LaunchQueue &, ProgramList<>) { return false; }
 template <class P, class... Rest>
-bool aot_map_dispatch(const Pending &p, const FusedArgs &a, dim3 grid, hipStream_t s, ProgramList<P, Rest...>) {
+bool aot_map_dispatch(const Pending &p, const FusedArgs &a, dim3 grid, LaunchQueue &s, ProgramList<P, Rest...>) {
     if (program_matches<P>(p)) {
         aot_map_launch<P>(a, grid, s);
         return true;
@@ -405,20 +405,20 @@ bool aot_map_dispatch(const Pending &p, const FusedArgs &a, dim3 grid, hipStream
 
 // Cached items per lane: 3 vectors of four (rows up to 12 * TPR elements; programs of a single leaf up to 16 vectors by 256 lanes,
 // rows up to 16384) or 10 single elements (rows up to 10 * TPR); longer rows take the re-reading instantiation.
-template <class P, int VEC> void aot_rows_launch(const FusedArgs &a, uint32_t *rowout, int tpr, dim3 grid, hipStream_t s) {
+template <class P, int VEC> void aot_rows_launch(const FusedArgs &a, uint32_t *rowout, int tpr, dim3 grid, LaunchQueue &s) {
     constexpr int CI = VEC == 4 ? 3 : 10;
     const bool fits = (uint64_t)(a.n / VEC) <= (uint64_t)CI * (uint32_t)tpr;
 #define CG_ROWS(TPR)                                                                                        \
     do {                                                                                                    \
         if (fits)                                                                                           \
-            hipLaunchKernelGGL((aot_rows_kernel<P, VEC, TPR, CI>), grid, dim3(kBlock), 0, s, a, rowout);     \
+            launch_kernel((aot_rows_kernel<P, VEC, TPR, CI>), grid, dim3(kBlock), 0, s, a, rowout);     \
         else                                                                                                \
-            hipLaunchKernelGGL((aot_rows_kernel<P, VEC, TPR, 0>), grid, dim3(kBlock), 0, s, a, rowout);      \
+            launch_kernel((aot_rows_kernel<P, VEC, TPR, 0>), grid, dim3(kBlock), 0, s, a, rowout);      \
     } while (0)
     if constexpr (VEC == 4 && P::nleaf == 1) {
         if (!fits && tpr == 256 && a.n <= 16384) {
-            if (a.n <= 8192) hipLaunchKernelGGL((aot_rows_kernel<P, VEC, 256, 8>), grid, dim3(kBlock), 0, s, a, rowout);
-            else hipLaunchKernelGGL((aot_rows_kernel<P, VEC, 256, 16>), grid, dim3(kBlock), 0, s, a, rowout);
+            if (a.n <= 8192) launch_kernel((aot_rows_kernel<P, VEC, 256, 8>), grid, dim3(kBlock), 0, s, a, rowout);
+            else launch_kernel((aot_rows_kernel<P, VEC, 256, 16>), grid, dim3(kBlock), 0, s, a, rowout);
             return;
         }
     }
@@ -427,12 +427,12 @@ template <class P, int VEC> void aot_rows_launch(const FusedArgs &a, uint32_t *r
     else CG_ROWS(256);
 #undef CG_ROWS
 }
-inline bool aot_rows_dispatch(const Pending &, const FusedArgs &, uint32_t *, int, dim3, hipStream_t, ProgramList<>) {
+inline bool aot_rows_dispatch(const Pending &, const FusedArgs &, uint32_t *, int, dim3, LaunchQueue &, ProgramList<>) {
     return false;
 }
 // tpr: lanes per row, one of 16 / 64 / 256 (shorter rows stay with the interpreter)
 template <class P, class... Rest>
-bool aot_rows_dispatch(const Pending &p, const FusedArgs &a, uint32_t *rowout, int tpr, dim3 grid, hipStream_t s,
+bool aot_rows_dispatch(const Pending &p, const FusedArgs &a, uint32_t *rowout, int tpr, dim3 grid, LaunchQueue &s,
                        ProgramList<P, Rest...>) {
     if (program_matches<P>(p)) {
         const bool words = all_words(a);

@@ -4,7 +4,7 @@
 
 namespace cg {
 
-bool launch_compiled_rows(const Pending &p, const FusedArgs &a, uint32_t *rowout, int tpr, dim3 grid, hipStream_t s) {
+bool launch_compiled_rows(const Pending &p, const FusedArgs &a, uint32_t *rowout, int tpr, dim3 grid, LaunchQueue &s) {
     return aot_rows_dispatch(p, a, rowout, tpr, grid, s, RowsPrograms{});
 }
 

@@ -51,7 +51,7 @@ static int launch_seg_kernel(cg_backend *be, const AttnArgs &g, const FusedArgs 
                                                    hipFuncAttributeMaxDynamicSharedMemorySize,
                                                    (int)seg_lds_bytes(MM, LPT * 4, kSegMaxChunk)) == hipSuccess;
     if (!lds_ok) return fail(CG_ERR_DEVICE, "decode attention: cannot reserve %zu bytes of LDS", seg_lds_bytes(MM, LPT * 4, kSegMaxChunk));
-    hipLaunchKernelGGL((decode_attention_seg_kernel<P, LPT, MM, PASSES, LOOP>), dim3(g.splits, batch), dim3(kSegBlock), lds, be->stream, g, a);
+    launch_kernel((decode_attention_seg_kernel<P, LPT, MM, PASSES, LOOP>), dim3(g.splits, batch), dim3(kSegBlock), lds, be->stream, g, a);
     return CG_OK;
 }
 
@@ -189,7 +189,7 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
 #undef CG_SEG_KERNEL
                 if (!rc) {
                     const uint64_t nrows = (uint64_t)f1.batch * g.M, waves = kBlock / 64;
-                    hipLaunchKernelGGL(decode_attention_combine_kernel, dim3((uint32_t)((nrows + waves - 1) / waves)), dim3(kBlock), 0,
+                    launch_kernel(decode_attention_combine_kernel, dim3((uint32_t)((nrows + waves - 1) / waves)), dim3(kBlock), 0,
                                        be->stream, g.part_o, g.part_ml, static_cast<uint32_t *>(out->buf->ptr), g.splits, g.M,
                                        (uint32_t)hd, nrows);
                 }
@@ -231,10 +231,10 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
         g.groups = make_fastdiv(g.M * (halves ? 2 : 1));
 #define CG_ROW_KERNEL(LPT, VS)                                                                                                     \
     do {                                                                                                                           \
-        if (passes == 5) hipLaunchKernelGGL((decode_attention_row_kernel<P, LPT, 5, false, VS>), grid, block, 0, be->stream, g, a, po);   \
-        else if (passes == 10) hipLaunchKernelGGL((decode_attention_row_kernel<P, LPT, 10, false, VS>), grid, block, 0, be->stream, g, a, po); \
-        else if (passes == 16) hipLaunchKernelGGL((decode_attention_row_kernel<P, LPT, 16, false, VS>), grid, block, 0, be->stream, g, a, po); \
-        else hipLaunchKernelGGL((decode_attention_row_kernel<P, LPT, 6, true, VS>), grid, block, 0, be->stream, g, a, po);          \
+        if (passes == 5) launch_kernel((decode_attention_row_kernel<P, LPT, 5, false, VS>), grid, block, 0, be->stream, g, a, po);   \
+        else if (passes == 10) launch_kernel((decode_attention_row_kernel<P, LPT, 10, false, VS>), grid, block, 0, be->stream, g, a, po); \
+        else if (passes == 16) launch_kernel((decode_attention_row_kernel<P, LPT, 16, false, VS>), grid, block, 0, be->stream, g, a, po); \
+        else launch_kernel((decode_attention_row_kernel<P, LPT, 6, true, VS>), grid, block, 0, be->stream, g, a, po);          \
     } while (0)
         if (hd == 64 && halves) CG_ROW_KERNEL(16, 2);
         else if (hd == 64) CG_ROW_KERNEL(16, 1);
@@ -243,7 +243,7 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
 #undef CG_ROW_KERNEL
         if (segmented) {
             const uint64_t nrows = (uint64_t)f1.batch * g.M, waves = kBlock / 64;
-            hipLaunchKernelGGL(decode_attention_combine_kernel, dim3((uint32_t)((nrows + waves - 1) / waves)), dim3(kBlock), 0,
+            launch_kernel(decode_attention_combine_kernel, dim3((uint32_t)((nrows + waves - 1) / waves)), dim3(kBlock), 0,
                                be->stream, g.part_o, g.part_ml, po, nseg, g.M, (uint32_t)hd, nrows);
             be->pool.free(part_o, co); // stream-ordered: later users queue behind the combine
             be->pool.free(part_ml, cml);
@@ -268,11 +268,11 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
         ProfScope prof(be, CG_K_GEMM_SKINNY, distinct_bytes(q) + distinct_bytes(kt) + distinct_bytes(v) + distinct_bytes(out));
         dim3 grid(g.splits, (uint32_t)f1.batch);
         if (hd == 64)
-            hipLaunchKernelGGL((decode_attention_kernel<P, 16>), grid, dim3(kBlock), 0, be->stream, g, a);
+            launch_kernel((decode_attention_kernel<P, 16>), grid, dim3(kBlock), 0, be->stream, g, a);
         else
-            hipLaunchKernelGGL((decode_attention_kernel<P, 32>), grid, dim3(kBlock), 0, be->stream, g, a);
+            launch_kernel((decode_attention_kernel<P, 32>), grid, dim3(kBlock), 0, be->stream, g, a);
         const uint64_t rows = (uint64_t)f1.batch * g.M, waves = kBlock / 64;
-        hipLaunchKernelGGL(decode_attention_combine_kernel, dim3((uint32_t)((rows + waves - 1) / waves)), dim3(kBlock), 0,
+        launch_kernel(decode_attention_combine_kernel, dim3((uint32_t)((rows + waves - 1) / waves)), dim3(kBlock), 0,
                            be->stream, g.part_o, g.part_ml, static_cast<uint32_t *>(out->buf->ptr), g.splits, g.M,
                            (uint32_t)hd, rows);
     }
@@ -417,12 +417,12 @@ int launch_prefill_attention(cg_backend *be, const Pending &p, const int64_t *pd
         ProfScope prof(be, CG_K_ATTENTION, flop);
         dim3 grid((uint32_t)nblocks, (uint32_t)ksplit);
         if (hd == 64)
-            hipLaunchKernelGGL((prefill_attention_kernel<64>), grid, dim3(kBlock), prefill_lds_bytes(64), be->stream, g, e);
+            launch_kernel((prefill_attention_kernel<64>), grid, dim3(kBlock), prefill_lds_bytes(64), be->stream, g, e);
         else
-            hipLaunchKernelGGL((prefill_attention_kernel<128>), grid, dim3(kBlock), prefill_lds_bytes(128), be->stream, g, e);
+            launch_kernel((prefill_attention_kernel<128>), grid, dim3(kBlock), prefill_lds_bytes(128), be->stream, g, e);
         if (ksplit > 1) {
             const uint64_t items = rows * (uint64_t)(hd / 4);
-            hipLaunchKernelGGL(prefill_attention_combine_kernel, dim3((uint32_t)((items + kBlock - 1) / kBlock)), dim3(kBlock), 0, be->stream,
+            launch_kernel(prefill_attention_combine_kernel, dim3((uint32_t)((items + kBlock - 1) / kBlock)), dim3(kBlock), 0, be->stream,
                                e.part_o, e.part_ml, e.out, (uint32_t)ksplit, (uint32_t)hd, rows);
         }
     }

@@ -429,13 +429,13 @@ int rows_kernels(cg_backend *be, const AttentionPlan &p, const float *q, uint32_
     if (!p.mix_scores)
         if (int rc = allow_lds(attention_mix_kernel<REP, MVW>, lds2)) return rc;
     const dim3 grid(nseg, p.kv_heads * groups, rows);
-    if (fresh) hipLaunchKernelGGL((attention_scores_kernel<REP, SVW, true>), grid, dim3(kThreads), lds1, be->stream, p, q, row0, nseg, scores, stats);
-    else hipLaunchKernelGGL((attention_scores_kernel<REP, SVW, false>), grid, dim3(kThreads), lds1, be->stream, p, q, row0, nseg, scores, stats);
+    if (fresh) launch_kernel((attention_scores_kernel<REP, SVW, true>), grid, dim3(kThreads), lds1, be->stream, p, q, row0, nseg, scores, stats);
+    else launch_kernel((attention_scores_kernel<REP, SVW, false>), grid, dim3(kThreads), lds1, be->stream, p, q, row0, nseg, scores, stats);
     if (p.mix_scores) return launch_mixed_rows(be, p, row0, rows, nseg, scores, parts, reinterpret_cast<float2 *>(parts + (size_t)rows * nseg * p.heads * p.vdim));
-    hipLaunchKernelGGL((attention_mix_kernel<REP, MVW>), grid, dim3(kThreads), lds2, be->stream, p, row0, nseg, scores, stats, nseg > 1 ? parts : p.out, nseg > 1);
+    launch_kernel((attention_mix_kernel<REP, MVW>), grid, dim3(kThreads), lds2, be->stream, p, row0, nseg, scores, stats, nseg > 1 ? parts : p.out, nseg > 1);
     if (nseg > 1) {
         const uint32_t n = p.heads * p.vdim;
-        hipLaunchKernelGGL(attention_sum_kernel, dim3((n + kThreads - 1) / kThreads, rows), dim3(kThreads), 0, be->stream, parts, nseg, n,
+        launch_kernel(attention_sum_kernel, dim3((n + kThreads - 1) / kThreads, rows), dim3(kThreads), 0, be->stream, parts, nseg, n,
                            p.out + (int64_t)row0 * n);
     }
     return launched("block_attention");
@@ -467,7 +467,7 @@ static int rotation_tables(cg_backend *be, AttentionPlan &p, uint64_t end) {
             delete b;
             return rc;
         }
-        hipLaunchKernelGGL(rotation_table_kernel, dim3((rows * pairs + kThreads - 1) / kThreads), dim3(kThreads), 0, be->stream, static_cast<float2 *>(b->ptr), rows, step,
+        launch_kernel(rotation_table_kernel, dim3((rows * pairs + kThreads - 1) / kThreads), dim3(kThreads), 0, be->stream, static_cast<float2 *>(b->ptr), rows, step,
                            p.rot_dims, p.rot_log2);
         *out = b;
         return launched("rotation_table");
@@ -519,12 +519,12 @@ int launch_attention(cg_backend *be, const AttentionPlan &plan) {
         q = static_cast<float *>(qbuf.p);
         auto aligned = [](const Rows &x) { return x.pitch % 4 == 0 && (reinterpret_cast<uintptr_t>(x.p) & 15) == 0; };
         const bool pieces = turned && !p.q_norm && !p.k_norm && p.dim % 4 == 0 && p.dim <= 256 && aligned(p.q) && aligned(p.k);
-        if (pieces && p.dim <= 32) hipLaunchKernelGGL((attention_turn_heads_kernel<8>), dim3(rows), dim3(kThreads), 0, be->stream, p, q);
-        else if (pieces && p.dim <= 64) hipLaunchKernelGGL((attention_turn_heads_kernel<16>), dim3(rows), dim3(kThreads), 0, be->stream, p, q);
-        else if (pieces && p.dim <= 128) hipLaunchKernelGGL((attention_turn_heads_kernel<32>), dim3(rows), dim3(kThreads), 0, be->stream, p, q);
-        else if (pieces) hipLaunchKernelGGL((attention_turn_heads_kernel<64>), dim3(rows), dim3(kThreads), 0, be->stream, p, q);
-        else if (turned) hipLaunchKernelGGL(attention_turn_kernel, dim3(rows), dim3(kThreads), (size_t)(p.rot_dims / 2) * sizeof(float2), be->stream, p, q);
-        else hipLaunchKernelGGL(attention_prepare_kernel, dim3(rows), dim3(kThreads), 0, be->stream, p, q);
+        if (pieces && p.dim <= 32) launch_kernel((attention_turn_heads_kernel<8>), dim3(rows), dim3(kThreads), 0, be->stream, p, q);
+        else if (pieces && p.dim <= 64) launch_kernel((attention_turn_heads_kernel<16>), dim3(rows), dim3(kThreads), 0, be->stream, p, q);
+        else if (pieces && p.dim <= 128) launch_kernel((attention_turn_heads_kernel<32>), dim3(rows), dim3(kThreads), 0, be->stream, p, q);
+        else if (pieces) launch_kernel((attention_turn_heads_kernel<64>), dim3(rows), dim3(kThreads), 0, be->stream, p, q);
+        else if (turned) launch_kernel(attention_turn_kernel, dim3(rows), dim3(kThreads), (size_t)(p.rot_dims / 2) * sizeof(float2), be->stream, p, q);
+        else launch_kernel(attention_prepare_kernel, dim3(rows), dim3(kThreads), 0, be->stream, p, q);
         if (int rc = launched("attention_prepare")) return rc;
         if (int rc = p.mix_scores ? launch_mixed_tiles(be, p, q) : launch_attention_tiles(be, p, q); rc != kDeclined) return rc;
     }

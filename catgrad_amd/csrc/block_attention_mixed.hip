@@ -723,16 +723,16 @@ void merge(cg_backend *be, const AttentionPlan &p, const float *parts, const flo
     if (segs <= 8) {
         const uint64_t total = (uint64_t)rows * n;
         if (p.vdim % 4 == 0)
-            hipLaunchKernelGGL((attention_merge_rows_kernel<4>), dim3((uint32_t)((total / 4 + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream, parts, stats, segs, row_pitch,
+            launch_kernel((attention_merge_rows_kernel<4>), dim3((uint32_t)((total / 4 + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream, parts, stats, segs, row_pitch,
                                seg_pitch, p.heads, p.vdim, p.zero_sink, total, out);
         else
-            hipLaunchKernelGGL((attention_merge_rows_kernel<1>), dim3((uint32_t)((total + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream, parts, stats, segs, row_pitch,
+            launch_kernel((attention_merge_rows_kernel<1>), dim3((uint32_t)((total + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream, parts, stats, segs, row_pitch,
                                seg_pitch, p.heads, p.vdim, p.zero_sink, total, out);
         return;
     }
     for (uint32_t r0 = 0; r0 < rows; r0 += 65535) {
         const uint32_t nr = std::min(rows - r0, 65535u);
-        hipLaunchKernelGGL(attention_merge_kernel, dim3((n + 63) / 64, nr), dim3(kMergeWaves * 64), 0, be->stream, parts + (uint64_t)r0 * row_pitch * p.vdim,
+        launch_kernel(attention_merge_kernel, dim3((n + 63) / 64, nr), dim3(kMergeWaves * 64), 0, be->stream, parts + (uint64_t)r0 * row_pitch * p.vdim,
                            stats + (uint64_t)r0 * row_pitch, segs, row_pitch, seg_pitch, p.heads, p.vdim, p.zero_sink, out + (uint64_t)r0 * n);
     }
 }
@@ -742,7 +742,7 @@ int mixed_rows(cg_backend *be, const AttentionPlan &p, uint32_t row0, uint32_t r
     const uint32_t rep = p.heads / p.kv_heads, groups = (rep + REP - 1) / REP, slots = p.talk ? p.heads : REP;
     const size_t lds = (size_t)mixed_floats(REP, slots, VW) * 4;
     if (int rc = allow_lds(reinterpret_cast<const void *>(&attention_mixed_rows_kernel<REP, VW>), lds)) return rc;
-    hipLaunchKernelGGL((attention_mixed_rows_kernel<REP, VW>), dim3(nseg, p.kv_heads * groups, rows), dim3(kThreads), lds, be->stream, p, row0, nseg, scores, parts, stats);
+    launch_kernel((attention_mixed_rows_kernel<REP, VW>), dim3(nseg, p.kv_heads * groups, rows), dim3(kThreads), lds, be->stream, p, row0, nseg, scores, parts, stats);
     merge(be, p, parts, stats, nseg, (uint64_t)nseg * p.heads, p.heads, rows, p.out + (uint64_t)row0 * p.heads * p.vdim);
     return launched("attention_mixed_rows");
 }
@@ -752,7 +752,7 @@ int launch_tiles(cg_backend *be, const AttentionPlan &p, const float *q, uint32_
     const uint32_t tiles = (p.S + kRowsT - 1) / kRowsT;
     const size_t h16 = (HPW * kTileWaves + 15) / 16 * 16, lds = (3 * h16 * kHeadPitch + h16 * (h16 + 4)) * 4;
     if (int rc = allow_lds(reinterpret_cast<const void *>(&attention_mixed_tiles_kernel<HPW, DT, VT, QREG, EXACT, SHARED>), lds)) return rc;
-    hipLaunchKernelGGL((attention_mixed_tiles_kernel<HPW, DT, VT, QREG, EXACT, SHARED>), dim3(tiles * splits, p.B), dim3(kTileWaves * 64), lds, be->stream, p, q, tiles, splits, dst,
+    launch_kernel((attention_mixed_tiles_kernel<HPW, DT, VT, QREG, EXACT, SHARED>), dim3(tiles * splits, p.B), dim3(kTileWaves * 64), lds, be->stream, p, q, tiles, splits, dst,
                        stats);
     return CG_OK;
 }
@@ -808,7 +808,7 @@ template <int REP, int DQ>
 static int step_kernels(cg_backend *be, const AttentionPlan &p, uint32_t chunk, uint32_t chunks, dim3 grid, size_t lds, float *parts, float2 *stats) {
     constexpr int PI = 8 / DQ; // keys of four lanes: 8 pieces per lane
     if (int rc = allow_lds(reinterpret_cast<const void *>(&attention_mixed_step_kernel<REP, DQ, PI>), lds)) return rc;
-    hipLaunchKernelGGL((attention_mixed_step_kernel<REP, DQ, PI>), grid, dim3(kThreads), lds, be->stream, p, chunk, chunks, parts, stats);
+    launch_kernel((attention_mixed_step_kernel<REP, DQ, PI>), grid, dim3(kThreads), lds, be->stream, p, chunk, chunks, parts, stats);
     return CG_OK;
 }
 

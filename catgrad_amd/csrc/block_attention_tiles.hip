@@ -339,10 +339,10 @@ template <int HPW, int DT, bool QREG> int run_tiles(cg_backend *be, const Attent
     const uint32_t tiles = (p.S + kRowsT - 1) / kRowsT, rep = p.heads / p.kv_heads;
     // heads of a stats wave: two that share their keys, or one
     if (rep % 2 == 0 && DT <= 4)
-        hipLaunchKernelGGL((attention_row_stats_kernel<2, DT>), dim3(tiles, (p.heads + 2 * kStatWaves - 1) / (2 * kStatWaves), p.B), dim3(kStatWaves * 64), 0,
+        launch_kernel((attention_row_stats_kernel<2, DT>), dim3(tiles, (p.heads + 2 * kStatWaves - 1) / (2 * kStatWaves), p.B), dim3(kStatWaves * 64), 0,
                            be->stream, p, q, stats);
     else
-        hipLaunchKernelGGL((attention_row_stats_kernel<1, DT>), dim3(tiles, (p.heads + kStatWaves - 1) / kStatWaves, p.B), dim3(kStatWaves * 64), 0, be->stream, p,
+        launch_kernel((attention_row_stats_kernel<1, DT>), dim3(tiles, (p.heads + kStatWaves - 1) / kStatWaves, p.B), dim3(kStatWaves * 64), 0, be->stream, p,
                            q, stats);
     const size_t h16 = (p.heads + 15) / 16 * 16, lds = (3 * h16 * kHeadPitch + 2 * p.heads * kRowsT + h16 * (h16 + 4)) * 4;
     const void *f = p.talk ? reinterpret_cast<const void *>(&attention_tiles_kernel<HPW, DT, QREG, true>)
@@ -352,8 +352,8 @@ template <int HPW, int DT, bool QREG> int run_tiles(cg_backend *be, const Attent
         if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute");
     }
     const dim3 grid(tiles * splits, p.B);
-    if (p.talk) hipLaunchKernelGGL((attention_tiles_kernel<HPW, DT, QREG, true>), grid, dim3(kTileWaves * 64), lds, be->stream, p, q, stats, tiles, splits, dst);
-    else hipLaunchKernelGGL((attention_tiles_kernel<HPW, DT, QREG, false>), grid, dim3(kTileWaves * 64), lds, be->stream, p, q, stats, tiles, splits, dst);
+    if (p.talk) launch_kernel((attention_tiles_kernel<HPW, DT, QREG, true>), grid, dim3(kTileWaves * 64), lds, be->stream, p, q, stats, tiles, splits, dst);
+    else launch_kernel((attention_tiles_kernel<HPW, DT, QREG, false>), grid, dim3(kTileWaves * 64), lds, be->stream, p, q, stats, tiles, splits, dst);
     return CG_OK;
 }
 template <int HPW> int run_tiles(cg_backend *be, const AttentionPlan &p, const float *q, float2 *stats, uint32_t splits, float *dst) {
@@ -384,7 +384,7 @@ int launch_attention_tiles(cg_backend *be, const AttentionPlan &p, const float *
              : p.heads <= 16 ? run_tiles<2>(be, p, q, stats, splits, dst)
                              : run_tiles<4>(be, p, q, stats, splits, dst);
     if (!rc && splits > 1)
-        hipLaunchKernelGGL(attention_parts_kernel, dim3((uint32_t)((n + 1023) / 1024)), dim3(256), 0, be->stream, dst, splits, n, p.out);
+        launch_kernel(attention_parts_kernel, dim3((uint32_t)((n + 1023) / 1024)), dim3(256), 0, be->stream, dst, splits, n, p.out);
     if (mem) be->pool.free(mem, mem_cls);
     if (parts) be->pool.free(parts, parts_cls);
     if (rc) return rc;

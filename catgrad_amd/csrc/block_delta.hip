@@ -694,7 +694,7 @@ template <int TPW, int CT> int scan(cg_backend *be, const DeltaPlan &p, const Ch
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&delta_scan_kernel<TPW, CT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute");
     }
-    hipLaunchKernelGGL((delta_scan_kernel<TPW, CT>), dim3((p.vdim + 16 * CT - 1) / (16 * CT), p.heads, p.B), dim3(CT * 256), lds, be->stream, p, a, state, p.out);
+    launch_kernel((delta_scan_kernel<TPW, CT>), dim3((p.vdim + 16 * CT - 1) / (16 * CT), p.heads, p.B), dim3(CT * 256), lds, be->stream, p, a, state, p.out);
     return CG_OK;
 }
 template <int CT> int scan(cg_backend *be, const DeltaPlan &p, const ChunkArrays &a, const float *state) {
@@ -721,9 +721,9 @@ int launch_channel_delta(cg_backend *be, const DeltaPlan &p) {
         const bool direct = p.S == 1 && p.state && p.taps == 4 && 2 * p.dim + p.vdim <= kStepThreads && p.dim <= kStepThreads / 4 && p.vdim <= kStepThreads / 4 && pieces(p.decay_w, p.decay_rank, p.decay) &&
                             pieces(p.gate_w, p.gate_rank, p.gate);
 #define CG_STEP(R, DIRECT)                                                                                                                \
-    if (DIRECT) hipLaunchKernelGGL((delta_step_kernel<R, 4, DIRECT>), grid, dim3(kStepThreads), 0, be->stream, p, lanes);                \
-    else if (p.taps == 4) hipLaunchKernelGGL((delta_step_kernel<R, 4, false>), grid, dim3(kStepThreads), 0, be->stream, p, lanes);       \
-    else hipLaunchKernelGGL((delta_step_kernel<R, 0, false>), grid, dim3(kStepThreads), 0, be->stream, p, lanes)
+    if (DIRECT) launch_kernel((delta_step_kernel<R, 4, DIRECT>), grid, dim3(kStepThreads), 0, be->stream, p, lanes);                \
+    else if (p.taps == 4) launch_kernel((delta_step_kernel<R, 4, false>), grid, dim3(kStepThreads), 0, be->stream, p, lanes);       \
+    else launch_kernel((delta_step_kernel<R, 0, false>), grid, dim3(kStepThreads), 0, be->stream, p, lanes)
         if (direct && held <= 4) { CG_STEP(4, true); }
         else if (direct && held <= 16) { CG_STEP(16, true); }
         else if (direct) { CG_STEP(32, true); } // (128 rows by four groups)
@@ -756,13 +756,13 @@ int launch_channel_delta(cg_backend *be, const DeltaPlan &p) {
         ProfScope prof(be, CG_K_RECURRENCE, flop * tokens * p.B);
         const size_t lds = (size_t)3 * kChunk * (a.dp + 4) * 4;
         const dim3 grid(a.chunks, p.heads, p.B);
-        if (p.taps == 4) hipLaunchKernelGGL((delta_chunk_kernel<4>), grid, dim3(kThreads), lds, be->stream, p, a, decay);
-        else hipLaunchKernelGGL((delta_chunk_kernel<0>), grid, dim3(kThreads), lds, be->stream, p, a, decay);
+        if (p.taps == 4) launch_kernel((delta_chunk_kernel<4>), grid, dim3(kThreads), lds, be->stream, p, a, decay);
+        else launch_kernel((delta_chunk_kernel<0>), grid, dim3(kThreads), lds, be->stream, p, a, decay);
         const float *state = c0 ? p.state_out : p.state;
         if (int rc = wide ? scan<2>(be, p, a, state) : scan<1>(be, p, a, state)) return rc;
     }
     const uint64_t n = (uint64_t)rows * p.heads;
-    hipLaunchKernelGGL(delta_finish_kernel, dim3((uint32_t)((n + kWaves - 1) / kWaves)), dim3(kThreads), 0, be->stream, p, gate, p.out, n);
+    launch_kernel(delta_finish_kernel, dim3((uint32_t)((n + kWaves - 1) / kWaves)), dim3(kThreads), 0, be->stream, p, gate, p.out, n);
     return launched("channel_delta");
 }
 

@@ -484,12 +484,12 @@ template <bool FIRST> int launch_tiles(cg_backend *be, const ExpertTileArgs &a, 
     const dim3 grid(tiles * a.tiles_n);
     const uint32_t tm = low ? 64 : 128;
     const size_t lds = bf16 ? (size_t)kStages * (tm + kTileN) * 64 : split::lds_bytes(tm, kTileN);
-    if (bf16 && low) hipLaunchKernelGGL((expert_tile_kernel<FIRST, 1>), grid, dim3(kThreads), lds, be->stream, a);
-    else if (bf16) hipLaunchKernelGGL((expert_tile_kernel<FIRST, 2>), grid, dim3(kThreads), lds, be->stream, a);
-    else if (low && far) hipLaunchKernelGGL((expert_split_kernel<FIRST, 2, 1, true>), grid, dim3(kThreads), lds, be->stream, a);
-    else if (low) hipLaunchKernelGGL((expert_split_kernel<FIRST, 2, 1, false>), grid, dim3(kThreads), lds, be->stream, a);
-    else if (far) hipLaunchKernelGGL((expert_split_kernel<FIRST, 2, 2, true>), grid, dim3(kThreads), lds, be->stream, a);
-    else hipLaunchKernelGGL((expert_split_kernel<FIRST, 2, 2, false>), grid, dim3(kThreads), lds, be->stream, a);
+    if (bf16 && low) launch_kernel((expert_tile_kernel<FIRST, 1>), grid, dim3(kThreads), lds, be->stream, a);
+    else if (bf16) launch_kernel((expert_tile_kernel<FIRST, 2>), grid, dim3(kThreads), lds, be->stream, a);
+    else if (low && far) launch_kernel((expert_split_kernel<FIRST, 2, 1, true>), grid, dim3(kThreads), lds, be->stream, a);
+    else if (low) launch_kernel((expert_split_kernel<FIRST, 2, 1, false>), grid, dim3(kThreads), lds, be->stream, a);
+    else if (far) launch_kernel((expert_split_kernel<FIRST, 2, 2, true>), grid, dim3(kThreads), lds, be->stream, a);
+    else launch_kernel((expert_split_kernel<FIRST, 2, 2, false>), grid, dim3(kThreads), lds, be->stream, a);
     return launched("expert_tiles");
 }
 
@@ -504,7 +504,7 @@ int launch_experts_first(cg_backend *be, const ExpertsPlan &p, float *hidden, ui
     const uint32_t per = std::max(1u, (uint32_t)((uint64_t)pairs * p.ff / ((uint64_t)be->compute_units * 8 * kWaves)));
     const uint32_t per_wave = std::min(per, 8u);
     const size_t lds = route_bytes(p);
-    hipStream_t s = be->stream;
+    LaunchQueue &s = be->stream;
     for (uint32_t first = 0; first < p.rows;) { // (the grid's y extent)
         const uint32_t n = std::min(p.rows - first, std::max(1u, 65535 / p.top));
         ExpertsPlan q = p;
@@ -515,7 +515,7 @@ int launch_experts_first(cg_backend *be, const ExpertsPlan &p, float *hidden, ui
         uint32_t *ch = chosen + (uint64_t)first * p.top;
         const dim3 grid((p.ff + kWaves * per_wave - 1) / (kWaves * per_wave), n * p.top);
         const uint32_t steps = (p.width + 64 * (bf16 ? 8 : 4) - 1) / (64 * (bf16 ? 8 : 4));
-#define CG_FIRST(BF, VE, ST) hipLaunchKernelGGL((expert_first_kernel<BF, VE, ST>), grid, dim3(kThreads), lds, s, q, per_wave, hid, ch)
+#define CG_FIRST(BF, VE, ST) launch_kernel((expert_first_kernel<BF, VE, ST>), grid, dim3(kThreads), lds, s, q, per_wave, hid, ch)
 #define CG_FIRST_ST(BF)                        \
     if (!vec) CG_FIRST(BF, false, 1);          \
     else if (steps <= 1) CG_FIRST(BF, true, 1); \
@@ -547,8 +547,8 @@ int launch_experts_second(cg_backend *be, const ExpertsPlan &p, const float *hid
     const dim3 grid((p.width + per - 1) / per, p.rows);
 #define CG_SECOND(BF, VE)                                                                                                                                            \
     {                                                                                                                                                                \
-        if (two) hipLaunchKernelGGL((expert_second_kernel<BF, VE, VE ? 2 : 1>), grid, dim3(kThreads), 0, be->stream, p, hidden, chosen, x, y, w ? *w : none, scale, out); \
-        else hipLaunchKernelGGL((expert_second_kernel<BF, VE, 1>), grid, dim3(kThreads), 0, be->stream, p, hidden, chosen, x, y, w ? *w : none, scale, out);           \
+        if (two) launch_kernel((expert_second_kernel<BF, VE, VE ? 2 : 1>), grid, dim3(kThreads), 0, be->stream, p, hidden, chosen, x, y, w ? *w : none, scale, out); \
+        else launch_kernel((expert_second_kernel<BF, VE, 1>), grid, dim3(kThreads), 0, be->stream, p, hidden, chosen, x, y, w ? *w : none, scale, out);           \
     }
     if (bf16 && vec) CG_SECOND(true, true)
     else if (bf16) CG_SECOND(true, false)
@@ -574,7 +574,7 @@ int launch_experts(cg_backend *be, const ExpertsPlan &p, float *y, int *y_fmt) {
         ProfScope prof(be, CG_K_GEMM_SKINNY, first_bytes(p, n) / 2);
         for (uint64_t at = 0; at < n; at += 65535) {
             const dim3 grid((p.width + kWaves - 1) / kWaves, (uint32_t)std::min<uint64_t>(n - at, 65535));
-#define CG_SLOTS(BF, VE) hipLaunchKernelGGL((expert_second_slots_kernel<BF, VE>), grid, dim3(kThreads), 0, be->stream, p, hidden + at * p.ff, chosen + at, y + at * p.width)
+#define CG_SLOTS(BF, VE) launch_kernel((expert_second_slots_kernel<BF, VE>), grid, dim3(kThreads), 0, be->stream, p, hidden + at * p.ff, chosen + at, y + at * p.width)
             if (bf16 && vec) CG_SLOTS(true, true);
             else if (bf16) CG_SLOTS(true, false);
             else if (vec) CG_SLOTS(false, true);
@@ -599,10 +599,10 @@ int launch_experts(cg_backend *be, const ExpertsPlan &p, float *y, int *y_fmt) {
     uint32_t *list = reinterpret_cast<uint32_t *>(weights + n), *count = list + n;
     {
         ProfScope prof(be, CG_K_GATHER, 4.0 * p.rows * p.experts + 20.0 * n);
-        hipLaunchKernelGGL(clear_kernel, dim3((p.experts + kThreads - 1) / kThreads), dim3(kThreads), 0, be->stream, count, p.experts);
+        launch_kernel(clear_kernel, dim3((p.experts + kThreads - 1) / kThreads), dim3(kThreads), 0, be->stream, count, p.experts);
         const uint32_t run = std::min(kMaxRun, (uint32_t)kWaves * std::max(1u, p.rows / (4 * be->compute_units * kWaves)));
-        hipLaunchKernelGGL(route_kernel, dim3((p.rows + run - 1) / run), dim3(kThreads), many_route_bytes(p), be->stream, p, run, routed, weights, count);
-        hipLaunchKernelGGL(route_lists_kernel, dim3((uint32_t)((n + kThreads - 1) / kThreads)), dim3(kThreads), (size_t)(p.experts + 1) * 8, be->stream, p.experts, (uint32_t)n, tm,
+        launch_kernel(route_kernel, dim3((p.rows + run - 1) / run), dim3(kThreads), many_route_bytes(p), be->stream, p, run, routed, weights, count);
+        launch_kernel(route_lists_kernel, dim3((uint32_t)((n + kThreads - 1) / kThreads)), dim3(kThreads), (size_t)(p.experts + 1) * 8, be->stream, p.experts, (uint32_t)n, tm,
                            max_tiles, routed, count, list, tiles);
         if (int rc = launched("route")) return rc;
     }

@@ -411,7 +411,7 @@ int launched(const char *what) {
 
 int launch_pair_embedding(cg_backend *be, const PairEmbeddingPlan &p) {
     ProfScope prof(be, CG_K_GATHER, (double)p.B * p.S * p.width * (4.0 + 2.0 * (p.table.fmt == kFmtBF16 ? 2.0 : 4.0)));
-    hipLaunchKernelGGL(pair_embedding_kernel, dim3(p.B * p.S), dim3(kThreads), 0, be->stream, p, be->fault_dev);
+    launch_kernel(pair_embedding_kernel, dim3(p.B * p.S), dim3(kThreads), 0, be->stream, p, be->fault_dev);
     return launched("pair_embedding");
 }
 
@@ -434,15 +434,15 @@ int launch_conv_rows(cg_backend *be, ConvRowsPlan p) {
     const uint32_t runs = (p.S + p.run - 1) / p.run;
     const dim3 grid(p.B * runs, p.groups * split);
     const size_t lds = (p.run + past) * 4;
-    hipStream_t s = be->stream;
+    LaunchQueue &s = be->stream;
 #define CG_CONV(T)                                                                                       \
-    if (vec) hipLaunchKernelGGL((conv_rows_kernel<4, T>), grid, dim3(kThreads), lds, s, p, split);        \
-    else hipLaunchKernelGGL((conv_rows_kernel<1, T>), grid, dim3(kThreads), lds, s, p, split)
+    if (vec) launch_kernel((conv_rows_kernel<4, T>), grid, dim3(kThreads), lds, s, p, split);        \
+    else launch_kernel((conv_rows_kernel<1, T>), grid, dim3(kThreads), lds, s, p, split)
     if (p.taps <= 1) { CG_CONV(1); }
     else if (p.taps <= 2) { CG_CONV(2); }
     else if (p.taps <= 3) { CG_CONV(3); }
     else if (p.taps == 4 && vec && p.run == 1 && taps)
-        hipLaunchKernelGGL(conv_token_kernel, grid, dim3(kThreads), 0, s, p, split);
+        launch_kernel(conv_token_kernel, grid, dim3(kThreads), 0, s, p, split);
     else if (p.taps <= 4) { CG_CONV(4); }
     else if (p.taps <= 8) { CG_CONV(8); }
     else if (p.taps <= kMaxTaps) { CG_CONV(kMaxTaps); }
@@ -454,7 +454,7 @@ int launch_conv_rows(cg_backend *be, ConvRowsPlan p) {
 int launch_side_gate(cg_backend *be, float *g, const Tokens &ids, const Table &table, uint32_t vocab, uint32_t first, uint32_t dim, uint32_t rows) {
     ProfScope prof(be, CG_K_ELEMENTWISE, 12.0 * rows * dim);
     const uint64_t n = (uint64_t)rows * dim;
-    hipLaunchKernelGGL(side_gate_kernel, dim3((uint32_t)((n + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream, g, ids, table, vocab, first, dim, rows,
+    launch_kernel(side_gate_kernel, dim3((uint32_t)((n + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream, g, ids, table, vocab, first, dim, rows,
                        be->fault_dev);
     return launched("side_gate");
 }
@@ -465,7 +465,7 @@ int launch_side_first(cg_backend *be, const Rows &x, uint32_t rows, const Weight
     const bool vec = w.k % vw == 0 && w.pitch % vw == 0 && aligned16(w.p) && x.pitch % 4 == 0 && aligned16(x.p);
     ProfScope prof(be, CG_K_GEMM_SKINNY, (double)w.n * w.k * (bf16 ? 2.0 : 4.0) + 4.0 * rows * ((double)w.k + w.n));
     const dim3 grid((w.n + kWaves - 1) / kWaves, rows);
-#define CG_FIRST(BF, VE) hipLaunchKernelGGL((side_first_kernel<BF, VE>), grid, dim3(kThreads), 0, be->stream, x, w, ids, table, vocab, first, g, be->fault_dev)
+#define CG_FIRST(BF, VE) launch_kernel((side_first_kernel<BF, VE>), grid, dim3(kThreads), 0, be->stream, x, w, ids, table, vocab, first, g, be->fault_dev)
     if (bf16 && vec) CG_FIRST(true, true);
     else if (bf16) CG_FIRST(true, false);
     else if (vec) CG_FIRST(false, true);
@@ -476,7 +476,7 @@ int launch_side_first(cg_backend *be, const Rows &x, uint32_t rows, const Weight
 
 template <bool BF16, int LANES> static int side_second(cg_backend *be, const Rows &x, const float *g, uint32_t rows, const Weight &w, const float *norm, float eps, float scale, float *out) {
     const uint32_t work = (w.n + kSideThreads / LANES - 1) / (kSideThreads / LANES);
-#define CG_SECOND(WK) hipLaunchKernelGGL((side_second_kernel<BF16, LANES, WK>), dim3(rows), dim3(kSideThreads), 0, be->stream, x, g, w, norm, eps, scale, out)
+#define CG_SECOND(WK) launch_kernel((side_second_kernel<BF16, LANES, WK>), dim3(rows), dim3(kSideThreads), 0, be->stream, x, g, w, norm, eps, scale, out)
     if (work <= 4) CG_SECOND(4);
     else if (work <= 8) CG_SECOND(8);
     else if (work <= 16) CG_SECOND(16);
@@ -504,8 +504,8 @@ int launch_side_second(cg_backend *be, const Rows &x, const float *g, uint32_t r
 int launch_side_sum(cg_backend *be, const Rows &x, const float *y, const float *norm, uint32_t rows, uint32_t width, float eps, float scale, float *out) {
     ProfScope prof(be, CG_K_REDUCE, 12.0 * rows * width);
     const bool vec = width % 4 == 0 && x.pitch % 4 == 0 && aligned16(x.p) && aligned16(y) && aligned16(norm) && aligned16(out);
-    if (vec) hipLaunchKernelGGL((side_sum_kernel<4>), dim3(rows), dim3(kThreads), 0, be->stream, x, y, norm, width, eps, scale, out);
-    else hipLaunchKernelGGL((side_sum_kernel<1>), dim3(rows), dim3(kThreads), 0, be->stream, x, y, norm, width, eps, scale, out);
+    if (vec) launch_kernel((side_sum_kernel<4>), dim3(rows), dim3(kThreads), 0, be->stream, x, y, norm, width, eps, scale, out);
+    else launch_kernel((side_sum_kernel<1>), dim3(rows), dim3(kThreads), 0, be->stream, x, y, norm, width, eps, scale, out);
     return launched("side_sum");
 }
 

@@ -283,8 +283,8 @@ template <int FMT, int OUT, int RT, bool WHOLE> __global__ __launch_bounds__(64 
 
 template <int FMT, int OUT, int RT> void launch_thin(cg_backend *be, const TileArgs &a) {
     const dim3 grid((a.N + 15) / 16, (a.M + 16 * RT - 1) / (16 * RT));
-    if (a.K % kTurnBytes == 0) hipLaunchKernelGGL((narrow_thin_kernel<FMT, OUT, RT, true>), grid, dim3(64 * kThinWaves), 0, be->stream, a);
-    else hipLaunchKernelGGL((narrow_thin_kernel<FMT, OUT, RT, false>), grid, dim3(64 * kThinWaves), 0, be->stream, a);
+    if (a.K % kTurnBytes == 0) launch_kernel((narrow_thin_kernel<FMT, OUT, RT, true>), grid, dim3(64 * kThinWaves), 0, be->stream, a);
+    else launch_kernel((narrow_thin_kernel<FMT, OUT, RT, false>), grid, dim3(64 * kThinWaves), 0, be->stream, a);
 }
 
 int launched(const char *what) {
@@ -312,9 +312,10 @@ template <int FMT, int OUT> int run_tiles(cg_backend *be, TileArgs a) {
         const double us = start + stage * stages * std::max(1.0, share * rounds) + (p > 1 ? 0.9 + 0.15 * p + 1.44e-6 * p * mn : 0.0);
         if (p == 1 || us < best) splits = p, best = us;
     }
-    // Few rows, or little work: without a second launch, where that is faster.  Fitted to 136 shapes of 9 to 1500 rows, each format and both
-    // heights timed: one row block while a compute unit has one workgroup, two beyond.
+    // Few rows, or little work: without a second launch, where that is faster by a tenth.  Fitted to 136 shapes of 9 to 1500 rows, each
+    // format and both heights timed, most within a tenth: one row block while a compute unit has one workgroup, two beyond.
     int high = 0;
+    best *= 0.9;
     for (int rt = 1; rt <= 2; rt++) {
         const uint64_t rows = (a.M + 16 * rt - 1) / (16 * rt);
         const double rounds = (double)(rows * ((a.N + 15) / 16)) / be->compute_units, turns = a.K / (double)(kThinWaves * kTurnBytes);
@@ -340,14 +341,14 @@ template <int FMT, int OUT> int run_tiles(cg_backend *be, TileArgs a) {
     const dim3 grid((uint32_t)tiles, splits);
     const size_t lds = (size_t)kStages * (tm + kTileN) * kStageBytes;
     if (splits > 1) {
-        if (low) hipLaunchKernelGGL((narrow_tile_kernel<FMT, kFmtWords, 1>), grid, dim3(kThreads), lds, be->stream, a);
-        else hipLaunchKernelGGL((narrow_tile_kernel<FMT, kFmtWords, 2>), grid, dim3(kThreads), lds, be->stream, a);
-        hipLaunchKernelGGL((sum_parts_kernel<OUT>), dim3((uint32_t)((mn / 4 + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream,
+        if (low) launch_kernel((narrow_tile_kernel<FMT, kFmtWords, 1>), grid, dim3(kThreads), lds, be->stream, a);
+        else launch_kernel((narrow_tile_kernel<FMT, kFmtWords, 2>), grid, dim3(kThreads), lds, be->stream, a);
+        launch_kernel((sum_parts_kernel<OUT>), dim3((uint32_t)((mn / 4 + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream,
                            static_cast<const float4v *>(parts), y, splits, mn / 4, a.N / 4, ld == a.N ? a.N / 4 : ld / 4);
         be->pool.free(parts, cls); // stream-ordered
     } else {
-        if (low) hipLaunchKernelGGL((narrow_tile_kernel<FMT, OUT, 1>), grid, dim3(kThreads), lds, be->stream, a);
-        else hipLaunchKernelGGL((narrow_tile_kernel<FMT, OUT, 2>), grid, dim3(kThreads), lds, be->stream, a);
+        if (low) launch_kernel((narrow_tile_kernel<FMT, OUT, 1>), grid, dim3(kThreads), lds, be->stream, a);
+        else launch_kernel((narrow_tile_kernel<FMT, OUT, 2>), grid, dim3(kThreads), lds, be->stream, a);
     }
     return launched("narrow_tiles");
 }

@@ -738,7 +738,7 @@ int few_rows_linear(cg_backend *be, const ProductInput &in, uint32_t rows, const
     const uint32_t pitch = staged_pitch(in.k);
     const size_t bytes = (size_t)M * pitch * 4;
     if (int rc = allow_lds(few_rows_linear_kernel<M, NC, BF16, VEC>, bytes)) return rc;
-    hipLaunchKernelGGL((few_rows_linear_kernel<M, NC, BF16, VEC>), dim3((w.n + kWaves * NC - 1) / (kWaves * NC)), dim3(kThreads), bytes, be->stream, in, rows, w,
+    launch_kernel((few_rows_linear_kernel<M, NC, BF16, VEC>), dim3((w.n + kWaves * NC - 1) / (kWaves * NC)), dim3(kThreads), bytes, be->stream, in, rows, w,
                        pitch, bias, scale, out);
     return CG_OK;
 }
@@ -748,7 +748,7 @@ int few_rows_residual(cg_backend *be, const Rows &x, const ResidualBranch *br, u
     const uint32_t p0 = staged_pitch(br[0].in.k), p1 = NB > 1 ? staged_pitch(br[1].in.k) : 0;
     const size_t bytes = (size_t)M * (p0 + p1) * 4;
     if (int rc = allow_lds(few_rows_residual_kernel<M, BF16, VEC, NB>, bytes)) return rc;
-    hipLaunchKernelGGL((few_rows_residual_kernel<M, BF16, VEC, NB>), dim3((width + kWaves - 1) / kWaves), dim3(kThreads), bytes, be->stream, x, br[0],
+    launch_kernel((few_rows_residual_kernel<M, BF16, VEC, NB>), dim3((width + kWaves - 1) / kWaves), dim3(kThreads), bytes, be->stream, x, br[0],
                        br[NB > 1 ? 1 : 0], rows, width, p0, p1, out);
     return CG_OK;
 }
@@ -771,7 +771,7 @@ template <bool BF16, int STEPS, int WAVES>
 static void launch_four_rows(cg_backend *be, const ProductInput &in, uint32_t rows, const Weight &w, const float *bias, float scale, float *out) {
     uint32_t iters;
     const uint32_t blocks = column_groups(be, w, &iters);
-    hipLaunchKernelGGL((four_rows_linear_kernel<BF16, STEPS, WAVES>), dim3(blocks), dim3(WAVES * 64), 0, be->stream, in, rows, w, iters, bias, scale, out);
+    launch_kernel((four_rows_linear_kernel<BF16, STEPS, WAVES>), dim3(blocks), dim3(WAVES * 64), 0, be->stream, in, rows, w, iters, bias, scale, out);
 }
 
 int launch_few_rows_linear(cg_backend *be, const ProductInput &in, uint32_t rows, const Weight &w, const float *bias, float scale, float *out) {
@@ -817,7 +817,7 @@ int launch_few_rows_linear(cg_backend *be, const ProductInput &in, uint32_t rows
 
 template <bool BF16, int STEPS, int WAVES> static void launch_four_rows2(cg_backend *be, FourRowsJob (&j)[2], uint32_t rows) {
     const uint32_t b0 = column_groups(be, j[0].w, &j[0].iters), b1 = column_groups(be, j[1].w, &j[1].iters);
-    hipLaunchKernelGGL((four_rows_linear2_kernel<BF16, STEPS, WAVES>), dim3(b0 + b1), dim3(WAVES * 64), 0, be->stream, j[0], j[1], b0, rows);
+    launch_kernel((four_rows_linear2_kernel<BF16, STEPS, WAVES>), dim3(b0 + b1), dim3(WAVES * 64), 0, be->stream, j[0], j[1], b0, rows);
 }
 
 int launch_few_rows_linear2(cg_backend *be, const ProductInput (&in)[2], uint32_t rows, const Weight (&w)[2], float *const (&out)[2]) {
@@ -848,11 +848,11 @@ template <bool BF16, int NG> static bool four_rows_residual(cg_backend *be, cons
     const dim3 grid((width + 4 * NG - 1) / (4 * NG)), block(WAVES * 64);
     const bool p0 = br[0].in.poly != nullptr, p1 = n > 1 && br[1].in.poly != nullptr;
     const ResidualBranch &b1 = br[n > 1 ? 1 : 0];
-    hipStream_t s = be->stream;
-    if (n == 2 && !p0 && p1) hipLaunchKernelGGL((four_rows_residual_kernel<BF16, 2, NG, WAVES, false, true>), grid, block, 0, s, x, br[0], b1, rows, width, out);
-    else if (n == 2 && !p0 && !p1) hipLaunchKernelGGL((four_rows_residual_kernel<BF16, 2, NG, WAVES, false, false>), grid, block, 0, s, x, br[0], b1, rows, width, out);
-    else if (n == 1 && p0) hipLaunchKernelGGL((four_rows_residual_kernel<BF16, 1, NG, WAVES, true, false>), grid, block, 0, s, x, br[0], b1, rows, width, out);
-    else if (n == 1) hipLaunchKernelGGL((four_rows_residual_kernel<BF16, 1, NG, WAVES, false, false>), grid, block, 0, s, x, br[0], b1, rows, width, out);
+    LaunchQueue &s = be->stream;
+    if (n == 2 && !p0 && p1) launch_kernel((four_rows_residual_kernel<BF16, 2, NG, WAVES, false, true>), grid, block, 0, s, x, br[0], b1, rows, width, out);
+    else if (n == 2 && !p0 && !p1) launch_kernel((four_rows_residual_kernel<BF16, 2, NG, WAVES, false, false>), grid, block, 0, s, x, br[0], b1, rows, width, out);
+    else if (n == 1 && p0) launch_kernel((four_rows_residual_kernel<BF16, 1, NG, WAVES, true, false>), grid, block, 0, s, x, br[0], b1, rows, width, out);
+    else if (n == 1) launch_kernel((four_rows_residual_kernel<BF16, 1, NG, WAVES, false, false>), grid, block, 0, s, x, br[0], b1, rows, width, out);
     else return false;
     return true;
 }
@@ -919,14 +919,14 @@ int launch_product_input(cg_backend *be, const ProductInput &in, uint32_t rows, 
     const int f = fmt == kFmtBF16 ? 2 : round_bf16 ? 1 : 0;
     const bool vec = !in.x2.p && in.k % 4 == 0 && in.x.pitch % 4 == 0 && aligned16(in.x.p) && in.k <= 4 * kThreads * 16;
     const int trips = (int)((in.k + 4 * kThreads - 1) / (4 * kThreads));
-    hipStream_t s = be->stream;
+    LaunchQueue &s = be->stream;
 #define CG_IN(F)                                                                                                                       \
-    if (!vec) hipLaunchKernelGGL((product_input_kernel<F>), dim3(rows), dim3(kThreads), 0, s, in, dst);                                 \
-    else if (trips <= 1) hipLaunchKernelGGL((product_input_vec_kernel<F, 1>), dim3(rows), dim3(kThreads), 0, s, in, dst);               \
-    else if (trips <= 2) hipLaunchKernelGGL((product_input_vec_kernel<F, 2>), dim3(rows), dim3(kThreads), 0, s, in, dst);               \
-    else if (trips <= 4) hipLaunchKernelGGL((product_input_vec_kernel<F, 4>), dim3(rows), dim3(kThreads), 0, s, in, dst);               \
-    else if (trips <= 8) hipLaunchKernelGGL((product_input_vec_kernel<F, 8>), dim3(rows), dim3(kThreads), 0, s, in, dst);               \
-    else hipLaunchKernelGGL((product_input_vec_kernel<F, 16>), dim3(rows), dim3(kThreads), 0, s, in, dst)
+    if (!vec) launch_kernel((product_input_kernel<F>), dim3(rows), dim3(kThreads), 0, s, in, dst);                                 \
+    else if (trips <= 1) launch_kernel((product_input_vec_kernel<F, 1>), dim3(rows), dim3(kThreads), 0, s, in, dst);               \
+    else if (trips <= 2) launch_kernel((product_input_vec_kernel<F, 2>), dim3(rows), dim3(kThreads), 0, s, in, dst);               \
+    else if (trips <= 4) launch_kernel((product_input_vec_kernel<F, 4>), dim3(rows), dim3(kThreads), 0, s, in, dst);               \
+    else if (trips <= 8) launch_kernel((product_input_vec_kernel<F, 8>), dim3(rows), dim3(kThreads), 0, s, in, dst);               \
+    else launch_kernel((product_input_vec_kernel<F, 16>), dim3(rows), dim3(kThreads), 0, s, in, dst)
     if (f == 0) { CG_IN(0); }
     else if (f == 1) { CG_IN(1); }
     else { CG_IN(2); }
@@ -938,7 +938,7 @@ int launch_affine_rows(cg_backend *be, float *y, uint32_t rows, uint32_t n, cons
     for (uint32_t r0 = 0; r0 < rows; r0 += 65535) { // (the grid's y extent)
         const uint32_t nr = rows - r0 < 65535 ? rows - r0 : 65535;
         ProfScope prof(be, CG_K_ELEMENTWISE, 8.0 * nr * n);
-        hipLaunchKernelGGL(affine_rows_kernel, dim3((n + kThreads - 1) / kThreads, nr), dim3(kThreads), 0, be->stream, y + (int64_t)r0 * n, n, bias, scale);
+        launch_kernel(affine_rows_kernel, dim3((n + kThreads - 1) / kThreads, nr), dim3(kThreads), 0, be->stream, y + (int64_t)r0 * n, n, bias, scale);
     }
     return launched("affine_rows");
 }
@@ -965,8 +965,8 @@ int launch_gated_sum(cg_backend *be, const Rows &x, const GatedTerm *t, int n, u
         }
         const uint32_t per = kThreads * (vec ? 4 : 1);
         const dim3 grid((width + per - 1) / per, nr);
-        if (vec) hipLaunchKernelGGL((gated_sum_kernel<4>), grid, dim3(kThreads), 0, be->stream, a, out + (int64_t)r0 * width);
-        else hipLaunchKernelGGL((gated_sum_kernel<1>), grid, dim3(kThreads), 0, be->stream, a, out + (int64_t)r0 * width);
+        if (vec) launch_kernel((gated_sum_kernel<4>), grid, dim3(kThreads), 0, be->stream, a, out + (int64_t)r0 * width);
+        else launch_kernel((gated_sum_kernel<1>), grid, dim3(kThreads), 0, be->stream, a, out + (int64_t)r0 * width);
     }
     return launched("gated_sum");
 }

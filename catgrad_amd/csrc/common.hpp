@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../include/catgrad_hip.h"
+#include "launches.hpp"
 
 namespace cg {
 
@@ -41,6 +42,7 @@ class Pool {
     void free(void *ptr, size_t cls);
     void trim();
     void stats(size_t *in_use, size_t *cached);
+    LaunchQueue *launches = nullptr; // of the stream: blocks go back to the device behind all that was launched
     static size_t size_class(size_t bytes);
 
   private:
@@ -129,7 +131,7 @@ struct cg_backend {
     std::atomic<long> live_tensors{0}; // heap handles that name this backend (see alloc_tensor)
     bool owner_gone = false;           // cg_backend_destroy has been called; the last handle released tears down
     int device = 0;
-    hipStream_t stream = nullptr;
+    cg::LaunchQueue stream;
     cg::Pool pool;
     uint32_t *fault_host = nullptr; // pinned, device-visible
     uint32_t *fault_dev = nullptr;

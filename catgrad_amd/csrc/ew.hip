@@ -197,9 +197,9 @@ static int try_transpose_copy(cg_backend *be, const EwArgs &a) {
     }
     if (blocks == 0 || blocks > 0x7FFFFFFFull) return kDeclined;
     t.vec = vec ? 1u : 0u;
-    if (eb == 4) hipLaunchKernelGGL(transpose_copy_kernel<4>, dim3((uint32_t)blocks), dim3(kBlock), 0, be->stream, t);
-    else if (eb == 2) hipLaunchKernelGGL(transpose_copy_kernel<2>, dim3((uint32_t)blocks), dim3(kBlock), 0, be->stream, t);
-    else hipLaunchKernelGGL(transpose_copy_kernel<1>, dim3((uint32_t)blocks), dim3(kBlock), 0, be->stream, t);
+    if (eb == 4) launch_kernel(transpose_copy_kernel<4>, dim3((uint32_t)blocks), dim3(kBlock), 0, be->stream, t);
+    else if (eb == 2) launch_kernel(transpose_copy_kernel<2>, dim3((uint32_t)blocks), dim3(kBlock), 0, be->stream, t);
+    else launch_kernel(transpose_copy_kernel<1>, dim3((uint32_t)blocks), dim3(kBlock), 0, be->stream, t);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "transposing copy launch");
 }
@@ -250,20 +250,20 @@ int launch_small_upload(cg_backend *be, uint32_t *dst, const uint32_t *host_word
     UploadWords v;
     memset(&v, 0, sizeof v);
     memcpy(v.w, host_words, (size_t)n * 4);
-    hipLaunchKernelGGL(small_upload_kernel, dim3(1), dim3(kUploadWords), 0, be->stream, dst, v, n);
+    launch_kernel(small_upload_kernel, dim3(1), dim3(kUploadWords), 0, be->stream, dst, v, n);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "upload launch");
 }
 
 int launch_small_readback(cg_backend *be, const uint32_t *src, uint32_t n, uint32_t seq) {
-    hipLaunchKernelGGL(small_readback_kernel, dim3(1), dim3(n > 1024 ? 1024 : 256), 0, be->stream, src, n, be->rb_dev, seq);
+    launch_kernel(small_readback_kernel, dim3(1), dim3(n > 1024 ? 1024 : 256), 0, be->stream, src, n, be->rb_dev, seq);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "read-back launch");
 }
 
 int launch_arange(cg_backend *be, cg_tensor *out) {
     uint32_t n = (uint32_t)out->dims[0];
-    hipLaunchKernelGGL(arange_kernel, dim3((n + 255) / 256), dim3(256), 0, be->stream,
+    launch_kernel(arange_kernel, dim3((n + 255) / 256), dim3(256), 0, be->stream,
                        static_cast<uint32_t *>(out->buf->ptr), n);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "arange launch");
@@ -273,7 +273,7 @@ int launch_bf16_widen(cg_backend *be, const void *src, void *dst, uint64_t n) {
     if (n == 0) return CG_OK;
     const uint64_t groups = n / 8;
     const uint32_t blocks = (uint32_t)std::min<uint64_t>(std::max<uint64_t>((groups + kBlock - 1) / kBlock, 1), 8192);
-    hipLaunchKernelGGL(bf16_widen_kernel, dim3(blocks), dim3(kBlock), 0, be->stream, static_cast<const uint16_t *>(src),
+    launch_kernel(bf16_widen_kernel, dim3(blocks), dim3(kBlock), 0, be->stream, static_cast<const uint16_t *>(src),
                        static_cast<uint32_t *>(dst), n);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "bf16 widen launch");
@@ -292,7 +292,7 @@ template <bool BF16> __global__ __launch_bounds__(kBlock) void narrow16_kernel(c
 int launch_f16_widen(cg_backend *be, const void *src, void *dst, uint64_t n) {
     if (n == 0) return CG_OK;
     const uint32_t blocks = (uint32_t)std::min<uint64_t>((n + kBlock - 1) / kBlock, 16384);
-    hipLaunchKernelGGL(f16_widen_kernel, dim3(blocks), dim3(kBlock), 0, be->stream, static_cast<const uint16_t *>(src),
+    launch_kernel(f16_widen_kernel, dim3(blocks), dim3(kBlock), 0, be->stream, static_cast<const uint16_t *>(src),
                        static_cast<uint32_t *>(dst), n);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "f16 widen launch");
@@ -303,10 +303,10 @@ int launch_narrow16(cg_backend *be, cg_dtype dt, const void *src, void *dst, uin
     if (int frc = flush_deferred(be)) return frc;
     const uint32_t blocks = (uint32_t)std::min<uint64_t>((n + kBlock - 1) / kBlock, 16384);
     if (dt == CG_BF16)
-        hipLaunchKernelGGL((narrow16_kernel<true>), dim3(blocks), dim3(kBlock), 0, be->stream, static_cast<const uint32_t *>(src),
+        launch_kernel((narrow16_kernel<true>), dim3(blocks), dim3(kBlock), 0, be->stream, static_cast<const uint32_t *>(src),
                            static_cast<uint16_t *>(dst), n);
     else
-        hipLaunchKernelGGL((narrow16_kernel<false>), dim3(blocks), dim3(kBlock), 0, be->stream, static_cast<const uint32_t *>(src),
+        launch_kernel((narrow16_kernel<false>), dim3(blocks), dim3(kBlock), 0, be->stream, static_cast<const uint32_t *>(src),
                            static_cast<uint16_t *>(dst), n);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "16-bit narrowing launch");
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(kBlock) void narrow8_kernel(const uint32_t *src, ui
 int launch_f8_widen(cg_backend *be, const void *src, void *dst, uint64_t n) {
     if (n == 0) return CG_OK;
     const uint32_t blocks = (uint32_t)std::min<uint64_t>((n + kBlock - 1) / kBlock, 16384);
-    hipLaunchKernelGGL(f8_widen_kernel, dim3(blocks), dim3(kBlock), 0, be->stream, static_cast<const uint8_t *>(src),
+    launch_kernel(f8_widen_kernel, dim3(blocks), dim3(kBlock), 0, be->stream, static_cast<const uint8_t *>(src),
                        static_cast<uint32_t *>(dst), n);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "fp8 widen launch");
@@ -330,7 +330,7 @@ int launch_narrow8(cg_backend *be, const void *src, void *dst, uint64_t n) {
     if (n == 0) return CG_OK;
     if (int frc = flush_deferred(be)) return frc;
     const uint32_t blocks = (uint32_t)std::min<uint64_t>((n + kBlock - 1) / kBlock, 16384);
-    hipLaunchKernelGGL(narrow8_kernel, dim3(blocks), dim3(kBlock), 0, be->stream, static_cast<const uint32_t *>(src),
+    launch_kernel(narrow8_kernel, dim3(blocks), dim3(kBlock), 0, be->stream, static_cast<const uint32_t *>(src),
                        static_cast<uint8_t *>(dst), n);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "fp8 narrowing launch");
@@ -341,7 +341,7 @@ int launch_widen(cg_backend *be, int fmt, const void *src, void *dst, uint64_t n
 }
 
 int launch_fill_word(cg_backend *be, void *ptr, uint32_t bits) {
-    hipLaunchKernelGGL(fill_word_kernel, dim3(1), dim3(1), 0, be->stream, static_cast<uint32_t *>(ptr), bits);
+    launch_kernel(fill_word_kernel, dim3(1), dim3(1), 0, be->stream, static_cast<uint32_t *>(ptr), bits);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "fill launch");
 }
@@ -391,11 +391,11 @@ int launch_gather(cg_backend *be, const cg_tensor *x, int dim, const cg_tensor *
     dim3 grid((uint32_t)((total + kBlock - 1) / kBlock)), block(kBlock);
     ProfScope prof(be, CG_K_GATHER, 2.0 * distinct_bytes(out) + distinct_bytes(idx));
     if (vec4)
-        hipLaunchKernelGGL((gather_kernel<4>), grid, block, 0, be->stream, static_cast<const uint32_t *>(xp),
+        launch_kernel((gather_kernel<4>), grid, block, 0, be->stream, static_cast<const uint32_t *>(xp),
                            static_cast<const uint32_t *>(ip), istride, op, (uint32_t)D, (uint32_t)inner,
                            make_fastdiv(ipr), ipr, make_fastdiv((uint32_t)J), (uint32_t)J, total, be->fault_dev);
     else
-        hipLaunchKernelGGL((gather_kernel<1>), grid, block, 0, be->stream, static_cast<const uint32_t *>(xp),
+        launch_kernel((gather_kernel<1>), grid, block, 0, be->stream, static_cast<const uint32_t *>(xp),
                            static_cast<const uint32_t *>(ip), istride, op, (uint32_t)D, (uint32_t)inner,
                            make_fastdiv(ipr), ipr, make_fastdiv((uint32_t)J), (uint32_t)J, total, be->fault_dev);
     hipError_t e = hipGetLastError();

@@ -92,9 +92,9 @@ template <int VEC, int OP, bool F, int NIN> int launch_variants(cg_backend *be, 
     if (blocks == 0) return CG_OK;
     dim3 grid((uint32_t)blocks), block(kBlock);
     if (a.g.nouter == 0)
-        hipLaunchKernelGGL((ew_kernel<OP, F, NIN, VEC, true>), grid, block, 0, be->stream, a);
+        launch_kernel((ew_kernel<OP, F, NIN, VEC, true>), grid, block, 0, be->stream, a);
     else
-        hipLaunchKernelGGL((ew_kernel<OP, F, NIN, VEC, false>), grid, block, 0, be->stream, a);
+        launch_kernel((ew_kernel<OP, F, NIN, VEC, false>), grid, block, 0, be->stream, a);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "element-wise kernel launch");
 }

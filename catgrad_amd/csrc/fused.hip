@@ -108,7 +108,7 @@ __global__ __launch_bounds__(kBlock) void silu_mul_f8_kernel(const uint8_t *g, c
     }
 }
 // Both tensors and the result dense in one of the two formats, from 16-byte addresses; bf16: the constant is one.
-static bool launch_dense_silu_mul(const Pending &p, const FusedArgs &a, hipStream_t s) {
+static bool launch_dense_silu_mul(const Pending &p, const FusedArgs &a, LaunchQueue &s) {
     const bool bf16 = program_matches<MapSiluMulBF16>(p);
     if (!bf16 && !program_matches<MapSiluMulF8>(p)) return false;
     const uint32_t fmt = bf16 ? kFmtBF16 : kFmtF8;
@@ -118,10 +118,10 @@ static bool launch_dense_silu_mul(const Pending &p, const FusedArgs &a, hipStrea
     const uint64_t n = a.g.inner, per = bf16 ? kBlock * 8 : kBlock * 16 * kSiluTrips;
     const dim3 grid((uint32_t)((n + per - 1) / per));
     if (bf16)
-        hipLaunchKernelGGL(silu_mul_bf16_kernel, grid, dim3(kBlock), 0, s, reinterpret_cast<const uint16_t *>(a.leaf[0].ptr),
+        launch_kernel(silu_mul_bf16_kernel, grid, dim3(kBlock), 0, s, reinterpret_cast<const uint16_t *>(a.leaf[0].ptr),
                            reinterpret_cast<const uint16_t *>(a.leaf[2].ptr), reinterpret_cast<uint16_t *>(const_cast<char *>(a.out.ptr)), n);
     else
-        hipLaunchKernelGGL(silu_mul_f8_kernel, grid, dim3(kBlock), 0, s, reinterpret_cast<const uint8_t *>(a.leaf[0].ptr),
+        launch_kernel(silu_mul_f8_kernel, grid, dim3(kBlock), 0, s, reinterpret_cast<const uint8_t *>(a.leaf[0].ptr),
                            reinterpret_cast<const uint8_t *>(a.leaf[2].ptr), reinterpret_cast<uint8_t *>(const_cast<char *>(a.out.ptr)), n, a.leaf[1].ubits);
     return true;
 }
@@ -145,14 +145,14 @@ int launch_fused(cg_backend *be, const cg_tensor *out, const Pending &p) {
     be->programs_interpreted++;
     if (a.g.vec == 4) {
         if (full)
-            hipLaunchKernelGGL((fused_kernel<4, true>), grid, block, 0, be->stream, a);
+            launch_kernel((fused_kernel<4, true>), grid, block, 0, be->stream, a);
         else
-            hipLaunchKernelGGL((fused_kernel<4, false>), grid, block, 0, be->stream, a);
+            launch_kernel((fused_kernel<4, false>), grid, block, 0, be->stream, a);
     } else {
         if (full)
-            hipLaunchKernelGGL((fused_kernel<1, true>), grid, block, 0, be->stream, a);
+            launch_kernel((fused_kernel<1, true>), grid, block, 0, be->stream, a);
         else
-            hipLaunchKernelGGL((fused_kernel<1, false>), grid, block, 0, be->stream, a);
+            launch_kernel((fused_kernel<1, false>), grid, block, 0, be->stream, a);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "fused element-wise launch");
@@ -187,7 +187,7 @@ int launch_fused_group(cg_backend *be, const cg_tensor *const *outs, const Pendi
     g.n = (uint32_t)n;
     for (int i = 0; i < n; i++) trace_program(be, *ps[i], ps[i]->ninstr, "map (grouped)", outs[i]->dims, outs[i]->rank);
     ProfScope prof(be, CG_K_ELEMENTWISE, bytes);
-    hipLaunchKernelGGL(aot_map_group_kernel, dim3(blocks), dim3(kBlock), 0, be->stream, g);
+    launch_kernel(aot_map_group_kernel, dim3(blocks), dim3(kBlock), 0, be->stream, g);
     be->programs_compiled += n;
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "grouped element-wise launch");
@@ -218,9 +218,9 @@ int launch_fused_reduce(cg_backend *be, int kind, bool f32, const Pending &p, in
 #define CG_LAUNCH(VEC, TPR)                                                                                  \
     do {                                                                                                     \
         if (full)                                                                                            \
-            hipLaunchKernelGGL((fused_reduce_kernel<VEC, TPR, true>), grid, block, 0, be->stream, a, op, kind, f);  \
+            launch_kernel((fused_reduce_kernel<VEC, TPR, true>), grid, block, 0, be->stream, a, op, kind, f);  \
         else                                                                                                 \
-            hipLaunchKernelGGL((fused_reduce_kernel<VEC, TPR, false>), grid, block, 0, be->stream, a, op, kind, f); \
+            launch_kernel((fused_reduce_kernel<VEC, TPR, false>), grid, block, 0, be->stream, a, op, kind, f); \
     } while (0)
     if (a.g.vec == 4) {
         switch (tpr) {

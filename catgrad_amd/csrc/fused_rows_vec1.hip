@@ -3,7 +3,7 @@
 
 namespace cg {
 
-void launch_interpreted_rows1(const FusedArgs &a, uint32_t *rowout, int tpr, bool full, dim3 grid, hipStream_t s) {
+void launch_interpreted_rows1(const FusedArgs &a, uint32_t *rowout, int tpr, bool full, dim3 grid, LaunchQueue &s) {
     launch_interpreted_rows<1>(a, rowout, tpr, full, grid, s);
 }
 

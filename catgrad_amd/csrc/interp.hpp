@@ -57,12 +57,12 @@ struct FusedArgs {
 
 // A row program that has a kernel compiled for it (aot_rows.hip) is launched with it: true.  `tpr` is the
 // number of lanes per row, 16 / 64 / 256; `grid` the launch's workgroups of 256 / tpr rows each.
-bool launch_compiled_rows(const Pending &p, const FusedArgs &a, uint32_t *rowout, int tpr, dim3 grid, hipStream_t s);
+bool launch_compiled_rows(const Pending &p, const FusedArgs &a, uint32_t *rowout, int tpr, dim3 grid, LaunchQueue &s);
 
 // Any row program through the interpreter, at four elements or one per work item (fused_rows_vec4.hip,
 // fused_rows_vec1.hip): `tpr` lanes per row, 4 / 16 / 64 / 256; `full`: no lane of the grid is idle.
-void launch_interpreted_rows4(const FusedArgs &a, uint32_t *rowout, int tpr, bool full, dim3 grid, hipStream_t s);
-void launch_interpreted_rows1(const FusedArgs &a, uint32_t *rowout, int tpr, bool full, dim3 grid, hipStream_t s);
+void launch_interpreted_rows4(const FusedArgs &a, uint32_t *rowout, int tpr, bool full, dim3 grid, LaunchQueue &s);
+void launch_interpreted_rows1(const FusedArgs &a, uint32_t *rowout, int tpr, bool full, dim3 grid, LaunchQueue &s);
 
 namespace {
 
@@ -431,13 +431,13 @@ __global__ __launch_bounds__(kBlock) void fused_rows_kernel(const FusedArgs a, u
 }
 
 template <int VEC>
-void launch_interpreted_rows(const FusedArgs &a, uint32_t *rowout, int tpr, bool full, dim3 grid, hipStream_t s) {
+void launch_interpreted_rows(const FusedArgs &a, uint32_t *rowout, int tpr, bool full, dim3 grid, LaunchQueue &s) {
 #define CG_LAUNCH(TPR)                                                                                  \
     do {                                                                                                \
         if (full)                                                                                       \
-            hipLaunchKernelGGL((fused_rows_kernel<VEC, TPR, true>), grid, dim3(kBlock), 0, s, a, rowout);  \
+            launch_kernel((fused_rows_kernel<VEC, TPR, true>), grid, dim3(kBlock), 0, s, a, rowout);  \
         else                                                                                            \
-            hipLaunchKernelGGL((fused_rows_kernel<VEC, TPR, false>), grid, dim3(kBlock), 0, s, a, rowout); \
+            launch_kernel((fused_rows_kernel<VEC, TPR, false>), grid, dim3(kBlock), 0, s, a, rowout); \
     } while (0)
     switch (tpr) {
     case 4: CG_LAUNCH(4); break;

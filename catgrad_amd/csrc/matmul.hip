@@ -2150,7 +2150,7 @@ int launch_matmul_group(cg_backend *be, const cg_tensor *x, const cg_tensor *con
     g.n = (uint32_t)n;
     ProfScope prof(be, CG_K_GEMM_SKINNY, bytes);
     const bool eight = g.p[0].M > 4, deep = xreg_trips(g.p[0].K) == 8;
-    auto launch = [&](auto kernel, auto... args) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, be->stream, args...); };
+    auto launch = [&](auto kernel, auto... args) { launch_kernel(kernel, dim3(blocks), dim3(kThreads), 0, be->stream, args...); };
     xreg_either(g.p[0].K, xreg ? 8 : xreg_trips(g.p[0].K), [&](auto whole) { // (the problems of a group share k)
         constexpr bool W = decltype(whole)::value;
         if (xreg) launch(skinny_kt_mfma_xreg_group_kernel<W, 4, 2, 8>, g);
@@ -2163,11 +2163,11 @@ int launch_matmul_group(cg_backend *be, const cg_tensor *x, const cg_tensor *con
         else if (xreg1 && eight) launch(skinny_kt_mfma_xreg_group_kernel<W, 8, 1, 4>, g);
         else if (xreg1) launch(skinny_kt_mfma_xreg_group_kernel<W, 4, 1, 4>, g);
         else if (g.p[0].M <= 1)
-            hipLaunchKernelGGL((skinny_kt_wide_group_kernel<1>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
+            launch_kernel((skinny_kt_wide_group_kernel<1>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
         else if (g.p[0].M <= 4)
-            hipLaunchKernelGGL((skinny_kt_wide_group_kernel<4>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
+            launch_kernel((skinny_kt_wide_group_kernel<4>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
         else
-            hipLaunchKernelGGL((skinny_kt_wide_group_kernel<8>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
+            launch_kernel((skinny_kt_wide_group_kernel<8>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
     });
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "grouped matmul launch");
@@ -2238,7 +2238,7 @@ int launch_matmul_group_rope(cg_backend *be, const cg_tensor *x, const cg_tensor
         hf.first[hf.n] = heads;
         finish_heads = heads;
     }
-    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, be->stream, g, rg, nf ? *nf : none); };
+    auto launch = [&](auto kernel) { launch_kernel(kernel, dim3(blocks), dim3(kThreads), 0, be->stream, g, rg, nf ? *nf : none); };
     xreg_either(g.p[0].K, xreg_trips(g.p[0].K), [&](auto whole) { // (the problems of a group share k)
         constexpr bool W = decltype(whole)::value;
         if (g.p[0].M > 4) {
@@ -2255,7 +2255,7 @@ int launch_matmul_group_rope(cg_backend *be, const cg_tensor *x, const cg_tensor
     });
     if (by_head) {
         const uint32_t threads = (hf.M * 128 + 63) / 64 * 64;
-        hipLaunchKernelGGL(head_norm_rope_finish_kernel, dim3(finish_heads), dim3(threads), 0, be->stream, hf);
+        launch_kernel(head_norm_rope_finish_kernel, dim3(finish_heads), dim3(threads), 0, be->stream, hf);
         be->pool.free(tmp, tmp_cls); // stream-ordered: later users queue behind the finishing launch
     }
     hipError_t e = hipGetLastError();
@@ -2291,7 +2291,7 @@ int launch_matmul_gated(cg_backend *be, const cg_tensor *x, const cg_tensor *yg,
         memset(&none, 0, sizeof none);
         const uint32_t groups = (ag.N + 3) / 4, iters = xreg_cols_iters(groups);
         const dim3 cgrid((groups + iters - 1) / iters);
-        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, cgrid, dim3(kThreads), 0, be->stream, ag, au.B, one, iters, nf ? *nf : none); };
+        auto launch = [&](auto kernel) { launch_kernel(kernel, cgrid, dim3(kThreads), 0, be->stream, ag, au.B, one, iters, nf ? *nf : none); };
         xreg_either(ag.K, xreg_trips(ag.K), [&](auto whole) {
             constexpr bool W = decltype(whole)::value;
             if (eight) {
@@ -2305,7 +2305,7 @@ int launch_matmul_gated(cg_backend *be, const cg_tensor *x, const cg_tensor *yg,
             }
         });
     } else {
-        auto launch = [&](auto kernel, auto... more) { hipLaunchKernelGGL(kernel, ggrid, dim3(kThreads), 0, be->stream, ag, au.B, one, more...); };
+        auto launch = [&](auto kernel, auto... more) { launch_kernel(kernel, ggrid, dim3(kThreads), 0, be->stream, ag, au.B, one, more...); };
         xreg_either(ag.K, xreg_trips(ag.K), [&](auto whole) {
             constexpr bool W = decltype(whole)::value;
             if (eight) {
@@ -2359,8 +2359,8 @@ int launch_matmul_residual(cg_backend *be, const cg_tensor *x, const cg_tensor *
     dim3 grid((uint32_t)((a.N + 3) / 4));
     const int eight = eight_trips(be, a.M, a.N, a.K);
     const dim3 grid8((uint32_t)((a.N + 7) / 8));
-    auto launch8 = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid8, dim3(kEightThreads), 0, be->stream, a, r); };
-    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, be->stream, a, r); };
+    auto launch8 = [&](auto kernel) { launch_kernel(kernel, grid8, dim3(kEightThreads), 0, be->stream, a, r); };
+    auto launch = [&](auto kernel) { launch_kernel(kernel, grid, dim3(kThreads), 0, be->stream, a, r); };
     const bool rows8 = a.M > 4;
     if (eight == 16) launch8(skinny_kt_mfma_eight_residual_kernel<4, 16>);
     else if (eight == 8 && rows8) launch8(skinny_kt_mfma_eight_residual_kernel<8, 8>);
@@ -2377,11 +2377,11 @@ int launch_matmul_residual(cg_backend *be, const cg_tensor *x, const cg_tensor *
             else launch(skinny_kt_mfma_xreg_residual_kernel<W, 4, 4>);
         });
     } else if (a.M <= 1)
-        hipLaunchKernelGGL((skinny_kt_wide_residual_kernel<1>), grid, dim3(kThreads), 0, be->stream, a, r);
+        launch_kernel((skinny_kt_wide_residual_kernel<1>), grid, dim3(kThreads), 0, be->stream, a, r);
     else if (a.M <= 4)
-        hipLaunchKernelGGL((skinny_kt_wide_residual_kernel<4>), grid, dim3(kThreads), 0, be->stream, a, r);
+        launch_kernel((skinny_kt_wide_residual_kernel<4>), grid, dim3(kThreads), 0, be->stream, a, r);
     else
-        hipLaunchKernelGGL((skinny_kt_wide_residual_kernel<8>), grid, dim3(kThreads), 0, be->stream, a, r);
+        launch_kernel((skinny_kt_wide_residual_kernel<8>), grid, dim3(kThreads), 0, be->stream, a, r);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "matmul with residual launch");
 }
@@ -2455,9 +2455,9 @@ static int pack_operand(cg_backend *be, Buffer *buf, const uint32_t *ptr, int64_
     const dim3 grid((uint32_t)((quads + kThreads - 1) / kThreads));
     {
         ProfScope prof(be, CG_K_PACK, (double)rows * (double)K * (4.0 + (kind == 3 ? 1.0 : 2.0)));
-        if (kind == 1) hipLaunchKernelGGL(pack_operand_kernel<1>, grid, dim3(kThreads), 0, be->stream, ptr, s_r, s_k, (uint32_t)rows, (uint32_t)K, dst);
-        else if (kind == 2) hipLaunchKernelGGL(pack_operand_kernel<2>, grid, dim3(kThreads), 0, be->stream, ptr, s_r, s_k, (uint32_t)rows, (uint32_t)K, dst);
-        else hipLaunchKernelGGL(pack_operand_kernel<3>, grid, dim3(kThreads), 0, be->stream, ptr, s_r, s_k, (uint32_t)rows, (uint32_t)K, dst);
+        if (kind == 1) launch_kernel(pack_operand_kernel<1>, grid, dim3(kThreads), 0, be->stream, ptr, s_r, s_k, (uint32_t)rows, (uint32_t)K, dst);
+        else if (kind == 2) launch_kernel(pack_operand_kernel<2>, grid, dim3(kThreads), 0, be->stream, ptr, s_r, s_k, (uint32_t)rows, (uint32_t)K, dst);
+        else launch_kernel(pack_operand_kernel<3>, grid, dim3(kThreads), 0, be->stream, ptr, s_r, s_k, (uint32_t)rows, (uint32_t)K, dst);
     }
     if (keep) {
         if (buf->packed.size() >= kMaxPackedPerBuffer) { // stream-ordered free: products already queued on it come first
@@ -2650,7 +2650,7 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
     const bool f32 = is_f(x->dt);
     const int half = x->dt == CG_BF16 ? 1 : x->dt == CG_F16 ? 2 : 0; // operands of the 16-bit matrix instructions
     const int kind = half ? half : x->dt == CG_F8 ? 3 : 0;           // the narrow kernels' operand format (0: none)
-    hipStream_t s = be->stream;
+    LaunchQueue &s = be->stream;
 
     // ---- the narrow dtypes' tiled kernels' plan (used by the last branch below; here because it decides how operands are addressed) ----
     // the 256 x 256 tile when it covers half of the chip (1024 x 2048 x 8192, 128 tiles: 53 us against 57 on 128 x 128 tiles, bf16;
@@ -2707,9 +2707,9 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
         uint64_t elems = (uint64_t)M * N;
         dim3 grid((uint32_t)((elems + kThreads - 1) / kThreads), (uint32_t)batch);
         if (f32)
-            hipLaunchKernelGGL((simple_gemm_kernel<true>), grid, dim3(kThreads), 0, s, a);
+            launch_kernel((simple_gemm_kernel<true>), grid, dim3(kThreads), 0, s, a);
         else
-            hipLaunchKernelGGL((simple_gemm_kernel<false>), grid, dim3(kThreads), 0, s, a);
+            launch_kernel((simple_gemm_kernel<false>), grid, dim3(kThreads), 0, s, a);
     } else if (skinny_packed) {
         // a decode-time linear layer of a narrow dtype: the weight matrix in memory as its dtype's patterns (as uploaded, or
         // narrowed once), read at 2 or 1 bytes a weight
@@ -2727,8 +2727,8 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
             const uint32_t groups = (uint32_t)((N + 3) / 4), iters = xreg_cols_iters(groups);
             const dim3 mgrid((groups + iters - 1) / iters);
 #define CG_PACKED_MFMA(KCH)                                                                                              \
-    if (half == 1) hipLaunchKernelGGL((skinny_kt_packed_mfma_kernel<1, KCH>), mgrid, dim3(kThreads), 0, s, a, pb, iters);      \
-    else hipLaunchKernelGGL((skinny_kt_packed_mfma_kernel<2, KCH>), mgrid, dim3(kThreads), 0, s, a, pb, iters);
+    if (half == 1) launch_kernel((skinny_kt_packed_mfma_kernel<1, KCH>), mgrid, dim3(kThreads), 0, s, a, pb, iters);      \
+    else launch_kernel((skinny_kt_packed_mfma_kernel<2, KCH>), mgrid, dim3(kThreads), 0, s, a, pb, iters);
             if (kch == 1) { CG_PACKED_MFMA(1) }
             else if (kch == 2) { CG_PACKED_MFMA(2) }
             else if (kch == 4) { CG_PACKED_MFMA(4) }
@@ -2739,9 +2739,9 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
             return me == hipSuccess ? CG_OK : hip_fail(me, "matmul launch");
         }
 #define CG_PACKED(MM)                                                                                                     \
-    if (kind == 1) hipLaunchKernelGGL((skinny_kt_packed_kernel<MM, 1>), pgrid, dim3(kThreads), 0, s, a, pb);                  \
-    else if (kind == 2) hipLaunchKernelGGL((skinny_kt_packed_kernel<MM, 2>), pgrid, dim3(kThreads), 0, s, a, pb);             \
-    else hipLaunchKernelGGL((skinny_kt_packed_kernel<MM, 3>), pgrid, dim3(kThreads), 0, s, a, pb);
+    if (kind == 1) launch_kernel((skinny_kt_packed_kernel<MM, 1>), pgrid, dim3(kThreads), 0, s, a, pb);                  \
+    else if (kind == 2) launch_kernel((skinny_kt_packed_kernel<MM, 2>), pgrid, dim3(kThreads), 0, s, a, pb);             \
+    else launch_kernel((skinny_kt_packed_kernel<MM, 3>), pgrid, dim3(kThreads), 0, s, a, pb);
         if (M <= 1) { CG_PACKED(1) }
         else if (M <= 4) { CG_PACKED(4) }
         else { CG_PACKED(8) }
@@ -2755,7 +2755,7 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
     else { CALL(8) }
         if (!vec) {
             dim3 grid((uint32_t)((N + 3) / 4), (uint32_t)batch);
-#define CG_CALL(MMV) hipLaunchKernelGGL((skinny_kt_kernel<MMV>), grid, dim3(kThreads), 0, s, a);
+#define CG_CALL(MMV) launch_kernel((skinny_kt_kernel<MMV>), grid, dim3(kThreads), 0, s, a);
             CG_MM_SWITCH(CG_CALL)
 #undef CG_CALL
         } else if (K <= 256) {
@@ -2763,9 +2763,9 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
             const uint32_t cols_per_block = 4 * (64 / lpc) * 4;
             dim3 grid((uint32_t)((N + cols_per_block - 1) / cols_per_block), (uint32_t)batch);
 #define CG_CALL(MMV)                                                                                          \
-    if (lpc == 16) hipLaunchKernelGGL((skinny_kt_narrow_kernel<MMV, 16>), grid, dim3(kThreads), 0, s, a);     \
-    else if (lpc == 32) hipLaunchKernelGGL((skinny_kt_narrow_kernel<MMV, 32>), grid, dim3(kThreads), 0, s, a); \
-    else hipLaunchKernelGGL((skinny_kt_narrow_kernel<MMV, 64>), grid, dim3(kThreads), 0, s, a);
+    if (lpc == 16) launch_kernel((skinny_kt_narrow_kernel<MMV, 16>), grid, dim3(kThreads), 0, s, a);     \
+    else if (lpc == 32) launch_kernel((skinny_kt_narrow_kernel<MMV, 32>), grid, dim3(kThreads), 0, s, a); \
+    else launch_kernel((skinny_kt_narrow_kernel<MMV, 64>), grid, dim3(kThreads), 0, s, a);
             CG_MM_SWITCH(CG_CALL)
 #undef CG_CALL
         } else {
@@ -2773,7 +2773,7 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
             const int64_t cols = N * batch;
             if (cols >= 16384) {
                 dim3 grid((uint32_t)((N + 15) / 16), (uint32_t)batch);
-#define CG_CALL(MMV) hipLaunchKernelGGL((skinny_kt_wide_kernel<MMV, 4, false>), grid, dim3(kThreads), 0, s, a);
+#define CG_CALL(MMV) launch_kernel((skinny_kt_wide_kernel<MMV, 4, false>), grid, dim3(kThreads), 0, s, a);
                 CG_MM_SWITCH(CG_CALL)
 #undef CG_CALL
             } else if (cols >= 4096 && M <= 4) { // the wider projections of a decode step: activations are fetched once per 8 columns
@@ -2781,31 +2781,31 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
                 xreg_either((uint32_t)K, xreg_trips((uint32_t)K), [&](auto whole) {
                     constexpr bool W = decltype(whole)::value;
                     if (xreg_trips((uint32_t)K) == 4)
-                        hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<W, 4, 2, 4>), grid, dim3(kThreads), 0, s, a);
+                        launch_kernel((skinny_kt_mfma_xreg_kernel<W, 4, 2, 4>), grid, dim3(kThreads), 0, s, a);
                     else
-                        hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<W, 4, 2, 8>), grid, dim3(kThreads), 0, s, a);
+                        launch_kernel((skinny_kt_mfma_xreg_kernel<W, 4, 2, 8>), grid, dim3(kThreads), 0, s, a);
                 });
             } else if (cols >= 2048 && xreg_narrow((uint32_t)M, (uint32_t)K)) {
                 dim3 grid((uint32_t)((N + 3) / 4), (uint32_t)batch);
                 xreg_either((uint32_t)K, xreg_trips((uint32_t)K), [&](auto whole) {
                     constexpr bool W = decltype(whole)::value;
                     if (M > 4 && xreg_trips((uint32_t)K) == 4)
-                        hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<W, 8, 1, 4>), grid, dim3(kThreads), 0, s, a);
+                        launch_kernel((skinny_kt_mfma_xreg_kernel<W, 8, 1, 4>), grid, dim3(kThreads), 0, s, a);
                     else if (M > 4)
-                        hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<W, 8, 1, 8>), grid, dim3(kThreads), 0, s, a);
+                        launch_kernel((skinny_kt_mfma_xreg_kernel<W, 8, 1, 8>), grid, dim3(kThreads), 0, s, a);
                     else if (xreg_trips((uint32_t)K) == 4)
-                        hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<W, 4, 1, 4>), grid, dim3(kThreads), 0, s, a);
+                        launch_kernel((skinny_kt_mfma_xreg_kernel<W, 4, 1, 4>), grid, dim3(kThreads), 0, s, a);
                     else
-                        hipLaunchKernelGGL((skinny_kt_mfma_xreg_kernel<W, 4, 1, 8>), grid, dim3(kThreads), 0, s, a);
+                        launch_kernel((skinny_kt_mfma_xreg_kernel<W, 4, 1, 8>), grid, dim3(kThreads), 0, s, a);
                 });
             } else if (cols >= 2048) {
                 dim3 grid((uint32_t)((N + 3) / 4), (uint32_t)batch);
-#define CG_CALL(MMV) hipLaunchKernelGGL((skinny_kt_wide_kernel<MMV, 1, false>), grid, dim3(kThreads), 0, s, a);
+#define CG_CALL(MMV) launch_kernel((skinny_kt_wide_kernel<MMV, 1, false>), grid, dim3(kThreads), 0, s, a);
                 CG_MM_SWITCH(CG_CALL)
 #undef CG_CALL
             } else {
                 dim3 grid((uint32_t)N, (uint32_t)batch);
-#define CG_CALL(MMV) hipLaunchKernelGGL((skinny_kt_wide_kernel<MMV, 1, true>), grid, dim3(kThreads), 0, s, a);
+#define CG_CALL(MMV) launch_kernel((skinny_kt_wide_kernel<MMV, 1, true>), grid, dim3(kThreads), 0, s, a);
                 CG_MM_SWITCH(CG_CALL)
 #undef CG_CALL
             }
@@ -2826,12 +2826,12 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
             dst = static_cast<uint32_t *>(scratch);
         }
         dim3 grid((uint32_t)((N + 63) / 64), (uint32_t)batch, (uint32_t)splits);
-#define CG_CALL(MMV) hipLaunchKernelGGL((skinny_nn_kernel<MMV>), grid, dim3(kThreads), 0, s, a, dst, kchunk);
+#define CG_CALL(MMV) launch_kernel((skinny_nn_kernel<MMV>), grid, dim3(kThreads), 0, s, a, dst, kchunk);
         CG_MM_SWITCH(CG_CALL)
 #undef CG_CALL
         if (splits > 1) {
             uint64_t total = (uint64_t)batch * M * N;
-            hipLaunchKernelGGL(splitk_reduce_kernel, dim3((uint32_t)((total + kThreads - 1) / kThreads)), dim3(kThreads),
+            launch_kernel(splitk_reduce_kernel, dim3((uint32_t)((total + kThreads - 1) / kThreads)), dim3(kThreads),
                                0, s, static_cast<const uint32_t *>(scratch), a.C, (uint32_t)splits, (uint32_t)(M * N),
                                total);
             be->pool.free(scratch, scratch_cls); // stream-ordered: later users queue behind the reduce
@@ -2905,15 +2905,15 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
                     const dim3 pgrid((uint32_t)std::min<uint64_t>(walked, (uint64_t)be->compute_units)); // its workgroups walk the tiles
                     if (prc) {
                     } else
-                    if (kind == 1 && narrow_out) hipLaunchKernelGGL((mfma_gemm_dlds_kernel<3, true>), pgrid, dim3(kThreads), kDldsLdsBytes, s, p);
-                    else if (kind == 1) hipLaunchKernelGGL((mfma_gemm_dlds_kernel<3, false>), pgrid, dim3(kThreads), kDldsLdsBytes, s, p);
-                    else if (kind == 2 && narrow_out) hipLaunchKernelGGL((mfma_gemm_dlds_kernel<4, true>), pgrid, dim3(kThreads), kDldsLdsBytes, s, p);
-                    else if (kind == 2) hipLaunchKernelGGL((mfma_gemm_dlds_kernel<4, false>), pgrid, dim3(kThreads), kDldsLdsBytes, s, p);
-                    else if (narrow_out) hipLaunchKernelGGL((mfma_gemm_dlds_kernel<5, true>), pgrid, dim3(kThreads), kDldsLdsBytes, s, p);
-                    else hipLaunchKernelGGL((mfma_gemm_dlds_kernel<5, false>), pgrid, dim3(kThreads), kDldsLdsBytes, s, p);
-                } else if (kind == 1) hipLaunchKernelGGL((mfma_gemm_kernel<false, false, 4, 4, 3>), grid, dim3(kThreads), gemm_lds_bytes(256, 256), s, p);
-                else if (kind == 2) hipLaunchKernelGGL((mfma_gemm_kernel<false, false, 4, 4, 4>), grid, dim3(kThreads), gemm_lds_bytes(256, 256), s, p);
-                else hipLaunchKernelGGL((mfma_gemm_kernel<false, false, 4, 4, 5>), grid, dim3(kThreads), gemm_lds_bytes(256, 256), s, p);
+                    if (kind == 1 && narrow_out) launch_kernel((mfma_gemm_dlds_kernel<3, true>), pgrid, dim3(kThreads), kDldsLdsBytes, s, p);
+                    else if (kind == 1) launch_kernel((mfma_gemm_dlds_kernel<3, false>), pgrid, dim3(kThreads), kDldsLdsBytes, s, p);
+                    else if (kind == 2 && narrow_out) launch_kernel((mfma_gemm_dlds_kernel<4, true>), pgrid, dim3(kThreads), kDldsLdsBytes, s, p);
+                    else if (kind == 2) launch_kernel((mfma_gemm_dlds_kernel<4, false>), pgrid, dim3(kThreads), kDldsLdsBytes, s, p);
+                    else if (narrow_out) launch_kernel((mfma_gemm_dlds_kernel<5, true>), pgrid, dim3(kThreads), kDldsLdsBytes, s, p);
+                    else launch_kernel((mfma_gemm_dlds_kernel<5, false>), pgrid, dim3(kThreads), kDldsLdsBytes, s, p);
+                } else if (kind == 1) launch_kernel((mfma_gemm_kernel<false, false, 4, 4, 3>), grid, dim3(kThreads), gemm_lds_bytes(256, 256), s, p);
+                else if (kind == 2) launch_kernel((mfma_gemm_kernel<false, false, 4, 4, 4>), grid, dim3(kThreads), gemm_lds_bytes(256, 256), s, p);
+                else launch_kernel((mfma_gemm_kernel<false, false, 4, 4, 5>), grid, dim3(kThreads), gemm_lds_bytes(256, 256), s, p);
             }
             if (ta) be->pool.free(ta, ca); // stream-ordered: later users queue behind the product
             if (tb) be->pool.free(tb, cb);
@@ -2924,9 +2924,9 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
 #define CG_GEMM_HALF(AF, BF, H)                                                                                    \
     do {                                                                                                           \
         if (big)                                                                                                   \
-            hipLaunchKernelGGL((mfma_gemm_kernel<AF, BF, 4, 4, H>), grid, dim3(kThreads), gemm_lds_bytes(256, 256, true), s, a); \
+            launch_kernel((mfma_gemm_kernel<AF, BF, 4, 4, H>), grid, dim3(kThreads), gemm_lds_bytes(256, 256, true), s, a); \
         else                                                                                                       \
-            hipLaunchKernelGGL((mfma_gemm_kernel<AF, BF, 2, 2, H>), grid, dim3(kThreads), gemm_lds_bytes(128, 128, true), s, a); \
+            launch_kernel((mfma_gemm_kernel<AF, BF, 2, 2, H>), grid, dim3(kThreads), gemm_lds_bytes(128, 128, true), s, a); \
     } while (0)
 #define CG_GEMM(AF, BF)                    \
     do {                                   \

@@ -512,7 +512,7 @@ template <int K, bool F> int launch_cols(cg_backend *be, const RowsArgs &a) {
     if (narrow_allowed && vec && R0 % 32 == 0 && (uint64_t)(R0 / 32) * (a.rows / R0) >= 256 && a.n >= 1024) {
         const uint64_t nblocks = (uint64_t)(R0 / 32) * (a.rows / R0);
         if (nblocks <= 0x7FFFFFFFull) {
-            hipLaunchKernelGGL((reduce_cols_narrow_kernel<K, F>), dim3((uint32_t)nblocks), dim3(kBlock), 0, be->stream, a, R0 / 32);
+            launch_kernel((reduce_cols_narrow_kernel<K, F>), dim3((uint32_t)nblocks), dim3(kBlock), 0, be->stream, a, R0 / 32);
             hipError_t ne = hipGetLastError();
             return ne == hipSuccess ? CG_OK : hip_fail(ne, "column reduction launch");
         }
@@ -532,11 +532,11 @@ template <int K, bool F> int launch_cols(cg_backend *be, const RowsArgs &a) {
     }
     const dim3 grid((uint32_t)blocks, segs);
     if (vec)
-        hipLaunchKernelGGL((reduce_cols_kernel<K, F, 4>), grid, dim3(kBlock), 0, be->stream, a, tiles0, seglen, segs, static_cast<long long *>(part));
+        launch_kernel((reduce_cols_kernel<K, F, 4>), grid, dim3(kBlock), 0, be->stream, a, tiles0, seglen, segs, static_cast<long long *>(part));
     else
-        hipLaunchKernelGGL((reduce_cols_kernel<K, F, 1>), grid, dim3(kBlock), 0, be->stream, a, tiles0, seglen, segs, static_cast<long long *>(part));
+        launch_kernel((reduce_cols_kernel<K, F, 1>), grid, dim3(kBlock), 0, be->stream, a, tiles0, seglen, segs, static_cast<long long *>(part));
     if (segs > 1) {
-        hipLaunchKernelGGL((reduce_cols_final_kernel<K, F>), dim3((a.rows + 63) / 64), dim3(kBlock), 0, be->stream,
+        launch_kernel((reduce_cols_final_kernel<K, F>), dim3((a.rows + 63) / 64), dim3(kBlock), 0, be->stream,
                            static_cast<const long long *>(part), a.out, segs, a.rows);
         be->pool.free(part, cls); // stream-ordered: later users queue behind the merge
     }
@@ -560,9 +560,9 @@ template <int K, bool F> int launch_rows(cg_backend *be, const RowsArgs &a) {
         void *part = nullptr;
         size_t cls = 0;
         if (be->pool.alloc((size_t)a.rows * segs * sizeof(long long), &part, &cls) == CG_OK) {
-            hipLaunchKernelGGL((reduce_segments_kernel<K, F>), dim3(segs, a.rows), dim3(kBlock), 0, be->stream, a,
+            launch_kernel((reduce_segments_kernel<K, F>), dim3(segs, a.rows), dim3(kBlock), 0, be->stream, a,
                                static_cast<long long *>(part), seglen);
-            hipLaunchKernelGGL((reduce_segments_final_kernel<K, F>), dim3(a.rows), dim3(64), 0, be->stream,
+            launch_kernel((reduce_segments_final_kernel<K, F>), dim3(a.rows), dim3(64), 0, be->stream,
                                static_cast<const long long *>(part), a.out, segs);
             be->pool.free(part, cls); // stream-ordered: later users queue behind the merge
             hipError_t e = hipGetLastError();
@@ -576,10 +576,10 @@ template <int K, bool F> int launch_rows(cg_backend *be, const RowsArgs &a) {
     uint32_t rpb = kBlock / tpr;
     dim3 grid((a.rows + rpb - 1) / rpb), block(kBlock);
     switch (tpr) {
-    case 4: hipLaunchKernelGGL((reduce_rows_kernel<K, F, 4>), grid, block, 0, be->stream, a); break;
-    case 16: hipLaunchKernelGGL((reduce_rows_kernel<K, F, 16>), grid, block, 0, be->stream, a); break;
-    case 64: hipLaunchKernelGGL((reduce_rows_kernel<K, F, 64>), grid, block, 0, be->stream, a); break;
-    default: hipLaunchKernelGGL((reduce_rows_kernel<K, F, 256>), grid, block, 0, be->stream, a); break;
+    case 4: launch_kernel((reduce_rows_kernel<K, F, 4>), grid, block, 0, be->stream, a); break;
+    case 16: launch_kernel((reduce_rows_kernel<K, F, 16>), grid, block, 0, be->stream, a); break;
+    case 64: launch_kernel((reduce_rows_kernel<K, F, 64>), grid, block, 0, be->stream, a); break;
+    default: launch_kernel((reduce_rows_kernel<K, F, 256>), grid, block, 0, be->stream, a); break;
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "reduction launch");
@@ -640,7 +640,7 @@ int launch_topk(cg_backend *be, const cg_tensor *x, int64_t k, cg_tensor *vals, 
     int rc = fill_rows_args(x, &a);
     if (rc) return rc;
     a.out = static_cast<uint32_t *>(vals->buf->ptr);
-    hipLaunchKernelGGL(topk_kernel, dim3(a.rows), dim3(kBlock), 0, be->stream, a, (uint32_t)k,
+    launch_kernel(topk_kernel, dim3(a.rows), dim3(kBlock), 0, be->stream, a, (uint32_t)k,
                        static_cast<uint32_t *>(idxs->buf->ptr));
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "topk launch");
@@ -661,7 +661,7 @@ static int launch_any(cg_backend *be, int mode, const cg_tensor *x, const cg_ten
     a.flag = be->flag_dev;
     dim3 grid((uint32_t)((a.g.total + kBlock - 1) / kBlock)), block(kBlock);
     bool f = is_f(x->dt);
-#define CG_ANY(MODE, F, VEC) hipLaunchKernelGGL((any_kernel<MODE, F, VEC>), grid, block, 0, be->stream, a)
+#define CG_ANY(MODE, F, VEC) launch_kernel((any_kernel<MODE, F, VEC>), grid, block, 0, be->stream, a)
     if (mode == 0) {
         if (a.g.vec == 4) { if (f) CG_ANY(0, true, 4); else CG_ANY(0, false, 4); }
         else { if (f) CG_ANY(0, true, 1); else CG_ANY(0, false, 1); }

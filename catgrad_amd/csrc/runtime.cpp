@@ -93,6 +93,7 @@ void Pool::trim() {
         take.swap(free_);
         cached_ = 0;
     }
+    if (launches) launches->drain();
     for (auto &kv : take) (void)hipFree(kv.second);
 }
 
@@ -756,6 +757,8 @@ static bool same_shape(const cg_tensor *a, const cg_tensor *b) {
 
 static int wait_and_check(cg_backend *be) {
     CG_HIP(hipStreamSynchronize(be->stream));
+    be->stream.waited();
+    CG_HIP(be->stream.error());
     if (!be->prof_pending.empty()) prof_drain(be);
     uint32_t f = *reinterpret_cast<volatile uint32_t *>(be->fault_host);
     if (f) {
@@ -778,6 +781,8 @@ static int wait_for_readback(cg_backend *be, uint32_t seq) {
         __builtin_ia32_pause();
     }
     std::atomic_thread_fence(std::memory_order_acquire);
+    be->stream.waited();
+    CG_HIP(be->stream.error());
     uint32_t f = *reinterpret_cast<volatile uint32_t *>(be->fault_host);
     if (f) {
         *reinterpret_cast<volatile uint32_t *>(be->fault_host) = 0;
@@ -2255,7 +2260,8 @@ int cg_backend_create(int device, cg_backend **out) {
     if (int nrc = noalloc_setup(device)) return nrc; // set-up of the entry point that may not allocate later
     cg_backend *b = new cg_backend;
     b->device = device;
-    CG_HIP(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
+    CG_HIP(b->stream.open(device));
+    b->pool.launches = &b->stream;
     CG_HIP(hipHostMalloc((void **)&b->fault_host, 64, hipHostMallocMapped));
     memset(b->fault_host, 0, 64);
     CG_HIP(hipHostGetDevicePointer((void **)&b->fault_dev, b->fault_host, 0));
@@ -2296,7 +2302,7 @@ static void backend_teardown(cg_backend *b) {
     (void)hipHostFree(b->flag_host);
     (void)hipHostFree(b->fault_host);
     (void)hipHostFree(b->rb_host);
-    (void)hipStreamDestroy(b->stream);
+    b->stream.close();
     delete b;
 }
 

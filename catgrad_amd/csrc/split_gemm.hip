@@ -201,15 +201,15 @@ int launch_split_gemm(cg_backend *be, MmArgs a, bool a_mfast, bool b_nfast) {
         splits = 1;
         a.ksplit = 0;
     }
-    hipLaunchKernelGGL(k, dim3((uint32_t)tiles, a.batch, (uint32_t)splits), dim3(all[t].threads), lds, be->stream, a);
+    launch_kernel(k, dim3((uint32_t)tiles, a.batch, (uint32_t)splits), dim3(all[t].threads), lds, be->stream, a);
     if (splits > 1) {
         const uint64_t total = mn * a.batch;
         const float *const from = static_cast<const float *>(parts);
         if (mn % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0)
-            hipLaunchKernelGGL((sum_splits_kernel<4>), dim3((uint32_t)((total / 4 + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream, from, y,
+            launch_kernel((sum_splits_kernel<4>), dim3((uint32_t)((total / 4 + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream, from, y,
                                (uint32_t)splits, (uint32_t)mn, total);
         else
-            hipLaunchKernelGGL((sum_splits_kernel<1>), dim3((uint32_t)((total + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream, from, y,
+            launch_kernel((sum_splits_kernel<1>), dim3((uint32_t)((total + kThreads - 1) / kThreads)), dim3(kThreads), 0, be->stream, from, y,
                                (uint32_t)splits, (uint32_t)mn, total);
         be->pool.free(parts, cls); // stream-ordered
     }

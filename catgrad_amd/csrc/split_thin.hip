@@ -182,11 +182,11 @@ double thin_gemm_cost(const cg_backend *be, const MmArgs &a, int *high) {
 int launch_thin_gemm(cg_backend *be, const MmArgs &a, int high) {
     const dim3 grid((a.N + 15) / 16, (a.M + 16 * high - 1) / (16 * high), a.batch), block(64 * kWaves);
     if (a.K % kTurn == 0) {
-        if (high == 1) hipLaunchKernelGGL((split_thin_kernel<1, true>), grid, block, 0, be->stream, a);
-        else hipLaunchKernelGGL((split_thin_kernel<2, true>), grid, block, 0, be->stream, a);
+        if (high == 1) launch_kernel((split_thin_kernel<1, true>), grid, block, 0, be->stream, a);
+        else launch_kernel((split_thin_kernel<2, true>), grid, block, 0, be->stream, a);
     } else {
-        if (high == 1) hipLaunchKernelGGL((split_thin_kernel<1, false>), grid, block, 0, be->stream, a);
-        else hipLaunchKernelGGL((split_thin_kernel<2, false>), grid, block, 0, be->stream, a);
+        if (high == 1) launch_kernel((split_thin_kernel<1, false>), grid, block, 0, be->stream, a);
+        else launch_kernel((split_thin_kernel<2, false>), grid, block, 0, be->stream, a);
     }
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "matmul launch");
