@@ -500,7 +500,7 @@ static int rotation_tables(cg_backend *be, AttentionPlan &p, uint64_t end) {
     return CG_OK;
 }
 
-int launch_attention(cg_backend *be, const AttentionPlan &plan) {
+int launch_attention(cg_backend *be, const AttentionPlan &plan, DeferredStep **later) {
     AttentionPlan p = plan;
     if (p.rot_dims)
         if (int rc = rotation_tables(be, p, p.position + p.S)) return rc;
@@ -511,7 +511,7 @@ int launch_attention(cg_backend *be, const AttentionPlan &plan) {
     for (uint32_t s = 0; s < p.S; s++) pairs += (double)std::min(p.window ? p.window : ~0u, p.cached + s + 1);
     ProfScope prof(be, CG_K_ATTENTION, pairs * p.B * p.heads * (2.0 * p.dim + 2.0 * p.vdim + (p.talk ? 2.0 * p.heads : 0.0)));
     if (p.mix_scores)
-        if (int rc = launch_mixed_step(be, p); rc != kDeclined) return rc;
+        if (int rc = launch_mixed_step(be, p, later); rc != kDeclined) return rc;
     Scratch qbuf(be);
     float *q = nullptr;
     if (!fresh) {

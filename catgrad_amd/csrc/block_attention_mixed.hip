@@ -13,6 +13,7 @@
 // Unfinished results carry {top, sum}: weights are 2^(score log2 e - top), `top` in units of log2.
 #include "blocks.hpp"
 #include "device_utils.hpp"
+#include "expert_first.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -433,10 +434,9 @@ __host__ __device__ inline StepLds step_lds(uint32_t S, uint32_t heads, uint32_t
 }
 
 template <int REP, int DQ, int PI>
-__global__ __launch_bounds__(kThreads, REP <= 4 ? 3 : 2) void attention_mixed_step_kernel(const AttentionPlan p, const uint32_t chunk, const uint32_t chunks, float *__restrict__ parts,
-                                                                        float2 *__restrict__ stats) {
-    extern __shared__ float lds[];
-    const uint32_t rep = p.heads / p.kv_heads, seg = blockIdx.x, nseg = gridDim.x, r = blockIdx.y, b = r / p.S, s = r - b * p.S;
+__device__ __forceinline__ void mixed_step(const AttentionPlan &p, const uint32_t chunk, const uint32_t chunks, float *__restrict__ parts, float2 *__restrict__ stats, const uint32_t seg,
+                                           const uint32_t nseg, const uint32_t r, float *const lds) {
+    const uint32_t rep = p.heads / p.kv_heads, b = r / p.S, s = r - b * p.S;
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63, pitch = chunk + 1, sub = threadIdx.x & 3;
     const StepLds at = step_lds(p.S, p.heads, p.kv_heads, p.dim, chunk, p.vdim);
     const uint32_t first = first_visible(p, p.cached + s) + seg * chunk * chunks, hi = p.cached + s + 1, end = min(hi, first + chunk * chunks);
@@ -664,6 +664,31 @@ __global__ __launch_bounds__(kThreads, REP <= 4 ? 3 : 2) void attention_mixed_st
     }
 }
 
+template <int REP, int DQ, int PI>
+__global__ __launch_bounds__(kThreads, REP <= 4 ? 3 : 2) void attention_mixed_step_kernel(const AttentionPlan p, const uint32_t chunk, const uint32_t chunks, float *__restrict__ parts,
+                                                                        float2 *__restrict__ stats) {
+    extern __shared__ float lds[];
+    mixed_step<REP, DQ, PI>(p, chunk, chunks, parts, stats, blockIdx.x, gridDim.x, blockIdx.y, lds);
+}
+// The same in the first segs * rows workgroups; the others compute the chosen experts' first products (their columns' blocks x, then
+// row * top + choice), which need nothing of the attention.
+template <int REP, int DQ, int PI, bool BF16>
+__global__ __launch_bounds__(kThreads, 3) void attention_step_experts_kernel(const AttentionPlan p, const uint32_t chunk, const uint32_t chunks, float *__restrict__ parts,
+                                                                             float2 *__restrict__ stats, const uint32_t segs, const ExpertsPlan e, const uint32_t per_wave,
+                                                                             const uint32_t blocks_x, float *__restrict__ hidden, uint32_t *__restrict__ chosen) {
+    extern __shared__ float lds[];
+    const uint32_t first = segs * p.B * p.S;
+    if (blockIdx.x < first) {
+        mixed_step<REP, DQ, PI>(p, chunk, chunks, parts, stats, blockIdx.x % segs, segs, blockIdx.x / segs, lds);
+        return;
+    }
+    const uint32_t i = blockIdx.x - first, by = i / blocks_x, bx = i - by * blocks_x;
+    constexpr uint32_t SPAN = 64 * (BF16 ? 8 : 4);
+    if (e.width <= 2 * SPAN) expert_first<BF16, true, 2>(e, per_wave, hidden, chosen, bx, by, lds);
+    else if (e.width <= 4 * SPAN) expert_first<BF16, true, 4>(e, per_wave, hidden, chosen, bx, by, lds);
+    else expert_first<BF16, true, 8>(e, per_wave, hidden, chosen, bx, by, lds);
+}
+
 int launched(const char *what) {
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, what);
@@ -804,20 +829,73 @@ int launch_mixed_tiles(cg_backend *be, const AttentionPlan &p, const float *q) {
     return launched("attention_mixed_tiles");
 }
 
-template <int REP, int DQ>
-static int step_kernels(cg_backend *be, const AttentionPlan &p, uint32_t chunk, uint32_t chunks, dim3 grid, size_t lds, float *parts, float2 *stats) {
+static uint32_t pieces_of(uint32_t dim) { return dim <= 32 ? 2 : dim <= 64 ? 4 : 8; } // 16-byte pieces of a key per lane
+
+template <int REP, int DQ> static int step_kernels(cg_backend *be, const DeferredStep &s) {
     constexpr int PI = 8 / DQ; // keys of four lanes: 8 pieces per lane
-    if (int rc = allow_lds(reinterpret_cast<const void *>(&attention_mixed_step_kernel<REP, DQ, PI>), lds)) return rc;
-    launch_kernel((attention_mixed_step_kernel<REP, DQ, PI>), grid, dim3(kThreads), lds, be->stream, p, chunk, chunks, parts, stats);
+    if (int rc = allow_lds(reinterpret_cast<const void *>(&attention_mixed_step_kernel<REP, DQ, PI>), s.lds)) return rc;
+    launch_kernel((attention_mixed_step_kernel<REP, DQ, PI>), dim3(s.segs, s.plan.B * s.plan.S), dim3(kThreads), s.lds, be->stream, s.plan, s.chunk, s.chunks, s.parts, s.stats);
     return CG_OK;
 }
+template <int REP, int DQ>
+static int step_kernels_beside(cg_backend *be, const DeferredStep &s, const ExpertsPlan &e, float *hidden, uint32_t *chosen) {
+    constexpr int PI = 8 / DQ;
+    const uint32_t per_wave = expert_first_columns(be, e), bx = (e.ff + kExpertWaves * per_wave - 1) / (kExpertWaves * per_wave);
+    const uint64_t blocks = (uint64_t)s.segs * s.plan.B * s.plan.S + (uint64_t)bx * e.rows * e.top;
+    const size_t lds = std::max(s.lds, route_bytes(e));
+    if (blocks > 0x7FFFFFFFull || lds > (64u << 10)) return kDeclined;
+    if (e.fmt == kFmtBF16)
+        launch_kernel((attention_step_experts_kernel<REP, DQ, PI, true>), dim3((uint32_t)blocks), dim3(kThreads), lds, be->stream, s.plan, s.chunk, s.chunks, s.parts, s.stats, s.segs,
+                      e, per_wave, bx, hidden, chosen);
+    else
+        launch_kernel((attention_step_experts_kernel<REP, DQ, PI, false>), dim3((uint32_t)blocks), dim3(kThreads), lds, be->stream, s.plan, s.chunk, s.chunks, s.parts, s.stats, s.segs,
+                      e, per_wave, bx, hidden, chosen);
+    return CG_OK;
+}
+static int merge_step(cg_backend *be, const DeferredStep &s) {
+    const AttentionPlan &p = s.plan;
+    merge(be, p, s.parts, s.stats, s.segs, (uint64_t)s.segs * p.heads, p.heads, p.B * p.S, p.out);
+    return launched("attention_mixed_step");
+}
 
-int launch_mixed_step(cg_backend *be, const AttentionPlan &p) {
+int run_step(cg_backend *be, const DeferredStep &s) {
+    const uint32_t rep = s.plan.heads / s.plan.kv_heads, dq = pieces_of(s.plan.dim);
+    int rc;
+#define CG_STEP(R) (dq == 2 ? step_kernels<R, 2>(be, s) : dq == 4 ? step_kernels<R, 4>(be, s) : step_kernels<R, 8>(be, s))
+    if (rep <= 1) rc = CG_STEP(1);
+    else if (rep <= 2) rc = CG_STEP(2);
+    else if (rep <= 4) rc = CG_STEP(4);
+    else rc = CG_STEP(8);
+#undef CG_STEP
+    return rc ? rc : merge_step(be, s);
+}
+
+// Heads of 33 to 128 columns, up to four to a kv head, and experts whose rows lie in 16-byte pieces: what the shared kernel is compiled for.
+static bool shares_launch(const AttentionPlan &p) { return pieces_of(p.dim) >= 4 && p.heads / p.kv_heads <= 4; }
+int run_step_beside_experts(cg_backend *be, const DeferredStep &s, const ExpertsPlan &e, float *hidden, uint32_t *chosen) {
+    const uint32_t rep = s.plan.heads / s.plan.kv_heads, dq = pieces_of(s.plan.dim), span = 64 * (e.fmt == kFmtBF16 ? 8 : 4);
+    if (!shares_launch(s.plan) || !vector_rows(e) || e.width > 8 * span) return kDeclined;
+    int rc;
+#define CG_STEP(R) (dq == 4 ? step_kernels_beside<R, 4>(be, s, e, hidden, chosen) : step_kernels_beside<R, 8>(be, s, e, hidden, chosen))
+    if (rep <= 1) rc = CG_STEP(1);
+    else if (rep <= 2) rc = CG_STEP(2);
+    else rc = CG_STEP(4);
+#undef CG_STEP
+    return rc ? rc : merge_step(be, s);
+}
+
+void drop_step(cg_backend *be, DeferredStep *s) {
+    if (s->mem) be->pool.free(s->mem, s->cls); // stream-ordered
+    for (cg_tensor *t : s->held) release(t);
+    delete s;
+}
+
+int launch_mixed_step(cg_backend *be, const AttentionPlan &p, DeferredStep **later) {
     const uint32_t rows = p.B * p.S, keys = p.cached + p.S, most = p.window ? std::min(p.window, keys) : keys, rep = p.heads / p.kv_heads, cols = p.kv_heads * p.vdim / 4;
     auto aligned = [](const Rows &x) { return x.pitch % 4 == 0 && (reinterpret_cast<uintptr_t>(x.p) & 15) == 0; };
     if (p.S > kFewRows || p.dim % 4 || p.vdim % 4 || rows > 65535 || p.q_norm || p.k_norm || rep > 8 || p.dim > 128 || cols > kThreads || !aligned(p.v)) return kDeclined;
     // chunks whose keys and values a workgroup holds in registers
-    const uint32_t turns = std::max(1u, (uint32_t)kThreads / cols), dq = p.dim <= 32 ? 2 : p.dim <= 64 ? 4 : 8, pairs = kThreads / 4 * (8 / dq);
+    const uint32_t turns = std::max(1u, (uint32_t)kThreads / cols), dq = pieces_of(p.dim), pairs = kThreads / 4 * (8 / dq);
     if (p.kv_heads > pairs) return kDeclined;
     uint32_t chunk = kMaxChunk;
     while (chunk * p.kv_heads > pairs || chunk > turns * kValuesAhead) chunk /= 2;
@@ -826,24 +904,27 @@ int launch_mixed_step(cg_backend *be, const AttentionPlan &p) {
     // as many workgroups as run at a time
     const uint32_t all = (most + chunk - 1) / chunk;
     const uint32_t resident = (rep <= 4 ? 3 : 2) * be->compute_units, chunks = (uint32_t)(((uint64_t)rows * all + resident - 1) / resident), nseg = (all + chunks - 1) / chunks;
-    Scratch mem(be);
+    DeferredStep *const s = new DeferredStep;
     const size_t n = (size_t)rows * nseg * p.heads;
-    if (int rc = mem.get(n * p.vdim * 4 + n * sizeof(float2))) return rc;
-    float *parts = static_cast<float *>(mem.p);
-    float2 *stats = reinterpret_cast<float2 *>(parts + n * p.vdim);
-    const dim3 grid(nseg, rows);
-    int rc;
-#define CG_STEP(R) (p.dim <= 32 ? step_kernels<R, 2>(be, p, chunk, chunks, grid, lds, parts, stats) \
-                    : p.dim <= 64 ? step_kernels<R, 4>(be, p, chunk, chunks, grid, lds, parts, stats) \
-                                  : step_kernels<R, 8>(be, p, chunk, chunks, grid, lds, parts, stats))
-    if (rep <= 1) rc = CG_STEP(1);
-    else if (rep <= 2) rc = CG_STEP(2);
-    else if (rep <= 4) rc = CG_STEP(4);
-    else rc = CG_STEP(8);
-#undef CG_STEP
-    if (rc) return rc;
-    merge(be, p, parts, stats, nseg, (uint64_t)nseg * p.heads, p.heads, rows, p.out);
-    return launched("attention_mixed_step");
+    if (int rc = be->pool.alloc(n * p.vdim * 4 + n * sizeof(float2), &s->mem, &s->cls)) {
+        s->mem = nullptr;
+        drop_step(be, s);
+        return rc;
+    }
+    s->plan = p;
+    s->chunk = chunk;
+    s->chunks = chunks;
+    s->segs = nseg;
+    s->lds = lds;
+    s->parts = static_cast<float *>(s->mem);
+    s->stats = reinterpret_cast<float2 *>(s->parts + n * p.vdim);
+    if (later && shares_launch(p) && !be->prof[CG_K_ATTENTION].every && !be->prof[CG_K_GEMM_SKINNY].every) {
+        *later = s;
+        return CG_OK;
+    }
+    const int rc = run_step(be, *s);
+    drop_step(be, s);
+    return rc;
 }
 
 } // namespace cg

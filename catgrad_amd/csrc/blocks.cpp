@@ -383,6 +383,16 @@ int cache_tail(cg_backend *be, const cg_tensor *all, int64_t keep, cg_tensor **o
 }
 
 } // namespace
+
+static int64_t numel_of(const DeferredStep &s) { return (int64_t)s.plan.B * s.plan.S * s.plan.heads * s.plan.vdim; } // of its result
+
+void flush_step(cg_backend *be) {
+    DeferredStep *const s = be->step;
+    be->step = nullptr;
+    if (hipSetDevice(be->device) != hipSuccess || run_step(be, *s) != CG_OK) be->stream.fail(hipErrorLaunchFailure);
+    drop_step(be, s);
+}
+
 } // namespace cg
 
 using namespace cg;
@@ -671,7 +681,17 @@ int cg_block_token_side(cg_backend *b, const cg_token_side_args *a, cg_tensor **
 }
 
 int cg_block_residual(cg_backend *b, cg_tensor *x, const cg_branch *br, size_t n, float eps, float scale, const cg_experts *experts, cg_tensor **out) {
-    Enter entered(b);
+    Enter entered(b, true);
+    // Attention that waits may share the experts' launch, if it is what the only branch reads and all else is in memory and none of its own
+    if (b && b->step) {
+        const DeferredStep &s = *b->step;
+        auto apart = [&](const cg_tensor *t) { return !t || (!t->pend && t->buf != s.out && t->buf != s.keys && t->buf != s.values); };
+        bool fits = experts && n == 1 && br && br->y && !br->y->pend && br->y->buf == s.out && !br->poly && !br->gate && apart(x) && apart(br->w) && apart(br->gate_bias);
+        for (const cg_tensor *t : {fits ? experts->h : nullptr, fits ? experts->logits : nullptr, fits ? experts->correction : nullptr, fits ? experts->gate_up : nullptr,
+                                   fits ? experts->down : nullptr})
+            fits = fits && apart(t);
+        if (!fits || !is_contiguous(br->y) || br->y->offset || numel(br->y) != numel_of(s)) flush_step(b);
+    }
     Held h;
     h.add(x);
     for (size_t i = 0; br && i < n; i++)
@@ -711,12 +731,21 @@ int cg_block_residual(cg_backend *b, cg_tensor *x, const cg_branch *br, size_t n
     if (rows > 0 && width > 0) {
         float *y = static_cast<float *>(o->buf->ptr);
         const bool plain = n == 1 && !r[0].in.poly && !r[0].gate.p && r[0].w.fmt == ep.fmt;
+        if (b->step && !(experts && rows <= kFewRows && plain)) flush_step(b);
         if (experts && rows <= kFewRows && (n == 0 || plain)) {
             Scratch tmp(b);
             void *hidden = nullptr, *chosen = nullptr;
             rc = tmp.get((size_t)rows * ep.top * ep.ff * 4, &hidden);
             if (!rc) rc = tmp.get((size_t)rows * ep.top * 4, &chosen);
-            if (!rc) rc = launch_experts_first(b, ep, static_cast<float *>(hidden), static_cast<uint32_t *>(chosen));
+            if (!rc) {
+                int both = kDeclined;
+                if (b->step && (both = run_step_beside_experts(b, *b->step, ep, static_cast<float *>(hidden), static_cast<uint32_t *>(chosen))) != kDeclined) {
+                    drop_step(b, b->step);
+                    b->step = nullptr;
+                }
+                if (b->step) flush_step(b);
+                rc = both != kDeclined ? both : launch_experts_first(b, ep, static_cast<float *>(hidden), static_cast<uint32_t *>(chosen));
+            }
             if (!rc)
                 rc = launch_experts_second(b, ep, static_cast<float *>(hidden), static_cast<uint32_t *>(chosen), xr, n ? r[0].in.x : Rows{}, n ? &r[0].w : nullptr, scale, y);
         } else if (!experts && scale == 1.0f && takes_few_rows_residual(r, (int)n, (uint32_t)rows)) {
@@ -809,19 +838,30 @@ int cg_block_attention(cg_backend *b, const cg_attention_args *a, cg_tensor **ou
     p.v_block = va->strides[1];
     const int64_t od[3] = {B, S, H * V};
     cg_tensor *o = nullptr, *ko = nullptr, *vo = nullptr;
+    DeferredStep *step = nullptr;
     int rc = new_dense(b, CG_F32, od, 3, &o);
     if (!rc) {
         p.out = static_cast<float *>(o->buf->ptr);
-        rc = launch_attention(b, p);
+        rc = launch_attention(b, p, &step);
     }
     const int64_t tail = window ? std::min<int64_t>(ka->dims[2], window - 1) : ka->dims[2];
     if (!rc) rc = cache_tail(b, ka, tail, &ko);
     if (!rc) rc = cache_tail(b, va, tail, &vo);
     if (rc) {
+        if (step) drop_step(b, step);
         release(o);
         release(ko);
         release(vo);
         return rc;
+    }
+    if (step) { // (its operands and results stay until it is launched)
+        step->out = o->buf;
+        step->keys = ka->buf;
+        step->values = va->buf;
+        step->held.swap(h.t);
+        retain(o);
+        step->held.push_back(o);
+        b->step = step;
     }
     *out = o;
     *k_out = ko;

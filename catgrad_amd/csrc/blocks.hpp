@@ -131,6 +131,9 @@ struct ExpertsPlan {
 int launch_experts(cg_backend *be, const ExpertsPlan &p, float *y, int *y_fmt);
 // A few rows: hidden[r, slot, 0 .. ff) (weights applied) and the chosen experts' numbers.
 int launch_experts_first(cg_backend *be, const ExpertsPlan &p, float *hidden, uint32_t *chosen);
+// Columns that a wave of it takes: enough workgroups for the device, not many more.  Whether its rows lie in 16-byte pieces.
+uint32_t expert_first_columns(const cg_backend *be, const ExpertsPlan &p);
+bool vector_rows(const ExpertsPlan &p);
 // out[r] = x[r] + scale * (y[r] . w^T + sum_slot hidden[r, slot] . down[chosen[r, slot]]^T), rows <= kFewRows
 int launch_experts_second(cg_backend *be, const ExpertsPlan &p, const float *hidden, const uint32_t *chosen, const Rows &x, const Rows &y, const Weight *w, float scale,
                           float *out);
@@ -161,14 +164,33 @@ __device__ __forceinline__ float2 rotation_at(const AttentionPlan &p, uint64_t p
     return make_float2(fmaf(a.x, b.x, -a.y * b.y), fmaf(a.x, b.y, a.y * b.x));
 }
 #endif
-int launch_attention(cg_backend *be, const AttentionPlan &p);
+// Attention over mixed scores of a few new tokens whose launch waits for the next call on its backend: a mixture of experts that does
+// not read its result, which comes next in a layer, shares the launch (either is bound by latency: 10 and 8 us, 12 together).
+// Any other call launches it first (Enter).
+struct DeferredStep {
+    AttentionPlan plan{};
+    uint32_t chunk = 0, chunks = 0, segs = 0;
+    size_t lds = 0;
+    void *mem = nullptr; // the segments' results (pool memory)
+    size_t cls = 0;
+    float *parts = nullptr;
+    float2 *stats = nullptr;
+    std::vector<cg_tensor *> held; // operands and results (retained)
+    const Buffer *out = nullptr, *keys = nullptr, *values = nullptr;
+};
+int run_step(cg_backend *be, const DeferredStep &s);
+// The same beside launch_experts_first's kernel; kDeclined: experts that do not go along.
+int run_step_beside_experts(cg_backend *be, const DeferredStep &s, const ExpertsPlan &p, float *hidden, uint32_t *chosen);
+void drop_step(cg_backend *be, DeferredStep *s);
+// later: set if the launch is left to run_step (only for plans that run_step_beside_experts may take), with what that needs but `held`.
+int launch_attention(cg_backend *be, const AttentionPlan &p, DeferredStep **later = nullptr);
 // More than a few new tokens, on the matrix instructions (q: the prepared queries); kDeclined: sizes it does not take.
 int launch_attention_tiles(cg_backend *be, const AttentionPlan &p, const float *q);
 // Soft-max over mixed scores (block_attention_mixed.hip).  `scores`: the scores' segments as attention_scores_kernel leaves
 // them, of the rows row0 .. row0 + rows - 1; parts / part_stats: memory of nseg results per (row, head).
 int launch_mixed_rows(cg_backend *be, const AttentionPlan &p, uint32_t row0, uint32_t rows, uint32_t nseg, const float *scores, float *parts, float2 *part_stats);
 int launch_mixed_tiles(cg_backend *be, const AttentionPlan &p, const float *q);
-int launch_mixed_step(cg_backend *be, const AttentionPlan &p);
+int launch_mixed_step(cg_backend *be, const AttentionPlan &p, DeferredStep **later);
 
 // ---- gated delta rule ------------------------------------------------------------------------------------------------
 struct DeltaPlan {

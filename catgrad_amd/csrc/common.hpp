@@ -111,6 +111,7 @@ template <class T> struct Pooled {
 
 struct LazyMm;
 struct DeferredWrite;
+struct DeferredStep;
 struct Buffer;
 }
 
@@ -150,6 +151,7 @@ struct cg_backend {
     std::string name;
     std::vector<cg::LazyMm *> lazy_open; // groupable lazy products not yet computed (not retained)
     std::vector<cg::DeferredWrite> deferred; // writes waiting to share a launch (see flush_deferred)
+    cg::DeferredStep *step = nullptr;        // attention waiting for the next call, which may share its launch (blocks.hpp)
     // Results that depend on constants only (the rotary tables every forward pass rebuilds from iota and
     // scalars) are kept, keyed by the program and its leaves, and handed out again instead of recomputed.
     // Buffers are retained here; the oldest entries go when the limits are reached.
@@ -320,9 +322,13 @@ struct Consume { // the consumed reference of a tensor argument (move semantics 
 // Every entry point that touches a backend's state holds the backend's lock for its whole duration
 // (declared first, so the tensor arguments it consumes are released under the lock too): handles may be
 // cloned, moved between threads and used from several threads; calls on one backend then run one at a time.
+void flush_step(cg_backend *be); // launches be->step; an error is the next waiting call's
 struct Enter {
-    explicit Enter(cg_backend *b) : b_(b) {
-        if (b_) b_->mu.lock();
+    // keep_step: the call launches nothing, or looks after be->step itself
+    explicit Enter(cg_backend *b, bool keep_step = false) : b_(b) {
+        if (!b_) return;
+        b_->mu.lock();
+        if (b_->step && !keep_step) flush_step(b_);
     }
     ~Enter() {
         if (b_) b_->mu.unlock();

@@ -42,6 +42,7 @@ class LaunchQueue {
     // The host has waited for the device: the launches up to the next time are counted anew.
     void waited() { direct_ = 0; }
     // What a launch that was handed over has come to, once (hipSuccess: no error since the last call).
+    void fail(hipError_t e) { failed_.store((int)e); }
     hipError_t error() { return failed_.load(std::memory_order_relaxed) ? (hipError_t)failed_.exchange(0) : hipSuccess; }
 
     // One caller at a time (the backend's lock); the arguments are copied.

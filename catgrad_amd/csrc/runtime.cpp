@@ -2420,7 +2420,7 @@ void cg_tensor_release(cg_tensor *t) {
     cg_backend *be = t->be;
     bool last;
     {
-        Enter entered(be); // the last holder of a deferred tensor also closes what it had open in the backend
+        Enter entered(be, true); // the last holder of a deferred tensor also closes what it had open in the backend
         release(t);
         last = be->owner_gone && be->live_tensors.load() == 0;
     }

@@ -191,12 +191,7 @@ class LufatarModel : public LayeredModel {
         t.talk = i.param(m + ".talk");
         t.k_cache = std::move(s[0]);
         t.v_cache = std::move(s[1]);
-        std::vector<Tensor> a = blocks::attention(i, std::move(t), c.attention, position);
-        s[0] = std::move(a[1]);
-        s[1] = std::move(a[2]);
-        std::vector<blocks::Branch> br;
-        br.push_back({std::move(a[0]), i.param(m + ".o"), Tensor(), Tensor(), Tensor()});
-        blocks::Experts ex;
+        blocks::Experts ex; // (in front of attention: nothing between the two calls, which share a launch for a few tokens)
         if (c.count) {
             ex.h = std::move(h[2]);
             ex.logits = std::move(h[1]);
@@ -205,6 +200,11 @@ class LufatarModel : public LayeredModel {
             ex.down = reshape(i, Shape{c.count, c_.width, c.ff}, i.param(f + ".second"));
             ex.options = c.experts;
         }
+        std::vector<Tensor> a = blocks::attention(i, std::move(t), c.attention, position);
+        s[0] = std::move(a[1]);
+        s[1] = std::move(a[2]);
+        std::vector<blocks::Branch> br;
+        br.push_back({std::move(a[0]), i.param(m + ".o"), Tensor(), Tensor(), Tensor()});
         x = blocks::residual(i, std::move(x), std::move(br), c_.eps, c_.mult, std::move(ex));
         blocks::SideOptions side;
         side.first = l * c_.side;
