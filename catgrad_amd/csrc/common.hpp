@@ -563,11 +563,14 @@ int launch_fused_rows(cg_backend *be, const cg_tensor *out, const Pending &p, co
 bool rows_program_compiled(const Pending &p);
 bool rows_max_program_begun(const Pending &p);
 int launch_arange(cg_backend *be, cg_tensor *out);
-// Copies n <= kReadbackWords words to be->rb_dev and then stores `seq` at word kReadbackWords of it, visible to the host.
-// (64 KiB.  The runtime's copy, us, and this one: behind a kernel 4096 words 30 and 23, 16384 33 and 27.  Behind a polled read-back, as of a step's
-// tokens, the runtime first retires all kernels in front of it: 6000 words 100 us more than here.  Only with nothing left to retire is its copy of
-// more than 16 KiB the faster one: 8192 words 13 and 17.)
-constexpr uint32_t kReadbackWords = 16384;
+// Copies n <= kReadbackWords words to be->rb_dev, a run of them per workgroup, each of which then stores `seq` at a word of its own behind
+// them (64 bytes apart), visible to the host: 16-byte stores of many compute units, and nobody waits for anybody.
+// (2 MiB: the rows of logits that a step hands back.  The runtime's copy waits for the stream, which retires every kernel in front of it: behind
+// one kernel 49152 words 41 us and 29 here, 151936 65 and 50, but behind the 150 to 200 of a decode step 60 to 100 more: a step of the
+// SmolLM2-135M shape 0.93 -> 0.82 ms, Qwen3-0.6B 1.42 -> 1.36, Llama-3.2-1B 1.25 -> 1.19.)
+constexpr uint32_t kReadbackWords = 524288, kReadbackGroups = 64;
+// Workgroups of a copy: 16384 words 25 us with one, 21 with four; more are not faster.
+inline uint32_t readback_groups(uint32_t n) { return n / 4096 < 1 ? 1 : n / 4096 > kReadbackGroups ? kReadbackGroups : n / 4096; }
 int launch_small_readback(cg_backend *be, const uint32_t *src, uint32_t n, uint32_t seq);
 // A few words from the host travel with the launch, as kernel arguments: n <= kUploadWords words to dst.
 constexpr uint32_t kUploadWords = 64;

@@ -229,14 +229,15 @@ int launch_elementwise(cg_backend *be, int op, cg_dtype dt, const cg_tensor *out
                           : launch_ew_vec<1>(be, op, dt, a);
 }
 
-__global__ void small_readback_kernel(const uint32_t *src, uint32_t n, uint32_t *dst, uint32_t seq) {
-    // one workgroup, since the number behind the words must not be seen before any of them: 16 bytes a lane where src allows it
-    const uint32_t quads = reinterpret_cast<uintptr_t>(src) % 16 == 0 ? n / 4 : 0;
-    for (uint32_t i = threadIdx.x; i < quads; i += blockDim.x) reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
-    for (uint32_t i = quads * 4 + threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
+__global__ __launch_bounds__(256) void small_readback_kernel(const uint32_t *src, uint32_t n, uint32_t *dst, uint32_t seq, uint32_t per) {
+    // a run of `per` words (whole 16-byte pieces) each; the number behind them must not be seen before any of a workgroup's own
+    const uint32_t first = blockIdx.x * per, last = min(n, first + per);
+    const uint32_t quads = reinterpret_cast<uintptr_t>(src) % 16 == 0 ? (last - first) / 4 : 0;
+    for (uint32_t i = threadIdx.x; i < quads; i += blockDim.x) reinterpret_cast<uint4 *>(dst + first)[i] = reinterpret_cast<const uint4 *>(src + first)[i];
+    for (uint32_t i = first + quads * 4 + threadIdx.x; i < last; i += blockDim.x) dst[i] = src[i];
     __threadfence_system();
     __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_store(dst + kReadbackWords, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (threadIdx.x == 0) __hip_atomic_store(dst + kReadbackWords + blockIdx.x * 16, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 struct UploadWords {
@@ -256,7 +257,8 @@ int launch_small_upload(cg_backend *be, uint32_t *dst, const uint32_t *host_word
 }
 
 int launch_small_readback(cg_backend *be, const uint32_t *src, uint32_t n, uint32_t seq) {
-    launch_kernel(small_readback_kernel, dim3(1), dim3(n > 1024 ? 1024 : 256), 0, be->stream, src, n, be->rb_dev, seq);
+    const uint32_t groups = readback_groups(n), per = ((n + groups - 1) / groups + 3) / 4 * 4;
+    launch_kernel(small_readback_kernel, dim3(groups), dim3(256), 0, be->stream, src, n, be->rb_dev, seq, per);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "read-back launch");
 }

@@ -769,14 +769,16 @@ static int wait_and_check(cg_backend *be) {
     return CG_OK;
 }
 
-// The read-back kernel with sequence number `seq` has run (and with it everything before it on the stream): polls the word
-// it writes last.  Launch timings that wait to be read need the stream itself; so does a device that does not answer
+// The read-back kernel with sequence number `seq` has run (and with it everything before it on the stream): polls the words
+// that its workgroups write last.  Launch timings that wait to be read need the stream itself; so does a device that does not answer
 // within a tenth of a second (a fault: the stream's own wait reports it).
-static int wait_for_readback(cg_backend *be, uint32_t seq) {
+static int wait_for_readback(cg_backend *be, uint32_t seq, uint32_t groups) {
     if (be->prof_pending.size() > 2048) return wait_and_check(be);
-    volatile uint32_t *word = be->rb_host + kReadbackWords;
+    volatile uint32_t *word = be->rb_host + kReadbackWords, *const end = word + 16 * groups;
     const auto t0 = std::chrono::steady_clock::now();
-    for (uint32_t spins = 0; *word != seq; spins++) {
+    for (uint32_t spins = 0;; spins++) {
+        while (word != end && *word == seq) word += 16;
+        if (word == end) break;
         if ((spins & 1023) == 1023 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(100)) return wait_and_check(be);
         __builtin_ia32_pause();
     }
@@ -2265,8 +2267,8 @@ int cg_backend_create(int device, cg_backend **out) {
     CG_HIP(hipHostMalloc((void **)&b->fault_host, 64, hipHostMallocMapped));
     memset(b->fault_host, 0, 64);
     CG_HIP(hipHostGetDevicePointer((void **)&b->fault_dev, b->fault_host, 0));
-    CG_HIP(hipHostMalloc((void **)&b->rb_host, (kReadbackWords + 16) * 4, hipHostMallocMapped));
-    memset(b->rb_host, 0, (kReadbackWords + 16) * 4);
+    CG_HIP(hipHostMalloc((void **)&b->rb_host, (kReadbackWords + 16 * kReadbackGroups) * 4, hipHostMallocMapped));
+    memset(b->rb_host, 0, (kReadbackWords + 16 * kReadbackGroups) * 4);
     CG_HIP(hipHostGetDevicePointer((void **)&b->rb_dev, b->rb_host, 0));
     if (const char *fr = getenv("CG_FAST_READBACK")) b->fast_readback = fr[0] != '0';
     CG_HIP(hipHostMalloc((void **)&b->flag_host, 64, hipHostMallocDefault));
@@ -2664,11 +2666,11 @@ static int copy_out(cg_backend *b, const cg_tensor *t, void *dst, size_t len) {
     const void *p;
     int rc = device_ptr(src, &p);
     if (!rc && b->fast_readback && len <= kReadbackWords) {
-        // a few words (the tokens of a decode step): copied by a kernel into pinned memory that the host polls — neither
+        // the tokens or the logits of a step: copied by a kernel into pinned memory that the host polls — neither
         // the runtime's staged copy nor its wake-up stands between the last kernel of a step and the first of the next
         const uint32_t seq = ++b->rb_seq;
         rc = launch_small_readback(b, static_cast<const uint32_t *>(p), (uint32_t)len, seq);
-        if (!rc) rc = wait_for_readback(b, seq);
+        if (!rc) rc = wait_for_readback(b, seq, readback_groups((uint32_t)len));
         if (!rc) memcpy(dst, b->rb_host, len * 4);
     } else if (!rc) {
         hipError_t e = hipMemcpyAsync(dst, p, len * 4, hipMemcpyDeviceToHost, b->stream);
