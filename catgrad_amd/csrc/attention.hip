@@ -188,10 +188,9 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
                 else CG_SEG_KERNEL(32, 8);
 #undef CG_SEG_KERNEL
                 if (!rc) {
-                    const uint64_t nrows = (uint64_t)f1.batch * g.M, waves = kBlock / 64;
-                    launch_kernel(decode_attention_combine_kernel, dim3((uint32_t)((nrows + waves - 1) / waves)), dim3(kBlock), 0,
-                                       be->stream, g.part_o, g.part_ml, static_cast<uint32_t *>(out->buf->ptr), g.splits, g.M,
-                                       (uint32_t)hd, nrows);
+                    const uint64_t nrows = (uint64_t)f1.batch * g.M;
+                    launch_kernel(decode_attention_combine_kernel, dim3((uint32_t)nrows), dim3(kBlock), 0, be->stream, g.part_o, g.part_ml, static_cast<uint32_t *>(out->buf->ptr), g.splits, g.M,
+                                  (uint32_t)hd);
                 }
             }
             be->pool.free(so, cso); // stream-ordered: later users queue behind the combine
@@ -242,9 +241,8 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
         else CG_ROW_KERNEL(32, 1);
 #undef CG_ROW_KERNEL
         if (segmented) {
-            const uint64_t nrows = (uint64_t)f1.batch * g.M, waves = kBlock / 64;
-            launch_kernel(decode_attention_combine_kernel, dim3((uint32_t)((nrows + waves - 1) / waves)), dim3(kBlock), 0,
-                               be->stream, g.part_o, g.part_ml, po, nseg, g.M, (uint32_t)hd, nrows);
+            const uint64_t nrows = (uint64_t)f1.batch * g.M;
+            launch_kernel(decode_attention_combine_kernel, dim3((uint32_t)nrows), dim3(kBlock), 0, be->stream, g.part_o, g.part_ml, po, nseg, g.M, (uint32_t)hd);
             be->pool.free(part_o, co); // stream-ordered: later users queue behind the combine
             be->pool.free(part_ml, cml);
         }
@@ -271,10 +269,9 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
             launch_kernel((decode_attention_kernel<P, 16>), grid, dim3(kBlock), 0, be->stream, g, a);
         else
             launch_kernel((decode_attention_kernel<P, 32>), grid, dim3(kBlock), 0, be->stream, g, a);
-        const uint64_t rows = (uint64_t)f1.batch * g.M, waves = kBlock / 64;
-        launch_kernel(decode_attention_combine_kernel, dim3((uint32_t)((rows + waves - 1) / waves)), dim3(kBlock), 0,
-                           be->stream, g.part_o, g.part_ml, static_cast<uint32_t *>(out->buf->ptr), g.splits, g.M,
-                           (uint32_t)hd, rows);
+        const uint64_t rows = (uint64_t)f1.batch * g.M;
+        launch_kernel(decode_attention_combine_kernel, dim3((uint32_t)rows), dim3(kBlock), 0, be->stream, g.part_o, g.part_ml, static_cast<uint32_t *>(out->buf->ptr), g.splits, g.M,
+                      (uint32_t)hd);
     }
     be->pool.free(po, co); // stream-ordered: later users queue behind the combine
     be->pool.free(pml, cml);

@@ -684,60 +684,58 @@ __global__ __launch_bounds__(kSegBlock) void decode_attention_seg_kernel(const A
     }
 }
 
-// out[b][m][n] = sum_c e^(m_c - g) o_c[n] / sum_c e^(m_c - g) l_c.  A wave per (batch entry, query
-// row): lane c first holds the statistics of chunk c (so each weight e^(m_c - g) is computed once
-// and handed round by lane broadcast), then lane n sums output element n (and n + 64) over the chunks.
-__global__ __launch_bounds__(kBlock) void decode_attention_combine_kernel(const float *part_o, const float *part_ml,
-                                                                          uint32_t *out, uint32_t splits, uint32_t M,
-                                                                          uint32_t hd, uint64_t rows) {
-    const uint32_t lane = threadIdx.x % 64;
-    const uint64_t r = (uint64_t)blockIdx.x * (kBlock / 64) + threadIdx.x / 64;
-    if (r >= rows) return;
-    const uint32_t m = (uint32_t)(r % M);
-    const uint64_t b = r / M;
+// out[b][m][n] = sum_c e^(m_c - g) o_c[n] / sum_c e^(m_c - g) l_c.  A workgroup per (batch entry, query row), whose waves share the
+// chunks: lane c first holds the statistics of chunk c (each wave computes each weight e^(m_c - g) once and reads it from that lane), then
+// lane n sums output element n (and n + 64) over the wave's chunks, and the waves' sums meet in LDS.
+// Bound by latency: one trip to memory.  A wave per row, with a shuffle per chunk, took 4.74 us for 16 rows of 32 chunks of 128; so 2.83.
+__global__ __launch_bounds__(kBlock) void decode_attention_combine_kernel(const float *part_o, const float *part_ml, uint32_t *out, uint32_t splits, uint32_t M, uint32_t hd) {
+    constexpr uint32_t kWaves = kBlock / 64, kTrip = 64, kMine = kTrip / kWaves; // chunks per trip, of which a wave takes every fourth
+    __shared__ float sums[kWaves][2][64];
+    const uint32_t lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const uint64_t r = blockIdx.x, b = r / M;
+    const uint32_t m = (uint32_t)(r - b * M);
     const float *ml = part_ml + (b * splits * M + m) * 2; // chunk c at + c * M * 2
     const float *po = part_o + (b * splits * M + m) * (uint64_t)hd; // chunk c at + c * M * hd
-    constexpr uint32_t kGroup = 32; // chunks per trip to memory
-    const bool wide = lane + 64 < hd;
-    float gmax = kF32Min;
-    float num0 = 0.0f, num1 = 0.0f, den = 0.0f;
-    for (uint32_t c0 = 0; c0 < splits; c0 += kGroup) {
-        // every load of the group is asked for before anything is used
-        float v0[kGroup], v1[kGroup];
+    const uint32_t d0 = min(lane, hd - 1), d1 = min(lane + 64, hd - 1);
+    float gmax = kF32Min, num0 = 0.0f, num1 = 0.0f, den = 0.0f;
+    for (uint32_t c0 = 0; c0 < splits; c0 += kTrip) {
+        // every load of the trip is asked for before anything is used (a chunk behind the last: the last one's, taken as zero)
+        const uint32_t c = min(c0 + lane, splits - 1);
+        const float2 mine = *reinterpret_cast<const float2 *>(ml + (uint64_t)c * M * 2);
+        float v0[kMine], v1[kMine];
 #pragma unroll
-        for (uint32_t k = 0; k < kGroup; k++) {
-            v0[k] = 0.0f;
-            v1[k] = 0.0f;
-            if (c0 + k < splits) {
-                const float *o = po + (uint64_t)(c0 + k) * M * hd;
-                if (lane < hd) v0[k] = o[lane];
-                if (wide) v1[k] = o[lane + 64];
-            }
+        for (uint32_t k = 0; k < kMine; k++) {
+            const float *o = po + (uint64_t)min(c0 + wave + k * kWaves, splits - 1) * M * hd;
+            v0[k] = o[d0];
+            v1[k] = o[d1];
         }
-        const uint32_t c = c0 + lane;
-        const bool mine = lane < kGroup && c < splits;
-        const float cm = mine ? ml[(uint64_t)c * M * 2] : kF32Min, cl = mine ? ml[(uint64_t)c * M * 2 + 1] : 0.0f;
-        float m2 = fmaxf(gmax, cm);
-        m2 = asf(group_fold<32>(asu(m2), LargerWords{}));
-        m2 = __shfl(m2, 0);
+        const bool there = c0 + lane < splits;
+        const float m2 = fmaxf(gmax, asf(wave_fold<1>(asu(there ? mine.x : kF32Min), LargerWords{})));
         // what was summed so far is relative to the old maximum
-        const float rescale = expf(gmax - m2);
+        const float rescale = expf(gmax - m2), w = there ? expf(mine.x - m2) : 0.0f;
+        gmax = m2;
         num0 *= rescale;
         num1 *= rescale;
-        den *= rescale;
-        gmax = m2;
-        const float w = mine ? expf(cm - gmax) : 0.0f;
-        den = fmaf(w, cl, den);
+        den = fmaf(w, there ? mine.y : 0.0f, den * rescale);
 #pragma unroll
-        for (uint32_t k = 0; k < kGroup; k++) {
-            const float wk = __shfl(w, (int)k);
-            num0 = fmaf(wk, v0[k], num0);
-            num1 = fmaf(wk, v1[k], num1);
+        for (uint32_t k = 0; k < kMine; k++) {
+            const uint32_t at = wave + k * kWaves;
+            const bool in = c0 + at < splits;
+            const float wk = asf((uint32_t)__builtin_amdgcn_readlane((int)asu(w), (int)at));
+            num0 = fmaf(wk, in ? v0[k] : 0.0f, num0);
+            num1 = fmaf(wk, in ? v1[k] : 0.0f, num1);
         }
     }
-    den = wave_add<1>(den);
-    if (lane < hd) out[r * hd + lane] = asu(num0 / den);
-    if (lane + 64 < hd) out[r * hd + lane + 64] = asu(num1 / den);
+    den = wave_add<1>(den); // (every wave has all chunks' sums)
+    sums[wave][0][lane] = num0;
+    sums[wave][1][lane] = num1;
+    __syncthreads();
+    const uint32_t d = threadIdx.x;
+    if (d >= hd) return; // (hd <= 128: the first two waves)
+    float s = 0.0f;
+#pragma unroll
+    for (uint32_t k = 0; k < kWaves; k++) s += sums[k][d / 64][d % 64];
+    out[r * hd + d] = asu(s / den);
 }
 
 // ---- prefill: causal attention of many query rows in one pass ---------------------------------------------------
