@@ -143,61 +143,71 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
     // V is pulled into a compute unit once.  As many segments as put a workgroup on every compute unit, at most
     // attn_seg_max() (each segment is one more partial result to merge), each a whole number of passes.  Taken for long
     // caches, and from 1024 positions when there are more query rows than compute units.  Measured with its combine launch
-    // against the kernels below (batch 4 x 8 KV heads x 4 rows, head_dim 64): 2100 positions 20.4 against 19.7 us (the segment
-    // kernel alone 13.6 against 19.7: what it saves, the combine launch and the hand-over to it cost again), 6000 positions 34.9
-    // against 34.9, 9000 positions 44 against 55, 12000 positions 53 against 64; batch 16 at 2100 positions 42 against 46.
-    // With at most 8 groups (a single sequence) the kernels below leave most of the device idle and the segments win from 2560
-    // positions on: 8 KV heads, head_dim 128: 3000 positions 17.2 against 28.3 us, 12000 positions 31.7 against 59.0; 3 KV
-    // heads, head_dim 64: 4500 positions 16.7 against 20.0, 12000 positions 22.1 against 40.5 (2100 positions: 15.8 against 15.8).
-    // So a single sequence takes the segments from 128 Ki cached values per KV head on (1024 positions of head_dim 128, 2048
-    // of 64): the Qwen3-0.6B shape's decode step (8 KV heads, head_dim 128, 16 query rows, 1024 to 1152 positions) takes 1.45
-    // to 1.53 ms with them against 1.64 to 1.66 ms with its 32 workgroups of the kernel below.
+    // against the kernels below (batch 4 x 8 KV heads x 4 rows, head_dim 64): 9000 positions 44 against 55, 12000 positions 53 against 64;
+    // batch 16 at 2100 positions 42 against 46.  A single sequence (at most 8 groups) leaves the kernels below most of the device idle:
+    // beyond kRowMaxT it always takes the segments (8 KV heads, head_dim 128: 12000 positions 31.7 against 59.0).
+    // Up to kRowMaxT by what either takes, in us: a row is its compute unit's share of the cache; the segments are two launches and the
+    // hand-over between them (1 us) up to what the device streams.  One row and one segment pair, SmolLM2-135M shape (3 KV heads of 64, one
+    // sequence) 512 positions 7.3 and 10.0, 1024 11.6 and 10.2, 2047 17.3 and 10.1; Qwen3-0.6B (8 of 128) 384 10.4 and 10.2, 512 12.1 and
+    // 10.2, 768 15.6 and 10.3, four sequences 512 12.7 and 10.9, 1024 19.2 and 15.0; Llama-3.2-1B (8 of 64) 1024 11.3 and 11.0, 1536 14.5
+    // and 11.1, four sequences 1536 15.5 and 14.4, 2047 18.4 and 16.0.
+    auto segments_win = [&] {
+        const double values = (double)T * (double)hd, mb = 8e-6 * values * (double)f1.batch;
+        const double row = 5.0 + 1.0e-4 * values * (qrows > 128 ? 1.3 : 1.0); // (more rows: a whole one per compute unit)
+        const double seg = std::max(10.2, 7.6 + 0.22 * mb) + (f1.M > 4 ? 2.5 : f1.M > 3 ? 1.0 : 0.0) + 1.0;
+        return T > kRowMaxT ? f1.batch <= 8 && T * hd >= 131072 : seg < row;
+    };
     // (Merging the segments inside the kernel — the workgroup that counts itself last at a device-scope counter reads the
     // others' results — was measured and costs what the combine launch costs: the stores must reach memory, the count must come
     // back and the loads go out again, 6 to 7 us in all; with a release / acquire fence per workgroup 24.0 against 19.3 us.)
-    if (be->attn_seg_from > 0 && (T >= be->attn_seg_from || (qrows > 256 && T >= 1024) || (f1.batch <= 8 && T * hd >= 131072))) {
+    if (be->attn_seg_from > 0 && (T >= be->attn_seg_from || (qrows > 256 && T >= 1024) || segments_win())) {
         const int64_t tpb = hd == 64 ? kSegBlock / 16 : kSegBlock / 32;
         int64_t want = std::min<int64_t>(attn_seg_max(), std::max<int64_t>(1, 256 / f1.batch));
         want = std::max<int64_t>(1, std::min<int64_t>(want, T / 64));
         const int64_t chunk = ((T + want - 1) / want + tpb - 1) / tpb * tpb;
         if (chunk <= kSegMaxChunk) {
+            const uint32_t other_chunk = g.chunk, other_splits = g.splits;
             g.chunk = (uint32_t)chunk;
             g.splits = (uint32_t)((T + chunk - 1) / chunk);
             const size_t o_b = (size_t)f1.batch * g.splits * g.M * hd * 4, ml_b = (size_t)f1.batch * g.splits * g.M * 2 * 4;
             void *so = nullptr, *sml = nullptr;
             size_t cso = 0, csml = 0;
-            rc = be->pool.alloc(o_b, &so, &cso);
-            if (rc) return rc;
-            rc = be->pool.alloc(ml_b, &sml, &csml);
-            if (rc) {
+            bool room = !be->pool.alloc(o_b, &so, &cso);
+            if (room && be->pool.alloc(ml_b, &sml, &csml)) {
                 be->pool.free(so, cso);
-                return rc;
+                room = false;
             }
-            g.part_o = static_cast<float *>(so);
-            g.part_ml = static_cast<float *>(sml);
-            be->programs_compiled++;
-            {
-                ProfScope prof(be, CG_K_GEMM_SKINNY, distinct_bytes(q) + distinct_bytes(kt) + distinct_bytes(v) + distinct_bytes(out));
-                const bool one_trip = chunk <= 5 * tpb;
-                const uint32_t nb = (uint32_t)f1.batch;
+            if (!room) { // the kernels below: up to kRowMaxT without scratch memory
+                (void)hipGetLastError();
+                g.chunk = other_chunk;
+                g.splits = other_splits;
+            } else {
+                g.part_o = static_cast<float *>(so);
+                g.part_ml = static_cast<float *>(sml);
+                be->programs_compiled++;
+                {
+                    ProfScope prof(be, CG_K_GEMM_SKINNY, distinct_bytes(q) + distinct_bytes(kt) + distinct_bytes(v) + distinct_bytes(out));
+                    const bool one_trip = chunk <= 5 * tpb;
+                    const uint32_t nb = (uint32_t)f1.batch;
 #define CG_SEG_KERNEL(LPT, MMV)                                                                    \
-    rc = one_trip ? launch_seg_kernel<P, LPT, MMV, 5, false>(be, g, a, nb) : launch_seg_kernel<P, LPT, MMV, 4, true>(be, g, a, nb)
-                if (hd == 64 && g.M <= 4) CG_SEG_KERNEL(16, 4);
-                else if (hd == 64) CG_SEG_KERNEL(16, 8);
-                else if (g.M <= 4) CG_SEG_KERNEL(32, 4);
-                else CG_SEG_KERNEL(32, 8);
+        rc = one_trip ? launch_seg_kernel<P, LPT, MMV, 5, false>(be, g, a, nb) : launch_seg_kernel<P, LPT, MMV, 4, true>(be, g, a, nb)
+                    if (hd == 64 && g.M <= 4) CG_SEG_KERNEL(16, 4);
+                    else if (hd == 64) CG_SEG_KERNEL(16, 8);
+                    else if (g.M <= 4) CG_SEG_KERNEL(32, 4);
+                    else CG_SEG_KERNEL(32, 8);
 #undef CG_SEG_KERNEL
-                if (!rc) {
-                    const uint64_t nrows = (uint64_t)f1.batch * g.M;
-                    launch_kernel(decode_attention_combine_kernel, dim3((uint32_t)nrows), dim3(kBlock), 0, be->stream, g.part_o, g.part_ml, static_cast<uint32_t *>(out->buf->ptr), g.splits, g.M,
-                                  (uint32_t)hd);
+                    if (!rc) {
+                        const uint64_t nrows = (uint64_t)f1.batch * g.M;
+                        launch_kernel(decode_attention_combine_kernel, dim3((uint32_t)nrows), dim3(kBlock), 0, be->stream, g.part_o, g.part_ml, static_cast<uint32_t *>(out->buf->ptr), g.splits, g.M,
+                                      (uint32_t)hd);
+                    }
                 }
+                be->pool.free(so, cso); // stream-ordered: later users queue behind the combine
+                be->pool.free(sml, csml);
+                if (rc) return rc;
+                hipError_t e = hipGetLastError();
+                return e == hipSuccess ? CG_OK : hip_fail(e, "decode attention launch");
             }
-            be->pool.free(so, cso); // stream-ordered: later users queue behind the combine
-            be->pool.free(sml, csml);
-            if (rc) return rc;
-            hipError_t e = hipGetLastError();
-            return e == hipSuccess ? CG_OK : hip_fail(e, "decode attention launch");
         }
     }
     const bool one_launch = T <= std::min<int64_t>(attn_whole_limit(), kRowMaxT) && (T <= 1024 || qrows <= 256);
