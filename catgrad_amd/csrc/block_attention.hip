@@ -7,7 +7,9 @@
 //   attention_turn_*_kernel   the same with rotations and unit heads
 //   attention_scores_kernel   a workgroup per (token, kv head, 128 keys): scores, and their maximum and sum per head; with a
 //                             few new tokens the preparation as well
-//   attention_mix_kernel      the same split: soft-max weights of every head, mixed, times the values of the kv head
+//   attention_columns_kernel  a few rows: a workgroup per (token, kv head, 16 columns of the values) over all keys, the soft-max
+//                             weights of every head, mixed, times the values
+//   attention_mix_kernel      other rows, split as the scores are: the same for 128 keys
 //   attention_sum_kernel      partial results of a token's key segments added up
 #include "blocks.hpp"
 #include "device_utils.hpp"
@@ -26,6 +28,12 @@ __device__ __forceinline__ float block_sum(float v, float *red) {
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     return (red[0] + red[1]) + (red[2] + red[3]);
+}
+__device__ __forceinline__ float2 block_sum2(float2 v, float2 *red) { // (the first use of `red`)
+    v = make_float2(wave_add<1>(v.x), wave_add<1>(v.y));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return make_float2((red[0].x + red[1].x) + (red[2].x + red[3].x), (red[0].y + red[1].y) + (red[2].y + red[3].y));
 }
 __device__ __forceinline__ float slope_of(uint32_t h, uint32_t heads) { return exp2f(-8.0f * (float)(h + 1) / (float)heads); }
 
@@ -185,14 +193,39 @@ __device__ __forceinline__ float row_squares(const float *__restrict__ x, uint32
     return m;
 }
 
+// The same in two parts, the loads and the sum, for rows whose loads a thread can hold.
+struct RowLoads {
+    float4 x[2];
+    bool held;
+    __device__ __forceinline__ void ask(const float *__restrict__ p, uint32_t n) {
+        held = n % 4 == 0 && n <= 8 * kThreads && (reinterpret_cast<uintptr_t>(p) & 15) == 0;
+        if (held)
+#pragma unroll
+            for (uint32_t i = 0; i < 2; i++) x[i] = reinterpret_cast<const float4 *>(p)[min(threadIdx.x + i * kThreads, n / 4 - 1)];
+    }
+    __device__ __forceinline__ float squares(const float *__restrict__ p, uint32_t n) const {
+        if (!held) return row_squares(p, n);
+        float m = 0.0f;
+#pragma unroll
+        for (uint32_t i = 0; i < 2; i++)
+            if (threadIdx.x + i * kThreads < n / 4) m = fmaf(x[i].x, x[i].x, fmaf(x[i].y, x[i].y, fmaf(x[i].z, x[i].z, fmaf(x[i].w, x[i].w, m))));
+        return m;
+    }
+};
+
 // Four lanes share a key; REP query heads of the kv head at a time (blockIdx.y = kv head and which of its head groups).
 // FRESH (a few new tokens): the queries and the new keys are normed here, from the projections as they are, and a token's
 // own workgroups of the last segment write its key and value rows into the cache; the cache is not read at new positions.
+// `exponentials`: behind the segment's maximum, instead of the scores.
+// A decode step runs a few dozen workgroups, each as long as its chain of loads: the rows that are normed and the first 128
+// values of every cached key are asked for together, at the start, and a query value in LDS is read once for both of a
+// thread's keys.  16 heads on 8 of 128 values: 5.9 us, where each loop asked for its own rows 7.3.
 template <int REP, int VW, bool FRESH>
-__global__ __launch_bounds__(kThreads) void attention_scores_kernel(const AttentionPlan p, const float *__restrict__ q, const uint32_t row0, const uint32_t nseg,
-                                                                    float *__restrict__ scores, float2 *__restrict__ stats) {
-    extern __shared__ float lds[]; // [REP][dim] queries, [REP][kSeg] scores, FRESH: [S][dim] new keys
+__global__ __launch_bounds__(kThreads, 4) void attention_scores_kernel(const AttentionPlan p, const float *__restrict__ q, const uint32_t row0, const uint32_t nseg,
+                                                                    float *__restrict__ scores, float2 *__restrict__ stats, const bool exponentials) {
+    extern __shared__ __align__(16) float lds[]; // [REP][dim] queries, [REP][kSeg] scores, FRESH: [S][dim] new keys
     __shared__ float red[kWaves];
+    __shared__ float2 red2[kWaves];
     const uint32_t rep = p.heads / p.kv_heads, groups = (rep + REP - 1) / REP;
     const uint32_t g = blockIdx.y / groups, h0 = g * rep + (blockIdx.y - g * groups) * REP, nh = min((uint32_t)REP, (g + 1) * rep - h0);
     const uint32_t r = row0 + blockIdx.z, b = r / p.S, s = r - b * p.S, seg = blockIdx.x;
@@ -200,26 +233,63 @@ __global__ __launch_bounds__(kThreads) void attention_scores_kernel(const Attent
     uint32_t lo, hi;
     visible(p, s, &lo, &hi);
     const uint32_t j0 = lo + seg * kSeg;
+    const float *K = p.keys + ((int64_t)b * p.kv_heads + g) * p.k_block;
+    const uint32_t sub = threadIdx.x & 3, nd = p.dim / VW, old = FRESH ? p.cached : hi; // old: the keys that are read from the cache
+    constexpr int KEYS = kSeg * 4 / kThreads, AHEAD = VW < 4 ? 1 : FRESH ? 8 : 4;
+    float4 kv[KEYS][AHEAD];
+    auto key_at = [&](int k) { return j0 + (threadIdx.x >> 2) + k * (kThreads / 4); };
+    auto ask_keys = [&] { // (clamped, not tested: the cache has a row for every new token)
+        if constexpr (VW == 4)
+#pragma unroll
+            for (int k = 0; k < KEYS; k++) {
+                const float4 *kp = reinterpret_cast<const float4 *>(K + (int64_t)min(key_at(k), max(old, 1u) - 1) * p.dim);
+#pragma unroll
+                for (int i = 0; i < AHEAD; i++) kv[k][i] = kp[min(sub + 4 * i, nd - 1)];
+            }
+    };
     if constexpr (FRESH) {
-        const uint32_t nq = p.heads * p.dim, nk = p.kv_heads * p.dim;
-        const float *qr = p.q.p + (int64_t)r * p.q.pitch;
+        const uint32_t nq = p.heads * p.dim, nk = p.kv_heads * p.dim, own = p.cached + s;
+        const float *qr = p.q.p + (int64_t)r * p.q.pitch, *kn = p.k.p + (int64_t)r * p.k.pitch;
+        const bool mine = own >= j0 && own < j0 + kSeg;
+        RowLoads ql, kl;
+        ql.held = kl.held = false;
+        if (p.q_norm) ql.ask(qr, nq);
+        const uint32_t e0 = min(h0 * p.dim + threadIdx.x, nq - 1), d0 = min(g * p.dim + threadIdx.x, nk - 1);
+        const float q0 = qr[e0], qw = p.q_norm ? p.q_norm[e0] : 1.0f;
+        float k0 = 0.0f, kw = 1.0f;
+        if (mine) {
+            if (p.k_norm) kl.ask(kn, nk);
+            k0 = kn[d0];
+            if (p.k_norm) kw = p.k_norm[d0];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        ask_keys();
+        __builtin_amdgcn_sched_barrier(0);
         float f = p.scale;
         if (p.temp_every) f *= 1.0f + p.temp_coef * logf((float)((p.position + s + 1) / p.temp_every + 1));
-        const float rms = p.q_norm ? 1.0f / sqrtf(block_sum(row_squares(qr, nq), red) / (float)nq + p.eps) : 1.0f;
+        float2 squares = make_float2(0.0f, 0.0f);
+        if (p.q_norm) squares.x = ql.squares(qr, nq);
+        if (mine && p.k_norm) squares.y = kl.squares(kn, nk);
+        if (p.q_norm || (mine && p.k_norm)) squares = block_sum2(squares, red2);
+        const float rms = p.q_norm ? 1.0f / sqrtf(squares.x / (float)nq + p.eps) : 1.0f;
         for (uint32_t i = threadIdx.x; i < REP * p.dim; i += kThreads) {
             const uint32_t h = i / p.dim, e = h0 * p.dim + i;
             float v = 0.0f;
-            if (h < nh) v = p.q_norm ? qr[e] * rms * p.q_norm[e] : qr[e];
+            if (h < nh) {
+                const float x = i < kThreads ? q0 : qr[e];
+                v = p.q_norm ? x * rms * (i < kThreads ? qw : p.q_norm[e]) : x;
+            }
             lds[i] = v * f;
         }
         for (uint32_t t = 0; t <= s; t++) { // the new keys among this workgroup's
             const uint32_t j = p.cached + t;
             if (j < j0 || j >= j0 + kSeg) continue;
             const float *kr = p.k.p + ((int64_t)b * p.S + t) * p.k.pitch;
-            const float fk = p.k_norm ? 1.0f / sqrtf(block_sum(row_squares(kr, nk), red) / (float)nk + p.eps) : 1.0f;
+            const float fk = p.k_norm ? 1.0f / sqrtf((t == s ? squares.y : block_sum(row_squares(kr, nk), red)) / (float)nk + p.eps) : 1.0f;
             float *kc = p.keys + ((int64_t)b * p.kv_heads + g) * p.k_block + (int64_t)j * p.dim;
             for (uint32_t d = threadIdx.x; d < p.dim; d += kThreads) {
-                const float v = p.k_norm ? kr[g * p.dim + d] * fk * p.k_norm[g * p.dim + d] : kr[g * p.dim + d];
+                const bool there = t == s && d < kThreads;
+                const float x = there ? k0 : kr[g * p.dim + d], v = p.k_norm ? x * fk * (there ? kw : p.k_norm[g * p.dim + d]) : x;
                 fresh[t * p.dim + d] = v;
                 if (t == s && h0 == g * rep) kc[d] = v;
             }
@@ -228,54 +298,82 @@ __global__ __launch_bounds__(kThreads) void attention_scores_kernel(const Attent
                     p.values[((int64_t)b * p.kv_heads + g) * p.v_block + (int64_t)j * p.vdim + d] = p.v.p[(int64_t)r * p.v.pitch + g * p.vdim + d];
         }
     } else {
+        ask_keys();
         for (uint32_t i = threadIdx.x; i < REP * p.dim; i += kThreads) {
             const uint32_t h = i / p.dim, d = i - h * p.dim;
             lds[i] = h < nh ? q[((int64_t)r * p.heads + h0 + h) * p.dim + d] : 0.0f;
         }
     }
     __syncthreads();
-    const float *K = p.keys + ((int64_t)b * p.kv_heads + g) * p.k_block;
-    const uint32_t sub = threadIdx.x & 3, nd = p.dim / VW;
-    for (uint32_t key = threadIdx.x >> 2; key < kSeg; key += kThreads / 4) {
-        const uint32_t j = j0 + key;
-        float acc[REP] = {};
-        if (j < hi) {
+    float acc[KEYS][REP] = {}, odd[KEYS][REP] = {}; // (two chains: half the rounding errors in a row)
+    if constexpr (VW == 4) {
+        auto row_at = [&](int k) -> const float4 * { // in the cache or among the new keys
+            const uint32_t j = key_at(k);
+            if (FRESH && j >= old && j < hi) return reinterpret_cast<const float4 *>(fresh + (j - old) * p.dim);
+            return reinterpret_cast<const float4 *>(K + (int64_t)min(j, max(old, 1u) - 1) * p.dim);
+        };
+        if constexpr (FRESH)
+#pragma unroll
+            for (int k = 0; k < KEYS; k++)
+                if (key_at(k) >= old && key_at(k) < hi)
+#pragma unroll
+                    for (int i = 0; i < AHEAD; i++) kv[k][i] = reinterpret_cast<const float4 *>(fresh + (key_at(k) - old) * p.dim)[min(sub + 4 * i, nd - 1)];
+        auto multiply = [&](uint32_t i, const float4(&x)[KEYS]) {
+#pragma unroll
+            for (int h = 0; h < REP; h++) {
+                const float4 w = *reinterpret_cast<const float4 *>(lds + h * p.dim + 4 * i);
+#pragma unroll
+                for (int k = 0; k < KEYS; k++) {
+                    acc[k][h] = fmaf(x[k].z, w.z, fmaf(x[k].x, w.x, acc[k][h]));
+                    odd[k][h] = fmaf(x[k].w, w.w, fmaf(x[k].y, w.y, odd[k][h]));
+                }
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++)
+            if (sub + 4 * i < nd) {
+                const float4 x[KEYS] = {kv[0][i], kv[1][i]};
+                multiply(sub + 4 * i, x);
+            }
+#pragma unroll 2
+        for (uint32_t i = sub + 4 * AHEAD; i < nd; i += 4) {
+            const float4 x[KEYS] = {row_at(0)[i], row_at(1)[i]};
+            multiply(i, x);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < KEYS; k++) {
+            const uint32_t j = key_at(k);
             auto walk = [&](const float *kp) {
 #pragma unroll 4
-                for (uint32_t i = sub; i < nd; i += 4) {
-                    float kv[VW];
-                    if constexpr (VW == 4) {
-                        const float4 t = *reinterpret_cast<const float4 *>(kp + 4 * i);
-                        kv[0] = t.x, kv[1] = t.y, kv[2] = t.z, kv[3] = t.w;
-                    } else {
-                        kv[0] = kp[i];
-                    }
+                for (uint32_t i = sub; i < nd; i += 4)
 #pragma unroll
-                    for (int h = 0; h < REP; h++)
-#pragma unroll
-                        for (int e = 0; e < VW; e++) acc[h] = fmaf(kv[e], lds[h * p.dim + VW * i + e], acc[h]);
-                }
+                    for (int h = 0; h < REP; h++) acc[k][h] = fmaf(kp[i], lds[h * p.dim + i], acc[k][h]);
             };
-            if (FRESH && j >= p.cached) walk(fresh + (j - p.cached) * p.dim);
+            if (j >= hi) continue;
+            if (FRESH && j >= old) walk(fresh + (j - old) * p.dim);
             else walk(K + (int64_t)j * p.dim);
         }
+    }
+#pragma unroll
+    for (int k = 0; k < KEYS; k++)
 #pragma unroll
         for (int h = 0; h < REP; h++) {
-            float v = acc[h];
-            v = add_across<2>(add_across<1>(v));
+            const uint32_t j = key_at(k);
+            float v = add_across<2>(add_across<1>(acc[k][h] + odd[k][h]));
             if (sub == 0) {
                 if (p.bias) v -= slope_of(h0 + h, p.heads) * (float)(int)(p.cached + s - j);
-                sc[h * kSeg + key] = j < hi ? v : -INFINITY;
+                sc[h * kSeg + j - j0] = j < hi ? v : -INFINITY;
             }
         }
-    }
     __syncthreads();
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (uint32_t h = wave; h < nh; h += kWaves) {
-        const float a = sc[h * kSeg + lane], c = sc[h * kSeg + 64 + lane];
-        float m = fmaxf(a, c);
-        m = asf(wave_fold<1>(asu(m), LargerWords{}));
-        const float l = m == -INFINITY ? 0.0f : wave_add<1>(expf(a - m) + expf(c - m));
+        float a = sc[h * kSeg + lane], c = sc[h * kSeg + 64 + lane];
+        const float m = asf(wave_fold<1>(asu(fmaxf(a, c)), LargerWords{}));
+        const bool none = m == -INFINITY;
+        const float ea = none ? 0.0f : expf(a - m), ec = none ? 0.0f : expf(c - m), l = wave_add<1>(ea + ec);
+        if (exponentials) a = ea, c = ec;
         const int64_t head = (int64_t)blockIdx.z * p.heads + h0 + h;
         float *o = scores + (head * nseg + seg) * kSeg;
         o[lane] = a;
@@ -386,6 +484,112 @@ __global__ __launch_bounds__(kThreads) void attention_mix_kernel(const Attention
     }
 }
 
+// The same for a few rows behind a cache of a few thousand keys: a workgroup per (16 columns of the values, heads of a kv head, token)
+// over all keys, a thread per key for the weights and per four columns of every 256th key for the products.  What bounds such a step
+// is the chain from one launch to the next, not bytes: this split ends in the results themselves where segments need a third launch
+// to add them, and its weights stay in the registers of the threads that made them, which read no exponentials of other threads.
+// The exponentials are taken once per 16 columns instead of once.
+// 16 heads on 8 of 128 values, 800 keys, one token: 5.5 us, where mixing by segments took 10.1 and adding them 3.8; 32 heads on 8 of 64 values, 7.9 for 16.6.
+constexpr int kColumns = 16, kColumnThreads = 1024, kColumnWaves = kColumnThreads / 64;
+constexpr uint64_t column_floats(uint32_t rep, uint32_t slots, uint32_t nseg) { return (uint64_t)nseg * ((slots + 15) / 16 * 16) * rep + rep * kColumnThreads + kColumnWaves * rep * kColumns; }
+
+template <int REP>
+__global__ __launch_bounds__(kColumnThreads) void attention_columns_kernel(const AttentionPlan p, const uint32_t row0, const uint32_t nseg,
+                                                                           const float *__restrict__ scores, const float2 *__restrict__ stats) {
+    extern __shared__ __align__(16) float lds[]; // [REP][threads] weights, [waves][REP][16] sums, [nseg][slots][REP] factors of the exponentials
+    const uint32_t rep = p.heads / p.kv_heads, groups = (rep + REP - 1) / REP;
+    const uint32_t g = blockIdx.y / groups, h0 = g * rep + (blockIdx.y - g * groups) * REP, nh = min((uint32_t)REP, (g + 1) * rep - h0);
+    const uint32_t r = row0 + blockIdx.z, b = r / p.S, s = r - b * p.S, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const uint32_t first = p.talk ? 0 : h0, nm = p.talk ? p.heads : nh;
+    float *wt = lds, *red = wt + REP * kColumnThreads, *tm = red + kColumnWaves * REP * kColumns;
+    uint32_t lo, hi;
+    visible(p, s, &lo, &hi);
+    const uint32_t keys = hi - lo, sub = tid & 3, turn = tid >> 2;
+    constexpr int TURNS = 4, HEADS = kColumnWaves; // rows of values and heads' exponentials in flight
+    const uint32_t padded = (nm + HEADS - 1) / HEADS * HEADS;
+    const float *V = p.values + ((int64_t)b * p.kv_heads + g) * p.v_block + (int64_t)lo * p.vdim + min(blockIdx.x * kColumns + 4 * sub, p.vdim - 4);
+    const float *sc = scores + ((int64_t)blockIdx.z * p.heads + first) * nseg * kSeg;
+    const float2 *st = stats + ((int64_t)blockIdx.z * p.heads + first) * nseg;
+    float x[HEADS];
+    float4 v[TURNS];
+    auto ask_scores = [&](uint32_t k0, uint32_t h) { // (clamped, not tested)
+        const uint32_t at = min(k0 + tid, nseg * kSeg - 1);
+#pragma unroll
+        for (int e = 0; e < HEADS; e++) x[e] = sc[min(h + e, nm - 1) * (nseg * kSeg) + at];
+    };
+    auto ask_values = [&](uint32_t k0) {
+#pragma unroll
+        for (int i = 0; i < TURNS; i++) v[i] = *reinterpret_cast<const float4 *>(V + (int64_t)min(k0 + turn + i * (kColumnThreads / 4), keys - 1) * p.vdim);
+    };
+    const float2 mine = st[min(wave, nm - 1) * nseg + min(lane, nseg - 1)];
+    auto mixing = [&](uint32_t h, int o) { // of head h in the results of head h0 + o
+        if (o >= nh || h >= nm) return 0.0f;
+        return p.talk ? p.talk[(int64_t)(h0 + o) * p.heads + h] : o == h ? 1.0f : 0.0f;
+    };
+    float talked[REP];
+#pragma unroll
+    for (int o = 0; o < REP; o++) talked[o] = mixing(wave, o);
+    __builtin_amdgcn_sched_barrier(0);
+    ask_scores(0, 0);
+    ask_values(0);
+    __builtin_amdgcn_sched_barrier(0);
+    for (uint32_t h = wave; h < padded; h += HEADS) { // a wave per head, a lane per segment; the heads behind the last one weigh nothing
+        float2 t = h == wave ? mine : st[min(h, nm - 1) * nseg + min(lane, nseg - 1)];
+        if (lane >= nseg) t = make_float2(-INFINITY, 0.0f);
+        const float m = fmaxf(p.zero_sink ? 0.0f : -INFINITY, asf(wave_fold<1>(asu(t.x), LargerWords{})));
+        const float up = t.y > 0.0f ? expf(t.x - m) : 0.0f;
+        const float f = up / (wave_add<1>(t.y > 0.0f ? t.y * up : 0.0f) + (p.zero_sink ? expf(-m) : 0.0f));
+        if (lane < nseg)
+#pragma unroll
+            for (int o = 0; o < REP; o++) tm[(lane * padded + h) * REP + o] = h < nm ? f * (h == wave ? talked[o] : mixing(h, o)) : 0.0f;
+    }
+    float acc[REP][4] = {};
+    for (uint32_t k0 = 0; k0 < keys; k0 += kColumnThreads) {
+        if (k0) {
+            ask_scores(k0, 0);
+            ask_values(k0);
+        }
+        __syncthreads();
+        if (k0 + (tid & ~63u) < keys) { // (the keys of a wave lie in one segment)
+            float w[REP] = {};
+            const float *f = tm + (k0 + tid) / kSeg * padded * REP;
+            for (uint32_t h = 0; h < nm; h += HEADS) {
+                if (h) ask_scores(k0, h);
+#pragma unroll
+                for (int e = 0; e < HEADS; e++)
+#pragma unroll
+                    for (int o = 0; o < REP; o++) w[o] = fmaf(f[(h + e) * REP + o], x[e], w[o]);
+            }
+#pragma unroll
+            for (int o = 0; o < REP; o++) wt[o * kColumnThreads + tid] = w[o];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < TURNS; i++) {
+            const uint32_t k = turn + i * (kColumnThreads / 4);
+            if (k0 + k < keys)
+#pragma unroll
+                for (int o = 0; o < REP; o++) {
+                    const float f = wt[o * kColumnThreads + k];
+                    acc[o][0] = fmaf(f, v[i].x, acc[o][0]), acc[o][1] = fmaf(f, v[i].y, acc[o][1]);
+                    acc[o][2] = fmaf(f, v[i].z, acc[o][2]), acc[o][3] = fmaf(f, v[i].w, acc[o][3]);
+                }
+        }
+    }
+#pragma unroll
+    for (int o = 0; o < REP; o++) { // (column 4 sub + e in row e of the lanes)
+        const float sum = four_sums(acc[o][0], acc[o][1], acc[o][2], acc[o][3]);
+        if ((lane & 15) < 4) red[(wave * REP + o) * kColumns + 4 * sub + (lane >> 4)] = sum;
+    }
+    __syncthreads();
+    const uint32_t o = tid / kColumns, c = tid % kColumns, d = blockIdx.x * kColumns + c;
+    if (o >= nh || d >= p.vdim) return;
+    float sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kColumnWaves; i++) sum += red[(i * REP + o) * kColumns + c];
+    p.out[((int64_t)r * p.heads + h0 + o) * p.vdim + d] = sum;
+}
+
 __global__ __launch_bounds__(kThreads) void attention_sum_kernel(const float *__restrict__ parts, const uint32_t nseg, const uint32_t n, float *__restrict__ out) {
     const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
     if (i >= n) return;
@@ -425,13 +629,26 @@ int rows_kernels(cg_backend *be, const AttentionPlan &p, const float *q, uint32_
     const bool fresh = !q; // a few new tokens, not prepared
     const size_t lds1 = ((size_t)REP * p.dim + REP * kSeg + (fresh ? p.S * p.dim : 0)) * 4;
     const size_t lds2 = (size_t)mix_floats(REP, slots, MVW) * 4;
+    // All keys of 16 columns in a workgroup, up to a lane per segment (8192 keys) and to workgroups for two a compute unit.  One token behind
+    // 100, 1500 and 7700 keys, 16 heads on 8 of 128 values: 11, 13 and 32 us with the scores, by segments 16, 21 and 52; eight tokens, 1500
+    // and 7700 keys: 26 and 156 for 31 and 157.  Beyond that the exponentials' reading, once per 16 columns, is no longer small.
+    const uint32_t chunks = (p.vdim + kColumns - 1) / kColumns;
+    const bool columns = MVW == 4 && !p.mix_scores && nseg <= 64 && (uint64_t)chunks * p.kv_heads * groups * rows <= 512 && column_floats(REP, slots, nseg) * 4 <= kMaxLds;
     if (int rc = fresh ? allow_lds(attention_scores_kernel<REP, SVW, true>, lds1) : allow_lds(attention_scores_kernel<REP, SVW, false>, lds1)) return rc;
-    if (!p.mix_scores)
+    if (!p.mix_scores && !columns)
         if (int rc = allow_lds(attention_mix_kernel<REP, MVW>, lds2)) return rc;
     const dim3 grid(nseg, p.kv_heads * groups, rows);
-    if (fresh) launch_kernel((attention_scores_kernel<REP, SVW, true>), grid, dim3(kThreads), lds1, be->stream, p, q, row0, nseg, scores, stats);
-    else launch_kernel((attention_scores_kernel<REP, SVW, false>), grid, dim3(kThreads), lds1, be->stream, p, q, row0, nseg, scores, stats);
+    if (fresh) launch_kernel((attention_scores_kernel<REP, SVW, true>), grid, dim3(kThreads), lds1, be->stream, p, q, row0, nseg, scores, stats, columns);
+    else launch_kernel((attention_scores_kernel<REP, SVW, false>), grid, dim3(kThreads), lds1, be->stream, p, q, row0, nseg, scores, stats, columns);
     if (p.mix_scores) return launch_mixed_rows(be, p, row0, rows, nseg, scores, parts, reinterpret_cast<float2 *>(parts + (size_t)rows * nseg * p.heads * p.vdim));
+    if constexpr (MVW == 4)
+        if (columns) {
+            const size_t lds = (size_t)column_floats(REP, slots, nseg) * 4;
+            const dim3 wgs(chunks, p.kv_heads * groups, rows);
+            if (int rc = allow_lds(attention_columns_kernel<REP>, lds)) return rc;
+            launch_kernel((attention_columns_kernel<REP>), wgs, dim3(kColumnThreads), lds, be->stream, p, row0, nseg, scores, stats);
+            return launched("block_attention");
+        }
     launch_kernel((attention_mix_kernel<REP, MVW>), grid, dim3(kThreads), lds2, be->stream, p, row0, nseg, scores, stats, nseg > 1 ? parts : p.out, nseg > 1);
     if (nseg > 1) {
         const uint32_t n = p.heads * p.vdim;
