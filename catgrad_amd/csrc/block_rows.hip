@@ -309,6 +309,13 @@ template <bool BF16> __device__ __forceinline__ void load_input(const ProductInp
 __device__ __forceinline__ float blocks_sum(float v) {
     return wave_add_up<4>(v);
 }
+// The same of a group's four columns, kept as [row j][column]: two columns share a register from the first step on, four from the second
+// (8 instructions for 4 x 8, at the end of every group's chain).
+__device__ __forceinline__ void keep_sums(f32x4 *dst, const f32x4 &v) {
+    const uint32_t lane = threadIdx.x & 63;
+    const float sum = four_sums(v[0], v[1], v[2], v[3]);
+    if ((lane & 15) < 4) reinterpret_cast<float *>(dst)[(lane & 3) * 4 + (lane >> 4)] = sum;
+}
 
 // A workgroup holds all of its waves' activations in registers (STEPS of 64 lanes' worth each) and walks column groups.
 // Weights, activations and the norm's gains are all asked for before anything is done with any of them: with the gains asked
@@ -363,10 +370,8 @@ __device__ __forceinline__ void four_rows_linear(const ProductInput &in, const u
 #pragma unroll
         for (int s = 0; s < STEPS; s++) acc = multiply<BF16>(wt[s], x[s], acc);
         if (g + 1 < g1) ask(g + 1);
-#pragma unroll
-        for (int r = 0; r < 4; r++) acc[r] = blocks_sum(acc[r]);
         f32x4(&mine)[WAVES][4] = sums[g & 1];
-        if (lane < 4) mine[wave][lane] = acc;
+        keep_sums(mine[wave], acc);
         __syncthreads(); // (two buffers: the next group's sums do not wait for these to be read)
         if (wave == (g - g0) % WAVES && lane < 16) { // lane (j, r): row j, column r of the group
             const uint32_t m = lane >> 2, c = lane & 3, n = g * 4 + c;
@@ -479,8 +484,9 @@ template <bool BF16, int NB, int NG, int WAVES, bool POLY0, bool POLY1>
 __global__ __launch_bounds__(WAVES * 64) void four_rows_residual_kernel(const Rows x, const ResidualBranch b0, const ResidualBranch b1, const uint32_t rows,
                                                                         const uint32_t width, float *__restrict__ out) {
     __shared__ f32x4 sums[NB][WAVES][NG][4][4]; // [branch][wave][group][term][row]
-    __shared__ float squares[NB][WAVES][3][4];
-    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63, n0 = blockIdx.x * NG * 4;
+    static_assert(WAVES % 4 == 0 && NG <= WAVES, "a quarter of the waves for each of four lanes, a wave per group");
+    __shared__ f32x4 squares[NB][WAVES][4]; // [branch][wave][row][term]
+    const uint32_t wave = threadIdx.x >> 6, n0 = blockIdx.x * NG * 4;
     BranchSums<NG> s[NB];
 #pragma unroll
     for (int b = 0; b < NB; b++) {
@@ -490,13 +496,15 @@ __global__ __launch_bounds__(WAVES * 64) void four_rows_residual_kernel(const Ro
             for (int g = 0; g < NG; g++) s[b].acc[g][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         s[b].m[0] = s[b].m[1] = s[b].m[2] = 0.0f;
     }
-    // thread e of the first 16 * NG: row m, column n; what it needs besides the sums is asked for first
-    const uint32_t e = threadIdx.x, m = e / (4 * NG), c = e % (4 * NG), n = min(n0 + c, width - 1), mr = min(m, rows - 1);
-    float xs = 0.0f, gate[NB] = {};
-    if (e < 16 * NG) {
+    // a wave per group of columns: lane (t, m, c), term t of row m, column n; what it needs besides the sums is asked for first
+    const uint32_t g = threadIdx.x >> 6, t = (threadIdx.x >> 4) & 3, m = (threadIdx.x >> 2) & 3, c = threadIdx.x & 3, n = min(n0 + 4 * g + c, width - 1), mr = min(m, rows - 1);
+    float xs = 0.0f, gate[NB] = {}, term[NB] = {};
+    if (g < NG) {
         xs = x.p[(int64_t)mr * x.pitch + n];
         if (b0.gate.p) gate[0] = b0.gate.p[(int64_t)mr * b0.gate.pitch + n] + (b0.gate_bias ? b0.gate_bias[n] : 0.0f);
         if (NB > 1 && b1.gate.p) gate[NB - 1] = b1.gate.p[(int64_t)mr * b1.gate.pitch + n] + (b1.gate_bias ? b1.gate_bias[n] : 0.0f);
+        if (POLY0) term[0] = b0.in.poly[t];
+        if (NB > 1 && POLY1) term[NB - 1] = b1.in.poly[t];
     }
     BranchLoads<BF16, NG> loads[NB];
     const uint32_t first = __builtin_amdgcn_readfirstlane(wave) * 16 * Frag<BF16>::W;
@@ -523,45 +531,34 @@ __global__ __launch_bounds__(WAVES * 64) void four_rows_residual_kernel(const Ro
         for (int t = 0; t < 4; t++) {
             if (t > 0 && !poly) break;
 #pragma unroll
-            for (int g = 0; g < NG; g++) {
-                f32x4 v;
-#pragma unroll
-                for (int r = 0; r < 4; r++) v[r] = blocks_sum(s[b].acc[g][t][r]);
-                if (lane < 4) sums[b][wave][g][t][lane] = v;
-            }
-            if (t < 3 && poly) {
-                const float q = blocks_sum(s[b].m[t]);
-                if (lane < 4) squares[b][wave][t][lane] = q;
-            }
+            for (int g = 0; g < NG; g++) keep_sums(sums[b][wave][g][t], s[b].acc[g][t]);
         }
+        if (poly) keep_sums(squares[b][wave], f32x4{s[b].m[0], s[b].m[1], s[b].m[2], 0.0f});
     }
     __syncthreads();
-    if (e >= 16 * NG || m >= rows || n0 + c >= width) return;
+    if (g >= NG) return;
 #pragma unroll
     for (int b = 0; b < NB; b++) {
         const ResidualBranch &br = b == 0 ? b0 : b1;
         const bool poly = b == 0 ? POLY0 : POLY1;
-        float y = 0.0f;
+        float v = 0.0f;
+        if (poly) { // a term of the polynomial
+            float q = 0.0f;
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            if (t > 0 && !poly) break;
-            float v = 0.0f, q = 0.0f;
-#pragma unroll
-            for (int i = 0; i < WAVES; i++) v += sums[b][i][c / 4][t][m][c % 4];
-            if (poly) {
-                if (t < 3) {
-#pragma unroll
-                    for (int i = 0; i < WAVES; i++) q += squares[b][i][t][m];
-                    v *= br.in.poly[t] / sqrtf(q / (float)br.in.k + br.in.eps);
-                } else {
-                    v *= br.in.poly[3];
-                }
+            for (int i = 0; i < WAVES; i++) {
+                v += sums[b][i][g][t][m][c];
+                q += squares[b][i][m][t];
             }
-            y += v;
+            v *= t < 3 ? term[b] / sqrtf(q / (float)br.in.k + br.in.eps) : term[b];
+        } else { // a quarter of the waves
+#pragma unroll
+            for (uint32_t i = 0; i < WAVES; i += 4) v += sums[b][i + t][g][0][m][c];
         }
+        const float y = wave_add<16>(v);
         xs += br.gate.p ? sigmoid(gate[b]) * y : y;
     }
-    out[(int64_t)m * width + n0 + c] = xs;
+    if (t > 0 || m >= rows || n0 + 4 * g + c >= width) return;
+    out[(int64_t)m * width + n] = xs;
 }
 
 // ---- many rows -------------------------------------------------------------------------------------------------------
