@@ -194,7 +194,9 @@ template <int VW, int TAPS> __global__ __launch_bounds__(kThreads) void conv_row
 // scales are known, where the kernel above makes six trips to memory one behind the other.  us above and here, with its timing: a token of 1024
 // columns in 4 groups 7.7 and 6.7, 256 of them 10.3 and 8.7, 500 of 2048 columns in 8 groups 21.0 and 17.5, a token of 4096 columns 10.2 and 8.0.
 typedef __attribute__((ext_vector_type(4))) float f32x4;
-__global__ __launch_bounds__(kThreads) void conv_token_kernel(const ConvRowsPlan p, const uint32_t parts) {
+// SUM (one token per sequence): its input is what side_sum_kernel below would have left, worked out here by every workgroup of the token, which
+// needs all of the row's mean square anyway: the launch between the two (2.6 us, and 1.5 from its end to the next one's first load) falls away.
+template <bool SUM> __global__ __launch_bounds__(kThreads) void conv_token_kernel(const ConvRowsPlan p, const uint32_t parts, const SideSum sum) {
     constexpr int TAPS = 4, PAST = TAPS - 1;
     static_assert(kWaves == TAPS, "a wave per row that a token looks at");
     __shared__ float scale[TAPS];
@@ -216,30 +218,74 @@ __global__ __launch_bounds__(kThreads) void conv_token_kernel(const ConvRowsPlan
             for (int j = 0; j < 4; j++) w[f][j] = load(taps[f] + (int64_t)(at + j) * TAPS);
         }
 #pragma unroll
-        for (int t = 0; t < TAPS; t++) {
+        for (int t = SUM; t < TAPS; t++) {
             const int32_t from = (int32_t)s - t;
             const bool fresh = from >= 0 || !has_state;
             const int64_t row = fresh ? (int64_t)b * p.S + max(from, 0) : (int64_t)b * PAST + (PAST + from);
             z[t] = load((fresh ? inputs : state) + row * (fresh ? p.x.pitch : (int64_t)p.width) + at);
         }
     };
-    ask(c_first);
+    struct Added { // four columns of the sum
+        f32x4 x, y, w;
+    };
+    auto ask_sum = [&](uint32_t c) {
+        const uint32_t at = min(c, p.width - 4);
+        auto get = [&](const float *q) { return *reinterpret_cast<const f32x4 *>(q + at); };
+        return Added{get(sum.x.p + (int64_t)b * sum.x.pitch), get(sum.y + (int64_t)b * p.width), get(sum.norm)};
+    };
+    float rms = 0.0f; // (of the sum's second term, times its factor)
+    auto added = [&](const Added &a) {
+        f32x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = fmaf(a.y[j] * rms, a.w[j], a.x[j]);
+        return v;
+    };
     float m = 0.0f;
+    Added own, group_first;
+    if constexpr (SUM) {
+        const f32x4 first = *reinterpret_cast<const f32x4 *>(sum.y + (int64_t)b * p.width + min(threadIdx.x * 4, p.width - 4));
+        group_first = ask_sum(g0 + lane * 4);
+        own = ask_sum(c_first);
+        ask(c_first);
+        for (uint32_t k = threadIdx.x * 4; k < p.width; k += kThreads * 4) { // (in side_sum_kernel's order)
+            const f32x4 v = k == threadIdx.x * 4 ? first : *reinterpret_cast<const f32x4 *>(sum.y + (int64_t)b * p.width + k);
+#pragma unroll
+            for (int j = 0; j < 4; j++) m = fmaf(v[j], v[j], m);
+        }
+        m = wave_total(m);
+        if (lane == 0) scale[wave] = m;
+        __syncthreads();
+        rms = sum.scale / sqrtf(((scale[0] + scale[1]) + (scale[2] + scale[3])) / (float)p.width + sum.eps);
+        m = 0.0f;
+    } else {
+        ask(c_first);
+    }
     const int32_t mine = (int32_t)s - PAST + (int32_t)wave; // (the token whose scale this wave takes)
     for (uint32_t k = lane * 4; k < size; k += 64 * 4) {
-        const f32x4 v = load(inputs + ((int64_t)b * p.S + max(mine, 0)) * p.x.pitch + g0 + k);
+        f32x4 v;
+        if constexpr (SUM) v = added(k == lane * 4 ? group_first : ask_sum(g0 + k));
+        else v = load(inputs + ((int64_t)b * p.S + max(mine, 0)) * p.x.pitch + g0 + k);
 #pragma unroll
         for (int j = 0; j < 4; j++) m = fmaf(v[j], v[j], m);
     }
-    const float sum = wave_total(m);
-    if (lane == 0) scale[wave] = 1.0f / sqrtf(sum / (float)size + p.eps);
-    __syncthreads();
+    const float unit = 1.0f / sqrtf(wave_total(m) / (float)size + p.eps);
+    if constexpr (!SUM) {
+        if (lane == 0) scale[wave] = unit;
+        __syncthreads();
+    }
     for (uint32_t c = c_first; c < c_end; c += kThreads * 4) {
-        if (c != c_first) ask(c);
+        if (c != c_first) {
+            ask(c);
+            if (SUM) own = ask_sum(c);
+        }
+        if constexpr (SUM) {
+            z[0] = added(own);
+            *reinterpret_cast<f32x4 *>(sum.out + (int64_t)b * p.width + c) = z[0];
+        }
 #pragma unroll
         for (int t = 0; t < TAPS; t++) {
             const bool fresh = (int32_t)s - t >= 0;
-            const float f = fresh ? scale[PAST - t] : 1.0f;
+            const float f = !fresh ? 1.0f : SUM ? unit : scale[PAST - t];
 #pragma unroll
             for (int j = 0; j < 4; j++) z[t][j] = fresh ? z[t][j] * f : has_state ? z[t][j] : 0.0f;
         }
@@ -415,7 +461,7 @@ int launch_pair_embedding(cg_backend *be, const PairEmbeddingPlan &p) {
     return launched("pair_embedding");
 }
 
-int launch_conv_rows(cg_backend *be, ConvRowsPlan p) {
+int launch_conv_rows(cg_backend *be, ConvRowsPlan p, const SideSum *sum) {
     const uint32_t cols = p.width / p.groups, past = p.taps - 1;
     // short runs while the device is not full, and a group's columns over several workgroups
     p.run = 1;
@@ -430,6 +476,8 @@ int launch_conv_rows(cg_backend *be, ConvRowsPlan p) {
         bytes += p.out[f].fmt == kFmtBF16 ? 2.0 : 4.0;
         vec = vec && aligned16(p.out[f].dst) && aligned16(p.out[f].gamma) && aligned16(p.out[f].conv);
     }
+    const bool token = p.taps > 3 && p.taps <= 4 && vec && p.run == 1 && taps;
+    if (sum && !(token && p.S == 1 && sum->x.pitch % 4 == 0 && aligned16(sum->x.p) && aligned16(sum->y) && aligned16(sum->norm) && aligned16(sum->out))) return kDeclined;
     ProfScope prof(be, CG_K_REDUCE, bytes * p.B * p.S * p.width);
     const uint32_t runs = (p.S + p.run - 1) / p.run;
     const dim3 grid(p.B * runs, p.groups * split);
@@ -441,8 +489,8 @@ int launch_conv_rows(cg_backend *be, ConvRowsPlan p) {
     if (p.taps <= 1) { CG_CONV(1); }
     else if (p.taps <= 2) { CG_CONV(2); }
     else if (p.taps <= 3) { CG_CONV(3); }
-    else if (p.taps == 4 && vec && p.run == 1 && taps)
-        launch_kernel(conv_token_kernel, grid, dim3(kThreads), 0, s, p, split);
+    else if (token && sum) launch_kernel(conv_token_kernel<true>, grid, dim3(kThreads), 0, s, p, split, *sum);
+    else if (token) launch_kernel(conv_token_kernel<false>, grid, dim3(kThreads), 0, s, p, split, SideSum{});
     else if (p.taps <= 4) { CG_CONV(4); }
     else if (p.taps <= 8) { CG_CONV(8); }
     else if (p.taps <= kMaxTaps) { CG_CONV(kMaxTaps); }
@@ -501,7 +549,10 @@ int launch_side_second(cg_backend *be, const Rows &x, const float *g, uint32_t r
 #undef CG_SIDE
 }
 
-int launch_side_sum(cg_backend *be, const Rows &x, const float *y, const float *norm, uint32_t rows, uint32_t width, float eps, float scale, float *out) {
+int launch_side_sum(cg_backend *be, const SideSum &a, uint32_t rows, uint32_t width) {
+    const Rows &x = a.x;
+    const float *const y = a.y, *const norm = a.norm, eps = a.eps, scale = a.scale;
+    float *const out = a.out;
     ProfScope prof(be, CG_K_REDUCE, 12.0 * rows * width);
     const bool vec = width % 4 == 0 && x.pitch % 4 == 0 && aligned16(x.p) && aligned16(y) && aligned16(norm) && aligned16(out);
     if (vec) launch_kernel((side_sum_kernel<4>), dim3(rows), dim3(kThreads), 0, be->stream, x, y, norm, width, eps, scale, out);

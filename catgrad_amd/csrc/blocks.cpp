@@ -386,11 +386,25 @@ int cache_tail(cg_backend *be, const cg_tensor *all, int64_t keep, cg_tensor **o
 
 static int64_t numel_of(const DeferredStep &s) { return (int64_t)s.plan.B * s.plan.S * s.plan.heads * s.plan.vdim; } // of its result
 
-void flush_step(cg_backend *be) {
-    DeferredStep *const s = be->step;
-    be->step = nullptr;
-    if (hipSetDevice(be->device) != hipSuccess || run_step(be, *s) != CG_OK) be->stream.fail(hipErrorLaunchFailure);
-    drop_step(be, s);
+static void drop_sum(cg_backend *be) {
+    DeferredSum *const s = be->sum;
+    be->sum = nullptr;
+    if (s->mem) be->pool.free(s->mem, s->cls); // stream-ordered
+    for (cg_tensor *t : s->held) release(t);
+    delete s;
+}
+
+void flush_waiting(cg_backend *be) {
+    const bool set = hipSetDevice(be->device) == hipSuccess;
+    if (DeferredStep *const s = be->step) {
+        be->step = nullptr;
+        if (!set || run_step(be, *s) != CG_OK) be->stream.fail(hipErrorLaunchFailure);
+        drop_step(be, s);
+    }
+    if (be->sum) {
+        if (!set || launch_side_sum(be, be->sum->sum, be->sum->rows, be->sum->width) != CG_OK) be->stream.fail(hipErrorLaunchFailure);
+        drop_sum(be);
+    }
 }
 
 } // namespace cg
@@ -522,7 +536,14 @@ int cg_block_pair_embedding(cg_backend *b, const cg_pair_embedding_args *a, cg_t
 }
 
 int cg_block_conv_linear(cg_backend *b, const cg_conv_linear_args *a, cg_tensor **y, cg_tensor **kept, cg_tensor **state_out) {
-    Enter entered(b);
+    Enter entered(b, true);
+    if (b && (b->step || b->sum)) { // a sum that waits goes along if its rows are what is filtered, and all else is in memory and none of them
+        auto apart = [&](const cg_tensor *t) { return !t || (!t->pend && t->buf != b->sum->out); };
+        bool fits = b->sum && a && a->x && !a->x->pend && a->x->buf == b->sum->out && is_contiguous(a->x) && !a->x->offset &&
+                    numel(a->x) == (int64_t)b->sum->rows * b->sum->width && apart(a->state);
+        for (size_t i = 0; fits && i < a->n && i < 2; i++) fits = apart(a->in[i].gamma) && apart(a->in[i].conv) && apart(a->in[i].w);
+        if (!fits) flush_waiting(b);
+    }
     if (!a) return fail(CG_ERR_ARG, "null argument");
     Held h;
     bool whole = a->x && a->state && y && kept && state_out;
@@ -585,7 +606,13 @@ int cg_block_conv_linear(cg_backend *b, const cg_conv_linear_args *a, cg_tensor 
     rc = new_dense(b, CG_F32, sd, 3, &so);
     if (!rc) {
         p.state_out = so->buf ? static_cast<float *>(so->buf->ptr) : nullptr;
-        rc = launch_conv_rows(b, p);
+        rc = kDeclined;
+        if (b->sum) {
+            if (p.width == b->sum->width) rc = launch_conv_rows(b, p, &b->sum->sum);
+            if (rc == kDeclined) flush_waiting(b);
+            else drop_sum(b);
+        }
+        if (rc == kDeclined) rc = launch_conv_rows(b, p);
     }
     ProductInput pi[2];
     for (size_t i = 0; i < a->n && !rc; i++) {
@@ -671,7 +698,18 @@ int cg_block_token_side(cg_backend *b, const cg_token_side_args *a, cg_tensor **
         second = launch_side_second(b, x, static_cast<const float *>(g), (uint32_t)rows, proj, norm, a->eps, a->scale, static_cast<float *>(o->buf->ptr));
     if (second != kDeclined) rc = second;
     if (!rc && second == kDeclined) rc = product({static_cast<const float *>(g), dim}, proj, pv, y);
-    if (!rc && second == kDeclined) rc = launch_side_sum(b, x, static_cast<const float *>(y), norm, (uint32_t)rows, (uint32_t)W, a->eps, a->scale, static_cast<float *>(o->buf->ptr));
+    if (!rc && second == kDeclined) {
+        const SideSum sum = {x, static_cast<const float *>(y), norm, static_cast<float *>(o->buf->ptr), a->eps, a->scale};
+        if (few && a->x->rank == 3 && a->x->dims[1] == 1 && !b->prof[CG_K_REDUCE].every) { // one token per sequence
+            b->sum = new DeferredSum{sum, (uint32_t)rows, (uint32_t)W, tmp.mem.back().first, tmp.mem.back().second, {}, o->buf};
+            tmp.mem.pop_back();
+            b->sum->held.swap(h.t);
+            retain(o);
+            b->sum->held.push_back(o);
+        } else {
+            rc = launch_side_sum(b, sum, (uint32_t)rows, (uint32_t)W);
+        }
+    }
     if (rc) {
         release(o);
         return rc;
@@ -682,6 +720,7 @@ int cg_block_token_side(cg_backend *b, const cg_token_side_args *a, cg_tensor **
 
 int cg_block_residual(cg_backend *b, cg_tensor *x, const cg_branch *br, size_t n, float eps, float scale, const cg_experts *experts, cg_tensor **out) {
     Enter entered(b, true);
+    if (b && b->sum) flush_waiting(b);
     // Attention that waits may share the experts' launch, if it is what the only branch reads and all else is in memory and none of its own
     if (b && b->step) {
         const DeferredStep &s = *b->step;
@@ -690,7 +729,7 @@ int cg_block_residual(cg_backend *b, cg_tensor *x, const cg_branch *br, size_t n
         for (const cg_tensor *t : {fits ? experts->h : nullptr, fits ? experts->logits : nullptr, fits ? experts->correction : nullptr, fits ? experts->gate_up : nullptr,
                                    fits ? experts->down : nullptr})
             fits = fits && apart(t);
-        if (!fits || !is_contiguous(br->y) || br->y->offset || numel(br->y) != numel_of(s)) flush_step(b);
+        if (!fits || !is_contiguous(br->y) || br->y->offset || numel(br->y) != numel_of(s)) flush_waiting(b);
     }
     Held h;
     h.add(x);
@@ -731,7 +770,7 @@ int cg_block_residual(cg_backend *b, cg_tensor *x, const cg_branch *br, size_t n
     if (rows > 0 && width > 0) {
         float *y = static_cast<float *>(o->buf->ptr);
         const bool plain = n == 1 && !r[0].in.poly && !r[0].gate.p && r[0].w.fmt == ep.fmt;
-        if (b->step && !(experts && rows <= kFewRows && plain)) flush_step(b);
+        if (b->step && !(experts && rows <= kFewRows && plain)) flush_waiting(b);
         if (experts && rows <= kFewRows && (n == 0 || plain)) {
             Scratch tmp(b);
             void *hidden = nullptr, *chosen = nullptr;
@@ -743,7 +782,7 @@ int cg_block_residual(cg_backend *b, cg_tensor *x, const cg_branch *br, size_t n
                     drop_step(b, b->step);
                     b->step = nullptr;
                 }
-                if (b->step) flush_step(b);
+                if (b->step) flush_waiting(b);
                 rc = both != kDeclined ? both : launch_experts_first(b, ep, static_cast<float *>(hidden), static_cast<uint32_t *>(chosen));
             }
             if (!rc)

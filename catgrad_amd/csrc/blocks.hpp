@@ -109,13 +109,31 @@ struct ConvRowsPlan {
         bool round; // words: rounded to bfloat16
     } out[2];
 };
-int launch_conv_rows(cg_backend *be, ConvRowsPlan p);
+// out = x + scale * y / sqrt(mean(y^2) + eps) * norm, by rows
+struct SideSum {
+    Rows x;
+    const float *y, *norm;
+    float *out;
+    float eps, scale;
+};
+// sum: what leaves the rows that are filtered, worked out on the way (kDeclined: sizes that do not go along)
+int launch_conv_rows(cg_backend *be, ConvRowsPlan p, const SideSum *sum = nullptr);
 
 int launch_side_gate(cg_backend *be, float *g, const Tokens &ids, const Table &table, uint32_t vocab, uint32_t first, uint32_t dim, uint32_t rows);
 // A few rows: g[r] = gelu(x[r] . w^T) * the rows' vectors; then out = x + scale * norm(g . w^T) (kDeclined: sizes it does not take).
 int launch_side_first(cg_backend *be, const Rows &x, uint32_t rows, const Weight &w, const Tokens &ids, const Table &table, uint32_t vocab, uint32_t first, float *g);
 int launch_side_second(cg_backend *be, const Rows &x, const float *g, uint32_t rows, const Weight &w, const float *norm, float eps, float scale, float *out);
-int launch_side_sum(cg_backend *be, const Rows &x, const float *y, const float *norm, uint32_t rows, uint32_t width, float eps, float scale, float *out);
+int launch_side_sum(cg_backend *be, const SideSum &a, uint32_t rows, uint32_t width);
+// The sum of one token per sequence, whose launch waits for the next call on its backend: the filters over what it leaves, which come
+// next in front of another layer, take it along.  Any other call launches it first (Enter).
+struct DeferredSum {
+    SideSum sum{};
+    uint32_t rows = 0, width = 0;
+    void *mem = nullptr; // its second term (pool memory)
+    size_t cls = 0;
+    std::vector<cg_tensor *> held; // operands and result (retained)
+    const Buffer *out = nullptr;
+};
 
 // ---- mixtures of experts ---------------------------------------------------------------------------------------------
 struct ExpertsPlan {

@@ -112,6 +112,7 @@ template <class T> struct Pooled {
 struct LazyMm;
 struct DeferredWrite;
 struct DeferredStep;
+struct DeferredSum;
 struct Buffer;
 }
 
@@ -152,6 +153,7 @@ struct cg_backend {
     std::vector<cg::LazyMm *> lazy_open; // groupable lazy products not yet computed (not retained)
     std::vector<cg::DeferredWrite> deferred; // writes waiting to share a launch (see flush_deferred)
     cg::DeferredStep *step = nullptr;        // attention waiting for the next call, which may share its launch (blocks.hpp)
+    cg::DeferredSum *sum = nullptr;          // the same of a sum of rows; never both
     // Results that depend on constants only (the rotary tables every forward pass rebuilds from iota and
     // scalars) are kept, keyed by the program and its leaves, and handed out again instead of recomputed.
     // Buffers are retained here; the oldest entries go when the limits are reached.
@@ -322,13 +324,13 @@ struct Consume { // the consumed reference of a tensor argument (move semantics 
 // Every entry point that touches a backend's state holds the backend's lock for its whole duration
 // (declared first, so the tensor arguments it consumes are released under the lock too): handles may be
 // cloned, moved between threads and used from several threads; calls on one backend then run one at a time.
-void flush_step(cg_backend *be); // launches be->step; an error is the next waiting call's
+void flush_waiting(cg_backend *be); // launches be->step or be->sum; an error is the next waiting call's
 struct Enter {
-    // keep_step: the call launches nothing, or looks after be->step itself
-    explicit Enter(cg_backend *b, bool keep_step = false) : b_(b) {
+    // keep: the call launches nothing, or looks after be->step and be->sum itself
+    explicit Enter(cg_backend *b, bool keep = false) : b_(b) {
         if (!b_) return;
         b_->mu.lock();
-        if (b_->step && !keep_step) flush_step(b_);
+        if ((b_->step || b_->sum) && !keep) flush_waiting(b_);
     }
     ~Enter() {
         if (b_) b_->mu.unlock();
