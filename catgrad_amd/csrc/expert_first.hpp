@@ -41,6 +41,7 @@ __device__ void choose_experts(const ExpertsPlan &p, uint32_t row, float *lds, u
             const uint32_t g = e / size, first = g * size;
             const float mine = choice[e];
             uint32_t rank = 0;
+#pragma unroll 8
             for (uint32_t j = first; j < first + size; j++) rank += beats(choice[j], j, mine, e);
             if (rank < 2) worth[2 * g + rank] = mine;
         }
@@ -48,6 +49,7 @@ __device__ void choose_experts(const ExpertsPlan &p, uint32_t row, float *lds, u
         for (uint32_t g = t; g < p.groups; g += N) {
             const float mine = worth[2 * g] + worth[2 * g + 1];
             uint32_t rank = 0;
+#pragma unroll 4
             for (uint32_t j = 0; j < p.groups; j++) rank += beats(worth[2 * j] + worth[2 * j + 1], j, mine, g);
             counts[g] = rank < p.keep ? 1.0f : 0.0f;
         }
@@ -59,7 +61,7 @@ __device__ void choose_experts(const ExpertsPlan &p, uint32_t row, float *lds, u
     for (uint32_t e = t; e < p.experts; e += N) {
         const float mine = choice[e];
         uint32_t rank = 0;
-#pragma unroll 4
+#pragma unroll 16
         for (uint32_t j = 0; j < p.experts; j++) rank += beats(choice[j], j, mine, e);
         if (rank < p.top) {
             chosen[rank] = e;
@@ -70,6 +72,9 @@ __device__ void choose_experts(const ExpertsPlan &p, uint32_t row, float *lds, u
 }
 
 // A workgroup of kExpertThreads: four waves' columns (block x, per_wave each, one after the other) of row * top + choice (block y).
+// In front of the first weight lie the choice and its loads, 4 us: so the columns are cut for one round of workgroups, and a wave's next
+// column is on its way while this one is multiplied.  The launch beside attention, 8 of 32 experts in bf16: 1024 columns of 2048 values
+// 23.4 -> 20.5 us (67 MB, 13 us at the device's rate), 384 of 1024 12.4 -> 11.8.
 // LDS: route_bytes(p).
 constexpr int kExpertThreads = 256, kExpertWaves = 4;
 inline size_t route_bytes(const ExpertsPlan &p) { return (route_floats(p.experts, p.groups) + 2 * (size_t)p.top) * 4; }
@@ -97,41 +102,79 @@ __device__ __forceinline__ void expert_first(const ExpertsPlan &p, const uint32_
 #pragma unroll
     for (int s = 0; s < STEPS; s++) take(s * SPAN + lane * W, x[s]);
     choose_experts<kExpertThreads>(p, row, lds, chosen, weight, threadIdx.x);
-    const uint32_t e = chosen[slot];
+    const uint32_t e = __builtin_amdgcn_readfirstlane(chosen[slot]);
     const float weigh = weight[slot];
     if (bx == 0 && threadIdx.x == 0) chosen_out[by] = e;
-    const uint32_t f0 = (bx * kExpertWaves + wave) * per_wave;
+    const uint32_t f0 = (bx * kExpertWaves + __builtin_amdgcn_readfirstlane(wave)) * per_wave, f1 = min(f0 + per_wave, p.ff);
+    if (f0 >= f1) return;
     constexpr uint32_t EB = BF16 ? 2 : 4;
-    for (uint32_t f = f0; f < min(f0 + per_wave, p.ff); f++) {
-        const char *g = static_cast<const char *>(p.gate_up) + ((uint64_t)e * 2 * p.ff + f) * p.width * EB, *u = g + (uint64_t)p.ff * p.width * EB;
-        float a = 0.0f, b = 0.0f;
-        if (p.width <= STEPS * SPAN) {
-            St wg[STEPS], wu[STEPS];
-#pragma unroll
-            for (int s = 0; s < STEPS; s++) { // (clamped: behind the last column x is zero)
-                const uint32_t k = min(s * SPAN + lane * W, p.width - W);
-                wg[s].load(g, k);
-                wu[s].load(u, k);
-            }
-#pragma unroll
-            for (int s = 0; s < STEPS; s++) {
-                a = wg[s].dot(x[s], a);
-                b = wu[s].dot(x[s], b);
-            }
-        } else {
+    auto column = [&](uint32_t f) { return static_cast<const char *>(p.gate_up) + ((uint64_t)e * 2 * p.ff + f) * p.width * EB; };
+    const uint64_t up = (uint64_t)p.ff * p.width * EB;
+    auto put = [&](uint32_t f, float a, float b) {
+        a = wave_total(a);
+        b = wave_total(b);
+        if (lane == 0) hidden[(uint64_t)by * p.ff + f] = weigh * activation(a, b, p.limit, p.slope);
+    };
+    if (p.width > STEPS * SPAN) {
+        for (uint32_t f = f0; f < f1; f++) {
+            const char *g = column(f);
+            float a = 0.0f, b = 0.0f;
             for (uint32_t k = lane * W; k < p.width; k += SPAN) {
                 St wg, wu;
                 wg.load(g, k);
-                wu.load(u, k);
+                wu.load(g + up, k);
                 float v[W];
                 take(k, v);
                 a = wg.dot(v, a);
                 b = wu.dot(v, b);
             }
+            put(f, a, b);
         }
-        a = wave_total(a);
-        b = wave_total(b);
-        if (lane == 0) hidden[(uint64_t)by * p.ff + f] = weigh * activation(a, b, p.limit, p.slope);
+        return;
+    }
+    // the next column, or the second half of eight steps, is asked for before this one is multiplied
+    constexpr int PART = STEPS < 4 ? STEPS : 4;
+    struct Piece {
+        St g[PART], u[PART];
+    };
+    auto ask = [&](uint32_t f, int first, Piece &c) {
+        const char *g = column(f);
+#pragma unroll
+        for (int s = 0; s < PART; s++) { // (clamped: behind the last column x is zero)
+            const uint32_t k = min((first + s) * SPAN + lane * W, p.width - W);
+            c.g[s].load(g, k);
+            c.u[s].load(g + up, k);
+        }
+    };
+    auto use = [&](const int first, const Piece &c, float &a, float &b) {
+#pragma unroll
+        for (int s = 0; s < PART; s++) {
+            a = c.g[s].dot(x[first + s], a);
+            b = c.u[s].dot(x[first + s], b);
+        }
+    };
+    Piece c0, c1;
+    ask(f0, 0, c0);
+    if constexpr (STEPS > PART) {
+        for (uint32_t f = f0; f < f1; f++) {
+            float a = 0.0f, b = 0.0f;
+            ask(f, PART, c1);
+            use(0, c0, a, b);
+            if (f + 1 < f1) ask(f + 1, 0, c0);
+            use(PART, c1, a, b);
+            put(f, a, b);
+        }
+    } else {
+        for (uint32_t f = f0; f < f1; f += 2) {
+            float a = 0.0f, b = 0.0f, c = 0.0f, d = 0.0f;
+            if (f + 1 < f1) ask(f + 1, 0, c1);
+            use(0, c0, a, b);
+            put(f, a, b);
+            if (f + 1 >= f1) break;
+            if (f + 2 < f1) ask(f + 2, 0, c0);
+            use(0, c1, c, d);
+            put(f + 1, c, d);
+        }
     }
 }
 
