@@ -414,7 +414,8 @@ template <int NG> struct BranchSums {
 };
 // Four steps of a branch (AHEAD * WAVES * 64 or 128 values of k) in registers: both branches' first ones are asked for before any is
 // multiplied.  2048 columns of 2048 + 8192 values of k, f32: 23.9 us with one branch behind the other, 21.1 so; bf16 14.7 and 14.1;
-// 1024 columns of 2048 + 3072: 10.2 and 10.1 (eight steps at a time: 10.4).
+// 1024 columns of 2048 + 3072: 10.2 and 10.1 (eight steps at a time: 10.4); 9.3 in a model's steps, 8.1 since the sums over lanes share
+// registers (keep_sums) and every term of the polynomial has a lane of its own in the end.
 template <bool BF16, int NG> struct BranchLoads {
     static constexpr int AHEAD = 4;
     Frag<BF16> wt[AHEAD][NG];
