@@ -395,16 +395,20 @@ static void drop_sum(cg_backend *be) {
 }
 
 void flush_waiting(cg_backend *be) {
-    const bool set = hipSetDevice(be->device) == hipSuccess;
+    int rc = CG_OK;
+    if (const hipError_t e = hipSetDevice(be->device)) rc = hip_fail(e, "hipSetDevice");
     if (DeferredStep *const s = be->step) {
         be->step = nullptr;
-        if (!set || run_step(be, *s) != CG_OK) be->stream.fail(hipErrorLaunchFailure);
+        if (!rc) rc = run_step(be, *s);
         drop_step(be, s);
     }
     if (be->sum) {
-        if (!set || launch_side_sum(be, be->sum->sum, be->sum->rows, be->sum->width) != CG_OK) be->stream.fail(hipErrorLaunchFailure);
+        if (!rc) rc = launch_side_sum(be, be->sum->sum, be->sum->rows, be->sum->width);
         drop_sum(be);
     }
+    if (!rc || be->late_rc) return;
+    be->late_rc = rc;
+    be->late_error = cg_last_error();
 }
 
 } // namespace cg

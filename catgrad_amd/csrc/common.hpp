@@ -154,6 +154,8 @@ struct cg_backend {
     std::vector<cg::DeferredWrite> deferred; // writes waiting to share a launch (see flush_deferred)
     cg::DeferredStep *step = nullptr;        // attention waiting for the next call, which may share its launch (blocks.hpp)
     cg::DeferredSum *sum = nullptr;          // the same of a sum of rows; never both
+    int late_rc = 0;                         // what launching one of them has come to, for the next call that waits (the first error is kept)
+    std::string late_error;
     // Results that depend on constants only (the rotary tables every forward pass rebuilds from iota and
     // scalars) are kept, keyed by the program and its leaves, and handed out again instead of recomputed.
     // Buffers are retained here; the oldest entries go when the limits are reached.

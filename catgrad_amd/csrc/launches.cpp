@@ -41,8 +41,7 @@ void LaunchQueue::wake() {
         thread_ = std::thread([this] { work(); });
     } catch (const std::system_error &) { // no thread to be had: what was handed over is passed on here, and so is what follows
         while (done_.load() != head_.load()) {
-            Slot &s = slots_[done_.load() % kSlots];
-            if (const hipError_t e = s.run(s.job, stream_)) failed_.store(e);
+            pass_on(slots_[done_.load() % kSlots]);
             done_.fetch_add(1);
         }
         awake_.store(false);
@@ -57,8 +56,7 @@ void LaunchQueue::work() {
     auto idle = std::chrono::steady_clock::now();
     for (uint32_t spins = 1;; spins++) {
         if (head_.load(std::memory_order_acquire) != n) {
-            Slot &s = slots_[n % kSlots];
-            if (const hipError_t e = s.run(s.job, stream_)) failed_.store(e);
+            pass_on(slots_[n % kSlots]);
             done_.store(++n, std::memory_order_release);
             spins = 0;
             continue;

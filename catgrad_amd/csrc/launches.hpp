@@ -41,9 +41,15 @@ class LaunchQueue {
     }
     // The host has waited for the device: the launches up to the next time are counted anew.
     void waited() { direct_ = 0; }
-    // What a launch that was handed over has come to, once (hipSuccess: no error since the last call).
-    void fail(hipError_t e) { failed_.store((int)e); }
-    hipError_t error() { return failed_.load(std::memory_order_relaxed) ? (hipError_t)failed_.exchange(0) : hipSuccess; }
+    // What the first launch that was handed over and failed since the last call has come to, and its kernel (hipSuccess: none).  Known when
+    // what was launched behind it is known to have run.
+    hipError_t error(const void **kernel) {
+        const hipError_t e = failed_.load(std::memory_order_acquire);
+        if (e == hipSuccess) return e;
+        *kernel = failed_kernel_;
+        failed_.store(hipSuccess, std::memory_order_release);
+        return e;
+    }
 
     // One caller at a time (the backend's lock); the arguments are copied.
     template <class... P, class... A> void launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, A &&...a) {
@@ -56,13 +62,15 @@ class LaunchQueue {
                 Slot &s = slots_[n % kSlots];
                 new (s.job) J{kernel, grid, block, lds, std::tuple<std::decay_t<P>...>(std::forward<A>(a)...)};
                 s.run = &J::run;
+                s.kernel = reinterpret_cast<const void *>(kernel);
                 head_.store(n + 1);          // (either this thread sees the other one asleep, or that one the launch)
                 if (!awake_.load()) wake();
                 return;
             }
         }
         drain();
-        kernel<<<grid, block, lds, stream_>>>(std::forward<A>(a)...);
+        J j{kernel, grid, block, lds, std::tuple<std::decay_t<P>...>(std::forward<A>(a)...)};
+        (void)J::run(&j, stream_); // (an error is the caller's hipGetLastError)
     }
 
   private:
@@ -71,6 +79,7 @@ class LaunchQueue {
     static constexpr int kDirect = 12;
     struct Slot {
         hipError_t (*run)(void *job, hipStream_t);
+        const void *kernel;
         alignas(16) unsigned char job[4096 + 128]; // (the arguments of a kernel are at most 4096 bytes)
     };
     template <class... P> struct Job {
@@ -79,7 +88,7 @@ class LaunchQueue {
         size_t lds;
         std::tuple<std::decay_t<P>...> args;
         static hipError_t run(void *p, hipStream_t stream) {
-            J_t &j = *static_cast<J_t *>(p);
+            Job &j = *static_cast<Job *>(p);
             return std::apply(
                 [&](auto &...a) {
                     void *at[sizeof...(P) + 1] = {&a...};
@@ -87,7 +96,6 @@ class LaunchQueue {
                 },
                 j.args);
         }
-        typedef Job J_t;
     };
     bool hands_over() {
         if (!slots_) return false;
@@ -96,6 +104,12 @@ class LaunchQueue {
     }
     void wake();
     void work();
+    void pass_on(Slot &s) {
+        const hipError_t e = s.run(s.job, stream_);
+        if (e == hipSuccess || failed_.load(std::memory_order_acquire) != hipSuccess) return; // (the first one is kept)
+        failed_kernel_ = s.kernel;
+        failed_.store(e, std::memory_order_release);
+    }
 
     int device_ = 0;
     hipStream_t stream_ = nullptr;
@@ -104,7 +118,8 @@ class LaunchQueue {
     alignas(64) std::atomic<uint64_t> head_{0}; // launches handed over
     alignas(64) std::atomic<uint64_t> done_{0}; // launches passed on
     std::atomic<bool> awake_{false};
-    std::atomic<int> failed_{0};
+    std::atomic<hipError_t> failed_{hipSuccess};
+    const void *failed_kernel_ = nullptr; // (written in front of failed_)
     bool stop_ = false;              // (under mu_)
     std::mutex mu_;
     std::condition_variable cv_;

@@ -755,18 +755,32 @@ static bool same_shape(const cg_tensor *a, const cg_tensor *b) {
     return true;
 }
 
+// What went wrong in front of a wait and has not been reported: launches made behind the call that asked for them, then what the kernels
+// found.  All of it is cleared, so that none of it becomes a later call's; the first error is what is said.
+static int reported(cg_backend *be) {
+    volatile uint32_t *const word = be->fault_host;
+    const uint32_t f = *word;
+    if (f) *word = 0;
+    const void *kernel = nullptr;
+    const hipError_t e = be->stream.error(&kernel);
+    if (const int rc = be->late_rc) {
+        be->late_rc = 0;
+        return fail(rc, "%s", be->late_error.c_str());
+    }
+    if (e != hipSuccess) {
+        const char *name = hipKernelNameRefByPtr(kernel, nullptr);
+        return fail(CG_ERR_DEVICE, "HIP error %d (%s) in the launch of %s", (int)e, hipGetErrorString(e), name ? name : "a kernel");
+    }
+    if (f & kFaultIndexRange) return fail(CG_ERR_RANGE, "index: index out of bounds (detected on device)");
+    if (f & kFaultDivZero) return fail(CG_ERR_RANGE, "attempt to divide by zero (detected on device)");
+    return CG_OK;
+}
+
 static int wait_and_check(cg_backend *be) {
     CG_HIP(hipStreamSynchronize(be->stream));
     be->stream.waited();
-    CG_HIP(be->stream.error());
     if (!be->prof_pending.empty()) prof_drain(be);
-    uint32_t f = *reinterpret_cast<volatile uint32_t *>(be->fault_host);
-    if (f) {
-        *reinterpret_cast<volatile uint32_t *>(be->fault_host) = 0;
-        if (f & kFaultIndexRange) return fail(CG_ERR_RANGE, "index: index out of bounds (detected on device)");
-        if (f & kFaultDivZero) return fail(CG_ERR_RANGE, "attempt to divide by zero (detected on device)");
-    }
-    return CG_OK;
+    return reported(be);
 }
 
 // The read-back kernel with sequence number `seq` has run (and with it everything before it on the stream): polls the words
@@ -784,14 +798,7 @@ static int wait_for_readback(cg_backend *be, uint32_t seq, uint32_t groups) {
     }
     std::atomic_thread_fence(std::memory_order_acquire);
     be->stream.waited();
-    CG_HIP(be->stream.error());
-    uint32_t f = *reinterpret_cast<volatile uint32_t *>(be->fault_host);
-    if (f) {
-        *reinterpret_cast<volatile uint32_t *>(be->fault_host) = 0;
-        if (f & kFaultIndexRange) return fail(CG_ERR_RANGE, "index: index out of bounds (detected on device)");
-        if (f & kFaultDivZero) return fail(CG_ERR_RANGE, "attempt to divide by zero (detected on device)");
-    }
-    return CG_OK;
+    return reported(be);
 }
 
 // fresh: dst is the whole of a buffer allocated for this very result (nothing else lives in it).
