@@ -831,11 +831,13 @@ int launch_mixed_tiles(cg_backend *be, const AttentionPlan &p, const float *q) {
 
 static uint32_t pieces_of(uint32_t dim) { return dim <= 32 ? 2 : dim <= 64 ? 4 : 8; } // 16-byte pieces of a key per lane
 
-template <int REP, int DQ> static int step_kernels(cg_backend *be, const DeferredStep &s) {
-    constexpr int PI = 8 / DQ; // keys of four lanes: 8 pieces per lane
-    if (int rc = allow_lds(reinterpret_cast<const void *>(&attention_mixed_step_kernel<REP, DQ, PI>), s.lds)) return rc;
-    launch_kernel((attention_mixed_step_kernel<REP, DQ, PI>), dim3(s.segs, s.plan.B * s.plan.S), dim3(kThreads), s.lds, be->stream, s.plan, s.chunk, s.chunks, s.parts, s.stats);
-    return CG_OK;
+typedef void (*StepKernel)(AttentionPlan, uint32_t, uint32_t, float *, float2 *);
+template <int REP> static StepKernel step_kernel(uint32_t dq) { // (PI: keys of four lanes, 8 pieces per lane)
+    return dq == 2 ? attention_mixed_step_kernel<REP, 2, 4> : dq == 4 ? attention_mixed_step_kernel<REP, 4, 2> : attention_mixed_step_kernel<REP, 8, 1>;
+}
+static StepKernel step_kernel(const AttentionPlan &p) {
+    const uint32_t rep = p.heads / p.kv_heads, dq = pieces_of(p.dim);
+    return rep <= 1 ? step_kernel<1>(dq) : rep <= 2 ? step_kernel<2>(dq) : rep <= 4 ? step_kernel<4>(dq) : step_kernel<8>(dq);
 }
 template <int REP, int DQ>
 static int step_kernels_beside(cg_backend *be, const DeferredStep &s, const ExpertsPlan &e, float *hidden, uint32_t *chosen) {
@@ -863,15 +865,8 @@ static int merge_step(cg_backend *be, const DeferredStep &s) {
 }
 
 int run_step(cg_backend *be, const DeferredStep &s) {
-    const uint32_t rep = s.plan.heads / s.plan.kv_heads, dq = pieces_of(s.plan.dim);
-    int rc;
-#define CG_STEP(R) (dq == 2 ? step_kernels<R, 2>(be, s) : dq == 4 ? step_kernels<R, 4>(be, s) : step_kernels<R, 8>(be, s))
-    if (rep <= 1) rc = CG_STEP(1);
-    else if (rep <= 2) rc = CG_STEP(2);
-    else if (rep <= 4) rc = CG_STEP(4);
-    else rc = CG_STEP(8);
-#undef CG_STEP
-    return rc ? rc : merge_step(be, s);
+    launch_kernel(step_kernel(s.plan), dim3(s.segs, s.plan.B * s.plan.S), dim3(kThreads), s.lds, be->stream, s.plan, s.chunk, s.chunks, s.parts, s.stats);
+    return merge_step(be, s);
 }
 
 // Heads of 33 to 128 columns, up to four to a kv head, and experts whose rows lie in 16-byte pieces: what the shared kernel is compiled for.
@@ -908,6 +903,8 @@ int launch_mixed_step(cg_backend *be, const AttentionPlan &p, DeferredStep **lat
     // as many workgroups as run at a time
     const uint32_t all = (most + chunk - 1) / chunk;
     const uint32_t resident = (rep <= 4 ? 3 : 2) * be->compute_units, chunks = (uint32_t)(((uint64_t)rows * all + resident - 1) / resident), nseg = (all + chunks - 1) / chunks;
+    // (here and not when it is launched: a refusal is this call's)
+    if (int rc = allow_lds(reinterpret_cast<const void *>(step_kernel(p)), lds)) return rc;
     DeferredStep *const s = new DeferredStep;
     const size_t n = (size_t)rows * nseg * p.heads;
     if (int rc = be->pool.alloc(n * p.vdim * 4 + n * sizeof(float2), &s->mem, &s->cls)) {

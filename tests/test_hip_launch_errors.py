@@ -1,5 +1,5 @@
-"""Launches that are refused behind the call that asked for them: the next wait says which one and why, once, and nothing of it is a later call's.
-A second process, in which chosen requests to the runtime are refused
+"""Launches that are refused behind the call that asked for them: the next wait says which one and why, once, and nothing of it is a later call's;
+what the host can tell before a launch is the call's own error.  A second process, in which chosen requests to the runtime are refused
 (no kernel runs that should not)."""
 import os
 import subprocess
@@ -14,18 +14,24 @@ SHIM = r"""
 #include <stddef.h>
 #include <atomic>
 struct dim { unsigned x, y, z; };
-static std::atomic<int> launch{0}, refused{0};
+static std::atomic<int> launch{0}, attribute{0}, refused{0};
 static void *next(const char *name) {
     void *runtime = dlopen("libamdhip64.so.7", RTLD_LAZY | RTLD_NOLOAD);
     return runtime ? dlsym(runtime, name) : nullptr;
 }
 extern "C" {
 void refuse_launch(int code) { refused = 0, launch = code; }        // the next launch comes to `code`
+void refuse_attribute(int code) { refused = 0, attribute = code; }  // so does every reservation, until it is 0 again
 int count(void) { return refused; }
 int hipLaunchKernel(const void *f, dim g, dim b, void **a, size_t l, void *s) {
     if (const int code = launch.exchange(0)) return refused++, code;
     static const auto to = (int (*)(const void *, dim, dim, void **, size_t, void *))next("hipLaunchKernel");
     return to ? to(f, g, b, a, l, s) : 999;
+}
+int hipFuncSetAttribute(const void *f, int what, int value) {
+    if (attribute) return refused++, attribute.load();
+    static const auto to = (int (*)(const void *, int, int))next("hipFuncSetAttribute");
+    return to ? to(f, what, value) : 999;
 }
 }
 """
@@ -35,6 +41,7 @@ import ctypes, sys
 shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)        # before the library: its requests come here first
 sys.path.insert(0, sys.argv[2])
 import numpy as np
+import block_cases as C
 from catgrad_amd import BackendPanic, HipBackend
 be = HipBackend(0)
 
@@ -77,6 +84,21 @@ refused(be.to_numpy, lambda: be.realize(be.index(table, 0, far)))
 be.realize(be.index(table, 0, far))
 assert "out of bounds" in error(be.sync)
 print("with a fault", flush=True)
+
+# attention over mixed scores whose launch waits for the next call: 71 KB of LDS to be reserved
+o = C.turned(32, 16, 128, 64, 16)
+t = C.attention_case(np.random.default_rng(0), 1, 6, o, norms=False)
+def attention():
+    c = {n: be.from_numpy(np.ones((1, 16, 5, d), dtype=np.float32)) for n, d in (("k_cache", 128), ("v_cache", 64))}
+    y, k, v = be.block_attention({**{n: be.from_numpy(t[n]) for n in ("q", "k", "v", "talk")}, **c}, position=5, **o)
+    return y
+shim.refuse_attribute(9)
+got = error(attention)
+assert shim.count() > 0
+shim.refuse_attribute(0)
+assert got and "HIP error 9" in got, got
+assert error(be.sync) is None
+assert np.isfinite(be.to_numpy(attention())).all()
 print("done", flush=True)
 """
 
