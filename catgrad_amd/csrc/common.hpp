@@ -42,7 +42,7 @@ class Pool {
     void free(void *ptr, size_t cls);
     void trim();
     void stats(size_t *in_use, size_t *cached);
-    LaunchQueue *launches = nullptr; // of the stream: blocks go back to the device behind all that was launched
+    cg_backend *owner = nullptr; // blocks go back to the device behind all that was launched, and what waits to be gives up its own
     static size_t size_class(size_t bytes);
 
   private:

@@ -68,6 +68,10 @@ int Pool::alloc(size_t bytes, void **ptr, size_t *cls) {
     hipError_t e = hipMalloc(&p, c);
     if (e != hipSuccess) {
         (void)hipGetLastError();
+        if (owner && (owner->step || owner->sum)) { // what waits for its launch holds memory (nothing waits behind this)
+            flush_waiting(owner);
+            return alloc(bytes, ptr, cls);
+        }
         trim();
         e = hipMalloc(&p, c);
         if (e != hipSuccess) return hip_fail(e, "hipMalloc");
@@ -93,7 +97,7 @@ void Pool::trim() {
         take.swap(free_);
         cached_ = 0;
     }
-    if (launches) launches->drain();
+    if (owner) owner->stream.drain();
     for (auto &kv : take) (void)hipFree(kv.second);
 }
 
@@ -2270,7 +2274,7 @@ int cg_backend_create(int device, cg_backend **out) {
     cg_backend *b = new cg_backend;
     b->device = device;
     CG_HIP(b->stream.open(device));
-    b->pool.launches = &b->stream;
+    b->pool.owner = b;
     CG_HIP(hipHostMalloc((void **)&b->fault_host, 64, hipHostMallocMapped));
     memset(b->fault_host, 0, 64);
     CG_HIP(hipHostGetDevicePointer((void **)&b->fault_dev, b->fault_host, 0));
