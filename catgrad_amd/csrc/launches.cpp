@@ -1,10 +1,40 @@
 // The thread that passes a backend's launches on (launches.hpp).
 #include "launches.hpp"
 
+#include <sched.h>
+
+#include <algorithm>
 #include <chrono>
+#include <cstdlib>
+#include <fstream>
+#include <string>
 #include <system_error>
 
 namespace cg {
+
+double usable_cores(const char *membership, const char *mount) {
+    cpu_set_t set;
+    double cores = sched_getaffinity(0, sizeof set, &set) == 0 ? std::max(CPU_COUNT(&set), 1) : 1e9; // (more cores than a set holds)
+    std::ifstream groups(membership);
+    for (std::string line; std::getline(groups, line);) { // "<hierarchy>:<controllers>:<path>"; the unified hierarchy names no controllers
+        const size_t a = line.find(':'), b = a == std::string::npos ? a : line.find(':', a + 1);
+        if (b == std::string::npos) continue;
+        const std::string what = "," + line.substr(a + 1, b - a - 1) + ",", root = std::string(mount) + (what == ",," ? "" : "/cpu");
+        if (what != ",," && what.find(",cpu,") == std::string::npos) continue;
+        for (std::string path = line.substr(b + 1);;) { // (a group has no more than those around it; in a container the path may be another one's)
+            const std::string at = root + (path == "/" ? "" : path);
+            std::string quota;
+            double given = 0, period = 0;
+            if (what == ",,") std::ifstream(at + "/cpu.max") >> quota >> period; // "max <period>" or "<quota> <period>"
+            else if (std::ifstream(at + "/cpu.cfs_quota_us") >> quota) std::ifstream(at + "/cpu.cfs_period_us") >> period;
+            if ((given = atof(quota.c_str())) > 0 && period > 0) cores = std::min(cores, given / period); // (no limit: "max", -1)
+            if (path.empty() || path == "/") break;
+            const size_t cut = path.rfind('/');
+            path.resize(cut == std::string::npos ? 0 : cut);
+        }
+    }
+    return cores;
+}
 
 hipError_t LaunchQueue::open(int device) {
     device_ = device;
@@ -37,16 +67,21 @@ void LaunchQueue::wake() {
         cv_.notify_one();
         return;
     }
-    try {
-        thread_ = std::thread([this] { work(); });
-    } catch (const std::system_error &) { // no thread to be had: what was handed over is passed on here, and so is what follows
-        while (done_.load() != head_.load()) {
-            pass_on(slots_[done_.load() % kSlots]);
-            done_.fetch_add(1);
+    // (here, where the thread takes over what the caller is bound to)
+    if (usable_cores() >= 2) {
+        try {
+            thread_ = std::thread([this] { work(); });
+            return;
+        } catch (const std::system_error &) {
         }
-        awake_.store(false);
-        slots_.reset();
     }
+    // no thread to be had, or no core for it: what was handed over is passed on here, and so is what follows
+    while (done_.load() != head_.load()) {
+        pass_on(slots_[done_.load() % kSlots]);
+        done_.fetch_add(1);
+    }
+    awake_.store(false);
+    slots_.reset();
 }
 
 void LaunchQueue::work() {
@@ -63,7 +98,11 @@ void LaunchQueue::work() {
         }
         __builtin_ia32_pause();
         if (spins == 1) idle = std::chrono::steady_clock::now();
-        if (spins % 64 || std::chrono::steady_clock::now() - idle < kLinger) continue;
+        if (spins % 64) continue;
+        if (std::chrono::steady_clock::now() - idle < kLinger) {
+            std::this_thread::yield();
+            continue;
+        }
         std::unique_lock<std::mutex> lk(mu_);
         awake_.store(false);
         if (head_.load() != n) { // handed over in the meantime

@@ -4,7 +4,8 @@
 // small model 1.25 ms, where its kernels take 0.8.  So a backend that launches many kernels between two waits of the host hands
 // them to a thread of its own, which does nothing but pass them on, in order, while the calling thread goes on (SmolLM2-135M shape
 // 1.25 -> 0.97 ms a step, Qwen3-0.6B shape 1.66 -> 1.42).  The thread sleeps while there is nothing to pass on, and a few launches do not wake
-// it: waking takes longer than they do.
+// it: waking takes longer than they do.  Two threads that wait for each other need two cores: a process that may use less launches
+// everything itself, and whoever waits longer than a launch takes lets others have its core.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -23,6 +24,15 @@
 
 namespace cg {
 
+// A turn of waiting for another thread; 512 of them take 20 us.
+inline void wait_turn(uint32_t &turns) {
+    if (++turns % 512) __builtin_ia32_pause();
+    else std::this_thread::yield();
+}
+// Cores that the calling thread and what it starts may use: what it is bound to, and the processor time that its control groups are given
+// (`membership` names them, `mount` is where they lie).
+double usable_cores(const char *membership = "/proc/self/cgroup", const char *mount = "/sys/fs/cgroup");
+
 class LaunchQueue {
   public:
     LaunchQueue() = default;
@@ -37,7 +47,7 @@ class LaunchQueue {
         return stream_;
     }
     void drain() {
-        while (done_.load(std::memory_order_acquire) != head_.load(std::memory_order_relaxed)) __builtin_ia32_pause();
+        for (uint32_t turns = 0; done_.load(std::memory_order_acquire) != head_.load(std::memory_order_relaxed);) wait_turn(turns);
     }
     // The host has waited for the device: the launches up to the next time are counted anew.
     void waited() { direct_ = 0; }
@@ -58,7 +68,7 @@ class LaunchQueue {
         if constexpr (sizeof(J) <= sizeof(Slot::job)) {
             if (hands_over()) {
                 const uint64_t n = head_.load(std::memory_order_relaxed);
-                while (n - done_.load(std::memory_order_acquire) >= kSlots) __builtin_ia32_pause();
+                for (uint32_t turns = 0; n - done_.load(std::memory_order_acquire) >= kSlots;) wait_turn(turns);
                 Slot &s = slots_[n % kSlots];
                 new (s.job) J{kernel, grid, block, lds, std::tuple<std::decay_t<P>...>(std::forward<A>(a)...)};
                 s.run = &J::run;

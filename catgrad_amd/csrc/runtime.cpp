@@ -794,11 +794,10 @@ static int wait_for_readback(cg_backend *be, uint32_t seq, uint32_t groups) {
     if (be->prof_pending.size() > 2048) return wait_and_check(be);
     volatile uint32_t *word = be->rb_host + kReadbackWords, *const end = word + 16 * groups;
     const auto t0 = std::chrono::steady_clock::now();
-    for (uint32_t spins = 0;; spins++) {
+    for (uint32_t turns = 0;; wait_turn(turns)) {
         while (word != end && *word == seq) word += 16;
         if (word == end) break;
-        if ((spins & 1023) == 1023 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(100)) return wait_and_check(be);
-        __builtin_ia32_pause();
+        if ((turns & 1023) == 1023 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(100)) return wait_and_check(be);
     }
     std::atomic_thread_fence(std::memory_order_acquire);
     be->stream.waited();

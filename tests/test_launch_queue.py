@@ -1,7 +1,7 @@
 """The queue between a backend and its launching thread (launches.hpp) on stand-ins for the runtime's calls: what a launch is given, in which order
 launches are passed on, and what becomes of one that fails.  No GPU: a "kernel" is a plain function that the stand-in calls."""
-import subprocess
 import os
+import subprocess
 
 import pytest
 
@@ -98,3 +98,88 @@ int main() {
     return !ok;
 }
 """, {"CG_LAUNCH_THREAD": thread})
+
+
+def test_one_core(tmp_path):
+    """A process that may use one core has every launch made by its caller."""
+    passes(tmp_path, r"""
+int main() {
+    auto &q = *queue();
+    for (int n = 0; n < 500; n++) launch(q, n);
+    q.drain();
+    bool ok = check(by_thread == 0, "no other thread");
+    ok &= check(seen.size() == 500, "all launched");
+    for (int n = 0; n < (int)seen.size(); n++) ok &= check(seen[n] == n, "in order");
+    q.close();
+    if (ok) printf("done\n");
+    return !ok;
+}
+""", prefix=("taskset", "-c", str(min(os.sched_getaffinity(0)))))
+
+
+@pytest.mark.skipif(len(os.sched_getaffinity(0)) < 2, reason="a process on one core has no other thread")
+def test_threads_moved_to_one_core(tmp_path):
+    """A wait lets the thread that it waits for have the core, in less than a scheduler's turn (0.6 ms of processor time a hand-over here)."""
+    passes(tmp_path, r"""
+#include <dirent.h>
+#include <sched.h>
+#include <time.h>
+int main() {
+    auto &q = *queue();
+    for (int n = 0; n < 100; n++) launch(q, n);
+    q.drain();
+    if (by_thread == 0) return printf("done\n"), 0; // (its control group has less than two cores)
+    cpu_set_t set, one;
+    sched_getaffinity(0, sizeof set, &set);
+    CPU_ZERO(&one);
+    for (int c = 0; c < CPU_SETSIZE; c++)
+        if (CPU_ISSET(c, &set)) {
+            CPU_SET(c, &one);
+            break;
+        }
+    DIR *d = opendir("/proc/self/task");
+    while (dirent *e = readdir(d))
+        if (int t = atoi(e->d_name)) sched_setaffinity(t, sizeof one, &one);
+    closedir(d);
+    timespec a, b;
+    clock_gettime(CLOCK_PROCESS_CPUTIME_ID, &a);
+    for (int i = 0; i < 200; i++) {
+        launch(q, i);
+        q.drain();
+    }
+    clock_gettime(CLOCK_PROCESS_CPUTIME_ID, &b);
+    const double us = ((b.tv_sec - a.tv_sec) * 1e6 + (b.tv_nsec - a.tv_nsec) * 1e-3) / 200;
+    printf("%.0f us of processor time a hand-over\n", us);
+    const bool ok = check(us < 250, "the wait gives way");
+    q.close();
+    if (ok) printf("done\n");
+    return !ok;
+}
+""")
+
+
+@pytest.mark.parametrize("membership,files,most", [
+    ("0::/\n", {"cpu.max": "max 100000"}, None),
+    ("0::/\n", {"cpu.max": "150000 100000"}, 1.5),
+    ("0::/a/b\n", {"a/cpu.max": "50000 100000", "a/b/cpu.max": "max 100000"}, 0.5),
+    ("0::/not/here\n", {"cpu.max": "100000 100000"}, 1.0),
+    ("5:memory:/a\n4:cpu,cpuacct:/a\n", {"cpu/a/cpu.cfs_quota_us": "25000", "cpu/a/cpu.cfs_period_us": "100000", "cpu/cpu.cfs_quota_us": "-1"}, 0.25),
+    ("3:cpuset:/a\n", {"cpu/a/cpu.cfs_quota_us": "25000", "cpu/a/cpu.cfs_period_us": "100000"}, None),
+    ("1:cpu:/\nnonsense\n0::x\n", {"cpu.max": "", "cpu/cpu.cfs_quota_us": "100000"}, None),
+], ids=lambda v: str(v) if isinstance(v, (float, type(None))) else "")
+def test_processor_time(tmp_path, membership, files, most):
+    """The least that a control group of the process is given, up to its bound cores."""
+    (tmp_path / "membership").write_text(membership)
+    for name, text in files.items():
+        (tmp_path / "mount" / name).parent.mkdir(parents=True, exist_ok=True)
+        (tmp_path / "mount" / name).write_text(text + "\n")
+    bound = len(os.sched_getaffinity(0))
+    want = bound if most is None else min(most, bound)
+    passes(tmp_path, r"""
+int main() {
+    const double got = cg::usable_cores("%s", "%s");
+    if (check(got == %r, "cores")) printf("done\n");
+    else printf("%%g\n", got);
+    return 0;
+}
+""" % (tmp_path / "membership", tmp_path / "mount", float(want)))
