@@ -2,6 +2,7 @@
 #include "launches.hpp"
 
 #include <sched.h>
+#include <unistd.h>
 
 #include <algorithm>
 #include <chrono>
@@ -9,8 +10,29 @@
 #include <fstream>
 #include <string>
 #include <system_error>
+#include <vector>
 
 namespace cg {
+namespace {
+
+// The open queues of the process, for its end.  (Never destroyed: a thread may close one while the process ends.)
+struct Open {
+    std::mutex mu;
+    std::vector<LaunchQueue *> all;
+    pid_t process = 0;
+};
+Open &open_queues() {
+    static Open *const o = new Open;
+    return *o;
+}
+void end_of_process() {
+    Open &o = open_queues();
+    if (getpid() != o.process) return; // (a forked child has none of the threads)
+    std::lock_guard<std::mutex> lk(o.mu);
+    for (LaunchQueue *q : o.all) q->end();
+}
+
+} // namespace
 
 double usable_cores(const char *membership, const char *mount) {
     cpu_set_t set;
@@ -41,10 +63,22 @@ hipError_t LaunchQueue::open(int device) {
     if (const hipError_t e = hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking)) return e;
     const char *t = getenv("CG_LAUNCH_THREAD"); // CG_LAUNCH_THREAD=0: every launch is the caller's
     if (!(t && t[0] == '0')) slots_.reset(new (std::nothrow) Slot[kSlots]);
+    Open &o = open_queues();
+    std::lock_guard<std::mutex> lk(o.mu);
+    if (!o.process) { // (behind the runtime's first call: what that leaves for the end of the process comes after this)
+        o.process = getpid();
+        (void)atexit(end_of_process);
+    }
+    o.all.push_back(this);
     return hipSuccess;
 }
 
 void LaunchQueue::close() {
+    {
+        Open &o = open_queues();
+        std::lock_guard<std::mutex> lk(o.mu);
+        o.all.erase(std::remove(o.all.begin(), o.all.end(), this), o.all.end());
+    }
     drain();
     if (thread_.joinable()) {
         {

@@ -40,6 +40,12 @@ class LaunchQueue {
     LaunchQueue &operator=(const LaunchQueue &) = delete;
     hipError_t open(int device);
     void close(); // everything handed over is on the stream; the thread ends, the stream goes
+    // The process ends with this queue open: what was handed over is on the stream, and from now on every launch is its caller's (the
+    // runtime goes next, and the thread must not be in it by then).
+    void end() {
+        ended_.store(true);
+        drain();
+    }
 
     // The stream, for anything but launch_kernel: what has been handed over is on it by then.
     operator hipStream_t() {
@@ -108,7 +114,7 @@ class LaunchQueue {
         }
     };
     bool hands_over() {
-        if (!slots_) return false;
+        if (!slots_ || ended_.load(std::memory_order_acquire)) return false;
         if (awake_.load(std::memory_order_acquire)) return true;
         return ++direct_ > kDirect;
     }
@@ -127,7 +133,7 @@ class LaunchQueue {
     std::unique_ptr<Slot[]> slots_;  // null: every launch is the caller's
     alignas(64) std::atomic<uint64_t> head_{0}; // launches handed over
     alignas(64) std::atomic<uint64_t> done_{0}; // launches passed on
-    std::atomic<bool> awake_{false};
+    std::atomic<bool> awake_{false}, ended_{false};
     std::atomic<hipError_t> failed_{hipSuccess};
     const void *failed_kernel_ = nullptr; // (written in front of failed_)
     bool stop_ = false;              // (under mu_)

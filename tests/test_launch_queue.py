@@ -183,3 +183,45 @@ int main() {
     return 0;
 }
 """ % (tmp_path / "membership", tmp_path / "mount", float(want)))
+
+
+@pytest.mark.parametrize("closed", [False, True])
+def test_end_of_process(tmp_path, closed):
+    """A process that ends with launches on their way has them made before the runtime goes, and none behind it."""
+    passes(tmp_path, r"""
+static void gone() {
+    runtime_gone = 1;
+    std::this_thread::sleep_for(std::chrono::milliseconds(20));
+    if (seen.size() == 60) printf("done\n");
+}
+int main() {
+    atexit(gone); // (the runtime's own, left there by its first call)
+    auto &q = *queue(), &other = *queue();
+    busy_us = 100;
+    for (int n = 0; n < 60; n++) launch(q, n);
+    if (%d) q.close();
+    other.close();
+    return 0;
+}
+""" % closed)
+
+
+def test_forked_child_ends(tmp_path):
+    """A forked child has none of its parent's threads: it ends without waiting for one."""
+    passes(tmp_path, r"""
+#include <sys/wait.h>
+int main() {
+    auto &q = *queue();
+    busy_us = 1000;
+    for (int n = 0; n < 60; n++) launch(q, n);
+    const pid_t child = fork();
+    if (!child) exit(7);
+    int status = 0;
+    for (int i = 0; i < 500 && !waitpid(child, &status, WNOHANG); i++) usleep(10000);
+    const bool ok = check(WIFEXITED(status) && WEXITSTATUS(status) == 7, "the child's own end");
+    if (!ok) kill(child, SIGKILL);
+    q.close();
+    if (ok) printf("done\n");
+    return !ok;
+}
+""".replace("#include <sys/wait.h>", "#include <signal.h>\n#include <sys/wait.h>"))
