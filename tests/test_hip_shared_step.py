@@ -4,13 +4,16 @@ import numpy as np
 import pytest
 
 import block_cases as C
+import kernel_names
 
 pytestmark = pytest.mark.gpu
 
 # query heads per kv head and head widths that the shared kernel is compiled for, one that it is not (16 columns), a model's width in one to
-# eight pieces of a wave's loads and beyond, rows whose length is not whole 16-byte pieces
+# eight pieces of a wave's loads and beyond, rows whose length is not whole 16-byte pieces; LDS for two workgroups
+SHARES = [True, True, True, True, True, True, False, False, False, False, True]
 CASES = [(4, 4, 64, 64, 256, "f32", 1, 1), (8, 4, 128, 128, 1024, "f32", 1, 1), (8, 2, 48, 32, 520, "bf16", 1, 2), (16, 8, 128, 128, 1024, "bf16", 2, 2), (8, 2, 96, 64, 2048, "f32", 1, 8),
-         (4, 2, 64, 64, 4096, "bf16", 1, 1), (4, 2, 64, 64, 4352, "f32", 1, 1), (4, 2, 64, 64, 262, "f32", 1, 1), (4, 2, 16, 16, 256, "f32", 1, 1), (16, 2, 64, 64, 256, "f32", 1, 1)]
+         (4, 2, 64, 64, 4096, "bf16", 1, 1), (4, 2, 64, 64, 4352, "f32", 1, 1), (4, 2, 64, 64, 262, "f32", 1, 1), (4, 2, 16, 16, 256, "f32", 1, 1), (16, 2, 64, 64, 256, "f32", 1, 1),
+         (32, 8, 128, 64, 256, "f32", 1, 8)]
 
 
 def run(be, case, between, seed=0):
@@ -95,3 +98,27 @@ def test_results_dropped(hip):
         del r, caches
     hip.sync()
     assert hip.pool_stats()[0] <= before + 4096
+
+
+def test_which_share(tmp_path):
+    """The kernel that both share runs where it should, once, and nowhere else."""
+    kernel_names.run(tmp_path, r"""
+from catgrad_amd import HipBackend
+import test_hip_shared_step as T
+be = HipBackend(0)
+
+
+def check(what, shares, *a):
+    names = launches(be, T.run, be, *a)
+    n = sum("attention_step_experts_kernel" in k for k in names)
+    print(what, n, flush=True)
+    assert n == shares and sum("attention_mixed_step_kernel" in k for k in names) == 1 - shares, names
+
+
+for case, shares in zip(T.CASES, T.SHARES):
+    check(case, int(shares), case, T.nothing)
+    check("with a wait", 0, case, T.waits)
+for f in (T.reads_result, T.reads_caches, T.drops_memory):
+    check(f.__name__, 0, T.CASES[1], f)
+print("done", flush=True)
+""")

@@ -5,11 +5,13 @@ import numpy as np
 import pytest
 
 import block_cases as C
+import kernel_names
 
 pytestmark = pytest.mark.gpu
 
 # sequences, width, groups, taps, outputs, whether there is a state: one to three pieces of a workgroup's loads, a group in two workgroups, groups shorter than a wave's piece and
 # longer than one; other numbers of taps, a width that is not whole 16-byte pieces (neither goes along)
+SHARES = [True] * 7 + [False] * 2
 CASES = [(1, 1024, 4, 4, 2, True), (3, 1024, 1, 4, 2, True), (2, 2048, 8, 4, 1, False), (1, 2304, 1, 4, 2, True), (8, 264, 2, 4, 1, True), (1, 96, 3, 4, 2, False), (1, 4096, 2, 4, 2, True),
          (2, 1024, 4, 3, 2, True), (1, 262, 2, 4, 1, True)]
 
@@ -86,3 +88,29 @@ def test_result_dropped(hip):
         run(hip, CASES[0], lambda be, z: None)
     hip.sync()
     assert hip.pool_stats()[0] <= before + 4096
+
+
+def test_which_share(tmp_path):
+    """The filters take the sum along where they should, and it runs by itself everywhere else."""
+    kernel_names.run(tmp_path, r"""
+from catgrad_amd import HipBackend
+import test_hip_shared_sum as T
+be = HipBackend(0)
+
+
+def check(what, shares, *a, **kw):
+    names = launches(be, T.run, be, *a, **kw)
+    own = sum("side_sum_kernel" in k for k in names)
+    print(what, own, flush=True)
+    assert own == 1 - shares, names
+    assert sum("conv_token_kernelILb1E" in k or "conv_token_kernel<true>" in k for k in names) == shares, names
+
+
+for case, shares in zip(T.CASES, T.SHARES):
+    check(case, int(shares), case, lambda be, z: None)
+    check("with a wait", 0, case, lambda be, z: be.sync())
+check("two tokens", 0, T.CASES[0], lambda be, z: None, S=2)
+for f in (T.reads_result, T.drops_memory, T.another_sum):
+    check(f.__name__, 0, T.CASES[0], f)
+print("done", flush=True)
+""")
