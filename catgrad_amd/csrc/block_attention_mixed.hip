@@ -842,14 +842,16 @@ static StepKernel step_kernel(const AttentionPlan &p) {
 template <int REP, int DQ>
 static int step_kernels_beside(cg_backend *be, const DeferredStep &s, const ExpertsPlan &e, float *hidden, uint32_t *chosen) {
     constexpr int PI = 8 / DQ;
-    // The experts' columns on what is resident beside attention (three workgroups a compute unit): those of a second round would start with the
-    // choice of the experts when the first ones end.
-    const uint32_t beside = std::max((uint32_t)be->compute_units, 3u * (uint32_t)be->compute_units - std::min(2u * (uint32_t)be->compute_units, s.segs * s.plan.B * s.plan.S));
+    const size_t lds = std::max(s.lds, route_bytes(e));
+    if (lds > (64u << 10)) return kDeclined;
+    // The experts' columns on what is resident beside attention (three workgroups a compute unit, two where its LDS holds no more): those of a
+    // second round would start with the choice of the experts when the first ones end.
+    const uint32_t units = be->compute_units, at_once = std::min<uint32_t>(3, (uint32_t)(kMaxLds / lds));
+    const uint32_t beside = std::max(units, at_once * units - std::min((at_once - 1) * units, s.segs * s.plan.B * s.plan.S));
     const uint64_t columns = (uint64_t)e.rows * e.top * e.ff;
     const uint32_t per_wave = (uint32_t)std::clamp<uint64_t>((columns + (uint64_t)beside * kExpertWaves - 1) / ((uint64_t)beside * kExpertWaves), 1, 16), bx = (e.ff + kExpertWaves * per_wave - 1) / (kExpertWaves * per_wave);
     const uint64_t blocks = (uint64_t)s.segs * s.plan.B * s.plan.S + (uint64_t)bx * e.rows * e.top;
-    const size_t lds = std::max(s.lds, route_bytes(e));
-    if (blocks > 0x7FFFFFFFull || lds > (64u << 10)) return kDeclined;
+    if (blocks > 0x7FFFFFFFull) return kDeclined;
     if (e.fmt == kFmtBF16)
         launch_kernel((attention_step_experts_kernel<REP, DQ, PI, true>), dim3((uint32_t)blocks), dim3(kThreads), lds, be->stream, s.plan, s.chunk, s.chunks, s.parts, s.stats, s.segs,
                       e, per_wave, bx, hidden, chosen);
