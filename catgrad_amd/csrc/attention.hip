@@ -145,17 +145,18 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
     // caches, and from 1024 positions when there are more query rows than compute units.  Measured with its combine launch
     // against the kernels below (batch 4 x 8 KV heads x 4 rows, head_dim 64): 9000 positions 44 against 55, 12000 positions 53 against 64;
     // batch 16 at 2100 positions 42 against 46.  A single sequence (at most 8 groups) leaves the kernels below most of the device idle:
-    // beyond kRowMaxT it always takes the segments (8 KV heads, head_dim 128: 12000 positions 31.7 against 59.0).
+    // beyond kRowMaxT it always takes the segments (8 KV heads, head_dim 128: 12000 positions 31.7 against 59.0; 3 of 64, 4500 16.7 and 20.0).
     // Up to kRowMaxT by what either takes, in us: a row is its compute unit's share of the cache; the segments are two launches and the
     // hand-over between them (1 us) up to what the device streams.  One row and one segment pair, SmolLM2-135M shape (3 KV heads of 64, one
     // sequence) 512 positions 7.3 and 10.0, 1024 11.6 and 10.2, 2047 17.3 and 10.1; Qwen3-0.6B (8 of 128) 384 10.4 and 10.2, 512 12.1 and
     // 10.2, 768 15.6 and 10.3, four sequences 512 12.7 and 10.9, 1024 19.2 and 15.0; Llama-3.2-1B (8 of 64) 1024 11.3 and 11.0, 1536 14.5
-    // and 11.1, four sequences 1536 15.5 and 14.4, 2047 18.4 and 16.0.
+    // and 11.1, four sequences 1536 15.5 and 14.4, 2047 18.4 and 16.0.  (So segments from 969 positions for the first, 485 and 644 for one and four
+    // sequences of the second, 1126 and 1646 of the third.)
     auto segments_win = [&] {
         const double values = (double)T * (double)hd, mb = 8e-6 * values * (double)f1.batch;
         const double row = 5.0 + 1.0e-4 * values * (qrows > 128 ? 1.3 : 1.0); // (more rows: a whole one per compute unit)
         const double seg = std::max(10.2, 7.6 + 0.22 * mb) + (f1.M > 4 ? 2.5 : f1.M > 3 ? 1.0 : 0.0) + 1.0;
-        return T > kRowMaxT ? f1.batch <= 8 && T * hd >= 131072 : seg < row;
+        return T > kRowMaxT ? f1.batch <= 8 : seg < row;
     };
     // (Merging the segments inside the kernel — the workgroup that counts itself last at a device-scope counter reads the
     // others' results — was measured and costs what the combine launch costs: the stores must reach memory, the count must come
@@ -177,7 +178,7 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
                 be->pool.free(so, cso);
                 room = false;
             }
-            if (!room) { // the kernels below: up to kRowMaxT without scratch memory
+            if (!room) { // the kernels below: a row per workgroup needs no scratch memory (up to kRowMaxT, beyond 1024 with at most 256 rows), the others ask for their own
                 (void)hipGetLastError();
                 g.chunk = other_chunk;
                 g.splits = other_splits;

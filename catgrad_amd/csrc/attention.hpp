@@ -687,7 +687,8 @@ __global__ __launch_bounds__(kSegBlock) void decode_attention_seg_kernel(const A
 // out[b][m][n] = sum_c e^(m_c - g) o_c[n] / sum_c e^(m_c - g) l_c.  A workgroup per (batch entry, query row), whose waves share the
 // chunks: lane c first holds the statistics of chunk c (each wave computes each weight e^(m_c - g) once and reads it from that lane), then
 // lane n sums output element n (and n + 64) over the wave's chunks, and the waves' sums meet in LDS.
-// Bound by latency: one trip to memory.  A wave per row, with a shuffle per chunk, took 4.74 us for 16 rows of 32 chunks of 128; so 2.83.
+// Bound by latency: one trip to memory.  A wave per row, with a shuffle per chunk, took 4.74 us for 16 rows of 32 chunks of 128; so 2.83 (3.33 in
+// Qwen3-0.6B's steps, behind the segments).
 __global__ __launch_bounds__(kBlock) void decode_attention_combine_kernel(const float *part_o, const float *part_ml, uint32_t *out, uint32_t splits, uint32_t M, uint32_t hd) {
     constexpr uint32_t kWaves = kBlock / 64, kTrip = 64, kMine = kTrip / kWaves; // chunks per trip, of which a wave takes every fourth
     __shared__ float sums[kWaves][2][64];

@@ -376,7 +376,8 @@ bool vector_rows(const ExpertsPlan &p) {
     const uint32_t vw = p.fmt == kFmtBF16 ? 8 : 4;
     return p.width % vw == 0 && p.ff % vw == 0 && aligned16(p.gate_up) && aligned16(p.down) && aligned16(p.h);
 }
-uint32_t expert_first_columns(const cg_backend *be, const ExpertsPlan &p) {
+// Columns that a wave takes where nothing runs beside: enough workgroups for the device, not many more.
+static uint32_t expert_first_columns(const cg_backend *be, const ExpertsPlan &p) {
     const uint32_t per = std::max(1u, (uint32_t)((uint64_t)p.rows * p.top * p.ff / ((uint64_t)be->compute_units * 8 * kWaves)));
     return std::min(per, 8u);
 }

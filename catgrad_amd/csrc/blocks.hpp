@@ -149,8 +149,7 @@ struct ExpertsPlan {
 int launch_experts(cg_backend *be, const ExpertsPlan &p, float *y, int *y_fmt);
 // A few rows: hidden[r, slot, 0 .. ff) (weights applied) and the chosen experts' numbers.
 int launch_experts_first(cg_backend *be, const ExpertsPlan &p, float *hidden, uint32_t *chosen);
-// Columns that a wave of it takes: enough workgroups for the device, not many more.  Whether its rows lie in 16-byte pieces.
-uint32_t expert_first_columns(const cg_backend *be, const ExpertsPlan &p);
+// Whether its rows lie in 16-byte pieces.
 bool vector_rows(const ExpertsPlan &p);
 // out[r] = x[r] + scale * (y[r] . w^T + sum_slot hidden[r, slot] . down[chosen[r, slot]]^T), rows <= kFewRows
 int launch_experts_second(cg_backend *be, const ExpertsPlan &p, const float *hidden, const uint32_t *chosen, const Rows &x, const Rows &y, const Weight *w, float scale,

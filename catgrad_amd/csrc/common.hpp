@@ -168,8 +168,8 @@ struct cg_backend {
     bool fuse = true; // defer element-wise ops and fuse them (CG_FUSE=0 switches it off)
     bool aot = true;  // use the compiled kernels for listed programs (CG_AOT=0: interpreter only)
     uint64_t programs_compiled = 0, programs_interpreted = 0; // launches of fused programs, by kernel kind
-    // decode-time attention over a cache of at least this many positions runs a workgroup per (KV head, segment of the
-    // cache) (CG_ATTN_SEG_FROM, read when the backend is created; 0: never)
+    // decode-time attention over a cache of at least this many positions always runs a workgroup per (KV head, segment of the
+    // cache), over a shorter one by the rule in launch_decode_attention (CG_ATTN_SEG_FROM, read when the backend is created; 0: never)
     int64_t attn_seg_from = 6001;
     bool narrow_storage = true;  // tensors of the narrow float dtypes keep 2- / 1-byte elements in memory (CG_NARROW_STORAGE=0: 32-bit words)
     int64_t narrow_from = 65536; // ... from this many elements on (CG_NARROW_FROM); smaller tensors stay 32-bit words: the kernels of a
@@ -569,9 +569,11 @@ bool rows_max_program_begun(const Pending &p);
 int launch_arange(cg_backend *be, cg_tensor *out);
 // Copies n <= kReadbackWords words to be->rb_dev, a run of them per workgroup, each of which then stores `seq` at a word of its own behind
 // them (64 bytes apart), visible to the host: 16-byte stores of many compute units, and nobody waits for anybody.
-// (2 MiB: the rows of logits that a step hands back.  The runtime's copy waits for the stream, which retires every kernel in front of it: behind
-// one kernel 49152 words 41 us and 29 here, 151936 65 and 50, but behind the 150 to 200 of a decode step 60 to 100 more: a step of the
-// SmolLM2-135M shape 0.93 -> 0.82 ms, Qwen3-0.6B 1.42 -> 1.36, Llama-3.2-1B 1.25 -> 1.19.)
+// (2 MiB, which each backend keeps pinned: the rows of logits that a step hands back.  The runtime's copy waits for the stream, which retires every
+// kernel in front of it: behind the 150 to 200 of a decode step 60 to 100 us, a step of the SmolLM2-135M shape 0.93 -> 0.82 ms, Qwen3-0.6B 1.42 ->
+// 1.36, Llama-3.2-1B 1.25 -> 1.19.  The runtime's copy and this one, us, with nothing in front of them: 256 words 22.5 and 10.1, 8192 11.4 and 11.3,
+// 49152 19.4 and 17.4, 151936 35.7 and 35.9, 262144 62 and 65, 524288 124 and 116; behind one kernel 8192 22.1 and 12.1, 151936 46.5 and 37.3,
+// 262144 76 and 70, 524288 135 and 119; behind 20 products 151936 134 and 117, 524288 219 and 202.  Beyond that not measured.)
 constexpr uint32_t kReadbackWords = 524288, kReadbackGroups = 64;
 // Workgroups of a copy: 16384 words 25 us with one, 21 with four; more are not faster.
 inline uint32_t readback_groups(uint32_t n) { return n / 4096 < 1 ? 1 : n / 4096 > kReadbackGroups ? kReadbackGroups : n / 4096; }

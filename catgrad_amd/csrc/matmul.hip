@@ -1670,7 +1670,7 @@ __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_group_rope_kerne
 // and this small launch finishes them: a workgroup per head of a product, a thread per (row, column) of the head; the
 // head's norm, the embedding and the store, op for op as the stand-alone programs (the sum of squares in runs of 16 columns).  A thread
 // norms its partner of the embedding as well, so that all loads go together and one barrier is enough: 4.8 -> 3.0 us for 24 heads
-// of 128.  Measured against one launch with a
+// of 128 (3.5 in the steps of the Qwen3-0.6B shape, 16 and 8 heads).  Measured against one launch with a
 // workgroup of 1024 threads per head (a compute unit streams about 25 GB/s on its own however deep its loads are queued,
 // so that launch is as slow as its heads are few: 23 to 29 us for the 32 heads of 128 x 1024 of the Qwen3-0.6B shape):
 // 9 + 3 us and a hand-over, 1.94 -> 1.66 ms per decode step of that shape.

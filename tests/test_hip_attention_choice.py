@@ -7,6 +7,7 @@ import sys
 import numpy as np
 import pytest
 
+import kernel_names
 import test_hip_no_room
 from cases import _np_decode_attention, decode_attention_ops, f32
 
@@ -23,6 +24,30 @@ def test_choice(hip, B, kvh, rep, hd, T):
     q, k, v = f32(400 + T, (B, kvh * rep, 1, hd)), f32(401 + T, (B, kvh, T, hd)), f32(402 + T, (B, kvh, T, hd))
     got = hip.to_numpy(decode_attention_ops(hip, hip.from_numpy(q), hip.from_numpy(k), hip.from_numpy(v), rep))
     np.testing.assert_allclose(got, _np_decode_attention(q, k, v, rep), rtol=1e-4, atol=1e-5)
+
+
+# the last length of rows and the first of segments
+EDGES = [(1, 8, 2, 128, 485), (1, 8, 4, 64, 1126), (1, 3, 3, 64, 969), (4, 8, 2, 128, 644), (4, 8, 4, 64, 1646), (1, 2, 8, 128, 680), (3, 2, 5, 64, 1360)]
+
+
+@pytest.mark.parametrize("B,kvh,rep,hd,T", [(*c[:4], c[4] + d) for c in EDGES for d in (-1, 0)])
+def test_edges(hip, B, kvh, rep, hd, T):
+    test_choice(hip, B, kvh, rep, hd, T)
+
+
+def test_which_is_chosen(tmp_path):
+    kernel_names.run(tmp_path, r"""
+from catgrad_amd import HipBackend
+from cases import decode_attention_ops, f32
+from test_hip_attention_choice import EDGES
+be = HipBackend(0)
+for B, kvh, rep, hd, first in EDGES:
+    for T, want in ((first - 1, "decode_attention_row_kernel"), (first, "decode_attention_seg_kernel")):
+        x = [be.from_numpy(f32(1, s)) for s in ((B, kvh * rep, 1, hd), (B, kvh, T, hd), (B, kvh, T, hd))]
+        names = [n for n in launches(be, lambda: be.realize(decode_attention_ops(be, *x, rep))) if "decode_attention" in n]
+        assert want in names[0] and len(names) == (2 if "seg" in want else 1), (B, kvh, rep, hd, T, names)
+print("done", flush=True)
+""")
 
 
 PROGRAM = r"""
