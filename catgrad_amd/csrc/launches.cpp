@@ -1,8 +1,8 @@
 // The thread that passes a backend's launches on (launches.hpp).
 #include "launches.hpp"
 
+#include <pthread.h>
 #include <sched.h>
-#include <unistd.h>
 
 #include <algorithm>
 #include <chrono>
@@ -19,7 +19,7 @@ namespace {
 struct Open {
     std::mutex mu;
     std::vector<LaunchQueue *> all;
-    pid_t process = 0;
+    bool watched = false;
 };
 Open &open_queues() {
     static Open *const o = new Open;
@@ -27,9 +27,14 @@ Open &open_queues() {
 }
 void end_of_process() {
     Open &o = open_queues();
-    if (getpid() != o.process) return; // (a forked child has none of the threads)
     std::lock_guard<std::mutex> lk(o.mu);
     for (LaunchQueue *q : o.all) q->end();
+}
+void before_fork() { open_queues().mu.lock(); }
+void behind_fork() { open_queues().mu.unlock(); }
+void in_child() {
+    for (LaunchQueue *q : open_queues().all) q->forked();
+    behind_fork();
 }
 
 } // namespace
@@ -65,9 +70,10 @@ hipError_t LaunchQueue::open(int device) {
     if (!(t && t[0] == '0')) slots_.reset(new (std::nothrow) Slot[kSlots]);
     Open &o = open_queues();
     std::lock_guard<std::mutex> lk(o.mu);
-    if (!o.process) { // (behind the runtime's first call: what that leaves for the end of the process comes after this)
-        o.process = getpid();
+    if (!o.watched) { // (behind the runtime's first call: what that leaves for the end of the process comes after this)
+        o.watched = true;
         (void)atexit(end_of_process);
+        (void)pthread_atfork(before_fork, behind_fork, in_child);
     }
     o.all.push_back(this);
     return hipSuccess;
@@ -80,33 +86,37 @@ void LaunchQueue::close() {
         o.all.erase(std::remove(o.all.begin(), o.all.end(), this), o.all.end());
     }
     drain();
-    if (thread_.joinable()) {
+    if (worker_) {
         {
-            std::lock_guard<std::mutex> lk(mu_);
-            stop_ = true;
+            std::lock_guard<std::mutex> lk(worker_->mu);
+            worker_->stop = true;
         }
-        cv_.notify_one();
-        thread_.join();
+        worker_->cv.notify_one();
+        worker_->thread.join();
+        worker_.reset();
     }
     if (stream_) (void)hipStreamDestroy(stream_);
     stream_ = nullptr;
 }
 
 void LaunchQueue::wake() {
-    {
-        std::lock_guard<std::mutex> lk(mu_);
-        awake_.store(true);
-    }
-    if (thread_.joinable()) {
-        cv_.notify_one();
+    if (worker_) {
+        {
+            std::lock_guard<std::mutex> lk(worker_->mu);
+            awake_.store(true);
+        }
+        worker_->cv.notify_one();
         return;
     }
     // (here, where the thread takes over what the caller is bound to)
     if (usable_cores() >= 2) {
         try {
-            thread_ = std::thread([this] { work(); });
+            worker_.reset(new Worker);
+            awake_.store(true);
+            worker_->thread = std::thread([this, w = worker_.get()] { work(*w); });
             return;
         } catch (const std::system_error &) {
+            worker_.reset();
         }
     }
     // no thread to be had, or no core for it: what was handed over is passed on here, and so is what follows
@@ -118,7 +128,7 @@ void LaunchQueue::wake() {
     slots_.reset();
 }
 
-void LaunchQueue::work() {
+void LaunchQueue::work(Worker &w) {
     constexpr auto kLinger = std::chrono::microseconds(300); // between a step's last launch and the next step's first
     (void)hipSetDevice(device_);
     uint64_t n = 0;
@@ -137,15 +147,15 @@ void LaunchQueue::work() {
             std::this_thread::yield();
             continue;
         }
-        std::unique_lock<std::mutex> lk(mu_);
+        std::unique_lock<std::mutex> lk(w.mu);
         awake_.store(false);
         if (head_.load() != n) { // handed over in the meantime
             awake_.store(true);
             spins = 0;
             continue;
         }
-        cv_.wait(lk, [this] { return awake_.load() || stop_; });
-        if (stop_) return;
+        w.cv.wait(lk, [&] { return awake_.load() || w.stop; });
+        if (w.stop) return;
         spins = 0;
     }
 }

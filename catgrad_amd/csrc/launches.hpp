@@ -46,6 +46,13 @@ class LaunchQueue {
         ended_.store(true);
         drain();
     }
+    // In a forked child, which has none of its parent's threads: what was handed over is the parent's, and every launch its caller's.
+    void forked() {
+        ended_.store(true);
+        awake_.store(false);
+        done_.store(head_.load());
+        (void)worker_.release(); // (never destroyed here: its thread waits in it, in the parent)
+    }
 
     // The stream, for anything but launch_kernel: what has been handed over is on it by then.
     operator hipStream_t() {
@@ -119,7 +126,8 @@ class LaunchQueue {
         return ++direct_ > kDirect;
     }
     void wake();
-    void work();
+    struct Worker;
+    void work(Worker &w);
     void pass_on(Slot &s) {
         const hipError_t e = s.run(s.job, stream_);
         if (e == hipSuccess || failed_.load(std::memory_order_acquire) != hipSuccess) return; // (the first one is kept)
@@ -136,10 +144,13 @@ class LaunchQueue {
     std::atomic<bool> awake_{false}, ended_{false};
     std::atomic<hipError_t> failed_{hipSuccess};
     const void *failed_kernel_ = nullptr; // (written in front of failed_)
-    bool stop_ = false;              // (under mu_)
-    std::mutex mu_;
-    std::condition_variable cv_;
-    std::thread thread_;
+    struct Worker {
+        bool stop = false;           // (under mu)
+        std::mutex mu;
+        std::condition_variable cv;
+        std::thread thread;
+    };
+    std::unique_ptr<Worker> worker_; // from the first launch that is handed over on
 };
 
 template <class... P, class... A> inline void launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, LaunchQueue &on, A &&...a) {

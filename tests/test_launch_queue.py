@@ -206,22 +206,34 @@ int main() {
 """ % closed)
 
 
-def test_forked_child_ends(tmp_path):
-    """A forked child has none of its parent's threads: it ends without waiting for one."""
+@pytest.mark.parametrize("asleep", [False, True])
+@pytest.mark.parametrize("child", ["exit(7);", "q.drain(); launch(q, 1000); q.close(); delete &q; if (seen.empty() || seen.back() != 1000) _exit(8); exit(7);"],
+                         ids=["ends", "closes"])
+def test_forked_child(tmp_path, child, asleep):
+    """A forked child has none of its parent's threads: it ends, or closes what it has inherited, without waiting for one; its launches are its own."""
     passes(tmp_path, r"""
+#include <signal.h>
 #include <sys/wait.h>
 int main() {
     auto &q = *queue();
     busy_us = 1000;
     for (int n = 0; n < 60; n++) launch(q, n);
+    if (%d) {
+        q.drain();
+        usleep(20000);
+    }
     const pid_t child = fork();
-    if (!child) exit(7);
+    if (!child) {
+        %s
+    }
     int status = 0;
-    for (int i = 0; i < 500 && !waitpid(child, &status, WNOHANG); i++) usleep(10000);
-    const bool ok = check(WIFEXITED(status) && WEXITSTATUS(status) == 7, "the child's own end");
-    if (!ok) kill(child, SIGKILL);
+    pid_t ended = 0;
+    for (int i = 0; i < 500 && !(ended = waitpid(child, &status, WNOHANG)); i++) usleep(10000);
+    const bool ok = check(ended == child && WIFEXITED(status) && WEXITSTATUS(status) == 7, "the child's own end");
+    if (!ok && !ended) kill(child, SIGKILL);
+    for (int n = 60; n < 120; n++) launch(q, n);
     q.close();
-    if (ok) printf("done\n");
+    if (ok && check(seen.size() == 120, "the parent's launches")) printf("done\n");
     return !ok;
 }
-""".replace("#include <sys/wait.h>", "#include <signal.h>\n#include <sys/wait.h>"))
+""" % (asleep, child))
