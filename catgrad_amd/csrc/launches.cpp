@@ -144,7 +144,7 @@ void LaunchQueue::work(Worker &w) {
         if (spins == 1) idle = std::chrono::steady_clock::now();
         if (spins % 64) continue;
         if (std::chrono::steady_clock::now() - idle < kLinger) {
-            std::this_thread::yield();
+            if (spins % 512 == 0) std::this_thread::yield(); // (not between the launches of a step)
             continue;
         }
         std::unique_lock<std::mutex> lk(w.mu);
