@@ -5,7 +5,8 @@
 // them to a thread of its own, which does nothing but pass them on, in order, while the calling thread goes on (SmolLM2-135M shape
 // 1.25 -> 0.97 ms a step, Qwen3-0.6B shape 1.66 -> 1.42).  The thread sleeps while there is nothing to pass on, and a few launches do not wake
 // it: waking takes longer than they do.  Two threads that wait for each other need two cores: a process that may use less launches
-// everything itself, and whoever waits longer than a launch takes lets others have its core.
+// everything itself, and whoever waits longer than a launch takes lets others have its core (SmolLM2-135M shape, 512 tokens and 16 steps on one
+// core: 24.7 ms, 392 with the thread and waits that keep the core; on two or more 18.7 to 20.4).
 #pragma once
 
 #include <hip/hip_runtime.h>
