@@ -223,7 +223,7 @@ struct Buffer : Pooled<Buffer> {
     RowStore *rs = nullptr;      // owned
     bool constant = false;       // the contents depend on constants only (iota, programs over such buffers)
     Buffer *successor = nullptr; // retained: the roomier buffer that blocks of this one migrate to on append
-    // Set by the product kernels that store a residual stream [rows <= 8, N]: per group of 4 columns and row
+    // Set by the product kernels that store a residual stream of two to eight rows [rows, N]: per group of 4 columns and row
     // the sum of squares of what was stored there, [side_blocks][side_rows] floats (4 for up to four rows, else 8).  An RMS norm over these rows that feeds
     // decode-time products needs no pass of its own then (see NormFuse).  Owned (pool memory).
     void *side = nullptr;
@@ -421,9 +421,9 @@ struct DeferredWrite {
 };
 
 // x / pow(sum(x*x) / n + eps, e) * gamma applied to the left operand while a decode-time product loads it:
-// the row sums come from the per-workgroup partial sums that the kernel which stored x left behind.
+// the row sums come from the per-workgroup partial sums that the kernel which stored x left behind; one row's the product works out.
 struct NormFuse {
-    const float *partials; // [blocks][4], [blocks][8] for more than four rows
+    const float *partials; // [blocks][4], [blocks][8] for more than four rows; one row: not used
     uint32_t blocks;
     const uint32_t *gamma; // [K]
     uint32_t n_bits, eps_bits, exp_bits;

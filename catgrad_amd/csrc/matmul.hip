@@ -42,6 +42,7 @@
 // reference's `matrixmultiply::sgemm`, which is why the contract for matmul is 1e-3
 // relative (ndarray.rs:750-816 makes no promise on order either).
 #include "gemm_args.hpp"
+#include "one_row.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -1026,10 +1027,8 @@ __device__ __forceinline__ uint32_t residual_sum(const MmResidual &r, const uint
 #ifndef CG_WIDE_UNROLL
 #define CG_WIDE_UNROLL 2
 #endif
-template <int MM, int COLS, bool SPLIT, bool RESIDUAL = false>
-__device__ __forceinline__ void skinny_kt_wide_body(const MmArgs &a, const uint32_t block_x, const uint32_t block_y,
-                                                    const MmResidual *res = nullptr) {
-    static_assert(!RESIDUAL || (COLS == 1 && !SPLIT), "the residual store is written for one column per wave");
+template <int MM, int COLS, bool SPLIT>
+__device__ __forceinline__ void skinny_kt_wide_body(const MmArgs &a, const uint32_t block_x, const uint32_t block_y) {
     constexpr int kWideUnroll = COLS == 1 ? CG_WIDE_UNROLL : 2;
     const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     const uint32_t group = SPLIT ? block_x : block_x * 4 + wave;
@@ -1039,18 +1038,6 @@ __device__ __forceinline__ void skinny_kt_wide_body(const MmArgs &a, const uint3
     batch_offsets(a, block_y, oa, ob);
     const uint32_t *A = a.A + oa;
     const uint32_t *B = a.B + ob;
-    uint32_t term[RESIDUAL ? MM : 1][4] = {};
-    if constexpr (RESIDUAL) {
-        // asked for before the walk along K, used after it
-        if (live && lane == 0) {
-#pragma unroll
-            for (int m = 0; m < MM; m++)
-#pragma unroll
-                for (int t = 0; t < 4; t++)
-                    if ((uint32_t)m < a.M && (uint32_t)t != res->slot && (uint32_t)t < res->nterms)
-                        term[m][t] = res->term[t][((uint64_t)block_y * a.M + m) * a.N + n0];
-        }
-    }
     float acc[COLS][MM];
 #pragma unroll
     for (int c = 0; c < COLS; c++)
@@ -1105,16 +1092,7 @@ __device__ __forceinline__ void skinny_kt_wide_body(const MmArgs &a, const uint3
         for (int c = 0; c < COLS; c++)
 #pragma unroll
             for (int m = 0; m < MM; m++)
-                if (n0 + c < a.N && (uint32_t)m < a.M) {
-                    uint32_t v = asu(acc[c][m]);
-                    if constexpr (RESIDUAL) {
-                        uint32_t t[4];
-#pragma unroll
-                        for (int i = 0; i < 4; i++) t[i] = (uint32_t)i == res->slot ? v : term[m][i];
-                        v = residual_sum(*res, t);
-                    }
-                    a.C[((uint64_t)block_y * a.M + m) * a.N + n0 + c] = v;
-                }
+                if (n0 + c < a.N && (uint32_t)m < a.M) a.C[((uint64_t)block_y * a.M + m) * a.N + n0 + c] = asu(acc[c][m]);
     }
 }
 
@@ -1123,16 +1101,11 @@ __global__ __launch_bounds__(kThreads) void skinny_kt_wide_kernel(const MmArgs a
     skinny_kt_wide_body<MM, COLS, SPLIT>(a, blockIdx.x, blockIdx.y);
 }
 
-template <int MM> __global__ __launch_bounds__(kThreads) void skinny_kt_wide_residual_kernel(const MmArgs a, const MmResidual r) {
-    skinny_kt_wide_body<MM, 1, false, true>(a, blockIdx.x, blockIdx.y, &r);
-}
-
 // Several products that share their left operand (the q / k / v projections of a decode step,
 // gate and up) in one launch: the workgroups are dealt to the problems in order.
 // Products too narrow for eight columns per workgroup still gain from the matrix-instruction kernel at four
 // columns per workgroup (one activation load per lane and trip instead of M) when its 2048-wide chunks of k are full.
-// With a single row it is 0.7 us behind the one-column-per-wave kernel at K = 2048 and level with it at K = 8192;
-// it is used all the same, because its residual store and its norm-applying loads save two launches per layer.
+// (One row: one_row.hip.)
 // Chunks of 2048 values of k when K is a multiple of that, of 1024 when of that (hidden sizes like 1024 or 3072); any
 // other K (a multiple of 4 above 256: hidden sizes like 576 or 1536) runs with a ragged last chunk, the waves of a
 // workgroup then interleaved every 64 values of k (xreg_lane_k) so that a short chunk still spreads over all four.
@@ -1173,11 +1146,6 @@ __device__ __forceinline__ uint32_t group_problem(const MmGroup &g, uint32_t &bl
     const uint32_t first = p == 0 ? g.first[0] : p == 1 ? g.first[1] : p == 2 ? g.first[2] : g.first[3];
     block_x = blockIdx.x - first;
     return p;
-}
-template <int MM> __global__ __launch_bounds__(kThreads) void skinny_kt_wide_group_kernel(const MmGroup g) {
-    uint32_t bx;
-    const uint32_t p = group_problem(g, bx);
-    skinny_kt_wide_body<MM, 1, false>(g.p[p], bx, 0);
 }
 
 // Skinny kernel on the 4x4x1 matrix instruction (16 independent 4x4 outer products per
@@ -1236,10 +1204,8 @@ template <int TRIPS, bool WHOLE, class F> __device__ __forceinline__ void xreg_c
 // every load leaves the compiler without a count of what is on its way, and it then waits for all of it before each of several groups.
 // The kernels below run for a few microseconds, most of them one trip to memory; around it nothing waits that need not: every load of
 // a chunk is on its way before the first wait, the sums over lanes stay out of LDS (four_sums), a norm's divisor is worked out
-// meanwhile, and the arguments come in two trips.  One row, us a launch with guarded loads, shuffles, the divisor at the end and
-// arguments field by field, and so: q, k and v with the rotary embedding 576 -> 960 7.3 and 5.2, 1024 -> 4096 9.0 and 6.7; gate and up
-// 576 -> 1536 7.4 and 5.9, 1024 -> 3072 8.5 and 7.8; the sums 576 -> 576 3.8 and 3.6, 2048 -> 1024 5.8 and 5.5.  Four rows: q, k and v
-// 2048 -> 3072 11.8 and 9.7, gate and up 2048 -> 8192 26.4 and 24.3.
+// meanwhile, and the arguments come in two trips.  Four rows, us a launch with guarded loads, shuffles, the divisor at the end and
+// arguments field by field, and so: q, k and v with the rotary embedding 2048 -> 3072 11.8 and 9.7, gate and up 2048 -> 8192 26.4 and 24.3.
 template <bool WHOLE, bool NT = false> __device__ __forceinline__ float4v xreg_at(const uint32_t *row, uint32_t k, uint32_t K) {
     const float4v *const p = reinterpret_cast<const float4v *>(row + (WHOLE ? k : min(k, K - 4)));
     if constexpr (NT) return __builtin_nontemporal_load(p);
@@ -2119,6 +2085,16 @@ static const void *native_ptr(const cg_tensor *t) {
     return static_cast<const char *>(t->buf->ptr) + t->offset * (int64_t)fmt_bytes(t->buf->fmt);
 }
 
+// One row: a kernel of its own (one_row.hip)
+static OneRowInput one_row_input(const MmArgs &a, const NormFuse *nf) {
+    OneRowInput in = {reinterpret_cast<const float *>(a.A), nullptr, a.K, 0, 0, 0};
+    if (nf) in = {in.x, reinterpret_cast<const float *>(nf->gamma), a.K, nf->n_bits, nf->eps_bits, nf->exp_bits};
+    return in;
+}
+static OneRowProduct one_row_product(const MmArgs &a) { // its row stored as it is
+    return {reinterpret_cast<const float *>(a.B), a.b_sn, a.N, 0, a.C, 0, nullptr, nullptr, a.N, 0};
+}
+
 int launch_matmul_group(cg_backend *be, const cg_tensor *x, const cg_tensor *const *ys, cg_tensor *const *outs, int n,
                         const NormFuse *nf) {
     if (int frc = flush_deferred(be)) return frc;
@@ -2138,9 +2114,13 @@ int launch_matmul_group(cg_backend *be, const cg_tensor *x, const cg_tensor *con
         all_wide = all_wide && a.N >= 8192;
         bytes += distinct_bytes(ys[i]) + distinct_bytes(outs[i]);
     }
+    if (takes_one_row(g.p[0].M, g.p[0].K)) {
+        OneRowGroup og = {one_row_input(g.p[0], nf), {}, (uint32_t)n};
+        for (int i = 0; i < n; i++) og.p[i] = one_row_product(g.p[i]);
+        ProfScope prof(be, CG_K_GEMM_SKINNY, bytes);
+        return launch_one_row_group(be, og);
+    }
     const bool xreg = !nf && all_wide && g.p[0].M <= 4;
-    const bool xreg1 = !xreg && xreg_narrow(g.p[0].M, g.p[0].K);
-    if (nf && !xreg1) return kDeclined;
     for (int i = 0; i < n && nf; i++)
         if (g.p[i].N >= 8192) return kDeclined; // a vocabulary-sized product: the kernel with more columns per wave, the norm on its own
     uint32_t blocks = 0;
@@ -2160,16 +2140,10 @@ int launch_matmul_group(cg_backend *be, const cg_tensor *x, const cg_tensor *con
         else if (nf && deep) launch(skinny_kt_mfma_xreg_group_norm_kernel<W, 4, 8>, g, *nf);
         else if (nf && eight) launch(skinny_kt_mfma_xreg_group_norm_kernel<W, 8, 4>, g, *nf);
         else if (nf) launch(skinny_kt_mfma_xreg_group_norm_kernel<W, 4, 4>, g, *nf);
-        else if (xreg1 && deep && eight) launch(skinny_kt_mfma_xreg_group_kernel<W, 8, 1, 8>, g);
-        else if (xreg1 && deep) launch(skinny_kt_mfma_xreg_group_kernel<W, 4, 1, 8>, g);
-        else if (xreg1 && eight) launch(skinny_kt_mfma_xreg_group_kernel<W, 8, 1, 4>, g);
-        else if (xreg1) launch(skinny_kt_mfma_xreg_group_kernel<W, 4, 1, 4>, g);
-        else if (g.p[0].M <= 1)
-            launch_kernel((skinny_kt_wide_group_kernel<1>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
-        else if (g.p[0].M <= 4)
-            launch_kernel((skinny_kt_wide_group_kernel<4>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
-        else
-            launch_kernel((skinny_kt_wide_group_kernel<8>), dim3(blocks), dim3(kThreads), 0, be->stream, g);
+        else if (deep && eight) launch(skinny_kt_mfma_xreg_group_kernel<W, 8, 1, 8>, g);
+        else if (deep) launch(skinny_kt_mfma_xreg_group_kernel<W, 4, 1, 8>, g);
+        else if (eight) launch(skinny_kt_mfma_xreg_group_kernel<W, 8, 1, 4>, g);
+        else launch(skinny_kt_mfma_xreg_group_kernel<W, 4, 1, 4>, g);
     });
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "grouped matmul launch");
@@ -2238,7 +2212,17 @@ int launch_matmul_group_rope(cg_backend *be, const cg_tensor *x, const cg_tensor
         }
     }
     auto launch = [&](auto kernel) { launch_kernel(kernel, dim3(blocks), dim3(kThreads), 0, be->stream, g, rg, nf ? *nf : none); };
-    xreg_either(g.p[0].K, xreg_trips(g.p[0].K), [&](auto whole) { // (the problems of a group share k)
+    if (takes_one_row(g.p[0].M, g.p[0].K)) {
+        OneRowGroup og = {one_row_input(g.p[0], nf), {}, (uint32_t)n};
+        for (int i = 0; i < n; i++) {
+            const RopeStore &st = rg.s[i];
+            og.p[i] = {reinterpret_cast<const float *>(g.p[i].B), g.p[i].b_sn, g.p[i].N, 0, st.dst, st.sh, st.cos, st.sin, st.hd, st.rope};
+        }
+        if (const int rc = launch_one_row_group(be, og)) {
+            if (tmp) be->pool.free(tmp, tmp_cls);
+            return rc;
+        }
+    } else xreg_either(g.p[0].K, xreg_trips(g.p[0].K), [&](auto whole) { // (the problems of a group share k)
         constexpr bool W = decltype(whole)::value;
         if (g.p[0].M > 4) {
             if (nf && wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 8, true, 8>);
@@ -2282,6 +2266,10 @@ int launch_matmul_gated(cg_backend *be, const cg_tensor *x, const cg_tensor *yg,
     if (ag.M > 4 && !nf) return kDeclined; // (more than four rows: a decode step's, whose norm comes along; others as a grouped product and the program)
     const bool short_chunks = xreg_trips(ag.K) == 4; // K a multiple of 1024 but not of 2048
     ProfScope prof(be, CG_K_GEMM_SKINNY, distinct_bytes(x) + distinct_bytes(yg) + distinct_bytes(yu) + distinct_bytes(out));
+    if (takes_one_row(ag.M, ag.K)) {
+        const OneRowGated g = {one_row_input(ag, nf), reinterpret_cast<const float *>(ag.B), reinterpret_cast<const float *>(au.B), ag.b_sn, ag.N, one, c};
+        return launch_one_row_gated(be, g);
+    }
     const dim3 ggrid((ag.N + 3) / 4);
     if (xreg_trips(ag.K) == 0) return kDeclined;
     const bool eight = ag.M > 4;
@@ -2341,6 +2329,12 @@ int launch_matmul_residual(cg_backend *be, const cg_tensor *x, const cg_tensor *
     r.order = (uint32_t)order;
     r.nterms = (uint32_t)nterms;
     r.partials = nullptr;
+    if (takes_one_row(a.M, a.K)) { // (its norm needs no sums that others left)
+        OneRowResidual o = {reinterpret_cast<const float *>(a.A), reinterpret_cast<const float *>(a.B), a.b_sn, a.N, a.K, {}, r.slot, r.order, r.nterms, a.C};
+        for (int t = 0; t < 4; t++) o.term[t] = r.term[t];
+        ProfScope prof(be, CG_K_GEMM_SKINNY, distinct_bytes(x) + distinct_bytes(y) + 4.0 * distinct_bytes(out));
+        return launch_one_row_residual(be, o);
+    }
     const uint32_t blocks = (uint32_t)((a.N + 3) / 4);
     if (keep_sums && out->offset == 0 && xreg_narrow(a.M, a.K) && !out->buf->side) {
         // the stored rows' sums of squares per workgroup, for an RMS norm that may follow (Buffer::side)
@@ -2366,7 +2360,7 @@ int launch_matmul_residual(cg_backend *be, const cg_tensor *x, const cg_tensor *
     else if (eight == 8) launch8(skinny_kt_mfma_eight_residual_kernel<4, 8>);
     else if (eight == 4 && rows8) launch8(skinny_kt_mfma_eight_residual_kernel<8, 4>);
     else if (eight == 4) launch8(skinny_kt_mfma_eight_residual_kernel<4, 4>);
-    else if (xreg_narrow(a.M, a.K)) {
+    else {
         const bool deep = xreg_trips(a.K) == 8;
         xreg_either(a.K, xreg_trips(a.K), [&](auto whole) {
             constexpr bool W = decltype(whole)::value;
@@ -2375,12 +2369,7 @@ int launch_matmul_residual(cg_backend *be, const cg_tensor *x, const cg_tensor *
             else if (rows8) launch(skinny_kt_mfma_xreg_residual_kernel<W, 8, 4>);
             else launch(skinny_kt_mfma_xreg_residual_kernel<W, 4, 4>);
         });
-    } else if (a.M <= 1)
-        launch_kernel((skinny_kt_wide_residual_kernel<1>), grid, dim3(kThreads), 0, be->stream, a, r);
-    else if (a.M <= 4)
-        launch_kernel((skinny_kt_wide_residual_kernel<4>), grid, dim3(kThreads), 0, be->stream, a, r);
-    else
-        launch_kernel((skinny_kt_wide_residual_kernel<8>), grid, dim3(kThreads), 0, be->stream, a, r);
+    }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? CG_OK : hip_fail(e, "matmul with residual launch");
 }
@@ -2770,7 +2759,10 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
         } else {
             // enough waves to cover 256 CUs several times over, else split K inside the block
             const int64_t cols = N * batch;
-            if (cols >= 16384) {
+            if (batch == 1 && cols >= 2048 && takes_one_row((uint32_t)M, (uint32_t)K)) {
+                const int orc = launch_one_row_group(be, {one_row_input(a, nullptr), {one_row_product(a)}, 1});
+                if (orc) return orc;
+            } else if (cols >= 16384) {
                 dim3 grid((uint32_t)((N + 15) / 16), (uint32_t)batch);
 #define CG_CALL(MMV) launch_kernel((skinny_kt_wide_kernel<MMV, 4, false>), grid, dim3(kThreads), 0, s, a);
                 CG_MM_SWITCH(CG_CALL)

@@ -160,7 +160,7 @@ Pending::~Pending() {
 }
 
 // Is x (still) the deferred program  h / pow(sum(h * h) / n + eps, e) * gamma  over the rows of a residual stream h
-// [1..8 rows, K] whose kernel left the partial sums of squares (Buffer::side)?  Then a decode-time product can apply
+// [1..8 rows, K] whose kernel left the partial sums of squares (Buffer::side; one row's products form them themselves)?  Then a decode-time product can apply
 // the norm while it loads h (K a multiple of 4 above 256) and the norm needs no launch.  Fills nf and the stand-in tensor
 // h (a borrowed view of the leaf's buffer: set h->buf to null before it goes out of scope).
 static bool norm_fuse_of(const cg_tensor *x, NormFuse *nf, cg_tensor *h) {
@@ -175,9 +175,8 @@ static bool norm_fuse_of(const cg_tensor *x, NormFuse *nf, cg_tensor *h) {
     const int64_t K = x->dims[r - 1], rows = K > 0 ? numel(x) / K : 0;
     if (K <= 256 || K % 4 != 0 || rows < 1 || rows > 8 || p->rowlen != K) return false;
     const LeafView &lh = p->leaf[0], &lg = p->leaf[4];
-    if (lh.uniform || lh.pw || lh.lazy || !lh.buf || !lh.buf->side || lh.offset != 0 || (int64_t)lh.buf->side_blocks * 4 != K ||
-        lh.buf->side_rows != (rows > 4 ? 8u : 4u))
-        return false;
+    if (lh.uniform || lh.pw || lh.lazy || !lh.buf || lh.offset != 0) return false;
+    if (rows > 1 && (!lh.buf->side || (int64_t)lh.buf->side_blocks * 4 != K || lh.buf->side_rows != (rows > 4 ? 8u : 4u))) return false;
     if (is_narrow_buf(lh.buf) || is_narrow_buf(lg.buf)) return false; // (the kernels read 32-bit words)
     if (!p->leaf[1].uniform || !p->leaf[2].uniform || !p->leaf[3].uniform) return false;
     if (lg.uniform || lg.pw || lg.lazy || !lg.buf || lg.offset % 4 != 0) return false;
