@@ -776,6 +776,7 @@ int launch_few_rows_linear(cg_backend *be, const ProductInput &in, uint32_t rows
     if (four_rows(in, rows, w) && !in.poly && in.k <= (w.fmt == kFmtBF16 ? 8192u : 4096u)) {
         const bool bf16 = w.fmt == kFmtBF16;
         ProfScope prof(be, CG_K_GEMM_SKINNY, (double)w.n * w.k * (bf16 ? 2.0 : 4.0) + 4.0 * rows * ((double)in.k + w.n));
+        if (rows == 1 && takes_block_one_row(in, w)) return launch_block_one_row(be, in, w, bias, scale, out);
         const uint32_t steps = (in.k + (bf16 ? 511 : 255)) / (bf16 ? 512 : 256); // of a workgroup of four waves
 #define CG_FOUR(BF)                                                                              \
     if (steps <= 1) launch_four_rows<BF, 1, 4>(be, in, rows, w, bias, scale, out);               \
@@ -828,6 +829,7 @@ int launch_few_rows_linear2(cg_backend *be, const ProductInput (&in)[2], uint32_
         bytes += (double)w[i].n * w[i].k * (bf16 ? 2.0 : 4.0) + 4.0 * rows * ((double)in[i].k + w[i].n);
     }
     ProfScope prof(be, CG_K_GEMM_SKINNY, bytes);
+    if (rows == 1 && takes_block_one_row(in[0], w[0]) && takes_block_one_row(in[1], w[1])) return launch_block_one_row2(be, in, w, out);
     const uint32_t steps = (in[0].k + (bf16 ? 511 : 255)) / (bf16 ? 512 : 256); // of a workgroup of four waves
 #define CG_FOUR(BF)                                                  \
     if (steps <= 1) launch_four_rows2<BF, 1, 4>(be, j, rows);        \
@@ -872,6 +874,7 @@ int launch_few_rows_residual(cg_backend *be, const Rows &x, const ResidualBranch
         double work = 8.0 * rows * width;
         for (int i = 0; i < n; i++) work += (double)br[i].w.n * br[i].w.k * (br[i].w.fmt == kFmtBF16 ? 2.0 : 4.0) + 4.0 * rows * ((double)br[i].in.k + width);
         ProfScope prof(be, CG_K_GEMM_SKINNY, work);
+        if (rows == 1 && takes_block_one_row_residual(br, n)) return launch_block_one_row_residual(be, x, br, n, width, out);
         const bool bf16 = br[0].w.fmt == kFmtBF16, two = width >= (uint32_t)be->compute_units * 8;
         if (two) bf16 ? four_rows_residual<true, 2>(be, x, br, n, rows, width, out) : four_rows_residual<false, 2>(be, x, br, n, rows, width, out);
         else bf16 ? four_rows_residual<true, 1>(be, x, br, n, rows, width, out) : four_rows_residual<false, 1>(be, x, br, n, rows, width, out);

@@ -52,6 +52,12 @@ struct ResidualBranch {
 // Whether launch_few_rows_residual takes these branches (one of them with 16-byte rows at most four rows deep, or LDS for all)
 bool takes_few_rows_residual(const ResidualBranch *br, int n, uint32_t rows);
 int launch_few_rows_residual(cg_backend *be, const Rows &x, const ResidualBranch *br, int n, uint32_t rows, uint32_t width, float *out);
+// The same of one row (block_one_row.hip), for operands that takes_* takes; called by the above.
+bool takes_block_one_row(const ProductInput &in, const Weight &w);
+int launch_block_one_row(cg_backend *be, const ProductInput &in, const Weight &w, const float *bias, float scale, float *out);
+int launch_block_one_row2(cg_backend *be, const ProductInput (&in)[2], const Weight (&w)[2], float *const (&out)[2]);
+bool takes_block_one_row_residual(const ResidualBranch *br, int n);
+int launch_block_one_row_residual(cg_backend *be, const Rows &x, const ResidualBranch *br, int n, uint32_t width, float *out);
 
 // y[rows, w.n] = x . w^T of dense bfloat16 patterns x [rows, w.k] on 128-wide tiles; kDeclined: operands it does not take.
 int launch_bf16_tiles(cg_backend *be, const void *x, uint32_t rows, const Weight &w, float *y);
