@@ -223,12 +223,6 @@ struct Buffer : Pooled<Buffer> {
     RowStore *rs = nullptr;      // owned
     bool constant = false;       // the contents depend on constants only (iota, programs over such buffers)
     Buffer *successor = nullptr; // retained: the roomier buffer that blocks of this one migrate to on append
-    // Set by the product kernels that store a residual stream of two to eight rows [rows, N]: per group of 4 columns and row
-    // the sum of squares of what was stored there, [side_blocks][side_rows] floats (4 for up to four rows, else 8).  An RMS norm over these rows that feeds
-    // decode-time products needs no pass of its own then (see NormFuse).  Owned (pool memory).
-    void *side = nullptr;
-    size_t side_cls = 0;
-    uint32_t side_blocks = 0, side_rows = 0;
     // Narrow copies of 2-D views of this buffer for the matrix instructions of its dtype (launch_matmul): [rows][k] of
     // 2-byte (f16 / bf16) or 1-byte (fp8) patterns, k contiguous, one entry per view (several slices of one weight buffer
     // each keep theirs; the oldest goes when the list is full).  A weight matrix is narrowed once and the copy kept while
@@ -421,10 +415,8 @@ struct DeferredWrite {
 };
 
 // x / pow(sum(x*x) / n + eps, e) * gamma applied to the left operand while a decode-time product loads it:
-// the row sums come from the per-workgroup partial sums that the kernel which stored x left behind; one row's the product works out.
+// (the product's kernel forms the rows' sums itself).
 struct NormFuse {
-    const float *partials; // [blocks][4], [blocks][8] for more than four rows; one row: not used
-    uint32_t blocks;
     const uint32_t *gamma; // [K]
     uint32_t n_bits, eps_bits, exp_bits;
 };
@@ -635,10 +627,9 @@ int launch_fused_group(cg_backend *be, const cg_tensor *const *outs, const Pendi
 // Writes that were put off so that they can share a launch (see DeferredWrite); every function
 // that launches a kernel or copies device memory calls this first.
 int flush_deferred(cg_backend *be, const Pending *also = nullptr);
-// nterms: 2 (out = t0 + t1) or 4.  out is a contiguous view (any offset).  keep_sums: out is the whole of its buffer, which
-// may then receive the partial sums of squares of the stored rows (Buffer::side).
+// nterms: 2 (out = t0 + t1) or 4.  out is a contiguous view (any offset).
 int launch_matmul_residual(cg_backend *be, const cg_tensor *x, const cg_tensor *y, const uint32_t *const *terms, int nterms,
-                           int slot, int order, cg_tensor *out, bool keep_sums);
+                           int slot, int order, cg_tensor *out);
 int launch_matmul_group(cg_backend *be, const cg_tensor *x, const cg_tensor *const *ys, cg_tensor *const *outs, int n,
                         const NormFuse *nf = nullptr);
 // Where the columns of a decode-time product go when the rotary embedding and the write into a KV cache (or into q's own

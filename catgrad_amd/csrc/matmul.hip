@@ -27,13 +27,8 @@
 //                      skinny_kt_wide / _narrow: a wave per output column (or per 4 columns, or a
 //                      column per 16/32 lanes for short K), 16-byte loads along K, wave shuffle
 //                      reduction;
-//                      skinny_kt_mfma_xreg_*: M <= 8 on the 4x4x1 matrix instruction with the
-//                      activations held in registers, in the variants the decode step needs:
-//                      _group (products that share their left operand in one launch), _group_rope
-//                      (the same with the rotary embedding and the KV-cache row writes in the
-//                      store), _gated / _cols_gated (two products and SiLU(g)*u in one launch),
-//                      _residual (the residual adds in the store, row sums of squares left
-//                      behind), _norm (an RMS norm applied to the left operand while it loads).
+//                      skinny_kt_mfma_xreg: batches of them on the 4x4x1 matrix instruction with the
+//                      activations held in registers; without a batch: skinny.hpp.
 //   skinny_nn_kernel   M <= 8 with N-contiguous B rows (p.V of a decode step), split over K
 //                      with a second pass that adds the partial sums.
 //   simple_gemm_kernel u32 (wrapping) and any shape the others decline.
@@ -42,7 +37,7 @@
 // reference's `matrixmultiply::sgemm`, which is why the contract for matmul is 1e-3
 // relative (ndarray.rs:750-816 makes no promise on order either).
 #include "gemm_args.hpp"
-#include "one_row.hpp"
+#include "skinny.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -1007,23 +1002,6 @@ template <int MM> __global__ __launch_bounds__(kThreads) void skinny_kt_kernel(c
 // 16-byte loads (COLS weight loads + M activation loads in flight per lane per trip; the
 // activation rows stay in L1/L2).  SPLIT: the four waves of the block share the columns
 // and split K, for shapes with too few columns to fill the chip.
-// A sum of four terms one of which is the product: out = (t0 + (t1 + t2)) + t3 (order 0) or
-// t0 + ((t1 + t2) + t3) (order 1), term[slot] being x.B^T and the others dense tensors of the
-// output's shape.  The residual adds of a decoder layer run in the store of the o / down projection.
-struct MmResidual {
-    const uint32_t *term[4];
-    uint32_t slot, order;
-    uint32_t nterms;  // 4, or 2: out = t0 + t1
-    float *partials;  // null, or [groups of four columns][4 or 8 rows]: per row the sum of squares of the four columns stored
-};
-// the sum, given all its terms
-__device__ __forceinline__ uint32_t residual_sum(const MmResidual &r, const uint32_t (&t)[4]) {
-    if (r.nterms == 2) return apply<kAdd, true>(t[0], t[1], 0, nullptr);
-    const uint32_t inner = apply<kAdd, true>(t[1], t[2], 0, nullptr);
-    return r.order == 0 ? apply<kAdd, true>(apply<kAdd, true>(t[0], inner, 0, nullptr), t[3], 0, nullptr)
-                        : apply<kAdd, true>(t[0], apply<kAdd, true>(inner, t[3], 0, nullptr), 0, nullptr);
-}
-
 #ifndef CG_WIDE_UNROLL
 #define CG_WIDE_UNROLL 2
 #endif
@@ -1101,18 +1079,13 @@ __global__ __launch_bounds__(kThreads) void skinny_kt_wide_kernel(const MmArgs a
     skinny_kt_wide_body<MM, COLS, SPLIT>(a, blockIdx.x, blockIdx.y);
 }
 
-// Several products that share their left operand (the q / k / v projections of a decode step,
-// gate and up) in one launch: the workgroups are dealt to the problems in order.
-// Products too narrow for eight columns per workgroup still gain from the matrix-instruction kernel at four
-// columns per workgroup (one activation load per lane and trip instead of M) when its 2048-wide chunks of k are full.
-// (One row: one_row.hip.)
 // Chunks of 2048 values of k when K is a multiple of that, of 1024 when of that (hidden sizes like 1024 or 3072); any
 // other K (a multiple of 4 above 256: hidden sizes like 576 or 1536) runs with a ragged last chunk, the waves of a
 // workgroup then interleaved every 64 values of k (xreg_lane_k) so that a short chunk still spreads over all four.
 static inline int xreg_trips(uint32_t K) {
     return K % 2048 == 0 ? 8 : K % 1024 == 0 ? 4 : (K % 4 == 0 && K > 256) ? (K > 1024 ? 8 : 4) : 0;
 }
-// Column groups per workgroup of the one-chunk gated kernel: as many as leave about two workgroups per compute unit
+// Column groups per workgroup of the packed kernel: as many as leave about two workgroups per compute unit
 // (env CG_XREG_ITERS=n forces n, for measurements).
 static inline uint32_t xreg_cols_iters(uint64_t groups) {
     static const int forced = [] {
@@ -1123,31 +1096,8 @@ static inline uint32_t xreg_cols_iters(uint64_t groups) {
     const uint64_t it = groups / 512;
     return (uint32_t)(it < 1 ? 1 : it > 4 ? 4 : it);
 }
-// Five to eight rows run on the same kernels with a second group of four rows: two activation loads and eight matrix
-// instructions per weight load instead of one and four.  Against the vector-unit kernels without the norms, gates and cache rows in
-// their loads and stores (up to 14 launches a layer instead of 5): Llama-3.2-1B shape, six sequences 2.44 -> 1.67 ms a step; SmolLM2-135M
-// shape, eight 1.93 -> 1.27; Qwen3-0.6B shape, five 2.8 -> 2.2.
-// Products without any of that: weights from memory, as a model's are, in us on the vector-unit kernels and here: 5 x 3072 x 8192 34 and 29, 8 x
-// 4096 x 4096 31 and 28.6, two of them in a launch 60 and 46, 8 x 2048 x 8192 31 and 24.  Weights that the last-level cache still holds from the call
-// before are faster on those: 5 x 3072 x 8192 22 and 26, 8 x 4096 x 4096 23 and 28, 8 x 2048 x 8192 22 and 23.
+// Five to eight rows: a second group of four.
 static inline bool xreg_narrow(uint32_t M, uint32_t K) { return M >= 1 && M <= 8 && xreg_trips(K) != 0; }
-constexpr int kMaxGroup = 4;
-struct MmGroup {
-    MmArgs p[kMaxGroup];
-    uint32_t first[kMaxGroup + 1]; // first workgroup of each problem; first[n] = grid size
-    uint32_t n;
-};
-__device__ __forceinline__ uint32_t group_problem(const MmGroup &g, uint32_t &block_x) {
-    // every slot of the prefix table is compared (the problems are in increasing order of their first workgroup), so the
-    // table is read from the argument block at once instead of one dependent scalar load per problem
-    uint32_t p = 0;
-#pragma unroll
-    for (int i = 1; i < kMaxGroup; i++) p += (uint32_t)i < g.n && blockIdx.x >= g.first[i] ? 1u : 0u;
-    const uint32_t first = p == 0 ? g.first[0] : p == 1 ? g.first[1] : p == 2 ? g.first[2] : g.first[3];
-    block_x = blockIdx.x - first;
-    return p;
-}
-
 // Skinny kernel on the 4x4x1 matrix instruction (16 independent 4x4 outer products per
 // issue): lane (b, j) = (lane / 4, lane % 4) feeds weight W[n0 + j][k] and activation
 // X[j][k] for the k values of block b, so one 16-byte weight load per lane drives four
@@ -1158,15 +1108,6 @@ __device__ __forceinline__ uint32_t group_problem(const MmGroup &g, uint32_t &bl
 // every 256 bytes), keep their share of the chunk's activations in registers (8 x 16 bytes
 // per lane and row group) and reuse it for CG groups of four columns, so the activation rows
 // are fetched once per 4 * CG columns.
-// RESIDUAL (CG = 1): the store adds the other terms of a four-term sum, as skinny_kt_wide_residual_kernel does.
-// GATED (CG = 2): the two column groups are the same four columns of two weight matrices, a.B and
-// `second` (same shape and strides), and the block writes g * (1 / (one + exp(-g))) * u for
-// g = x.B^T, u = x.second^T: the SiLU-gated pair of an MLP block without writing g and u.
-// pow(sum / n + eps, e): the divisor of an RMS norm from its row's sum of squares, in the program's own ops
-__device__ __forceinline__ uint32_t norm_divisor(const NormFuse &nf, float sum) {
-    const uint32_t mean = apply<kDiv, true>(asu(sum), nf.n_bits, 0, nullptr);
-    return apply<kPow, true>(apply<kAdd, true>(mean, nf.eps_bits, 0, nullptr), nf.exp_bits, 0, nullptr);
-}
 // Where a lane's k values lie inside a chunk of TRIPS * 256: trip t covers k0 + kb + ks * t .. + 3.  Whole chunks: a wave
 // takes a quarter of the chunk in a row (2 KiB in a row of each weight row: measured 12 % faster on the gate / up pair than
 // interleaving the waves every 256 bytes).  A ragged last chunk: the waves interleaved every 64 values of k, so that what
@@ -1218,35 +1159,17 @@ template <bool WHOLE> __device__ __forceinline__ float4v xreg_within(float4v v, 
     }
     return v;
 }
-// This thread's share of a norm's partial sums, [blocks][MM] floats: the first 2 * MM rounds, clamped likewise, and their sum with the rest
-template <int MM> __device__ __forceinline__ void xreg_ask_sums(const NormFuse &nf, float (&pv)[2 * MM]) {
-#pragma unroll
-    for (int u = 0; u < 2 * MM; u++) pv[u] = nf.partials[min(threadIdx.x + u * kThreads, nf.blocks * MM - 1)];
-}
-template <int MM> __device__ __forceinline__ float xreg_sums(const NormFuse &nf, const float (&pv)[2 * MM]) {
-    float s = 0.0f;
-#pragma unroll
-    for (int u = 0; u < 2 * MM; u++) s += threadIdx.x + u * kThreads < nf.blocks * MM ? pv[u] : 0.0f;
-    for (uint32_t i = threadIdx.x + 2 * MM * kThreads; i < nf.blocks * MM; i += kThreads) s += nf.partials[i];
-    return s;
-}
-template <bool WHOLE, int MM, int CG, bool GATED, bool RESIDUAL, bool NORM, int TRIPS>
-__device__ __forceinline__ void skinny_kt_mfma_xreg_body(const MmArgs &a, const uint32_t block_x, const uint32_t block_y, const uint32_t *second = nullptr,
-                                                         const uint32_t one = 0, const MmResidual *res = nullptr, const NormFuse *nf = nullptr) {
+template <bool WHOLE, int MM, int CG, int TRIPS> __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_kernel(const MmArgs a) {
     static_assert(MM == 4 || MM == 8, "one or two groups of four rows");
-    static_assert(!GATED || CG == 2, "a gated pair is two column groups");
-    static_assert(!(GATED && RESIDUAL), "one epilogue at a time");
     constexpr int G = MM / 4;
     const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     const uint32_t j = lane % 4, b = lane / 4;
-    const uint32_t n0 = block_x * (GATED ? 4 : 4 * CG);
+    const uint32_t n0 = blockIdx.x * (4 * CG);
     int64_t oa, ob;
-    batch_offsets(a, block_y, oa, ob);
+    batch_offsets(a, blockIdx.y, oa, ob);
     const uint32_t *wrow[CG];
 #pragma unroll
-    for (int c = 0; c < CG; c++)
-        wrow[c] = GATED ? (c == 0 ? a.B : second) + ob + (int64_t)min(n0 + j, a.N - 1) * a.b_sn
-                        : a.B + ob + (int64_t)min(n0 + 4 * c + j, a.N - 1) * a.b_sn;
+    for (int c = 0; c < CG; c++) wrow[c] = a.B + ob + (int64_t)min(n0 + 4 * c + j, a.N - 1) * a.b_sn;
     const uint32_t *xrow[G];
 #pragma unroll
     for (int g = 0; g < G; g++) xrow[g] = a.A + oa + (int64_t)min((uint32_t)(4 * g) + j, a.M - 1) * a.a_sm;
@@ -1255,23 +1178,6 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body(const MmArgs &a, const 
     for (int c = 0; c < CG; c++)
 #pragma unroll
         for (int g = 0; g < G; g++) acc[c][g] = (float4v){0.f, 0.f, 0.f, 0.f};
-    // the sum's other terms for the value this thread will store: asked for before the walk along K
-    uint32_t term[4] = {};
-    if constexpr (RESIDUAL) {
-        const uint32_t c = threadIdx.x / (MM * 4) % CG, m = min(threadIdx.x / 4 % MM, a.M - 1), col = min(n0 + 4 * c + threadIdx.x % 4, a.N - 1);
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-            if ((uint32_t)t != res->slot && (uint32_t)t < res->nterms) term[t] = res->term[t][((uint64_t)block_y * a.M + m) * a.N + col];
-    }
-    // NORM: the products are taken of x * gamma and divided by d_m = pow(sum(x[m]^2) / n + eps, e) where they are stored:
-    // (x / d * gamma) . w = ((x * gamma) . w) / d.  The row sums are put together from the partial sums that the kernel
-    // which stored x left (always in the same order); thread t takes entries t, t + 256, ... of [blocks][MM], all of row
-    // t % MM.  They are asked for in front of all else, and the divisor (a power, in a few hundred instructions that nothing hides
-    // at a kernel's end) is worked out while the first weights are on their way.
-    __shared__ float nsum[4][MM];
-    uint32_t divisor = 0;
-    float pv[2 * MM];
-    if constexpr (NORM) xreg_ask_sums<MM>(*nf, pv);
     // of every chunk of TRIPS * 256 values of k (2048 or 1024) a wave takes a quarter in a row (TRIPS trips of 64)
     uint32_t kb, ks;
     xreg_lane_k<TRIPS, WHOLE>(wave, b, kb, ks);
@@ -1280,314 +1186,15 @@ __device__ __forceinline__ void skinny_kt_mfma_xreg_body(const MmArgs &a, const 
         constexpr int T = decltype(trips)::value;
         float4v xr[G][T];
 #pragma unroll
-        for (int t = 0; t < T; t++) {
-            const uint32_t k = k0 + kb + ks * t;
-#pragma unroll
-            for (int g = 0; g < G; g++) xr[g][t] = xreg_at<WHOLE>(xrow[g], k, a.K);
-        }
-        float4v gm[NORM ? T : 1]; // asked for with the activations, multiplied in once the first weights are on their way
-        if constexpr (NORM) {
-#pragma unroll
-            for (int t = 0; t < T; t++) {
-                const uint32_t k = k0 + kb + ks * t;
-                gm[t] = xreg_at<WHOLE>(nf->gamma, k, a.K);
-            }
-        }
-        float4v ws[CG][T];
-        auto ask = [&](int c) {
-#pragma unroll
-            for (int t = 0; t < T; t++) ws[c][t] = xreg_at<WHOLE>(wrow[c], k0 + kb + ks * t, a.K);
-        };
-        if constexpr (NORM) { // all in front of the wait for the partial sums
-#pragma unroll
-            for (int c = 0; c < CG; c++) ask(c);
-        }
-#pragma unroll
-        for (int c = 0; c < CG; c++) {
-            float4v (&w)[T] = ws[c];
-            if constexpr (!NORM) ask(c);
-            if constexpr (!WHOLE || NORM) __builtin_amdgcn_sched_barrier(0); // (what follows stays behind all of the loads)
-            if constexpr (NORM) {
-                if (c == 0 && k0 == 0) { // (the same for every thread)
-                    const float s = wave_add<MM>(xreg_sums<MM>(*nf, pv));
-                    if (lane < MM) nsum[wave][lane] = s;
-                    __syncthreads();
-                    if (threadIdx.x < MM * 4 * (GATED ? 1 : CG)) divisor = norm_divisor(*nf, (nsum[0][threadIdx.x / 4 % MM] + nsum[1][threadIdx.x / 4 % MM]) + (nsum[2][threadIdx.x / 4 % MM] + nsum[3][threadIdx.x / 4 % MM]));
-                }
-            }
-            if constexpr (NORM) {
-                if (c == 0) {
-#pragma unroll
-                    for (int t = 0; t < T; t++)
-#pragma unroll
-                        for (int g = 0; g < G; g++)
-#pragma unroll
-                            for (int e = 0; e < 4; e++) xr[g][t][e] = asf(apply<kMul, true>(asu(xr[g][t][e]), asu(gm[t][e]), 0, nullptr));
-                }
-            }
-            if constexpr (!WHOLE) {
-#pragma unroll
-                for (int t = 0; t < T; t++) {
-                    w[t] = xreg_within<WHOLE>(w[t], k0 + kb + ks * t, a.K);
-#pragma unroll
-                    for (int g = 0; g < G; g++)
-                        if (c == 0) xr[g][t] = xreg_within<WHOLE>(xr[g][t], k0 + kb + ks * t, a.K);
-                }
-            }
-#pragma unroll
-            for (int t = 0; t < T; t++)
-#pragma unroll
-                for (int g = 0; g < G; g++) {
-                    acc[c][g] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[g][t][0], w[t][0], acc[c][g], 0, 0, 0);
-                    acc[c][g] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[g][t][1], w[t][1], acc[c][g], 0, 0, 0);
-                    acc[c][g] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[g][t][2], w[t][2], acc[c][g], 0, 0, 0);
-                    acc[c][g] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[g][t][3], w[t][3], acc[c][g], 0, 0, 0);
-                }
-        }
-    };
-    for (; k0 < a.K; k0 += TRIPS * 256) xreg_chunk<TRIPS, WHOLE>(a.K - k0, chunk);
-    __shared__ float part[4][CG * MM * 4];
-#pragma unroll
-    for (int c = 0; c < CG; c++)
-#pragma unroll
-        for (int g = 0; g < G; g++) {
-            const float v = four_sums(acc[c][g][0], acc[c][g][1], acc[c][g][2], acc[c][g][3]); // of row g * 4 + b / 4
-            if (b % 4 == 0) part[wave][(c * MM + 4 * g) * 4 + b + j] = v;
-        }
-    __syncthreads();
-    if constexpr (GATED) {
-        if (threadIdx.x < MM * 4) {
-            const uint32_t t = threadIdx.x, u_at = MM * 4 + t, m = t / 4, col = n0 + t % 4;
-            uint32_t gv = asu((part[0][t] + part[1][t]) + (part[2][t] + part[3][t]));
-            uint32_t uv = asu((part[0][u_at] + part[1][u_at]) + (part[2][u_at] + part[3][u_at]));
-            if constexpr (NORM) {
-                gv = apply<kDiv, true>(gv, divisor, 0, nullptr);
-                uv = apply<kDiv, true>(uv, divisor, 0, nullptr);
-            }
-            // the ops of the deferred program, in its order
-            const uint32_t e = apply<kExp, true>(apply<kNeg, true>(gv, 0, 0, nullptr), 0, 0, nullptr);
-            const uint32_t sg = apply<kDiv, true>(one, apply<kAdd, true>(one, e, 0, nullptr), 0, nullptr);
-            const uint32_t r = apply<kMul, true>(apply<kMul, true>(gv, sg, 0, nullptr), uv, 0, nullptr);
-            if (col < a.N && m < a.M) a.C[((uint64_t)block_y * a.M + m) * a.N + col] = r;
-        }
-    } else if (threadIdx.x < CG * MM * 4) {
-        const uint32_t c = threadIdx.x / (MM * 4), m = threadIdx.x / 4 % MM, col = n0 + 4 * c + threadIdx.x % 4;
-        uint32_t v = asu((part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]));
-        if constexpr (NORM) v = apply<kDiv, true>(v, divisor, 0, nullptr);
-        if constexpr (RESIDUAL) {
-#pragma unroll
-            for (int t = 0; t < 4; t++) term[t] = (uint32_t)t == res->slot ? v : term[t];
-            v = residual_sum(*res, term);
-        }
-        const bool stored = col < a.N && m < a.M;
-        if (stored) a.C[((uint64_t)block_y * a.M + m) * a.N + col] = v;
-        if constexpr (RESIDUAL) {
-            // threads 0 .. 4 MM - 1 = (row m, column n0 + t % 4): the row's sum of squares over the block's four columns
-            if (res->partials) {
-                float q = stored ? asf(v) * asf(v) : 0.0f;
-                q += asf(row_rotated<0xB1>(asu(q))); // (of the lane 1 away, then 2)
-                q += asf(row_rotated<0x4E>(asu(q)));
-                if (threadIdx.x % 4 == 0) res->partials[(uint64_t)block_x * MM + m] = q;
-            }
-        }
-    }
-}
-template <bool WHOLE, int MM, int CG, int TRIPS> __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_kernel(const MmArgs a) {
-    skinny_kt_mfma_xreg_body<WHOLE, MM, CG, false, false, false, TRIPS>(a, blockIdx.x, blockIdx.y);
-}
-template <bool WHOLE, int MM, int TRIPS>
-__global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_gated_kernel(const MmArgs a, const uint32_t *second, uint32_t one) {
-    skinny_kt_mfma_xreg_body<WHOLE, MM, 2, true, false, false, TRIPS>(a, blockIdx.x, blockIdx.y, second, one);
-}
-template <bool WHOLE, int MM, int TRIPS>
-__global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_residual_kernel(const MmArgs a, const MmResidual r) {
-    skinny_kt_mfma_xreg_body<WHOLE, MM, 1, false, true, false, TRIPS>(a, blockIdx.x, blockIdx.y, nullptr, 0, &r);
-}
-// The same sum with residual terms for up to four rows, eight columns and all of K by eight waves: an eighth of a chunk of K each,
-// every load of a chunk asked for before the first product.  The kernel above fetches as many bytes of activations as of weights
-// (four columns per workgroup), and a compute unit's path to L2 bounds it; here the activations are half of the weights' bytes.
-// 4 x 8192 x 2048 (64 MiB of weights): 17.2 us above, 15.9 here; 4 x 2048 x 2048: 6.5 and 6.2.  With an arg-max of the sum behind
-// both: 4 x 4096 x 2048 24.8 and 24.4, 4 x 6144 x 2048 28.4 and 27.9, 4 x 16384 x 2048 45.8 and 45.4; from 3072 columns on
-// equal within 1 %.
-constexpr int kEightThreads = 512;
-template <int MM, int TRIPS>
-__global__ __launch_bounds__(kEightThreads, 2) void skinny_kt_mfma_eight_residual_kernel(const MmArgs a, const MmResidual res) {
-    const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 4, b = lane / 4;
-    const uint32_t n0 = blockIdx.x * 8;
-    const uint32_t *const w0 = a.B + (int64_t)min(n0 + j, a.N - 1) * a.b_sn, *const w1 = a.B + (int64_t)min(n0 + 4 + j, a.N - 1) * a.b_sn;
-    constexpr int G = MM / 4, kOut = 8 * MM; // row groups; values of the workgroup's result
-    const uint32_t *x[G];
-#pragma unroll
-    for (int g = 0; g < G; g++) x[g] = a.A + (int64_t)min((uint32_t)(4 * g) + j, a.M - 1) * a.a_sm;
-    // the sum's other terms for the value this thread will store
-    const uint32_t tc = threadIdx.x / (4 * MM), tm = threadIdx.x / 4 % MM, tcol = n0 + 4 * tc + threadIdx.x % 4;
-    const bool stored = threadIdx.x < kOut && tcol < a.N && tm < a.M;
-    uint32_t term[4] = {};
-    const uint64_t term_at = (uint64_t)min(tm, a.M - 1) * a.N + min(tcol, a.N - 1);
-#pragma unroll
-    for (int t = 0; t < 4; t++)
-        if ((uint32_t)t != res.slot && (uint32_t)t < res.nterms) term[t] = res.term[t][term_at];
-    float4v acc[2][G] = {};
-    for (uint32_t k0 = wave * (TRIPS * 64) + b * 4; k0 < a.K; k0 += TRIPS * kEightThreads) { // (K: whole chunks)
-        float4v xr[G][TRIPS], wr[2][TRIPS];
-#pragma unroll
-        for (int t = 0; t < TRIPS; t++) {
-            wr[0][t] = *reinterpret_cast<const float4v *>(w0 + k0 + 64 * t);
-            wr[1][t] = *reinterpret_cast<const float4v *>(w1 + k0 + 64 * t);
-#pragma unroll
-            for (int g = 0; g < G; g++) xr[g][t] = *reinterpret_cast<const float4v *>(x[g] + k0 + 64 * t);
-        }
-        __builtin_amdgcn_sched_barrier(0); // (or the compiler asks for a few at a time)
-#pragma unroll
-        for (int t = 0; t < TRIPS; t++)
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-#pragma unroll
-                for (int c = 0; c < 2; c++)
-#pragma unroll
-                    for (int g = 0; g < G; g++) acc[c][g] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[g][t][e], wr[c][t][e], acc[c][g], 0, 0, 0);
-    }
-    __shared__ float part[8][kOut];
-#pragma unroll
-    for (int c = 0; c < 2; c++)
-#pragma unroll
-        for (int g = 0; g < G; g++) {
-            const float v = four_sums(acc[c][g][0], acc[c][g][1], acc[c][g][2], acc[c][g][3]); // of row g * 4 + b / 4
-            if (b % 4 == 0) part[wave][(c * MM + 4 * g) * 4 + b + j] = v;
-        }
-    __syncthreads();
-    if (threadIdx.x >= kOut) return;
-    const uint32_t t = threadIdx.x;
-    uint32_t v = asu(((part[0][t] + part[1][t]) + (part[2][t] + part[3][t])) + ((part[4][t] + part[5][t]) + (part[6][t] + part[7][t])));
-#pragma unroll
-    for (int k = 0; k < 4; k++) term[k] = (uint32_t)k == res.slot ? v : term[k];
-    v = residual_sum(res, term);
-    if (stored) a.C[(uint64_t)tm * a.N + tcol] = v;
-    if (res.partials) { // the rows' sums of squares over four columns each, as above
-        float q = stored ? asf(v) * asf(v) : 0.0f;
-        q += asf(row_rotated<0xB1>(asu(q)));
-        q += asf(row_rotated<0x4E>(asu(q)));
-        if (t % 4 == 0 && n0 + 4 * tc < a.N) res.partials[((uint64_t)blockIdx.x * 2 + tc) * MM + tm] = q;
-    }
-}
-// trips of 64 values of k per wave and chunk; 0: K is not whole chunks, or there are too few columns for a workgroup per compute unit
-static inline int eight_trips(const cg_backend *be, uint32_t M, uint32_t N, uint32_t K) {
-    if (M > 8 || (uint64_t)N < 8ull * be->compute_units) return 0;
-    return K % 8192 == 0 && M <= 4 ? 16 : K % 4096 == 0 ? 8 : K % 2048 == 0 ? 4 : 0; // (16 trips of eight rows: more registers than there are)
-}
-// the gated pair with the RMS norm of the left operand applied on load
-template <bool WHOLE, int MM, int TRIPS>
-__global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_gated_norm_kernel(const MmArgs a, const uint32_t *second, uint32_t one,
-                                                                                  const NormFuse nf) {
-    skinny_kt_mfma_xreg_body<WHOLE, MM, 2, true, false, true, TRIPS>(a, blockIdx.x, blockIdx.y, second, one, nullptr, &nf);
-}
-template <bool WHOLE, int MM, int CG, int TRIPS> __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_group_kernel(const MmGroup g) {
-    uint32_t bx;
-    const uint32_t p = group_problem(g, bx);
-    skinny_kt_mfma_xreg_body<WHOLE, MM, CG, false, false, false, TRIPS>(g.p[p], bx, 0);
-}
-template <bool WHOLE, int MM, int TRIPS>
-__global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_group_norm_kernel(const MmGroup g, const NormFuse nf) {
-    uint32_t bx;
-    const uint32_t p = group_problem(g, bx);
-    skinny_kt_mfma_xreg_body<WHOLE, MM, 1, false, false, true, TRIPS>(g.p[p], bx, 0, nullptr, 0, nullptr, &nf);
-}
-
-// The grouped products of an attention block's decode step (q, k, v: a few rows, the same left operand) with the
-// rotary embedding and the move into the KV cache done where they are stored: a workgroup owns two groups of four
-// columns half a head apart (the pair the embedding mixes; next to each other for a product stored as it is) and
-// writes column n = head * hd + d of row m to dst[m * sb + head * sh + d] (see RopeStore).  The embedding's ops are
-// those of the deferred program cos * x + sin * concat(-x2, x1), in its order.  M <= MM, K a multiple of TRIPS * 256,
-// N a multiple of hd (of 8 without the embedding).
-struct RopeGroup {
-    RopeStore s[kMaxGroup];
-};
-template <bool WHOLE, int MM, bool NORM, int TRIPS>
-__global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_group_rope_kernel(const MmGroup g, const RopeGroup rg, const NormFuse nf) {
-    __shared__ float nsum[4][MM];
-    uint32_t divisor = 0;
-    float pv[2 * MM];
-    if constexpr (NORM) xreg_ask_sums<MM>(nf, pv); // (the norm as in skinny_kt_mfma_xreg_body)
-    uint32_t bx;
-    const uint32_t p = group_problem(g, bx);
-    // (everything that the problem's number leads to asked for at once, not field by field on the way)
-    struct {
-        const uint32_t *A, *B;
-        uint32_t M, N, K;
-        int64_t a_sm, b_sn;
-    } a = {g.p[p].A, g.p[p].B, g.p[p].M, g.p[p].N, g.p[p].K, g.p[p].a_sm, g.p[p].b_sn};
-    struct {
-        uint32_t *dst;
-        int64_t sb, sh;
-        const uint32_t *cos, *sin;
-        uint32_t hd, rope;
-    } rs = {rg.s[p].dst, rg.s[p].sb, rg.s[p].sh, rg.s[p].cos, rg.s[p].sin, rg.s[p].hd, rg.s[p].rope};
-    asm volatile("" : "+s"(a.M), "+s"(a.N), "+s"(a.K), "+s"(a.a_sm), "+s"(a.b_sn), "+s"(rs.sb), "+s"(rs.sh), "+s"(rs.hd), "+s"(rs.rope)
-                 : "s"(a.A), "s"(a.B), "s"(rs.dst), "s"(rs.cos), "s"(rs.sin));
-    if constexpr (NORM) asm volatile("" ::"s"(nf.gamma), "s"(nf.n_bits), "s"(nf.eps_bits), "s"(nf.exp_bits));
-    const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const uint32_t j = lane % 4, b = lane / 4;
-    const uint32_t span = rs.rope ? rs.hd : 8, per = span / 8;
-    const uint32_t n0 = bx / per * span + bx % per * 4;
-    const uint32_t nc[2] = {n0, n0 + span / 2};
-    const uint32_t *wrow[2];
-#pragma unroll
-    for (int c = 0; c < 2; c++) wrow[c] = a.B + (int64_t)min(nc[c] + j, a.N - 1) * a.b_sn;
-    constexpr int G = MM / 4, kOut = 8 * MM; // row groups; values of the workgroup's result: at most a wave's lanes
-    const uint32_t *xrow[G];
-#pragma unroll
-    for (int g = 0; g < G; g++) xrow[g] = a.A + (int64_t)min((uint32_t)(4 * g) + j, a.M - 1) * a.a_sm;
-    float4v acc[2][G] = {};
-    // the embedding's factors for the value this thread will store: asked for before the walk along K
-    uint32_t cs = 0, sn = 0;
-    if (rs.rope && threadIdx.x < kOut) {
-        const uint32_t d = (nc[threadIdx.x / (4 * MM)] + threadIdx.x % 4) % rs.hd;
-        cs = rs.cos[d];
-        sn = rs.sin[d];
-    }
-    uint32_t kb, ks;
-    xreg_lane_k<TRIPS, WHOLE>(wave, b, kb, ks);
-    auto at = [&](const uint32_t *row, uint32_t k) { return xreg_at<WHOLE>(row, k, a.K); };
-    uint32_t k0 = 0;
-    auto chunk = [&](auto trips) __attribute__((always_inline)) {
-        constexpr int T = decltype(trips)::value;
-        float4v xr[G][T];
-#pragma unroll
         for (int t = 0; t < T; t++)
 #pragma unroll
-            for (int g = 0; g < G; g++) xr[g][t] = at(xrow[g], k0 + kb + ks * t);
-        float4v gm[NORM ? T : 1];
-        if constexpr (NORM) {
+            for (int g = 0; g < G; g++) xr[g][t] = xreg_at<WHOLE>(xrow[g], k0 + kb + ks * t, a.K);
 #pragma unroll
-            for (int t = 0; t < T; t++) gm[t] = at(nf.gamma, k0 + kb + ks * t);
-        }
-        float4v ws[2][T];
+        for (int c = 0; c < CG; c++) {
+            float4v w[T];
 #pragma unroll
-        for (int c = 0; c < 2; c++)
-#pragma unroll
-            for (int t = 0; t < T; t++) ws[c][t] = at(wrow[c], k0 + kb + ks * t);
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-            float4v (&w)[T] = ws[c];
-            if constexpr (!WHOLE || NORM) __builtin_amdgcn_sched_barrier(0); // (what follows stays behind all of the loads)
-            if constexpr (NORM) {
-                if (c == 0 && k0 == 0) { // (the same for every thread)
-                    const float s = wave_add<MM>(xreg_sums<MM>(nf, pv));
-                    if (lane < MM) nsum[wave][lane] = s;
-                    __syncthreads();
-                    if (threadIdx.x < 64) divisor = norm_divisor(nf, (nsum[0][threadIdx.x / 4 % MM] + nsum[1][threadIdx.x / 4 % MM]) + (nsum[2][threadIdx.x / 4 % MM] + nsum[3][threadIdx.x / 4 % MM]));
-                }
-            }
-            if constexpr (NORM) {
-                if (c == 0) {
-#pragma unroll
-                    for (int t = 0; t < T; t++)
-#pragma unroll
-                        for (int g = 0; g < G; g++)
-#pragma unroll
-                            for (int e = 0; e < 4; e++) xr[g][t][e] = asf(apply<kMul, true>(asu(xr[g][t][e]), asu(gm[t][e]), 0, nullptr));
-                }
-            }
+            for (int t = 0; t < T; t++) w[t] = xreg_at<WHOLE>(wrow[c], k0 + kb + ks * t, a.K);
+            if constexpr (!WHOLE) __builtin_amdgcn_sched_barrier(0); // (what follows stays behind all of the loads)
             if constexpr (!WHOLE) {
 #pragma unroll
                 for (int t = 0; t < T; t++) {
@@ -1606,26 +1213,19 @@ __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_group_rope_kerne
         }
     };
     for (; k0 < a.K; k0 += TRIPS * 256) xreg_chunk<TRIPS, WHOLE>(a.K - k0, chunk);
-    __shared__ float part[4][kOut];
+    __shared__ float part[4][CG * MM * 4];
 #pragma unroll
-    for (int c = 0; c < 2; c++)
+    for (int c = 0; c < CG; c++)
 #pragma unroll
         for (int g = 0; g < G; g++) {
             const float v = four_sums(acc[c][g][0], acc[c][g][1], acc[c][g][2], acc[c][g][3]); // of row g * 4 + b / 4
             if (b % 4 == 0) part[wave][(c * MM + 4 * g) * 4 + b + j] = v;
         }
     __syncthreads();
-    if (threadIdx.x < 64) { // the first wave: lanes 0 .. kOut - 1 hold (column group, row, column), any others idle along
-        const uint32_t t = threadIdx.x % kOut, c = t / (4 * MM), m = t / 4 % MM, col = nc[c] + t % 4;
-        uint32_t v = asu((part[0][t] + part[1][t]) + (part[2][t] + part[3][t]));
-        if constexpr (NORM) v = apply<kDiv, true>(v, divisor, 0, nullptr);
-        const uint32_t other = across<4 * MM>(v); // the same row's column half a head away
-        if (rs.rope) {
-            // lower half: rotate_half reads -x[d + hd / 2]; upper half: x[d - hd / 2]
-            const uint32_t rot = c == 0 ? apply<kNeg, true>(other, 0, 0, nullptr) : other;
-            v = apply<kAdd, true>(apply<kMul, true>(cs, v, 0, nullptr), apply<kMul, true>(sn, rot, 0, nullptr), 0, nullptr);
-        }
-        if (threadIdx.x < kOut && col < a.N && m < a.M) rs.dst[(int64_t)m * rs.sb + (int64_t)(col / rs.hd) * rs.sh + col % rs.hd] = v;
+    if (threadIdx.x < CG * MM * 4) {
+        const uint32_t c = threadIdx.x / (MM * 4), m = threadIdx.x / 4 % MM, col = n0 + 4 * c + threadIdx.x % 4;
+        const uint32_t v = asu((part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]));
+        if (col < a.N && m < a.M) a.C[((uint64_t)blockIdx.y * a.M + m) * a.N + col] = v;
     }
 }
 
@@ -1641,9 +1241,9 @@ __global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_group_rope_kerne
 // so that launch is as slow as its heads are few: 23 to 29 us for the 32 heads of 128 x 1024 of the Qwen3-0.6B shape):
 // 9 + 3 us and a hand-over, 1.94 -> 1.66 ms per decode step of that shape.
 struct HeadFinish {
-    RopeStore s[kMaxGroup];
-    const uint32_t *src[kMaxGroup];
-    uint32_t N[kMaxGroup];
+    RopeStore s[kMaxSkinny];
+    const uint32_t *src[kMaxSkinny];
+    uint32_t N[kMaxSkinny];
     uint32_t n, M;
 };
 constexpr int kFinishThreads = 1024;
@@ -1686,131 +1286,6 @@ __global__ __launch_bounds__(kFinishThreads) void head_norm_rope_finish_kernel(c
         v = apply<kAdd, true>(apply<kMul, true>(cs, v, 0, nullptr), apply<kMul, true>(sn, rot, 0, nullptr), 0, nullptr);
     }
     rs.dst[(int64_t)m * rs.sb + (int64_t)head * rs.sh + d] = v;
-}
-
-// The gated pair when K is exactly one chunk (TRIPS * 256: the hidden size of the model): the workgroup asks for its
-// share of the activations (and of gamma, and of the row sums of an RMS norm) ONCE and walks `iters` consecutive
-// groups of four columns with them, the next group's weights always on their way while the current group is
-// multiplied, reduced and stored.  Measured on the 1B-shape decode step: the activation, gamma and partial-sum loads
-// of a workgroup that owns a single column group cost a fifth of the kernel's time although they all hit in L2 (they
-// are three quarters as many bytes again as the weights); four groups per workgroup take 29.5 instead of 34.3 us for
-// the 128 MiB of gate + up, more leave too few workgroups in flight.  For q / k / v and o (a quarter of the columns)
-// one group per workgroup stays the fastest.  Weights are read with the non-temporal hint.
-// M <= MM, batch folded away (one batch entry).  Epilogues as in skinny_kt_mfma_xreg_body.
-template <bool WHOLE, int MM, bool NORM, int CHUNK, int TRIPS>
-__device__ __forceinline__ void skinny_kt_mfma_xreg_cols_gated_impl(const MmArgs &a, const uint32_t *second, uint32_t one, uint32_t iters, const NormFuse &nf) {
-    const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const uint32_t j = lane % 4, b = lane / 4;
-    uint32_t kb, ks; // this lane's k: kb + ks t (beyond K, in a chunk that K does not fill: zeros)
-    xreg_lane_k<CHUNK, WHOLE>(wave, b, kb, ks);
-    constexpr int G = MM / 4, kOut = 4 * MM; // row groups; values of one product in a group of columns
-    float pv[2 * MM];
-    if constexpr (NORM) xreg_ask_sums<MM>(nf, pv);
-    float4v xr[G][TRIPS];
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-        const uint32_t *xrow = a.A + (int64_t)min((uint32_t)(4 * g) + j, a.M - 1) * a.a_sm;
-#pragma unroll
-        for (int t = 0; t < TRIPS; t++) xr[g][t] = xreg_at<WHOLE>(xrow, kb + ks * t, a.K);
-    }
-    float4v gm[NORM ? TRIPS : 1];
-    if constexpr (NORM) {
-#pragma unroll
-        for (int t = 0; t < TRIPS; t++) gm[t] = xreg_at<WHOLE>(nf.gamma, kb + ks * t, a.K);
-    }
-    __shared__ float part[2][4][2 * kOut];
-    __shared__ float nsum[4][MM];
-    const uint32_t groups = (a.N + 3) / 4;
-    float4v wg[TRIPS], wu[TRIPS]; // the group's four columns of the two weight matrices
-    auto ask = [&](float4v (&w)[TRIPS], const uint32_t *base, uint32_t n0) {
-        const uint32_t *row = base + (int64_t)min(n0 + j, a.N - 1) * a.b_sn;
-#pragma unroll
-        for (int t = 0; t < TRIPS; t++) w[t] = xreg_at<WHOLE, true>(row, kb + ks * t, a.K);
-    };
-    auto multiply = [&](float4v (&sum)[G], float4v (&w)[TRIPS]) {
-        if constexpr (!WHOLE) {
-#pragma unroll
-            for (int t = 0; t < TRIPS; t++) w[t] = xreg_within<WHOLE>(w[t], kb + ks * t, a.K);
-        }
-#pragma unroll
-        for (int t = 0; t < TRIPS; t++)
-#pragma unroll
-            for (int g = 0; g < G; g++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) sum[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[g][t][e], w[t][e], sum[g], 0, 0, 0);
-    };
-    const uint32_t first_grp = blockIdx.x * iters;
-    if (first_grp >= groups) return; // the same for every thread of the workgroup
-    ask(wg, a.B, first_grp * 4);
-    ask(wu, second, first_grp * 4);
-    if constexpr (!WHOLE || NORM) __builtin_amdgcn_sched_barrier(0); // (what follows stays behind the loads)
-    uint32_t divisor = 0;
-    if constexpr (NORM) { // (the norm as in skinny_kt_mfma_xreg_body)
-        const float s = wave_add<MM>(xreg_sums<MM>(nf, pv));
-        if (lane < MM) nsum[wave][lane] = s;
-        __syncthreads();
-        if (threadIdx.x < kOut) {
-            const uint32_t m = threadIdx.x / 4;
-            divisor = norm_divisor(nf, (nsum[0][m] + nsum[1][m]) + (nsum[2][m] + nsum[3][m]));
-        }
-        // (x / d * gamma) . w = ((x * gamma) . w) / d: gamma goes in once, while the first weights are on their way; the row
-        // sums of squares are put together from the partial sums, always in the same order
-#pragma unroll
-        for (int t = 0; t < TRIPS; t++)
-#pragma unroll
-            for (int g = 0; g < G; g++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) xr[g][t][e] = asf(apply<kMul, true>(asu(xr[g][t][e]), asu(gm[t][e]), 0, nullptr));
-    }
-    if constexpr (!WHOLE) {
-#pragma unroll
-        for (int g = 0; g < G; g++)
-#pragma unroll
-            for (int t = 0; t < TRIPS; t++) xr[g][t] = xreg_within<WHOLE>(xr[g][t], kb + ks * t, a.K);
-    }
-    for (uint32_t it = 0; it < iters; it++) {
-        const uint32_t grp = first_grp + it;
-        if (grp >= groups) break;
-        const uint32_t n0 = grp * 4;
-        float4v acc_g[G] = {}, acc_u[G] = {};
-        const bool more = it + 1 < iters && grp + 1 < groups;
-        multiply(acc_g, wg);
-        if (more) ask(wg, a.B, n0 + 4); // on its way through the rest of this group
-        multiply(acc_u, wu);
-        if (more) ask(wu, second, n0 + 4);
-        float (*pt)[2 * kOut] = part[it & 1];
-#pragma unroll
-        for (int g = 0; g < G; g++) {
-            const float vg = four_sums(acc_g[g][0], acc_g[g][1], acc_g[g][2], acc_g[g][3]); // of row g * 4 + b / 4
-            const float vu = four_sums(acc_u[g][0], acc_u[g][1], acc_u[g][2], acc_u[g][3]);
-            if (b % 4 == 0) {
-                pt[wave][16 * g + b + j] = vg;
-                pt[wave][kOut + 16 * g + b + j] = vu;
-            }
-        }
-        __syncthreads(); // (the buffer written two groups ago was read before the barrier of the group in between)
-        if (threadIdx.x < kOut) {
-            const uint32_t t = threadIdx.x, m = t / 4, col = n0 + t % 4;
-            uint32_t gv = asu((pt[0][t] + pt[1][t]) + (pt[2][t] + pt[3][t]));
-            uint32_t uv = asu((pt[0][kOut + t] + pt[1][kOut + t]) + (pt[2][kOut + t] + pt[3][kOut + t]));
-            if constexpr (NORM) {
-                gv = apply<kDiv, true>(gv, divisor, 0, nullptr);
-                uv = apply<kDiv, true>(uv, divisor, 0, nullptr);
-            }
-            // the ops of the deferred program, in its order
-            const uint32_t e = apply<kExp, true>(apply<kNeg, true>(gv, 0, 0, nullptr), 0, 0, nullptr);
-            const uint32_t sg = apply<kDiv, true>(one, apply<kAdd, true>(one, e, 0, nullptr), 0, nullptr);
-            const uint32_t r = apply<kMul, true>(apply<kMul, true>(gv, sg, 0, nullptr), uv, 0, nullptr);
-            if (col < a.N && m < a.M) a.C[(uint64_t)m * a.N + col] = r;
-        }
-    }
-}
-template <bool WHOLE, int MM, bool NORM, int TRIPS>
-__global__ __launch_bounds__(kThreads) void skinny_kt_mfma_xreg_cols_gated_kernel(const MmArgs a, const uint32_t *second, uint32_t one,
-                                                                                  uint32_t iters, const NormFuse nf) {
-    xreg_chunk<TRIPS, WHOLE>(a.K, [&](auto trips) __attribute__((always_inline)) {
-        skinny_kt_mfma_xreg_cols_gated_impl<WHOLE, MM, NORM, TRIPS, decltype(trips)::value>(a, second, one, iters, nf);
-    });
 }
 
 // Vectorised skinny kernel for short K (K <= 4*LPC, e.g. q.K^T of a decode step with
@@ -2085,102 +1560,70 @@ static const void *native_ptr(const cg_tensor *t) {
     return static_cast<const char *>(t->buf->ptr) + t->offset * (int64_t)fmt_bytes(t->buf->fmt);
 }
 
-// One row: a kernel of its own (one_row.hip)
-static OneRowInput one_row_input(const MmArgs &a, const NormFuse *nf) {
-    OneRowInput in = {reinterpret_cast<const float *>(a.A), nullptr, a.K, 0, 0, 0};
-    if (nf) in = {in.x, reinterpret_cast<const float *>(nf->gamma), a.K, nf->n_bits, nf->eps_bits, nf->exp_bits};
+// One to eight rows, k contiguous in 16-byte pieces, one batch entry: skinny.hpp
+static SkinnyInput skinny_input(const MmArgs &a, const NormFuse *nf) {
+    SkinnyInput in = {reinterpret_cast<const float *>(a.A), nullptr, a.a_sm, a.M, a.K, 0, 0, 0};
+    if (nf) {
+        in.gamma = reinterpret_cast<const float *>(nf->gamma);
+        in.n_bits = nf->n_bits;
+        in.eps_bits = nf->eps_bits;
+        in.exp_bits = nf->exp_bits;
+    }
     return in;
 }
-static OneRowProduct one_row_product(const MmArgs &a) { // its row stored as it is
-    return {reinterpret_cast<const float *>(a.B), a.b_sn, a.N, 0, a.C, 0, nullptr, nullptr, a.N, 0};
+static SkinnyProduct skinny_product(const MmArgs &a) { // its rows stored as they are
+    return {reinterpret_cast<const float *>(a.B), a.b_sn, a.N, 0, a.C, a.N, 0, nullptr, nullptr, a.N, 0};
 }
+static bool skinny_operands(const MmArgs &a) { return a.a_vec && a.b_vec && a.a_sk == 1 && a.b_sk == 1 && takes_skinny(a.M, a.K); }
 
 int launch_matmul_group(cg_backend *be, const cg_tensor *x, const cg_tensor *const *ys, cg_tensor *const *outs, int n,
                         const NormFuse *nf) {
     if (int frc = flush_deferred(be)) return frc;
-    if (n < (nf ? 1 : 2) || n > kMaxGroup || x->dt != CG_F32) return kDeclined;
-    MmGroup g;
-    memset(&g, 0, sizeof g);
+    if (n < (nf ? 1 : 2) || n > kMaxSkinny || x->dt != CG_F32) return kDeclined;
+    SkinnyGroup g = {};
+    MmArgs first;
     double bytes = distinct_bytes(x);
-    bool all_wide = true;
     for (int i = 0; i < n; i++) {
+        MmArgs a;
         MmFold f;
-        int rc = make_mm_args(x, ys[i], outs[i]->buf->ptr, &g.p[i], &f);
+        int rc = make_mm_args(x, ys[i], outs[i]->buf->ptr, &a, &f);
         if (rc) return rc;
-        const MmArgs &a = g.p[i];
-        const bool vec = a.a_vec && a.b_vec && a.a_sk == 1 && a.K % 4 == 0;
-        if (f.batch != 1 || a.M > 8 || a.b_sk != 1 || !vec || a.K <= 256 || a.N < 4) return kDeclined;
-        if (i > 0 && (a.M != g.p[0].M || a.K != g.p[0].K || a.a_sm != g.p[0].a_sm)) return kDeclined;
-        all_wide = all_wide && a.N >= 8192;
+        if (f.batch != 1 || !skinny_operands(a) || a.N < 4) return kDeclined;
+        if (i == 0) first = a;
+        else if (a.M != first.M || a.K != first.K || a.a_sm != first.a_sm) return kDeclined;
+        g.p[i] = skinny_product(a);
         bytes += distinct_bytes(ys[i]) + distinct_bytes(outs[i]);
     }
-    if (takes_one_row(g.p[0].M, g.p[0].K)) {
-        OneRowGroup og = {one_row_input(g.p[0], nf), {}, (uint32_t)n};
-        for (int i = 0; i < n; i++) og.p[i] = one_row_product(g.p[i]);
-        ProfScope prof(be, CG_K_GEMM_SKINNY, bytes);
-        return launch_one_row_group(be, og);
-    }
-    const bool xreg = !nf && all_wide && g.p[0].M <= 4;
-    for (int i = 0; i < n && nf; i++)
-        if (g.p[i].N >= 8192) return kDeclined; // a vocabulary-sized product: the kernel with more columns per wave, the norm on its own
-    uint32_t blocks = 0;
-    for (int i = 0; i < n; i++) {
-        g.first[i] = blocks;
-        blocks += xreg ? (g.p[i].N + 7) / 8 : (g.p[i].N + 3) / 4;
-    }
-    g.first[n] = blocks;
-    g.n = (uint32_t)n;
+    g.in = skinny_input(first, nf);
+    g.count = (uint32_t)n;
     ProfScope prof(be, CG_K_GEMM_SKINNY, bytes);
-    const bool eight = g.p[0].M > 4, deep = xreg_trips(g.p[0].K) == 8;
-    auto launch = [&](auto kernel, auto... args) { launch_kernel(kernel, dim3(blocks), dim3(kThreads), 0, be->stream, args...); };
-    xreg_either(g.p[0].K, xreg ? 8 : xreg_trips(g.p[0].K), [&](auto whole) { // (the problems of a group share k)
-        constexpr bool W = decltype(whole)::value;
-        if (xreg) launch(skinny_kt_mfma_xreg_group_kernel<W, 4, 2, 8>, g);
-        else if (nf && deep && eight) launch(skinny_kt_mfma_xreg_group_norm_kernel<W, 8, 8>, g, *nf);
-        else if (nf && deep) launch(skinny_kt_mfma_xreg_group_norm_kernel<W, 4, 8>, g, *nf);
-        else if (nf && eight) launch(skinny_kt_mfma_xreg_group_norm_kernel<W, 8, 4>, g, *nf);
-        else if (nf) launch(skinny_kt_mfma_xreg_group_norm_kernel<W, 4, 4>, g, *nf);
-        else if (deep && eight) launch(skinny_kt_mfma_xreg_group_kernel<W, 8, 1, 8>, g);
-        else if (deep) launch(skinny_kt_mfma_xreg_group_kernel<W, 4, 1, 8>, g);
-        else if (eight) launch(skinny_kt_mfma_xreg_group_kernel<W, 8, 1, 4>, g);
-        else launch(skinny_kt_mfma_xreg_group_kernel<W, 4, 1, 4>, g);
-    });
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? CG_OK : hip_fail(e, "grouped matmul launch");
+    return launch_skinny_group(be, g);
 }
 
 int launch_matmul_group_rope(cg_backend *be, const cg_tensor *x, const cg_tensor *const *ys, const RopeStore *stores, int n,
                              const NormFuse *nf) {
-    if (n < 1 || n > kMaxGroup || x->dt != CG_F32) return kDeclined;
-    MmGroup g;
-    RopeGroup rg;
-    memset(&g, 0, sizeof g);
-    memset(&rg, 0, sizeof rg);
+    if (n < 1 || n > kMaxSkinny || x->dt != CG_F32) return kDeclined;
+    SkinnyGroup g = {};
+    MmArgs first;
     double bytes = distinct_bytes(x);
-    uint32_t blocks = 0;
     bool by_head = false; // some product's heads are normed: two launches (see head_norm_rope_finish_kernel)
     for (int i = 0; i < n; i++) by_head = by_head || stores[i].hgamma != nullptr;
     for (int i = 0; i < n; i++) {
+        MmArgs a;
         MmFold f;
-        int rc = make_mm_args(x, ys[i], stores[i].dst, &g.p[i], &f);
+        int rc = make_mm_args(x, ys[i], stores[i].dst, &a, &f);
         if (rc) return rc;
-        const MmArgs &a = g.p[i];
         const RopeStore &st = stores[i];
-        const bool vec = a.a_vec && a.b_vec && a.a_sk == 1 && a.K % 4 == 0;
-        if (f.batch != 1 || !xreg_narrow(a.M, a.K) || a.b_sk != 1 || !vec || a.N >= 8192) return kDeclined;
-        if (i > 0 && (a.M != g.p[0].M || a.K != g.p[0].K || a.a_sm != g.p[0].a_sm)) return kDeclined;
+        if (f.batch != 1 || !skinny_operands(a) || a.N >= 8192) return kDeclined;
+        if (i == 0) first = a;
+        else if (a.M != first.M || a.K != first.K || a.a_sm != first.a_sm) return kDeclined;
         if (st.hd < 8 || st.hd % 8 || a.N % st.hd || !st.dst || (st.rope && (!st.cos || !st.sin))) return kDeclined;
         if (by_head && (st.hd % 16 || st.hd > 128)) return kDeclined;
-        rg.s[i] = st;
-        g.first[i] = blocks;
-        blocks += a.N / 8;
+        g.p[i] = {reinterpret_cast<const float *>(a.B), a.b_sn, a.N, 0, st.dst, st.sb, st.sh, st.cos, st.sin, st.hd, st.rope};
         bytes += distinct_bytes(ys[i]) + 4.0 * (double)a.M * a.N;
     }
-    g.first[n] = blocks;
-    g.n = (uint32_t)n;
-    NormFuse none;
-    memset(&none, 0, sizeof none);
-    const bool wide = xreg_trips(g.p[0].K) == 8;
+    g.in = skinny_input(first, nf);
+    g.count = (uint32_t)n;
     ProfScope prof(be, CG_K_GEMM_SKINNY, bytes);
     HeadFinish hf;
     void *tmp = nullptr;
@@ -2188,66 +1631,43 @@ int launch_matmul_group_rope(cg_backend *be, const cg_tensor *x, const cg_tensor
     uint32_t finish_heads = 0, finish_hd = 0;
     if (by_head) { // the normed products go to scratch memory as they are (see head_norm_rope_finish_kernel)
         memset(&hf, 0, sizeof hf);
-        hf.M = g.p[0].M;
+        hf.M = first.M;
         uint64_t words = 0;
         for (int i = 0; i < n; i++)
-            if (stores[i].hgamma) words += (uint64_t)g.p[i].M * g.p[i].N;
+            if (stores[i].hgamma) words += (uint64_t)first.M * g.p[i].n;
         if (int arc = be->pool.alloc(words * 4, &tmp, &tmp_cls)) return arc;
         uint32_t *at = static_cast<uint32_t *>(tmp);
         for (int i = 0; i < n; i++) {
             if (!stores[i].hgamma) continue;
             const uint32_t k = hf.n++;
+            SkinnyProduct &p = g.p[i]; // column n of row m to at[m * N + n]
             hf.s[k] = stores[i];
             hf.src[k] = at;
-            hf.N[k] = g.p[i].N;
-            finish_heads = std::max(finish_heads, g.p[i].N / stores[i].hd);
+            hf.N[k] = p.n;
+            finish_heads = std::max(finish_heads, p.n / stores[i].hd);
             finish_hd = std::max(finish_hd, stores[i].hd);
-            RopeStore &plain = rg.s[i]; // column n of row m to at[m * N + n]
-            plain.dst = at;
-            plain.sb = g.p[i].N;
-            plain.sh = stores[i].hd;
-            plain.rope = 0;
-            plain.hgamma = nullptr;
-            at += (uint64_t)g.p[i].M * g.p[i].N;
+            p.dst = at;
+            p.sb = p.n;
+            p.sh = stores[i].hd;
+            p.rope = 0;
+            at += (uint64_t)first.M * p.n;
         }
     }
-    auto launch = [&](auto kernel) { launch_kernel(kernel, dim3(blocks), dim3(kThreads), 0, be->stream, g, rg, nf ? *nf : none); };
-    if (takes_one_row(g.p[0].M, g.p[0].K)) {
-        OneRowGroup og = {one_row_input(g.p[0], nf), {}, (uint32_t)n};
-        for (int i = 0; i < n; i++) {
-            const RopeStore &st = rg.s[i];
-            og.p[i] = {reinterpret_cast<const float *>(g.p[i].B), g.p[i].b_sn, g.p[i].N, 0, st.dst, st.sh, st.cos, st.sin, st.hd, st.rope};
-        }
-        if (const int rc = launch_one_row_group(be, og)) {
-            if (tmp) be->pool.free(tmp, tmp_cls);
-            return rc;
-        }
-    } else xreg_either(g.p[0].K, xreg_trips(g.p[0].K), [&](auto whole) { // (the problems of a group share k)
-        constexpr bool W = decltype(whole)::value;
-        if (g.p[0].M > 4) {
-            if (nf && wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 8, true, 8>);
-            else if (nf) launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 8, true, 4>);
-            else if (wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 8, false, 8>);
-            else launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 8, false, 4>);
-        } else {
-            if (nf && wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 4, true, 8>);
-            else if (nf) launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 4, true, 4>);
-            else if (wide) launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 4, false, 8>);
-            else launch(skinny_kt_mfma_xreg_group_rope_kernel<W, 4, false, 4>);
-        }
-    });
+    int rc = launch_skinny_group(be, g);
     if (by_head) {
         const uint32_t threads = (hf.M * finish_hd + 63) / 64 * 64;
-        launch_kernel(head_norm_rope_finish_kernel, dim3(finish_heads, hf.n), dim3(threads), 0, be->stream, hf);
+        if (!rc) {
+            launch_kernel(head_norm_rope_finish_kernel, dim3(finish_heads, hf.n), dim3(threads), 0, be->stream, hf);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) rc = hip_fail(e, "head norm launch");
+        }
         be->pool.free(tmp, tmp_cls); // stream-ordered: later users queue behind the finishing launch
     }
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? CG_OK : hip_fail(e, "grouped matmul with rotary store launch");
+    return rc;
 }
 
 // out = g * (1 / (one + exp(-g))) * u with g = x.yg, u = x.yu: two decode-time linear layers and
-// the program between them and the next product in one launch.  Declines unless the 4x4x1
-// kernel takes the shapes.
+// the program between them and the next product in one launch.
 int launch_matmul_gated(cg_backend *be, const cg_tensor *x, const cg_tensor *yg, const cg_tensor *yu, uint32_t one,
                         cg_tensor *out, const NormFuse *nf) {
     if (int frc = flush_deferred(be)) return frc;
@@ -2258,120 +1678,27 @@ int launch_matmul_gated(cg_backend *be, const cg_tensor *x, const cg_tensor *yg,
     int rc = make_mm_args(x, yg, c, &ag, &fg);
     if (!rc) rc = make_mm_args(x, yu, c, &au, &fu);
     if (rc) return rc;
-    const bool vec = ag.a_vec && ag.b_vec && au.b_vec && ag.a_sk == 1 && ag.K % 4 == 0;
-    if (fg.batch != 1 || fu.batch != 1 || ag.M > 8 || ag.b_sk != 1 || au.b_sk != 1 || !vec || ag.K <= 256 || ag.N < 512 ||
-        au.N != ag.N || au.K != ag.K || au.M != ag.M || au.b_sn != ag.b_sn)
+    if (fg.batch != 1 || fu.batch != 1 || !skinny_operands(ag) || !skinny_operands(au) || ag.N < 512 || au.N != ag.N || au.K != ag.K || au.M != ag.M || au.b_sn != ag.b_sn)
         return kDeclined;
-    if (nf && xreg_trips(ag.K) == 0) return kDeclined;
     if (ag.M > 4 && !nf) return kDeclined; // (more than four rows: a decode step's, whose norm comes along; others as a grouped product and the program)
-    const bool short_chunks = xreg_trips(ag.K) == 4; // K a multiple of 1024 but not of 2048
     ProfScope prof(be, CG_K_GEMM_SKINNY, distinct_bytes(x) + distinct_bytes(yg) + distinct_bytes(yu) + distinct_bytes(out));
-    if (takes_one_row(ag.M, ag.K)) {
-        const OneRowGated g = {one_row_input(ag, nf), reinterpret_cast<const float *>(ag.B), reinterpret_cast<const float *>(au.B), ag.b_sn, ag.N, one, c};
-        return launch_one_row_gated(be, g);
-    }
-    const dim3 ggrid((ag.N + 3) / 4);
-    if (xreg_trips(ag.K) == 0) return kDeclined;
-    const bool eight = ag.M > 4;
-    if ((int)ag.K <= xreg_trips(ag.K) * 256) { // one chunk of k (full or not): see skinny_kt_mfma_xreg_cols_gated_kernel
-        NormFuse none;
-        memset(&none, 0, sizeof none);
-        const uint32_t groups = (ag.N + 3) / 4, iters = xreg_cols_iters(groups);
-        const dim3 cgrid((groups + iters - 1) / iters);
-        auto launch = [&](auto kernel) { launch_kernel(kernel, cgrid, dim3(kThreads), 0, be->stream, ag, au.B, one, iters, nf ? *nf : none); };
-        xreg_either(ag.K, xreg_trips(ag.K), [&](auto whole) {
-            constexpr bool W = decltype(whole)::value;
-            if (eight) {
-                if (short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<W, 8, true, 4>);
-                else launch(skinny_kt_mfma_xreg_cols_gated_kernel<W, 8, true, 8>);
-            } else {
-                if (nf && short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<W, 4, true, 4>);
-                else if (nf) launch(skinny_kt_mfma_xreg_cols_gated_kernel<W, 4, true, 8>);
-                else if (short_chunks) launch(skinny_kt_mfma_xreg_cols_gated_kernel<W, 4, false, 4>);
-                else launch(skinny_kt_mfma_xreg_cols_gated_kernel<W, 4, false, 8>);
-            }
-        });
-    } else {
-        auto launch = [&](auto kernel, auto... more) { launch_kernel(kernel, ggrid, dim3(kThreads), 0, be->stream, ag, au.B, one, more...); };
-        xreg_either(ag.K, xreg_trips(ag.K), [&](auto whole) {
-            constexpr bool W = decltype(whole)::value;
-            if (eight) {
-                if (short_chunks) launch(skinny_kt_mfma_xreg_gated_norm_kernel<W, 8, 4>, *nf);
-                else launch(skinny_kt_mfma_xreg_gated_norm_kernel<W, 8, 8>, *nf);
-            } else {
-                if (nf && short_chunks) launch(skinny_kt_mfma_xreg_gated_norm_kernel<W, 4, 4>, *nf);
-                else if (nf) launch(skinny_kt_mfma_xreg_gated_norm_kernel<W, 4, 8>, *nf);
-                else if (short_chunks) launch(skinny_kt_mfma_xreg_gated_kernel<W, 4, 4>);
-                else launch(skinny_kt_mfma_xreg_gated_kernel<W, 4, 8>);
-            }
-        });
-    }
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? CG_OK : hip_fail(e, "gated matmul launch");
+    return launch_skinny_gated(be, {skinny_input(ag, nf), reinterpret_cast<const float *>(ag.B), reinterpret_cast<const float *>(au.B), ag.b_sn, ag.N, one, c});
 }
 
-// out = a sum of four terms, term[slot] = x.y, the other three dense tensors of out's shape
-// (device pointers); `order` as in MmResidual.  Declines unless the one-column-per-wave kernel
-// is what the product would run on anyway.
+// out = a sum of two or four terms, term[slot] = x.y, the others dense tensors of out's shape (device pointers); `order` as in SkinnyResidual.
 int launch_matmul_residual(cg_backend *be, const cg_tensor *x, const cg_tensor *y, const uint32_t *const *terms, int nterms,
-                           int slot, int order, cg_tensor *out, bool keep_sums) {
+                           int slot, int order, cg_tensor *out) {
     if (int frc = flush_deferred(be)) return frc;
     if (x->dt != CG_F32) return kDeclined;
     MmArgs a;
     MmFold f;
     int rc = make_mm_args(x, y, static_cast<uint32_t *>(out->buf->ptr) + out->offset, &a, &f);
     if (rc) return rc;
-    const bool vec = a.a_vec && a.b_vec && a.a_sk == 1 && a.K % 4 == 0;
-    if (f.batch != 1 || a.M > 8 || a.b_sk != 1 || !vec || a.K <= 256 || a.N < 512 || a.N >= 8192) return kDeclined;
-    MmResidual r;
-    for (int t = 0; t < 4; t++) r.term[t] = t == slot || t >= nterms ? nullptr : terms[t];
-    r.slot = (uint32_t)slot;
-    r.order = (uint32_t)order;
-    r.nterms = (uint32_t)nterms;
-    r.partials = nullptr;
-    if (takes_one_row(a.M, a.K)) { // (its norm needs no sums that others left)
-        OneRowResidual o = {reinterpret_cast<const float *>(a.A), reinterpret_cast<const float *>(a.B), a.b_sn, a.N, a.K, {}, r.slot, r.order, r.nterms, a.C};
-        for (int t = 0; t < 4; t++) o.term[t] = r.term[t];
-        ProfScope prof(be, CG_K_GEMM_SKINNY, distinct_bytes(x) + distinct_bytes(y) + 4.0 * distinct_bytes(out));
-        return launch_one_row_residual(be, o);
-    }
-    const uint32_t blocks = (uint32_t)((a.N + 3) / 4);
-    if (keep_sums && out->offset == 0 && xreg_narrow(a.M, a.K) && !out->buf->side) {
-        // the stored rows' sums of squares per workgroup, for an RMS norm that may follow (Buffer::side)
-        Buffer *ob = out->buf;
-        const uint32_t rows = a.M > 4 ? 8 : 4;
-        if (be->pool.alloc((size_t)blocks * rows * sizeof(float), &ob->side, &ob->side_cls) == CG_OK) {
-            ob->side_blocks = blocks;
-            ob->side_rows = rows;
-            r.partials = static_cast<float *>(ob->side);
-        } else {
-            ob->side = nullptr;
-        }
-    }
+    if (f.batch != 1 || !skinny_operands(a) || a.N < 512 || a.N >= 8192) return kDeclined;
+    SkinnyResidual r = {skinny_input(a, nullptr), reinterpret_cast<const float *>(a.B), a.b_sn, a.N, {}, (uint32_t)slot, (uint32_t)order, (uint32_t)nterms, a.C};
+    for (int t = 0; t < nterms; t++) r.term[t] = t == slot ? nullptr : terms[t];
     ProfScope prof(be, CG_K_GEMM_SKINNY, distinct_bytes(x) + distinct_bytes(y) + 4.0 * distinct_bytes(out));
-    dim3 grid((uint32_t)((a.N + 3) / 4));
-    const int eight = eight_trips(be, a.M, a.N, a.K);
-    const dim3 grid8((uint32_t)((a.N + 7) / 8));
-    auto launch8 = [&](auto kernel) { launch_kernel(kernel, grid8, dim3(kEightThreads), 0, be->stream, a, r); };
-    auto launch = [&](auto kernel) { launch_kernel(kernel, grid, dim3(kThreads), 0, be->stream, a, r); };
-    const bool rows8 = a.M > 4;
-    if (eight == 16) launch8(skinny_kt_mfma_eight_residual_kernel<4, 16>);
-    else if (eight == 8 && rows8) launch8(skinny_kt_mfma_eight_residual_kernel<8, 8>);
-    else if (eight == 8) launch8(skinny_kt_mfma_eight_residual_kernel<4, 8>);
-    else if (eight == 4 && rows8) launch8(skinny_kt_mfma_eight_residual_kernel<8, 4>);
-    else if (eight == 4) launch8(skinny_kt_mfma_eight_residual_kernel<4, 4>);
-    else {
-        const bool deep = xreg_trips(a.K) == 8;
-        xreg_either(a.K, xreg_trips(a.K), [&](auto whole) {
-            constexpr bool W = decltype(whole)::value;
-            if (deep && rows8) launch(skinny_kt_mfma_xreg_residual_kernel<W, 8, 8>);
-            else if (deep) launch(skinny_kt_mfma_xreg_residual_kernel<W, 4, 8>);
-            else if (rows8) launch(skinny_kt_mfma_xreg_residual_kernel<W, 8, 4>);
-            else launch(skinny_kt_mfma_xreg_residual_kernel<W, 4, 4>);
-        });
-    }
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? CG_OK : hip_fail(e, "matmul with residual launch");
+    return launch_skinny_residual(be, r);
 }
 
 // ---- narrow operands for the 16-bit and 8-bit matrix instructions ---------------------------------------------------
@@ -2496,7 +1823,7 @@ template <int KIND> __device__ __forceinline__ void widen_weights(const uint4v &
     }
 }
 // The same for at most four rows of the 16-bit dtypes on the matrix instruction v_mfma_f32_4x4x4_{bf16_1k,f16}: the layout
-// of skinny_kt_mfma_xreg_body (lane (b, j) = (lane / 4, lane % 4) feeds weight row n0 + j and activation row j for the k of
+// of skinny_kt_mfma_xreg_kernel (lane (b, j) = (lane / 4, lane % 4) feeds weight row n0 + j and activation row j for the k of
 // block b) with 8 k per lane and trip instead of 4: one 16-byte load of narrow weights drives two instructions.  The
 // activations, which are f32 words in memory, are narrowed (exact) into registers ONCE per workgroup — all of K, 16
 // registers per 2048 — and the workgroup walks `iters` consecutive groups of four columns with them, the next group's
@@ -2759,8 +2086,8 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
         } else {
             // enough waves to cover 256 CUs several times over, else split K inside the block
             const int64_t cols = N * batch;
-            if (batch == 1 && cols >= 2048 && takes_one_row((uint32_t)M, (uint32_t)K)) {
-                const int orc = launch_one_row_group(be, {one_row_input(a, nullptr), {one_row_product(a)}, 1});
+            if (batch == 1 && cols >= 2048 && skinny_operands(a)) {
+                const int orc = launch_skinny_group(be, {skinny_input(a, nullptr), {skinny_product(a)}, 1});
                 if (orc) return orc;
             } else if (cols >= 16384) {
                 dim3 grid((uint32_t)((N + 15) / 16), (uint32_t)batch);

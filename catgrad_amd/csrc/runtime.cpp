@@ -128,7 +128,6 @@ void drop_packed(Buffer *b) {
 void buffer_release(Buffer *b) {
     while (b && b->rc.fetch_sub(1) == 1) {
         if (b->ptr) b->be->pool.free(b->ptr, b->cls);
-        if (b->side) b->be->pool.free(b->side, b->side_cls);
         drop_packed(b);
         buffer_release(b->wide); // (a widened copy has none of its own: one level deep)
         Buffer *next = b->successor;
@@ -160,7 +159,7 @@ Pending::~Pending() {
 }
 
 // Is x (still) the deferred program  h / pow(sum(h * h) / n + eps, e) * gamma  over the rows of a residual stream h
-// [1..8 rows, K] whose kernel left the partial sums of squares (Buffer::side; one row's products form them themselves)?  Then a decode-time product can apply
+// [1..8 rows, K]?  Then a decode-time product can apply
 // the norm while it loads h (K a multiple of 4 above 256) and the norm needs no launch.  Fills nf and the stand-in tensor
 // h (a borrowed view of the leaf's buffer: set h->buf to null before it goes out of scope).
 static bool norm_fuse_of(const cg_tensor *x, NormFuse *nf, cg_tensor *h) {
@@ -176,7 +175,6 @@ static bool norm_fuse_of(const cg_tensor *x, NormFuse *nf, cg_tensor *h) {
     if (K <= 256 || K % 4 != 0 || rows < 1 || rows > 8 || p->rowlen != K) return false;
     const LeafView &lh = p->leaf[0], &lg = p->leaf[4];
     if (lh.uniform || lh.pw || lh.lazy || !lh.buf || lh.offset != 0) return false;
-    if (rows > 1 && (!lh.buf->side || (int64_t)lh.buf->side_blocks * 4 != K || lh.buf->side_rows != (rows > 4 ? 8u : 4u))) return false;
     if (is_narrow_buf(lh.buf) || is_narrow_buf(lg.buf)) return false; // (the kernels read 32-bit words)
     if (!p->leaf[1].uniform || !p->leaf[2].uniform || !p->leaf[3].uniform) return false;
     if (lg.uniform || lg.pw || lg.lazy || !lg.buf || lg.offset % 4 != 0) return false;
@@ -186,8 +184,6 @@ static bool norm_fuse_of(const cg_tensor *x, NormFuse *nf, cg_tensor *h) {
         if (x->dims[d] != 1 && lg.strides[d] != (d == r - 1 ? 1 : 0)) return false;
         st *= x->dims[d];
     }
-    nf->partials = static_cast<const float *>(lh.buf->side);
-    nf->blocks = lh.buf->side_blocks;
     nf->gamma = static_cast<const uint32_t *>(lg.buf->ptr) + lg.offset;
     nf->n_bits = p->leaf[1].ubits;
     nf->eps_bits = p->leaf[2].ubits;
@@ -1004,8 +1000,7 @@ static int try_gated_pair(cg_backend *be, const cg_tensor *dst, const Pending &p
 
 // A sum of four dense terms, one of them a product nobody has needed yet (the residual stream after the
 // o or down projection): the adds run in the product's store.
-// fresh: dst is a whole new buffer, so the row sums of squares of what is stored may be kept with it.
-static int try_residual_store(cg_backend *be, const cg_tensor *dst, const Pending &p, bool fresh) {
+static int try_residual_store(cg_backend *be, const cg_tensor *dst, const Pending &p) {
     static const uint8_t orders[2][3][2] = {{{1, 2}, {0, 8}, {9, 3}}, {{1, 2}, {8, 3}, {0, 9}}};
     if (p.nred != 0 || !is_contiguous(dst) || dst->dt != CG_F32) return kDeclined;
     int order = -1;
@@ -1051,7 +1046,7 @@ static int try_residual_store(cg_backend *be, const cg_tensor *dst, const Pendin
         int xrc = ensure_concrete(m->x);
         if (xrc) return xrc;
     }
-    int rc = launch_matmul_residual(be, m->x, m->y, terms, nterms, slot, order, const_cast<cg_tensor *>(dst), fresh && dst->offset == 0);
+    int rc = launch_matmul_residual(be, m->x, m->y, terms, nterms, slot, order, const_cast<cg_tensor *>(dst));
     if (rc == CG_OK) {
         lazy_mm_close(m);
         be->programs_compiled++;
@@ -1065,7 +1060,7 @@ static int run_pending(cg_backend *be, const cg_tensor *dst, const Pending &p, b
     if (narrow_dst && p.nred > 0) return fail(CG_ERR_ARG, "internal error: a narrow buffer written by a kernel that stores words");
     if (be->aot && !narrow_dst) {
         int grc = try_gated_pair(be, dst, p);
-        if (grc == kDeclined) grc = try_residual_store(be, dst, p, fresh);
+        if (grc == kDeclined) grc = try_residual_store(be, dst, p);
         if (grc != kDeclined) return grc;
     }
     {
@@ -3561,11 +3556,6 @@ int cg_concat(cg_backend *b, cg_tensor *x, cg_tensor *y, size_t dim, cg_tensor *
         if (rc) return rc;
         x->buf->elems = nx + ny;
         drop_packed(x->buf);
-        if (x->buf->side) { // row sums kept for the rows this buffer held so far do not describe the grown tensor
-            b->pool.free(x->buf->side, x->buf->side_cls);
-            x->buf->side = nullptr;
-            x->buf->side_blocks = 0;
-        }
         x->dims[dim] = od[dim];
         set_row_major(x);
         retain(x);
