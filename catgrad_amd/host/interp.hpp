@@ -248,48 +248,71 @@ class Interpreter {
 // DSL spellings.  `I` plays the role of the `Builder`; argument orders are those of
 // catgrad/src/category/lang/ops.rs:165-218 (e.g. `broadcast(builder, shape, x)` emits
 // the operands [x, shape]; `reshape(builder, shape, x)` emits [shape, x]).
+// Unless a term is being recorded, an operation is the backend call itself, checked as tensor_op() checks it: a decode step issues
+// thousands, and the vectors of arguments and results cost as much as the calls (SmolLM2-135M shape: 0.79 -> 0.72 ms a step).
 namespace ops {
 using I = Interpreter;
-inline Tensor add(I &i, Tensor x, Tensor y) { return i.run1(TensorOp::Add, vals(std::move(x), std::move(y))); }
-inline Tensor sub(I &i, Tensor x, Tensor y) { return i.run1(TensorOp::Sub, vals(std::move(x), std::move(y))); }
-inline Tensor mul(I &i, Tensor x, Tensor y) { return i.run1(TensorOp::Mul, vals(std::move(x), std::move(y))); }
-inline Tensor div(I &i, Tensor x, Tensor y) { return i.run1(TensorOp::Div, vals(std::move(x), std::move(y))); }
-inline Tensor pow(I &i, Tensor x, Tensor y) { return i.run1(TensorOp::Pow, vals(std::move(x), std::move(y))); }
-inline Tensor lt(I &i, Tensor x, Tensor y) { return i.run1(TensorOp::LT, vals(std::move(x), std::move(y))); }
-inline Tensor lte(I &i, Tensor x, Tensor y) { return i.run1(TensorOp::LTE, vals(std::move(x), std::move(y))); }
-inline Tensor gte(I &i, Tensor x, Tensor y) { return i.run1(TensorOp::GTE, vals(std::move(x), std::move(y))); }
+namespace detail {
+inline void same_dtype(const Tensor &x, const Tensor &y) { // as cgh::detail::same_dtype
+    if (x.dtype() != y.dtype()) throw InterpreterError("TypeError: mixed dtypes");
+}
+inline Tensor binary(I &i, TensorOp op, cg_binary_op call, Tensor x, Tensor y) {
+    if (i.recorder) return i.run1(op, vals(std::move(x), std::move(y)));
+    same_dtype(x, y);
+    return i.backend.binary(call, std::move(x), std::move(y));
+}
+inline Tensor unary(I &i, TensorOp op, cg_unary_op call, Tensor x) {
+    return i.recorder ? i.run1(op, vals(std::move(x))) : i.backend.unary(call, std::move(x));
+}
+} // namespace detail
+inline Tensor add(I &i, Tensor x, Tensor y) { return detail::binary(i, TensorOp::Add, CG_ADD, std::move(x), std::move(y)); }
+inline Tensor sub(I &i, Tensor x, Tensor y) { return detail::binary(i, TensorOp::Sub, CG_SUB, std::move(x), std::move(y)); }
+inline Tensor mul(I &i, Tensor x, Tensor y) { return detail::binary(i, TensorOp::Mul, CG_MUL, std::move(x), std::move(y)); }
+inline Tensor div(I &i, Tensor x, Tensor y) { return detail::binary(i, TensorOp::Div, CG_DIV, std::move(x), std::move(y)); }
+inline Tensor pow(I &i, Tensor x, Tensor y) { return detail::binary(i, TensorOp::Pow, CG_POW, std::move(x), std::move(y)); }
+inline Tensor lt(I &i, Tensor x, Tensor y) { return detail::binary(i, TensorOp::LT, CG_LT, std::move(x), std::move(y)); }
+inline Tensor lte(I &i, Tensor x, Tensor y) { return detail::binary(i, TensorOp::LTE, CG_LTE, std::move(x), std::move(y)); }
+inline Tensor gte(I &i, Tensor x, Tensor y) { return detail::binary(i, TensorOp::GTE, CG_GTE, std::move(x), std::move(y)); }
 // lang/ops.rs:241-249: the operand is borrowed (`&Var`), so the operation reads a clone; it has no result
 inline void probe(I &i, const std::string &label, const Tensor &x) { i.run(Op::probe(label), vals(Tensor(x))); }
-inline Tensor neg(I &i, Tensor x) { return i.run1(TensorOp::Neg, vals(std::move(x))); }
-inline Tensor exp(I &i, Tensor x) { return i.run1(TensorOp::Exp, vals(std::move(x))); }
-inline Tensor sin(I &i, Tensor x) { return i.run1(TensorOp::Sin, vals(std::move(x))); }
-inline Tensor cos(I &i, Tensor x) { return i.run1(TensorOp::Cos, vals(std::move(x))); }
-inline Tensor sum(I &i, Tensor x) { return i.run1(TensorOp::Sum, vals(std::move(x))); }
-inline Tensor max(I &i, Tensor x) { return i.run1(TensorOp::Max, vals(std::move(x))); }
-inline Tensor argmax(I &i, Tensor x) { return i.run1(TensorOp::Argmax, vals(std::move(x))); }
-inline Tensor matmul(I &i, Tensor x, Tensor y) { return i.run1(TensorOp::MatMul, vals(std::move(x), std::move(y))); }
-inline Tensor cast(I &i, Tensor x, cg_dtype d) { return i.run1(TensorOp::Cast, vals(std::move(x), d)); }
+inline Tensor neg(I &i, Tensor x) { return detail::unary(i, TensorOp::Neg, CG_NEG, std::move(x)); }
+inline Tensor exp(I &i, Tensor x) { return detail::unary(i, TensorOp::Exp, CG_EXP, std::move(x)); }
+inline Tensor sin(I &i, Tensor x) { return detail::unary(i, TensorOp::Sin, CG_SIN, std::move(x)); }
+inline Tensor cos(I &i, Tensor x) { return detail::unary(i, TensorOp::Cos, CG_COS, std::move(x)); }
+inline Tensor sum(I &i, Tensor x) { return i.recorder ? i.run1(TensorOp::Sum, vals(std::move(x))) : i.backend.sum(std::move(x)); }
+inline Tensor max(I &i, Tensor x) { return i.recorder ? i.run1(TensorOp::Max, vals(std::move(x))) : i.backend.max(std::move(x)); }
+inline Tensor argmax(I &i, Tensor x) { return i.recorder ? i.run1(TensorOp::Argmax, vals(std::move(x))) : i.backend.argmax(std::move(x)); }
+inline Tensor matmul(I &i, Tensor x, Tensor y) {
+    if (i.recorder) return i.run1(TensorOp::MatMul, vals(std::move(x), std::move(y)));
+    detail::same_dtype(x, y);
+    return i.backend.matmul(std::move(x), std::move(y));
+}
+inline Tensor cast(I &i, Tensor x, cg_dtype d) { return i.recorder ? i.run1(TensorOp::Cast, vals(std::move(x), d)) : i.backend.cast(std::move(x), d); }
 inline Tensor nat_to_u32(I &i, size_t n) { return i.run1(TensorOp::NatToU32, vals(n)); }
 inline Tensor arange(I &i, size_t end) { return i.run1(TensorOp::Arange, vals(end)); }
-inline Tensor broadcast(I &i, const Shape &s, Tensor x) { return i.run1(TensorOp::Broadcast, vals(std::move(x), s)); }
-inline Tensor reshape(I &i, const Shape &s, Tensor x) { return i.run1(TensorOp::Reshape, vals(s, std::move(x))); }
+inline Tensor broadcast(I &i, const Shape &s, Tensor x) {
+    return i.recorder ? i.run1(TensorOp::Broadcast, vals(std::move(x), s)) : i.backend.broadcast(std::move(x), s);
+}
+inline Tensor reshape(I &i, const Shape &s, Tensor x) {
+    return i.recorder ? i.run1(TensorOp::Reshape, vals(s, std::move(x))) : i.backend.reshape(std::move(x), s);
+}
 inline Tensor transpose(I &i, size_t d0, size_t d1, Tensor x) {
-    return i.run1(TensorOp::Transpose, vals(std::move(x), d0, d1));
+    return i.recorder ? i.run1(TensorOp::Transpose, vals(std::move(x), d0, d1)) : i.backend.transpose(std::move(x), d0, d1);
 }
 inline Tensor index(I &i, size_t dim, Tensor idx, Tensor x) {
-    return i.run1(TensorOp::Index, vals(std::move(x), dim, std::move(idx)));
+    return i.recorder ? i.run1(TensorOp::Index, vals(std::move(x), dim, std::move(idx))) : i.backend.index(std::move(x), dim, std::move(idx));
 }
 inline Tensor slice(I &i, size_t dim, size_t start, size_t len, Tensor x) {
-    return i.run1(TensorOp::Slice, vals(std::move(x), dim, start, len));
+    return i.recorder ? i.run1(TensorOp::Slice, vals(std::move(x), dim, start, len)) : i.backend.slice(std::move(x), dim, start, len);
 }
 inline Tensor concat(I &i, size_t dim, Tensor x, Tensor y) {
-    return i.run1(TensorOp::Concat, vals(std::move(x), std::move(y), dim));
+    return i.recorder ? i.run1(TensorOp::Concat, vals(std::move(x), std::move(y), dim)) : i.backend.concat(std::move(x), std::move(y), dim);
 }
 inline Shape shape(const Tensor &x) { return x.shape(); }
 inline cg_dtype dtype(const Tensor &x) { return x.dtype(); }
 // stdlib/ops.rs:16-24: lit + broadcast
-inline Tensor lit(I &i, float v) { return i.run1(Op::scalar(v), vals()); }
-inline Tensor lit(I &i, uint32_t v) { return i.run1(Op::scalar(v), vals()); }
+inline Tensor lit(I &i, float v) { return i.recorder ? i.run1(Op::scalar(v), vals()) : i.backend.ndarray_from_vec_f32(&v, 1, Shape{}); }
+inline Tensor lit(I &i, uint32_t v) { return i.recorder ? i.run1(Op::scalar(v), vals()) : i.backend.ndarray_from_vec_u32(&v, 1, Shape{}); }
 inline Tensor constant(I &i, float v, const Shape &s) { return broadcast(i, s, lit(i, v)); }
 // stdlib/ops.rs:26-30
 inline Tensor inverse(I &i, Tensor x) {
