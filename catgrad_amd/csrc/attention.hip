@@ -44,20 +44,53 @@ static int64_t attn_seg_max() {
     return n;
 }
 
-template <class P, int LPT, int MM, int PASSES, bool LOOP>
-static int launch_seg_kernel(cg_backend *be, const AttnArgs &g, const FusedArgs &a, uint32_t batch) {
+template <class P, int LPT, int MM, int PASSES, bool LOOP, class Heads>
+static int launch_seg_kernel(cg_backend *be, const AttnArgs &g, const FusedArgs &a, uint32_t batch, const Heads &heads) {
     const size_t lds = seg_lds_bytes(MM, LPT * 4, g.chunk);
-    static const bool lds_ok = hipFuncSetAttribute(reinterpret_cast<const void *>(&decode_attention_seg_kernel<P, LPT, MM, PASSES, LOOP>),
+    static const bool lds_ok = hipFuncSetAttribute(reinterpret_cast<const void *>(&decode_attention_seg_kernel<P, LPT, MM, PASSES, LOOP, Heads>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize,
                                                    (int)seg_lds_bytes(MM, LPT * 4, kSegMaxChunk)) == hipSuccess;
     if (!lds_ok) return fail(CG_ERR_DEVICE, "decode attention: cannot reserve %zu bytes of LDS", seg_lds_bytes(MM, LPT * 4, kSegMaxChunk));
-    launch_kernel((decode_attention_seg_kernel<P, LPT, MM, PASSES, LOOP>), dim3(g.splits, batch), dim3(kSegBlock), lds, be->stream, g, a);
+    launch_kernel((decode_attention_seg_kernel<P, LPT, MM, PASSES, LOOP, Heads>), dim3(g.splits, batch), dim3(kSegBlock), lds, be->stream, g, a, heads);
     return CG_OK;
+}
+
+// The open heads as the attention g over a cache of T positions reads them: its q and the newest row of its K, no other products.
+static bool take_open_heads(const cg_backend *be, const AttnArgs &g, int64_t entries, RawHeads *raw) {
+    const OpenHeads *h = be->heads;
+    if (!h || h->count != 2) return false;
+    const uint32_t *const newest = g.Kc + (int64_t)(g.T - 1) * g.k_st;
+    const int q = h->p[0].to.dst == g.Q ? 0 : 1;
+    const OpenHeads::Product &pq = h->p[q], &pk = h->p[1 - q];
+    if (pq.to.dst != g.Q || pk.to.dst != newest || pq.to.hd != g.hd || pk.to.hd != g.hd || !pq.to.rope || !pk.to.rope) return false;
+    const int64_t seqs = h->rows, heads = pk.n / g.hd;
+    if (entries != seqs * heads || (int64_t)pq.n != heads * g.M * g.hd || (g.M > 1 && g.q_sm != pq.to.sh)) return false;
+    // the batch axes: the KV heads, then the sequences, or both as one axis
+    auto lies = [&](const OpenHeads::Product &p, const int64_t *step, int64_t per_head) {
+        const int64_t head = step[0], seq = g.nb == 2 ? step[1] : step[0] * heads;
+        if (g.nb == 0) return entries == 1;
+        if (g.nb == 1 && heads == 1) return seqs == 1 || step[0] == p.to.sb;
+        return (heads == 1 || head == per_head * p.to.sh) && (seqs == 1 || seq == p.to.sb);
+    };
+    if (g.nb > 2 || (g.nb == 2 && (g.bd[0] != heads || g.bd[1] != seqs))) return false;
+    if (!lies(pq, g.q_bs, g.M) || !lies(pk, g.k_bs, 1)) return false;
+    auto rows = [](const OpenHeads::Product &p) {
+        auto f = [](const uint32_t *w) { return reinterpret_cast<const float *>(w); };
+        return HeadRows{f(p.src), f(p.to.hgamma), f(p.to.cos), f(p.to.sin), p.n, p.to.hn_n_bits, p.to.hn_eps_bits, p.to.hn_exp_bits};
+    };
+    *raw = {rows(pq), rows(pk), make_fastdiv((uint32_t)heads)};
+    auto aligned = [](const HeadRows &r) {
+        for (const float *at : {r.src, r.gamma, r.cos, r.sin})
+            if (reinterpret_cast<uintptr_t>(at) % 16) return false;
+        return true;
+    };
+    return aligned(raw->q) && aligned(raw->k);
 }
 
 int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdims, int prank, const cg_tensor *q,
                             const cg_tensor *kt, const cg_tensor *v, cg_tensor *out) {
-    if (int frc = flush_deferred(be)) return frc;
+    if (!be->deferred.empty()) // (open heads may wait: see take_open_heads; where this declines, the next launch takes them along)
+        if (int frc = flush_deferred(be)) return frc;
     using P = WordsOnly<RowsSoftmaxCausal>; // (the scores of an open product are f32, and so is all that meets them)
     if (!be->aot || !program_matches<P>(p) || !p.leaf[0].lazy || p.leaf[0].lazy->result || p.reduced) return kDeclined;
     cg_tensor pd; // the soft-max result as a dense descriptor: the left operand of p.V
@@ -134,6 +167,10 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
     g.q_sm = f1.a_sm;
     g.k_st = f1.b_sn;
     g.v_st = f2.b_sk;
+    RawHeads raw;
+    const bool open = take_open_heads(be, g, f1.batch, &raw);
+    if (be->heads && !open)
+        if (int hrc = launch_open_heads(be)) return hrc;
     // One workgroup per query row: a cache of up to kRowMaxT positions in one launch with nothing to combine (beyond
     // 1024 positions only while the workgroups fit the compute units in one round: a row costs its compute unit
     // T x head_dim x 4 multiply-adds); longer caches in segments of at most kRowMaxT positions per workgroup, merged by the
@@ -191,12 +228,17 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
                     const bool one_trip = chunk <= 5 * tpb;
                     const uint32_t nb = (uint32_t)f1.batch;
 #define CG_SEG_KERNEL(LPT, MMV)                                                                    \
-        rc = one_trip ? launch_seg_kernel<P, LPT, MMV, 5, false>(be, g, a, nb) : launch_seg_kernel<P, LPT, MMV, 4, true>(be, g, a, nb)
-                    if (hd == 64 && g.M <= 4) CG_SEG_KERNEL(16, 4);
-                    else if (hd == 64) CG_SEG_KERNEL(16, 8);
-                    else if (g.M <= 4) CG_SEG_KERNEL(32, 4);
-                    else CG_SEG_KERNEL(32, 8);
+        rc = one_trip ? launch_seg_kernel<P, LPT, MMV, 5, false>(be, g, a, nb, heads) : launch_seg_kernel<P, LPT, MMV, 4, true>(be, g, a, nb, heads)
+                    auto launch = [&](const auto &heads) {
+                        if (hd == 64 && g.M <= 4) CG_SEG_KERNEL(16, 4);
+                        else if (hd == 64) CG_SEG_KERNEL(16, 8);
+                        else if (g.M <= 4) CG_SEG_KERNEL(32, 4);
+                        else CG_SEG_KERNEL(32, 8);
+                    };
 #undef CG_SEG_KERNEL
+                    if (open) launch(raw);
+                    else launch(NoHeads{});
+                    if (open && !rc) drop_open_heads(be);
                     if (!rc) {
                         const uint64_t nrows = (uint64_t)f1.batch * g.M;
                         launch_kernel(decode_attention_combine_kernel, dim3((uint32_t)nrows), dim3(kBlock), 0, be->stream, g.part_o, g.part_ml, static_cast<uint32_t *>(out->buf->ptr), g.splits, g.M,
@@ -221,6 +263,9 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
         const int64_t seglen = segmented ? ((T + nseg - 1) / nseg + 63) / 64 * 64 : T;
         g.chunk = (uint32_t)seglen;
         g.splits = (uint32_t)f1.batch; // (this kernel has no chunks: the field carries the number of batch entries)
+        const bool halves = qrows * nseg * 2 <= attn_row_halves_below(); // two workgroups per row still leave compute units idle
+        if (open && !halves) // (with whole rows of the output the registers don't hold an open head besides K and V)
+            if (int hrc = launch_open_heads(be)) return hrc;
         void *part_o = nullptr, *part_ml = nullptr;
         size_t co = 0, cml = 0;
         if (segmented) {
@@ -236,20 +281,29 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
         g.part_ml = static_cast<float *>(part_ml);
         const int64_t per_pass = hd == 64 ? kRowBlock / 16 : kRowBlock / 32;
         const int passes = seglen <= 5 * per_pass ? 5 : seglen <= 10 * per_pass ? 10 : seglen <= 16 * per_pass ? 16 : 0;
-        const bool halves = qrows * nseg * 2 <= attn_row_halves_below(); // two workgroups per row still leave compute units idle
         const dim3 grid((uint32_t)((f1.batch + 7) / 8 * 8 * g.M * (halves ? 2 : 1)), nseg), block(kRowBlock);
         g.groups = make_fastdiv(g.M * (halves ? 2 : 1));
 #define CG_ROW_KERNEL(LPT, VS)                                                                                                     \
     do {                                                                                                                           \
-        if (passes == 5) launch_kernel((decode_attention_row_kernel<P, LPT, 5, false, VS>), grid, block, 0, be->stream, g, a, po);   \
-        else if (passes == 10) launch_kernel((decode_attention_row_kernel<P, LPT, 10, false, VS>), grid, block, 0, be->stream, g, a, po); \
-        else if (passes == 16) launch_kernel((decode_attention_row_kernel<P, LPT, 16, false, VS>), grid, block, 0, be->stream, g, a, po); \
-        else launch_kernel((decode_attention_row_kernel<P, LPT, 6, true, VS>), grid, block, 0, be->stream, g, a, po);          \
+        if (passes == 5) launch_kernel((decode_attention_row_kernel<P, LPT, 5, false, VS, H>), grid, block, 0, be->stream, g, a, po, heads);   \
+        else if (passes == 10) launch_kernel((decode_attention_row_kernel<P, LPT, 10, false, VS, H>), grid, block, 0, be->stream, g, a, po, heads); \
+        else if (passes == 16) launch_kernel((decode_attention_row_kernel<P, LPT, 16, false, VS, H>), grid, block, 0, be->stream, g, a, po, heads); \
+        else launch_kernel((decode_attention_row_kernel<P, LPT, 6, true, VS, H>), grid, block, 0, be->stream, g, a, po, heads);          \
     } while (0)
-        if (hd == 64 && halves) CG_ROW_KERNEL(16, 2);
-        else if (hd == 64) CG_ROW_KERNEL(16, 1);
-        else if (halves) CG_ROW_KERNEL(32, 2);
-        else CG_ROW_KERNEL(32, 1);
+        if (open && halves) {
+            typedef RawHeads H;
+            const RawHeads &heads = raw;
+            if (hd == 64) CG_ROW_KERNEL(16, 2);
+            else CG_ROW_KERNEL(32, 2);
+            drop_open_heads(be);
+        } else {
+            typedef NoHeads H;
+            const NoHeads heads;
+            if (hd == 64 && halves) CG_ROW_KERNEL(16, 2);
+            else if (hd == 64) CG_ROW_KERNEL(16, 1);
+            else if (halves) CG_ROW_KERNEL(32, 2);
+            else CG_ROW_KERNEL(32, 1);
+        }
 #undef CG_ROW_KERNEL
         if (segmented) {
             const uint64_t nrows = (uint64_t)f1.batch * g.M;
@@ -260,6 +314,8 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
         hipError_t e = hipGetLastError();
         return e == hipSuccess ? CG_OK : hip_fail(e, "decode attention launch");
     }
+    if (open)
+        if (int hrc = launch_open_heads(be)) return hrc;
     const size_t o_bytes = (size_t)f1.batch * g.splits * g.M * hd * 4, ml_bytes = (size_t)f1.batch * g.splits * g.M * 2 * 4;
     void *po = nullptr, *pml = nullptr;
     size_t co = 0, cml = 0;

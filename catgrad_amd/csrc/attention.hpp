@@ -68,6 +68,50 @@ struct AttnArgs {
     FastDiv vbdiv[kMaxBatchAxes];
 };
 
+// q and the cache's newest row of K as the products left them (see OpenHeads): the kernels below apply the heads' RMS norm and the
+// rotary embedding themselves, op for op but for the order of the sum of squares, and store the results where the launch that they
+// save would have.  A wave finishes a row, behind the first loads of K, and the rows cross to the others through LDS.  The newest row's
+// score is taken from there: the cache does not hold that row until the launch ends (what is loaded in its place is not used).
+// head_norm_rope_finish_kernel takes 3.3 us and the hand-over behind it; here it hides behind K: Qwen3-0.6B's steps at 1050 positions
+// (8 KV heads of 128, 2 query heads each) 7.41 us with finished heads, 7.48 so.  (Every wave finishing the rows for itself: the
+// registers do not hold it all, 13.7.)
+struct NoHeads {};
+struct HeadRows { // of one product: HD columns a head, piece l of a row to lane l
+    const float *src, *gamma, *cos, *sin;
+    uint32_t n, n_bits, eps_bits, exp_bits; // n: columns of a row
+};
+struct RawHeads {
+    HeadRows q, k;
+    FastDiv heads; // KV heads: batch entry = sequence * heads + KV head
+};
+template <int LPT> struct OpenHead { // a wave's: a lane's piece of a row and the one that the embedding mixes it with, and the factors of both
+    float4v x, other, gamma, gamma_other, cos, sin;
+    __device__ __forceinline__ void load(const HeadRows &h, uint64_t row, uint32_t l) {
+        const uint32_t l2 = l ^ (LPT / 2);
+        auto piece = [](const float *p, uint32_t at) { return *reinterpret_cast<const float4v *>(p + at * 4); };
+        x = piece(h.src + row, l);
+        other = piece(h.src + row, l2);
+        gamma = piece(h.gamma, l);
+        gamma_other = piece(h.gamma, l2);
+        cos = piece(h.cos, l);
+        sin = piece(h.sin, l);
+    }
+    __device__ __forceinline__ float4v finish(const HeadRows &h, uint32_t l) const {
+        float ss = row16_sum(fmaf(x[3], x[3], fmaf(x[2], x[2], fmaf(x[1], x[1], x[0] * x[0]))));
+        if (LPT == 32) ss = asf(fold_rows(asu(ss), AddWords{}));
+        const uint32_t mean = apply<kAdd, true>(apply<kDiv, true>(asu(ss), h.n_bits, 0, nullptr), h.eps_bits, 0, nullptr);
+        // (a square root where the exponent is one half, as in every model's norms; the power where they differ)
+        const float r = h.exp_bits == 0x3F000000u && asf(mean) > 0.0f ? sqrtf(asf(mean)) : asf(apply<kPow, true>(mean, h.exp_bits, 0, nullptr));
+        float4v v;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float own = x[j] / r * gamma[j], mixed = other[j] / r * gamma_other[j];
+            v[j] = cos[j] * own + sin[j] * (l < LPT / 2 ? -mixed : mixed);
+        }
+        return v;
+    }
+};
+
 // Operand offsets of batch entry b, and its first row in the soft-max program's [rows, T] space.  Two axes are read without a test (as a
 // rule there are no more): a test in front of every axis is a trip to the argument block for every axis, a third of a microsecond each
 // before the first load of K goes out.
@@ -287,9 +331,10 @@ __global__ __launch_bounds__(kBlock) void decode_attention_kernel(const AttnArgs
 // units pull on V (used when the launch would otherwise leave half of them idle).
 constexpr int kRowBlock = 1024;
 constexpr int kRowMaxT = 4096;
-template <class P, int LPT, int PASSES, bool LOOP, int VS>
-__global__ __launch_bounds__(kRowBlock) void decode_attention_row_kernel(const AttnArgs g, const FusedArgs a, uint32_t *out) {
+template <class P, int LPT, int PASSES, bool LOOP, int VS, class Heads>
+__global__ __launch_bounds__(kRowBlock) void decode_attention_row_kernel(const AttnArgs g, const FusedArgs a, uint32_t *out, const Heads heads) {
     constexpr int HD = LPT * 4;
+    constexpr bool RAW = std::is_same<Heads, RawHeads>::value;
     constexpr int TPB = kRowBlock / LPT; // positions per pass
     constexpr int SPAN = TPB * PASSES;    // positions per trip to memory
     constexpr int LPV = LPT / VS;         // lanes per position in the V phase
@@ -336,7 +381,18 @@ __global__ __launch_bounds__(kRowBlock) void decode_attention_row_kernel(const A
     float4v ka[PASSES], kb[LOOP ? PASSES : 1];
     float4v va[PASSES_V], vb[LOOP ? PASSES_V : 1];
     // (loads come back in the order in which they are asked for: the query and K, the leaves, V)
-    const float4v qf = *reinterpret_cast<const float4v *>(g.Q + oq + (int64_t)m * g.q_sm + l * 4);
+    float4v qf;
+    const bool last = RAW && t_first + T == g.T; // this workgroup's positions end with the newest row
+    const uint32_t cached = T - last;
+    const uint32_t uwave = __builtin_amdgcn_readfirstlane(wave);
+    OpenHead<LPT> mine; // the first wave finishes q, the second the newest row
+    if constexpr (RAW) {
+        const uint32_t seq = fastdiv(b, heads.heads), head = b - seq * heads.heads.d;
+        if (uwave == 0) mine.load(heads.q, (uint64_t)seq * heads.q.n + (head * g.M + m) * HD, l);
+        else if (uwave == 1) mine.load(heads.k, (uint64_t)seq * heads.k.n + head * HD, l);
+    } else {
+        qf = *reinterpret_cast<const float4v *>(g.Q + oq + (int64_t)m * g.q_sm + l * 4);
+    }
     ask_k_at(ka, 0);
     // the soft-max program's other leaves at this thread's positions (tid, tid + 1024, ...)
     LeafWords<P, 1> w[IPL];
@@ -351,20 +407,41 @@ __global__ __launch_bounds__(kRowBlock) void decode_attention_row_kernel(const A
     if constexpr (V_EARLY) ask_v_at(va, 0);
 
     // ---- scores of the whole row
+    auto score_of = [&](const float4v &k) {
+        float v = fmaf(qf[3], k[3], fmaf(qf[2], k[2], fmaf(qf[1], k[1], qf[0] * k[0])));
+        v = row16_sum(v);
+        if (LPT == 32) v = asf(fold_rows(asu(v), AddWords{}));
+        return v;
+    };
+    if constexpr (RAW) {
+        float *const rows = &red[0][0]; // q, the newest row (red itself is needed behind the soft-max)
+        if (uwave < 2) {
+            const float4v v = mine.finish(uwave == 0 ? heads.q : heads.k, l);
+            if (lane < LPT) {
+                *reinterpret_cast<float4v *>(rows + uwave * HD + l * 4) = v;
+                uint32_t *const to = const_cast<uint32_t *>(uwave == 0 ? g.Q + oq + (int64_t)m * g.q_sm : g.Kc + ok + (int64_t)(g.T - 1) * g.k_st);
+                if (part == 0 && (uwave == 0 ? seg == 0 : last && m == 0)) *reinterpret_cast<float4v *>(to + l * 4) = v;
+            }
+        }
+        __syncthreads();
+        qf = *reinterpret_cast<const float4v *>(rows + l * 4);
+        if (last && uwave == 0) {
+            const float v = score_of(*reinterpret_cast<const float4v *>(rows + HD + l * 4));
+            if (lane == 0) sc[cached] = v;
+        }
+    }
     auto score = [&](const float4v (&f)[PASSES], uint32_t first, auto full) {
 #pragma unroll
         for (int ps = 0; ps < PASSES; ps++) {
             const uint32_t t = first + sub + ps * TPB;
-            if (decltype(full)::value || first + ps * TPB < T) { // the same for the whole workgroup
-                float v = fmaf(qf[3], f[ps][3], fmaf(qf[2], f[ps][2], fmaf(qf[1], f[ps][1], qf[0] * f[ps][0])));
-                v = row16_sum(v);
-                if (LPT == 32) v = asf(fold_rows(asu(v), AddWords{}));
-                if (l == 0 && (decltype(full)::value || t < T)) sc[t] = v;
+            if (decltype(full)::value || first + ps * TPB < cached) { // the same for the whole workgroup
+                const float v = score_of(f[ps]);
+                if (l == 0 && (decltype(full)::value || t < cached)) sc[t] = v;
             }
         }
     };
     auto score_at = [&](const float4v (&f)[PASSES], uint32_t first) {
-        if (first + SPAN <= T) score(f, first, whole_trip);
+        if (first + SPAN <= cached) score(f, first, whole_trip);
         else score(f, first, ragged);
     };
     if constexpr (LOOP) {
@@ -488,9 +565,10 @@ constexpr int kSegMaxChunk = 2048; // most positions per workgroup: their scores
 constexpr size_t seg_lds_bytes(int mm, int hd, uint32_t chunk) {
     return ((size_t)mm * ((chunk + 63) / 64 * 64) + (size_t)(kSegBlock / 64) * mm * hd) * sizeof(float);
 }
-template <class P, int LPT, int MM, int PASSES, bool LOOP>
-__global__ __launch_bounds__(kSegBlock) void decode_attention_seg_kernel(const AttnArgs g, const FusedArgs a) {
+template <class P, int LPT, int MM, int PASSES, bool LOOP, class Heads>
+__global__ __launch_bounds__(kSegBlock) void decode_attention_seg_kernel(const AttnArgs g, const FusedArgs a, const Heads heads) {
     constexpr int HD = LPT * 4;
+    constexpr bool RAW = std::is_same<Heads, RawHeads>::value;
     constexpr int TPB = kSegBlock / LPT; // positions per pass
     constexpr int SPAN = TPB * PASSES;    // positions per trip to memory
     constexpr int WAVES = kSegBlock / 64;
@@ -524,9 +602,19 @@ __global__ __launch_bounds__(kSegBlock) void decode_attention_seg_kernel(const A
     float4v ka[PASSES], kb[LOOP ? PASSES : 1];
     float4v va[PASSES], vb[LOOP ? PASSES : 1];
     float4v qf[MM];
+    const bool last = RAW && split + 1 == g.splits; // this segment ends with the newest row
+    const uint32_t cached = n - last;
+    const uint32_t uwave = __builtin_amdgcn_readfirstlane(wave);
+    OpenHead<LPT> mine; // a wave finishes a row of q each, the next one the newest row of K
+    if constexpr (RAW) {
+        const uint32_t seq = fastdiv(b, heads.heads), head = b - seq * heads.heads.d;
+        if (uwave < g.M) mine.load(heads.q, (uint64_t)seq * heads.q.n + (head * g.M + uwave) * HD, l);
+        else if (uwave == g.M) mine.load(heads.k, (uint64_t)seq * heads.k.n + head * HD, l);
+    } else {
 #pragma unroll
-    for (int m = 0; m < MM; m++) {
-        qf[m] = *reinterpret_cast<const float4v *>(g.Q + oq + (int64_t)min((uint32_t)m, g.M - 1) * g.q_sm + l * 4);
+        for (int m = 0; m < MM; m++) {
+            qf[m] = *reinterpret_cast<const float4v *>(g.Q + oq + (int64_t)min((uint32_t)m, g.M - 1) * g.q_sm + l * 4);
+        }
     }
     ask_k(ka, 0);
     // the soft-max phase gives a wave a query row (waves M.. have none); its lanes take positions lane, lane + 64, ...
@@ -540,26 +628,56 @@ __global__ __launch_bounds__(kSegBlock) void decode_attention_seg_kernel(const A
         ask_v(va, 0); // the whole segment is in flight: the registers hold both
     }
 
+
     // ---- scores of the segment, all rows of the group
+    auto score_of = [&](int m, const float4v &k) {
+        float v = fmaf(qf[m][3], k[3], fmaf(qf[m][2], k[2], fmaf(qf[m][1], k[1], qf[m][0] * k[0])));
+        v = row16_sum(v);
+        if (LPT == 32) v = asf(fold_rows(asu(v), AddWords{}));
+        return v;
+    };
+    if constexpr (RAW) {
+        static_assert(MM < WAVES, "a wave per row");
+        // (red is needed behind the soft-max: until then it holds the finished rows, K's behind q's)
+        if (uwave <= g.M) {
+            const float4v v = mine.finish(uwave < g.M ? heads.q : heads.k, l);
+            if (lane < LPT) {
+                *reinterpret_cast<float4v *>(red + uwave * HD + l * 4) = v;
+                uint32_t *const to = const_cast<uint32_t *>(uwave < g.M ? g.Q + oq + (int64_t)uwave * g.q_sm : g.Kc + ok + (int64_t)(g.T - 1) * g.k_st);
+                if (uwave < g.M ? split == 0 : last) *reinterpret_cast<float4v *>(to + l * 4) = v;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < MM; m++) qf[m] = *reinterpret_cast<const float4v *>(red + min((uint32_t)m, g.M - 1) * HD + l * 4);
+        if (last && uwave == 0) {
+            const float4v newest = *reinterpret_cast<const float4v *>(red + g.M * HD + l * 4);
+#pragma unroll
+            for (int m = 0; m < MM; m++) {
+                if ((uint32_t)m < g.M) {
+                    const float v = score_of(m, newest);
+                    if (lane == 0) sc[m * cap + cached] = v;
+                }
+            }
+        }
+    }
     auto score = [&](const float4v (&f)[PASSES], uint32_t first, auto full) {
 #pragma unroll
         for (int ps = 0; ps < PASSES; ps++) {
             const uint32_t t = first + sub + ps * TPB;
-            if (decltype(full)::value || first + ps * TPB < n) { // the same for the whole workgroup
+            if (decltype(full)::value || first + ps * TPB < cached) { // the same for the whole workgroup
 #pragma unroll
                 for (int m = 0; m < MM; m++) {
                     if ((uint32_t)m < g.M) {
-                        float v = fmaf(qf[m][3], f[ps][3], fmaf(qf[m][2], f[ps][2], fmaf(qf[m][1], f[ps][1], qf[m][0] * f[ps][0])));
-                        v = row16_sum(v);
-                        if (LPT == 32) v = asf(fold_rows(asu(v), AddWords{}));
-                        if (l == 0 && (decltype(full)::value || t < n)) sc[m * cap + t] = v;
+                        const float v = score_of(m, f[ps]);
+                        if (l == 0 && (decltype(full)::value || t < cached)) sc[m * cap + t] = v;
                     }
                 }
             }
         }
     };
     auto score_at = [&](const float4v (&f)[PASSES], uint32_t first) {
-        if (first + SPAN <= n) score(f, first, whole_trip);
+        if (first + SPAN <= cached) score(f, first, whole_trip);
         else score(f, first, ragged);
     };
     if constexpr (LOOP) {

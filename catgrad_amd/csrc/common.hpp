@@ -111,6 +111,7 @@ template <class T> struct Pooled {
 
 struct LazyMm;
 struct DeferredWrite;
+struct OpenHeads;
 struct DeferredStep;
 struct DeferredSum;
 struct Buffer;
@@ -152,6 +153,8 @@ struct cg_backend {
     std::string name;
     std::vector<cg::LazyMm *> lazy_open; // groupable lazy products not yet computed (not retained)
     std::vector<cg::DeferredWrite> deferred; // writes waiting to share a launch (see flush_deferred)
+    cg::OpenHeads *heads = nullptr;          // q and k of a decode step, their heads' norms not yet applied (owned)
+    bool keep_heads = false;                 // such heads may stay so: the caller puts the attention over them off
     cg::DeferredStep *step = nullptr;        // attention waiting for the next call, which may share its launch (blocks.hpp)
     cg::DeferredSum *sum = nullptr;          // the same of a sum of rows; never both
     int late_rc = 0;                         // what launching one of them has come to, for the next call that waits (the first error is kept)
@@ -646,9 +649,27 @@ struct RopeStore {
     uint32_t hn_n_bits, hn_eps_bits, hn_exp_bits;
 };
 // The products x . ys[i] (one row per batch entry, the same x) with such a store each; kDeclined when the shapes are not
-// the grouped kernel's.  nf as in launch_matmul_group.
+// the grouped kernel's.  nf as in launch_matmul_group.  Products with normed heads are left to be->heads.
 int launch_matmul_group_rope(cg_backend *be, const cg_tensor *x, const cg_tensor *const *ys, const RopeStore *stores, int n,
                              const NormFuse *nf);
+
+// Products whose heads are still to be normed (RopeStore::hgamma): their rows lie in scratch memory, n columns each.  The norm, the
+// embedding and the store run in decode-time attention as it loads q and the cache's newest row (take_open_heads in attention.hip) or,
+// when anything else is launched first, in a launch of their own (flush_deferred).
+struct OpenHeads {
+    struct Product {
+        RopeStore to;
+        const uint32_t *src;
+        uint32_t n;
+    };
+    uint32_t rows = 0, count = 0;
+    Product p[4];
+    void *scratch = nullptr;
+    size_t cls = 0;
+    std::vector<Buffer *> held; // what the stores read and write (retained)
+};
+int launch_open_heads(cg_backend *be); // be->heads in a launch of their own
+void drop_open_heads(cg_backend *be);  // be->heads are done with: to be called behind the launch that reads them
 
 // Decode-time attention in one pass: out = softmax-program(q . kT) . v, where `p` is the deferred
 // soft-max program whose leaf 0 is the (never computed) lazy product q . kT and (pdims, prank) its

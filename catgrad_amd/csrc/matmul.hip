@@ -1230,10 +1230,11 @@ template <bool WHOLE, int MM, int CG, int TRIPS> __global__ __launch_bounds__(kT
 }
 
 // The store above for products whose heads go through an RMS norm of their own first (RopeStore::hgamma, the q / k norm of
-// Qwen3): the norm needs the sum of squares over all hd columns of a head, which lie with hd / 8 workgroups of the
-// eight-columns-per-workgroup kernel, and workgroups cannot exchange values inside a launch for less than a launch costs.
-// So that kernel leaves those products plain (rows already divided by the input norm) in scratch memory, N columns a row,
-// and this small launch finishes them: a workgroup per head of a product, a thread per (row, column) of the head; the
+// Qwen3): the norm needs the sum of squares over all hd columns of a head, which lie with several workgroups of the
+// products' kernel, and workgroups cannot exchange values inside a launch for less than a launch costs.
+// So that kernel leaves those products plain (rows already divided by the input norm) in scratch memory, N columns a row.  Decode-time
+// attention finishes them as it loads them (see OpenHeads); where something else comes first or the attention is none of those kernels',
+// this small launch does: a workgroup per head of a product, a thread per (row, column) of the head; the
 // head's norm, the embedding and the store, op for op as the stand-alone programs (the sum of squares in runs of 16 columns).  A thread
 // norms its partner of the embedding as well, so that all loads go together and one barrier is enough: 4.8 -> 3.0 us for 24 heads
 // of 128 (3.5 in the steps of the Qwen3-0.6B shape, 16 and 8 heads).  Measured against one launch with a
@@ -1625,45 +1626,61 @@ int launch_matmul_group_rope(cg_backend *be, const cg_tensor *x, const cg_tensor
     g.in = skinny_input(first, nf);
     g.count = (uint32_t)n;
     ProfScope prof(be, CG_K_GEMM_SKINNY, bytes);
-    HeadFinish hf;
-    void *tmp = nullptr;
-    size_t tmp_cls = 0;
-    uint32_t finish_heads = 0, finish_hd = 0;
-    if (by_head) { // the normed products go to scratch memory as they are (see head_norm_rope_finish_kernel)
-        memset(&hf, 0, sizeof hf);
-        hf.M = first.M;
-        uint64_t words = 0;
-        for (int i = 0; i < n; i++)
-            if (stores[i].hgamma) words += (uint64_t)first.M * g.p[i].n;
-        if (int arc = be->pool.alloc(words * 4, &tmp, &tmp_cls)) return arc;
-        uint32_t *at = static_cast<uint32_t *>(tmp);
-        for (int i = 0; i < n; i++) {
-            if (!stores[i].hgamma) continue;
-            const uint32_t k = hf.n++;
-            SkinnyProduct &p = g.p[i]; // column n of row m to at[m * N + n]
-            hf.s[k] = stores[i];
-            hf.src[k] = at;
-            hf.N[k] = p.n;
-            finish_heads = std::max(finish_heads, p.n / stores[i].hd);
-            finish_hd = std::max(finish_hd, stores[i].hd);
-            p.dst = at;
-            p.sb = p.n;
-            p.sh = stores[i].hd;
-            p.rope = 0;
-            at += (uint64_t)first.M * p.n;
-        }
+    if (!by_head) return launch_skinny_group(be, g);
+    uint64_t words = 0; // the normed products go to scratch memory as they are
+    for (int i = 0; i < n; i++)
+        if (stores[i].hgamma) words += (uint64_t)first.M * g.p[i].n;
+    void *scratch = nullptr;
+    size_t cls = 0;
+    if (int arc = be->pool.alloc(words * 4, &scratch, &cls)) return arc;
+    OpenHeads *const heads = new OpenHeads;
+    heads->rows = first.M;
+    heads->scratch = scratch;
+    heads->cls = cls;
+    uint32_t *at = static_cast<uint32_t *>(scratch);
+    for (int i = 0; i < n; i++) {
+        if (!stores[i].hgamma) continue;
+        SkinnyProduct &p = g.p[i]; // column n of row m to at[m * N + n]
+        heads->p[heads->count++] = {stores[i], at, p.n};
+        p.dst = at;
+        p.sb = p.n;
+        p.sh = stores[i].hd;
+        p.rope = 0;
+        at += (uint64_t)first.M * p.n;
     }
-    int rc = launch_skinny_group(be, g);
-    if (by_head) {
-        const uint32_t threads = (hf.M * finish_hd + 63) / 64 * 64;
-        if (!rc) {
-            launch_kernel(head_norm_rope_finish_kernel, dim3(finish_heads, hf.n), dim3(threads), 0, be->stream, hf);
-            const hipError_t e = hipGetLastError();
-            if (e != hipSuccess) rc = hip_fail(e, "head norm launch");
-        }
-        be->pool.free(tmp, tmp_cls); // stream-ordered: later users queue behind the finishing launch
-    }
+    be->heads = heads;
+    const int rc = launch_skinny_group(be, g);
+    if (rc) drop_open_heads(be);
     return rc;
+}
+
+void drop_open_heads(cg_backend *be) {
+    OpenHeads *const h = be->heads;
+    be->heads = nullptr;
+    be->pool.free(h->scratch, h->cls); // stream-ordered: later users queue behind the launch that reads it
+    for (Buffer *b : h->held) buffer_release(b);
+    delete h;
+}
+
+int launch_open_heads(cg_backend *be) {
+    const OpenHeads &h = *be->heads;
+    HeadFinish f;
+    memset(&f, 0, sizeof f);
+    f.n = h.count;
+    f.M = h.rows;
+    uint32_t heads = 0, hd = 0;
+    for (uint32_t i = 0; i < h.count; i++) {
+        f.s[i] = h.p[i].to;
+        f.src[i] = h.p[i].src;
+        f.N[i] = h.p[i].n;
+        heads = std::max(heads, h.p[i].n / h.p[i].to.hd);
+        hd = std::max(hd, h.p[i].to.hd);
+    }
+    ProfScope prof(be, CG_K_GEMM_SKINNY, 8.0 * f.M * heads * hd * f.n);
+    launch_kernel(head_norm_rope_finish_kernel, dim3(heads, f.n), dim3((f.M * hd + 63) / 64 * 64), 0, be->stream, f);
+    const hipError_t e = hipGetLastError();
+    drop_open_heads(be);
+    return e == hipSuccess ? CG_OK : hip_fail(e, "head norm launch");
 }
 
 // out = g * (1 / (one + exp(-g))) * u with g = x.yg, u = x.yu: two decode-time linear layers and

@@ -1368,17 +1368,33 @@ static int try_rope_stores(cg_backend *be, std::vector<DeferredWrite> &w, const 
     h.buf = nullptr;
     if (rc) return rc;
     be->programs_compiled++;
+    if (be->heads) { // the buffers outlive the programs
+        auto hold = [&](Buffer *b) {
+            b->rc.fetch_add(1);
+            be->heads->held.push_back(b);
+        };
+        for (int i = 0; i < n; i++) {
+            if (!ms[i]->head_norm) continue;
+            hold(w[i].dst->buf);
+            hold(ms[i]->hn_gamma);
+            for (int l = 0; l < w[i].prog->nleaf; l++)
+                if (w[i].prog->leaf[l].buf) hold(w[i].prog->leaf[l].buf);
+        }
+    }
     for (int i = 0; i < n; i++) lazy_mm_close(ms[i]); // they go away with the programs, never computed on their own
     return CG_OK;
 }
 
 int flush_deferred(cg_backend *be, const Pending *also) {
+    if (be->heads)
+        if (int hrc = launch_open_heads(be)) return hrc; // (older than the writes)
     if (be->deferred.empty()) return CG_OK;
     std::vector<DeferredWrite> w;
     w.swap(be->deferred); // the launches below come back here and find nothing to do
     int rc = try_rope_stores(be, w, also);
     if (rc != kDeclined) {
         for (DeferredWrite &d : w) drop_deferred(d);
+        if (!rc && be->heads && !be->keep_heads) rc = launch_open_heads(be);
         return rc;
     }
     rc = CG_OK;
@@ -2325,6 +2341,7 @@ void cg_backend_destroy(cg_backend *b) {
         (void)hipSetDevice(b->device);
         for (DeferredWrite &d : b->deferred) drop_deferred(d); // nobody can read them any more
         b->deferred.clear();
+        if (b->heads) drop_open_heads(b);
         const_memo_clear(b);
         (void)hipStreamSynchronize(b->stream);
         prof_drain(b);
@@ -3030,7 +3047,12 @@ static int matmul_entry(cg_backend *b, cg_tensor *x, cg_tensor *y, cg_tensor **o
         norm_x = norm_fuse_of(x, &nfx, &hx);
         hx.buf = nullptr;
     }
-    if (!norm_x && (x->pend || x->split >= r - 2)) rc = ensure_concrete(x);
+    if (!norm_x && (x->pend || x->split >= r - 2)) {
+        // (decode-time q for a product that is put off below: the attention which absorbs that can finish q's heads)
+        b->keep_heads = b->fuse && b->aot && r == 4 && x->dims[r - 2] <= 8 && (x->dims[r - 1] == 64 || x->dims[r - 1] == 128);
+        rc = ensure_concrete(x);
+        b->keep_heads = false;
+    }
     if (!rc && (y->pend || y->split >= r - 2)) rc = ensure_concrete(y);
     if (!rc && x->split >= 0 && y->split >= 0 && (x->split != y->split || x->split_inner != y->split_inner))
         rc = ensure_concrete(y);
