@@ -1,7 +1,7 @@
 // The delta rule with a state that decays channel by channel (cg_block_channel_delta).
 //
 // A few new tokens (a decode step): delta_step_kernel, a workgroup per (sequence, head) that does everything from the
-// convolutions to the gated norm, the state in registers from the first token to the last.
+// convolutions to the gated norm, the state in registers from the first token to the last; delta_token_kernel for one token.
 //
 // More: chunks of 16 tokens.  With G_t the sum of the logarithms of the decays from the chunk's start to token t (per key
 // channel), S_0 the state before the chunk and S the one behind it,
@@ -464,62 +464,17 @@ template <int TAPS> __device__ __forceinline__ float conv_step(const DeltaPlan &
     }
 }
 
-// A lane's quarter of w . x for up to kDotQuads * 16 values of k, 16 bytes at a time: asked for, and added up over its quad of lanes
-constexpr int kDotQuads = 8;
-struct DotLoads {
-    float4 a[kDotQuads], c[kDotQuads];
-    // (w and x: the same for all lanes, so that a lane's addresses are 32-bit offsets)
-    __device__ __forceinline__ void ask(const float *__restrict__ w, uint32_t row, const float *__restrict__ x, uint32_t n, uint32_t sub) {
-#pragma unroll
-        for (int j = 0; j < kDotQuads; j++) {
-            const uint32_t at = min(sub + 4 * j, n / 4 - 1);
-            a[j] = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(w) + (row * n + at * 4) * 4);
-            c[j] = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(x) + at * 16);
-        }
-    }
-    __device__ __forceinline__ float value(uint32_t n, uint32_t sub) const {
-        float s = 0.0f;
-#pragma unroll
-        for (int j = 0; j < kDotQuads; j++) {
-            const float t = fmaf(a[j].x, c[j].x, fmaf(a[j].y, c[j].y, fmaf(a[j].z, c[j].z, a[j].w * c[j].w)));
-            s += sub + 4 * j < n / 4 ? t : 0.0f;
-        }
-        return add_across<2>(add_across<1>(s));
-    }
-};
-
-// Thread (c, group) holds rows group, group + groups, ... (at most R) of column c of the head's state.
-// DIRECT: one token behind a state; a thread has at most one channel of the convolutions and a row of each factored projection, and these have ranks of at
-// most 128 in 16-byte pieces (launch_delta_step).  Then all of a token's loads are asked for together, and ahead of the state, whose
-// 64 KB for 128 x 128 a compute unit takes 2 us to fetch: nothing of the token waits for it.  One after the other: 14.9 us, 13.1 so
-// (what is left is mostly the state and the factors, 200 KB through one compute unit).
-template <int R, int TAPS, bool DIRECT> __global__ __launch_bounds__(kStepThreads) void delta_step_kernel(const DeltaPlan p, const uint32_t lanes) {
+// Thread (c, group) holds rows group, group + groups, ... (at most R) of column c of the head's state.  (One token's loads together and
+// ahead of the state, as in delta_token_kernel, cost two tokens 2.9 us: 21.9 so, 19.0 without.)
+template <int R, int TAPS> __global__ __launch_bounds__(kStepThreads) void delta_step_kernel(const DeltaPlan p, const uint32_t lanes) {
     __shared__ float q[257], k[257], g[257], v[kStepThreads], gate[kStepThreads], part[kStepThreads], red[kStepThreads / 64];
     __shared__ float2 red2[kStepThreads / 64];
     const uint32_t h = blockIdx.x, b = blockIdx.y, rep = p.heads / p.kv_heads, kh = h / rep, D = p.dim, V = p.vdim, kc = p.kv_heads * D;
     const uint32_t tid = threadIdx.x, c = tid & (lanes - 1), group = tid / lanes, groups = kStepThreads / lanes;
     const int64_t sb = ((int64_t)b * p.heads + h) * D * V;
     constexpr uint32_t ROWS = kStepThreads / 4; // rows of the factored projections per round
-    ConvLoads<TAPS ? TAPS : 1, true> conv;
-    DotLoads dot[DIRECT ? 2 : 1];
-    auto channel_of = [&](uint32_t u) { return u < D ? kh * D + u : u < 2 * D ? kc + kh * D + u - D : 2 * kc + h * V + u - 2 * D; };
-    auto ask = [&](uint32_t t) {
-        const int64_t r = (int64_t)b * p.S + t;
-        conv.ask(p, b, (int)t, channel_of(min(tid, 2 * D + V - 1)));
-        dot[0].ask(p.decay_w + (int64_t)h * D * p.decay_rank, min(tid / 4, D - 1), p.decay.p + r * p.decay.pitch, p.decay_rank, tid & 3);
-        dot[DIRECT].ask(p.gate_w + (int64_t)h * V * p.gate_rank, min(tid / 4, V - 1), p.gate.p + r * p.gate.pitch, p.gate_rank, tid & 3);
-    };
-    float dt_bias = 0.0f, a_log = 0.0f, beta_in = 0.0f, weight = 0.0f;
-    if constexpr (DIRECT) {
-        ask(0);
-        a_log = p.a_log[h];
-        dt_bias = p.dt_bias[h * D + min(tid / 4, D - 1)];
-        beta_in = p.beta.p[(int64_t)b * p.beta.pitch + h];
-        weight = p.norm[min(c, V - 1)];
-        __builtin_amdgcn_sched_barrier(0);
-    }
     float S[R];
-    if (DIRECT || p.state) { // (clamped, not tested: no load waits)
+    if (p.state) { // (clamped, not tested: no load waits)
         const char *const src = reinterpret_cast<const char *>(p.state + sb);
         const uint32_t col = min(c, V - 1);
 #pragma unroll
@@ -529,21 +484,9 @@ template <int R, int TAPS, bool DIRECT> __global__ __launch_bounds__(kStepThread
         for (int i = 0; i < R; i++) S[i] = 0.0f;
     }
     if (tid == 0) q[D] = k[D] = g[D] = 0.0f; // what the rows behind the last one read
-    for (uint32_t t = 0; t < (DIRECT ? 1 : p.S); t++) {
+    for (uint32_t t = 0; t < p.S; t++) {
         const int64_t r = (int64_t)b * p.S + t;
         float sq = 0.0f, sk = 0.0f;
-        if constexpr (DIRECT) {
-            const float x = conv.value(p, (int)t);
-            if (tid < 2 * D + V) {
-                (tid < D ? q[tid] : tid < 2 * D ? k[tid - D] : v[tid - 2 * D]) = x;
-                sq = tid < D ? x * x : 0.0f;
-                sk = tid >= D && tid < 2 * D ? x * x : 0.0f;
-            }
-            const uint32_t e = tid / 4;
-            const float decay = dot[0].value(p.decay_rank, tid & 3), open = dot[DIRECT].value(p.gate_rank, tid & 3);
-            if ((tid & 3) == 0 && e < D) g[e] = exp2_of(log2_decay(a_log, decay + dt_bias));
-            if ((tid & 3) == 0 && e < V) gate[e] = sigmoid(open);
-        } else
         for (uint32_t u = tid; u < 2 * D + V; u += kStepThreads) {
             const bool is_q = u < D, is_k = !is_q && u < 2 * D;
             const uint32_t e = is_q ? u : is_k ? u - D : u - 2 * D;
@@ -552,7 +495,7 @@ template <int R, int TAPS, bool DIRECT> __global__ __launch_bounds__(kStepThread
             sk = is_k ? fmaf(x, x, sk) : sk;
             (is_q ? q : is_k ? k : v)[e] = x;
         }
-        for (uint32_t u = tid / 4; !DIRECT && u < D + V; u += ROWS) { // the two factored projections
+        for (uint32_t u = tid / 4; u < D + V; u += ROWS) { // the two factored projections
             const bool is_g = u < D;
             const uint32_t e = is_g ? u : u - D;
             const float a = quad_dot(is_g ? p.decay_w + ((int64_t)h * D + e) * p.decay_rank : p.gate_w + ((int64_t)h * V + e) * p.gate_rank,
@@ -563,11 +506,11 @@ template <int R, int TAPS, bool DIRECT> __global__ __launch_bounds__(kStepThread
             }
         }
         step_sum2(sq, sk, red2);
-        if (DIRECT || t == 0) // rows behind the last one hold what the clamped loads brought
+        if (t == 0) // rows behind the last one hold what the clamped loads brought
 #pragma unroll
             for (int i = 0; i < R; i++) S[i] = group + i * groups < D ? S[i] : 0.0f;
         const float fq = 1.0f / sqrtf(sq + 1e-6f) * (1.0f / sqrtf((float)D)), fk = 1.0f / sqrtf(sk + 1e-6f);
-        const float beta = sigmoid(DIRECT ? beta_in : p.beta.p[r * p.beta.pitch + h]);
+        const float beta = sigmoid(p.beta.p[r * p.beta.pitch + h]);
         float read = 0.0f; // (the sums above end behind a barrier: q, k, v, g and gate are there)
 #pragma unroll
         for (int i = 0; i < R; i++) {
@@ -594,14 +537,163 @@ template <int R, int TAPS, bool DIRECT> __global__ __launch_bounds__(kStepThread
         if (group == 0)
             for (uint32_t i = 0; i < groups; i++) y += part[i * lanes + c];
         const float f = 1.0f / sqrtf(step_sum(group == 0 && c < V ? y * y : 0.0f, red) / (float)V + p.eps);
-        if (group == 0 && c < V) p.out[r * p.heads * V + h * V + c] = y * f * (DIRECT ? weight : p.norm[c]) * gate[c];
-        if (!DIRECT) __syncthreads(); // the next token overwrites what this one reads
+        if (group == 0 && c < V) p.out[r * p.heads * V + h * V + c] = y * f * p.norm[c] * gate[c];
+        __syncthreads(); // the next token overwrites what this one reads
     }
     keep_inputs(p, b, h);
 #pragma unroll
     for (int i = 0; i < R; i++) {
         const uint32_t d = group + i * groups;
         if (d < D && c < V) p.state_out[sb + (int64_t)d * V + c] = S[i];
+    }
+}
+
+// One token behind a state of at most 128 x 128, V a multiple of 4: a workgroup per (sequence, head), which reads 130 KB of state and
+// factors and writes 64.  A compute unit takes 2 us to fetch and store these, so everything is asked for at the start, the
+// token's inputs ahead of the state, and what lies behind is kept short: a thread holds R rows of four columns (16 bytes to a load, a
+// quarter of the reads of g, k and q from LDS), both of the state's products are taken before it is written, in one pass,
+//     q . S' = q . (g S) + (q . k) u,   u = beta (v - k . (g S)),
+// so that two barriers are enough, either factored projection has four waves to itself (one vector to fetch, not two), and the
+// convolutions' inputs are kept from the registers that hold them.  Heads of 128 x 128, 32-bit steps behind 777 tokens of a model of
+// width 1024: 12.5 us before (a column a thread, a pass and four barriers more), 6.2 so.
+constexpr uint32_t kTokenDim = 128;
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef f4 f4_words __attribute__((aligned(4))); // from any word's address
+// LV: lanes side by side on a row of the state (V at most 4 LV).  Q: 16-byte pieces of the factors' rows to a lane, four lanes to a row.
+template <int LV, int Q> __global__ __launch_bounds__(kStepThreads) void delta_token_kernel(const DeltaPlan p) {
+    constexpr int WAVES = kStepThreads / 64, GROUPS = kStepThreads / LV, R = kTokenDim / GROUPS, HALF = kStepThreads / 2;
+    static_assert(R % 4 == 0 && (LV == 32 || LV == 16), "rows in fours, whole or half waves' rows");
+    __shared__ __attribute__((aligned(16))) float q[kTokenDim], k[kTokenDim], g[kTokenDim], v[kTokenDim], gate[kTokenDim], part[WAVES][2][LV][4], part_qk[WAVES];
+    __shared__ float2 red[WAVES];
+    const uint32_t h = blockIdx.x, b = blockIdx.y, rep = p.heads / p.kv_heads, kh = h / rep, D = p.dim, V = p.vdim, kc = p.kv_heads * D, C = 2 * kc + p.heads * V;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid / 64), c = tid % LV, d0 = tid / LV * R;
+    const int64_t sb = ((int64_t)b * p.heads + h) * D * V;
+    // ---- the token's inputs
+    const bool has_channel = tid < 2 * D + V;
+    const uint32_t u0 = min(tid, 2 * D + V - 1), ch = u0 < D ? kh * D + u0 : u0 < 2 * D ? kc + kh * D + u0 - D : 2 * kc + h * V + u0 - 2 * D;
+    ConvLoads<4, true> conv;
+    conv.ask(p, b, 0, ch);
+    const bool is_gate = wave >= WAVES / 2;
+    const uint32_t n = is_gate ? p.gate_rank : p.decay_rank, rows = is_gate ? V : D, sub = tid & 3, e0 = tid % HALF / 4;
+    const float *const w = is_gate ? p.gate_w + (int64_t)h * V * n : p.decay_w + (int64_t)h * D * n;
+    const float *const x = is_gate ? p.gate.p + (int64_t)b * p.gate.pitch : p.decay.p + (int64_t)b * p.decay.pitch;
+    f4 in[Q], factor[2][Q];
+#pragma unroll
+    for (int j = 0; j < Q; j++) {
+        const uint32_t at = min(sub + 4 * j, n / 4 - 1); // (clamped, not tested: no load waits)
+        in[j] = *reinterpret_cast<const f4 *>(reinterpret_cast<const char *>(x) + at * 16);
+#pragma unroll
+        for (uint32_t i = 0; i < 2; i++) factor[i][j] = *reinterpret_cast<const f4 *>(reinterpret_cast<const char *>(w) + (min(e0 + i * (HALF / 4), rows - 1) * n + at * 4) * 4);
+    }
+    float dt_bias[2];
+#pragma unroll
+    for (uint32_t i = 0; i < 2; i++) dt_bias[i] = p.dt_bias[h * D + min(e0 + i * (HALF / 4), D - 1)];
+    const float a_log = p.a_log[h], beta_in = p.beta.p[(int64_t)b * p.beta.pitch + h];
+    const uint32_t col = min(4 * c, V - 4);
+    const f4 weight = *reinterpret_cast<const f4_words *>(p.norm + col);
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- the state
+    f4 S[R];
+    const char *const src = reinterpret_cast<const char *>(p.state + sb);
+#pragma unroll
+    for (uint32_t i = 0; i < R; i++) S[i] = *reinterpret_cast<const f4 *>(src + (min(d0 + i, D - 1) * V + col) * 4);
+    __builtin_amdgcn_sched_barrier(0); // (what follows stays behind all of the loads)
+
+    if (tid >= D && tid < kTokenDim) q[tid] = k[tid] = g[tid] = 0.0f;
+    const float y_conv = conv.value(p, 0);
+    if (has_channel) (tid < D ? q[tid] : tid < 2 * D ? k[tid - D] : v[tid - 2 * D]) = y_conv;
+    const float sq = wave_add<1>(tid < D ? y_conv * y_conv : 0.0f), sk = wave_add<1>(tid >= D && tid < 2 * D ? y_conv * y_conv : 0.0f);
+    if (lane == 0) red[wave] = make_float2(sq, sk);
+#pragma unroll
+    for (uint32_t i = 0; i < 2; i++) {
+        float s = 0.0f;
+#pragma unroll
+        for (int j = 0; j < Q; j++) {
+            const float t = fmaf(factor[i][j][0], in[j][0], fmaf(factor[i][j][1], in[j][1], fmaf(factor[i][j][2], in[j][2], factor[i][j][3] * in[j][3])));
+            s += sub + 4 * j < n / 4 ? t : 0.0f;
+        }
+        s = add_across<2>(add_across<1>(s));
+        const uint32_t e = e0 + i * (HALF / 4);
+        if (sub == 0 && e < rows) (is_gate ? gate : g)[e] = is_gate ? sigmoid(s) : exp2_of(log2_decay(a_log, s + dt_bias[i]));
+    }
+    if (has_channel && (h % rep == 0 || tid >= 2 * D)) { // the inputs that the next token's convolutions need
+        float *const keep = p.conv_out + (int64_t)b * 3 * C + ch;
+#pragma unroll
+        for (int j = 0; j < 3; j++) keep[(int64_t)j * C] = j == 2 || p.conv_state ? conv.x[j + 1] : 0.0f;
+    }
+    __syncthreads();
+    float nq = 0.0f, nk = 0.0f;
+#pragma unroll
+    for (int i = 0; i < WAVES; i++) nq += red[i].x, nk += red[i].y;
+    const float fq = 1.0f / sqrtf(nq + 1e-6f) * (1.0f / sqrtf((float)D)), fk = 1.0f / sqrtf(nk + 1e-6f), beta = sigmoid(beta_in);
+    float kk[R], qk = 0.0f;
+    f4 read = {}, out = {};
+#pragma unroll
+    for (int i0 = 0; i0 < R; i0 += 4) {
+        const f4 k4 = *reinterpret_cast<const f4 *>(k + d0 + i0), q4 = *reinterpret_cast<const f4 *>(q + d0 + i0), g4 = *reinterpret_cast<const f4 *>(g + d0 + i0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const bool there = d0 + i0 + i < D; // rows behind the last one hold what the clamped loads brought
+            const float qq = q4[i] * fq;
+            kk[i0 + i] = k4[i] * fk;
+            qk = fmaf(qq, kk[i0 + i], qk);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float s = there ? S[i0 + i][j] * g4[i] : 0.0f;
+                S[i0 + i][j] = s;
+                read[j] = fmaf(s, kk[i0 + i], read[j]);
+                out[j] = fmaf(s, qq, out[j]);
+            }
+        }
+    }
+    // over the wave's rows: q's sums to the lower half of its lanes, k's to the upper half
+    f4 both;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const auto halves = __builtin_amdgcn_permlane32_swap(asu(out[j]), asu(read[j]), false, false);
+        both[j] = asf((uint32_t)halves[0]) + asf((uint32_t)halves[1]);
+        if constexpr (LV == 16) both[j] = asf(fold_rows(asu(both[j]), AddWords{}));
+    }
+    const auto halves = __builtin_amdgcn_permlane32_swap(asu(qk), asu(qk), false, false);
+    qk = asf((uint32_t)halves[0]) + asf((uint32_t)halves[1]);
+    if constexpr (LV == 16) qk = asf(fold_rows(asu(qk), AddWords{}));
+    if (lane % 32 < LV) *reinterpret_cast<f4 *>(part[wave][lane / 32][c]) = both;
+    if (lane == 0) part_qk[wave] = qk;
+    __syncthreads();
+    const bool column = 4 * c < V;
+    f4 u = {};
+#pragma unroll
+    for (int i = 0; i < WAVES; i++) u += *reinterpret_cast<const f4 *>(part[i][1][c]);
+    const f4 v4 = *reinterpret_cast<const f4 *>(v + col);
+#pragma unroll
+    for (int j = 0; j < 4; j++) u[j] = column ? beta * (v4[j] - u[j]) : 0.0f;
+    if (wave == 0) { // (a wave for the norm and the gate)
+        f4 y = {};
+        float sum = 0.0f;
+        qk = 0.0f;
+#pragma unroll
+        for (int i = 0; i < WAVES; i++) {
+            y += *reinterpret_cast<const f4 *>(part[i][0][c]);
+            qk += part_qk[i];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            y[j] = fmaf(qk, u[j], y[j]);
+            sum = fmaf(y[j], y[j], sum);
+        }
+        const bool stores = column && lane < LV;
+        const float f = 1.0f / sqrtf(wave_add<1>(stores ? sum : 0.0f) / (float)V + p.eps);
+        const f4 open = *reinterpret_cast<const f4 *>(gate + col);
+#pragma unroll
+        for (int j = 0; j < 4; j++) y[j] = y[j] * f * weight[j] * open[j];
+        if (stores) *reinterpret_cast<f4 *>(p.out + ((int64_t)b * p.heads + h) * V + col) = y;
+    }
+    char *const dst = reinterpret_cast<char *>(p.state_out + sb);
+#pragma unroll
+    for (uint32_t i = 0; i < R; i++) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) S[i][j] = fmaf(kk[i], u[j], S[i][j]);
+        if (column && d0 + i < D) *reinterpret_cast<f4 *>(dst + ((d0 + i) * V + col) * 4) = S[i];
     }
 }
 
@@ -688,6 +780,14 @@ bool step_shape(const DeltaPlan &p, uint32_t *lanes, uint32_t *rows) {
     return *rows <= 64;
 }
 
+// What delta_token_kernel is written for: all that it loads in 16-byte pieces lies in such.
+bool takes_token(const DeltaPlan &p) {
+    auto aligned = [](const float *at) { return (reinterpret_cast<uintptr_t>(at) & 15) == 0; };
+    auto pieces = [&](const float *w, uint32_t rank, const Rows &x) { return rank >= 4 && rank <= 128 && rank % 4 == 0 && x.pitch % 4 == 0 && aligned(w) && aligned(x.p); };
+    return p.S == 1 && p.state && p.taps == 4 && p.dim <= kTokenDim && p.vdim <= kTokenDim && p.vdim % 4 == 0 && aligned(p.state) && pieces(p.decay_w, p.decay_rank, p.decay) &&
+           pieces(p.gate_w, p.gate_rank, p.gate);
+}
+
 template <int TPW, int CT> int scan(cg_backend *be, const DeltaPlan &p, const ChunkArrays &a, const float *state) {
     const size_t lds = (size_t)(2 * chunk_lds_floats(64 * TPW) + CT * 4 * 2 * 64 * 4) * 4;
     if (lds > (64 << 10)) {
@@ -715,22 +815,22 @@ int launch_channel_delta(cg_backend *be, const DeltaPlan &p) {
     if (step_shape(p, &lanes, &held)) {
         ProfScope prof(be, CG_K_RECURRENCE, flop * rows);
         const dim3 grid(p.heads, p.B);
-        auto pieces = [](const float *w, uint32_t rank, const Rows &x) {
-            return rank >= 4 && rank <= 16 * kDotQuads && rank % 4 == 0 && x.pitch % 4 == 0 && ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x.p)) & 15) == 0;
-        };
-        const bool direct = p.S == 1 && p.state && p.taps == 4 && 2 * p.dim + p.vdim <= kStepThreads && p.dim <= kStepThreads / 4 && p.vdim <= kStepThreads / 4 && pieces(p.decay_w, p.decay_rank, p.decay) &&
-                            pieces(p.gate_w, p.gate_rank, p.gate);
-#define CG_STEP(R, DIRECT)                                                                                                                \
-    if (DIRECT) launch_kernel((delta_step_kernel<R, 4, DIRECT>), grid, dim3(kStepThreads), 0, be->stream, p, lanes);                \
-    else if (p.taps == 4) launch_kernel((delta_step_kernel<R, 4, false>), grid, dim3(kStepThreads), 0, be->stream, p, lanes);       \
-    else launch_kernel((delta_step_kernel<R, 0, false>), grid, dim3(kStepThreads), 0, be->stream, p, lanes)
-        if (direct && held <= 4) { CG_STEP(4, true); }
-        else if (direct && held <= 16) { CG_STEP(16, true); }
-        else if (direct) { CG_STEP(32, true); } // (128 rows by four groups)
-        else if (held <= 4) { CG_STEP(4, false); }
-        else if (held <= 16) { CG_STEP(16, false); }
-        else if (held <= 32) { CG_STEP(32, false); }
-        else { CG_STEP(64, false); }
+        if (takes_token(p)) {
+            auto token = [&](auto kernel) { launch_kernel(kernel, grid, dim3(kStepThreads), 0, be->stream, p); };
+            const bool short_rows = std::max(p.decay_rank, p.gate_rank) <= 64;
+            if (p.vdim > 64 && short_rows) token(delta_token_kernel<32, 4>);
+            else if (p.vdim > 64) token(delta_token_kernel<32, 8>);
+            else if (short_rows) token(delta_token_kernel<16, 4>);
+            else token(delta_token_kernel<16, 8>);
+            return launched("channel_delta token");
+        }
+#define CG_STEP(R)                                                                                                                \
+    if (p.taps == 4) launch_kernel((delta_step_kernel<R, 4>), grid, dim3(kStepThreads), 0, be->stream, p, lanes);       \
+    else launch_kernel((delta_step_kernel<R, 0>), grid, dim3(kStepThreads), 0, be->stream, p, lanes)
+        if (held <= 4) { CG_STEP(4); }
+        else if (held <= 16) { CG_STEP(16); }
+        else if (held <= 32) { CG_STEP(32); }
+        else { CG_STEP(64); }
 #undef CG_STEP
         return launched("channel_delta step");
     }
