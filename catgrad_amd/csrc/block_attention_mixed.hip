@@ -410,6 +410,11 @@ __global__ __launch_bounds__(kTileWaves * 64) void attention_mixed_tiles_kernel(
 // Keys are taken in chunks of `chunk`, a workgroup takes `chunks` of them.  Their keys and values are asked for first and
 // arrive while the queries are prepared: four lanes share a key of a kv head (PI such keys per four lanes, DQ 16-byte pieces
 // per lane), a thread has four columns of a kv head's values (for every turns-th key of the chunk).
+// A workgroup's chain of loads, short sums and barriers is what a step takes, the last segment's above all, which has the new key to
+// prepare: so all loads are asked for before anything waits (both tables of the rotation and the new key among them), the new values are
+// stored from the registers that weigh them, heads take sixteen bytes a lane, so that two of 128 share a wave and no pair of the
+// rotation crosses lanes, and nothing divides (StepDivs).  330 positions, 16 heads of 128 beside 8 of 32 experts of 384 x 1024 in bfloat16: 11.9 us
+// with the parts after one another and three workgroups a compute unit, whose registers did not hold the values on their way; 8.1 so.
 constexpr uint32_t kMaxChunk = 64, kValuesAhead = 8;
 struct StepLds { // floats
     uint32_t q, fresh, talk, raw, mixed, state, total;
@@ -434,20 +439,20 @@ __host__ __device__ inline StepLds step_lds(uint32_t S, uint32_t heads, uint32_t
 }
 
 template <int REP, int DQ, int PI>
-__device__ __forceinline__ void mixed_step(const AttentionPlan &p, const uint32_t chunk, const uint32_t chunks, float *__restrict__ parts, float2 *__restrict__ stats, const uint32_t seg,
+__device__ __forceinline__ void mixed_step(const AttentionPlan &p, const StepDivs &divs, const uint32_t chunk, const uint32_t chunks, float *__restrict__ parts, float2 *__restrict__ stats, const uint32_t seg,
                                            const uint32_t nseg, const uint32_t r, float *const lds) {
-    const uint32_t rep = p.heads / p.kv_heads, b = r / p.S, s = r - b * p.S;
-    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63, pitch = chunk + 1, sub = threadIdx.x & 3;
+    const uint32_t vec = p.vdim / 4, cols = p.kv_heads * vec, rep = fastdiv(p.heads * vec, divs.cols), b = fastdiv(r, divs.tokens), s = r - b * p.S;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, pitch = chunk + 1, sub = threadIdx.x & 3, shift = __builtin_ctz(chunk); // (chunk: a power of two)
     const StepLds at = step_lds(p.S, p.heads, p.kv_heads, p.dim, chunk, p.vdim);
     const uint32_t first = first_visible(p, p.cached + s) + seg * chunk * chunks, hi = p.cached + s + 1, end = min(hi, first + chunk * chunks);
-    const uint32_t vec = p.vdim / 4, cols = p.kv_heads * vec, turns = max(1u, kThreads / cols);
-    const uint32_t mine = threadIdx.x % cols, my_turn = threadIdx.x / cols; // (more columns than threads: turns 1, a second round)
-    const bool has_values = cols > kThreads || my_turn < turns;
+    const uint32_t turns = fastdiv((uint32_t)kThreads, divs.cols); // (at most kThreads columns)
+    const uint32_t my_turn = fastdiv(threadIdx.x, divs.cols), mine = threadIdx.x - my_turn * cols, my_group = fastdiv(mine, divs.vec), my_column = (mine - my_group * vec) * 4;
+    const bool has_values = my_turn < turns;
     f32x4 k[PI][DQ], v[kValuesAhead];
     auto key_of = [&](uint32_t j0, int i, uint32_t *g, uint32_t *key) {
         const uint32_t pair = (threadIdx.x >> 2) + i * (kThreads / 4);
-        *g = min(pair / chunk, p.kv_heads - 1);
-        *key = pair - pair / chunk * chunk;
+        *g = min(pair >> shift, p.kv_heads - 1);
+        *key = pair & (chunk - 1);
         return pair < chunk * p.kv_heads;
     };
     // (rows that are not there or not in the cache are clamped into it: what they hold is replaced or hidden)
@@ -461,93 +466,107 @@ __device__ __forceinline__ void mixed_step(const AttentionPlan &p, const uint32_
             for (int d = 0; d < DQ; d++) k[i][d] = *reinterpret_cast<const f32x4 *>(src + min((uint32_t)(d * 16 + sub * 4), p.dim - 4));
         }
     };
-    auto value_row = [&](uint32_t j, uint32_t g) { // new ones come from the projections
-        return j < p.cached ? p.values + ((int64_t)b * p.kv_heads + g) * p.v_block + (int64_t)j * p.vdim
-                            : p.v.p + ((int64_t)b * p.S + (min(j, hi - 1) - p.cached)) * p.v.pitch + g * p.vdim;
-    };
-    auto ask_values = [&](uint32_t j0, uint32_t c) {
-        const uint32_t g = min(c / vec, p.kv_heads - 1), d = (c - c / vec * vec) * 4;
+    // (new ones come from the projections; a lane chooses: see pinned)
+    global_float *const cached_values = pinned(p.values), *const new_values = pinned(p.v.p);
+    typedef const __attribute__((address_space(1))) f32x4 global_f32x4;
+    global_float *const cached_column = cached_values + ((int64_t)b * p.kv_heads + my_group) * p.v_block + my_column;
+    global_float *const new_column = new_values + ((int64_t)b * p.S - p.cached) * p.v.pitch + my_group * p.vdim + my_column;
+    auto ask_values = [&](uint32_t j0) {
 #pragma unroll
         for (uint32_t e = 0; e < kValuesAhead; e++)
-            if (e * turns < chunk) v[e] = *reinterpret_cast<const f32x4 *>(value_row(min(j0 + my_turn % turns + e * turns, hi - 1), g) + d);
+            if (e * turns < chunk) {
+                const uint32_t j = min(j0 + min(my_turn, turns - 1) + e * turns, hi - 1);
+                global_float *const old_row = cached_column + (int64_t)j * p.vdim, *const new_row = new_column + (int64_t)j * p.v.pitch;
+                v[e] = *reinterpret_cast<global_f32x4 *>(j < p.cached ? old_row : new_row);
+            }
     };
-    // a wave's heads: values lane and lane + 64 of each (one of a kind where a head is shorter)
-    constexpr int QH = 4, QV = DQ > 4 ? 2 : 1;
-    constexpr uint32_t kWaves = kThreads / 64;
-    float qv[QH][QV];
-    const uint32_t d0 = min(lane, p.dim - 1), d1 = min(lane + 64, p.dim - 1);
-    auto ask_heads = [&](const float *src, uint32_t h0, uint32_t n) {
-#pragma unroll
-        for (int i = 0; i < QH; i++) {
-            const float *x = src + min(h0 + i * kWaves + wave, n - 1) * p.dim;
-            qv[i][0] = x[d0];
-            if (QV > 1) qv[i][QV - 1] = x[d1];
-        }
-    };
-    float2 turn[QV];
+    // heads of a token: LPH lanes to a head, four values (two pairs of the rotation) a lane, HPP heads at a time in a wave
+    constexpr uint32_t kWaves = kThreads / 64, LPH = DQ * 4, HPP = 64 / LPH, QP = 2;
+    typedef f32x4 f32x4_words __attribute__((aligned(4))); // from any word's address
+    const uint32_t own_head = wave * HPP + lane / LPH, d = lane % LPH * 4, d_in = min(d, p.dim - 4);
+    auto head_at = [&](const float *src, uint32_t h, uint32_t n) { return *reinterpret_cast<const f32x4_words *>(src + min(h, n - 1) * p.dim + d_in); };
+    // a token's rotation: both tables asked for (no load behind waits for them), and put together
+    float2 fine[2] = {}, coarse[2] = {}, turn[2];
     auto ask_turn = [&](uint32_t t) {
+        if (!p.rot_dims) return;
+        const uint32_t pairs = p.rot_dims / 2;
+        const uint64_t position = p.position + t;
 #pragma unroll
-        for (int v = 0; v < QV; v++) {
-            const uint32_t d = lane + 64 * v;
-            turn[v] = make_float2(1.0f, 0.0f);
-            if (d < p.rot_dims) turn[v] = rotation_at(p, p.position + t, d / 2);
-            if (!(d & 1)) turn[v].y = -turn[v].y;
+        for (uint32_t v = 0; v < 2; v++) {
+            const uint32_t i = min(d / 2 + v, pairs - 1);
+            fine[v] = p.rot_fine[(position % kRotFine) * pairs + i];
+            coarse[v] = p.rot_coarse[(position / kRotFine) * pairs + i];
         }
     };
-    ask_heads(p.q.p + (int64_t)r * p.q.pitch, 0, p.heads);
-    ask_turn(s);
-    ask_keys(first);
-    ask_values(first, mine);
-
+    auto settle_turn = [&] {
+#pragma unroll
+        for (uint32_t v = 0; v < 2; v++) {
+            const float2 a = fine[v], b = coarse[v];
+            turn[v] = d + 2 * v < p.rot_dims ? make_float2(fmaf(a.x, b.x, -a.y * b.y), fmaf(a.x, b.y, a.y * b.x)) : make_float2(1.0f, 0.0f);
+        }
+    };
     const uint32_t t0 = first > p.cached ? first - p.cached : 0, t1 = end > p.cached && end > first ? end - p.cached : 0; // new keys [t0, t1)
-    for (uint32_t i = threadIdx.x; i < p.heads * p.heads; i += kThreads) { // (transposed: lanes side by side read other heads' columns)
-        const uint32_t h = i / p.heads, g = i - h * p.heads;
-        lds[at.talk + g * p.heads + h] = p.talk ? p.talk[i] : h == g ? 1.0f : 0.0f;
+    const float *const q_row = p.q.p + (int64_t)r * p.q.pitch;
+    auto new_key = [&](uint32_t t, uint32_t h0) { return head_at(p.k.p + ((int64_t)b * p.S + t) * p.k.pitch, h0 + own_head, p.kv_heads); };
+    f32x4 qv[QP], kv = {};
+#pragma unroll
+    for (uint32_t i = 0; i < QP; i++) qv[i] = head_at(q_row, i * kWaves * HPP + own_head, p.heads);
+    if (t0 < t1) kv = new_key(t0, 0);
+    ask_turn(s);
+    const uint32_t pairs_of_heads = p.heads * p.heads;
+    const float talk_ahead = p.talk ? p.talk[min(threadIdx.x, pairs_of_heads - 1)] : 0.0f;
+    __builtin_amdgcn_sched_barrier(0);
+    ask_keys(first);
+    __builtin_amdgcn_sched_barrier(0);
+    ask_values(first);
+    __builtin_amdgcn_sched_barrier(0); // (what follows stays behind these loads)
+
+    for (uint32_t i = threadIdx.x; i < pairs_of_heads; i += kThreads) { // (transposed: lanes side by side read other heads' columns)
+        const uint32_t h = fastdiv(i, divs.heads), g = i - h * p.heads;
+        lds[at.talk + g * p.heads + h] = p.talk ? (i < kThreads ? talk_ahead : p.talk[i]) : h == g ? 1.0f : 0.0f;
     }
+    settle_turn();
     for (uint32_t h = threadIdx.x; h < p.heads; h += kThreads) {
         lds[at.state + h] = kNone;
         lds[at.state + p.heads + h] = 0.0f;
     }
-    // the heads of a token: turned, at a mean square of one, times f
-    auto put_heads = [&](uint32_t h0, uint32_t n, float f, float *dst, float *cache, int64_t cache_pitch) {
+    // a head: turned, at a mean square of one, times f
+    auto put_head = [&](const f32x4 &given, uint32_t h, uint32_t n, float f, float *dst, float *cache, int64_t cache_pitch) {
+        f32x4 x;
 #pragma unroll
-        for (int i = 0; i < QH; i++) {
-            const uint32_t h = h0 + i * kWaves + wave;
-            float x[QV], m = 0.0f;
-#pragma unroll
-            for (int v = 0; v < QV; v++) {
-                x[v] = fmaf(qv[i][v], turn[v].x, asf(across<1>(asu(qv[i][v]))) * turn[v].y);
-                if (lane + 64 * v < p.dim) m = fmaf(x[v], x[v], m);
-            }
-            float g = f;
-            if (p.unit_heads) g /= sqrtf(wave_total(m) / (float)p.dim + p.eps);
-#pragma unroll
-            for (int v = 0; v < QV; v++)
-                if (h < n && lane + 64 * v < p.dim) {
-                    dst[h * p.dim + lane + 64 * v] = x[v] * g;
-                    if (cache) cache[h * cache_pitch + lane + 64 * v] = x[v] * g;
-                }
+        for (uint32_t v = 0; v < 4; v += 2) {
+            x[v] = fmaf(given[v], turn[v / 2].x, given[v + 1] * -turn[v / 2].y);
+            x[v + 1] = fmaf(given[v + 1], turn[v / 2].x, given[v] * turn[v / 2].y);
+        }
+        if (p.unit_heads) {
+            float m = d < p.dim ? fmaf(x[3], x[3], fmaf(x[2], x[2], fmaf(x[1], x[1], x[0] * x[0]))) : 0.0f;
+            m = add_across<4>(add_across<2>(add_across<1>(m)));
+            if constexpr (LPH > 8) m = add_across<8>(m);
+            if constexpr (LPH > 16) m = add_across<16>(m);
+            f /= sqrtf(m / (float)p.dim + p.eps);
+        }
+        x *= f;
+        if (h < n && d < p.dim) {
+            *reinterpret_cast<f32x4 *>(dst + h * p.dim + d) = x;
+            if (cache) *reinterpret_cast<f32x4_words *>(cache + h * cache_pitch + d) = x;
         }
     };
     float temp = p.scale;
     if (p.temp_every) temp *= 1.0f + p.temp_coef * logf((float)((p.position + s + 1) / p.temp_every + 1));
-    for (uint32_t h0 = 0; h0 < p.heads; h0 += QH * kWaves) {
-        if (h0) ask_heads(p.q.p + (int64_t)r * p.q.pitch, h0, p.heads);
-        put_heads(h0, p.heads, temp, lds + at.q, nullptr, 0);
-    }
+#pragma unroll
+    for (uint32_t i = 0; i < QP; i++) put_head(qv[i], i * kWaves * HPP + own_head, p.heads, temp, lds + at.q, nullptr, 0);
+    for (uint32_t h = QP * kWaves * HPP + own_head; h < p.heads; h += kWaves * HPP) put_head(head_at(q_row, h, p.heads), h, p.heads, temp, lds + at.q, nullptr, 0);
     for (uint32_t t = t0; t < t1; t++) {
-        if (t != s || t > t0) ask_turn(t);
+        if (t != s || t > t0) {
+            ask_turn(t);
+            settle_turn();
+        }
         float *cache = t == s ? p.keys + (int64_t)b * p.kv_heads * p.k_block + (int64_t)(p.cached + t) * p.dim : nullptr; // its own workgroup's
-        for (uint32_t h0 = 0; h0 < p.kv_heads; h0 += QH * kWaves) {
-            ask_heads(p.k.p + ((int64_t)b * p.S + t) * p.k.pitch, h0, p.kv_heads);
-            put_heads(h0, p.kv_heads, 1.0f, lds + at.fresh + t * p.kv_heads * p.dim, cache, p.k_block);
+        for (uint32_t h0 = 0; h0 < p.kv_heads; h0 += kWaves * HPP) {
+            if (t > t0 || h0) kv = new_key(t, h0);
+            put_head(kv, h0 + own_head, p.kv_heads, 1.0f, lds + at.fresh + t * p.kv_heads * p.dim, cache, p.k_block);
         }
     }
-    if (t1 == s + 1 && t0 <= s) // the last segment: this token's values
-        for (uint32_t i = threadIdx.x; i < p.kv_heads * p.vdim; i += kThreads) {
-            const uint32_t g = i / p.vdim, d = i - g * p.vdim;
-            p.values[((int64_t)b * p.kv_heads + g) * p.v_block + (int64_t)(p.cached + s) * p.vdim + d] = p.v.p[(int64_t)r * p.v.pitch + i];
-        }
     __syncthreads();
     f32x4 acc[REP] = {};
     for (uint32_t j0 = first; j0 < end; j0 += chunk) {
@@ -586,7 +605,7 @@ __device__ __forceinline__ void mixed_step(const AttentionPlan &p, const uint32_
         if (j0 + chunk < end) ask_keys(j0 + chunk); // on their way meanwhile
         __syncthreads();
         for (uint32_t i = threadIdx.x; i < p.heads * chunk; i += kThreads) {
-            const uint32_t key = i / p.heads, h = i - key * p.heads;
+            const uint32_t key = fastdiv(i, divs.heads), h = i - key * p.heads;
             float w = 0.0f;
 #pragma unroll 8
             for (uint32_t g = 0; g < p.heads; g++) w = fmaf(lds[at.talk + g * p.heads + h], lds[at.raw + g * pitch + key], w);
@@ -616,15 +635,17 @@ __device__ __forceinline__ void mixed_step(const AttentionPlan &p, const uint32_
         }
         __syncthreads();
         // a thread's columns: results of this chunk for one kv head's query heads, REP at a time
-        auto weigh = [&](uint32_t c, uint32_t h0, f32x4(&o)[REP]) {
-            const uint32_t g = c / vec;
+        auto weigh = [&](f32x4(&o)[REP]) {
+            const uint32_t g = my_group;
 #pragma unroll
             for (uint32_t e = 0; e < kValuesAhead; e++) {
-                const uint32_t key = my_turn % turns + e * turns;
+                const uint32_t key = my_turn + e * turns;
                 if (key >= keys) break;
+                if (j0 + key == p.cached + s) // this token's values, in the last segment
+                    *reinterpret_cast<f32x4 *>(p.values + ((int64_t)b * p.kv_heads + g) * p.v_block + (int64_t)(p.cached + s) * p.vdim + my_column) = v[e];
 #pragma unroll
                 for (int h = 0; h < REP; h++) {
-                    const float w = lds[at.mixed + (g * rep + min(h0 + h, rep - 1)) * pitch + key];
+                    const float w = lds[at.mixed + (g * rep + min((uint32_t)h, rep - 1)) * pitch + key];
 #pragma unroll
                     for (int d = 0; d < 4; d++) o[h][d] = fmaf(w, v[e][d], o[h][d]);
                 }
@@ -632,11 +653,11 @@ __device__ __forceinline__ void mixed_step(const AttentionPlan &p, const uint32_
         };
         if (has_values) {
 #pragma unroll
-            for (int h = 0; h < REP; h++) acc[h] *= lds[at.state + 2 * p.heads + (mine / vec) * rep + min((uint32_t)h, rep - 1)];
-            weigh(mine, 0, acc);
+            for (int h = 0; h < REP; h++) acc[h] *= lds[at.state + 2 * p.heads + my_group * rep + min((uint32_t)h, rep - 1)];
+            weigh(acc);
         }
         if (j0 + chunk < end) {
-            ask_values(j0 + chunk, mine);
+            ask_values(j0 + chunk);
             __syncthreads();
         }
     }
@@ -650,7 +671,7 @@ __device__ __forceinline__ void mixed_step(const AttentionPlan &p, const uint32_
 #pragma unroll
                 for (int h = 0; h < REP; h++) {
                     if (h >= (int)rep) break;
-                    f32x4 *o = reinterpret_cast<f32x4 *>(lds + at.q + ((mine / vec) * rep + h) * p.vdim + (mine % vec) * 4);
+                    f32x4 *o = reinterpret_cast<f32x4 *>(lds + at.q + (my_group * rep + h) * p.vdim + my_column);
                     *o = t ? *o + acc[h] : acc[h];
                 }
             }
@@ -660,26 +681,27 @@ __device__ __forceinline__ void mixed_step(const AttentionPlan &p, const uint32_
     } else if (has_values) {
 #pragma unroll
         for (int h = 0; h < REP; h++)
-            if (h < (int)rep) *reinterpret_cast<f32x4 *>(dst + ((mine / vec) * rep + h) * p.vdim + (mine % vec) * 4) = acc[h];
+            if (h < (int)rep) *reinterpret_cast<f32x4 *>(dst + (my_group * rep + h) * p.vdim + my_column) = acc[h];
     }
 }
 
 template <int REP, int DQ, int PI>
-__global__ __launch_bounds__(kThreads, REP <= 4 ? 3 : 2) void attention_mixed_step_kernel(const AttentionPlan p, const uint32_t chunk, const uint32_t chunks, float *__restrict__ parts,
+__global__ __launch_bounds__(kThreads, 2) void attention_mixed_step_kernel(const AttentionPlan p, const StepDivs divs, const uint32_t chunk, const uint32_t chunks, float *__restrict__ parts,
                                                                         float2 *__restrict__ stats) {
     extern __shared__ float lds[];
-    mixed_step<REP, DQ, PI>(p, chunk, chunks, parts, stats, blockIdx.x, gridDim.x, blockIdx.y, lds);
+    mixed_step<REP, DQ, PI>(p, divs, chunk, chunks, parts, stats, blockIdx.x, gridDim.x, blockIdx.y, lds);
 }
 // The same in the first segs * rows workgroups; the others compute the chosen experts' first products (their columns' blocks x, then
 // row * top + choice), which need nothing of the attention.
 template <int REP, int DQ, int PI, bool BF16>
-__global__ __launch_bounds__(kThreads, 3) void attention_step_experts_kernel(const AttentionPlan p, const uint32_t chunk, const uint32_t chunks, float *__restrict__ parts,
+__global__ __launch_bounds__(kThreads, 2) void attention_step_experts_kernel(const AttentionPlan p, const StepDivs divs, const uint32_t chunk, const uint32_t chunks, float *__restrict__ parts,
                                                                              float2 *__restrict__ stats, const uint32_t segs, const ExpertsPlan e, const uint32_t per_wave,
                                                                              const uint32_t blocks_x, float *__restrict__ hidden, uint32_t *__restrict__ chosen) {
     extern __shared__ float lds[];
     const uint32_t first = segs * p.B * p.S;
     if (blockIdx.x < first) {
-        mixed_step<REP, DQ, PI>(p, chunk, chunks, parts, stats, blockIdx.x % segs, segs, blockIdx.x / segs, lds);
+        const uint32_t r = fastdiv(blockIdx.x, divs.segs);
+        mixed_step<REP, DQ, PI>(p, divs, chunk, chunks, parts, stats, blockIdx.x - r * segs, segs, r, lds);
         return;
     }
     const uint32_t i = blockIdx.x - first, by = i / blocks_x, bx = i - by * blocks_x;
@@ -831,7 +853,7 @@ int launch_mixed_tiles(cg_backend *be, const AttentionPlan &p, const float *q) {
 
 static uint32_t pieces_of(uint32_t dim) { return dim <= 32 ? 2 : dim <= 64 ? 4 : 8; } // 16-byte pieces of a key per lane
 
-typedef void (*StepKernel)(AttentionPlan, uint32_t, uint32_t, float *, float2 *);
+typedef void (*StepKernel)(AttentionPlan, StepDivs, uint32_t, uint32_t, float *, float2 *);
 template <int REP> static StepKernel step_kernel(uint32_t dq) { // (PI: keys of four lanes, 8 pieces per lane)
     return dq == 2 ? attention_mixed_step_kernel<REP, 2, 4> : dq == 4 ? attention_mixed_step_kernel<REP, 4, 2> : attention_mixed_step_kernel<REP, 8, 1>;
 }
@@ -844,19 +866,19 @@ static int step_kernels_beside(cg_backend *be, const DeferredStep &s, const Expe
     constexpr int PI = 8 / DQ;
     const size_t lds = std::max(s.lds, route_bytes(e));
     if (lds > (64u << 10)) return kDeclined;
-    // The experts' columns on what is resident beside attention (three workgroups a compute unit, two where its LDS holds no more): those of a
+    // The experts' columns on what is resident beside attention (two workgroups a compute unit): those of a
     // second round would start with the choice of the experts when the first ones end.
-    const uint32_t units = be->compute_units, at_once = std::min<uint32_t>(3, (uint32_t)(kMaxLds / lds));
+    const uint32_t units = be->compute_units, at_once = std::min<uint32_t>(2, (uint32_t)(kMaxLds / lds));
     const uint32_t beside = std::max(units, at_once * units - std::min((at_once - 1) * units, s.segs * s.plan.B * s.plan.S));
     const uint64_t columns = (uint64_t)e.rows * e.top * e.ff;
     const uint32_t per_wave = (uint32_t)std::clamp<uint64_t>((columns + (uint64_t)beside * kExpertWaves - 1) / ((uint64_t)beside * kExpertWaves), 1, 16), bx = (e.ff + kExpertWaves * per_wave - 1) / (kExpertWaves * per_wave);
     const uint64_t blocks = (uint64_t)s.segs * s.plan.B * s.plan.S + (uint64_t)bx * e.rows * e.top;
     if (blocks > 0x7FFFFFFFull) return kDeclined;
     if (e.fmt == kFmtBF16)
-        launch_kernel((attention_step_experts_kernel<REP, DQ, PI, true>), dim3((uint32_t)blocks), dim3(kThreads), lds, be->stream, s.plan, s.chunk, s.chunks, s.parts, s.stats, s.segs,
+        launch_kernel((attention_step_experts_kernel<REP, DQ, PI, true>), dim3((uint32_t)blocks), dim3(kThreads), lds, be->stream, s.plan, s.divs, s.chunk, s.chunks, s.parts, s.stats, s.segs,
                       e, per_wave, bx, hidden, chosen);
     else
-        launch_kernel((attention_step_experts_kernel<REP, DQ, PI, false>), dim3((uint32_t)blocks), dim3(kThreads), lds, be->stream, s.plan, s.chunk, s.chunks, s.parts, s.stats, s.segs,
+        launch_kernel((attention_step_experts_kernel<REP, DQ, PI, false>), dim3((uint32_t)blocks), dim3(kThreads), lds, be->stream, s.plan, s.divs, s.chunk, s.chunks, s.parts, s.stats, s.segs,
                       e, per_wave, bx, hidden, chosen);
     return CG_OK;
 }
@@ -867,7 +889,7 @@ static int merge_step(cg_backend *be, const DeferredStep &s) {
 }
 
 int run_step(cg_backend *be, const DeferredStep &s) {
-    launch_kernel(step_kernel(s.plan), dim3(s.segs, s.plan.B * s.plan.S), dim3(kThreads), s.lds, be->stream, s.plan, s.chunk, s.chunks, s.parts, s.stats);
+    launch_kernel(step_kernel(s.plan), dim3(s.segs, s.plan.B * s.plan.S), dim3(kThreads), s.lds, be->stream, s.plan, s.divs, s.chunk, s.chunks, s.parts, s.stats);
     return merge_step(be, s);
 }
 
@@ -904,7 +926,7 @@ int launch_mixed_step(cg_backend *be, const AttentionPlan &p, DeferredStep **lat
     if (lds > kMaxLds / 2) return kDeclined;
     // as many workgroups as run at a time
     const uint32_t all = (most + chunk - 1) / chunk;
-    const uint32_t resident = (rep <= 4 ? 3 : 2) * be->compute_units, chunks = (uint32_t)(((uint64_t)rows * all + resident - 1) / resident), nseg = (all + chunks - 1) / chunks;
+    const uint32_t resident = 2 * be->compute_units, chunks = (uint32_t)(((uint64_t)rows * all + resident - 1) / resident), nseg = (all + chunks - 1) / chunks;
     // (here and not when it is launched: a refusal is this call's)
     if (int rc = allow_lds(reinterpret_cast<const void *>(step_kernel(p)), lds)) return rc;
     DeferredStep *const s = new DeferredStep;
@@ -915,6 +937,7 @@ int launch_mixed_step(cg_backend *be, const AttentionPlan &p, DeferredStep **lat
         return rc;
     }
     s->plan = p;
+    s->divs = {make_fastdiv(p.S), make_fastdiv(p.heads), make_fastdiv(p.vdim / 4), make_fastdiv(cols), make_fastdiv(nseg)};
     s->chunk = chunk;
     s->chunks = chunks;
     s->segs = nseg;

@@ -188,10 +188,14 @@ __device__ __forceinline__ float2 rotation_at(const AttentionPlan &p, uint64_t p
 }
 #endif
 // Attention over mixed scores of a few new tokens whose launch waits for the next call on its backend: a mixture of experts that does
-// not read its result, which comes next in a layer, shares the launch (either is bound by latency: 10 and 8 us, 12 together).
+// not read its result, which comes next in a layer, shares the launch (either is bound by latency: 10 and 8 us alone where both were 12 together, now 8).
 // Any other call launches it first (Enter).
+struct StepDivs { // what the kernels divide by, as multiplications
+    FastDiv tokens, heads, vec, cols, segs; // new tokens; heads; 16-byte pieces of a value row, of all kv heads' value rows; segments
+};
 struct DeferredStep {
     AttentionPlan plan{};
+    StepDivs divs{};
     uint32_t chunk = 0, chunks = 0, segs = 0;
     size_t lds = 0;
     void *mem = nullptr; // the segments' results (pool memory)

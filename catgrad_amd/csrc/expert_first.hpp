@@ -71,10 +71,66 @@ __device__ void choose_experts(const ExpertsPlan &p, uint32_t row, float *lds, u
     __syncthreads();
 }
 
+// The choice by a wave alone, a lane to an expert: scores are ranked in registers, and nothing waits for LDS or a barrier.  At most 64 experts, their
+// groups (where groups are dropped) of a power of two members.  (Every wave of a workgroup chooses for itself, so a comparison is three instructions:
+// ties are resolved behind the ranks.)
+__host__ __device__ inline bool wave_chooses(const ExpertsPlan &p) {
+    const uint32_t size = p.experts / p.groups;
+    return p.experts <= 64 && (p.keep >= p.groups || (size & (size - 1)) == 0);
+}
+struct WaveChoice {
+    float logit, correction, own; // own: the lane's expert's score
+    uint32_t rank;                // how many choices are better (none: the lane has no expert)
+    __device__ __forceinline__ void ask(const ExpertsPlan &p, uint32_t row) { // (clamped, not tested: no load waits)
+        const uint32_t e = min(threadIdx.x & 63, p.experts - 1);
+        logit = p.logits[(int64_t)row * p.experts + e];
+        correction = p.correction ? p.correction[e] : 0.0f;
+    }
+    template <int DIST> static __device__ __forceinline__ void best_two(float &first, float &second) {
+        const float f = asf(across<DIST>(asu(first))), s = asf(across<DIST>(asu(second)));
+        second = fmaxf(fminf(first, f), fmaxf(second, s));
+        first = fmaxf(first, f);
+    }
+    static __device__ __forceinline__ float lane_of(float v, uint32_t lane) { return asf(__builtin_amdgcn_readlane(asu(v), lane)); }
+    __device__ __forceinline__ void choose(const ExpertsPlan &p) {
+        const uint32_t e = threadIdx.x & 63;
+        own = sigmoid(logit);
+        float choice = p.correction ? own + correction : own;
+        if (p.keep < p.groups) {
+            const uint32_t shift = __builtin_ctz(p.experts / p.groups), size = 1u << shift, g = e >> shift;
+            float first = choice, second = size > 1 ? -INFINITY : 0.0f;
+            if (size > 1) best_two<1>(first, second);
+            if (size > 2) best_two<2>(first, second);
+            if (size > 4) best_two<4>(first, second);
+            if (size > 8) best_two<8>(first, second);
+            if (size > 16) best_two<16>(first, second);
+            if (size > 32) best_two<32>(first, second);
+            const float worth = first + second;
+            uint32_t before = 0;
+            for (uint32_t j = 0; j < p.groups; j++) before += beats(lane_of(worth, j << shift), j, worth, g);
+            if (before >= p.keep) choice = -INFINITY;
+        }
+        rank = 0;
+#pragma unroll 8
+        for (uint32_t j = 0; j < p.experts; j++) rank += lane_of(choice, j) > choice;
+        if (e >= p.experts) rank = 64;
+    }
+    // the expert in a place and its weight (0 and 0 where scores that are not numbers leave the place untaken)
+    __device__ __forceinline__ uint32_t in_place(uint32_t slot, float *weight) const {
+        uint64_t there = 0;
+        uint32_t r = slot; // equal choices share the first of their places and take them in the order of the experts
+        while (!(there = __ballot(rank == r)) && r) r--;
+        for (; r < slot; r++) there &= there - 1;
+        const uint32_t e = there ? (uint32_t)__builtin_ctzll(there) : 0;
+        *weight = there ? lane_of(own, e) : 0.0f;
+        return e;
+    }
+};
+
 // A workgroup of kExpertThreads: four waves' columns (block x, per_wave each, one after the other) of row * top + choice (block y).
-// In front of the first weight lie the choice and its loads, 4 us: so the columns are cut for one round of workgroups, and a wave's next
-// column is on its way while this one is multiplied.  The launch beside attention, 8 of 32 experts in bf16: 1024 columns of 2048 values
-// 23.4 -> 20.5 us (67 MB, 13 us at the device's rate), 384 of 1024 12.4 -> 11.8.
+// In front of the first weight lie the choice and its loads (3.0 us with barriers, 1.6 by waves, a third of it the way of the logits): so the columns are cut for one round of
+// workgroups, and a wave's next column is on its way while this one is multiplied.  The launch beside attention, 8 of 32 experts in bf16: 1024 columns of 2048 values
+// 23.4 -> 20.5 us (67 MB, 13 us at the device's rate), 384 of 1024 12.4 -> 11.8 (and 8.1 with the choice by waves, see there and mixed_step).
 // LDS: route_bytes(p).
 constexpr int kExpertThreads = 256, kExpertWaves = 4;
 inline size_t route_bytes(const ExpertsPlan &p) { return (route_floats(p.experts, p.groups) + 2 * (size_t)p.top) * 4; }
@@ -86,24 +142,47 @@ __device__ __forceinline__ void expert_first(const ExpertsPlan &p, const uint32_
     const uint32_t row = by / p.top, slot = by - row * p.top, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     uint32_t *chosen = reinterpret_cast<uint32_t *>(lds + route_floats(p.experts, p.groups));
     float *weight = reinterpret_cast<float *>(chosen + p.top);
-    // the row of h, this lane's values of it in registers where they fit
+    const bool by_wave = wave_chooses(p);
+    WaveChoice choice;
+    if (by_wave) choice.ask(p, row);
+    // the row of h, this lane's values of it in registers where they fit: words or pairs of bfloat16 patterns until the choice is made
     float x[STEPS][W];
-    auto take = [&](uint32_t k, float(&o)[W]) { // (clamped; zeros behind the last column)
+    const bool narrow = p.h_fmt == kFmtBF16;
+    typedef uint32_t __attribute__((aligned(2))) pair;
+    auto ask_h = [&](uint32_t k, float(&o)[W]) { // (clamped)
         const int64_t at = (int64_t)row * p.width + min(k, p.width - W);
-        if (p.h_fmt == kFmtBF16) {
+        if (narrow) {
+            const uint16_t *const src = static_cast<const uint16_t *>(p.h) + at;
+            if constexpr (W == 1) {
+                o[0] = asf(src[0]);
+            } else {
 #pragma unroll
-            for (uint32_t i = 0; i < W; i++) o[i] = asf((uint32_t) static_cast<const uint16_t *>(p.h)[at + i] << 16);
+                for (uint32_t i = 0; i < W / 2; i++) o[i] = asf(reinterpret_cast<const pair *>(src)[i]);
+            }
         } else {
             St::input(static_cast<const float *>(p.h), at, o);
+        }
+    };
+    auto settle_h = [&](uint32_t k, float(&o)[W]) { // (zeros behind the last column)
+        if (narrow) {
+#pragma unroll
+            for (int i = (int)W - 1; i >= 0; i--) o[i] = asf(W > 1 && i % 2 ? asu(o[i / 2]) & 0xFFFF0000u : asu(o[i / 2]) << 16);
         }
 #pragma unroll
         for (uint32_t i = 0; i < W; i++) o[i] = k < p.width ? o[i] : 0.0f;
     };
 #pragma unroll
-    for (int s = 0; s < STEPS; s++) take(s * SPAN + lane * W, x[s]);
-    choose_experts<kExpertThreads>(p, row, lds, chosen, weight, threadIdx.x);
-    const uint32_t e = __builtin_amdgcn_readfirstlane(chosen[slot]);
-    const float weigh = weight[slot];
+    for (int s = 0; s < STEPS; s++) ask_h(s * SPAN + lane * W, x[s]);
+    uint32_t e;
+    float weigh;
+    if (by_wave) {
+        choice.choose(p);
+        e = choice.in_place(slot, &weigh);
+    } else {
+        choose_experts<kExpertThreads>(p, row, lds, chosen, weight, threadIdx.x);
+        e = __builtin_amdgcn_readfirstlane(chosen[slot]);
+        weigh = weight[slot];
+    }
     if (bx == 0 && threadIdx.x == 0) chosen_out[by] = e;
     const uint32_t f0 = (bx * kExpertWaves + __builtin_amdgcn_readfirstlane(wave)) * per_wave, f1 = min(f0 + per_wave, p.ff);
     if (f0 >= f1) return;
@@ -124,7 +203,8 @@ __device__ __forceinline__ void expert_first(const ExpertsPlan &p, const uint32_
                 wg.load(g, k);
                 wu.load(g + up, k);
                 float v[W];
-                take(k, v);
+                ask_h(k, v);
+                settle_h(k, v);
                 a = wg.dot(v, a);
                 b = wu.dot(v, b);
             }
@@ -155,6 +235,8 @@ __device__ __forceinline__ void expert_first(const ExpertsPlan &p, const uint32_
     };
     Piece c0, c1;
     ask(f0, 0, c0);
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) settle_h(s * SPAN + lane * W, x[s]);
     if constexpr (STEPS > PART) {
         for (uint32_t f = f0; f < f1; f++) {
             float a = 0.0f, b = 0.0f;
