@@ -1,5 +1,5 @@
 // The decoder blocks' products of one row of activations (one token of one sequence), for weights whose rows lie in 16-byte pieces: as
-// in one_row.hip a workgroup's waves share k, every load is asked for at the start, and one barrier is enough: what a norm multiplies a
+// in skinny_kernel.hpp a workgroup's waves share k, every load is asked for at the start, and one barrier is enough: what a norm multiplies a
 // row by is a factor of the sums (for the polynomial one, of the sums of z, z^2, z^3 and 1 each).  Activations stay in 32 bits, also
 // beside bfloat16 weights.  Against the kernels of up to four rows (block_rows.hip), us a launch in the steps of models of width 1024:
 // 1024 -> 8328 with a norm, f32, 9.7 and 7.6; the sum of 2048 -> 1024 and of the polynomial norm's 3072 -> 1024, f32, 7.9 and 6.0; two products
