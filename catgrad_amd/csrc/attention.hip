@@ -55,10 +55,17 @@ static int launch_seg_kernel(cg_backend *be, const AttnArgs &g, const FusedArgs 
     return CG_OK;
 }
 
-// The open heads as the attention g over a cache of T positions reads them: its q and the newest row of its K, no other products.
-static bool take_open_heads(const cg_backend *be, const AttnArgs &g, int64_t entries, RawHeads *raw) {
+// The open heads as the attention g over a cache of T positions reads them: its q and the newest row of its K, no other products.  What
+// else it loads, v and the soft-max program's leaves, must not lie where the heads are to be stored: the kernels ask for V and the leaves
+// before they store a finished row, so that a V which is K's own cache would be read without its newest row.
+static bool take_open_heads(const cg_backend *be, const AttnArgs &g, int64_t entries, const Pending &p, const cg_tensor *v, RawHeads *raw) {
     const OpenHeads *h = be->heads;
     if (!h || h->count != 2) return false;
+    for (const Buffer *b : h->destinations) {
+        if (v->buf == b) return false;
+        for (int l = 0; l < p.nleaf; l++)
+            if (p.leaf[l].buf == b || p.leaf[l].buf2 == b) return false;
+    }
     const uint32_t *const newest = g.Kc + (int64_t)(g.T - 1) * g.k_st;
     const int q = h->p[0].to.dst == g.Q ? 0 : 1;
     const OpenHeads::Product &pq = h->p[q], &pk = h->p[1 - q];
@@ -168,7 +175,7 @@ int launch_decode_attention(cg_backend *be, const Pending &p, const int64_t *pdi
     g.k_st = f1.b_sn;
     g.v_st = f2.b_sk;
     RawHeads raw;
-    const bool open = take_open_heads(be, g, f1.batch, &raw);
+    const bool open = take_open_heads(be, g, f1.batch, p, v, &raw);
     if (be->heads && !open)
         if (int hrc = launch_open_heads(be)) return hrc;
     // One workgroup per query row: a cache of up to kRowMaxT positions in one launch with nothing to combine (beyond

@@ -666,7 +666,8 @@ struct OpenHeads {
     Product p[4];
     void *scratch = nullptr;
     size_t cls = 0;
-    std::vector<Buffer *> held; // what the stores read and write (retained)
+    std::vector<Buffer *> held;               // what the stores read and write (retained)
+    std::vector<const Buffer *> destinations; // of these, what they write
 };
 int launch_open_heads(cg_backend *be); // be->heads in a launch of their own
 void drop_open_heads(cg_backend *be);  // be->heads are done with: to be called behind the launch that reads them

@@ -1376,6 +1376,7 @@ static int try_rope_stores(cg_backend *be, std::vector<DeferredWrite> &w, const 
         for (int i = 0; i < n; i++) {
             if (!ms[i]->head_norm) continue;
             hold(w[i].dst->buf);
+            be->heads->destinations.push_back(w[i].dst->buf);
             hold(ms[i]->hn_gamma);
             for (int l = 0; l < w[i].prog->nleaf; l++)
                 if (w[i].prog->leaf[l].buf) hold(w[i].prog->leaf[l].buf);
