@@ -548,18 +548,20 @@ template <int R, int TAPS> __global__ __launch_bounds__(kStepThreads) void delta
     }
 }
 
-// One token behind a state of at most 128 x 128, V a multiple of 4: a workgroup per (sequence, head), which reads 130 KB of state and
+// One token behind a state of at most 128 x 128, V at least 4: a workgroup per (sequence, head), which reads 130 KB of state and
 // factors and writes 64.  A compute unit takes 2 us to fetch and store these, so everything is asked for at the start, the
 // token's inputs ahead of the state, and what lies behind is kept short: a thread holds R rows of four columns (16 bytes to a load, a
 // quarter of the reads of g, k and q from LDS), both of the state's products are taken before it is written, in one pass,
 //     q . S' = q . (g S) + (q . k) u,   u = beta (v - k . (g S)),
 // so that two barriers are enough, either factored projection has four waves to itself (one vector to fetch, not two), and the
 // convolutions' inputs are kept from the registers that hold them.  Heads of 128 x 128, 32-bit steps behind 777 tokens of a model of
-// width 1024: 12.5 us before (a column a thread, a pass and four barriers more), 6.2 so.
+// width 1024: 12.5 us before (a column a thread, a pass and four barriers more), 6.2 so.  (128 x 126, whose rows begin at any word: 13.6 on
+// the general kernel, 6.5.)
 constexpr uint32_t kTokenDim = 128;
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef f4 f4_words __attribute__((aligned(4))); // from any word's address
-// LV: lanes side by side on a row of the state (V at most 4 LV).  Q: 16-byte pieces of the factors' rows to a lane, four lanes to a row.
+// LV: lanes side by side on a row of the state (V at most 4 LV; where V is no multiple of 4 the last lane's columns begin with some of the
+// lane's before it: the same sums to the bit, counted once).  Q: 16-byte pieces of the factors' rows to a lane, four lanes to a row.
 template <int LV, int Q> __global__ __launch_bounds__(kStepThreads) void delta_token_kernel(const DeltaPlan p) {
     constexpr int WAVES = kStepThreads / 64, GROUPS = kStepThreads / LV, R = kTokenDim / GROUPS, HALF = kStepThreads / 2;
     static_assert(R % 4 == 0 && (LV == 32 || LV == 16), "rows in fours, whole or half waves' rows");
@@ -596,7 +598,7 @@ template <int LV, int Q> __global__ __launch_bounds__(kStepThreads) void delta_t
     f4 S[R];
     const char *const src = reinterpret_cast<const char *>(p.state + sb);
 #pragma unroll
-    for (uint32_t i = 0; i < R; i++) S[i] = *reinterpret_cast<const f4 *>(src + (min(d0 + i, D - 1) * V + col) * 4);
+    for (uint32_t i = 0; i < R; i++) S[i] = *reinterpret_cast<const f4_words *>(src + (min(d0 + i, D - 1) * V + col) * 4);
     __builtin_amdgcn_sched_barrier(0); // (what follows stays behind all of the loads)
 
     if (tid >= D && tid < kTokenDim) q[tid] = k[tid] = g[tid] = 0.0f;
@@ -664,7 +666,7 @@ template <int LV, int Q> __global__ __launch_bounds__(kStepThreads) void delta_t
     f4 u = {};
 #pragma unroll
     for (int i = 0; i < WAVES; i++) u += *reinterpret_cast<const f4 *>(part[i][1][c]);
-    const f4 v4 = *reinterpret_cast<const f4 *>(v + col);
+    const f4 v4 = *reinterpret_cast<const f4_words *>(v + col);
 #pragma unroll
     for (int j = 0; j < 4; j++) u[j] = column ? beta * (v4[j] - u[j]) : 0.0f;
     if (wave == 0) { // (a wave for the norm and the gate)
@@ -679,21 +681,21 @@ template <int LV, int Q> __global__ __launch_bounds__(kStepThreads) void delta_t
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             y[j] = fmaf(qk, u[j], y[j]);
-            sum = fmaf(y[j], y[j], sum);
+            sum = col + j >= 4 * c ? fmaf(y[j], y[j], sum) : sum;
         }
         const bool stores = column && lane < LV;
         const float f = 1.0f / sqrtf(wave_add<1>(stores ? sum : 0.0f) / (float)V + p.eps);
-        const f4 open = *reinterpret_cast<const f4 *>(gate + col);
+        const f4 open = *reinterpret_cast<const f4_words *>(gate + col);
 #pragma unroll
         for (int j = 0; j < 4; j++) y[j] = y[j] * f * weight[j] * open[j];
-        if (stores) *reinterpret_cast<f4 *>(p.out + ((int64_t)b * p.heads + h) * V + col) = y;
+        if (stores) *reinterpret_cast<f4_words *>(p.out + ((int64_t)b * p.heads + h) * V + col) = y;
     }
     char *const dst = reinterpret_cast<char *>(p.state_out + sb);
 #pragma unroll
     for (uint32_t i = 0; i < R; i++) {
 #pragma unroll
         for (int j = 0; j < 4; j++) S[i][j] = fmaf(kk[i], u[j], S[i][j]);
-        if (column && d0 + i < D) *reinterpret_cast<f4 *>(dst + ((d0 + i) * V + col) * 4) = S[i];
+        if (column && d0 + i < D) *reinterpret_cast<f4_words *>(dst + ((d0 + i) * V + col) * 4) = S[i];
     }
 }
 
@@ -780,11 +782,11 @@ bool step_shape(const DeltaPlan &p, uint32_t *lanes, uint32_t *rows) {
     return *rows <= 64;
 }
 
-// What delta_token_kernel is written for: all that it loads in 16-byte pieces lies in such.
+// What delta_token_kernel is written for: the factored projections' rows lie in 16-byte pieces.
 bool takes_token(const DeltaPlan &p) {
     auto aligned = [](const float *at) { return (reinterpret_cast<uintptr_t>(at) & 15) == 0; };
     auto pieces = [&](const float *w, uint32_t rank, const Rows &x) { return rank >= 4 && rank <= 128 && rank % 4 == 0 && x.pitch % 4 == 0 && aligned(w) && aligned(x.p); };
-    return p.S == 1 && p.state && p.taps == 4 && p.dim <= kTokenDim && p.vdim <= kTokenDim && p.vdim % 4 == 0 && aligned(p.state) && pieces(p.decay_w, p.decay_rank, p.decay) &&
+    return p.S == 1 && p.state && p.taps == 4 && p.dim <= kTokenDim && p.vdim <= kTokenDim && p.vdim >= 4 && pieces(p.decay_w, p.decay_rank, p.decay) &&
            pieces(p.gate_w, p.gate_rank, p.gate);
 }
 

@@ -349,7 +349,7 @@ def delta_reference(t, b, o):
     return y.reshape(S, -1), state, raw[S:]
 
 
-def run_delta(be, t, o, portions):
+def run_delta(be, t, o, portions, behind=5):
     B, taps = t["q"].shape[0], t["conv_q"].shape[1]
     H, G, D, V = o["heads"], o["kv_heads"], o["dim"], o["vdim"]
     state, conv = be.zeros((B, H, D, V), 0), be.zeros((B, taps - 1, 2 * G * D + H * V), 0)
@@ -357,15 +357,15 @@ def run_delta(be, t, o, portions):
     small = {n: be.from_numpy(a) for n, a in t.items() if n not in seq}
     at, outs = 0, []
     for n in portions:
-        part = {c: part_of_rows(be, t[c][:, at:at + n]) for c in seq}
+        part = {c: part_of_rows(be, t[c][:, at:at + n], behind=behind) for c in seq}
         out, state, conv = be.block_channel_delta({**part, **small, "state": state.move(), "conv_state": conv.move()}, **o)
         at += n
         outs.append(be.to_numpy(out))
     return np.concatenate(outs, 1), be.to_numpy(state), be.to_numpy(conv)
 
 
-def check_delta(be, t, o, portions, tol=1e-4):
-    got, state, conv = run_delta(be, t, o, portions)
+def check_delta(be, t, o, portions, tol=1e-4, behind=5):
+    got, state, conv = run_delta(be, t, o, portions, behind)
     for b in range(t["q"].shape[0]):
         want, s, c = delta_reference(t, b, o)
         close(got[b], want, tol, f"channel delta {o}, portions {portions[:6]}, sequence {b}")
