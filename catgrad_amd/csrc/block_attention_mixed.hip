@@ -474,7 +474,7 @@ __device__ __forceinline__ void mixed_step(const AttentionPlan &p, const StepDiv
     auto ask_values = [&](uint32_t j0) {
 #pragma unroll
         for (uint32_t e = 0; e < kValuesAhead; e++)
-            if (e * turns < chunk) {
+            if (!e || e * turns < chunk) { // (the first one without a test: a wait in front of it then serves the others, where each would have its own)
                 const uint32_t j = min(j0 + min(my_turn, turns - 1) + e * turns, hi - 1);
                 global_float *const old_row = cached_column + (int64_t)j * p.vdim, *const new_row = new_column + (int64_t)j * p.v.pitch;
                 v[e] = *reinterpret_cast<global_f32x4 *>(j < p.cached ? old_row : new_row);
@@ -484,7 +484,7 @@ __device__ __forceinline__ void mixed_step(const AttentionPlan &p, const StepDiv
     constexpr uint32_t kWaves = kThreads / 64, LPH = DQ * 4, HPP = 64 / LPH, QP = 2;
     typedef f32x4 f32x4_words __attribute__((aligned(4))); // from any word's address
     const uint32_t own_head = wave * HPP + lane / LPH, d = lane % LPH * 4, d_in = min(d, p.dim - 4);
-    auto head_at = [&](const float *src, uint32_t h, uint32_t n) { return *reinterpret_cast<const f32x4_words *>(src + min(h, n - 1) * p.dim + d_in); };
+    auto head_at = [&](const float *src, uint32_t h, uint32_t n) -> f32x4 { return *reinterpret_cast<const f32x4_words *>(src + min(h, n - 1) * p.dim + d_in); };
     // a token's rotation: both tables asked for (no load behind waits for them), and put together
     float2 fine[2] = {}, coarse[2] = {}, turn[2];
     auto ask_turn = [&](uint32_t t) {
@@ -641,8 +641,6 @@ __device__ __forceinline__ void mixed_step(const AttentionPlan &p, const StepDiv
             for (uint32_t e = 0; e < kValuesAhead; e++) {
                 const uint32_t key = my_turn + e * turns;
                 if (key >= keys) break;
-                if (j0 + key == p.cached + s) // this token's values, in the last segment
-                    *reinterpret_cast<f32x4 *>(p.values + ((int64_t)b * p.kv_heads + g) * p.v_block + (int64_t)(p.cached + s) * p.vdim + my_column) = v[e];
 #pragma unroll
                 for (int h = 0; h < REP; h++) {
                     const float w = lds[at.mixed + (g * rep + min((uint32_t)h, rep - 1)) * pitch + key];
@@ -659,6 +657,11 @@ __device__ __forceinline__ void mixed_step(const AttentionPlan &p, const StepDiv
         if (j0 + chunk < end) {
             ask_values(j0 + chunk);
             __syncthreads();
+        } else if (has_values && end == hi) { // this token's values, from the last segment (with a store where chunks follow, waits are for the next one's keys too)
+            const uint32_t own = hi - 1 - j0;
+#pragma unroll
+            for (uint32_t e = 0; e < kValuesAhead; e++)
+                if (my_turn + e * turns == own) *reinterpret_cast<f32x4 *>(p.values + ((int64_t)b * p.kv_heads + my_group) * p.v_block + (int64_t)(p.cached + s) * p.vdim + my_column) = v[e];
         }
     }
     __syncthreads();
