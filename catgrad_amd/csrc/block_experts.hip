@@ -434,17 +434,23 @@ int launch_experts_second(cg_backend *be, const ExpertsPlan &p, const float *hid
         vec = vec && w->k % vw == 0 && w->pitch % vw == 0 && aligned16(w->p) && y.pitch % 4 == 0 && aligned16(y.p);
     }
     ProfScope prof(be, CG_K_GEMM_SKINNY, first_bytes(p, p.rows * p.top) / 2 + (w ? (double)w->n * w->k * (bf16 ? 2.0 : 4.0) : 0.0));
+    // pieces of a wave at a time: as many as leave the fewest rounds, and of these the fewest, since those behind the last are loaded too
+    // (4 rows of 1024, 32 pieces in 32 bits: five at a time 21.4 us, four 19.4; 8 of 512, 3 in bfloat16: three 5.0, one 4.1)
+    constexpr uint32_t kMost = 6; // (what the registers hold beside four columns' sums)
     const uint32_t span = 64 * (bf16 ? 8 : 4), pieces = p.top * ((p.ff + span - 1) / span) + (w ? (w->k + span - 1) / span : 0);
+    const uint32_t rounds = (pieces + kMost * kWaves - 1) / (kMost * kWaves), at_once = (pieces + rounds * kWaves - 1) / (rounds * kWaves);
     const dim3 grid((p.width + 3) / 4, p.rows);
     static_assert(kWaves == 4, "columns of a workgroup, a wave each or four to all");
     auto launch = [&](auto kernel) { launch_kernel(kernel, grid, dim3(kThreads), 0, be->stream, p, hidden, chosen, x, y, w ? *w : none, scale, out); };
     auto either = [&](auto b) {
         constexpr bool BF = decltype(b)::value;
         if (!vec) launch(expert_second_kernel<BF, false, 4>);
-        else if (pieces <= 3 * kWaves) launch(expert_second_kernel<BF, true, 3>);
-        else if (pieces <= 4 * kWaves) launch(expert_second_kernel<BF, true, 4>);
-        else if (pieces > 5 * kWaves && pieces <= 6 * kWaves) launch(expert_second_kernel<BF, true, 6>);
-        else launch(expert_second_kernel<BF, true, 5>);
+        else if (at_once == 1) launch(expert_second_kernel<BF, true, 1>);
+        else if (at_once == 2) launch(expert_second_kernel<BF, true, 2>);
+        else if (at_once == 3) launch(expert_second_kernel<BF, true, 3>);
+        else if (at_once == 4) launch(expert_second_kernel<BF, true, 4>);
+        else if (at_once == 5) launch(expert_second_kernel<BF, true, 5>);
+        else launch(expert_second_kernel<BF, true, kMost>);
     };
     if (bf16) either(std::true_type{});
     else either(std::false_type{});
