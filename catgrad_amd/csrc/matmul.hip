@@ -1575,6 +1575,16 @@ static SkinnyInput skinny_input(const MmArgs &a, const NormFuse *nf) {
 static SkinnyProduct skinny_product(const MmArgs &a) { // its rows stored as they are
     return {reinterpret_cast<const float *>(a.B), a.b_sn, a.N, 0, a.C, a.N, 0, nullptr, nullptr, a.N, 0};
 }
+// Whether a product that shares its launch with no other goes there too.  Lanes whose values lie behind the end of a wave's share of k idle
+// (see with_cut), which costs more than the barriers and the sums that it saves: us a launch there and on the matrix instruction's kernel
+// 5 x 2052 x 12288 39.5 and 24.9, 4 x 260 x 8192 6.3 and 4.6, but 8 x 2048 x 12288 19.8 and 33.9.  One row of fewer columns takes as long
+// there or up to a tenth longer (1 x 4096 x 8192 22.0 and 20.4).  From 16384 columns on the other side is skinny_kt_wide_kernel: 1 x 1024 x
+// 32768 20.8 and 30.8, 5 x 260 x 49152 32.1 and 21.8.
+static bool skinny_alone(const MmArgs &a) {
+    const uint32_t cut = a.M == 1 ? (a.K <= 4096 ? 1024 : 8192) : a.K <= 1024 ? 1024 : 2048, whole = (a.K + cut - 1) / cut * cut;
+    const bool many = a.N >= 16384, rounds = a.M > 1 && a.K > cut;
+    return (a.M > 1 || many) && 16ull * a.K >= (many || rounds ? 15ull : 9ull) * whole;
+}
 static bool skinny_operands(const MmArgs &a) { return a.a_vec && a.b_vec && a.a_sk == 1 && a.b_sk == 1 && takes_skinny(a.M, a.K); }
 
 int launch_matmul_group(cg_backend *be, const cg_tensor *x, const cg_tensor *const *ys, cg_tensor *const *outs, int n,
@@ -2103,7 +2113,7 @@ static int product(cg_backend *be, const cg_tensor *x, const cg_tensor *y, cg_te
         } else {
             // enough waves to cover 256 CUs several times over, else split K inside the block
             const int64_t cols = N * batch;
-            if (batch == 1 && cols >= 2048 && skinny_operands(a)) {
+            if (batch == 1 && cols >= 2048 && skinny_operands(a) && skinny_alone(a)) {
                 const int orc = launch_skinny_group(be, {skinny_input(a, nullptr), {skinny_product(a)}, 1});
                 if (orc) return orc;
             } else if (cols >= 16384) {
