@@ -69,8 +69,8 @@ struct AttnArgs {
 };
 
 // q and the cache's newest row of K as the products left them (see OpenHeads): the kernels below apply the heads' RMS norm and the
-// rotary embedding themselves, op for op but for the order of the sum of squares, and store the results where the launch that they
-// save would have.  A wave finishes a row, behind the first loads of K, and the rows cross to the others through LDS.  The newest row's
+// rotary embedding themselves, op for op as the launch that they save but for the order of the sum of squares, and store the results where
+// that would have.  A wave finishes a row, behind the first loads of K, and the rows cross to the others through LDS.  The newest row's
 // score is taken from there: the cache does not hold that row until the launch ends (what is loaded in its place is not used).
 // head_norm_rope_finish_kernel takes 3.3 us and the hand-over behind it; here it hides behind K: Qwen3-0.6B's steps at 1050 positions
 // (8 KV heads of 128, 2 query heads each) 7.41 us with finished heads, 7.48 so.  (Every wave finishing the rows for itself: the
@@ -99,9 +99,7 @@ template <int LPT> struct OpenHead { // a wave's: a lane's piece of a row and th
     __device__ __forceinline__ float4v finish(const HeadRows &h, uint32_t l) const {
         float ss = row16_sum(fmaf(x[3], x[3], fmaf(x[2], x[2], fmaf(x[1], x[1], x[0] * x[0]))));
         if (LPT == 32) ss = asf(fold_rows(asu(ss), AddWords{}));
-        const uint32_t mean = apply<kAdd, true>(apply<kDiv, true>(asu(ss), h.n_bits, 0, nullptr), h.eps_bits, 0, nullptr);
-        // (a square root where the exponent is one half, as in every model's norms; the power where they differ)
-        const float r = h.exp_bits == 0x3F000000u && asf(mean) > 0.0f ? sqrtf(asf(mean)) : asf(apply<kPow, true>(mean, h.exp_bits, 0, nullptr));
+        const float r = norm_divisor(ss, h.n_bits, h.eps_bits, h.exp_bits);
         float4v v;
 #pragma unroll
         for (int j = 0; j < 4; j++) {

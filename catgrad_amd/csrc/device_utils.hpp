@@ -315,6 +315,15 @@ __device__ __forceinline__ uint32_t apply(uint32_t a, uint32_t b, uint32_t c, ui
     return 0u;
 }
 
+// What an RMS norm divides a row by, pow(sum / n + eps, e), in the norm's own ops but for the power: a square root where e is one half, as in
+// every model's norms (powf takes 0.7 us of a launch of 5; where they are not the same, at and below zero, it stays).  For every kernel that
+// applies such a norm beside other work, so that a row's divisor does not depend on which of them it is.
+__device__ __forceinline__ float norm_divisor(float squares, uint32_t n_bits, uint32_t eps_bits, uint32_t exp_bits) {
+    const uint32_t mean = apply<kAdd, true>(apply<kDiv, true>(asu(squares), n_bits, 0, nullptr), eps_bits, 0, nullptr);
+    if (exp_bits == 0x3F000000u && asf(mean) > 0.0f) return sqrtf(asf(mean));
+    return asf(apply<kPow, true>(mean, exp_bits, 0, nullptr));
+}
+
 // Sum over the 64 lanes of a wave, for every lane: inside rows of 16 lanes by shifts, then from row to row, all without LDS.
 template <int CTRL, int ROWS> __device__ __forceinline__ float add_shifted(float v) {
     return v + asf((uint32_t)__builtin_amdgcn_update_dpp(0, (int)asu(v), CTRL, ROWS, 0xF, true));

@@ -1235,8 +1235,8 @@ template <bool WHOLE, int MM, int CG, int TRIPS> __global__ __launch_bounds__(kT
 // So that kernel leaves those products plain (rows already divided by the input norm) in scratch memory, N columns a row.  Decode-time
 // attention finishes them as it loads them (see OpenHeads); where something else comes first or the attention is none of those kernels',
 // this small launch does: a workgroup per head of a product, a thread per (row, column) of the head; the
-// head's norm, the embedding and the store, op for op as the stand-alone programs (the sum of squares in runs of 16 columns).  A thread
-// norms its partner of the embedding as well, so that all loads go together and one barrier is enough: 4.8 -> 3.0 us for 24 heads
+// head's norm, the embedding and the store, op for op as the stand-alone programs but for norm_divisor's square root and the order of the
+// sum of squares (in runs of 16 columns).  A thread norms its partner of the embedding as well, so that all loads go together and one barrier is enough: 4.8 -> 3.0 us for 24 heads
 // of 128 (3.5 in the steps of the Qwen3-0.6B shape, 16 and 8 heads).  Measured against one launch with a
 // workgroup of 1024 threads per head (a compute unit streams about 25 GB/s on its own however deep its loads are queued,
 // so that launch is as slow as its heads are few: 23 to 29 us for the 32 heads of 128 x 1024 of the Qwen3-0.6B shape):
@@ -1278,8 +1278,7 @@ __global__ __launch_bounds__(kFinishThreads) void head_norm_rope_finish_kernel(c
     if (!mine) return;
     ss = 0.0f;
     for (uint32_t c = 0; c < hd / 16; c++) ss += runs[m * (hd / 16) + c];
-    const uint32_t mean = apply<kDiv, true>(asu(ss), rs.hn_n_bits, 0, nullptr);
-    const uint32_t r = apply<kPow, true>(apply<kAdd, true>(mean, rs.hn_eps_bits, 0, nullptr), rs.hn_exp_bits, 0, nullptr);
+    const uint32_t r = asu(norm_divisor(ss, rs.hn_n_bits, rs.hn_eps_bits, rs.hn_exp_bits));
     v = apply<kMul, true>(apply<kDiv, true>(v, r, 0, nullptr), hg, 0, nullptr);
     if (rs.rope) {
         const uint32_t other = apply<kMul, true>(apply<kDiv, true>(v2, r, 0, nullptr), hg2, 0, nullptr);

@@ -25,13 +25,7 @@ namespace {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 
-// pow(sum / n + eps, e) in the norm's own ops; a square root where e is one half, as in every model's norms (the power takes 0.7 us of a
-// launch of 5; where they are not the same, at and below zero, it stays)
-__device__ __forceinline__ float divisor_of(const SkinnyInput &in, float squares) {
-    const uint32_t mean = apply<kAdd, true>(apply<kDiv, true>(asu(squares), in.n_bits, 0, nullptr), in.eps_bits, 0, nullptr);
-    if (in.exp_bits == 0x3F000000u && asf(mean) > 0.0f) return sqrtf(asf(mean));
-    return asf(apply<kPow, true>(mean, in.exp_bits, 0, nullptr));
-}
+__device__ __forceinline__ float divisor_of(const SkinnyInput &in, float squares) { return norm_divisor(squares, in.n_bits, in.eps_bits, in.exp_bits); }
 
 // The sums of N values over a wave into dst[0 .. N)
 template <int N, class Of> __device__ __forceinline__ void keep_lane_sums(float *dst, Of of) {

@@ -32,6 +32,18 @@ def close(got, want, bound, what):
     assert np.abs(got - want).max() <= bound, what
 
 
+def finish(be, t, shape, gain, tables, pos):
+    """Heads of a product, normed and embedded."""
+    B, n, hd = shape
+    flat = be.reshape(be.transpose(be.reshape(t.move(), (B, 1, n, hd)).move(), 1, 2).move(), (B * n, hd))
+    y = cases._rmsnorm_ops(be, flat, gain, hd, (B * n, hd))
+    del flat  # (the norm stays open if nobody else holds the product)
+    y = be.reshape(y.move(), (B, n, 1, hd))
+    c, s = (be.broadcast(be.reshape(be.slice(a, 0, pos, 1).move(), (1, 1, 1, hd)).move(), (B, n, 1, hd)) for a in tables)
+    mixed = cases._rot_half(be, y, hd // 2)
+    return be.add(be.mul(c.move(), y.move()).move(), be.mul(s.move(), mixed.move()).move())
+
+
 def run(B, kvh, rep, hd, T, segments, shared=False, between=lambda: None):
     be = backend_with_env(**({"CG_ATTN_SEG_FROM": "1"} if segments else {}))
     H, rng = kvh * rep, np.random.default_rng(T + hd)
@@ -48,17 +60,7 @@ def run(B, kvh, rep, hd, T, segments, shared=False, between=lambda: None):
         x = r(B, 1, K)
         tx = be.from_numpy(x)
         q, k, v = (cases._linear(be, tx, a) for a in tw)
-
-        def finish(t, n, gain):
-            flat = be.reshape(be.transpose(be.reshape(t.move(), (B, 1, n, hd)).move(), 1, 2).move(), (B * n, hd))
-            y = cases._rmsnorm_ops(be, flat, gain, hd, (B * n, hd))
-            del flat  # (the norm stays open if nobody else holds the product)
-            y = be.reshape(y.move(), (B, n, 1, hd))
-            c, s = (be.broadcast(be.reshape(be.slice(a, 0, pos, 1).move(), (1, 1, 1, hd)).move(), (B, n, 1, hd)) for a in tt)
-            mixed = cases._rot_half(be, y, hd // 2)
-            return be.add(be.mul(c.move(), y.move()).move(), be.mul(s.move(), mixed.move()).move())
-
-        q, k = finish(q, H, tg[0].clone()), finish(k, kvh, tg[1].clone())
+        q, k = finish(be, q, (B, H, hd), tg[0].clone(), tt, pos), finish(be, k, (B, kvh, hd), tg[1].clone(), tt, pos)
         v = be.transpose(be.reshape(v.move(), (B, 1, kvh, hd)).move(), 1, 2)
         tk = be.concat(tk.move(), k.move(), 2)
         if not shared:
@@ -100,6 +102,36 @@ def test_one_cache_for_keys_and_values(B, kvh, rep, hd, T, segments):
     run(B, kvh, rep, hd, T, segments, shared=True)
 
 
+def rows_of(T, hd, apart):
+    """q and the newest row of K of a step behind T positions, from whole numbers; `apart`: over one cache, so that the heads get a launch of their own."""
+    be = backend_with_env()
+    B, kvh, rep = 2, 3, 2
+    H, rng = kvh * rep, np.random.default_rng(hd)
+    whole = lambda *s: rng.integers(-3, 4, s).astype(np.float32)  # noqa: E731
+    tw = [be.from_numpy(whole(n * hd, K)) for n in (H, kvh, kvh)]
+    gains = [be.from_numpy(rng.uniform(0.5, 1.5, hd).astype(np.float32)) for _ in range(2)]
+    angle = rng.uniform(0, 6.28, (T + 2, hd)).astype(np.float32)
+    tables = [be.from_numpy(f(angle)) for f in (np.cos, np.sin)]
+    tk, tv = (be.from_numpy(whole(B, kvh, T, hd)) for _ in range(2))
+    for pos in (T, T + 1):
+        tx = be.from_numpy(whole(B, 1, K))
+        q, k, v = (cases._linear(be, tx, a) for a in tw)
+        q, k = finish(be, q, (B, H, hd), gains[0].clone(), tables, pos), finish(be, k, (B, kvh, hd), gains[1].clone(), tables, pos)
+        v = be.transpose(be.reshape(v.move(), (B, 1, kvh, hd)).move(), 1, 2)
+        tk, tv = be.concat(tk.move(), k.move(), 2), be.concat(tv.move(), v.move(), 2)
+        held = q.clone()
+        be.to_numpy(cases.decode_attention_ops(be, q, tk.clone(), (tk if apart else tv).clone(), rep))
+    return [be.to_numpy(held), be.to_numpy(be.slice(tk, 2, T + 1, 1))]
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("T", [37, 300])
+def test_rows_do_not_depend_on_the_launch(T, hd):
+    """Sums of squares of whole numbers are exact in any order: all that follows them is the same to the bit."""
+    for a, b in zip(rows_of(T, hd, False), rows_of(T, hd, True)):
+        np.testing.assert_array_equal(a, b)
+
+
 def test_which_kernels(tmp_path):
     """Attention finishes the heads of the step that appends in place, or one launch of its own does."""
     kernel_names.run(tmp_path, r"""
@@ -113,5 +145,8 @@ for steps, expected in ((T.ROWS, (0, 1, 0)), (T.SEGMENTS, (0, 0, 1)), (T.APART, 
         row, seg = (sum("decode_attention_%s_kernel" % k in n and "RawHeads" in n for n in names) for k in ("row", "seg"))
         print(step, own, row, seg, flush=True)
         assert (own, row, seg) == expected, names
+for apart in (False, True):
+    names = launches(be, T.rows_of, 300, 64, apart)
+    assert sum("RawHeads" in n for n in names) == 1 - apart, names
 print("done", flush=True)
 """)
