@@ -26,7 +26,8 @@ def close(got, want, tol, what=""):
 
 
 def part_of_rows(be, x, before=8, behind=5):
-    """x [.., n] as a view of the columns before .. before + n of wider rows."""
+    """x [.., n] as a view of the columns before .. before + n of wider rows.  (n a multiple of 4 and `behind` too: rows at 16 bytes, which
+    the kernels for few rows want; else others run.)"""
     wide = np.concatenate([np.full(x.shape[:-1] + (before,), 7.0), x, np.full(x.shape[:-1] + (behind,), -9.0)], -1).astype(np.float32)
     return be.slice(be.from_numpy(wide), x.ndim - 1, before, x.shape[-1])
 
@@ -88,7 +89,7 @@ RESIDUAL = [  # rows, width, [(K, poly, gate)], weight dtype
     (70, 256, [(512, False, True), (768, True, True)], "bf16"), (33, 130, [(52, False, False), (48, True, True)], "f32"), (65, 96, [(64, False, True)], "f32")]
 
 
-def run_residual(be, case, seed=0):
+def run_residual(be, case, seed=0, behind=5):
     rows, width, parts, dt = case
     rng = np.random.default_rng(seed)
     eps = 2e-3
@@ -98,7 +99,7 @@ def run_residual(be, case, seed=0):
         y, w = rng.standard_normal((1, rows, K)).astype(np.float32), bf16(rng.standard_normal((width, K)) * K ** -0.5)
         g, gb = rng.standard_normal((1, rows, width)).astype(np.float32), rng.standard_normal(width).astype(np.float32)
         c = rng.standard_normal(4).astype(np.float32)
-        d = {"y": part_of_rows(be, y) if i else be.from_numpy(y), "w": weight(be, w, dt)}
+        d = {"y": part_of_rows(be, y, behind=behind) if i else be.from_numpy(y), "w": weight(be, w, dt)}
         z = y[0].astype(np.float64)
         if poly:
             d["poly"] = be.from_numpy(c)
@@ -167,14 +168,14 @@ def attention_case(rng, B, S, o, norms=True, talk=True):
     return {n: a.astype(np.float32) for n, a in t.items()}
 
 
-def run_attention(be, t, o, portions):
+def run_attention(be, t, o, portions, behind=5):
     """The sequence in portions of these lengths, through the cache: [B, S, heads * vdim]."""
     B = t["q"].shape[0]
     kc, vc = be.zeros((B, o["kv_heads"], 0, o["dim"]), 0), be.zeros((B, o["kv_heads"], 0, o["vdim"]), 0)
     small = {n: be.from_numpy(t[n]) for n in ("q_norm", "k_norm", "talk") if n in t}
     at, outs = 0, []
     for n in portions:
-        part = {c: part_of_rows(be, t[c][:, at:at + n]) for c in ("q", "k", "v")}
+        part = {c: part_of_rows(be, t[c][:, at:at + n], behind=behind) for c in ("q", "k", "v")}
         out, kc, vc = be.block_attention({**part, **small, "k_cache": kc.move(), "v_cache": vc.move()}, position=at, **o)
         at += n
         w = o.get("window")
@@ -184,8 +185,8 @@ def run_attention(be, t, o, portions):
     return np.concatenate(outs, 1)
 
 
-def check_attention(be, t, o, portions, tol=3e-5):
-    got = run_attention(be, t, o, portions)
+def check_attention(be, t, o, portions, tol=3e-5, behind=5):
+    got = run_attention(be, t, o, portions, behind)
     for b in range(t["q"].shape[0]):
         want = attention_reference(t["q"][b], t["k"][b], t["v"][b], o, t.get("q_norm"), t.get("k_norm"), t.get("talk"))
         close(got[b], want, tol, f"attention {o}, portions {portions[:6]}, sequence {b}")
@@ -264,10 +265,10 @@ MIXED = {  # name: (options, batch, portions, norms, talk)
 }
 
 
-def run_mixed_case(be, name):
+def run_mixed_case(be, name, behind=5):
     o, B, portions, norms, talk = MIXED[name]
     rng = np.random.default_rng(sum(map(ord, name)))
-    check_attention(be, attention_case(rng, B, sum(portions), o, norms, talk), o, portions, tol=6e-5)
+    check_attention(be, attention_case(rng, B, sum(portions), o, norms, talk), o, portions, tol=6e-5, behind=behind)
 
 
 def run_mixed_needles(be, o, portions):
@@ -494,7 +495,7 @@ def experts_reference(t, top, groups, keep, limit):
     return out
 
 
-def run_experts(be, case, seed=0, change=None):
+def run_experts(be, case, seed=0, change=None, behind=5):
     rows, width, count, top, groups, keep, ff, K, dt = case
     rng = np.random.default_rng(seed + rows)
     t = expert_case(rng, rows, width, count, ff, dt)
@@ -505,7 +506,7 @@ def run_experts(be, case, seed=0, change=None):
     if K:
         y, w = rng.standard_normal((1, rows, K)).astype(np.float32), bf16(rng.standard_normal((width, K)) * K ** -0.5)
         want = want + scale * (y[0].astype(np.float64) @ w.T)
-        br = [{"y": part_of_rows(be, y), "w": weight(be, w, dt)}]
+        br = [{"y": part_of_rows(be, y, behind=behind), "w": weight(be, w, dt)}]
     want = want + scale * experts_reference(t, top, groups, keep, limit)
     ex = {n: be.from_numpy(t[n]) for n in ("logits", "correction")}
     ex["h"] = be.from_numpy(t["h"]) if dt == "f32" else be.cast(be.from_numpy(t["h"]), BF16)
