@@ -315,7 +315,7 @@ def measure(config, steps, warmup, batch=None, prefill=None, decode=None, seed=0
             "bound": "hbm", "bytes_per_step": step_bytes, "achieved": round(step_rate / 1e9, 2), "peak": HBM_PEAK / 1e9,
             "unit": "GB/s", "frac": round(step_rate / HBM_PEAK, 4),
             "skinny_gemm_kernels": {
-                "kernels": "skinny_kt_wide / skinny_kt_mfma_xreg / skinny_kt_narrow / skinny_nn (M <= 8)",
+                "kernels": "skinny_group / skinny_gated / skinny_residual / head_norm_rope_finish; skinny_kt_* / skinny_nn (M <= 8)",
                 "achieved": round(skinny_rate / 1e9, 2), "unit": "GB/s", "frac": round(skinny_rate / HBM_PEAK, 4),
                 "launches_timed": n_s, "avg_launch_us": round(ms_s / max(n_s, 1) * 1e3, 3),
                 "timed_in": "an untimed pass of its own, before the timed region (every 8th launch)",

@@ -417,8 +417,8 @@ struct DeferredWrite {
     Pending *prog = nullptr;  // owned
 };
 
-// x / pow(sum(x*x) / n + eps, e) * gamma applied to the left operand while a decode-time product loads it:
-// (the product's kernel forms the rows' sums itself).
+// x / pow(sum(x*x) / n + eps, e) * gamma applied to the left operand while a decode-time product loads it (the
+// product's kernel forms the rows' sums itself).
 struct NormFuse {
     const uint32_t *gamma; // [K]
     uint32_t n_bits, eps_bits, exp_bits;

@@ -27,8 +27,8 @@
 //                      skinny_kt_wide / _narrow: a wave per output column (or per 4 columns, or a
 //                      column per 16/32 lanes for short K), 16-byte loads along K, wave shuffle
 //                      reduction;
-//                      skinny_kt_mfma_xreg: batches of them on the 4x4x1 matrix instruction with the
-//                      activations held in registers; without a batch: skinny.hpp.
+//                      skinny_kt_mfma_xreg: batches of them, and products alone that skinny_alone leaves here, on the
+//                      4x4x1 matrix instruction with the activations held in registers; others: skinny.hpp.
 //   skinny_nn_kernel   M <= 8 with N-contiguous B rows (p.V of a decode step), split over K
 //                      with a second pass that adds the partial sums.
 //   simple_gemm_kernel u32 (wrapping) and any shape the others decline.
@@ -1103,11 +1103,10 @@ static inline bool xreg_narrow(uint32_t M, uint32_t K) { return M >= 1 && M <= 8
 // X[j][k] for the k values of block b, so one 16-byte weight load per lane drives four
 // instructions that update all 4 (rows) x 4 (columns) partial sums of the block.  Against
 // the FMA kernels this needs a quarter of the vector issue slots.  The four waves of a
-// workgroup split each 2048-wide chunk of k into runs of 512 (a wave reads 2 KiB in a row of
-// each weight row: measured 12 % faster on the gate / up pair than interleaving the waves
-// every 256 bytes), keep their share of the chunk's activations in registers (8 x 16 bytes
+// workgroup split each 2048-wide chunk of k into runs of 512, keep their share of the chunk's activations in registers (8 x 16 bytes
 // per lane and row group) and reuse it for CG groups of four columns, so the activation rows
 // are fetched once per 4 * CG columns.
+//
 // Where a lane's k values lie inside a chunk of TRIPS * 256: trip t covers k0 + kb + ks * t .. + 3.  Whole chunks: a wave
 // takes a quarter of the chunk in a row (2 KiB in a row of each weight row: measured 12 % faster on the gate / up pair than
 // interleaving the waves every 256 bytes).  A ragged last chunk: the waves interleaved every 64 values of k, so that what
@@ -1122,8 +1121,7 @@ template <class F> static void xreg_either(uint32_t K, int trips, F f) { // f(is
     else f(std::false_type{});
 }
 // A chunk's work with as many trips as what is left of K has (or one more): f(their number, as a constant).  Trips that lie behind K
-// altogether would be asked for like any others, clamped.  us with all of a chunk's trips and so: 4 x 512 x 8192 twice in a launch 23.6 and
-// 14.7, 4 x 2308 x 12288 24.7 and 19.1, with a residual sum 30.0 and 24.5.
+// altogether would be asked for like any others, clamped: 4 x 2308 x 12288 24.7 us with all of a chunk's trips, 19.1 so.
 template <int TRIPS, bool WHOLE, class F> __device__ __forceinline__ void xreg_chunk(uint32_t left, F f) {
     static_assert(TRIPS == 8 || TRIPS == 4, "chunks of 2048 or 1024");
     constexpr std::integral_constant<int, TRIPS> all{};
@@ -1143,14 +1141,10 @@ template <int TRIPS, bool WHOLE, class F> __device__ __forceinline__ void xreg_c
 }
 // Four values of a row from k on, and what they count for: zeros behind K.  Loads behind K are clamped, not tested: a test in front of
 // every load leaves the compiler without a count of what is on its way, and it then waits for all of it before each of several groups.
-// The kernels below run for a few microseconds, most of them one trip to memory; around it nothing waits that need not: every load of
-// a chunk is on its way before the first wait, the sums over lanes stay out of LDS (four_sums), a norm's divisor is worked out
-// meanwhile, and the arguments come in two trips.  Four rows, us a launch with guarded loads, shuffles, the divisor at the end and
-// arguments field by field, and so: q, k and v with the rotary embedding 2048 -> 3072 11.8 and 9.7, gate and up 2048 -> 8192 26.4 and 24.3.
-template <bool WHOLE, bool NT = false> __device__ __forceinline__ float4v xreg_at(const uint32_t *row, uint32_t k, uint32_t K) {
-    const float4v *const p = reinterpret_cast<const float4v *>(row + (WHOLE ? k : min(k, K - 4)));
-    if constexpr (NT) return __builtin_nontemporal_load(p);
-    else return *p;
+// The kernel below runs for a few microseconds, most of them one trip to memory; around it nothing waits that need not: every load of
+// a chunk is on its way before the first wait, and the sums over lanes stay out of LDS (four_sums).
+template <bool WHOLE> __device__ __forceinline__ float4v xreg_at(const uint32_t *row, uint32_t k, uint32_t K) {
+    return *reinterpret_cast<const float4v *>(row + (WHOLE ? k : min(k, K - 4)));
 }
 template <bool WHOLE> __device__ __forceinline__ float4v xreg_within(float4v v, uint32_t k, uint32_t K) {
     if constexpr (!WHOLE) {

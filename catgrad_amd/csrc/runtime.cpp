@@ -203,8 +203,8 @@ static bool norm_fuse_of(const cg_tensor *x, NormFuse *nf, cg_tensor *h) {
 }
 
 // t0 + t1 with one term a decode-time product nobody has needed yet and of the extent that the products' residual
-// store takes (the residual stream after an o or down projection): worth computing where it stands — the add runs
-// in the product's store and the row sums of squares come with it — rather than carrying it into a longer program.
+// store takes (the residual stream after an o or down projection): worth computing where it stands, with the add in
+// the product's store, rather than carrying it into a longer program.
 static bool residual_sum_open(const cg_tensor *x) {
     const Pending *p = x->pend;
     if (!p || !x->be->aot || x->dt != CG_F32 || p->nleaf != 2 || p->ninstr != 1 || p->nred != 0) return false;

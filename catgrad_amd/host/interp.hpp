@@ -5,7 +5,8 @@
 //   * `Interpreter` owns the backend and the `Parameters` map; `param()` is the `Load`
 //     operation, which clones the stored tensor (interpreter/interpreter.rs:56-59).
 //   * namespace `ops` gives the DSL spellings of catgrad/src/category/lang/ops.rs and
-//     catgrad/src/stdlib/ops.rs; every call goes through `tensor_op()`.
+//     catgrad/src/stdlib/ops.rs; while a term is recorded every call is one of `tensor_op()`'s, else most
+//     are the backend call itself with the same checks.
 // Values are moved into operations and cloned on fan-out, which is the evaluator's
 // lifetime model (catgrad/src/abstract_interpreter/eval.rs:44-49,107-116).  Shape, Nat
 // and Dtype computations run on the host and issue no backend call (eval.rs:122-187).
