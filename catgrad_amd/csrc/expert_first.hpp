@@ -130,7 +130,7 @@ struct WaveChoice {
 // A workgroup of kExpertThreads: four waves' columns (block x, per_wave each, one after the other) of row * top + choice (block y).
 // In front of the first weight lie the choice and its loads (3.0 us with barriers, 1.6 by waves, a third of it the way of the logits): so the columns are cut for one round of
 // workgroups, and a wave's next column is on its way while this one is multiplied.  The launch beside attention, 8 of 32 experts in bf16: 1024 columns of 2048 values
-// 23.4 -> 20.5 us (67 MB, 13 us at the device's rate), 384 of 1024 12.4 -> 11.8 (and 8.1 with the choice by waves, see there and mixed_step).
+// 23.4 -> 20.5 us (67 MB, 13 us at the device's rate), 384 of 1024 12.4 -> 11.8 (now, with mixed_step's loads all ahead, 9.4, and 7.7 to 8.1 with the choice by waves).
 // LDS: route_bytes(p).
 constexpr int kExpertThreads = 256, kExpertWaves = 4;
 inline size_t route_bytes(const ExpertsPlan &p) { return (route_floats(p.experts, p.groups) + 2 * (size_t)p.top) * 4; }
