@@ -4,39 +4,18 @@ import numpy as np
 import pytest
 
 import block_cases as C
-import kernel_names
 
 pytestmark = pytest.mark.gpu
 
+
 # (heads, KV heads, key channels, value channels, ranks)
-TOKEN = [
+@pytest.mark.parametrize("heads,kv,dim,vdim,ranks", [
     (1, 1, 1, 4, (4, 4)), (2, 1, 31, 60, (64, 60)), (4, 2, 32, 64, (8, 64)), (2, 2, 128, 64, (68, 4)),  # four lanes' sixteenths of a row
     (2, 1, 127, 68, (64, 12)), (3, 3, 65, 128, (4, 128)), (2, 1, 128, 124, (72, 128)),  # eighths
-    (2, 1, 3, 5, (4, 4)), (2, 1, 64, 62, (8, 8)), (2, 2, 40, 63, (72, 8)), (3, 3, 128, 65, (64, 64)), (2, 1, 127, 127, (128, 4))]  # values that fill no lane
-GENERAL = [(2, 1, 129, 64, (8, 8)), (2, 1, 64, 132, (8, 8)), (2, 2, 16, 3, (8, 8)), (2, 2, 16, 16, (132, 8)), (2, 2, 16, 16, (8, 10))]  # the general kernel's
-
-
-def run(be, heads, kv, dim, vdim, ranks):
+    (2, 1, 129, 64, (8, 8)), (2, 1, 64, 132, (8, 8)), (2, 1, 64, 62, (8, 8)), (2, 2, 16, 16, (132, 8)), (2, 2, 16, 16, (8, 10)),  # the general kernel's
+])
+def test_one_token_behind_a_state(hip, heads, kv, dim, vdim, ranks):
     rng = np.random.default_rng(dim + 1000 * vdim)
     o = C.delta_options(heads, kv, dim, vdim)
-    # (rows of the factored projections' inputs at 16 bytes)
-    C.check_delta(be, C.delta_case(rng, 2, 24, o, 4, *ranks), o, [19, 1, 1, 2, 1], behind=8)
-    C.check_delta(be, C.delta_case(rng, 1, 4, o, 4, *ranks, decay_at=6.0), o, [1, 1, 1, 1], behind=8)
-
-
-@pytest.mark.parametrize("heads,kv,dim,vdim,ranks", TOKEN + GENERAL)
-def test_one_token_behind_a_state(hip, heads, kv, dim, vdim, ranks):
-    run(hip, heads, kv, dim, vdim, ranks)
-
-
-def test_which_kernel(tmp_path):
-    kernel_names.run(tmp_path, r"""
-from catgrad_amd import HipBackend
-import test_hip_delta_token as T
-be = HipBackend(0)
-for sizes in T.TOKEN + T.GENERAL:
-    n = sum("delta_token_kernel" in k for k in launches(be, T.run, be, *sizes))
-    print(sizes, n, flush=True)
-    assert n == (6 if sizes in T.TOKEN else 0)  # (of seven single tokens one has no state yet)
-print("done", flush=True)
-""")
+    C.check_delta(hip, C.delta_case(rng, 2, 24, o, 4, *ranks), o, [19, 1, 1, 2, 1])
+    C.check_delta(hip, C.delta_case(rng, 1, 4, o, 4, *ranks, decay_at=6.0), o, [1, 1, 1, 1])

@@ -3,8 +3,6 @@ residual sums and RMS norms in the loads, at the edges of the waves' shares of k
 import numpy as np
 import pytest
 
-import kernel_names
-
 pytestmark = pytest.mark.gpu
 
 # every number of trips, whole and ragged; shares that end inside a quad of lanes' values; one and several rounds of 8192
@@ -37,15 +35,6 @@ def constant(hip, v, shape):
     return hip.broadcast(hip.ndarray_from_vec_f32([v], ()), shape)
 
 
-def norm_of(hip, x, gamma, power, eps):
-    """x / pow(sum(x x) / n + eps, e) * gamma, every handle given away at its last use: so the norm is left to the products that read it."""
-    _, rows, K = x.shape
-    h, row = hip.from_numpy(x), (1, rows, 1)
-    s = hip.div(hip.sum(hip.mul(h, h).move()).move(), constant(hip, float(K), row).move())
-    d = hip.pow(hip.add(s.move(), constant(hip, eps, row).move()).move(), constant(hip, power, row).move())
-    return hip.mul(hip.div(h, hip.broadcast(d.move(), x.shape).move()).move(), hip.broadcast(gamma, x.shape).move())
-
-
 @pytest.mark.parametrize("power,eps", [(0.5, 1e-5), (0.25, 1e-5), (0.5, 0.0)])
 @pytest.mark.parametrize("rows", [1, 2, 4, 7])
 @pytest.mark.parametrize("K", KS)
@@ -58,7 +47,11 @@ def test_norm_and_gate(hip, K, rows, power, eps):
     tg, tw = hip.from_numpy(gamma), [hip.from_numpy(a) for a in w]
 
     def normed():
-        return norm_of(hip, x, tg, power, eps)
+        h = hip.from_numpy(x)
+        row = (1, rows, 1)
+        s = hip.div(hip.sum(hip.mul(h, h).move()).move(), constant(hip, float(K), row).move())
+        d = hip.pow(hip.add(s.move(), constant(hip, eps, row).move()).move(), constant(hip, power, row).move())
+        return hip.mul(hip.div(h, hip.broadcast(d, (1, rows, K)).move()).move(), hip.broadcast(tg, (1, rows, K)).move())
 
     f = x[0].astype(np.float64)
     y = f / (np.mean(f * f, -1, keepdims=True) + eps) ** power * gamma
@@ -77,67 +70,3 @@ def test_norm_and_gate(hip, K, rows, power, eps):
     s = want[0] / (1.0 + np.exp(-want[0]))
     # silu' <= 1.1; the sigmoid's own roundings
     assert (np.abs(got - s * want[1]) <= 1.1 * bound[0] * np.abs(want[1]) + np.abs(s) * bound[1] + 2.0 ** -20 * np.abs(s * want[1])).all()
-
-
-@pytest.mark.parametrize("rows", [2, 3, 5, 8])
-@pytest.mark.parametrize("K", [1020, 1028, 2048, 2052, 4100])
-def test_eight_columns(hip, K, rows):
-    """Products of at least 8192 columns share the rows among eight: their last workgroup's columns, alone, in pairs and behind a norm."""
-    rng = np.random.default_rng(K + rows)
-    x = rng.integers(-3, 4, (1, rows, K)).astype(np.float32)
-    for N in (8193, 8199):
-        w = [rng.integers(-3, 4, (n, K)).astype(np.float32) for n in (N, 8192)]
-        tx, tw = hip.from_numpy(x), [hip.from_numpy(a) for a in w]
-        np.testing.assert_array_equal(hip.to_numpy(linear(hip, tx, tw[0]))[0], x[0] @ w[0].T)
-        for y, a in zip([linear(hip, tx, t) for t in tw], w):
-            np.testing.assert_array_equal(hip.to_numpy(y)[0], x[0] @ a.T)
-        gamma = rng.uniform(0.5, 1.5, K).astype(np.float32)
-        got = hip.to_numpy(linear(hip, norm_of(hip, x, hip.from_numpy(gamma), 0.5, 1e-5), tw[0]))[0]
-        f = x[0].astype(np.float64)
-        y = f / np.sqrt(np.mean(f * f, -1, keepdims=True) + 1e-5) * gamma
-        assert (np.abs(got - y @ w[0].astype(np.float64).T) <= (K / 16 + 64) * 2.0 ** -24 * (np.abs(y) @ np.abs(w[0]).T)).all()
-
-
-# rows, K, columns of a product alone, and whether it is worth these kernels (their lanes busy, or enough columns)
-ALONE = [(2, 1024, 2050, True), (4, 576, 2050, True), (4, 572, 2050, False), (2, 1028, 2050, False), (8, 2048, 2050, True), (5, 2052, 2050, False), (8, 3840, 2050, True),
-         (8, 2560, 2050, False), (1, 2048, 16380, False), (1, 960, 16384, True), (1, 956, 16384, False), (8, 576, 16384, False)]
-
-
-def alone(hip, rows, K, N):
-    rng = np.random.default_rng(K)
-    x, w = rng.integers(-3, 4, (1, rows, K)).astype(np.float32), rng.integers(-3, 4, (N, K)).astype(np.float32)
-    np.testing.assert_array_equal(hip.to_numpy(linear(hip, hip.from_numpy(x), hip.from_numpy(w)))[0], x[0] @ w.T)
-
-
-def test_which_kernels(tmp_path):
-    """The kernels with the norm in their loads run where it stands in front of the products, eight columns where there are enough, and a
-    product alone goes where the rule says."""
-    kernel_names.run(tmp_path, r"""
-import re
-from catgrad_amd import HipBackend
-import test_hip_skinny as T
-be = HipBackend(0)
-
-
-def count(names, pattern):
-    return sum(bool(re.search(pattern, n)) for n in names)
-
-
-for rows, K in ((1, 260), (1, 4100), (2, 1024), (4, 3084), (7, 8196)):
-    names = launches(be, T.test_norm_and_gate, be, K, rows, 0.5, 1e-5)
-    print("norm", rows, K, flush=True)
-    # (one product, three, and the gated pair, each with the norm in its loads)
-    assert count(names, r"skinny_group_kernel.*Li4ELb1EE") == 2 and count(names, r"skinny_gated_kernel.*Lb1EE") == 1 and not count(names, "fused"), names
-    names = launches(be, T.test_whole_numbers, be, K, rows)
-    # (three widths: a group of three, a residual sum; the products alone are below)
-    assert count(names, r"skinny_group_kernel.*Li4ELb0EE") >= 3 and count(names, "skinny_residual_kernel") == 3, names
-for rows, K in ((2, 1028), (8, 2052)):
-    names = launches(be, T.test_eight_columns, be, K, rows)
-    print("eight", rows, K, flush=True)
-    assert count(names, r"skinny_group_kernel.*Li8ELb1EE") == 2 and count(names, r"skinny_group_kernel.*Li8ELb0EE") == 2, names
-for rows, K, N, there in T.ALONE:
-    names = launches(be, T.alone, be, rows, K, N)
-    print("alone", rows, K, N, flush=True)
-    assert count(names, "skinny_group_kernel") == there, names
-print("done", flush=True)
-""")
