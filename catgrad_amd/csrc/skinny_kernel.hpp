@@ -157,6 +157,7 @@ template <class F> void with_cut(uint32_t rows, uint32_t K, F f) {
     else if (K <= 2048) go(one, two, four, once);
     else if (K <= 3072) go(one, std::integral_constant<int, 3>{}, four, once);
     else if (K <= 4096) go(one, four, four, once);
+    else if (K <= 6144) go(one, std::integral_constant<int, 3>{}, eight, once); // (a fourth trip of idle lanes: the gated pair 1 x 4100 x 2052 18.8 us, 15.5 without, 1 x 5120 x 4608 35.9 and 30.4)
     else go(one, four, eight, loop);
 }
 

@@ -52,6 +52,13 @@ def test_norm_left_to_the_products(hip, K, rows, power, eps):
     assert (np.abs(got - s * want[1]) <= 1.1 * bound[0] * np.abs(want[1]) + np.abs(s) * bound[1] + 2.0 ** -20 * np.abs(s * want[1])).all()
 
 
+@pytest.mark.parametrize("K", [5120, 5124, 6140, 6144, 6148])
+def test_one_row_in_three_trips(hip, K):
+    """Eight waves of one row share up to 6144 values of k in three trips (4100 is among the others' sizes)."""
+    whole.test_whole_numbers(hip, K, 1)
+    test_norm_left_to_the_products(hip, K, 1, 0.5, 1e-5)
+
+
 @pytest.mark.parametrize("rows", [2, 3, 5, 8])
 @pytest.mark.parametrize("K", [1020, 1028, 2048, 2052, 4100])
 def test_eight_columns(hip, K, rows):
