@@ -1568,15 +1568,23 @@ static SkinnyInput skinny_input(const MmArgs &a, const NormFuse *nf) {
 static SkinnyProduct skinny_product(const MmArgs &a) { // its rows stored as they are
     return {reinterpret_cast<const float *>(a.B), a.b_sn, a.N, 0, a.C, a.N, 0, nullptr, nullptr, a.N, 0};
 }
-// Whether a product that shares its launch with no other goes there too.  Lanes whose values lie behind the end of a wave's share of k idle
-// (see with_cut), which costs more than the barriers and the sums that it saves: us a launch there and on the matrix instruction's kernel
-// 5 x 2052 x 12288 39.5 and 24.9, 4 x 260 x 8192 6.3 and 4.6, but 8 x 2048 x 12288 19.8 and 33.9.  One row of fewer columns takes as long
-// there or up to a tenth longer (1 x 4096 x 8192 22.0 and 20.4).  From 16384 columns on the other side is skinny_kt_wide_kernel: 1 x 1024 x
-// 32768 20.8 and 30.8, 5 x 260 x 49152 32.1 and 21.8.
+// Whether a product that shares its launch with no other goes there too: where enough of the lanes' loads are values, `least` sixteenths of a
+// whole cut of k (see with_cut).  What is enough differs by the rows that share a lane's weights, by the columns (from 8192 on eight a
+// workgroup) and, from 16384 columns on, where the other side is skinny_kt_wide_kernel.  Weights from memory, us a launch on the other side and here:
+//   1 row    4096 x 8190 26.1, 22.9; 2304 x 4096 10.4, 8.7; 576 x 4096 5.1, 4.8; less than 9 / 16: 1028 x 12288 11.5, 12.6; 260 x 8190 5.0, 5.6
+//   2 rows   3584 x 8190 23.4, 20.5; 2052 x 4096 9.2, 9.2; 260 x 16384 9.9, 7.6; but 1028 x 4096 6.1, 6.9
+//   4 rows   3584 x 4096 14.6, 13.8; 4100 x 12288 40.0, 36.4; 2880 x 32768 70.2, 66.9; 260 x 16384 10.4, 9.6; but 2560 x 8190 19.2, 21.8; 2304 x 16384 29.7, 31.9
+//   8 rows   3584 x 3584 29.6, 17.4; 2304 x 8190 32.1, 27.2; 5120 x 8194 60.8, 46.8; 960 x 32768 34.2, 26.9; but 2052 x 12288 36.1, 41.5; 3072 x 16384 49.2, 58.6
 static bool skinny_alone(const MmArgs &a) {
-    const uint32_t cut = a.M == 1 ? (a.K <= 4096 ? 1024 : 8192) : a.K <= 1024 ? 1024 : 2048, whole = (a.K + cut - 1) / cut * cut;
-    const bool many = a.N >= 16384, rounds = a.M > 1 && a.K > cut;
-    return (a.M > 1 || many) && 16ull * a.K >= (many || rounds ? 15ull : 9ull) * whole;
+    const uint32_t M = a.M, K = a.K, cut = M > 1 ? (K <= 1024 ? 1024 : 2048) : K <= 4096 ? 1024 : K <= 6144 ? 6144 : 8192, whole = (K + cut - 1) / cut * cut;
+    const bool many = a.N >= 16384, rounds = M > 1 && K > 2048;
+    uint32_t least = 9;
+    if (M > 1 && K > 6144) least = 0; // (one idle part of four rounds and more: 8 x 9216 x 18000 160.9, 135)
+    else if (M == 2) least = many || rounds ? 0 : 9;
+    else if (M > 2 && M <= 4) least = rounds ? (K > 4096 ? 0 : many ? 11 : 14) : many && K <= 1024 ? 0 : 9;
+    else if (M > 4 && many) least = K <= 1024 ? 12 : 15;
+    else if (M > 4 && rounds && a.N >= 8192) least = M > 6 ? 9 : 13; // (this side takes as long for five rows as for eight: 2560 x 12288 37.5 and 42.0, 46.1 and 42.8)
+    return 16ull * K >= (uint64_t)least * whole;
 }
 static bool skinny_operands(const MmArgs &a) { return a.a_vec && a.b_vec && a.a_sk == 1 && a.b_sk == 1 && takes_skinny(a.M, a.K); }
 

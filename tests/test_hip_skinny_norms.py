@@ -78,9 +78,12 @@ def test_eight_columns(hip, K, rows):
         assert (np.abs(got - y @ w[0].astype(np.float64).T) <= (K / 16 + 64) * 2.0 ** -24 * (np.abs(y) @ np.abs(w[0]).T)).all()
 
 
-# rows, K, columns of a product alone, and whether it is worth these kernels (their lanes busy, or enough columns)
-ALONE = [(2, 1024, 2050, True), (4, 576, 2050, True), (4, 572, 2050, False), (2, 1028, 2050, False), (8, 2048, 2050, True), (5, 2052, 2050, False), (8, 3840, 2050, True),
-         (8, 2560, 2050, False), (1, 2048, 16380, False), (1, 960, 16384, True), (1, 956, 16384, False), (8, 576, 16384, False)]
+# rows, K, columns of a product alone, and whether it is worth these kernels (enough of the lanes busy for its rows and columns)
+ALONE = [(1, 576, 2050, True), (1, 572, 2050, False), (1, 1028, 16384, False), (1, 4100, 2050, True), (1, 6148, 2050, True), (1, 8196, 2050, False), (1, 956, 16384, True),
+         (2, 1024, 2050, True), (2, 1028, 2050, False), (2, 2052, 2050, True), (2, 260, 16384, True), (2, 260, 16380, False),
+         (4, 576, 2050, True), (4, 572, 2050, False), (3, 3580, 2050, False), (3, 3584, 2050, True), (4, 4100, 2050, True), (4, 2812, 16384, False), (4, 2816, 16384, True), (3, 260, 16384, True),
+         (8, 2048, 2050, True), (5, 2052, 2050, False), (5, 2304, 8188, True), (8, 2560, 2050, True), (6, 3324, 8192, False), (5, 3328, 8192, True), (7, 2304, 8192, True), (7, 2300, 8192, False), (8, 6148, 8194, True),
+         (8, 764, 16384, False), (8, 768, 16384, True), (5, 3836, 16384, False), (5, 3840, 16384, True), (8, 6148, 16384, True)]
 
 
 def alone(hip, rows, K, N):
